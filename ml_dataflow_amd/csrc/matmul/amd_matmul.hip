@@ -72,11 +72,82 @@ static int launch_staged(const GemmParams & p, long grid, hipStream_t stream) {
 }
 
 /* direct-to-LDS kernel: static LDS */
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool PK, bool QK, int MODE, int GATHER = GATHER_NONE>
-static int launch_direct(const GemmParams & p, long grid, hipStream_t stream) {
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PK, bool QK, int MODE, int GATHER = GATHER_NONE>
+static int launch_direct_tile(const GemmParams & p, long grid, hipStream_t stream) {
 	constexpr int threads = WAVES_M * WAVES_N * 64;
-	hipLaunchKernelGGL((gemm_bf16_direct_kernel<BM, BN, WAVES_M, WAVES_N, PK, QK, MODE, GATHER>), dim3((unsigned int) grid), dim3(threads), 0, stream, p);
+	hipLaunchKernelGGL((gemm_bf16_direct_kernel<BM, BN, WAVES_M, WAVES_N, PK, QK, MODE, GATHER, STAGES>), dim3((unsigned int) ((grid + 7) & ~7L)), dim3(threads), 0, stream, p);
 	return check_launch();
+}
+
+static long tiles_of(long extent, long tile) { return (extent + tile - 1) / tile; }
+
+/* The work-group tiles of the direct kernel, and which of them a problem runs on (BIG: the persistent kernels instead).
+ *
+ * A problem with few tiles takes as long as one work-group needs for its k-tiles, and what a k-tile costs one work-group
+ * grows much more slowly than its tile: measured on problems of 88 to 512 tiles, K of 1024-4096 (microseconds per k-tile
+ * and work-group with the compute units sharing the load) 64 x 32: 0.20-0.28, 64 x 64: 0.21-0.31, 64 x 128: 0.29-0.44,
+ * 128 x 128 with three stages and eight waves: 0.47-0.66, two of them with two stages on one compute unit: 0.50 each (0.56
+ * alone), the persistent 256 x 256: 1.1-1.4.  So the cheapest tile is the one with the least (rounds of tiles over the
+ * compute units) x (cost of a k-tile), small tiles while they still fit one round and larger ones behind that.  1408 x
+ * 2048 x 256 takes 10 us on 64 x 64 tiles (29 on 128 x 128 with one k-tile in flight, which this replaced), 4096 x 4096 x
+ * 512 31 us on 64 x 128 (55), 4096 x 4096 x 2048 66 us on pairs of 128 x 128 (92 on the persistent kernel). */
+enum { TILE_64x32, TILE_64x64, TILE_64x128, TILE_128x128, TILE_128x128_PAIR, TILE_BIG, NUM_TILES };
+static const struct { int bm, bn, cost; } TILES[NUM_TILES] = {{64, 32, 21}, {64, 64, 25}, {64, 128, 36}, {128, 128, 58}, {128, 128, 50}, {256, 256, 130}};
+#define TILE_PAIR_COST_ALONE 62      /* of a k-tile of the pair's tile where it has the compute unit to itself, or its lines come from HBM */
+
+/* tiles of the launch for tile `which`.  Ragged N: the group sizes are on the device; a group of the mean size has on
+ * average half a tile more than its rows fill, and at least one */
+static long tiles_in_launch(int which, int mode, const GemmParams & p) {
+	const long tm = tiles_of(p.M, TILES[which].bm), bn = TILES[which].bn;
+	if (mode == MODE_SINGLE) {
+		return tm * tiles_of(p.N, bn);
+	}
+	if (mode == MODE_RAGGED_K) {
+		return tm * tiles_of(p.N, bn) * p.num_groups;
+	}
+	const long filled = p.N < p.num_groups ? p.N : p.num_groups;
+	const long tn = p.N / bn + filled / 2;
+	return tm * (tn > filled ? tn : filled);
+}
+
+/* upper bound for the grid */
+static long grid_of(int which, int mode, const GemmParams & p) {
+	if (mode != MODE_RAGGED_N) {
+		return tiles_in_launch(which, mode, p);
+	}
+	return tiles_of(p.M, TILES[which].bm) * ((long) p.N / TILES[which].bn + (p.N < p.num_groups ? p.N : p.num_groups));
+}
+
+static int choose_tile(int mode, const GemmParams & p, long cu_count) {
+	const bool big_ok = p.M >= 256 && (mode == MODE_RAGGED_N || p.N >= 256);
+	int best = TILE_64x32;
+	long best_cost = 0;
+	for (int which = 0; which < NUM_TILES; which++) {
+		if (which == TILE_BIG && !big_ok) {
+			continue;
+		}
+		const long tiles = tiles_in_launch(which, mode, p);
+		const bool alone = which == TILE_128x128_PAIR && (tiles <= cu_count || mode == MODE_RAGGED_N);
+		const long cost = tiles_of(tiles, cu_count) * (alone ? TILE_PAIR_COST_ALONE : TILES[which].cost);
+		if (which == 0 || cost < best_cost) {
+			best = which;
+			best_cost = cost;
+		}
+	}
+	return best;
+}
+
+/* the direct kernel on one of its tiles */
+template <bool PK, bool QK, int MODE, int GATHER = GATHER_NONE>
+static int launch_direct(const GemmParams & p, int which, hipStream_t stream) {
+	const long grid = grid_of(which, MODE, p);
+	switch (which) {
+		case TILE_64x32: return launch_direct_tile<64, 32, 2, 2, 4, PK, QK, MODE, GATHER>(p, grid, stream);
+		case TILE_64x64: return launch_direct_tile<64, 64, 2, 2, 4, PK, QK, MODE, GATHER>(p, grid, stream);
+		case TILE_64x128: return launch_direct_tile<64, 128, 2, 2, 3, PK, QK, MODE, GATHER>(p, grid, stream);
+		case TILE_128x128: return launch_direct_tile<128, 128, 4, 2, 3, PK, QK, MODE, GATHER>(p, grid, stream);
+		default: return launch_direct_tile<128, 128, 4, 2, 2, PK, QK, MODE, GATHER>(p, grid, stream);
+	}
 }
 
 /* the direct kernel with four stages, for the partial products of a split along K (amd_matmul's few-tile problems) */
@@ -162,15 +233,15 @@ static bool w4_ok(const GemmParams & p) {
 }
 
 static long round_up8(long v) { return (v + 7) & ~7L; }
-static long tiles_of(long extent, long tile) { return (extent + tile - 1) / tile; }
 
 #define BIG_TILE 256, 256, 4, 2          /* 8 waves, wave tile 64 x 128 */
 #define WIDE_TILE 256, 288, 4, 2         /* 8 waves, wave tile 64 x 144: the token side of the ragged-N launches, see launch_gemm */
 #define SMALL_TILE 128, 128, 2, 2        /* 4 waves, wave tile 64 x 64 */
 
-/* grid_big / grid_small: work-group counts for the two tile sizes; `direct` selects the fast kernel */
+/* `direct`: the operands suit the direct-to-LDS kernels.  grid_big / grid_small: work-group counts of the persistent kernel
+ * and of the register-staged one; grid_wide: tiles of 288 token rows (ragged N) */
 template <int MODE>
-static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct, bool big, long grid_big, long grid_small, long cu_count, hipStream_t stream,
+static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct, long grid_big, long grid_small, long cu_count, hipStream_t stream,
 					   long grid_wide = 0) {
 	/* to_trans_a = 1 means A is stored [M][K] (k contiguous); to_trans_b = 1 means B is stored [K][N] (k-major) */
 	const bool pk = !transa;
@@ -178,6 +249,10 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 	if (grid_big <= 0 || grid_small <= 0) {
 		return 0;
 	}
+	/* a caller that named one of the persistent kernels gets it wherever it has enough tiles for half the compute units */
+	const bool named = kernel_choice != AMD_MATMUL_KERNEL_AUTO && p.M >= 256 && (MODE == MODE_RAGGED_N ? (long) p.N / 256 * tiles_of(p.M, 256) : p.N >= 256 ? grid_big : 0) >= 128;
+	const int tile = named ? TILE_BIG : choose_tile(MODE, p, cu_count);
+	const bool big = tile == TILE_BIG;
 	const bool four_ok = direct && big && !qk && w4_ok(p);
 	const bool wide_only = kernel_choice == AMD_MATMUL_KERNEL_FOUR_WAVES_384;
 	bool either = kernel_choice == AMD_MATMUL_KERNEL_AUTO;
@@ -264,7 +339,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 #define PICK(PK, QK) do { \
 		if (direct) { \
 			return big ? launch_stream<BIG_TILE, PK, QK, MODE>(p, grid_big, cu_count, stream) \
-					   : launch_direct<SMALL_TILE, PK, QK, MODE>(p, round_up8(grid_small), stream); \
+					   : launch_direct<PK, QK, MODE>(p, tile, stream); \
 		} \
 		return launch_staged<SMALL_TILE, PK, QK, MODE>(p, round_up8(grid_small), stream); \
 	} while (0)
@@ -273,7 +348,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 #define PICK_GATHER(PK) do { \
 			if (direct) { \
 				return big ? launch_stream<BIG_TILE, PK, false, MODE_RAGGED_N, GATHER_Q_ROWS>(p, grid_big, cu_count, stream) \
-						   : launch_direct<SMALL_TILE, PK, false, MODE_RAGGED_N, GATHER_Q_ROWS>(p, round_up8(grid_small), stream); \
+						   : launch_direct<PK, false, MODE_RAGGED_N, GATHER_Q_ROWS>(p, tile, stream); \
 			} \
 			return launch_staged<SMALL_TILE, PK, false, MODE_RAGGED_N>(p, round_up8(grid_small), stream); \
 		} while (0)
@@ -285,7 +360,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 		/* gathered A: the k-rows of the reduction are fetched through the row map (both operands are k-major here) */
 		if (direct) {
 			return big ? launch_stream<BIG_TILE, true, true, MODE_RAGGED_K, GATHER_P_KROWS>(p, grid_big, cu_count, stream)
-					   : launch_direct<SMALL_TILE, true, true, MODE_RAGGED_K, GATHER_P_KROWS>(p, round_up8(grid_small), stream);
+					   : launch_direct<true, true, MODE_RAGGED_K, GATHER_P_KROWS>(p, tile, stream);
 		}
 		return launch_staged<SMALL_TILE, true, true, MODE_RAGGED_K>(p, round_up8(grid_small), stream);
 	}
@@ -401,10 +476,9 @@ static int run_matmul(Dataflow_Handle * dataflow_handle, int stream_id, GemmPara
 		return -1;
 	}
 	const bool direct = operand_direct_ok(p.A, !transa, p.M, p.K, 0) && operand_direct_ok(p.B, transb != 0, p.N, p.K, 0);
-	/* small problems: 128x128 tiles fill the device better; large ones amortise operand traffic with 256x256 */
 	const long grid_big = tiles_of(p.M, 256) * tiles_of(p.N, 256);
 	const long grid_small = tiles_of(p.M, 128) * tiles_of(p.N, 128);
-	const bool big = grid_big >= cu_count / 2 && p.M >= 256 && p.N >= 256;
+	const bool big = grid_big >= cu_count / 2 && p.M >= 256 && p.N >= 256;     /* enough tiles without splitting K */
 	/* Few tiles and a long K (the router's GEMMs: 64 experts on one side): split K over the idle compute units,
 	 * fp32 partial sums in the caller's workspace, one reduction pass.  Without a workspace that is large enough
 	 * (and 16-byte aligned) the problem runs unsplit. */
@@ -434,7 +508,7 @@ static int run_matmul(Dataflow_Handle * dataflow_handle, int stream_id, GemmPara
 			return check_launch();
 		}
 	}
-	return launch_gemm<MODE_SINGLE>(p, transa, transb, direct, big, grid_big, grid_small, cu_count, stream);
+	return launch_gemm<MODE_SINGLE>(p, transa, transb, direct, grid_big, grid_small, cu_count, stream);
 }
 
 /* Ragged K without a C operand: D_g = alpha * (sum over no rows) = 0 for a group without rows.  The GEMM kernels give such
@@ -649,9 +723,8 @@ extern "C" int amd_grouped_matmul(Dataflow_Handle * dataflow_handle, int stream_
 		/* upper bound of n-tiles: every group may end in one partial tile */
 		const long grid_big = tiles_of(p.M, 256) * ((long) p.N / 256 + p.num_groups);
 		const long grid_small = tiles_of(p.M, 128) * ((long) p.N / 128 + p.num_groups);
-		const bool big = p.M >= 256 && (long) p.N / 256 * tiles_of(p.M, 256) >= 128;
 		const long grid_wide = tiles_of(p.M, 256) * ((long) p.N / 288 + p.num_groups);
-		return launch_gemm<MODE_RAGGED_N>(p, transa, transb, direct, big, grid_big, grid_small, extra_cu_count(op_extra), stream, grid_wide);
+		return launch_gemm<MODE_RAGGED_N>(p, transa, transb, direct, grid_big, grid_small, extra_cu_count(op_extra), stream, grid_wide);
 	}
 	if (ragged == AMD_GROUPED_RAGGED_K) {
 		if (transa != 0 || transb != 1 || p.N < 1) {
@@ -662,7 +735,6 @@ extern "C" int amd_grouped_matmul(Dataflow_Handle * dataflow_handle, int stream_
 		const bool direct = operand_direct_ok(p.A, true, p.M, p.K, 0) && operand_direct_ok(p.B, true, p.N, p.K, 0) && (p.strideD % 4 == 0);
 		const long grid_big = tiles_of(p.M, 256) * tiles_of(p.N, 256) * p.num_groups;
 		const long grid_small = tiles_of(p.M, 128) * tiles_of(p.N, 128) * p.num_groups;
-		const bool big = p.M >= 256 && p.N >= 256 && grid_big >= 128;
 		if (p.C == nullptr) {
 			const long long count = (long long) p.M * p.N;
 			const long long blocks = (count / 8 + 255) / 256;
@@ -672,7 +744,7 @@ extern "C" int amd_grouped_matmul(Dataflow_Handle * dataflow_handle, int stream_
 				return -1;
 			}
 		}
-		return launch_gemm<MODE_RAGGED_K>(p, transa, transb, direct, big, grid_big, grid_small, extra_cu_count(op_extra), stream);
+		return launch_gemm<MODE_RAGGED_K>(p, transa, transb, direct, grid_big, grid_small, extra_cu_count(op_extra), stream);
 	}
 	fprintf(stderr, "Error: unknown ragged dimension %d...\n", ragged);
 	return -1;

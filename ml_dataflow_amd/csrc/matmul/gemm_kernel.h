@@ -8,9 +8,10 @@
  *       compute unit walks over many output tiles with the operand stream of the direct kernel below, the MFMA
  *       operands one k-step ahead in registers, and a line-coalesced epilogue through its own LDS scratch.
  *
- *   gemm_bf16_direct_kernel   one work-group per output tile (128 x 128 tiles, small problems).  Operand tiles go from global memory straight into LDS with
- *       16-byte buffer loads (no VGPR staging); out-of-range rows and the k tail are zero-filled by the buffer
- *       bounds check.  Two LDS stages: the loads of k-tile i+1 are in flight while k-tile i is multiplied.
+ *   gemm_bf16_direct_kernel   one work-group per output tile (64 x 32 to 128 x 128, small problems).  Operand tiles go from
+ *       global memory straight into LDS with 16-byte buffer loads (no VGPR staging); out-of-range rows and the k tail are
+ *       zero-filled by the buffer bounds check.  Two to four LDS stages: the loads of the next k-tiles are in flight
+ *       while k-tile i is multiplied.
  *       Operands stored k-contiguous are kept [row][64] in LDS (16-byte chunks XOR-swizzled by row) and read
  *       with ds_read_b128; operands stored k-major are kept [64][rows] (32-byte groups XOR-swizzled by k) and
  *       read with the transposing ds_read_b64_tr_b16, so no layout needs an explicit transpose.
@@ -757,12 +758,18 @@ __device__ __forceinline__ void dma_load16(uint32_t voff, i32x4 rsrc, uint32_t l
 
 #define VOFF_INVALID 0xFFFFFFFFu
 
-/* k-major LDS tile ([64 k][ROWS]): the 16-byte chunk (8 rows) c of k-row k sits at chunk c ^ kmajor_swizzle(k).  A
+/* k-major LDS tile ([64 k][ROWS]): the 16-byte chunk (8 rows) c of k-row k sits at chunk c ^ kmajor_swizzle<ROWS>(k).  A
  * fragment read takes, per 16-lane group, 32 bytes (16 rows) of each of four consecutive k-rows, and the groups that
  * are served together read k-rows 8 apart: bits 0-1 of k spread the four k-rows of a group over the banks, bit 3 the
  * two groups. */
+template <int ROWS>
 __device__ __forceinline__ int kmajor_swizzle(int k) {
-	return ((k & 3) << 2) ^ (((k >> 3) & 1) << 1);
+	static_assert(ROWS >= 128 || ROWS == 64 || ROWS == 32, "k-rows of 32, 64 or at least 128 elements");
+	if (ROWS >= 128) {
+		return ((k & 3) << 2) ^ (((k >> 3) & 1) << 1);
+	}
+	/* a k-row of 128 bytes: its place in the banks already follows bit 0 of k; of 64 bytes: bits 0-1 */
+	return ROWS == 64 ? ((k & 2) ^ (((k >> 3) & 1) << 2)) : (((k >> 3) & 1) << 1);
 }
 
 /* Loads one operand panel (ROWS rows of the operand, all of K) k-tile by k-tile into its LDS tile layout.
@@ -778,7 +785,7 @@ __device__ __forceinline__ int kmajor_swizzle(int k) {
  *   holds global chunk slot ^ ((row >> 1) & 7) of that row.  Consecutive loads of a lane are THREADS/8 rows apart.
  *   Rows past rows_total fall behind the end of the buffer and read as zero; the k tail needs a check.
  * k-major operand ([K][rows_total] in memory, [64][ROWS] in LDS): LDS chunk id -> (k = id/(ROWS/8), slot)
- *   holds global row-chunk slot ^ kmajor_swizzle(k) of that k.  Consecutive loads are THREADS/(ROWS/8) k apart: 8 (the
+ *   holds global row-chunk slot ^ kmajor_swizzle<ROWS>(k) of that k.  Consecutive loads are THREADS/(ROWS/8) k apart: 8 (the
  *   swizzle then alternates between a lane's even and odd loads, which are two chunks apart in the row) or 16.
  *   k past K falls behind the end of the buffer; rows past rows_total need a check (fixed per lane).
  * A lane whose chunk is not valid loads from offset 0xFFFFFFFF, which is out of range of any descriptor.
@@ -833,8 +840,8 @@ struct TileLoader {
 		} else {
 			constexpr int CPR = ROWS / 8;
 			const int k = tid / CPR;
-			const int mc = (tid % CPR) ^ kmajor_swizzle(k);
-			const int mc_odd = (tid % CPR) ^ kmajor_swizzle(k + KSTEP);
+			const int mc = (tid % CPR) ^ kmajor_swizzle<ROWS>(k);
+			const int mc_odd = (tid % CPR) ^ kmajor_swizzle<ROWS>(k + KSTEP);
 			kchunk = 0;
 			lane_ok = row0 + (mc << 3) < rows_total;
 			lane_ok_odd = row0 + (mc_odd << 3) < rows_total;
@@ -884,8 +891,8 @@ struct TileLoader {
 		constexpr int CPR = ROWS / 8;
 		const int tid = threadIdx.x % THREADS;
 		const int k = tid / CPR;
-		const int mc = (tid % CPR) ^ kmajor_swizzle(k);
-		const int mc_odd = (tid % CPR) ^ kmajor_swizzle(k + KSTEP);
+		const int mc = (tid % CPR) ^ kmajor_swizzle<ROWS>(k);
+		const int mc_odd = (tid % CPR) ^ kmajor_swizzle<ROWS>(k + KSTEP);
 		kchunk = 0;
 		lane_ok = row0 + (mc << 3) < rows_total;
 		lane_ok_odd = row0 + (mc_odd << 3) < rows_total;
@@ -957,21 +964,22 @@ __device__ __forceinline__ bf16x8 read_fragment(const bf16_t * tile, int row_bas
 		const int lg = lane & 15;
 		const int r0 = row_base + ((lg & 3) << 2);
 		const int k_lo = 32 * s + ((lane >> 4) << 3) + (lg >> 2), k_hi = k_lo + 4;
-		s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *) LDS_PTR(tile + k_lo * ROWS + (r0 ^ (kmajor_swizzle(k_lo) << 3))));
-		s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *) LDS_PTR(tile + k_hi * ROWS + (r0 ^ (kmajor_swizzle(k_hi) << 3))));
+		s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *) LDS_PTR(tile + k_lo * ROWS + (r0 ^ (kmajor_swizzle<ROWS>(k_lo) << 3))));
+		s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *) LDS_PTR(tile + k_hi * ROWS + (r0 ^ (kmajor_swizzle<ROWS>(k_hi) << 3))));
 		s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 		return __builtin_bit_cast(bf16x8, both);
 	}
 }
 
-/* STAGES: 2, or 4 for the launches that split K over otherwise idle compute units (few tiles, the router's GEMMs): those
- * are short streams of operand bytes with nothing to reuse, and what one k-tile in flight per compute unit fetches in a
- * memory round trip is a third of what HBM delivers; with four stages three k-tiles are in flight.  A split then has to
- * be a multiple of four k-tiles long. */
+/* STAGES LDS stages keep STAGES - 1 k-tiles in flight per work-group.  Problems of few tiles are short streams of operand
+ * bytes with nothing to reuse: a k-tile costs them the memory round trip divided by the k-tiles in flight, so they run on
+ * three or four stages of small tiles (1408 x 2048 x 256: 30 us with 128 x 128 tiles and two stages, 23 us with four, 10.5
+ * us with 64 x 64 tiles and four; eight stages leave room for one work-group per compute unit and lose what they gain).
+ * Two stages where two work-groups of a compute unit hide each other's waits (the host's table of tiles). */
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool P_KMAJOR, bool Q_KMAJOR, int MODE, int GATHER = 0, int STAGES = 2>
 __global__ void __launch_bounds__(WAVES_M * WAVES_N * 64)
 gemm_bf16_direct_kernel(GemmParams p) {
-	static_assert(STAGES == 2 || STAGES == 4, "two stages, or four");
+	static_assert(STAGES >= 2 && STAGES <= 8, "at least two stages");
 	constexpr int THREADS = WAVES_M * WAVES_N * 64;
 	constexpr int WTM = BM / WAVES_M;
 	constexpr int WTN = BN / WAVES_N;
@@ -1084,22 +1092,25 @@ gemm_bf16_direct_kernel(GemmParams p) {
 			COMPUTE_STAGE(stage1);
 		}
 	} else {
-		/* Iteration for k-tile kt (stage kt mod 4): the loads of kt, kt+1, kt+2 are out; wait until only the two younger
-		 * ones are (loads complete in order), barrier -- kt is visible, and nobody reads the stage of kt-1 any more --
-		 * start kt+3 into that stage, multiply kt.  The split is a multiple of four k-tiles (or ends with K), so what is
-		 * multiplied past its end are k-tiles past K: zeros; the loads that run ahead into the next split's k-tiles are
-		 * never multiplied. */
+		/* Iteration for k-tile kt (stage kt mod STAGES): the loads of kt .. kt + STAGES - 2 are out; wait until only those
+		 * behind kt are (loads complete in order), barrier -- kt is visible, and nobody reads the stage of kt-1 any more --
+		 * start the load of kt + STAGES - 1 into that stage, multiply kt.  Loads that run ahead past the end are never
+		 * multiplied. */
 		constexpr uint32_t STAGE_BYTES = (BM + BN) * BK * 2;
-		ISSUE_STAGE(stage0_addr, kt_begin);
-		ISSUE_STAGE(stage0_addr + STAGE_BYTES, kt_begin + 1);
-		ISSUE_STAGE(stage0_addr + 2 * STAGE_BYTES, kt_begin + 2);
-		for (int kt = kt_begin; kt < k_tiles; kt += 4) {
+		static_assert((STAGES - 2) * LOADS_PER_STAGE < 64, "vmcnt is a 6-bit counter");
+		#pragma unroll
+		for (int u = 0; u < STAGES - 1; u++) {
+			ISSUE_STAGE(stage0_addr + u * STAGE_BYTES, kt_begin + u);
+		}
+		for (int kt = kt_begin; kt < k_tiles; kt += STAGES) {
 			#pragma unroll
-			for (int u = 0; u < 4; u++) {
-				WAIT_VMCNT(2 * LOADS_PER_STAGE);
-				__syncthreads();
-				ISSUE_STAGE(stage0_addr + ((u + 3) & 3) * STAGE_BYTES, kt + u + 3);
-				COMPUTE_STAGE(stages[u]);
+			for (int u = 0; u < STAGES; u++) {
+				if (kt + u < k_tiles) {
+					WAIT_VMCNT((STAGES - 2) * LOADS_PER_STAGE);
+					__syncthreads();
+					ISSUE_STAGE(stage0_addr + ((u + STAGES - 1) % STAGES) * STAGE_BYTES, kt + u + STAGES - 1);
+					COMPUTE_STAGE(stages[u]);
+				}
 			}
 		}
 	}

@@ -498,6 +498,22 @@ def test_matmul_split_k_through_the_workspace(backend, oracle, transa, transb, M
     check_matmul(got, O.matmul(oracle, transa, transb, M, K, N, A, Bm, alpha=0.5, beta=1.0, Cin=Cin), K)
 
 
+@pytest.mark.parametrize("transa,transb", [(1, 0), (0, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("M,K,N", [(72, 200, 33), (8, 8, 32), (1000, 136, 1000), (1024, 64, 968), (2048, 264, 1000), (2000, 56, 1024), (4000, 72, 1000), (4096, 520, 2000)])
+def test_matmul_tiles_of_the_direct_kernel(backend, oracle, transa, transb, M, K, N):
+    """Sizes the dispatch gives to each of the small work-group tiles (64 x 32, 64 x 64, 64 x 128, 128 x 128 alone and in
+    pairs): whole and partial last tiles, fewer k-tiles than stages, k tails."""
+    print("case tile ta=%d tb=%d M=%d K=%d N=%d" % (transa, transb, M, K, N), flush=True)
+    if transb:
+        N = (N + 7) & ~7
+    rng = np.random.default_rng(M + K + N)
+    A = normal_bf16(rng, (M, K) if transa else (K, M))
+    Bm = normal_bf16(rng, (K, N) if transb else (N, K), 0.05)
+    Cin = normal_bf16(rng, (N, M))
+    got = run_gpu_matmul(backend, transa, transb, M, K, N, A, Bm, 0.5, 1.0, Cin)
+    check_matmul(got, O.matmul(oracle, transa, transb, M, K, N, A, Bm, alpha=0.5, beta=1.0, Cin=Cin), K)
+
+
 def test_matmul_random_shapes(backend, oracle):
     """Seeded random problems over every kernel the dispatch can pick (128-tile direct, 256-tile streaming, split-K,
     the general path for sizes that are not multiples of 8), all four layouts, with and without a C operand."""
