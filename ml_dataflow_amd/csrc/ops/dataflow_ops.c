@@ -9,37 +9,93 @@
  */
 #include "dataflow_amd_ops.h"
 
+#include <pthread.h>
+#include <stdatomic.h>
 #include <stdio.h>
 #include <string.h>
 
 #define I_S DATAFLOW_INT_SCALAR
 #define F_S DATAFLOW_FP32_SCALAR
 
-static void fill_skeleton(Op_Skeleton * skeleton, const char * base, DataflowDatatype dt0, DataflowDatatype dt1,
-						  int num_args, const DataflowDatatype * arg_dtypes) {
+/* Skeletons that have been filled once in this process.  A skeleton is a function of its base name and type tags, and its
+ * fingerprint (a SHA-256 over 388 bytes) and formatted nickname were most of what the host spent on a submission beside
+ * the launch itself (1.3 of 4.4 us): every later submission of the op copies the first one's.  Slots are only ever added,
+ * published by the count behind them, so readers need no lock; a full table leaves further ops unremembered. */
+#define MAX_KNOWN_SKELETONS 128
+typedef struct known_skeleton {
+	const char * base;                /* the string literal the op's setter passes: compared by address */
+	DataflowDatatype dt0, dt1;
+	int num_args, listed;
+	DataflowDatatype tags[MAX_OP_ARGS];
+	Op_Skeleton skeleton;
+} Known_Skeleton;
+static Known_Skeleton known[MAX_KNOWN_SKELETONS];
+static atomic_int num_known;
+static pthread_mutex_t known_lock = PTHREAD_MUTEX_INITIALIZER;
+
+static int recall_skeleton(Op_Skeleton * skeleton, const char * base, DataflowDatatype dt0, DataflowDatatype dt1,
+						   int num_args, int listed, const DataflowDatatype * tags) {
+	const int n = atomic_load_explicit(&num_known, memory_order_acquire);
+	for (int i = 0; i < n; i++) {
+		const Known_Skeleton * k = &known[i];
+		if (k->base == base && k->dt0 == dt0 && k->dt1 == dt1 && k->num_args == num_args && k->listed == listed
+			&& memcmp(k->tags, tags, (size_t) listed * sizeof(DataflowDatatype)) == 0) {
+			*skeleton = k->skeleton;
+			return 1;
+		}
+	}
+	return 0;
+}
+
+static void remember_skeleton(const Op_Skeleton * skeleton, const char * base, DataflowDatatype dt0, DataflowDatatype dt1,
+							  int num_args, int listed, const DataflowDatatype * tags) {
+	pthread_mutex_lock(&known_lock);
+	const int n = atomic_load_explicit(&num_known, memory_order_relaxed);
+	if (n < MAX_KNOWN_SKELETONS) {
+		Known_Skeleton * k = &known[n];
+		k->base = base;
+		k->dt0 = dt0;
+		k->dt1 = dt1;
+		k->num_args = num_args;
+		k->listed = listed;
+		memcpy(k->tags, tags, (size_t) listed * sizeof(DataflowDatatype));
+		k->skeleton = *skeleton;
+		atomic_store_explicit(&num_known, n + 1, memory_order_release);
+	}
+	pthread_mutex_unlock(&known_lock);
+}
+
+/* `listed` type tags are set, `num_args` is the argument count written beside them (one skeleton's list is the longer).
+ * four_types: two element types that come in front of dt0 and dt1 in the nickname (the op that has four), or NULL */
+static void fill_skeleton_listed(Op_Skeleton * skeleton, const char * base, const DataflowDatatype * four_types,
+								 DataflowDatatype dt0, DataflowDatatype dt1, int num_args, int listed, const DataflowDatatype * arg_dtypes) {
+	if (recall_skeleton(skeleton, base, dt0, dt1, num_args, listed, arg_dtypes)) {
+		return;
+	}
 	Op_Skeleton_Header * header = &(skeleton->header);
 	/* the nickname field is hashed in full, so everything after the text must be zero */
 	memset(header->op_nickname, 0, sizeof(header->op_nickname));
-	if (dt0 == DATAFLOW_NONE) {
-		snprintf(header->op_nickname, MAX_OP_NICKNAME_SIZE, "%s", base);
-	} else if (dt1 == DATAFLOW_NONE) {
-		snprintf(header->op_nickname, MAX_OP_NICKNAME_SIZE, "%s_%s", base, dataflow_datatype_as_string(dt0));
-	} else {
-		snprintf(header->op_nickname, MAX_OP_NICKNAME_SIZE, "%s_%s_%s", base, dataflow_datatype_as_string(dt0), dataflow_datatype_as_string(dt1));
+	int at = snprintf(header->op_nickname, MAX_OP_NICKNAME_SIZE, "%s", base);
+	if (four_types) {
+		at += snprintf(header->op_nickname + at, (size_t) (MAX_OP_NICKNAME_SIZE - at), "_%s_%s", dataflow_datatype_as_string(four_types[0]), dataflow_datatype_as_string(four_types[1]));
+	}
+	if (dt0 != DATAFLOW_NONE) {
+		at += snprintf(header->op_nickname + at, (size_t) (MAX_OP_NICKNAME_SIZE - at), "_%s", dataflow_datatype_as_string(dt0));
+		if (dt1 != DATAFLOW_NONE) {
+			snprintf(header->op_nickname + at, (size_t) (MAX_OP_NICKNAME_SIZE - at), "_%s", dataflow_datatype_as_string(dt1));
+		}
 	}
 	header->num_args = num_args;
 	for (int i = 0; i < MAX_OP_ARGS; i++) {
-		header->arg_dtypes[i] = (i < num_args) ? arg_dtypes[i] : DATAFLOW_NONE;
+		header->arg_dtypes[i] = (i < listed) ? arg_dtypes[i] : DATAFLOW_NONE;
 	}
 	dataflow_do_fingerprinting(header, sizeof(Op_Skeleton_Header), skeleton->identifier.fingerprint);
+	remember_skeleton(skeleton, base, dt0, dt1, num_args, listed, arg_dtypes);
 }
 
-/* for the one skeleton whose tag list is longer than its argument count: `listed` tags are set, then hashed */
-static void fill_skeleton_listed(Op_Skeleton * skeleton, const char * base, DataflowDatatype dt0, DataflowDatatype dt1,
-								 int num_args, int listed, const DataflowDatatype * arg_dtypes) {
-	fill_skeleton(skeleton, base, dt0, dt1, listed, arg_dtypes);
-	skeleton->header.num_args = num_args;
-	dataflow_do_fingerprinting(&(skeleton->header), sizeof(Op_Skeleton_Header), skeleton->identifier.fingerprint);
+static void fill_skeleton(Op_Skeleton * skeleton, const char * base, DataflowDatatype dt0, DataflowDatatype dt1,
+						  int num_args, const DataflowDatatype * arg_dtypes) {
+	fill_skeleton_listed(skeleton, base, NULL, dt0, dt1, num_args, num_args, arg_dtypes);
 }
 
 void dataflow_set_matmul_skeleton(Op_Skeleton * skeleton) {
@@ -121,7 +177,7 @@ void dataflow_set_default_rms_norm_bwd_x_skeleton(Op_Skeleton * skeleton, Datafl
 
 void dataflow_set_default_rms_norm_bwd_w_skeleton(Op_Skeleton * skeleton, DataflowDatatype fwd, DataflowDatatype bwd) {
 	const DataflowDatatype t[9] = {I_S, I_S, F_S, DATAFLOW_FP32, fwd, bwd, DATAFLOW_FP32, DATAFLOW_INT, DATAFLOW_UINT64_SCALAR};
-	fill_skeleton_listed(skeleton, "default_rms_norm_bwd_w", fwd, bwd, 8, 9, t);
+	fill_skeleton_listed(skeleton, "default_rms_norm_bwd_w", NULL, fwd, bwd, 8, 9, t);
 }
 
 void dataflow_set_default_rms_norm_bwd_w_combine_skeleton(Op_Skeleton * skeleton, DataflowDatatype bwd) {
@@ -134,9 +190,8 @@ void dataflow_set_default_rms_norm_bwd_w_combine_skeleton(Op_Skeleton * skeleton
 void dataflow_set_default_adamw_step_skeleton(Op_Skeleton * skeleton, DataflowDatatype param_dt, DataflowDatatype grad_dt,
 											  DataflowDatatype mean_dt, DataflowDatatype var_dt) {
 	const DataflowDatatype t[11] = {DATAFLOW_UINT64_SCALAR, I_S, F_S, F_S, F_S, F_S, F_S, param_dt, grad_dt, mean_dt, var_dt};
-	char base[MAX_OP_NICKNAME_SIZE];
-	snprintf(base, sizeof(base), "default_adamw_step_%s_%s", dataflow_datatype_as_string(param_dt), dataflow_datatype_as_string(grad_dt));
-	fill_skeleton(skeleton, base, mean_dt, var_dt, 11, t);
+	const DataflowDatatype front[2] = {param_dt, grad_dt};
+	fill_skeleton_listed(skeleton, "default_adamw_step", front, mean_dt, var_dt, 11, 11, t);
 }
 
 /* ---- casts (set_op_skeletons.c:92-156): the nicknames carry no dtype suffix, the argument tags do ---- */
