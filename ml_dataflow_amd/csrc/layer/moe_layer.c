@@ -8,6 +8,7 @@
  * grouped one without the backward recompute of the expert outputs.
  */
 #include "moe_layer.h"
+#include "layer_ops.h"
 
 #include <stdio.h>
 #include <stdlib.h>
@@ -193,18 +194,11 @@ static int stream_wait(Dataflow_Handle * h, int waiter, int signaller) {
 
 /* ------------------------------------------------------------------ forward */
 
-int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L, int T, void * X, void * logit_bias, void * out, int schedule) {
-	if (check_call(L, T, schedule)) {
-		return -1;
-	}
-	if (T == 0) {
-		return 0;
-	}
+/* the routing as the reference submits it, op by op */
+static int route_by_ops(Dataflow_Handle * h, int cs, Amd_Moe_Layer * L, int T, void * X, void * logit_bias) {
 	const DataflowDatatype dt = L->dt;
 	const DataflowDatatype cdt = DATAFLOW_FP32;
-	const int D = L->model_dim, E = L->num_experts, K = L->top_k, H = L->expert_dim;
-	const uint64_t el = 2;
-
+	const int D = L->model_dim, E = L->num_experts, K = L->top_k;
 	/* 1. router logits (bf16 out), dataflow_transformer.c:2710-2717 */
 	CHECK(dataflow_submit_matmul(h, cs, dt, dt, logit_bias ? dt : DATAFLOW_NONE, dt, cdt, 1, 0, E, D, T,
 								 1.0f, logit_bias ? 1.0f : 0.0f, L->w_router, X, logit_bias, L->x_routed,
@@ -226,6 +220,29 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 	/* 3. mapping, :2781-2784 */
 	CHECK(dataflow_submit_default_build_expert_mapping(h, cs, T, E, K, L->chosen_experts, L->expert_counts_cumsum,
 													   L->expert_mapping, L->token_mapping), "failed to submit build expert mapping");
+	return 0;
+}
+
+int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L, int T, void * X, void * logit_bias, void * out, int schedule) {
+	if (check_call(L, T, schedule)) {
+		return -1;
+	}
+	if (T == 0) {
+		return 0;
+	}
+	const DataflowDatatype dt = L->dt;
+	const DataflowDatatype cdt = DATAFLOW_FP32;
+	const int D = L->model_dim, E = L->num_experts, K = L->top_k, H = L->expert_dim;
+	const uint64_t el = 2;
+
+	/* router logits, selection, counts and mapping (dataflow_transformer.c:2710-2784): one op where its limits hold */
+	if (E <= LAYER_ROUTE_MAX_EXPERTS && K <= 32 && T <= (1 << 17) && L->kernel_workspace_bytes >= LAYER_ROUTE_WORKSPACE(T, E)) {
+		CHECK(layer_submit_route_tokens(h, cs, T, E, K, D, X, L->w_router, logit_bias, L->x_routed, L->token_expert_weights, L->chosen_experts,
+										L->expert_counts, L->expert_counts_cumsum, L->host_expert_counts, L->expert_mapping, L->token_mapping,
+										L->kernel_workspace_bytes, L->kernel_workspace), "failed to submit routing");
+	} else if (route_by_ops(h, cs, L, T, X, logit_bias)) {
+		return -1;
+	}
 
 	L->last_forward_tokens = T;
 	L->host_counts_synced = 0;

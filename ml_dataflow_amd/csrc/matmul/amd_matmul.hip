@@ -26,6 +26,7 @@
 #include "gemm_kernel.h"
 #include "gemm_w4_kernel.h"
 #include "gemm_typed_kernel.h"
+#include "route_kernel.h"
 
 /* ------------------------------------------------------------------ host side */
 
@@ -150,19 +151,23 @@ static int launch_direct(const GemmParams & p, int which, hipStream_t stream) {
 	}
 }
 
-/* the direct kernel with four stages, for the partial products of a split along K (amd_matmul's few-tile problems) */
-static int launch_split_deep(const GemmParams & p, int transa, int transb, long grid, hipStream_t stream) {
+/* The partial products of a split along K (few tiles): the direct kernel with four stages, on 64 x 64 tiles where one side
+ * has no more rows than that (the router's GEMMs of up to 64 experts: half of a 128 x 128 tile would be padding) */
+static int launch_split(const GemmParams & p, int transa, int transb, hipStream_t stream) {
 	const bool pk = !transa;
 	const bool qk = transb != 0;
-#define DEEP(PK, QK) do { \
-		hipLaunchKernelGGL((gemm_bf16_direct_kernel<128, 128, 2, 2, PK, QK, MODE_SINGLE, GATHER_NONE, 4>), dim3((unsigned int) grid), dim3(256), 0, stream, p); \
-		return check_launch(); \
+	const bool narrow = p.M <= 64 || p.N <= 64;
+	const long tiles = narrow ? tiles_of(p.M, 64) * tiles_of(p.N, 64) : tiles_of(p.M, 128) * tiles_of(p.N, 128);
+	const long grid = tiles * p.split_k;
+#define SPLIT(PK, QK) do { \
+		return narrow ? launch_direct_tile<64, 64, 2, 2, 4, PK, QK, MODE_SINGLE>(p, grid, stream) \
+					  : launch_direct_tile<128, 128, 2, 2, 4, PK, QK, MODE_SINGLE>(p, grid, stream); \
 	} while (0)
-	if (!pk && !qk) { DEEP(false, false); }
-	if (pk && !qk) { DEEP(true, false); }
-	if (pk && qk) { DEEP(true, true); }
-	DEEP(false, true);
-#undef DEEP
+	if (!pk && !qk) { SPLIT(false, false); }
+	if (pk && !qk) { SPLIT(true, false); }
+	if (pk && qk) { SPLIT(true, true); }
+	SPLIT(false, true);
+#undef SPLIT
 }
 
 /* streaming kernel: one persistent work-group per compute unit (LDS allows no more), a multiple of 8 so every die gets the same share */
@@ -455,6 +460,37 @@ static long extra_cu_count(void * op_extra) {
 	return op_extra ? ((MatmulExtra *) op_extra)->cu_count : 256;
 }
 
+/* Few tiles and a long K (the router's GEMMs: 64 experts on one side): split K over the idle compute units, fp32 partial
+ * sums in `workspace`, added up by the pass behind.  Without a workspace that is large enough (and 16-byte aligned) the
+ * problem runs unsplit; `must_fit`: that is an error instead.  1 and the split in `p`, 0: unsplit, -1: error. */
+static int plan_split(GemmParams & p, bool direct, float * workspace, uint64_t workspace_bytes, long cu_count, bool must_fit) {
+	const bool big = tiles_of(p.M, 256) * tiles_of(p.N, 256) >= cu_count / 2 && p.M >= 256 && p.N >= 256;     /* enough tiles as it is */
+	const long k_tiles = tiles_of(p.K, BK);
+	long splits = direct && !big ? cu_count / (tiles_of(p.M, 128) * tiles_of(p.N, 128)) : 1;
+	if (splits < 2 || k_tiles < 8 || !workspace || (((uintptr_t) workspace) & 15)) {
+		return 0;
+	}
+	long per = tiles_of(k_tiles, splits);
+	per = per < 4 ? 4 : (per + 3) & ~3L;                /* at least as many as the kernel's stages */
+	splits = tiles_of(k_tiles, per);
+	const uint64_t count = (uint64_t) p.M * (uint64_t) p.N;
+	if (splits < 2) {
+		return 0;
+	}
+	if (workspace_bytes / 4 / (uint64_t) splits < count) {
+		if (must_fit) {
+			fprintf(stderr, "Error: this %d x %d x %d matmul splits along K into %ld parts of %lu partial sums each, more than the %lu-byte scratch holds; use the matmul op with a workspace...\n",
+					p.M, p.K, p.N, splits, (unsigned long) count, (unsigned long) workspace_bytes);
+			return -1;
+		}
+		return 0;
+	}
+	p.partial = workspace;
+	p.split_k = (int) splits;
+	p.kt_per_split = (int) per;
+	return 1;
+}
+
 /* shared by amd_matmul and amd_matmul_no_alloc: checks, kernel choice, launch.  `workspace` (may be NULL) holds the fp32
  * partial sums of a split along K; `must_fit`: a split that the workspace cannot hold is an error instead of running
  * unsplit */
@@ -478,35 +514,19 @@ static int run_matmul(Dataflow_Handle * dataflow_handle, int stream_id, GemmPara
 	const bool direct = operand_direct_ok(p.A, !transa, p.M, p.K, 0) && operand_direct_ok(p.B, transb != 0, p.N, p.K, 0);
 	const long grid_big = tiles_of(p.M, 256) * tiles_of(p.N, 256);
 	const long grid_small = tiles_of(p.M, 128) * tiles_of(p.N, 128);
-	const bool big = grid_big >= cu_count / 2 && p.M >= 256 && p.N >= 256;     /* enough tiles without splitting K */
-	/* Few tiles and a long K (the router's GEMMs: 64 experts on one side): split K over the idle compute units,
-	 * fp32 partial sums in the caller's workspace, one reduction pass.  Without a workspace that is large enough
-	 * (and 16-byte aligned) the problem runs unsplit. */
-	const long k_tiles = tiles_of(p.K, BK);
-	long splits = direct && !big ? cu_count / grid_small : 1;
-	if (splits >= 2 && k_tiles >= 8 && workspace && aligned16(workspace)) {
-		long per = tiles_of(k_tiles, splits);
-		per = per < 4 ? 4 : per;
-		per = (per + 3) & ~3L;                      /* the four-stage kernel takes its k-tiles in fours */
-		splits = tiles_of(k_tiles, per);
-		const uint64_t count = (uint64_t) p.M * (uint64_t) p.N;
-		if (splits >= 2 && must_fit && workspace_bytes / 4 / (uint64_t) splits < count) {
-			fprintf(stderr, "Error: this %d x %d x %d matmul splits along K into %ld parts of %lu partial sums each, more than the %lu-byte scratch holds; use the matmul op with a workspace...\n",
-					p.M, p.K, p.N, splits, (unsigned long) count, (unsigned long) workspace_bytes);
+	const int split = plan_split(p, direct, workspace, workspace_bytes, cu_count, must_fit);
+	if (split < 0) {
+		return -1;
+	}
+	if (split) {
+		if (launch_split(p, transa, transb, stream)) {
 			return -1;
 		}
-		if (splits >= 2 && workspace_bytes / 4 / (uint64_t) splits >= count) {
-			p.partial = workspace;
-			p.split_k = (int) splits;
-			p.kt_per_split = (int) per;
-			if (launch_split_deep(p, transa, transb, (grid_small * splits + 7) & ~7L, stream)) {
-				return -1;
-			}
-			const long blocks = (long) ((count + 255) / 256);
-			hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned int) (blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream,
-							   (const float *) workspace, (int) splits, (long long) count, p.alpha, p.beta, p.C, p.D);
-			return check_launch();
-		}
+		const uint64_t count = (uint64_t) p.M * (uint64_t) p.N;
+		const long blocks = (long) ((count + 255) / 256);
+		hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned int) (blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream,
+						   (const float *) workspace, p.split_k, (long long) count, p.alpha, p.beta, p.C, p.D);
+		return check_launch();
 	}
 	return launch_gemm<MODE_SINGLE>(p, transa, transb, direct, grid_big, grid_small, cu_count, stream);
 }
@@ -748,4 +768,88 @@ extern "C" int amd_grouped_matmul(Dataflow_Handle * dataflow_handle, int stream_
 	}
 	fprintf(stderr, "Error: unknown ragged dimension %d...\n", ragged);
 	return -1;
+}
+
+/* The layer's routing in one op (../layer/layer_ops.h): router product, selection, counts, prefix sum, permutation. */
+extern "C" int amd_route_tokens(Dataflow_Handle * dataflow_handle, int stream_id, Op * op, void * op_extra) {
+	void ** a = op->op_args;
+	RouteParams r;
+	memset(&r, 0, sizeof(r));
+	r.T = *((int *) a[0]);
+	r.E = *((int *) a[1]);
+	r.K = *((int *) a[2]);
+	GemmParams p;
+	memset(&p, 0, sizeof(p));
+	p.M = r.E;
+	p.K = *((int *) a[3]);
+	p.N = r.T;
+	p.B = (const bf16_t *) *((uint64_t *) a[4]);
+	p.A = (const bf16_t *) *((uint64_t *) a[5]);
+	p.C = (const bf16_t *) *((uint64_t *) a[6]);
+	p.D = (bf16_t *) *((uint64_t *) a[7]);
+	p.alpha = 1.0f;
+	p.beta = p.C ? 1.0f : 0.0f;
+	r.bias = p.C;
+	r.x_routed = p.D;
+	r.weights = (float *) *((uint64_t *) a[8]);
+	r.chosen = (uint16_t *) *((uint64_t *) a[9]);
+	r.expert_counts = (int *) *((uint64_t *) a[10]);
+	r.expert_counts_cumsum = (int *) *((uint64_t *) a[11]);
+	r.host_expert_counts = (int *) *((uint64_t *) a[12]);
+	r.expert_mapping = (int *) *((uint64_t *) a[13]);
+	r.token_mapping = (int *) *((uint64_t *) a[14]);
+	const uint64_t workspace_bytes = *((uint64_t *) a[15]);
+	uint8_t * workspace = (uint8_t *) *((uint64_t *) a[16]);
+
+	r.counts_pitch = 16;
+	while (r.counts_pitch < r.E) {
+		r.counts_pitch *= 2;
+	}
+	const long blocks = tiles_of(r.T, ROUTE_TOKENS);
+	const uint64_t counts_bytes = ((uint64_t) blocks * (uint64_t) r.counts_pitch + 255) & ~255UL;
+	if (r.T < 1 || r.E < 1 || r.E > ROUTE_MAX_EXPERTS || r.K < 1 || r.K > r.E || r.K > SELECT_MAX_K || p.K < 1 || !p.A || !p.B || !p.D
+		|| blocks * (r.counts_pitch / 16) > 2047L * ROUTE_MAP_THREADS || !workspace || (((uintptr_t) workspace) & 15) || workspace_bytes < counts_bytes) {
+		fprintf(stderr, "Error: bad arguments of the routing op (%d tokens, %d experts, top %d, model dim %d, %lu bytes of workspace)...\n",
+				r.T, r.E, r.K, p.K, (unsigned long) workspace_bytes);
+		return -1;
+	}
+	hipStream_t stream;
+	if (resolve_stream(dataflow_handle, stream_id, &stream)) {
+		return -1;
+	}
+	if (hipSetDevice(dataflow_handle->device_id) != hipSuccess) {
+		fprintf(stderr, "Error: hipSetDevice failed in the routing op...\n");
+		return -1;
+	}
+	r.counts = workspace;
+	float * partial = (float *) (workspace + counts_bytes);
+	const long cu_count = extra_cu_count(op_extra);
+	const bool direct = operand_direct_ok(p.A, false, p.M, p.K, 0) && operand_direct_ok(p.B, false, p.N, p.K, 0);
+	if (plan_split(p, direct, partial, workspace_bytes - counts_bytes, cu_count, false)) {
+		r.partial = partial;
+		r.splits = p.split_k;
+		if (launch_split(p, 1, 0, stream)) {
+			return -1;
+		}
+	} else if (launch_gemm<MODE_SINGLE>(p, 1, 0, direct, tiles_of(p.M, 256) * tiles_of(p.N, 256), tiles_of(p.M, 128) * tiles_of(p.N, 128), cu_count, stream)) {
+		return -1;
+	}
+	int lanes = 1;                                      /* one slot per lane */
+	while (lanes < r.K) {
+		lanes *= 2;
+	}
+	/* Few tokens: selection and permutation in one work-group, one launch less in a chain of which nothing else is left.
+	 * Its one compute unit adds up the partial sums at 20-30 GB/s a wave: bounded, so that it stays below a launch. */
+	if (r.T <= ROUTE_SMALL_TOKENS && r.T * lanes <= ROUTE_SMALL_THREADS && (long) r.T * r.E * (r.splits > 1 ? r.splits : 1) <= ROUTE_SMALL_PARTIALS) {
+		int threads = (r.T * lanes + WAVE - 1) / WAVE * WAVE;
+		threads = threads < 256 ? 256 : threads;
+		hipLaunchKernelGGL(route_small_kernel, dim3(1), dim3((unsigned int) threads), 0, stream, r, lanes);
+		return check_launch();
+	}
+	hipLaunchKernelGGL(route_select_kernel, dim3((unsigned int) blocks), dim3((unsigned int) (ROUTE_TOKENS * lanes < 256 ? 256 : ROUTE_TOKENS * lanes)), 0, stream, r, lanes);
+	if (check_launch()) {
+		return -1;
+	}
+	hipLaunchKernelGGL(route_map_kernel, dim3((unsigned int) tiles_of(blocks, ROUTE_MAP_WAVES)), dim3(ROUTE_MAP_THREADS), 0, stream, r, (int) blocks);
+	return check_launch();
 }

@@ -8,6 +8,7 @@
  * libdataflowops/src/submit_ops/{moe_ops.c, matmul_op.c, mlp_misc_ops.c}.
  */
 #include "dataflow_amd_ops.h"
+#include "skeletons.h"
 
 #include <pthread.h>
 #include <stdatomic.h>
@@ -93,10 +94,11 @@ static void fill_skeleton_listed(Op_Skeleton * skeleton, const char * base, cons
 	remember_skeleton(skeleton, base, dt0, dt1, num_args, listed, arg_dtypes);
 }
 
-static void fill_skeleton(Op_Skeleton * skeleton, const char * base, DataflowDatatype dt0, DataflowDatatype dt1,
-						  int num_args, const DataflowDatatype * arg_dtypes) {
+void dataflow_fill_skeleton(Op_Skeleton * skeleton, const char * base, DataflowDatatype dt0, DataflowDatatype dt1,
+							int num_args, const DataflowDatatype * arg_dtypes) {
 	fill_skeleton_listed(skeleton, base, NULL, dt0, dt1, num_args, num_args, arg_dtypes);
 }
+#define fill_skeleton dataflow_fill_skeleton
 
 void dataflow_set_matmul_skeleton(Op_Skeleton * skeleton) {
 	/* num_procs, 5 dtype tags, 2 transpose flags, M K N, alpha beta, A B C D, workspace bytes, workspace */

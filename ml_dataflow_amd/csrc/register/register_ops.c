@@ -12,6 +12,7 @@
 #define _GNU_SOURCE
 #include "dataflow_amd.h"
 #include "dataflow_amd_ops.h"
+#include "../layer/layer_ops.h"
 
 #include <dlfcn.h>
 #include <limits.h>
@@ -148,6 +149,24 @@ static int register_external(Dataflow_Handle * handle, const char * dir) {
 	return added;
 }
 
+/* the layer driver's own ops: in the table like the others, but no part of the operator interface (and of the count that
+ * registration reports) */
+static int register_layer_ops(Dataflow_Handle * handle, const char * dir) {
+	enum { N = 1 };
+	Op_Skeleton skeletons[N];
+	layer_set_route_tokens_skeleton(&skeletons[0]);
+	char * symbols[N] = {"amd_route_tokens"};
+	char * init_symbols[N] = {"amd_matmul_init"};
+	char lib[PATH_MAX];
+	snprintf(lib, sizeof(lib), "%s/%s", dir, MATMUL_LIB);
+	int added = (handle->register_external_code)(handle, lib, N, skeletons, symbols, init_symbols);
+	if (added != N) {
+		fprintf(stderr, "Error: failed to register the layer's ops, expected %d functions, got %d...\n", N, added);
+		return -1;
+	}
+	return added;
+}
+
 int dataflow_register_default_ops(Dataflow_Handle * dataflow_handle) {
 	if (!dataflow_handle || !dataflow_handle->register_native_code || !dataflow_handle->register_external_code) {
 		fprintf(stderr, "Error: cannot register ops on an uninitialised handle...\n");
@@ -162,7 +181,7 @@ int dataflow_register_default_ops(Dataflow_Handle * dataflow_handle) {
 		return -1;
 	}
 	int native = register_native(dataflow_handle, dir);
-	if (native < 0) {
+	if (native < 0 || register_layer_ops(dataflow_handle, dir) < 0) {
 		return -1;
 	}
 	return external + native;
