@@ -319,9 +319,10 @@ int default_adamw_step_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handl
 		fprintf(stderr, "Error: adamw step needs a step number of at least 1 (bias correction divides by 1 - beta^step), got %d...\n", step_num);
 		return -1;
 	}
-	uint64_t groups = (num_els + 2047) / 2048;               /* 8 elements per lane */
-	if (groups > 8192) {
-		groups = 8192;
+	uint64_t groups = (num_els + 2047) / 2048;               /* 8 elements per lane: every vector has a lane of its own */
+	if (groups > 0x7fffffffUL) {
+		fprintf(stderr, "Error: adamw step over %lu elements needs too many work-groups...\n", (unsigned long) num_els);
+		return -1;
 	}
 	set_1d(cfg, (unsigned int) groups, 256, 0);
 	return 0;

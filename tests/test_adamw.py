@@ -88,3 +88,9 @@ def test_gpu_matches_oracle(backend, oracle, n, step, offset):
         assert be.read(bufs[0].ptr, (1,), np.uint16)[0] == param[0]             # nothing written in front of the arrays
     # step numbers below 1 are rejected
     assert be.lib.dataflow_submit_default_adamw_step(be.hp, 1, BF, BF, BF, BF, n, 0, 1e-3, 0.9, 0.999, 0.0, 1e-8, *ptrs) == -1
+
+
+@pytest.mark.gpu
+def test_gpu_matches_oracle_beyond_the_caches(backend, oracle):
+    """past the size from which the arrays are accessed non-temporally, with a tail that is no whole vector"""
+    test_gpu_matches_oracle(backend, oracle, (1 << 25) + 13, 3, 0)
