@@ -237,14 +237,94 @@ static bool w4_ok(const GemmParams & p) {
 		   (p.M % 8 == 0) && ((((uintptr_t) p.D) & 15) == 0);
 }
 
+/* one tiling of a ragged-N launch without C; grid: an upper bound on the tiles that is the same for all of its tilings */
+template <bool PK, int GATHER>
+static int launch_ragged_n_tiling(int tiling, const GemmParams & p, long grid, long cu_count, hipStream_t stream) {
+	switch (tiling) {
+		case RAGGED_N_384: return launch_w4d<PK, MODE_RAGGED_N, GATHER>(p, grid, cu_count, stream);
+		case RAGGED_N_288: return launch_stream<256, 288, 4, 2, PK, false, MODE_RAGGED_N, GATHER>(p, grid, cu_count, stream);
+		case RAGGED_N_224: return launch_stream<256, 224, 4, 2, PK, false, MODE_RAGGED_N, GATHER>(p, grid, cu_count, stream);
+		default: return launch_stream<256, 192, 4, 2, PK, false, MODE_RAGGED_N, GATHER>(p, grid, cu_count, stream);
+	}
+}
+
+static int launch_ragged_n(int candidates, const GemmParams & p, bool pk, long grid, long cu_count, hipStream_t stream) {
+	GemmParams q = p;
+	q.candidates = (candidates & (candidates - 1)) ? candidates : 0;
+	for (int tiling = RAGGED_N_TILINGS - 1; tiling >= 0; tiling--) {
+		if (!((candidates >> tiling) & 1)) {
+			continue;
+		}
+		int r;
+		if (p.gather) {
+			r = pk ? launch_ragged_n_tiling<true, GATHER_Q_ROWS>(tiling, q, grid, cu_count, stream)
+				   : launch_ragged_n_tiling<false, GATHER_Q_ROWS>(tiling, q, grid, cu_count, stream);
+		} else {
+			r = pk ? launch_ragged_n_tiling<true, GATHER_NONE>(tiling, q, grid, cu_count, stream)
+				   : launch_ragged_n_tiling<false, GATHER_NONE>(tiling, q, grid, cu_count, stream);
+		}
+		if (r) {
+			return r;
+		}
+	}
+	return 0;
+}
+
+/* The tilings a ragged-N launch without C is dispatched on; the device takes the cheapest of them for the real group sizes.
+ * A launch that loses costs a few microseconds, so only those are candidates that could win, seen from the mean group:
+ *   288: always, the safe one for uneven groups.
+ *   384: where it wins with all groups the same size; where it does not, uneven groups only make it lose by more (short
+ *        groups fill a 384-row tile worse).
+ *   224 or 192: with groups one standard deviation of an even router (the root of the mean) above the mean, so that
+ *        the usual spread does not spill into a further tile; where 384 does not win there too, and where it is ahead of
+ *        288 by twice what a losing launch costs (FINER_TILE_MARGIN: 6.6 us at 3.3 ns per round, k-tile and fetched row).  No
+ *        tiling is faster than the weights arrive, 4.4 TB/s where a group is one tile (STREAMED_WEIGHTS): 32 groups of
+ *        170 rows, 2048 x 1408, take 57-60 us on either tile, 1408 x 2048, whose tiles leave a quarter of the compute
+ *        units idle, 45 instead of 52. */
+#define FINER_TILE_MARGIN 200000
+#define STREAMED_WEIGHTS(bytes) ((bytes) / 145)
+static long larger(long a, long b) { return a > b ? a : b; }
+static int ragged_n_candidates(const GemmParams & p, long cu_count, bool four_ok) {
+	const long tiles_m = tiles_of(p.M, 256), k_tiles = tiles_of(p.K, BK);
+	long groups = cu_count & ~7L;
+	groups = groups < 8 ? 8 : groups;
+	const long rows = p.num_groups > 0 && p.N / p.num_groups > 0 ? p.N / p.num_groups : 1;
+	long above = rows;                                       /* rows + sqrt(rows) */
+	for (long r = 1; r * r <= rows; r++) {
+		above = rows + r;
+	}
+#define EVEN_ROUNDS(group_rows, tile_rows) tiles_of(tiles_m * p.num_groups * tiles_of((group_rows), (tile_rows)), groups)
+	const long narrow = EVEN_ROUNDS(rows, 288);
+	const long wide = EVEN_ROUNDS(rows, 384);
+	int candidates = 1 << RAGGED_N_288;
+	const bool wide_wins = four_ok && WIDE_TILE_COST(wide, k_tiles) < NARROW_TILE_COST(narrow, k_tiles);
+	if (wide_wins) {
+		candidates |= 1 << RAGGED_N_384;
+	}
+	int finer = RAGGED_N_224;
+	long cost = ragged_n_cost(finer, EVEN_ROUNDS(above, 224), k_tiles);
+	const long cost_192 = ragged_n_cost(RAGGED_N_192, EVEN_ROUNDS(above, 192), k_tiles);
+	if (cost_192 < cost) {
+		finer = RAGGED_N_192;
+		cost = cost_192;
+	}
+	const bool wide_wins_above = wide_wins && WIDE_TILE_COST(EVEN_ROUNDS(above, 384), k_tiles) < cost;
+	const long streamed = STREAMED_WEIGHTS((long) p.num_groups * p.M * p.K * 2);
+	if (!wide_wins_above && larger(cost, streamed) + FINER_TILE_MARGIN < larger(NARROW_TILE_COST(narrow, k_tiles), streamed)) {
+		candidates |= 1 << finer;
+	}
+#undef EVEN_ROUNDS
+	return candidates;
+}
+
 static long round_up8(long v) { return (v + 7) & ~7L; }
 
 #define BIG_TILE 256, 256, 4, 2          /* 8 waves, wave tile 64 x 128 */
-#define WIDE_TILE 256, 288, 4, 2         /* 8 waves, wave tile 64 x 144: the token side of the ragged-N launches, see launch_gemm */
 #define SMALL_TILE 128, 128, 2, 2        /* 4 waves, wave tile 64 x 64 */
 
 /* `direct`: the operands suit the direct-to-LDS kernels.  grid_big / grid_small: work-group counts of the persistent kernel
- * and of the register-staged one; grid_wide: tiles of 288 token rows (ragged N) */
+ * and of the register-staged one; grid_wide: tiles of 192 token rows (ragged N), which bounds
+ * the count of the larger ones too */
 template <int MODE>
 static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct, long grid_big, long grid_small, long cu_count, hipStream_t stream,
 					   long grid_wide = 0) {
@@ -260,47 +340,9 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 	const bool big = tile == TILE_BIG;
 	const bool four_ok = direct && big && !qk && w4_ok(p);
 	const bool wide_only = kernel_choice == AMD_MATMUL_KERNEL_FOUR_WAVES_384;
-	bool either = kernel_choice == AMD_MATMUL_KERNEL_AUTO;
-	if (MODE == MODE_RAGGED_N && either && p.num_groups > 0) {
-		/* The second launch costs a few microseconds even where it returns at once.  With all groups the same size the
-		 * rule of ragged_n_prefers_384 can be evaluated here; where the narrow tiling wins then, uneven groups only make
-		 * it win by more (short groups fill a 384-row tile worse), and the eight-wave kernel is launched alone. */
-		const long rows = (long) p.N / p.num_groups;
-		const long tiles_m = tiles_of(p.M, 256);
-		long groups = cu_count & ~7L;
-		groups = groups < 8 ? 8 : groups;
-		const long narrow = tiles_of(tiles_m * p.num_groups * tiles_of(rows > 0 ? rows : 1, 288), groups);
-		const long wide = tiles_of(tiles_m * p.num_groups * tiles_of(rows > 0 ? rows : 1, 384), groups);
-		const long k_tiles = tiles_of(p.K, BK);
-		if (!(WIDE_TILE_COST(wide, k_tiles) < NARROW_TILE_COST(narrow, k_tiles))) {
-			either = false;
-		}
-	}
-	if (MODE == MODE_RAGGED_N && four_ok && grid_wide > 0 && (wide_only || either)) {
-		/* grid_wide counts tiles of 288 rows: an upper bound for tiles of 384.  With the choice left open both kernels
-		 * are launched and the work-groups decide from the group sizes which of them runs (GemmParams::arbitrate). */
-		GemmParams q = p;
-		if (either) {
-			q.arbitrate = ARBITRATE_NARROW;
-			int r;
-			if (p.gather) {
-				r = pk ? launch_stream<WIDE_TILE, true, false, MODE_RAGGED_N, GATHER_Q_ROWS>(q, grid_wide, cu_count, stream)
-					   : launch_stream<WIDE_TILE, false, false, MODE_RAGGED_N, GATHER_Q_ROWS>(q, grid_wide, cu_count, stream);
-			} else {
-				r = pk ? launch_stream<WIDE_TILE, true, false, MODE_RAGGED_N>(q, grid_wide, cu_count, stream)
-					   : launch_stream<WIDE_TILE, false, false, MODE_RAGGED_N>(q, grid_wide, cu_count, stream);
-			}
-			if (r) {
-				return r;
-			}
-			q.arbitrate = ARBITRATE_WIDE;
-		}
-		if (p.gather) {
-			if (pk) { return launch_w4d<true, MODE_RAGGED_N, GATHER_Q_ROWS>(q, grid_wide, cu_count, stream); }
-			return launch_w4d<false, MODE_RAGGED_N, GATHER_Q_ROWS>(q, grid_wide, cu_count, stream);
-		}
-		if (pk) { return launch_w4d<true, MODE_RAGGED_N>(q, grid_wide, cu_count, stream); }
-		return launch_w4d<false, MODE_RAGGED_N>(q, grid_wide, cu_count, stream);
+	const bool either = kernel_choice == AMD_MATMUL_KERNEL_AUTO;
+	if (MODE == MODE_RAGGED_N && four_ok && grid_wide > 0 && wide_only) {
+		return launch_ragged_n(1 << RAGGED_N_384, p, pk, grid_wide, cu_count, stream);
 	}
 	if (MODE == MODE_SINGLE && four_ok && p.split_k <= 1 && (wide_only || either)) {
 		/* a single problem's tiles are known here: the same rule as for the ragged launches, against the 256 x 256 tiles
@@ -330,16 +372,11 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 		return launch_w4<false, MODE_SINGLE>(p, tiles, cu_count, stream);
 	}
 	if (MODE == MODE_RAGGED_N && direct && big && grid_wide > 0 && !qk && !(p.C && p.beta != 0.0f)) {
-		/* Token rows in tiles of 288: a launch takes as long as its tiles are many (a k-tile step is paced by the
+		/* Token rows in tiles of up to 384: a launch takes as long as its tiles are many (a k-tile step is paced by the
 		 * latency of the operand stream, not by the multiplies), and a group of slightly more than a multiple of 256
 		 * rows -- every second expert when the mean is such a multiple -- then needs no extra, nearly empty tile.
 		 * Every element is accumulated over k in the same order as in the 256-row tiles: results are bit-identical. */
-		if (p.gather) {
-			if (pk) { return launch_stream<WIDE_TILE, true, false, MODE_RAGGED_N, GATHER_Q_ROWS>(p, grid_wide, cu_count, stream); }
-			return launch_stream<WIDE_TILE, false, false, MODE_RAGGED_N, GATHER_Q_ROWS>(p, grid_wide, cu_count, stream);
-		}
-		if (pk) { return launch_stream<WIDE_TILE, true, false, MODE_RAGGED_N>(p, grid_wide, cu_count, stream); }
-		return launch_stream<WIDE_TILE, false, false, MODE_RAGGED_N>(p, grid_wide, cu_count, stream);
+		return launch_ragged_n(either ? ragged_n_candidates(p, cu_count, four_ok) : 1 << RAGGED_N_288, p, pk, grid_wide, cu_count, stream);
 	}
 #define PICK(PK, QK) do { \
 		if (direct) { \
@@ -743,7 +780,7 @@ extern "C" int amd_grouped_matmul(Dataflow_Handle * dataflow_handle, int stream_
 		/* upper bound of n-tiles: every group may end in one partial tile */
 		const long grid_big = tiles_of(p.M, 256) * ((long) p.N / 256 + p.num_groups);
 		const long grid_small = tiles_of(p.M, 128) * ((long) p.N / 128 + p.num_groups);
-		const long grid_wide = tiles_of(p.M, 256) * ((long) p.N / 288 + p.num_groups);
+		const long grid_wide = tiles_of(p.M, 256) * ((long) p.N / 192 + p.num_groups);
 		return launch_gemm<MODE_RAGGED_N>(p, transa, transb, direct, grid_big, grid_small, extra_cu_count(op_extra), stream, grid_wide);
 	}
 	if (ragged == AMD_GROUPED_RAGGED_K) {

@@ -3,8 +3,8 @@
  *
  * Three kernels share the tile resolver:
  *
- *   gemm_bf16_stream_kernel   the fast path for large problems (256 x 256 tiles, or 256 x 288 for the token rows of a
- *       ragged-N launch without a C operand): one persistent work-group per
+ *   gemm_bf16_stream_kernel   the fast path for large problems (256 x 256 tiles, or 256 x 288, 224 or 192 for the token
+ *       rows of a ragged-N launch without a C operand): one persistent work-group per
  *       compute unit walks over many output tiles with the operand stream of the direct kernel below, the MFMA
  *       operands one k-step ahead in registers, and a line-coalesced epilogue through its own LDS scratch.
  *
@@ -67,13 +67,11 @@ struct GemmParams {
 	float * partial;
 	int split_k;                   /* 0 or 1: off */
 	int kt_per_split;              /* even */
-	/* Ragged-N launches without C that both the eight-wave kernel (token rows in tiles of 288) and the four-wave
-	 * kernel with the 256 x 384 tile can take are launched on both; each work-group counts the tiles of the two tilings
-	 * from the device prefix sum (ragged_n_prefers_384) and the kernel that loses returns at once.
-	 * 0: run; ARBITRATE_NARROW: run unless the 384 tiling wins; ARBITRATE_WIDE: run only if it wins */
-	int arbitrate;
+	/* Ragged-N launches without C that several tilings can take are launched on each candidate; every work-group counts
+	 * the tiles of the tilings from the device prefix sum (ragged_n_choice) and the kernels that lose return at once.
+	 * One bit per tiling, RAGGED_N_288 always among them; 0: run */
+	int candidates;
 };
-enum { ARBITRATE_NONE = 0, ARBITRATE_NARROW = 1, ARBITRATE_WIDE = 2 };
 
 struct Tile {
 	const bf16_t * P;              /* M-side operand of this problem */
@@ -155,21 +153,60 @@ __device__ __forceinline__ long count_tiles(const GemmParams & p) {
 	return (long) __builtin_amdgcn_readfirstlane((int) total_n_tiles) * tiles_m;
 }
 
-/* Which tiling of the token rows is cheaper for this launch.  A launch takes (rounds of tiles over the work-groups) x
+/* Which tiling of the token rows is cheapest for this launch.  A launch takes (rounds of tiles over the work-groups) x
  * (time of a tile), and a k-tile step is paced by the bytes it fetches: 256 + 288 rows against 256 + 384 rows of 128
  * bytes, the larger tile at 3 % fewer bytes per clock plus what 1.6 k-tiles take per tile (its tiles change over
  * with fewer loads in flight; measured over group sizes of 256-2048 rows, K of 1024-4096 and the layer's launches: 3-7 %
  * at 64 k-tiles, 7-15 % at 16).  The 384 tiling wins where the groups are long enough to fill its tiles and the rounds
- * come out even; with short or very uneven groups the narrower tile wastes less.  Every work-group of both launches
- * computes the same answer.  Both sides are scaled by the k-tiles of a tile. */
+ * come out even; with short or very uneven groups the narrower tiles waste less.  Tiles of 224 and 192 rows serve the
+ * sizes between: 32 groups of 430 rows, 1408 x 2048, take 85 us in two rounds of 224 and 97 in two of 288; 170 rows
+ * 42 us on 192 (53 on 288), 24 groups of 512 rows, 1536 x 3008, 134 (158).  They are charged 7 % per byte: a round of
+ * them costs 0-8 % more per k-tile and fetched row than one of 288 (2.6-3.7 ns for K of 1408-4096), most where the
+ * weights of many m-tiles come from HBM (64 groups of about 375 rows, 2048 x 4096: 407 us on 384, 434 on 224).
+ * A launch is dispatched on every candidate tiling (bits of GemmParams::candidates) and every work-group of them
+ * computes the same answer.  All sides are scaled by the k-tiles of a tile. */
 #define WIDE_TILE_COST(rounds, k_tiles) ((rounds) * (256 + 384) * (103 * (k_tiles) + 160))
 #define NARROW_TILE_COST(rounds, k_tiles) ((rounds) * (256 + 288) * 100 * (k_tiles))
-__device__ __forceinline__ bool ragged_n_prefers_384(const GemmParams & p) {
+#define FINER_TILE_COST(rounds, rows, k_tiles) ((rounds) * (256 + (rows)) * 107 * (k_tiles))
+enum { RAGGED_N_288, RAGGED_N_384, RAGGED_N_224, RAGGED_N_192, RAGGED_N_TILINGS };
+
+__host__ __device__ __forceinline__ int ragged_n_rows(int tiling) {
+	return tiling == RAGGED_N_288 ? 288 : tiling == RAGGED_N_384 ? 384 : tiling == RAGGED_N_224 ? 224 : 192;
+}
+__host__ __device__ __forceinline__ long ragged_n_cost(int tiling, long rounds, long k_tiles) {
+	return tiling == RAGGED_N_384 ? WIDE_TILE_COST(rounds, k_tiles) : tiling == RAGGED_N_288 ? NARROW_TILE_COST(rounds, k_tiles)
+		 : FINER_TILE_COST(rounds, ragged_n_rows(tiling), k_tiles);
+}
+
+/* the cheapest of the candidates for the group sizes at hand */
+__device__ __forceinline__ int ragged_n_choice(const GemmParams & p) {
+	const int lane = threadIdx.x & 63;
+	int tiles[RAGGED_N_TILINGS] = {0, 0, 0, 0};
+	for (int g = lane; g < p.num_groups; g += 64) {
+		const int rows = p.cumsum[g] - (g ? p.cumsum[g - 1] : 0);
+		#pragma unroll
+		for (int i = 0; i < RAGGED_N_TILINGS; i++) {
+			tiles[i] += (rows + ragged_n_rows(i) - 1) / ragged_n_rows(i);
+		}
+	}
 	const long groups = gridDim.x;
-	const long narrow = (count_tiles<256, 288, MODE_RAGGED_N>(p) + groups - 1) / groups;
-	const long wide = (count_tiles<256, 384, MODE_RAGGED_N>(p) + groups - 1) / groups;
+	const long tiles_m = (p.M + 255) / 256;
 	const long k_tiles = (p.K + BK - 1) / BK;
-	return WIDE_TILE_COST(wide, k_tiles) < NARROW_TILE_COST(narrow, k_tiles);
+	int best = RAGGED_N_288;
+	long least = 0;
+	#pragma unroll
+	for (int i = 0; i < RAGGED_N_TILINGS; i++) {
+		#pragma unroll
+		for (int off = 32; off > 0; off >>= 1) {
+			tiles[i] += __shfl_xor(tiles[i], off, 64);
+		}
+		const long cost = ragged_n_cost(i, (tiles[i] * tiles_m + groups - 1) / groups, k_tiles);
+		if (i == RAGGED_N_288 || (((p.candidates >> i) & 1) && cost < least)) {
+			best = i;
+			least = cost;
+		}
+	}
+	return __builtin_amdgcn_readfirstlane(best);
 }
 
 /* Order of the tiles of one problem (tiles_m x tiles_n of them, `lid` counts them): the work-groups of a die run 32
@@ -1179,8 +1216,10 @@ gemm_bf16_stream_kernel(GemmParams p) {
 	const int wm = (wave % WAVES_M) * WTM;
 	const int wn = (wave / WAVES_M) * WTN;
 
-	if (MODE == MODE_RAGGED_N && p.arbitrate == ARBITRATE_NARROW && ragged_n_prefers_384(p)) {
-		return;                                             /* the 256 x 384 launch behind this one does the work */
+	static_assert(MODE != MODE_RAGGED_N || BN == 256 || BN == 288 || BN == 224 || BN == 192, "a tiling of ragged_n_choice, or the one for launches with C");
+	constexpr int TILING = BN == 288 ? RAGGED_N_288 : BN == 224 ? RAGGED_N_224 : RAGGED_N_192;
+	if (MODE == MODE_RAGGED_N && p.candidates && ragged_n_choice(p) != TILING) {
+		return;                                             /* another tiling's launch does the work */
 	}
 	const long total = count_tiles<BM, BN, MODE>(p);
 	const long chunk = (total + 7) >> 3;                    /* tiles per die */

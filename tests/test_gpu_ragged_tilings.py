@@ -1,0 +1,61 @@
+"""The tilings of a ragged-N launch without C (token rows in tiles of 288, 384, 224 or 192, chosen from the group sizes)
+against the one of 288 rows: bit for bit.  Every element is accumulated over k in the same order whatever the tile."""
+import ctypes as C
+import os
+
+import numpy as np
+import pytest
+
+from ml_dataflow_amd import binding as B
+from util import normal_bf16
+
+pytestmark = pytest.mark.gpu
+
+BF, CS = B.DATAFLOW_BF16, 1
+AUTO, EIGHT = 0, 8
+
+# mean rows that the short tilings are candidates at (170: 192 rows, 430: 224, 650 x 3 m-tiles: three rounds of either),
+# with groups on both sides of one, two and three tiles; the last two are so uneven that another candidate wins
+COUNTS = {
+    "192": [170, 191, 192, 160, 165, 150, 168, 180, 155, 172, 166, 190, 1, 0, 192, 187] * 2,
+    "224": [430, 447, 448, 425, 410, 420, 435, 400, 445, 415, 428, 223, 224, 432, 440, 444] * 2,
+    "three": [650, 575, 576, 577, 671, 672, 640, 660, 655, 630, 645, 670, 668, 600, 620, 665] * 2,
+    "one large": [2000] + [110] * 30 + [1],
+    "spilling": [449, 450, 193, 385, 580, 673, 455, 460] * 4,
+}
+
+
+@pytest.mark.parametrize("gathered", [False, True])
+@pytest.mark.parametrize("transa", [1, 0])
+@pytest.mark.parametrize("name", sorted(COUNTS))
+@pytest.mark.parametrize("M,K", [(1408, 1536), (1000, 1544)])      # whole k-tiles; a k tail, a partial m-tile, no 384 rows
+def test_tilings_bit_identical(backend, M, K, name, transa, gathered):
+    be = backend
+    lib = C.CDLL(os.path.join(os.path.dirname(B.__file__), "lib", "libamd_matmul.so"))
+    lib.amd_matmul_select_kernel.argtypes = [C.c_int]
+    counts = np.array(COUNTS[name], dtype=np.int32)
+    G, total, src_rows = len(counts), int(counts.sum()), 777
+    print("case tilings %s M=%d K=%d ta=%d gathered=%s rows=%d" % (name, M, K, transa, gathered, total), flush=True)
+    rng = np.random.default_rng(M + K + total + transa)
+    W = normal_bf16(rng, (G * M * K,), 0.05)
+    X = normal_bf16(rng, (src_rows if gathered else total, K))
+    d_W, d_X, d_cum = be.upload(W), be.upload(X), be.upload(np.cumsum(counts).astype(np.int32))
+    d_map = be.upload(rng.integers(0, src_rows, size=total).astype(np.int32))
+    guard = 64                                                         # rows behind the last group keep their value
+    got = {}
+    for kernel in (EIGHT, AUTO):
+        d_D = be.upload(np.full((total + guard, M), 0x4242, dtype=np.uint16))
+        assert lib.amd_matmul_select_kernel(kernel) == 0
+        head = (be.hp, CS, BF, BF, B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, transa, 0, B.AMD_GROUPED_RAGGED_N, M, K, total, G, d_cum.ptr, 1.0, 0.0,
+                d_W.ptr, M * K * 2, d_X.ptr, None, d_D.ptr, 0)
+        ret = be.lib.dataflow_submit_amd_grouped_matmul_gathered(*head, d_map.ptr, src_rows) if gathered else be.lib.dataflow_submit_amd_grouped_matmul(*head)
+        assert lib.amd_matmul_select_kernel(AUTO) == 0
+        assert ret == 0
+        be.sync(CS)
+        got[kernel] = be.read(d_D.ptr, (total + guard, M), np.uint16)
+        d_D.free()
+    assert (got[AUTO][total:] == 0x4242).all() and (got[EIGHT][total:] == 0x4242).all()
+    bad = got[AUTO] != got[EIGHT]
+    assert not bad.any(), "%d of %d elements differ, first at %s" % (int(bad.sum()), bad.size, np.argwhere(bad)[:4].tolist())
+    for d in (d_W, d_X, d_cum, d_map):
+        d.free()

@@ -78,7 +78,7 @@ def test_ablation_switches_drop_only_what_they_name(tmp_path):
 
 def test_bench_restates_the_tiling_rule_of_the_kernels():
     """bench.py names the kernel function behind each launch class (for the roofline object's dominant kernel) and its sweep
-    workload prints what the rule picks: both restate ragged_n_prefers_384 of gemm_kernel.h and must carry its constants."""
+    workload prints what the rule picks: both restate ragged_n_choice of gemm_kernel.h and must carry its constants."""
     header = open(os.path.join(ROOT, "ml_dataflow_amd", "csrc", "matmul", "gemm_kernel.h")).read()
     wide = re.search(r"#define WIDE_TILE_COST\(rounds, k_tiles\) \(\(rounds\) \* \(256 \+ 384\) \* \((\d+) \* \(k_tiles\) \+ (\d+)\)\)", header)
     narrow = re.search(r"#define NARROW_TILE_COST\(rounds, k_tiles\) \(\(rounds\) \* \(256 \+ 288\) \* (\d+) \* \(k_tiles\)\)", header)
