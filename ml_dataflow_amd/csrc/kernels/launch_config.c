@@ -320,9 +320,8 @@ int default_adamw_step_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handl
 		return -1;
 	}
 	uint64_t groups = (num_els + 2047) / 2048;               /* 8 elements per lane: every vector has a lane of its own */
-	if (groups > 0x7fffffffUL) {
-		fprintf(stderr, "Error: adamw step over %lu elements needs too many work-groups...\n", (unsigned long) num_els);
-		return -1;
+	if (groups > 0xffffffffUL / 256) {                       /* a launch has less than 2^32 lanes; the kernel strides over the rest */
+		groups = 0xffffffffUL / 256;
 	}
 	set_1d(cfg, (unsigned int) groups, 256, 0);
 	return 0;

@@ -45,11 +45,12 @@ __device__ __forceinline__ void adamw_vector(uint64_t i, u32x4 * param, const u3
 	}
 }
 
-/* Launch: grid = ceil(num_els / 2048), block = 256: one vector per lane (the loop only takes the tail of an unaligned
- * call).  A grid bounded at 8192 work-groups that stride over the arrays keeps 32 places of each array open at 32 KiB
- * distances per compute unit and streamed at 4.0-4.5 TB/s; in order of the work-groups it is 5.6-5.9 (277 M elements:
- * 979 -> 695 us, 657 with non-temporal accesses; 805 M: 2490 -> 2068, 2059).  Arrays that the 256 MiB memory-side cache
- * could hold keep their plain accesses (8 M elements: 19.9 us against 20.4). */
+/* Launch: grid = ceil(num_els / 2048), block = 256: one vector per lane (the loops only take the tail, an unaligned
+ * call, or what lies beyond the 2^32 lanes of the largest launch).  A grid bounded at 8192 work-groups that stride over
+ * the arrays keeps 32 places of each array open at 32 KiB distances per compute unit and streamed at 4.0-4.5 TB/s; in
+ * order of the work-groups it is 5.6-5.9 (277 M elements: 979 -> 695 us, 657 with non-temporal accesses; 805 M: 2490 ->
+ * 2068, 2059).  Arrays that the 256 MiB memory-side cache could hold keep their plain accesses (8 M elements: 19.9 us
+ * against 20.4). */
 #define ADAMW_STREAM_ELS (1ull << 25)
 extern "C" __global__ void __launch_bounds__(256)
 default_adamw_step_bf16_bf16_bf16_bf16_kernel(uint64_t num_els, int step_num, float lr, float beta1, float beta2, float weight_decay,
@@ -62,11 +63,11 @@ default_adamw_step_bf16_bf16_bf16_bf16_kernel(uint64_t num_els, int step_num, fl
 	const uint64_t nvec = aligned ? (num_els >> 3) : 0;
 	u32x4 * const p4 = (u32x4 *) param, * const m4 = (u32x4 *) mean, * const v4 = (u32x4 *) var;
 	const u32x4 * const g4 = (const u32x4 *) grad;
-	if (tid < nvec) {
+	for (uint64_t i = tid; i < nvec; i += nthreads) {
 		if (num_els > ADAMW_STREAM_ELS) {
-			adamw_vector<true>(tid, p4, g4, m4, v4, lr, beta1, beta2, weight_decay, epsilon, corr1, corr2);
+			adamw_vector<true>(i, p4, g4, m4, v4, lr, beta1, beta2, weight_decay, epsilon, corr1, corr2);
 		} else {
-			adamw_vector<false>(tid, p4, g4, m4, v4, lr, beta1, beta2, weight_decay, epsilon, corr1, corr2);
+			adamw_vector<false>(i, p4, g4, m4, v4, lr, beta1, beta2, weight_decay, epsilon, corr1, corr2);
 		}
 	}
 	for (uint64_t i = (nvec << 3) + tid; i < num_els; i += nthreads) {
