@@ -21,37 +21,34 @@ __device__ __forceinline__ void adamw_element(float & p, float g, float & m, flo
 	v = v_t;
 }
 
-/* One 16-byte vector of each array: read, updated, written; STREAM: past the caches both ways. */
-template <bool STREAM>
+/* One 16-byte vector of each array: read, updated, written, past the caches both ways. */
 __device__ __forceinline__ void adamw_vector(uint64_t i, u32x4 * param, const u32x4 * grad, u32x4 * mean, u32x4 * var, float lr, float beta1, float beta2,
 											 float weight_decay, float epsilon, float corr1, float corr2) {
 	float p[8], g[8], m[8], v[8];
-	unpack8(STREAM ? __builtin_nontemporal_load(param + i) : param[i], p);
+	unpack8(__builtin_nontemporal_load(param + i), p);
 	unpack8(__builtin_nontemporal_load(grad + i), g);
-	unpack8(STREAM ? __builtin_nontemporal_load(mean + i) : mean[i], m);
-	unpack8(STREAM ? __builtin_nontemporal_load(var + i) : var[i], v);
+	unpack8(__builtin_nontemporal_load(mean + i), m);
+	unpack8(__builtin_nontemporal_load(var + i), v);
 	#pragma unroll
 	for (int e = 0; e < 8; e++) {
 		adamw_element(p[e], g[e], m[e], v[e], lr, beta1, beta2, weight_decay, epsilon, corr1, corr2);
 	}
-	if (STREAM) {
-		__builtin_nontemporal_store(pack8(p), param + i);
-		__builtin_nontemporal_store(pack8(m), mean + i);
-		__builtin_nontemporal_store(pack8(v), var + i);
-	} else {
-		param[i] = pack8(p);
-		mean[i] = pack8(m);
-		var[i] = pack8(v);
-	}
+	__builtin_nontemporal_store(pack8(p), param + i);
+	__builtin_nontemporal_store(pack8(m), mean + i);
+	__builtin_nontemporal_store(pack8(v), var + i);
 }
 
 /* Launch: grid = ceil(num_els / 2048), block = 256: one vector per lane (the loops only take the tail, an unaligned
- * call, or what lies beyond the 2^32 lanes of the largest launch).  A grid bounded at 8192 work-groups that stride over
- * the arrays keeps 32 places of each array open at 32 KiB distances per compute unit and streamed at 4.0-4.5 TB/s; in
- * order of the work-groups it is 5.6-5.9 (277 M elements: 979 -> 695 us, 657 with non-temporal accesses; 805 M: 2490 ->
- * 2068, 2059).  Arrays that the 256 MiB memory-side cache could hold keep their plain accesses (8 M elements: 19.9 us
- * against 20.4). */
-#define ADAMW_STREAM_ELS (1ull << 25)
+ * call, or what lies beyond the 2^32 lanes of the largest launch).
+ * A lane's first vector stands in front of the loop: there the four loads are issued together; inside the loop the
+ * compiler waits for each before it issues the next, four memory round trips in a row.
+ * Every array is accessed non-temporally at every size, in one form: with a plain and a non-temporal form behind a
+ * branch on the size, the compiler merges the two and drops the hint.  Each step passes over all four arrays once, and a
+ * training step passes over far more than the 256 MiB memory-side cache in between.
+ * Measured, us per launch: each load behind the one before / issued together / and non-temporal, with arrays that were
+ * not touched by the last launches: 1 M elements 8.0 / 7.1 / 6.0; 8 M 27.6 / 25.3 / 24.1; 34 M 95 / 87 / 83; 277 M 693 /
+ * 670 / 641 (6.0 TB/s); 805 M 2005 / 1969 / 1884.  Launched over and over on the same arrays, sizes that the cache
+ * holds are fastest with plain accesses (25 M: 68.6 / 59.2 / 61.0), all others as above. */
 extern "C" __global__ void __launch_bounds__(256)
 default_adamw_step_bf16_bf16_bf16_bf16_kernel(uint64_t num_els, int step_num, float lr, float beta1, float beta2, float weight_decay,
 											  float epsilon, bf16_t * param, const bf16_t * grad, bf16_t * mean, bf16_t * var) {
@@ -63,11 +60,10 @@ default_adamw_step_bf16_bf16_bf16_bf16_kernel(uint64_t num_els, int step_num, fl
 	const uint64_t nvec = aligned ? (num_els >> 3) : 0;
 	u32x4 * const p4 = (u32x4 *) param, * const m4 = (u32x4 *) mean, * const v4 = (u32x4 *) var;
 	const u32x4 * const g4 = (const u32x4 *) grad;
-	for (uint64_t i = tid; i < nvec; i += nthreads) {
-		if (num_els > ADAMW_STREAM_ELS) {
-			adamw_vector<true>(i, p4, g4, m4, v4, lr, beta1, beta2, weight_decay, epsilon, corr1, corr2);
-		} else {
-			adamw_vector<false>(i, p4, g4, m4, v4, lr, beta1, beta2, weight_decay, epsilon, corr1, corr2);
+	if (tid < nvec) {
+		adamw_vector(tid, p4, g4, m4, v4, lr, beta1, beta2, weight_decay, epsilon, corr1, corr2);
+		for (uint64_t i = tid + nthreads; i < nvec; i += nthreads) {
+			adamw_vector(i, p4, g4, m4, v4, lr, beta1, beta2, weight_decay, epsilon, corr1, corr2);
 		}
 	}
 	for (uint64_t i = (nvec << 3) + tid; i < num_els; i += nthreads) {

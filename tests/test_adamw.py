@@ -1,6 +1,12 @@
 """AdamW step of the layer's weights: the oracle pinned against the fp64 closed form, the HIP kernel against the
 oracle through the C ABI.  Values: one bf16 rounding of the result plus the fp32 rounding of its terms (the moment update can cancel; powf, sqrtf,
 the divisions and fused multiply-adds differ by an fp32 rounding between libm / the host compiler and the device)."""
+import ctypes as C
+import os
+import re
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -92,5 +98,53 @@ def test_gpu_matches_oracle(backend, oracle, n, step, offset):
 
 @pytest.mark.gpu
 def test_gpu_matches_oracle_beyond_the_caches(backend, oracle):
-    """past the size from which the arrays are accessed non-temporally, with a tail that is no whole vector"""
+    """four arrays that the 256 MiB memory-side cache does not hold together, with a tail that is no whole vector"""
     test_gpu_matches_oracle(backend, oracle, (1 << 25) + 13, 3, 0)
+
+
+def test_kernel_issues_its_loads_together_and_non_temporally(tmp_path):
+    """The two things the kernel's speed rests on are the compiler's to undo, so they are read from the assembly of the
+    kernel's own source: a lane's first four vector loads are in flight together, and every vector access carries nt."""
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ml_dataflow_amd", "csrc")
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    flags = re.search(r"^HIPFLAGS = (.*)$", open(os.path.join(csrc, "Makefile")).read(), flags=re.M).group(1)
+    flags = flags.replace("$(ARCH)", "gfx950").replace("$(INC)", "").split()
+    source, asm = tmp_path / "adamw.hip", tmp_path / "adamw.s"
+    source.write_text('#include "moe_common.h"\n#include "optimizer.hip"\n')
+    subprocess.run([hipcc, *flags, "-I", os.path.join(csrc, "kernels"), "-S", "--cuda-device-only", "-o", str(asm), str(source)], check=True, capture_output=True)
+    body = re.search(r"^default_adamw_step_bf16_bf16_bf16_bf16_kernel:(.*?)s_endpgm", asm.read_text(), flags=re.M | re.S).group(1)
+    lines = [line.strip() for line in body.splitlines()]
+    vector = [line for line in lines if re.match(r"global_(load|store)_dwordx4\b", line)]
+    assert vector and all(re.search(r"\bnt\b", line) for line in vector), vector
+    loads = [i for i, line in enumerate(lines) if line.startswith("global_load_dwordx4")]
+    assert len(loads) >= 4
+    assert not [line for line in lines[loads[0]:loads[3]] if line.startswith("s_waitcnt") and "vmcnt" in line]
+
+
+@pytest.mark.gpu
+def test_gpu_strides_beyond_the_lanes_of_a_launch(backend, oracle):
+    """the kernel itself on a grid of fewer lanes than vectors, as a launch of more than 2^32 vectors would have: 3 groups
+    for 8 groups' worth and a tail"""
+    from ml_dataflow_amd import binding as B
+    print("case adamw strided", flush=True)
+    be, n, step = backend, 8 * 2048 + 13, 4
+    param, grad, mean, var = make(np.random.default_rng(7), n)
+    bufs = [be.upload(a) for a in (param, grad, mean, var)]
+    hip = C.CDLL("libamdhip64.so")
+    module, kernel = C.c_void_p(), C.c_void_p()
+    assert hip.hipModuleLoad(C.byref(module), os.path.join(B.LIB_DIR, "hip_kernels_gfx950.hsaco").encode()) == 0
+    assert hip.hipModuleGetFunction(C.byref(kernel), module, b"default_adamw_step_bf16_bf16_bf16_bf16_kernel") == 0
+    args = [C.c_uint64(n), C.c_int(step)] + [C.c_float(HP[k]) for k in ("lr", "beta1", "beta2", "weight_decay", "epsilon")] + [C.c_void_p(b.ptr) for b in bufs]
+    params = (C.c_void_p * len(args))(*[C.cast(C.byref(a), C.c_void_p) for a in args])
+    assert hip.hipModuleLaunchKernel(kernel, 3, 1, 1, 256, 1, 1, 0, C.c_void_p(be.stream(1)), params, None) == 0
+    be.sync(1)
+    p, m, v = param.copy(), mean.copy(), var.copy()
+    oracle.oracle_adamw_step(n, step, HP["lr"], HP["beta1"], HP["beta2"], HP["weight_decay"], HP["epsilon"], O.ptr(p), O.ptr(grad), O.ptr(m), O.ptr(v))
+    scales = (np.abs(bf16_to_f64(param)).max(), max(np.abs(bf16_to_f64(mean)).max(), np.abs(bf16_to_f64(grad)).max()), np.abs(bf16_to_f64(var)).max())
+    for buf, want, sc in zip((bufs[0], bufs[2], bufs[3]), (p, m, v), scales):
+        near(be.read(buf.ptr, (n,), np.uint16), bf16_to_f64(want), sc, rel=2.0 ** -7)
+    assert hip.hipModuleUnload(module) == 0
+    for buf in bufs:
+        buf.free()
