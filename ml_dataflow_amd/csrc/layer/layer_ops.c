@@ -19,6 +19,12 @@ void layer_set_route_tokens_skeleton(Op_Skeleton * skeleton) {
 	dataflow_fill_skeleton(skeleton, "amd_route_tokens", DATAFLOW_BF16, DATAFLOW_NONE, 17, t);
 }
 
+int layer_has_route_tokens(Dataflow_Handle * handle) {
+	Op_Skeleton skeleton;
+	layer_set_route_tokens_skeleton(&skeleton);
+	return dataflow_find_table(&handle->op_table, skeleton.identifier.fingerprint, false, NULL) >= 0;
+}
+
 int layer_submit_route_tokens(Dataflow_Handle * handle, int stream_id, int num_tokens, int num_experts, int top_k, int model_dim,
 							  void * X, void * w_router, void * logit_bias, void * x_routed, float * token_expert_weights,
 							  uint16_t * chosen_experts, int * expert_counts, int * expert_counts_cumsum, int * host_expert_counts,
