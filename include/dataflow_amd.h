@@ -239,6 +239,7 @@ typedef struct hip_function_config {
 } Hip_Function_Config;
 
 typedef struct hip_function Hip_Function;
+#define HIP_MAX_STOOD_IN 3
 
 /* value type of the op table. Counterpart of Cuda_Function (cuda_dataflow_handle.h:47-64). */
 struct hip_function {
@@ -249,6 +250,9 @@ struct hip_function {
 	int (*hip_external_func)(Dataflow_Handle * dataflow_handle, int stream_id, Op * op, void * op_extra);
 	void * op_extra;
 	Op_Skeleton op_skeleton;
+	/* of an op that stands in for several others: what implemented those (function_handle, or hip_external_func) when it was
+	 * registered, so that its caller can tell whether one of them has been replaced since; unused entries NULL */
+	const void * stands_in_for[HIP_MAX_STOOD_IN];
 };
 
 /* optional per-kernel attribute hook looked up in the launch-config library (cuda_dataflow_handle.h:66) */

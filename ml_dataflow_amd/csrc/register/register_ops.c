@@ -164,6 +164,10 @@ static int register_layer_ops(Dataflow_Handle * handle, const char * dir) {
 		fprintf(stderr, "Error: failed to register the layer's ops, expected %d functions, got %d...\n", N, added);
 		return -1;
 	}
+	if (layer_bind_route_tokens(handle)) {
+		fprintf(stderr, "Error: the layer's routing op needs the matmul, select_experts and build_expert_mapping in the table...\n");
+		return -1;
+	}
 	return added;
 }
 

@@ -53,3 +53,114 @@ def test_a_handle_without_the_routing_op_is_routed_op_by_op(schedule):
     names = NotingHandle().forward(schedule)
     assert names[:3] == ROUTED_BY_OPS
     assert not [name for name in names if name.startswith("amd_route_tokens")]
+
+
+class HipFunction(C.Structure):
+    """include/dataflow_amd.h: Hip_Function"""
+    _fields_ = [("config", C.c_int * 2), ("is_native", C.c_bool), ("function_handle", C.c_void_p), ("set_launch_config", C.c_void_p),
+                ("hip_external_func", C.c_void_p), ("op_extra", C.c_void_p), ("op_skeleton", B.OpSkeleton), ("stands_in_for", C.c_void_p * 3)]
+
+
+def skeleton_of(lib, name):
+    """the skeletons of the three ops that routing consists of, and of the op that stands in for them"""
+    sk = B.OpSkeleton()
+    if name == "matmul":
+        lib.dataflow_set_matmul_skeleton(C.byref(sk))
+    elif name == "select_experts":
+        lib.dataflow_set_default_select_experts_skeleton(C.byref(sk), B.DATAFLOW_BF16)
+    elif name == "build_expert_mapping":
+        lib.dataflow_set_default_build_expert_mapping_skeleton(C.byref(sk))
+    else:
+        sk.header.op_nickname = b"amd_route_tokens_BF16"
+        sk.header.num_args = 17
+        tags = [B.DATAFLOW_INT_SCALAR] * 4 + [B.DATAFLOW_BF16] * 4 + [B.DATAFLOW_FP32, B.DATAFLOW_UINT16] + [B.DATAFLOW_INT] * 5 + [B.DATAFLOW_UINT64_SCALAR, B.DATAFLOW_VOID]
+        sk.header.arg_dtypes = (C.c_int * B.MAX_OP_ARGS)(*tags)
+        assert lib.dataflow_do_fingerprinting(C.byref(sk.header), C.sizeof(sk.header), sk.fingerprint) == 0
+    return sk
+
+
+ROUTING_OPS = ("matmul", "select_experts", "build_expert_mapping")
+
+
+@pytest.mark.parametrize("replaced", [None, *ROUTING_OPS])
+def test_the_routing_op_gives_way_to_a_replaced_one(replaced):
+    """a table as registration leaves it, then another implementation under one of the three skeletons"""
+    noting = NotingHandle(C.sizeof(HipFunction))
+    lib, table = noting.lib, C.byref(noting.h.op_table)
+    implementations = {"matmul": 0x1000, "select_experts": 0x2000, "build_expert_mapping": 0x3000}
+
+    def insert(name, **fields):
+        sk = skeleton_of(lib, name)
+        fn = HipFunction(op_skeleton=sk, **fields)
+        assert lib.dataflow_insert_table(table, C.cast(sk.fingerprint, C.c_void_p), C.cast(C.byref(fn), C.c_void_p)) == 0
+
+    def insert_op(name, implementation):
+        insert(name, is_native=name != "matmul", **{"hip_external_func" if name == "matmul" else "function_handle": implementation})
+
+    for name in ROUTING_OPS:
+        insert_op(name, implementations[name])
+    insert("route", hip_external_func=0x4000, stands_in_for=(C.c_void_p * 3)(*[implementations[name] for name in ROUTING_OPS]))
+    if replaced:
+        assert lib.dataflow_remove_table(table, C.cast(skeleton_of(lib, replaced).fingerprint, C.c_void_p), None) == 0
+        insert_op(replaced, 0x5000)
+    for schedule in (B.AMD_MOE_PER_EXPERT, B.AMD_MOE_GROUPED, B.AMD_MOE_FUSED):
+        names = noting.forward(schedule)
+        if replaced:
+            assert names[:3] == ROUTED_BY_OPS
+        else:
+            assert names[0] == "amd_route_tokens_BF16" and not set(ROUTED_BY_OPS[1:]) & set(names)
+
+
+@pytest.mark.gpu
+def test_gpu_replaced_select_experts_is_the_one_that_runs():
+    """registration notes the real implementations; the op sequence takes over when one of them is exchanged for the same
+    kernel out of a second load of the code object, with the same results"""
+    import os
+
+    import numpy as np
+
+    from ml_dataflow_amd import Backend, MoeLayer
+    from util import normal_bf16
+    print("case replaced select_experts", flush=True)
+    be = Backend(0)
+    rng = np.random.default_rng(5)
+    layer = MoeLayer(be, T, D, E, K, H)
+    layer.load_weights(*(normal_bf16(rng, s, 0.02) for s in ((E, D), (E, H, D), (E, H, D), (E, D, H))))
+    X, resid = normal_bf16(rng, (T, D)), normal_bf16(rng, (T, D))
+    d_X = be.upload(X)
+    names, kind = [], dict(B.DataflowHandle._fields_)["submit_op"]
+    submit = kind(C.cast(be.h.submit_op, C.c_void_p).value)          # a pointer of its own, not the handle's field
+
+    def note(handle, op, stream):
+        names.append(op.contents.op_skeleton.header.op_nickname.decode())
+        return submit(handle, op, stream)
+
+    noting = kind(note)
+    be.h.submit_op = noting
+
+    def forward():
+        names.clear()
+        d_out = be.upload(resid)
+        layer.forward(T, d_X.ptr, d_out.ptr, None, B.AMD_MOE_GROUPED)
+        be.sync()
+        return be.read(d_out.ptr, (T, D), np.uint16)
+
+    first = forward()
+    assert names[0] == "amd_route_tokens_BF16" and "default_select_experts_BF16" not in names
+    hip = C.CDLL("libamdhip64.so")
+    module, kernel = C.c_void_p(), C.c_void_p()
+    assert hip.hipModuleLoad(C.byref(module), os.path.join(B.LIB_DIR, "hip_kernels_gfx950.hsaco").encode()) == 0
+    assert hip.hipModuleGetFunction(C.byref(kernel), module, b"default_select_experts_bf16_kernel") == 0
+    key = C.cast(skeleton_of(be.lib, "select_experts").fingerprint, C.c_void_p)
+    entry = HipFunction()
+    assert be.lib.dataflow_remove_table(C.byref(be.h.op_table), key, C.cast(C.byref(entry), C.c_void_p)) == 0
+    assert entry.is_native and entry.function_handle != kernel.value
+    entry.function_handle = kernel.value
+    assert be.lib.dataflow_insert_table(C.byref(be.h.op_table), key, C.cast(C.byref(entry), C.c_void_p)) == 0
+    second = forward()
+    assert names[:3] == ROUTED_BY_OPS
+    assert (first == second).all()
+    be.h.submit_op = submit
+    layer.free()
+    be.close()
+    assert hip.hipModuleUnload(module) == 0
