@@ -13,8 +13,8 @@
 /* Router product, selection, counts, prefix sum and dispatch permutation: what dataflow_submit_matmul (logits = X Wr^T +
  * bias), clearing the count arrays, dataflow_submit_default_select_experts and dataflow_submit_default_build_expert_mapping
  * leave, bit for bit, from at most four launches (../matmul/route_kernel.h).
- * Up to 512 experts and 32 slots; the workspace (16-byte aligned) holds LAYER_ROUTE_WORKSPACE bytes and, where there is
- * room, the partial sums of a router product split along its K. */
+ * Up to 512 experts and 32 slots; the workspace (16-byte aligned) has at least LAYER_ROUTE_WORKSPACE bytes.  The router
+ * product is split along its K where the matmul would split it with that workspace. */
 #define LAYER_ROUTE_MAX_EXPERTS 512
 #define LAYER_ROUTE_WORKSPACE(tokens, experts) (((uint64_t) (tokens) + 31) / 32 * (2 * (uint64_t) (experts) + 16) + 256)
 LAYER_OPS_HIDDEN void layer_set_route_tokens_skeleton(Op_Skeleton * skeleton);

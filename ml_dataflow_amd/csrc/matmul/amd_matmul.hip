@@ -528,6 +528,15 @@ static int plan_split(GemmParams & p, bool direct, float * workspace, uint64_t w
 	return 1;
 }
 
+/* the pass behind the partial products: D from their sums */
+static int launch_split_reduce(const GemmParams & p, hipStream_t stream) {
+	const uint64_t count = (uint64_t) p.M * (uint64_t) p.N;
+	const long blocks = (long) ((count + 255) / 256);
+	hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned int) (blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream,
+					   (const float *) p.partial, p.split_k, (long long) count, p.alpha, p.beta, p.C, p.D);
+	return check_launch();
+}
+
 /* shared by amd_matmul and amd_matmul_no_alloc: checks, kernel choice, launch.  `workspace` (may be NULL) holds the fp32
  * partial sums of a split along K; `must_fit`: a split that the workspace cannot hold is an error instead of running
  * unsplit */
@@ -559,11 +568,7 @@ static int run_matmul(Dataflow_Handle * dataflow_handle, int stream_id, GemmPara
 		if (launch_split(p, transa, transb, stream)) {
 			return -1;
 		}
-		const uint64_t count = (uint64_t) p.M * (uint64_t) p.N;
-		const long blocks = (long) ((count + 255) / 256);
-		hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned int) (blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream,
-						   (const float *) workspace, p.split_k, (long long) count, p.alpha, p.beta, p.C, p.D);
-		return check_launch();
+		return launch_split_reduce(p, stream);
 	}
 	return launch_gemm<MODE_SINGLE>(p, transa, transb, direct, grid_big, grid_small, cu_count, stream);
 }
@@ -858,14 +863,22 @@ extern "C" int amd_route_tokens(Dataflow_Handle * dataflow_handle, int stream_id
 		fprintf(stderr, "Error: hipSetDevice failed in the routing op...\n");
 		return -1;
 	}
-	r.counts = workspace;
-	float * partial = (float *) (workspace + counts_bytes);
 	const long cu_count = extra_cu_count(op_extra);
 	const bool direct = operand_direct_ok(p.A, false, p.M, p.K, 0) && operand_direct_ok(p.B, false, p.N, p.K, 0);
-	if (plan_split(p, direct, partial, workspace_bytes - counts_bytes, cu_count, false)) {
-		r.partial = partial;
-		r.splits = p.split_k;
+	r.counts = workspace;
+	/* The product is split where the matmul op splits it, by the whole workspace: another order of the sums would be another
+	 * rounding of the logits.  Selection adds up the partial sums itself if the counts fit behind them; if they do not, the
+	 * sums are reduced first and the counts then overwrite them. */
+	if (plan_split(p, direct, (float *) workspace, workspace_bytes, cu_count, false)) {
 		if (launch_split(p, 1, 0, stream)) {
+			return -1;
+		}
+		const uint64_t partial_bytes = ((uint64_t) p.split_k * (uint64_t) r.T * (uint64_t) r.E * sizeof(float) + 255) & ~255UL;
+		if (partial_bytes <= workspace_bytes && counts_bytes <= workspace_bytes - partial_bytes) {
+			r.partial = p.partial;
+			r.splits = p.split_k;
+			r.counts = workspace + partial_bytes;
+		} else if (launch_split_reduce(p, stream)) {
 			return -1;
 		}
 	} else if (launch_gemm<MODE_SINGLE>(p, 1, 0, direct, tiles_of(p.M, 256) * tiles_of(p.N, 256), tiles_of(p.M, 128) * tiles_of(p.N, 128), cu_count, stream)) {

@@ -22,6 +22,28 @@ def outputs(be, L, T, E, K):
             "host_counts": np.ctypeslib.as_array(C.cast(L.host_expert_counts, C.POINTER(C.c_int32)), (E,)).copy()}
 
 
+def compare(be, L, layer, T, E, K, D, d_X, d_out, d_bias):
+    """a forward, then the same routing op by op; returns what both left"""
+    layer.forward(T, d_X.ptr, d_out.ptr, d_bias.ptr if d_bias else None, B.AMD_MOE_FUSED)
+    got = outputs(be, L, T, E, K)
+    be.zero(L.x_routed, T * E * 2, CS)
+    be.zero(L.expert_counts, (E + 1) * 4, CS)
+    be.zero(L.expert_counts_cumsum, E * 4, CS)
+    be.zero(L.expert_mapping, T * K * 4, CS)
+    be.zero(L.token_mapping, T * K * 4, CS)
+    lib, hp, bptr = be.lib, be.hp, d_bias.ptr if d_bias else None
+    assert lib.dataflow_submit_matmul(hp, CS, BF, BF, BF if d_bias else B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 1, 0, E, D, T, 1.0, 1.0 if d_bias else 0.0,
+                                      L.w_router, d_X.ptr, bptr, L.x_routed, L.kernel_workspace_bytes, L.kernel_workspace) == 0
+    assert lib.dataflow_submit_default_select_experts(hp, CS, BF, T, E, K, L.x_routed, L.token_expert_weights, L.chosen_experts, L.expert_counts,
+                                                      L.expert_counts_cumsum, L.host_expert_counts) == 0
+    assert lib.dataflow_submit_default_build_expert_mapping(hp, CS, T, E, K, L.chosen_experts, L.expert_counts_cumsum, L.expert_mapping,
+                                                            L.token_mapping) == 0
+    want = outputs(be, L, T, E, K)
+    for name in want:
+        assert (got[name] == want[name]).all(), name
+    return got
+
+
 @pytest.mark.parametrize("T,E,K,D,bias", [
     (1, 8, 2, 64, False), (16, 64, 8, 4096, False), (31, 5, 3, 512, True), (128, 64, 8, 1024, False), (129, 64, 8, 1024, True),
     (256, 8, 2, 512, False), (257, 8, 2, 512, False), (255, 17, 4, 64, True), (1000, 7, 1, 2048, False), (3001, 32, 4, 2048, True),
@@ -39,22 +61,33 @@ def test_routing_equals_the_op_sequence(backend, T, E, K, D, bias):
     be.zero(L.slab, L.slab_bytes, CS)
     be.sync(CS)
     be.write(L.w_router, Wr)
-    layer.forward(T, d_X.ptr, d_out.ptr, d_bias.ptr if bias else None, B.AMD_MOE_FUSED)
-    got = outputs(be, L, T, E, K)
-    be.zero(L.x_routed, T * E * 2, CS)
-    be.zero(L.expert_counts, (E + 1) * 4, CS)
-    be.zero(L.expert_counts_cumsum, E * 4, CS)
-    be.zero(L.expert_mapping, T * K * 4, CS)
-    be.zero(L.token_mapping, T * K * 4, CS)
-    lib, hp, bptr = be.lib, be.hp, d_bias.ptr if bias else None
-    assert lib.dataflow_submit_matmul(hp, CS, BF, BF, BF if bias else B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 1, 0, E, D, T, 1.0, 1.0 if bias else 0.0,
-                                      L.w_router, d_X.ptr, bptr, L.x_routed, L.kernel_workspace_bytes, L.kernel_workspace) == 0
-    assert lib.dataflow_submit_default_select_experts(hp, CS, BF, T, E, K, L.x_routed, L.token_expert_weights, L.chosen_experts, L.expert_counts,
-                                                      L.expert_counts_cumsum, L.host_expert_counts) == 0
-    assert lib.dataflow_submit_default_build_expert_mapping(hp, CS, T, E, K, L.chosen_experts, L.expert_counts_cumsum, L.expert_mapping,
-                                                            L.token_mapping) == 0
-    want = outputs(be, L, T, E, K)
-    for name in want:
-        assert (got[name] == want[name]).all(), name
+    got = compare(be, L, layer, T, E, K, D, d_X, d_out, d_bias)
+    assert got["counts"][:E].sum() == T * K
+    layer.free()
+
+
+@pytest.mark.parametrize("T,E,K,D,room", [(512, 64, 8, 4096, -4), (512, 64, 8, 4096, 0), (512, 64, 8, 4096, 1020), (512, 64, 8, 4096, 1024),
+                                          (100, 20, 4, 2048, 0), (3001, 32, 4, 2048, 100), (256, 8, 2, 1024, 0)])
+def test_routing_splits_the_product_as_the_matmul_does(backend, T, E, K, D, room):
+    """a workspace of the partial sums' size plus `room` bytes: without it the product runs unsplit, in another order of its
+    sums; the counts that the routing keeps there too (1024 bytes for 512 tokens and 64 experts) do not take it from them"""
+    print("case routing workspace T=%d E=%d K=%d D=%d room=%d" % (T, E, K, D, room), flush=True)
+    be = backend
+    k_tiles, cus = (D + 63) // 64, be.device_info.cu_count
+    splits = cus // (((T + 127) // 128) * ((E + 127) // 128))
+    per = max(4, (-(-k_tiles // splits) + 3) & ~3)
+    splits = -(-k_tiles // per)
+    assert splits > 1
+    rng = np.random.default_rng(T + E + K + D)
+    X, Wr = normal_bf16(rng, (T, D)), normal_bf16(rng, (E, D), 0.02)
+    layer = MoeLayer(be, T, D, E, K, 256)
+    L = layer.L
+    assert L.kernel_workspace_bytes >= splits * T * E * 4 + room
+    L.kernel_workspace_bytes = splits * T * E * 4 + room            # what the ops are told: the layer's own is larger
+    d_X, d_out = be.upload(X), be.alloc(T * D * 2)
+    be.zero(L.slab, L.slab_bytes, CS)
+    be.sync(CS)
+    be.write(L.w_router, Wr)
+    got = compare(be, L, layer, T, E, K, D, d_X, d_out, None)
     assert got["counts"][:E].sum() == T * K
     layer.free()
