@@ -238,7 +238,7 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 	/* router logits, selection, counts and mapping (dataflow_transformer.c:2710-2784): one op where the handle has it and
 	 * its limits hold */
 	if (E <= LAYER_ROUTE_MAX_EXPERTS && K <= 32 && T <= (1 << 17) && L->kernel_workspace_bytes >= LAYER_ROUTE_WORKSPACE(T, E)
-		&& layer_has_route_tokens(h)) {
+		&& ((uintptr_t) L->kernel_workspace & 15) == 0 && layer_has_route_tokens(h)) {
 		CHECK(layer_submit_route_tokens(h, cs, T, E, K, D, X, L->w_router, logit_bias, L->x_routed, L->token_expert_weights, L->chosen_experts,
 										L->expert_counts, L->expert_counts_cumsum, L->host_expert_counts, L->expert_mapping, L->token_mapping,
 										L->kernel_workspace_bytes, L->kernel_workspace), "failed to submit routing");

@@ -82,33 +82,45 @@ def skeleton_of(lib, name):
 ROUTING_OPS = ("matmul", "select_experts", "build_expert_mapping")
 
 
+class RegisteredHandle(NotingHandle):
+    """with a table as registration leaves it: the three ops, and the one that stands in for them"""
+
+    def __init__(self):
+        super().__init__(C.sizeof(HipFunction))
+        for i, name in enumerate(ROUTING_OPS):
+            self.insert_op(name, 0x1000 * (i + 1))
+        self.insert("route", hip_external_func=0x4000, stands_in_for=(C.c_void_p * 3)(0x1000, 0x2000, 0x3000))
+
+    def insert(self, name, **fields):
+        sk = skeleton_of(self.lib, name)
+        fn = HipFunction(op_skeleton=sk, **fields)
+        assert self.lib.dataflow_insert_table(C.byref(self.h.op_table), C.cast(sk.fingerprint, C.c_void_p), C.cast(C.byref(fn), C.c_void_p)) == 0
+
+    def insert_op(self, name, implementation):
+        self.insert(name, is_native=name != "matmul", **{"hip_external_func" if name == "matmul" else "function_handle": implementation})
+
+
 @pytest.mark.parametrize("replaced", [None, *ROUTING_OPS])
 def test_the_routing_op_gives_way_to_a_replaced_one(replaced):
     """a table as registration leaves it, then another implementation under one of the three skeletons"""
-    noting = NotingHandle(C.sizeof(HipFunction))
+    noting = RegisteredHandle()
     lib, table = noting.lib, C.byref(noting.h.op_table)
-    implementations = {"matmul": 0x1000, "select_experts": 0x2000, "build_expert_mapping": 0x3000}
-
-    def insert(name, **fields):
-        sk = skeleton_of(lib, name)
-        fn = HipFunction(op_skeleton=sk, **fields)
-        assert lib.dataflow_insert_table(table, C.cast(sk.fingerprint, C.c_void_p), C.cast(C.byref(fn), C.c_void_p)) == 0
-
-    def insert_op(name, implementation):
-        insert(name, is_native=name != "matmul", **{"hip_external_func" if name == "matmul" else "function_handle": implementation})
-
-    for name in ROUTING_OPS:
-        insert_op(name, implementations[name])
-    insert("route", hip_external_func=0x4000, stands_in_for=(C.c_void_p * 3)(*[implementations[name] for name in ROUTING_OPS]))
     if replaced:
         assert lib.dataflow_remove_table(table, C.cast(skeleton_of(lib, replaced).fingerprint, C.c_void_p), None) == 0
-        insert_op(replaced, 0x5000)
+        noting.insert_op(replaced, 0x5000)
     for schedule in (B.AMD_MOE_PER_EXPERT, B.AMD_MOE_GROUPED, B.AMD_MOE_FUSED):
         names = noting.forward(schedule)
         if replaced:
             assert names[:3] == ROUTED_BY_OPS
         else:
             assert names[0] == "amd_route_tokens_BF16" and not set(ROUTED_BY_OPS[1:]) & set(names)
+
+
+@pytest.mark.parametrize("changes", [{"kernel_workspace": (9 << 24) + 8}, {"kernel_workspace_bytes": 256}, {"num_experts": 520}])
+def test_the_routing_op_gives_way_where_its_limits_do_not_hold(changes):
+    """a workspace off a 16-byte boundary, one too small for the counts, more experts than it takes: all of which the ops take"""
+    names = RegisteredHandle().forward(B.AMD_MOE_FUSED, **changes)
+    assert names[:3] == ROUTED_BY_OPS
 
 
 @pytest.mark.gpu
