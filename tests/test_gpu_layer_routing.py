@@ -91,3 +91,44 @@ def test_routing_splits_the_product_as_the_matmul_does(backend, T, E, K, D, room
     got = compare(be, L, layer, T, E, K, D, d_X, d_out, None)
     assert got["counts"][:E].sum() == T * K
     layer.free()
+
+
+NEG_INF, INF, NAN = 0xFF80, 0x7F80, 0x7FC0
+
+
+@pytest.mark.parametrize("T,E,K,D,offset", [(40, 8, 2, 64, 0), (100, 20, 4, 512, 1), (33, 7, 3, 512, 0), (256, 64, 4, 1024, 1), (300, 64, 8, 1024, 0),
+                                            (700, 13, 5, 2048, 1), (1000, 32, 4, 64, 1), (290, 512, 9, 576, 0), (64, 40, 32, 512, 0)])
+def test_routing_of_masked_infinite_and_nan_logits(backend, T, E, K, D, offset):
+    """experts masked with a bias of -inf, down to rows with fewer than K experts left (slots without an expert) and with none;
+    NaN and +inf logits; offset 1: a bias that starts 2 bytes off every larger alignment"""
+    print("case routing special T=%d E=%d K=%d D=%d offset=%d" % (T, E, K, D, offset), flush=True)
+    be = backend
+    rng = np.random.default_rng(T + E + K + D)
+    X, Wr = normal_bf16(rng, (T, D)), normal_bf16(rng, (E, D), 0.02)
+    bias = normal_bf16(rng, (T, E))
+    bias[rng.random((T, E)) < 0.3] = NEG_INF
+    bias[0] = NEG_INF                                     # no expert left
+    bias[1, :], bias[1, E // 2] = NEG_INF, 0              # one
+    bias[2, :], bias[2, E - K:] = NEG_INF, 0              # just enough
+    bias[3, 1] = NAN
+    bias[4, :] = NAN
+    bias[5, E - 1] = INF
+    bias[6, 0], bias[6, 2] = INF, NAN
+    bias[T - 1, :K - 1], bias[T - 1, K - 1:] = 0, NEG_INF  # one too few, in the last token
+    layer = MoeLayer(be, T, D, E, K, 256)
+    L = layer.L
+    d_X, d_out = be.upload(X), be.alloc(T * D * 2)
+    d_bias = be.upload(np.concatenate([np.zeros(offset, np.uint16), bias.ravel()]))
+    d_bias.ptr += 2 * offset
+    be.zero(L.slab, L.slab_bytes, CS)                     # the mappings of slots without an expert are left as they are: in range
+    be.sync(CS)
+    be.write(L.w_router, Wr)
+    got = compare(be, L, layer, T, E, K, D, d_X, d_out, d_bias)
+    d_bias.ptr -= 2 * offset
+    assert (got["chosen"][0] == 0xFFFF).all() and sorted(got["chosen"][1])[0] == E // 2 and (got["chosen"][4] == 0xFFFF).all()
+    assert sorted(got["chosen"][2]) == list(range(E - K, E))
+    assert (got["chosen"][T - 1] == 0xFFFF).sum() == 1 and (got["chosen"][5] == E - 1).any() and (got["chosen"][6] == 0).any()
+    valid = got["chosen"] < E
+    assert (got["counts"][:E] == np.bincount(got["chosen"][valid], minlength=E)).all()
+    assert (np.sort(got["token_mapping"][valid]) == np.arange(valid.sum())).all()
+    layer.free()
