@@ -53,7 +53,8 @@ struct RouteParams {
 template <int AHEAD, int SPLITS>
 __device__ __forceinline__ void route_stage_quads(const RouteParams & p, uint32_t * __restrict__ tile, int t0, int quads, int items, int c0) {
 	const long long count = (long long) p.T * p.E;
-	const bool whole = (p.E & 3) == 0;                   /* then a quad is whole and aligned */
+	const bool whole = (p.E & 3) == 0;                   /* then a quad is whole, and aligned in the partial sums */
+	const bool whole_logits = whole && (((uintptr_t) p.x_routed) & 7) == 0;
 	const float * __restrict__ partial = p.partial;
 	for (int i0 = threadIdx.x; i0 < items; i0 += AHEAD * (int) blockDim.x) {
 		long long at[AHEAD];
@@ -123,7 +124,7 @@ __device__ __forceinline__ void route_stage_quads(const RouteParams & p, uint32_
 				}
 				const uint32_t lo = bits[0] | (bits[1] << 16), hi = bits[2] | (bits[3] << 16);
 				if (partial) {
-					if (whole) {
+					if (whole_logits) {
 						*((u32x2 *) (p.x_routed + at[u])) = u32x2{lo, hi};
 					} else {
 						#pragma unroll

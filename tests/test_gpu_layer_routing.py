@@ -132,3 +132,23 @@ def test_routing_of_masked_infinite_and_nan_logits(backend, T, E, K, D, offset):
     assert (got["counts"][:E] == np.bincount(got["chosen"][valid], minlength=E)).all()
     assert (np.sort(got["token_mapping"][valid]) == np.arange(valid.sum())).all()
     layer.free()
+
+
+def test_routing_writes_logits_at_any_element(backend):
+    """x_routed 2 bytes off an 8-byte boundary, rows of whole quads: element by element, nothing in front or behind touched"""
+    print("case routing unaligned logits", flush=True)
+    be, (T, E, K, D) = backend, (31, 20, 4, 512)
+    rng = np.random.default_rng(3)
+    X, Wr = normal_bf16(rng, (T, D)), normal_bf16(rng, (E, D), 0.02)
+    layer = MoeLayer(be, T, D, E, K, 256)
+    L = layer.L
+    d_X, d_out = be.upload(X), be.alloc(T * D * 2)
+    d_logits = be.upload(np.full(T * E + 8, 0x1234, np.uint16))
+    be.zero(L.slab, L.slab_bytes, CS)
+    be.sync(CS)
+    be.write(L.w_router, Wr)
+    L.x_routed = d_logits.ptr + 2
+    compare(be, L, layer, T, E, K, D, d_X, d_out, None)
+    around = be.read(d_logits.ptr, (T * E + 8,), np.uint16)
+    assert around[0] == 0x1234 and (around[T * E + 1:] == 0x1234).all()
+    layer.free()
