@@ -88,6 +88,25 @@ class HipEvents:
         return float(ms.value)
 
 
+def submit_route_tokens(be, layer, T, d_X, d_bias, stream_id):
+    """The op the layer routes with (router product, selection, counts, permutation: csrc/layer/layer_ops.h).  It is the layer
+    driver's own, without a submit wrapper, so it goes to the handle as an op built here."""
+    from ml_dataflow_amd import binding as B
+    L, op = layer.L, B.Op()
+    header = op.op_skeleton.header
+    header.op_nickname, header.num_args = b"amd_route_tokens_BF16", 17
+    tags = [B.DATAFLOW_INT_SCALAR] * 4 + [B.DATAFLOW_BF16] * 4 + [B.DATAFLOW_FP32, B.DATAFLOW_UINT16] + [B.DATAFLOW_INT] * 5 + [B.DATAFLOW_UINT64_SCALAR, B.DATAFLOW_VOID]
+    header.arg_dtypes = (C.c_int * B.MAX_OP_ARGS)(*tags)
+    if be.lib.dataflow_do_fingerprinting(C.byref(header), C.sizeof(header), op.op_skeleton.fingerprint) != 0:
+        return -1
+    pointers = [d_X.ptr, L.w_router, d_bias.ptr if d_bias else None, L.x_routed, L.token_expert_weights, L.chosen_experts, L.expert_counts,
+                L.expert_counts_cumsum, L.host_expert_counts, L.expert_mapping, L.token_mapping]
+    args = [C.c_int(v) for v in (T, layer.E, layer.K, layer.D)] + [C.c_void_p(v) for v in pointers] + [C.c_uint64(L.kernel_workspace_bytes), C.c_void_p(L.kernel_workspace)]
+    for i, value in enumerate(args):
+        op.op_args[i] = C.addressof(value)
+    return be.h.submit_op(be.hp, C.byref(op), stream_id)
+
+
 def replay_step_with_events(be, layer, T, d_X, d_out, d_dY, d_dX, d_bias, backward, ev, stream, fused, first=False):
     """Submits the grouped (or fused) schedule op by op (same ops, same order as amd_moe_layer_forward/_backward, all
     on the compute stream) with an event pair around every launch; returns [(kernel class, ms)].  first: the weight-gradient
@@ -119,15 +138,7 @@ def replay_step_with_events(be, layer, T, d_X, d_out, d_dY, d_dX, d_bias, backwa
     def wc(ptr):
         return None if first else ptr
 
-    bias = d_bias.ptr if d_bias else None
-    timed("router_gemm", lib.dataflow_submit_matmul, hp, CS, BF, BF, BF if bias else NONE, BF, F32, 1, 0, E, D, T, 1.0, 1.0 if bias else 0.0,
-          L.w_router, d_X.ptr, bias, L.x_routed, L.kernel_workspace_bytes, ws)
-    be.zero(L.expert_counts, (E + 1) * 4, CS)
-    be.zero(L.expert_counts_cumsum, E * 4, CS)
-    timed("select_experts", lib.dataflow_submit_default_select_experts, hp, CS, BF, T, E, K, L.x_routed, L.token_expert_weights, L.chosen_experts,
-          L.expert_counts, L.expert_counts_cumsum, L.host_expert_counts)
-    timed("build_expert_mapping", lib.dataflow_submit_default_build_expert_mapping, hp, CS, T, E, K, L.chosen_experts, L.expert_counts_cumsum,
-          L.expert_mapping, L.token_mapping)
+    timed("route_tokens", submit_route_tokens, be, layer, T, d_X, d_bias, CS)
     if fused:
         # no dispatch copy in the fused forward: the up-projection's loaders gather the rows of X through expert_mapping
         timed("gemm_up13", lib.dataflow_submit_amd_grouped_matmul_gathered, hp, CS, BF, BF, NONE, BF, F32, 1, 0, B.AMD_GROUPED_RAGGED_N, 2 * H, D, R, E, cum,
@@ -278,8 +289,8 @@ def algorithmic_work(T, D, E, K, H, fused):
         "combine_grad": ("hbm", 2.0 * R * D + (2.0 if fused else 4.0) * T * D + 4.0 * T * K),
         "swiglu": ("hbm", 6.0 * R * H), "swiglu_bwd_x": ("hbm", 10.0 * R * H), "swiglu_bwd_x_routed": ("hbm", 12.0 * R * H + 18.0 * R),
         "router_bwd_x": ("hbm", 2.0 * T * D + 4.0 * R * D + 10.0 * R),
-        "select_experts": ("hbm", 2.0 * T * E + 6.0 * T * K + 12.0 * E),
-        "build_expert_mapping": ("hbm", 10.0 * T * K),
+        # X and the router weight read; logits, weights, ids, both mappings and the counts written
+        "route_tokens": ("hbm", 2.0 * T * D + 2.0 * E * D + 2.0 * T * E + 14.0 * T * K + 12.0 * E),
         "router_gate_bwd_x": ("hbm", 10.0 * T * K),
         # RMS norm around the layer (reported beside the layer's kernels, not part of the timed step)
         "rms_norm": ("hbm", 4.0 * T * D + 4.0 * T), "rms_norm_bwd_x": ("hbm", 10.0 * T * D),

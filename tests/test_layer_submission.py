@@ -31,18 +31,23 @@ class NotingHandle:
         self.hash = HASH(lambda key, size: key[31] % size)
         assert self.lib.dataflow_init_table(C.byref(self.h.op_table), C.cast(self.hash, C.c_void_p), 32, value_bytes, 64, 256, 0.75, 0.1) == 0
 
-    def forward(self, schedule, **changes):
-        """the ops of one forward; no pointer of the layer is followed but that of the counts on the host"""
+    def layer(self, **changes):
+        """no pointer of it is followed but that of the counts on the host"""
         layer = B.AmdMoeLayer(max_tokens=T, model_dim=D, num_experts=E, top_k=K, expert_dim=H, dt=B.DATAFLOW_BF16, expert_stride_bytes=3 * H * D * 2)
         for i, (name, kind) in enumerate(B.AmdMoeLayer._fields_):
             if kind is C.c_void_p:
                 setattr(layer, name, (i + 1) << 24)
         layer.w3, layer.dw3 = layer.w1 + H * D * 2, layer.dw1 + H * D * 2
         layer.kernel_workspace_bytes = 1 << 23
-        counts = (C.c_int * E)(*[T * K // E] * E)
-        layer.host_expert_counts = C.addressof(counts)
+        self.counts = (C.c_int * E)(*[T * K // E] * E)
+        layer.host_expert_counts = C.addressof(self.counts)
         for name, value in changes.items():
             setattr(layer, name, value)
+        return layer
+
+    def forward(self, schedule, **changes):
+        """the ops of one forward"""
+        layer = self.layer(**changes)
         self.names.clear()
         assert self.lib.amd_moe_layer_forward(C.pointer(self.h), 1, 2, C.byref(layer), T, 1 << 32, None, 2 << 32, schedule) == 0
         return list(self.names)
@@ -121,6 +126,32 @@ def test_the_routing_op_gives_way_where_its_limits_do_not_hold(changes):
     """a workspace off a 16-byte boundary, one too small for the counts, more experts than it takes: all of which the ops take"""
     names = RegisteredHandle().forward(B.AMD_MOE_FUSED, **changes)
     assert names[:3] == ROUTED_BY_OPS
+
+
+@pytest.mark.parametrize("first", [False, True])
+@pytest.mark.parametrize("schedule", [B.AMD_MOE_GROUPED, B.AMD_MOE_FUSED])
+def test_the_benchmark_times_the_ops_the_layer_submits(schedule, first):
+    """bench.py's kernel table comes from a replay of the step op by op: the same ops in the same order as the layer's own"""
+    import bench
+    noting = RegisteredHandle()
+    lib, hp, layer = noting.lib, C.pointer(noting.h), noting.layer()
+    flag = B.AMD_MOE_FIRST_MICRO_BATCH if first else 0
+    assert lib.amd_moe_layer_forward(hp, 1, 2, C.byref(layer), T, 1 << 32, None, 2 << 32, schedule) == 0
+    assert lib.amd_moe_layer_backward(hp, 1, 2, C.byref(layer), T, 1 << 32, 3 << 32, 4 << 32, schedule | flag) == 0
+    submitted = list(noting.names)
+    noting.names.clear()
+
+    class Stub:
+        def __init__(self, **fields):
+            self.__dict__.update(fields)
+
+    be = Stub(lib=lib, h=noting.h, hp=hp, zero=lambda *a: None, sync=lambda *a: None)
+    ev = Stub(new=lambda: None, record=lambda *a: None, elapsed_ms=lambda *a: 0.0)
+    buffers = [Stub(ptr=n << 32) for n in (1, 2, 3, 4)]
+    rows = bench.replay_step_with_events(be, Stub(L=layer, T=T, D=D, E=E, K=K, H=H), T, *buffers, None, True, ev, None, schedule == B.AMD_MOE_FUSED, first)
+    assert noting.names == submitted
+    work = bench.algorithmic_work(T, D, E, K, H, schedule == B.AMD_MOE_FUSED)
+    assert len(rows) == len(submitted) and all(name in work for name, _ in rows)
 
 
 @pytest.mark.gpu
