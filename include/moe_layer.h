@@ -1,7 +1,8 @@
 /*
  * moe_layer.h -- host-side driver of one mixture-of-experts layer on top of a Dataflow_Handle.
  *
- * It submits the same operator sequence as the MoE part of the reference's transformer block:
+ * It does the work of the MoE part of the reference's transformer block, by its operator sequence or a shorter one with the
+ * same results:
  *   forward   libdataflowmodels/src/transformer/src/dataflow_transformer.c:2700-2986
  *   bwd_x     dataflow_transformer.c:3386-3719
  *   bwd_w     dataflow_transformer.c:4013-4185
@@ -9,6 +10,13 @@
  * x_routed, token_expert_weights, chosen_experts, expert_counts, expert_counts_cumsum, expert_mapping,
  * token_mapping, x_1, x_3, x_expert_zones, kernelWorkspace) and the same per-expert weight layout
  * (prep_transformer.c:152-160: w1, w3, w2 of expert e stored back to back, experts at a fixed stride).
+ *
+ * Routing, on every schedule: the router product, selection, counts and mapping (dataflow_transformer.c:2710-2784) are one
+ * op of the layer's own, bit-identical to the reference's sequence of matmul, fills, select_experts and
+ * build_expert_mapping with the same workspace.  That sequence is submitted instead where the handle does not hold the op
+ * (its ops were registered one by one), where one of those ops has been replaced in the handle's table since it was
+ * registered, with more than 512 experts, 32 slots or 131072 tokens, and with a workspace that is not 16-byte aligned or
+ * has less than ceil(tokens / 32) * (2 * experts + 16) + 256 bytes.
  *
  * Three schedules; the first two produce the same results bit for bit:
  *   AMD_MOE_PER_EXPERT  the reference's: sync after routing, read host_expert_counts, then a host loop over

@@ -47,8 +47,9 @@ __device__ __forceinline__ void adamw_vector(uint64_t i, u32x4 * param, const u3
  * training step passes over far more than the 256 MiB memory-side cache in between.
  * Measured, us per launch: each load behind the one before / issued together / and non-temporal, with arrays that were
  * not touched by the last launches: 1 M elements 8.0 / 7.1 / 6.0; 8 M 27.6 / 25.3 / 24.1; 34 M 95 / 87 / 83; 277 M 693 /
- * 670 / 641 (6.0 TB/s); 805 M 2005 / 1969 / 1884.  Launched over and over on the same arrays, sizes that the cache
- * holds are fastest with plain accesses (25 M: 68.6 / 59.2 / 61.0), all others as above. */
+ * 670 / 641 (6.0 TB/s); 805 M 2005 / 1969 / 1884.  Launched over and over on the same arrays: the same order or no
+ * difference, but for 17 to 34 M elements, which the cache holds and plain accesses serve 1-6 % faster (25 M: 68.6 /
+ * 59.2 / 61.0). */
 extern "C" __global__ void __launch_bounds__(256)
 default_adamw_step_bf16_bf16_bf16_bf16_kernel(uint64_t num_els, int step_num, float lr, float beta1, float beta2, float weight_decay,
 											  float epsilon, bf16_t * param, const bf16_t * grad, bf16_t * mean, bf16_t * var) {

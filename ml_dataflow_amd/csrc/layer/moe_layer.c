@@ -1,11 +1,12 @@
 /*
  * moe_layer.c -- submits the MoE layer's operator sequence to a Dataflow_Handle (see include/moe_layer.h).
  *
- * The per-expert schedule restates, op for op, the MoE part of
- * libdataflowmodels/src/transformer/src/dataflow_transformer.c (forward :2700-2986, bwd_x :3386-3719,
- * bwd_w :4013-4185) including its stream fork/join and workspace halving; the grouped schedule replaces
- * each host loop over experts by one grouped launch and never waits for the device; the fused schedule is the
- * grouped one without the backward recompute of the expert outputs.
+ * The per-expert schedule restates the MoE part of libdataflowmodels/src/transformer/src/dataflow_transformer.c
+ * (forward :2700-2986, bwd_x :3386-3719, bwd_w :4013-4185) including its stream fork/join and workspace halving; the
+ * grouped schedule replaces each host loop over experts by one grouped launch and never waits for the device; the
+ * fused schedule is the grouped one without the backward recompute of the expert outputs.  What follows the routing is
+ * restated op for op; the routing itself (:2710-2784) is one op with the same results on all three schedules, or the
+ * reference's ops where that one is not there or does not apply (layer_ops.h).
  */
 #include "moe_layer.h"
 #include "layer_ops.h"

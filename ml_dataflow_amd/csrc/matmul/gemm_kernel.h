@@ -66,7 +66,7 @@ struct GemmParams {
 	 * (no alpha, beta or C) to partial[ks][n * M + m]; splitk_reduce_kernel turns them into D */
 	float * partial;
 	int split_k;                   /* 0 or 1: off */
-	int kt_per_split;              /* even */
+	int kt_per_split;              /* a multiple of 4, as the host plans it; the kernel takes any */
 	/* Ragged-N launches without C that several tilings can take are launched on each candidate; every work-group counts
 	 * the tiles of the tilings from the device prefix sum (ragged_n_choice) and the kernels that lose return at once.
 	 * One bit per tiling, RAGGED_N_288 always among them; 0: run */
@@ -1063,8 +1063,9 @@ gemm_bf16_direct_kernel(GemmParams p) {
 		}
 	}
 
-	/* a split of K is an even number of k-tiles, so the stage that the loop multiplies beyond an odd count only
-	 * ever holds k-tiles past K (zeros), never the next split's */
+	/* A split ends where the next begins.  The loop over more than two stages stops there; the two-stage loop multiplies
+	 * one stage beyond an odd count, which holds zeros past K but would hold the next split's k-tile in front of it, so
+	 * splits run with more stages. */
 	int k_tiles = (t.K + BK - 1) / BK;
 	if (split >= 0) {
 		k_tiles = min(k_tiles, kt_begin + p.kt_per_split);
