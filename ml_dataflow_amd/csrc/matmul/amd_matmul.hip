@@ -91,7 +91,9 @@ static long tiles_of(long extent, long tile) { return (extent + tile - 1) / tile
  * alone), the persistent 256 x 256: 1.1-1.4.  So the cheapest tile is the one with the least (rounds of tiles over the
  * compute units) x (cost of a k-tile), small tiles while they still fit one round and larger ones behind that.  1408 x
  * 2048 x 256 takes 10 us on 64 x 64 tiles (29 on 128 x 128 with one k-tile in flight, which this replaced), 4096 x 4096 x
- * 512 31 us on 64 x 128 (55), 4096 x 4096 x 2048 66 us on pairs of 128 x 128 (92 on the persistent kernel). */
+ * 512 31 us on 64 x 128 (55), 4096 x 4096 x 2048 66 us on pairs of 128 x 128 (92 on the persistent kernel).  The rule has
+ * no term per tile and is applied at every K: how the tiles compare where K is so short that a tile's epilogue takes as
+ * long as its k-tiles (short groups of a ragged-K launch) has not been measured. */
 enum { TILE_64x32, TILE_64x64, TILE_64x128, TILE_128x128, TILE_128x128_PAIR, TILE_BIG, NUM_TILES };
 static const struct { int bm, bn, cost; } TILES[NUM_TILES] = {{64, 32, 21}, {64, 64, 25}, {64, 128, 36}, {128, 128, 58}, {128, 128, 50}, {256, 256, 130}};
 #define TILE_PAIR_COST_ALONE 62      /* of a k-tile of the pair's tile where it has the compute unit to itself, or its lines come from HBM */
