@@ -34,6 +34,8 @@ int amd_grouped_matmul(Dataflow_Handle * dataflow_handle, int stream_id, Op * op
  * as for dataflow_submit_matmul), with the fp32 partial sums of the split kept in a device array of the library itself
  * instead of a caller's workspace.  The call makes no allocation of any kind.  C is ignored when NULL or beta == 0.
  * Limit: a problem whose split needs more than 8 MiB of partial sums (splits * M * N * 4 bytes) is refused with -1.
+ * Operands whose rows are not 16-byte aligned, which the op copies to padded rows in the workspace, are copied to the
+ * same array where copies and partial sums fit; where they do not, the problem runs as the op runs it without a workspace.
  * Every call on a device shares that device's array: calls that overlap on one device (two streams, two host
  * threads) race on it.  Needs a handle on which dataflow_register_default_ops has run (that is where the array's
  * address on the handle's device is looked up). */

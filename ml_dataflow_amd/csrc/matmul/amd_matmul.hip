@@ -13,7 +13,7 @@
  * The kernels live in gemm_kernel.h (eight waves), gemm_w4_kernel.h (four waves) and gemm_typed_kernel.h (element
  * types beside all-bf16); this file decodes the op arguments, checks them on the host and picks a kernel: the
  * direct-to-LDS kernels when every operand is 16-byte aligned with a contiguous extent that is a multiple of 8
- * elements, the register-staged kernel otherwise; for large ragged-N launches without a C operand the choice between
+ * elements, or a workspace holds padded copies of those that are not (pad_operands), the register-staged kernel otherwise; for large ragged-N launches without a C operand the choice between
  * the eight-wave kernel and the four-wave 256 x 384 one is left to the device (launch_gemm).
  */
 #include <stdio.h>
@@ -121,8 +121,8 @@ static long grid_of(int which, int mode, const GemmParams & p) {
 	return tiles_of(p.M, TILES[which].bm) * ((long) p.N / TILES[which].bn + (p.N < p.num_groups ? p.N : p.num_groups));
 }
 
-static int choose_tile(int mode, const GemmParams & p, long cu_count) {
-	const bool big_ok = p.M >= 256 && (mode == MODE_RAGGED_N || p.N >= 256);
+static int choose_tile(int mode, const GemmParams & p, long cu_count, bool persistent_ok = true) {
+	const bool big_ok = persistent_ok && p.M >= 256 && (mode == MODE_RAGGED_N || p.N >= 256);
 	int best = TILE_64x32;
 	long best_cost = 0;
 	for (int which = 0; which < NUM_TILES; which++) {
@@ -539,11 +539,97 @@ static int launch_split_reduce(const GemmParams & p, hipStream_t stream) {
 	return check_launch();
 }
 
+/* ---- operands that the 16-byte loads cannot fetch (an odd number of experts: the rows of the router's gradient) ----
+ *
+ * The register-staged kernel fetches such an operand element by element, 5 us per k-tile of 128 x 128, unsplit along K: the
+ * router's weight gradient of 46398 tokens and 33 experts (1024 x 46398 x 33) took 3828 us, its input gradient
+ * 93.  A copy with its rows padded to a multiple of 8 elements (zeros) in the caller's workspace costs a pass over that
+ * operand (4-6 us here), and the copy then runs on the direct kernel, split along K where the matmul op splits.  A training step of
+ * that layer (dim 1024, top 8, expert dim 640) takes 5582 us instead of 9998, one of 1132 tokens and 59 experts 717 instead of
+ * 792.  Below PAD_MIN_STEPS rounds of staged tiles x k-tiles the staged kernel is done by the time a second launch starts. */
+#define PAD_MIN_STEPS 2
+
+__global__ void __launch_bounds__(256) pad_rows_kernel(const bf16_t * __restrict__ src, long long rows, int extent, int pitch, u32x4 * __restrict__ dst) {
+	const int chunks = pitch >> 3;                       /* 16-byte chunks of a padded row */
+	const long long total = rows * chunks;
+	const long long stride = (long long) gridDim.x * 256;
+	for (long long i = (long long) blockIdx.x * 256 + threadIdx.x; i < total; i += stride) {
+		const long long r = i / chunks;
+		const int c = (int) (i - r * chunks) * 8;
+		const bf16_t * s = src + r * extent + c;
+		uint32_t e[8];
+		#pragma unroll
+		for (int j = 0; j < 8; j++) {
+			e[j] = c + j < extent ? (uint32_t) s[j] : 0u;
+		}
+		dst[i] = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
+	}
+}
+
+/* Copies of the operands of `p` that need one, at the start of the workspace, which is advanced past them; `p` then
+ * describes the padded problem.  1: done, 0: does not apply or does not fit (`p` as it was), -1: error. */
+static int pad_operands(GemmParams & p, int transa, int transb, uint8_t *& workspace, uint64_t & workspace_bytes, long cu_count, hipStream_t stream) {
+	if (!workspace || (((uintptr_t) workspace) & 15) || p.K < 1
+		|| tiles_of(tiles_of(p.M, 128) * tiles_of(p.N, 128), cu_count) * tiles_of(p.K, BK) < PAD_MIN_STEPS) {
+		return 0;
+	}
+	const bool copy_a = !operand_direct_ok(p.A, !transa, p.M, p.K, 0), copy_b = !operand_direct_ok(p.B, transb != 0, p.N, p.K, 0);
+	const long pitch_a = round_up8(transa ? p.K : p.M), pitch_b = round_up8(transb ? p.N : p.K);
+	/* row lengths and K as ints, and what operand_direct_ok allows of a contiguous extent */
+	if (pitch_a > (transa ? 1L << 22 : 1L << 24) || pitch_b > (transb ? 1L << 24 : 1L << 22)) {
+		return 0;
+	}
+	const long rows_a = transa ? p.M : p.K, rows_b = transb ? p.K : p.N;
+	const uint64_t bytes_a = copy_a ? (((uint64_t) rows_a * (uint64_t) pitch_a * 2u) + 255) & ~255UL : 0;
+	const uint64_t bytes_b = copy_b ? (((uint64_t) rows_b * (uint64_t) pitch_b * 2u) + 255) & ~255UL : 0;
+	if (workspace_bytes < bytes_a || workspace_bytes - bytes_a < bytes_b) {
+		return 0;
+	}
+	for (int which = 0; which < 2; which++) {
+		if (!(which ? copy_b : copy_a)) {
+			continue;
+		}
+		const long rows = which ? rows_b : rows_a, pitch = which ? pitch_b : pitch_a;
+		const int extent = which ? (transb ? p.N : p.K) : (transa ? p.K : p.M);
+		const long blocks = tiles_of(rows * (pitch / 8), 256);
+		u32x4 * dst = (u32x4 *) (workspace + (which ? bytes_a : 0));
+		hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned int) (blocks < 16384 ? blocks : 16384)), dim3(256), 0, stream,
+						   which ? p.B : p.A, (long long) rows, extent, (int) pitch, dst);
+		if (check_launch()) {
+			return -1;
+		}
+		(which ? p.B : p.A) = (const bf16_t *) dst;
+	}
+	workspace += bytes_a + bytes_b;
+	workspace_bytes -= bytes_a + bytes_b;
+	if (copy_a && !transa) {
+		p.pitchA = (int) pitch_a;
+	}
+	if (copy_b && transb) {
+		p.pitchB = (int) pitch_b;
+	}
+	if ((copy_a && transa) || (copy_b && !transb)) {
+		p.k_rows = p.K;
+		p.K = (int) round_up8(p.K);
+	}
+	return 1;
+}
+
+/* a padded problem that is not split: the direct kernel on its cheapest tile */
+static int launch_padded(const GemmParams & p, int transa, int transb, long cu_count, hipStream_t stream) {
+	const int tile = choose_tile(MODE_SINGLE, p, cu_count, false);
+	const bool pk = !transa, qk = transb != 0;
+	if (!pk && !qk) { return launch_direct<false, false, MODE_SINGLE>(p, tile, stream); }
+	if (pk && !qk) { return launch_direct<true, false, MODE_SINGLE>(p, tile, stream); }
+	if (pk && qk) { return launch_direct<true, true, MODE_SINGLE>(p, tile, stream); }
+	return launch_direct<false, true, MODE_SINGLE>(p, tile, stream);
+}
+
 /* shared by amd_matmul and amd_matmul_no_alloc: checks, kernel choice, launch.  `workspace` (may be NULL) holds the fp32
  * partial sums of a split along K; `must_fit`: a split that the workspace cannot hold is an error instead of running
  * unsplit */
 static int run_matmul(Dataflow_Handle * dataflow_handle, int stream_id, GemmParams & p, int transa, int transb,
-					  float * workspace, uint64_t workspace_bytes, long cu_count, bool must_fit) {
+					  uint8_t * workspace, uint64_t workspace_bytes, long cu_count, bool must_fit) {
 	if (p.M < 0 || p.N < 0 || p.K < 0 || !p.D || ((p.M > 0 && p.N > 0 && p.K > 0) && (!p.A || !p.B))) {
 		fprintf(stderr, "Error: bad matmul arguments M=%d K=%d N=%d A=%p B=%p D=%p...\n", p.M, p.K, p.N, (void *) p.A, (void *) p.B, (void *) p.D);
 		return -1;
@@ -562,7 +648,12 @@ static int run_matmul(Dataflow_Handle * dataflow_handle, int stream_id, GemmPara
 	const bool direct = operand_direct_ok(p.A, !transa, p.M, p.K, 0) && operand_direct_ok(p.B, transb != 0, p.N, p.K, 0);
 	const long grid_big = tiles_of(p.M, 256) * tiles_of(p.N, 256);
 	const long grid_small = tiles_of(p.M, 128) * tiles_of(p.N, 128);
-	const int split = plan_split(p, direct, workspace, workspace_bytes, cu_count, must_fit);
+	const int padded = direct ? 0 : pad_operands(p, transa, transb, workspace, workspace_bytes, cu_count, stream);
+	if (padded < 0) {
+		return -1;
+	}
+	/* a padded problem whose split does not fit runs unsplit: it was never refused for that */
+	const int split = plan_split(p, direct || padded, (float *) workspace, workspace_bytes, cu_count, must_fit && !padded);
 	if (split < 0) {
 		return -1;
 	}
@@ -571,6 +662,9 @@ static int run_matmul(Dataflow_Handle * dataflow_handle, int stream_id, GemmPara
 			return -1;
 		}
 		return launch_split_reduce(p, stream);
+	}
+	if (padded) {
+		return launch_padded(p, transa, transb, cu_count, stream);
 	}
 	return launch_gemm<MODE_SINGLE>(p, transa, transb, direct, grid_big, grid_small, cu_count, stream);
 }
@@ -685,7 +779,7 @@ extern "C" int amd_matmul(Dataflow_Handle * dataflow_handle, int stream_id, Op *
 		return -1;
 	}
 	const uint64_t workspace_bytes = *((uint64_t *) a[17]);
-	float * workspace = (float *) *((uint64_t *) a[18]);
+	uint8_t * workspace = (uint8_t *) *((uint64_t *) a[18]);
 	return run_matmul(dataflow_handle, stream_id, p, transa, transb, workspace, workspace_bytes, extra_cu_count(op_extra), false);
 }
 
@@ -713,7 +807,7 @@ extern "C" int amd_matmul_no_alloc(Dataflow_Handle * dataflow_handle, int stream
 	p.alpha = alpha; p.beta = beta;
 	p.A = (const bf16_t *) A; p.B = (const bf16_t *) B; p.C = (beta == 0.0f) ? NULL : (const bf16_t *) C; p.D = (bf16_t *) D;
 	Hip_Device_Info * info = (Hip_Device_Info *) dataflow_handle->device_info;
-	return run_matmul(dataflow_handle, stream_id, p, to_trans_a, to_trans_b, (float *) scratch_of_device[dev], AMD_MATMUL_SCRATCH_BYTES,
+	return run_matmul(dataflow_handle, stream_id, p, to_trans_a, to_trans_b, (uint8_t *) scratch_of_device[dev], AMD_MATMUL_SCRATCH_BYTES,
 					  info ? info->cu_count : 256, true);
 }
 

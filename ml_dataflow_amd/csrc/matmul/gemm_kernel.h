@@ -67,6 +67,11 @@ struct GemmParams {
 	float * partial;
 	int split_k;                   /* 0 or 1: off */
 	int kt_per_split;              /* a multiple of 4, as the host plans it; the kernel takes any */
+	/* Operands copied to padded rows (single problems on the direct kernel only; 0: not padded): elements from one k-row
+	 * to the next of a k-major operand, and the k-rows a k-major operand has where K was rounded up for a k-contiguous one
+	 * (those past them read as zero, like the padding they are multiplied with) */
+	int pitchA, pitchB;
+	int k_rows;
 	/* Ragged-N launches without C that several tilings can take are launched on each candidate; every work-group counts
 	 * the tiles of the tilings from the device prefix sum (ragged_n_choice) and the kernels that lose return at once.
 	 * One bit per tiling, RAGGED_N_288 always among them; 0: run */
@@ -859,8 +864,9 @@ struct TileLoader {
 	uint32_t row_bytes;      /* uniform, k-major GATHER: bytes of one source row */
 	uint32_t kmap_rows;      /* uniform, k-major GATHER: rows of the source */
 
-	/* `operand`: first element of the operand (of this group); row0: first of the panel's rows; row0 < rows_total */
-	__device__ __forceinline__ void init(const bf16_t * operand, int row0, int rows_total, int K) {
+	/* `operand`: first element of the operand (of this group); row0: first of the panel's rows; row0 < rows_total; pitch:
+	 * elements from one k-row of a k-major operand to the next, at least rows_total */
+	__device__ __forceinline__ void init(const bf16_t * operand, int row0, int rows_total, int K, int pitch) {
 		const int tid = threadIdx.x % THREADS;
 		if (!KMAJOR) {
 			const int row = tid >> 3;
@@ -884,11 +890,15 @@ struct TileLoader {
 			lane_ok_odd = row0 + (mc_odd << 3) < rows_total;
 			odd_delta = (uint32_t) ((mc_odd - mc) * 16);
 			base = (uint64_t) (operand + row0);
-			extent = (uint64_t) K * (uint64_t) rows_total * 2u - (uint64_t) row0 * 2u;
-			lane_voff = ((uint32_t) k * (uint32_t) rows_total + (uint32_t) (mc << 3)) * 2u;
-			step = (uint32_t) (THREADS / CPR) * (uint32_t) rows_total * 2u;
-			ktile = (uint64_t) BK * (uint64_t) rows_total * 2u;
+			extent = (uint64_t) K * (uint64_t) pitch * 2u - (uint64_t) row0 * 2u;
+			lane_voff = ((uint32_t) k * (uint32_t) pitch + (uint32_t) (mc << 3)) * 2u;
+			step = (uint32_t) (THREADS / CPR) * (uint32_t) pitch * 2u;
+			ktile = (uint64_t) BK * (uint64_t) pitch * 2u;
 		}
+	}
+
+	__device__ __forceinline__ void init(const bf16_t * operand, int row0, int rows_total, int K) {
+		init(operand, row0, rows_total, K, rows_total);
 	}
 
 	/* GATHER: `source` has source_rows rows of K elements (below 4 GiB in all); map[r] is the source row of the panel's
@@ -1073,15 +1083,16 @@ gemm_bf16_direct_kernel(GemmParams p) {
 
 	TileLoader<P_KMAJOR, BM, THREADS, GATHER == GATHER_P_KROWS> ldP;
 	TileLoader<Q_KMAJOR, BN, THREADS, GATHER == GATHER_Q_ROWS> ldQ;
+	const int k_rows = MODE == MODE_SINGLE && p.k_rows ? p.k_rows : t.K;
 	if (GATHER == GATHER_P_KROWS) {
 		ldP.init_gather_k(t.P, t.Pmap, t.m0, t.M, t.K, p.gather_rows);
 	} else {
-		ldP.init(t.P, t.m0, t.M, t.K);
+		ldP.init(t.P, t.m0, t.M, P_KMAJOR ? k_rows : t.K, MODE == MODE_SINGLE && p.pitchA ? p.pitchA : t.M);
 	}
 	if (GATHER == GATHER_Q_ROWS) {
 		ldQ.init_gather(t.Q, t.Qmap, t.n0, t.N, t.K, p.gather_rows);
 	} else {
-		ldQ.init(t.Q, t.n0, t.N, t.K);
+		ldQ.init(t.Q, t.n0, t.N, Q_KMAJOR ? k_rows : t.K, MODE == MODE_SINGLE && p.pitchB ? p.pitchB : t.N);
 	}
 
 	/* the descriptors end with the operand of this problem: anything outside reads as zero */

@@ -550,6 +550,51 @@ def test_matmul_unaligned_shapes_take_the_scalar_path(backend, oracle, M, K, N):
         check_matmul(got, O.matmul(oracle, transa, transb, M, K, N, A, Bm), K)
 
 
+@pytest.mark.parametrize("transa,transb,M,K,N", [
+    (0, 1, 1024, 3000, 33),      # router weight gradient, odd number of experts: B's rows padded, K split
+    (0, 0, 512, 33, 2000),       # router input gradient: B's rows and with them K padded, A's k-rows end before the padded K
+    (0, 0, 203, 77, 1500),       # A's rows (along M) and B's (along K)
+    (0, 1, 203, 1500, 77),       # both k-major and odd
+    (1, 0, 131, 1001, 300),      # both k-contiguous and odd
+    (1, 1, 65, 1031, 193),
+    (0, 1, 8, 129, 1),           # one padded row of 8
+    (1, 0, 1030, 7, 2050)])      # K shorter than the loads
+def test_matmul_unaligned_operands_padded_through_the_workspace(backend, oracle, transa, transb, M, K, N):
+    """Operands whose rows are not a multiple of 8 elements, with a workspace that holds padded copies: the bar of the other
+    matmuls, with and without C, and at a base that is not 16-byte aligned.  A workspace too small for the copies gives the
+    bits of the run without one.  Products of the padding are 0 * 0, so an infinity stays in its own rows."""
+    print("case padded ta=%d tb=%d M=%d K=%d N=%d" % (transa, transb, M, K, N), flush=True)
+    rng = np.random.default_rng(M + K + N)
+    A = normal_bf16(rng, (M, K) if transa else (K, M))
+    Bm = normal_bf16(rng, (K, N) if transb else (N, K), 0.05)
+    Cin = normal_bf16(rng, (N, M))
+    big = 64 * M * N * 4 + 4 * (M + N + 64) * (K + 64)
+    want = O.matmul(oracle, transa, transb, M, K, N, A, Bm)
+    check_matmul(run_gpu_matmul(backend, transa, transb, M, K, N, A, Bm, 1.0, 0.0, None, big), want, K)
+    check_matmul(run_gpu_matmul(backend, transa, transb, M, K, N, A, Bm, 0.5, 1.0, Cin, big),
+                 O.matmul(oracle, transa, transb, M, K, N, A, Bm, alpha=0.5, beta=1.0, Cin=Cin), K)
+    staged = run_gpu_matmul(backend, transa, transb, M, K, N, A, Bm, 1.0, 0.0, None)
+    assert (run_gpu_matmul(backend, transa, transb, M, K, N, A, Bm, 1.0, 0.0, None, 64) == staged).all()
+    A.reshape(-1)[-1] = 0x7F80                            # the last element: m = M - 1, k = K - 1
+    got = run_gpu_matmul(backend, transa, transb, M, K, N, A, Bm, 1.0, 0.0, None, big)
+    finite = (got & 0x7F80) != 0x7F80
+    assert finite[:, :M - 1].all() and not finite[:, M - 1].any()
+
+
+def test_matmul_misaligned_bases_padded_through_the_workspace(backend, oracle):
+    be, rng = backend, np.random.default_rng(5)
+    M, K, N = 200, 264, 328
+    A, Bm = normal_bf16(rng, (M, K)), normal_bf16(rng, (N, K), 0.05)
+    d_A, d_B = be.upload(np.concatenate([[np.uint16(0)], A.reshape(-1)]).astype(np.uint16)), be.upload(np.concatenate([np.zeros(3, np.uint16), Bm.reshape(-1)]).astype(np.uint16))
+    d_D, d_ws = be.alloc(M * N * 2), be.alloc(8 << 20)
+    assert be.lib.dataflow_submit_matmul(be.hp, CS, BF, BF, B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 1, 0, M, K, N, 1.0, 0.0,
+                                         d_A.ptr + 2, d_B.ptr + 6, None, d_D.ptr, 8 << 20, d_ws.ptr) == 0
+    be.sync(CS)
+    check_matmul(be.read(d_D.ptr, (N, M), np.uint16), O.matmul(oracle, 1, 0, M, K, N, A, Bm), K)
+    for buf in (d_A, d_B, d_D, d_ws):
+        buf.free()
+
+
 def test_matmul_special_cases(backend):
     be = backend
     rng = np.random.default_rng(1)
