@@ -124,6 +124,79 @@ __device__ __forceinline__ long xcd_remap(long b, long total) {
 	return (b & 7) * chunk + (b >> 3);
 }
 
+/* Inclusive sum over the lanes of a wave, and the value of the lane below (lane 0: `first`), in cross-lane moves of the
+ * vector unit.  Every ragged launch starts with such a scan of the group sizes, a persistent work-group does one per tile
+ * with the matrix pipes idle, and a shuffle through the LDS costs about a hundred clocks where a move costs eight (with
+ * 32-bit divisions by the tiles of a row: a forward of 256 tokens 30.6 -> 28.9 us, a training step of 8192 tokens, 64
+ * experts, dim 4096 5124 -> 5063). */
+__device__ __forceinline__ int wave_inclusive_sum(int v) {
+	v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);      /* row_shr:1, 2, 4, 8 */
+	v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+	v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+	v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+	v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);      /* row_bcast:15, :31 */
+	v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+	return v;
+}
+__device__ __forceinline__ int wave_lane_below(int v, int first) { return __builtin_amdgcn_update_dpp(first, v, 0x138, 0xF, 0xF, false); }
+
+/* ragged N: groups base .. base + 63, one per lane: end and start of the group's rows, tiles of BN rows in the groups up to
+ * and including it and in it alone; rows_before: rows of the groups in front of `base` */
+struct GroupScan { int end, start, incl, mine; };
+template <int BN>
+__device__ __forceinline__ GroupScan scan_groups(const GemmParams & p, int base, int lane, int rows_before) {
+	const int g = base + lane;
+	GroupScan s;
+	s.end = g < p.num_groups ? p.cumsum[g] : 0;
+	s.start = wave_lane_below(s.end, rows_before);
+	s.mine = g < p.num_groups ? (s.end - s.start + BN - 1) / BN : 0;
+	s.incl = wave_inclusive_sum(s.mine);
+	return s;
+}
+
+/* ragged N: the group of n-tile `nt` of the launch, its rows and which of its n-tiles that is */
+struct FoundGroup { int g, start, rows, nt; };
+__device__ __forceinline__ bool find_in_scan(const GemmParams & p, const GroupScan & s, int base, int lane, int tiles_before, int nt, FoundGroup & f) {
+	const uint64_t past = __ballot(base + lane < p.num_groups && tiles_before + s.incl > nt);
+	if (!past) {
+		return false;
+	}
+	const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long) past) - 1);
+	f.g = base + src;
+	f.start = __builtin_amdgcn_readlane(s.start, src);
+	f.rows = __builtin_amdgcn_readlane(s.end, src) - f.start;
+	f.nt = nt - (tiles_before + __builtin_amdgcn_readlane(s.incl, src) - __builtin_amdgcn_readlane(s.mine, src));
+	return true;
+}
+template <int BN>
+__device__ __forceinline__ FoundGroup find_group(const GemmParams & p, int lane, int nt) {
+	FoundGroup f = {0, 0, 0, 0};
+	int tiles_before = 0, rows_before = 0;
+	for (int base = 0; base < p.num_groups; base += 64) {
+		const GroupScan s = scan_groups<BN>(p, base, lane, rows_before);
+		if (find_in_scan(p, s, base, lane, tiles_before, nt, f)) {
+			break;
+		}
+		tiles_before += __builtin_amdgcn_readlane(s.incl, 63);
+		rows_before = __builtin_amdgcn_readlane(s.end, min(63, p.num_groups - base - 1));
+	}
+	return f;
+}
+/* the same in scalar registers (the compiler does not see that a value carried round a loop is the same in every lane) */
+__device__ __forceinline__ FoundGroup uniform_group(const FoundGroup & f) {
+	return FoundGroup{__builtin_amdgcn_readfirstlane(f.g), __builtin_amdgcn_readfirstlane(f.start), __builtin_amdgcn_readfirstlane(f.rows), __builtin_amdgcn_readfirstlane(f.nt)};
+}
+template <int BN>
+__device__ __forceinline__ int count_n_tiles(const GemmParams & p, int lane) {
+	int tiles = 0, rows_before = 0;
+	for (int base = 0; base < p.num_groups; base += 64) {
+		const GroupScan s = scan_groups<BN>(p, base, lane, rows_before);
+		tiles += __builtin_amdgcn_readlane(s.incl, 63);
+		rows_before = __builtin_amdgcn_readlane(s.end, min(63, p.num_groups - base - 1));
+	}
+	return __builtin_amdgcn_readfirstlane(tiles);
+}
+
 /* number of tiles of the launch (ragged-N: read from the device prefix sum) */
 template <int BM, int BN, int MODE>
 __device__ __forceinline__ long count_tiles(const GemmParams & p) {
@@ -134,28 +207,7 @@ __device__ __forceinline__ long count_tiles(const GemmParams & p) {
 	if (MODE == MODE_RAGGED_K) {
 		return (long) tiles_m * ((p.N + BN - 1) / BN) * p.num_groups;
 	}
-	const int lane = threadIdx.x & 63;
-	long total_n_tiles = 0;
-	int carry_rows = 0;
-	for (int base = 0; base < p.num_groups; base += 64) {
-		const int g = base + lane;
-		const int c = (g < p.num_groups) ? p.cumsum[g] : 0;
-		int prev = __shfl_up(c, 1, 64);
-		if (lane == 0) {
-			prev = carry_rows;
-		}
-		int tiles = (g < p.num_groups) ? (c - prev + BN - 1) / BN : 0;
-		#pragma unroll
-		for (int off = 1; off < 64; off <<= 1) {
-			int up = __shfl_up(tiles, off, 64);
-			if (lane >= off) {
-				tiles += up;
-			}
-		}
-		total_n_tiles += __shfl(tiles, 63, 64);
-		carry_rows = __shfl(c, min(63, p.num_groups - base - 1), 64);
-	}
-	return (long) __builtin_amdgcn_readfirstlane((int) total_n_tiles) * tiles_m;
+	return (long) count_n_tiles<BN>(p, threadIdx.x & 63) * tiles_m;
 }
 
 /* Which tiling of the token rows is cheapest for this launch.  A launch takes (rounds of tiles over the work-groups) x
@@ -194,18 +246,15 @@ __device__ __forceinline__ int ragged_n_choice(const GemmParams & p) {
 			tiles[i] += (rows + ragged_n_rows(i) - 1) / ragged_n_rows(i);
 		}
 	}
-	const long groups = gridDim.x;
-	const long tiles_m = (p.M + 255) / 256;
+	const unsigned int groups = gridDim.x;
+	const unsigned int tiles_m = (unsigned int) (p.M + 255) / 256;
 	const long k_tiles = (p.K + BK - 1) / BK;
 	int best = RAGGED_N_288;
 	long least = 0;
 	#pragma unroll
 	for (int i = 0; i < RAGGED_N_TILINGS; i++) {
-		#pragma unroll
-		for (int off = 32; off > 0; off >>= 1) {
-			tiles[i] += __shfl_xor(tiles[i], off, 64);
-		}
-		const long cost = ragged_n_cost(i, (tiles[i] * tiles_m + groups - 1) / groups, k_tiles);
+		const unsigned int all = (unsigned int) __builtin_amdgcn_readlane(wave_inclusive_sum(tiles[i]), 63) * tiles_m;
+		const long cost = ragged_n_cost(i, (all + groups - 1) / groups, k_tiles);
 		if (i == RAGGED_N_288 || (((p.candidates >> i) & 1) && cost < least)) {
 			best = i;
 			least = cost;
@@ -255,62 +304,27 @@ __device__ __forceinline__ bool resolve_tile_id(const GemmParams & p, long id, T
 		return true;
 	}
 	if (MODE == MODE_RAGGED_N) {
-		const int lane = threadIdx.x & 63;
-		const int nt = (int) (id / tiles_m);                /* finds the group: a group owns tiles_m * (its n-tiles) consecutive ids */
-		int found_g = 0, found_prev = 0, found_rows = 0, found_nt = 0;
-		int tiles_before = 0;
-		int carry_rows = 0;
-		for (int base = 0; base < p.num_groups; base += 64) {
-			const int g = base + lane;
-			const int c = (g < p.num_groups) ? p.cumsum[g] : 0;
-			int prev = __shfl_up(c, 1, 64);
-			if (lane == 0) {
-				prev = carry_rows;
-			}
-			const int mine = (g < p.num_groups) ? (c - prev + BN - 1) / BN : 0;
-			int incl = mine;
-			#pragma unroll
-			for (int off = 1; off < 64; off <<= 1) {
-				int up = __shfl_up(incl, off, 64);
-				if (lane >= off) {
-					incl += up;
-				}
-			}
-			const uint64_t past = __ballot((g < p.num_groups) && (tiles_before + incl > nt));
-			if (past) {
-				const int src = __ffsll((long long) past) - 1;
-				found_g = base + src;
-				found_prev = __shfl(prev, src, 64);
-				found_rows = __shfl(c - prev, src, 64);
-				found_nt = nt - (tiles_before + __shfl(incl - mine, src, 64));
-				break;
-			}
-			tiles_before += __shfl(incl, 63, 64);
-			carry_rows = __shfl(c, min(63, p.num_groups - base - 1), 64);
-		}
-		found_g = __builtin_amdgcn_readfirstlane(found_g);
-		found_prev = __builtin_amdgcn_readfirstlane(found_prev);
-		found_rows = __builtin_amdgcn_readfirstlane(found_rows);
-		found_nt = __builtin_amdgcn_readfirstlane(found_nt);
-		/* found_nt counted whole rows of tiles_m ids inside the group; redo the split with the blocked order */
+		/* finds the group: a group owns tiles_m * (its n-tiles) consecutive ids */
+		const int nt = (int) ((unsigned int) id / (unsigned int) tiles_m);
+		const FoundGroup f = uniform_group(find_group<BN>(p, threadIdx.x & 63, nt));
+		/* f.nt counts whole rows of tiles_m ids inside the group; redo the split with the blocked order */
 		int tm, tn;
-		tile_in_problem(found_nt * tiles_m + (int) (id % tiles_m), tiles_m, (found_rows + BN - 1) / BN, tm, tn);
-		found_nt = tn;
-		t.P = p.A + (long long) found_g * p.strideA;
-		t.Q = p.gather ? p.B : p.B + (long long) found_prev * p.K;
-		t.Qmap = p.gather ? p.gather + found_prev : nullptr;
+		tile_in_problem(f.nt * tiles_m + ((int) id - nt * tiles_m), tiles_m, (f.rows + BN - 1) / BN, tm, tn);
+		t.P = p.A + (long long) f.g * p.strideA;
+		t.Q = p.gather ? p.B : p.B + (long long) f.start * p.K;
+		t.Qmap = p.gather ? p.gather + f.start : nullptr;
 		t.Pmap = nullptr;
-		t.C = p.C ? p.C + (long long) found_prev * p.M : nullptr;
-		t.D = p.D + (long long) found_prev * p.M;
-		t.M = p.M; t.N = found_rows; t.K = p.K;
+		t.C = p.C ? p.C + (long long) f.start * p.M : nullptr;
+		t.D = p.D + (long long) f.start * p.M;
+		t.M = p.M; t.N = f.rows; t.K = p.K;
 		t.m0 = tm * BM;
-		t.n0 = found_nt * BN;
+		t.n0 = tn * BN;
 		return true;
 	}
 	const int tiles_n = (p.N + BN - 1) / BN;
-	const long per_group = (long) tiles_m * tiles_n;
-	const int g = (int) (id / per_group);
-	const long r = id % per_group;
+	const unsigned int per_group = (unsigned int) tiles_m * (unsigned int) tiles_n;
+	const int g = (int) ((unsigned int) id / per_group);
+	const unsigned int r = (unsigned int) id - (unsigned int) g * per_group;
 	const int hi = p.cumsum[g];
 	const int lo = g ? p.cumsum[g - 1] : 0;
 	if (hi - lo <= 0) {
@@ -342,87 +356,41 @@ __device__ __forceinline__ bool resolve_tile(const GemmParams & p, Tile & t) {
 		}
 		t.P = p.A; t.Q = p.B; t.Qmap = nullptr; t.Pmap = nullptr; t.C = p.C; t.D = p.D;
 		t.M = p.M; t.N = p.N; t.K = p.K;
-		t.m0 = (int) (id % tiles_m) * BM;
-		t.n0 = (int) (id / tiles_m) * BN;
+		const int tn = (int) ((unsigned int) id / (unsigned int) tiles_m);
+		t.m0 = ((int) id - tn * tiles_m) * BM;
+		t.n0 = tn * BN;
 		return true;
 	}
 	if (MODE == MODE_RAGGED_N) {
 		/* Tile order: group, then n-tile, then m-tile (fastest).  The per-group tile counts come from the device-side
-		 * prefix sum; every wave scans them on its own, 64 groups per step with one coalesced load and shuffles,
-		 * instead of walking the array with dependent scalar loads. */
+		 * prefix sum; every wave scans them on its own, 64 groups per step, one per lane; up to 64 groups the total and the
+		 * group of this work-group's tile come from one scan. */
 		const int lane = threadIdx.x & 63;
-		long total_n_tiles = 0;
-		int carry_rows = 0;
-		for (int base = 0; base < p.num_groups; base += 64) {
-			const int g = base + lane;
-			const int c = (g < p.num_groups) ? p.cumsum[g] : 0;
-			int prev = __shfl_up(c, 1, 64);
-			if (lane == 0) {
-				prev = carry_rows;
-			}
-			int tiles = (g < p.num_groups) ? (c - prev + BN - 1) / BN : 0;
-			#pragma unroll
-			for (int off = 1; off < 64; off <<= 1) {
-				int up = __shfl_up(tiles, off, 64);
-				if (lane >= off) {
-					tiles += up;
-				}
-			}
-			total_n_tiles += __shfl(tiles, 63, 64);
-			carry_rows = __shfl(c, min(63, p.num_groups - base - 1), 64);
-		}
-		total_n_tiles = __builtin_amdgcn_readfirstlane((int) total_n_tiles);
-		const long total = total_n_tiles * tiles_m;
+		const GroupScan first = scan_groups<BN>(p, 0, lane, 0);
+		const bool one_scan = p.num_groups <= 64;
+		const unsigned int total = (unsigned int) (one_scan ? __builtin_amdgcn_readlane(first.incl, 63) : count_n_tiles<BN>(p, lane)) * (unsigned int) tiles_m;
 		const long id = xcd_remap(blockIdx.x, total);
 		if (id >= total) {
 			return false;
 		}
-		const int nt = (int) (id / tiles_m);
-		const int tm = (int) (id % tiles_m);
-		int found_g = 0, found_prev = 0, found_rows = 0, found_nt = 0;
-		int tiles_before = 0;
-		carry_rows = 0;
-		for (int base = 0; base < p.num_groups; base += 64) {
-			const int g = base + lane;
-			const int c = (g < p.num_groups) ? p.cumsum[g] : 0;
-			int prev = __shfl_up(c, 1, 64);
-			if (lane == 0) {
-				prev = carry_rows;
-			}
-			const int mine = (g < p.num_groups) ? (c - prev + BN - 1) / BN : 0;
-			int incl = mine;
-			#pragma unroll
-			for (int off = 1; off < 64; off <<= 1) {
-				int up = __shfl_up(incl, off, 64);
-				if (lane >= off) {
-					incl += up;
-				}
-			}
-			const uint64_t past = __ballot((g < p.num_groups) && (tiles_before + incl > nt));
-			if (past) {
-				const int src = __ffsll((long long) past) - 1;
-				found_g = base + src;
-				found_prev = __shfl(prev, src, 64);
-				found_rows = __shfl(c - prev, src, 64);
-				found_nt = nt - (tiles_before + __shfl(incl - mine, src, 64));
-				break;
-			}
-			tiles_before += __shfl(incl, 63, 64);
-			carry_rows = __shfl(c, min(63, p.num_groups - base - 1), 64);
+		const int nt = (int) ((unsigned int) id / (unsigned int) tiles_m);
+		const int tm = (int) id - nt * tiles_m;
+		FoundGroup f = {0, 0, 0, 0};
+		if (one_scan) {
+			find_in_scan(p, first, 0, lane, 0, nt, f);
+		} else {
+			f = find_group<BN>(p, lane, nt);
 		}
-		found_g = __builtin_amdgcn_readfirstlane(found_g);
-		found_prev = __builtin_amdgcn_readfirstlane(found_prev);
-		found_rows = __builtin_amdgcn_readfirstlane(found_rows);
-		found_nt = __builtin_amdgcn_readfirstlane(found_nt);
-		t.P = p.A + (long long) found_g * p.strideA;
-		t.Q = p.gather ? p.B : p.B + (long long) found_prev * p.K;
-		t.Qmap = p.gather ? p.gather + found_prev : nullptr;
+		f = uniform_group(f);
+		t.P = p.A + (long long) f.g * p.strideA;
+		t.Q = p.gather ? p.B : p.B + (long long) f.start * p.K;
+		t.Qmap = p.gather ? p.gather + f.start : nullptr;
 		t.Pmap = nullptr;
-		t.C = p.C ? p.C + (long long) found_prev * p.M : nullptr;
-		t.D = p.D + (long long) found_prev * p.M;
-		t.M = p.M; t.N = found_rows; t.K = p.K;
+		t.C = p.C ? p.C + (long long) f.start * p.M : nullptr;
+		t.D = p.D + (long long) f.start * p.M;
+		t.M = p.M; t.N = f.rows; t.K = p.K;
 		t.m0 = tm * BM;
-		t.n0 = found_nt * BN;
+		t.n0 = f.nt * BN;
 		return true;
 	}
 	/* MODE_RAGGED_K: tile order: group, n-tile, m-tile */
@@ -433,8 +401,8 @@ __device__ __forceinline__ bool resolve_tile(const GemmParams & p, Tile & t) {
 	if (id >= total) {
 		return false;
 	}
-	int g = (int) (id / per_group);
-	long r = id % per_group;
+	int g = (int) ((unsigned int) id / (unsigned int) per_group);
+	unsigned int r = (unsigned int) id - (unsigned int) g * (unsigned int) per_group;
 	int hi = p.cumsum[g];
 	int lo = g ? p.cumsum[g - 1] : 0;
 	if (hi - lo <= 0) {
@@ -447,8 +415,9 @@ __device__ __forceinline__ bool resolve_tile(const GemmParams & p, Tile & t) {
 	t.C = p.C ? p.C + (long long) g * p.strideD : nullptr;
 	t.D = p.D + (long long) g * p.strideD;
 	t.M = p.M; t.N = p.N; t.K = hi - lo;
-	t.m0 = (int) (r % tiles_m) * BM;
-	t.n0 = (int) (r / tiles_m) * BN;
+	const int tn = (int) (r / (unsigned int) tiles_m);
+	t.m0 = ((int) r - tn * tiles_m) * BM;
+	t.n0 = tn * BN;
 	return true;
 }
 
@@ -1046,7 +1015,7 @@ gemm_bf16_direct_kernel(GemmParams p) {
 	int kt_begin = 0;
 	int split = -1;
 	if (MODE == MODE_SINGLE && p.split_k > 1) {
-		const long tiles = (long) ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+		const unsigned int tiles = (unsigned int) ((p.M + BM - 1) / BM) * (unsigned int) ((p.N + BN - 1) / BN);
 		split = (int) (blockIdx.x / tiles);
 		if (split >= p.split_k || !resolve_tile_id<BM, BN, MODE>(p, blockIdx.x - split * tiles, t)) {
 			return;

@@ -59,3 +59,40 @@ def test_tilings_bit_identical(backend, M, K, name, transa, gathered):
     assert not bad.any(), "%d of %d elements differ, first at %s" % (int(bad.sum()), bad.size, np.argwhere(bad)[:4].tolist())
     for d in (d_W, d_X, d_cum, d_map):
         d.free()
+
+
+@pytest.mark.parametrize("kernel,M,K,rows", [(AUTO, 72, 64, 2000), (EIGHT, 256, 64, 33400), (384, 256, 128, 50000)])
+@pytest.mark.parametrize("G", [1, 2, 63, 64, 65, 127, 128, 129, 200])
+def test_group_of_every_row_at_the_edges_of_the_scan(backend, G, kernel, M, K, rows):
+    """The group of a tile is found by a scan over 64 groups at a time: group counts on both sides of one, two and three
+    steps, empty groups at the lanes where a step begins and ends.  The operands are whole numbers whose sums bf16 holds
+    exactly (at most 256), so the result is exact."""
+    print("case scan G=%d kernel=%d M=%d K=%d" % (G, kernel, M, K), flush=True)
+    be = backend
+    lib = C.CDLL(os.path.join(os.path.dirname(B.__file__), "lib", "libamd_matmul.so"))
+    lib.amd_matmul_select_kernel.argtypes = [C.c_int]
+    rng = np.random.default_rng(G + M)
+    share = rng.random(G) + 0.1
+    for g in (0, 15, 16, 31, 32, 62, 63, 64, 126, 127, 128, 191):
+        if g < G - 1:
+            share[g] = 0.0
+    counts = np.floor(share / share.sum() * rows).astype(np.int64)
+    counts[-1] += rows - counts.sum()
+    W = rng.integers(-2, 3, size=(G, M, K)).astype(np.float32)
+    X = rng.integers(-2, 3, size=(rows, K)).astype(np.float32)
+    X[:, 256 // 4:] = 0.0                                              # |sum| <= 64 products of at most 4
+    as_bf16 = lambda a: (a.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    want, row = np.empty((rows, M), dtype=np.float32), 0
+    for g in range(G):
+        want[row:row + counts[g]] = X[row:row + counts[g]] @ W[g].T
+        row += int(counts[g])
+    d_W, d_X, d_cum, d_D = be.upload(as_bf16(W)), be.upload(as_bf16(X)), be.upload(np.cumsum(counts).astype(np.int32)), be.alloc(rows * M * 2)
+    assert lib.amd_matmul_select_kernel(kernel) == 0
+    ret = be.lib.dataflow_submit_amd_grouped_matmul(be.hp, CS, BF, BF, B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 1, 0, B.AMD_GROUPED_RAGGED_N, M, K, rows, G,
+                                                    d_cum.ptr, 1.0, 0.0, d_W.ptr, M * K * 2, d_X.ptr, None, d_D.ptr, 0)
+    assert lib.amd_matmul_select_kernel(AUTO) == 0
+    assert ret == 0
+    be.sync(CS)
+    assert (be.read(d_D.ptr, (rows, M), np.uint16) == as_bf16(want)).all()
+    for d in (d_W, d_X, d_cum, d_D):
+        d.free()
