@@ -224,6 +224,31 @@ FUSED_GEMM_KERNEL_OF_CLASS = {
 }
 
 
+def ragged_n_tile_rows(M, K, rows, groups, work_groups=256):
+    """Token rows per tile of a ragged-N launch without C: ragged_n_tiling (csrc/matmul/amd_matmul.hip), restated.  The
+    cheapest tiling for the group sizes that an even router gives."""
+    mean, kt = rows / groups, -(-K // 64)
+    sizes = [round(mean + sign * q * mean ** 0.5) for q in (0.104, 0.319, 0.549, 0.812, 1.150, 1.732) for sign in (1.0, -1.0)]
+
+    def rounds(tile_rows):
+        tiles = [-(-max(size, 0) // tile_rows) for size in sizes]
+        average = sum(tiles) / 12.0
+        spread = (max(sum(t * t for t in tiles) / 12.0 - average ** 2, 0.0) * groups) ** 0.5
+        return sum(weight * -(-(-(-M // 256) * round(average * groups + 0.5 * side * spread)) // work_groups)
+                   for side, weight in ((-1, 0.25), (0, 0.5), (1, 0.25)))
+
+    streamed = groups * M * K * 2.0 / 200
+    best, cost = 288, rounds(288) * 544 * 100 * kt
+    if K % 128 == 0 and M % 8 == 0 and rounds(384) * 640 * (103 * kt + 160) < cost:
+        best, cost = 384, rounds(384) * (256 + 384) * (103 * kt + 160)
+    cost = max(cost, streamed)
+    for tile_rows in (224, 192):
+        finer = max(rounds(tile_rows) * (256 + tile_rows) * 107 * kt, streamed)
+        if finer < cost:
+            best, cost = tile_rows, finer
+    return best
+
+
 def norm_kernels_with_events(be, T, D, d_X, d_dY, d_dX, ev, stream, backward):
     """The RMS norm that feeds the layer and its backward passes (the calls of dataflow_transformer.c:2567, 3726, 3749),
     each between an event pair; returns [(kernel class, ms)].  rms_norm_bwd_w covers both of its kernels."""
@@ -404,8 +429,7 @@ def sustained_gemm(args):
 def tiling_sweep(args):
     """amd_grouped_matmul (ragged N, no C operand, random bf16 operands) per case on kernel 8, kernel 384 and the default
     choice: three rounds of --steps launches each (8 unless given), alternating, HIP events around each round, the fastest
-    round per kernel.  `rule` is what ragged_n_choice (gemm_kernel.h) picks between 288 and 384 rows from the group sizes,
-    restated here."""
+    round per kernel.  `rule` is what the tile costs of gemm_kernel.h say between 288 and 384 rows for these group sizes."""
     from ml_dataflow_amd import Backend, binding as B
     be = Backend(0)
     ev, stream = HipEvents(), be.stream(1)
@@ -786,23 +810,13 @@ def main():
         name = _W4 if args.gemm_kernel == 4 else _W4D
         four = {"gemm_up13": name % "false, 1, 1", "gemm_tn": name % "false, 1, 0", "gemm_nn": name % "true, 1, 0", "gemm_dx13": name % "true, 1, 0"}
         if args.gemm_kernel == 0:
-            # the library's rule (ragged_n_choice in gemm_kernel.h), from the same group sizes: which launches ran on 256 x 384 tiles
+            # the library's rule: which launches ran on tiles of 384, 224 or 192 token rows
             rows_m = {"gemm_up13": 2 * H, "gemm_tn": D, "gemm_nn": H, "gemm_dx13": D}
             k_of = {"gemm_up13": D, "gemm_tn": H, "gemm_nn": D, "gemm_dx13": 2 * H}
             for cls in list(four):
-                tiles_m = -(-rows_m[cls] // 256)
-                narrow = tiles_m * int(sum(-(-int(c) // 288) for c in counts))
-                wide = tiles_m * int(sum(-(-int(c) // 384) for c in counts))
-                groups = max(8, min(256, (tiles_m * (T * K // 192 + E) + 7) // 8 * 8))
-                even = T * K // E                          # the host's first look: all groups the same size
-                even_narrow, even_wide = tiles_m * E * -(-max(even, 1) // 288), tiles_m * E * -(-max(even, 1) // 384)
-                kt = -(-k_of[cls] // 64)
-                wide_cost, narrow_cost = 640 * (103 * kt + 160), 544 * 100 * kt
-                takes_wide = k_of[cls] % 128 == 0 and rows_m[cls] % 8 == 0 and \
-                    -(-even_wide // 256) * wide_cost < -(-even_narrow // 256) * narrow_cost and \
-                    -(-wide // groups) * wide_cost < -(-narrow // groups) * narrow_cost
-                if not takes_wide:
-                    del four[cls]
+                tile_rows = ragged_n_tile_rows(rows_m[cls], k_of[cls], T * K, E)
+                if tile_rows != 384:
+                    four[cls] = kernel_of_class[cls].replace("288", str(tile_rows))
         kernel_of_class.update(four)
     by_kernel = {}
     for k, v in gemms.items():

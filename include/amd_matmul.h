@@ -50,10 +50,9 @@ int amd_matmul_no_alloc(Dataflow_Handle * dataflow_handle, int stream_id, int to
  *     operand bytes per flop), every wave loading straight into the LDS and multiplying, its own token rows reloaded
  *     without the barrier.
  *   FOUR_WAVES: one loading wave (operands through its registers) and three multiplying waves, 256 x 288 tiles.
- *   AUTO (the default): ragged-N launches that both EIGHT_WAVES and FOUR_WAVES_384 can take are launched on both, and the
- *     work-groups decide from the group sizes on the device which of the two does the work (the other returns at once):
- *     the larger tile where the groups fill it and the rounds of tiles over the compute units come out no worse.
- *     For a single problem the same rule is evaluated on the host.  Everything else runs EIGHT_WAVES.
+ *   AUTO (the default): a ragged-N launch runs on the cheapest of the tilings of both (tiles of 384, 288, 224 or 192 token
+ *     rows) for the group sizes that an even router gives: the number of tiles, in rounds over the compute units.
+ *     For a single problem, whose tiles are known, tiles of 384 against those of 256.  Everything else runs EIGHT_WAVES.
  * The four-wave kernels are taken only where their limits hold (no C operand, N-side operand k-contiguous, K a multiple
  * of 128 and at most 2^21, M a multiple of 8, 16-byte aligned D), the eight-wave kernel elsewhere.  Results are
  * bit-identical whichever kernel runs.  The choice is process-wide; the environment variable AMD_MATMUL_KERNEL ("auto",

@@ -13,9 +13,10 @@
  * The kernels live in gemm_kernel.h (eight waves), gemm_w4_kernel.h (four waves) and gemm_typed_kernel.h (element
  * types beside all-bf16); this file decodes the op arguments, checks them on the host and picks a kernel: the
  * direct-to-LDS kernels when every operand is 16-byte aligned with a contiguous extent that is a multiple of 8
- * elements, or a workspace holds padded copies of those that are not (pad_operands), the register-staged kernel otherwise; for large ragged-N launches without a C operand the choice between
- * the eight-wave kernel and the four-wave 256 x 384 one is left to the device (launch_gemm).
+ * elements, or a workspace holds padded copies of those that are not (pad_operands), the register-staged kernel otherwise; large
+ * ragged-N launches without a C operand run on one of four tilings (ragged_n_tiling).
  */
+#include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -239,7 +240,7 @@ static bool w4_ok(const GemmParams & p) {
 		   (p.M % 8 == 0) && ((((uintptr_t) p.D) & 15) == 0);
 }
 
-/* one tiling of a ragged-N launch without C; grid: an upper bound on the tiles that is the same for all of its tilings */
+/* a ragged-N launch without C on one of its tilings; grid: an upper bound on the tiles */
 template <bool PK, int GATHER>
 static int launch_ragged_n_tiling(int tiling, const GemmParams & p, long grid, long cu_count, hipStream_t stream) {
 	switch (tiling) {
@@ -250,73 +251,70 @@ static int launch_ragged_n_tiling(int tiling, const GemmParams & p, long grid, l
 	}
 }
 
-static int launch_ragged_n(int candidates, const GemmParams & p, bool pk, long grid, long cu_count, hipStream_t stream) {
-	GemmParams q = p;
-	q.candidates = (candidates & (candidates - 1)) ? candidates : 0;
-	for (int tiling = RAGGED_N_TILINGS - 1; tiling >= 0; tiling--) {
-		if (!((candidates >> tiling) & 1)) {
-			continue;
-		}
-		int r;
-		if (p.gather) {
-			r = pk ? launch_ragged_n_tiling<true, GATHER_Q_ROWS>(tiling, q, grid, cu_count, stream)
-				   : launch_ragged_n_tiling<false, GATHER_Q_ROWS>(tiling, q, grid, cu_count, stream);
-		} else {
-			r = pk ? launch_ragged_n_tiling<true, GATHER_NONE>(tiling, q, grid, cu_count, stream)
-				   : launch_ragged_n_tiling<false, GATHER_NONE>(tiling, q, grid, cu_count, stream);
-		}
-		if (r) {
-			return r;
-		}
+static int launch_ragged_n(int tiling, const GemmParams & p, bool pk, long grid, long cu_count, hipStream_t stream) {
+	if (p.gather) {
+		return pk ? launch_ragged_n_tiling<true, GATHER_Q_ROWS>(tiling, p, grid, cu_count, stream)
+				  : launch_ragged_n_tiling<false, GATHER_Q_ROWS>(tiling, p, grid, cu_count, stream);
 	}
-	return 0;
+	return pk ? launch_ragged_n_tiling<true, GATHER_NONE>(tiling, p, grid, cu_count, stream)
+			  : launch_ragged_n_tiling<false, GATHER_NONE>(tiling, p, grid, cu_count, stream);
 }
 
-/* The tilings a ragged-N launch without C is dispatched on; the device takes the cheapest of them for the real group sizes.
- * A launch that loses costs a few microseconds, so only those are candidates that could win, seen from the mean group:
- *   288: always, the safe one for uneven groups.
- *   384: where it wins with all groups the same size; where it does not, uneven groups only make it lose by more (short
- *        groups fill a 384-row tile worse).
- *   224 or 192: with groups one standard deviation of an even router (the root of the mean) above the mean, so that
- *        the usual spread does not spill into a further tile; where 384 does not win there too, and where it is ahead of
- *        288 by twice what a losing launch costs (FINER_TILE_MARGIN: 6.6 us at 3.3 ns per round, k-tile and fetched row).  No
- *        tiling is faster than the weights arrive, 4.4 TB/s where a group is one tile (STREAMED_WEIGHTS): 32 groups of
- *        170 rows, 2048 x 1408, take 57-60 us on either tile, 1408 x 2048, whose tiles leave a quarter of the compute
- *        units idle, 45 instead of 52. */
-#define FINER_TILE_MARGIN 200000
-#define STREAMED_WEIGHTS(bytes) ((bytes) / 145)
-static long larger(long a, long b) { return a > b ? a : b; }
-static int ragged_n_candidates(const GemmParams & p, long cu_count, bool four_ok) {
-	const long tiles_m = tiles_of(p.M, 256), k_tiles = tiles_of(p.K, BK);
+/* Tiles of `tile_rows` rows of all groups together, as an even router deals the rows: a group's share is near-normal with the
+ * mean's root as standard deviation, seen here at twelve equally likely quantiles.  spread: standard deviation of the result. */
+static double expected_n_tiles(const GemmParams & p, long tile_rows, double * spread) {
+	static const double QUANTILES[6] = {0.104, 0.319, 0.549, 0.812, 1.150, 1.732};
+	const double rows = (double) p.N / p.num_groups, deviation = sqrt(rows);
+	double sum = 0.0, squares = 0.0;
+	for (int i = 0; i < 12; i++) {
+		const double r = rint(rows + (i & 1 ? -1.0 : 1.0) * QUANTILES[i / 2] * deviation);
+		const double tiles = r > 0.0 ? (double) tiles_of((long) r, tile_rows) : 0.0;
+		sum += tiles;
+		squares += tiles * tiles;
+	}
+	const double mean = sum / 12.0, variance = squares / 12.0 - mean * mean;
+	*spread = variance > 0.0 ? sqrt(variance * p.num_groups) : 0.0;
+	return mean * p.num_groups;
+}
+
+/* Rounds of those tiles over the work-groups of a launch; a few tiles more or less decide over a whole round, so half a
+ * standard deviation to both sides counts a quarter each */
+static double expected_rounds(const GemmParams & p, long tile_rows, long groups) {
+	double spread;
+	const double n_tiles = expected_n_tiles(p, tile_rows, &spread);
+	double rounds = 0.0;
+	for (int side = -1; side <= 1; side++) {
+		rounds += (side ? 0.25 : 0.5) * (double) tiles_of(tiles_of(p.M, 256) * lrint(n_tiles + 0.5 * side * spread), groups);
+	}
+	return rounds;
+}
+
+/* The tiling a ragged-N launch without C runs on: the cheapest for the group sizes that an even router gives.  The sizes
+ * themselves are on the device; launching several tilings and letting their work-groups agree on one from the real sizes,
+ * as this did before, costs 3 us for each that returns at once, more than the real sizes tell better.  Over 310 launches
+ * of the layer's kind (8-64 experts, 30-9000 rows each, K 512-4096) the launches then took 4.7 % longer than the best of
+ * all tilings and take 1.9 % longer now; with a Zipf router, whose largest group is eight times the mean, 5.6 and 4.4 % (100
+ * launches).  A training step of 65536 tokens, 64 experts, dim 4096: 37.75 -> 36.99 ms, a forward of 8192 tokens, 32 experts, dim 2048:
+ * 638 -> 622 us.  No tiling is faster than the weights arrive (STREAMED_WEIGHTS: 6 TB/s). */
+#define STREAMED_WEIGHTS(bytes) ((bytes) / 200)
+static double larger(double a, double b) { return a > b ? a : b; }
+static int ragged_n_tiling(const GemmParams & p, long cu_count, bool four_ok) {
+	const long k_tiles = tiles_of(p.K, BK);
 	long groups = cu_count & ~7L;
 	groups = groups < 8 ? 8 : groups;
-	const long rows = p.num_groups > 0 && p.N / p.num_groups > 0 ? p.N / p.num_groups : 1;
-	long above = rows;                                       /* rows + sqrt(rows) */
-	for (long r = 1; r * r <= rows; r++) {
-		above = rows + r;
-	}
-#define EVEN_ROUNDS(group_rows, tile_rows) tiles_of(tiles_m * p.num_groups * tiles_of((group_rows), (tile_rows)), groups)
-	const long narrow = EVEN_ROUNDS(rows, 288);
-	const long wide = EVEN_ROUNDS(rows, 384);
-	int candidates = 1 << RAGGED_N_288;
+	const double narrow = expected_rounds(p, 288, groups), wide = expected_rounds(p, 384, groups);
 	const bool wide_wins = four_ok && WIDE_TILE_COST(wide, k_tiles) < NARROW_TILE_COST(narrow, k_tiles);
-	if (wide_wins) {
-		candidates |= 1 << RAGGED_N_384;
+	const double streamed = STREAMED_WEIGHTS((double) p.num_groups * p.M * p.K * 2.0);
+	int best = wide_wins ? RAGGED_N_384 : RAGGED_N_288;
+	double cost = larger(wide_wins ? WIDE_TILE_COST(wide, k_tiles) : NARROW_TILE_COST(narrow, k_tiles), streamed);
+	for (int rows = 224; rows >= 192; rows -= 32) {
+		const double finer = larger(FINER_TILE_COST(expected_rounds(p, rows, groups), rows, k_tiles), streamed);
+		if (finer < cost) {
+			best = rows == 224 ? RAGGED_N_224 : RAGGED_N_192;
+			cost = finer;
+		}
 	}
-	int finer = RAGGED_N_224;
-	long cost = ragged_n_cost(finer, EVEN_ROUNDS(above, 224), k_tiles);
-	const long cost_192 = ragged_n_cost(RAGGED_N_192, EVEN_ROUNDS(above, 192), k_tiles);
-	if (cost_192 < cost) {
-		finer = RAGGED_N_192;
-		cost = cost_192;
-	}
-	const bool wide_wins_above = wide_wins && WIDE_TILE_COST(EVEN_ROUNDS(above, 384), k_tiles) < cost;
-	const long streamed = STREAMED_WEIGHTS((long) p.num_groups * p.M * p.K * 2);
-	if (!wide_wins_above && larger(cost, streamed) + FINER_TILE_MARGIN < larger(NARROW_TILE_COST(narrow, k_tiles), streamed)) {
-		candidates |= 1 << finer;
-	}
-#undef EVEN_ROUNDS
-	return candidates;
+	return best;
 }
 
 static long round_up8(long v) { return (v + 7) & ~7L; }
@@ -344,7 +342,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 	const bool wide_only = kernel_choice == AMD_MATMUL_KERNEL_FOUR_WAVES_384;
 	const bool either = kernel_choice == AMD_MATMUL_KERNEL_AUTO;
 	if (MODE == MODE_RAGGED_N && four_ok && grid_wide > 0 && wide_only) {
-		return launch_ragged_n(1 << RAGGED_N_384, p, pk, grid_wide, cu_count, stream);
+		return launch_ragged_n(RAGGED_N_384, p, pk, grid_wide, cu_count, stream);
 	}
 	if (MODE == MODE_SINGLE && four_ok && p.split_k <= 1 && (wide_only || either)) {
 		/* a single problem's tiles are known here: the same rule as for the ragged launches, against the 256 x 256 tiles
@@ -378,7 +376,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 		 * latency of the operand stream, not by the multiplies), and a group of slightly more than a multiple of 256
 		 * rows -- every second expert when the mean is such a multiple -- then needs no extra, nearly empty tile.
 		 * Every element is accumulated over k in the same order as in the 256-row tiles: results are bit-identical. */
-		return launch_ragged_n(either ? ragged_n_candidates(p, cu_count, four_ok) : 1 << RAGGED_N_288, p, pk, grid_wide, cu_count, stream);
+		return launch_ragged_n(either ? ragged_n_tiling(p, cu_count, four_ok) : RAGGED_N_288, p, pk, grid_wide, cu_count, stream);
 	}
 #define PICK(PK, QK) do { \
 		if (direct) { \

@@ -72,10 +72,6 @@ struct GemmParams {
 	 * (those past them read as zero, like the padding they are multiplied with) */
 	int pitchA, pitchB;
 	int k_rows;
-	/* Ragged-N launches without C that several tilings can take are launched on each candidate; every work-group counts
-	 * the tiles of the tilings from the device prefix sum (ragged_n_choice) and the kernels that lose return at once.
-	 * One bit per tiling, RAGGED_N_288 always among them; 0: run */
-	int candidates;
 };
 
 struct Tile {
@@ -220,48 +216,11 @@ __device__ __forceinline__ long count_tiles(const GemmParams & p) {
  * 42 us on 192 (53 on 288), 24 groups of 512 rows, 1536 x 3008, 134 (158).  They are charged 7 % per byte: a round of
  * them costs 0-8 % more per k-tile and fetched row than one of 288 (2.6-3.7 ns for K of 1408-4096), most where the
  * weights of many m-tiles come from HBM (64 groups of about 375 rows, 2048 x 4096: 407 us on 384, 434 on 224).
- * A launch is dispatched on every candidate tiling (bits of GemmParams::candidates) and every work-group of them
- * computes the same answer.  All sides are scaled by the k-tiles of a tile. */
+ * All sides are scaled by the k-tiles of a tile; the host compares them for the tiles it expects (ragged_n_tiling). */
 #define WIDE_TILE_COST(rounds, k_tiles) ((rounds) * (256 + 384) * (103 * (k_tiles) + 160))
 #define NARROW_TILE_COST(rounds, k_tiles) ((rounds) * (256 + 288) * 100 * (k_tiles))
 #define FINER_TILE_COST(rounds, rows, k_tiles) ((rounds) * (256 + (rows)) * 107 * (k_tiles))
 enum { RAGGED_N_288, RAGGED_N_384, RAGGED_N_224, RAGGED_N_192, RAGGED_N_TILINGS };
-
-__host__ __device__ __forceinline__ int ragged_n_rows(int tiling) {
-	return tiling == RAGGED_N_288 ? 288 : tiling == RAGGED_N_384 ? 384 : tiling == RAGGED_N_224 ? 224 : 192;
-}
-__host__ __device__ __forceinline__ long ragged_n_cost(int tiling, long rounds, long k_tiles) {
-	return tiling == RAGGED_N_384 ? WIDE_TILE_COST(rounds, k_tiles) : tiling == RAGGED_N_288 ? NARROW_TILE_COST(rounds, k_tiles)
-		 : FINER_TILE_COST(rounds, ragged_n_rows(tiling), k_tiles);
-}
-
-/* the cheapest of the candidates for the group sizes at hand */
-__device__ __forceinline__ int ragged_n_choice(const GemmParams & p) {
-	const int lane = threadIdx.x & 63;
-	int tiles[RAGGED_N_TILINGS] = {0, 0, 0, 0};
-	for (int g = lane; g < p.num_groups; g += 64) {
-		const int rows = p.cumsum[g] - (g ? p.cumsum[g - 1] : 0);
-		#pragma unroll
-		for (int i = 0; i < RAGGED_N_TILINGS; i++) {
-			tiles[i] += (rows + ragged_n_rows(i) - 1) / ragged_n_rows(i);
-		}
-	}
-	const unsigned int groups = gridDim.x;
-	const unsigned int tiles_m = (unsigned int) (p.M + 255) / 256;
-	const long k_tiles = (p.K + BK - 1) / BK;
-	int best = RAGGED_N_288;
-	long least = 0;
-	#pragma unroll
-	for (int i = 0; i < RAGGED_N_TILINGS; i++) {
-		const unsigned int all = (unsigned int) __builtin_amdgcn_readlane(wave_inclusive_sum(tiles[i]), 63) * tiles_m;
-		const long cost = ragged_n_cost(i, (all + groups - 1) / groups, k_tiles);
-		if (i == RAGGED_N_288 || (((p.candidates >> i) & 1) && cost < least)) {
-			best = i;
-			least = cost;
-		}
-	}
-	return __builtin_amdgcn_readfirstlane(best);
-}
 
 /* Order of the tiles of one problem (tiles_m x tiles_n of them, `lid` counts them): the work-groups of a die run 32
  * consecutive tiles at a time, and what they fetch is one operand panel per distinct m-tile plus one per distinct
@@ -1197,11 +1156,7 @@ gemm_bf16_stream_kernel(GemmParams p) {
 	const int wm = (wave % WAVES_M) * WTM;
 	const int wn = (wave / WAVES_M) * WTN;
 
-	static_assert(MODE != MODE_RAGGED_N || BN == 256 || BN == 288 || BN == 224 || BN == 192, "a tiling of ragged_n_choice, or the one for launches with C");
-	constexpr int TILING = BN == 288 ? RAGGED_N_288 : BN == 224 ? RAGGED_N_224 : RAGGED_N_192;
-	if (MODE == MODE_RAGGED_N && p.candidates && ragged_n_choice(p) != TILING) {
-		return;                                             /* another tiling's launch does the work */
-	}
+	static_assert(MODE != MODE_RAGGED_N || BN == 256 || BN == 288 || BN == 224 || BN == 192, "a tiling of ragged_n_tiling, or the one for launches with C");
 	const long total = count_tiles<BM, BN, MODE>(p);
 	const long chunk = (total + 7) >> 3;                    /* tiles per die */
 	const long die = blockIdx.x & 7;
