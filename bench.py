@@ -225,8 +225,8 @@ FUSED_GEMM_KERNEL_OF_CLASS = {
 
 
 def ragged_n_tile_rows(M, K, rows, groups, work_groups=256):
-    """Token rows per tile of a ragged-N launch without C: ragged_n_tiling (csrc/matmul/amd_matmul.hip), restated.  The
-    cheapest tiling for the group sizes that an even router gives."""
+    """Token rows per tile of a ragged-N launch without C: the first tiling of ragged_n_tilings (csrc/matmul/amd_matmul.hip),
+    restated: the cheapest for the group sizes that an even router gives."""
     mean, kt = rows / groups, -(-K // 64)
     sizes = [round(mean + sign * q * mean ** 0.5) for q in (0.104, 0.319, 0.549, 0.812, 1.150, 1.732) for sign in (1.0, -1.0)]
 

@@ -14,7 +14,7 @@
  * types beside all-bf16); this file decodes the op arguments, checks them on the host and picks a kernel: the
  * direct-to-LDS kernels when every operand is 16-byte aligned with a contiguous extent that is a multiple of 8
  * elements, or a workspace holds padded copies of those that are not (pad_operands), the register-staged kernel otherwise; large
- * ragged-N launches without a C operand run on one of four tilings (ragged_n_tiling).
+ * ragged-N launches without a C operand run on one of four tilings (ragged_n_tilings).
  */
 #include <math.h>
 #include <stdio.h>
@@ -251,37 +251,53 @@ static int launch_ragged_n_tiling(int tiling, const GemmParams & p, long grid, l
 	}
 }
 
-static int launch_ragged_n(int tiling, const GemmParams & p, bool pk, long grid, long cu_count, hipStream_t stream) {
-	if (p.gather) {
-		return pk ? launch_ragged_n_tiling<true, GATHER_Q_ROWS>(tiling, p, grid, cu_count, stream)
-				  : launch_ragged_n_tiling<false, GATHER_Q_ROWS>(tiling, p, grid, cu_count, stream);
+/* on every tiling of `tilings` (bits) */
+static int launch_ragged_n(int tilings, const GemmParams & p, bool pk, long grid, long cu_count, hipStream_t stream) {
+	GemmParams q = p;
+	q.candidates = (tilings & (tilings - 1)) ? tilings : 0;
+	for (int tiling = RAGGED_N_TILINGS - 1; tiling >= 0; tiling--) {
+		if (!((tilings >> tiling) & 1)) {
+			continue;
+		}
+		int r;
+		if (p.gather) {
+			r = pk ? launch_ragged_n_tiling<true, GATHER_Q_ROWS>(tiling, q, grid, cu_count, stream)
+				   : launch_ragged_n_tiling<false, GATHER_Q_ROWS>(tiling, q, grid, cu_count, stream);
+		} else {
+			r = pk ? launch_ragged_n_tiling<true, GATHER_NONE>(tiling, q, grid, cu_count, stream)
+				   : launch_ragged_n_tiling<false, GATHER_NONE>(tiling, q, grid, cu_count, stream);
+		}
+		if (r) {
+			return r;
+		}
 	}
-	return pk ? launch_ragged_n_tiling<true, GATHER_NONE>(tiling, p, grid, cu_count, stream)
-			  : launch_ragged_n_tiling<false, GATHER_NONE>(tiling, p, grid, cu_count, stream);
+	return 0;
 }
 
-/* Tiles of `tile_rows` rows of all groups together, as an even router deals the rows: a group's share is near-normal with the
- * mean's root as standard deviation, seen here at twelve equally likely quantiles.  spread: standard deviation of the result. */
-static double expected_n_tiles(const GemmParams & p, long tile_rows, double * spread) {
-	static const double QUANTILES[6] = {0.104, 0.319, 0.549, 0.812, 1.150, 1.732};
+/* Tiles of `tile_rows` rows of all groups together.  Even: as an even router deals the rows, a group's share near-normal with the
+ * mean's root as standard deviation.  Uneven: shares that fall like a power (0.9) of the group's rank, the largest 4.1 times
+ * the mean.  Either is seen at twelve equally likely quantiles.  spread: standard deviation of the result. */
+static double expected_n_tiles(const GemmParams & p, long tile_rows, bool uneven, double * spread) {
+	static const double NORMAL[6] = {0.104, 0.319, 0.549, 0.812, 1.150, 1.732};
+	static const double SHARES[12] = {4.122, 1.855, 1.223, 0.921, 0.743, 0.624, 0.540, 0.476, 0.427, 0.387, 0.354, 0.327};
 	const double rows = (double) p.N / p.num_groups, deviation = sqrt(rows);
 	double sum = 0.0, squares = 0.0;
 	for (int i = 0; i < 12; i++) {
-		const double r = rint(rows + (i & 1 ? -1.0 : 1.0) * QUANTILES[i / 2] * deviation);
+		const double r = rint(uneven ? rows * SHARES[i] : rows + (i & 1 ? -1.0 : 1.0) * NORMAL[i / 2] * deviation);
 		const double tiles = r > 0.0 ? (double) tiles_of((long) r, tile_rows) : 0.0;
 		sum += tiles;
 		squares += tiles * tiles;
 	}
 	const double mean = sum / 12.0, variance = squares / 12.0 - mean * mean;
-	*spread = variance > 0.0 ? sqrt(variance * p.num_groups) : 0.0;
+	*spread = variance > 0.0 && !uneven ? sqrt(variance * p.num_groups) : 0.0;
 	return mean * p.num_groups;
 }
 
 /* Rounds of those tiles over the work-groups of a launch; a few tiles more or less decide over a whole round, so half a
  * standard deviation to both sides counts a quarter each */
-static double expected_rounds(const GemmParams & p, long tile_rows, long groups) {
+static double expected_rounds(const GemmParams & p, long tile_rows, bool uneven, long groups) {
 	double spread;
-	const double n_tiles = expected_n_tiles(p, tile_rows, &spread);
+	const double n_tiles = expected_n_tiles(p, tile_rows, uneven, &spread);
 	double rounds = 0.0;
 	for (int side = -1; side <= 1; side++) {
 		rounds += (side ? 0.25 : 0.5) * (double) tiles_of(tiles_of(p.M, 256) * lrint(n_tiles + 0.5 * side * spread), groups);
@@ -289,32 +305,41 @@ static double expected_rounds(const GemmParams & p, long tile_rows, long groups)
 	return rounds;
 }
 
-/* The tiling a ragged-N launch without C runs on: the cheapest for the group sizes that an even router gives.  The sizes
- * themselves are on the device; launching several tilings and letting their work-groups agree on one from the real sizes,
- * as this did before, costs 3 us for each that returns at once, more than the real sizes tell better.  Over 310 launches
- * of the layer's kind (8-64 experts, 30-9000 rows each, K 512-4096) the launches then took 4.7 % longer than the best of
- * all tilings and take 1.9 % longer now; with a Zipf router, whose largest group is eight times the mean, 5.6 and 4.4 % (100
- * launches).  A training step of 65536 tokens, 64 experts, dim 4096: 37.75 -> 36.99 ms, a forward of 8192 tokens, 32 experts, dim 2048:
- * 638 -> 622 us.  No tiling is faster than the weights arrive (STREAMED_WEIGHTS: 6 TB/s). */
+/* expected costs of the tilings, and the cheapest.  No tiling is faster than the weights arrive (STREAMED_WEIGHTS: 6 TB/s). */
 #define STREAMED_WEIGHTS(bytes) ((bytes) / 200)
 static double larger(double a, double b) { return a > b ? a : b; }
-static int ragged_n_tiling(const GemmParams & p, long cu_count, bool four_ok) {
+static int cheapest_tiling(const GemmParams & p, long groups, bool four_ok, bool uneven, double cost[RAGGED_N_TILINGS]) {
 	const long k_tiles = tiles_of(p.K, BK);
-	long groups = cu_count & ~7L;
-	groups = groups < 8 ? 8 : groups;
-	const double narrow = expected_rounds(p, 288, groups), wide = expected_rounds(p, 384, groups);
-	const bool wide_wins = four_ok && WIDE_TILE_COST(wide, k_tiles) < NARROW_TILE_COST(narrow, k_tiles);
+	const double narrow = expected_rounds(p, 288, uneven, groups), wide = expected_rounds(p, 384, uneven, groups);
 	const double streamed = STREAMED_WEIGHTS((double) p.num_groups * p.M * p.K * 2.0);
-	int best = wide_wins ? RAGGED_N_384 : RAGGED_N_288;
-	double cost = larger(wide_wins ? WIDE_TILE_COST(wide, k_tiles) : NARROW_TILE_COST(narrow, k_tiles), streamed);
-	for (int rows = 224; rows >= 192; rows -= 32) {
-		const double finer = larger(FINER_TILE_COST(expected_rounds(p, rows, groups), rows, k_tiles), streamed);
-		if (finer < cost) {
-			best = rows == 224 ? RAGGED_N_224 : RAGGED_N_192;
-			cost = finer;
+	int best = four_ok && WIDE_TILE_COST(wide, k_tiles) < NARROW_TILE_COST(narrow, k_tiles) ? RAGGED_N_384 : RAGGED_N_288;
+	cost[RAGGED_N_288] = larger(NARROW_TILE_COST(narrow, k_tiles), streamed);
+	cost[RAGGED_N_384] = larger(WIDE_TILE_COST(wide, k_tiles), streamed);
+	for (int tiling = RAGGED_N_224; tiling <= RAGGED_N_192; tiling++) {
+		const long rows = ragged_n_rows(tiling);
+		cost[tiling] = larger(FINER_TILE_COST(expected_rounds(p, rows, uneven, groups), rows, k_tiles), streamed);
+		if (cost[tiling] < cost[best]) {
+			best = tiling;
 		}
 	}
 	return best;
+}
+
+/* The tilings a ragged-N launch without C goes out on, as bits: the cheapest for the group sizes that an even router gives, and where
+ * that one costs 5 % and 4 us more than another with very uneven groups, that other one too: the sizes are on the device, whose
+ * work-groups then agree on one of the two from the real sizes (ragged_n_choice).  A launch that loses costs 3 us, so both
+ * go out only there.  Over 310 launches of the layer's kind (8-64 experts, 30-9000 rows each, K 512-4096) one launch on the
+ * expected tiling takes 1.9 % longer than the best of all tilings and this rule 2.5 %; up to three launches, among them 288 always,
+ * took 4.7 %.  With a Zipf router, whose largest group is eight times the mean (100 launches), 4.5, 3.2 and 5.6 %: one of
+ * 2979 tokens, 36 experts, top 4, dim 832 lost 9 % to the single launch.  us: a training step of 65536 tokens, 64 experts, dim
+ * 4096 37.75 -> 36.99 ms, a forward of 8192 tokens, 32 experts, dim 2048 638 -> 622. */
+#define SECOND_TILING_MARGIN 121000
+static int ragged_n_tilings(const GemmParams & p, long cu_count, bool four_ok) {
+	long groups = cu_count & ~7L;
+	groups = groups < 8 ? 8 : groups;
+	double even[RAGGED_N_TILINGS], uneven[RAGGED_N_TILINGS];
+	const int first = cheapest_tiling(p, groups, four_ok, false, even), second = cheapest_tiling(p, groups, four_ok, true, uneven);
+	return uneven[first] < 1.05 * uneven[second] + SECOND_TILING_MARGIN ? 1 << first : 1 << first | 1 << second;
 }
 
 static long round_up8(long v) { return (v + 7) & ~7L; }
@@ -342,7 +367,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 	const bool wide_only = kernel_choice == AMD_MATMUL_KERNEL_FOUR_WAVES_384;
 	const bool either = kernel_choice == AMD_MATMUL_KERNEL_AUTO;
 	if (MODE == MODE_RAGGED_N && four_ok && grid_wide > 0 && wide_only) {
-		return launch_ragged_n(RAGGED_N_384, p, pk, grid_wide, cu_count, stream);
+		return launch_ragged_n(1 << RAGGED_N_384, p, pk, grid_wide, cu_count, stream);
 	}
 	if (MODE == MODE_SINGLE && four_ok && p.split_k <= 1 && (wide_only || either)) {
 		/* a single problem's tiles are known here: the same rule as for the ragged launches, against the 256 x 256 tiles
@@ -376,7 +401,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 		 * latency of the operand stream, not by the multiplies), and a group of slightly more than a multiple of 256
 		 * rows -- every second expert when the mean is such a multiple -- then needs no extra, nearly empty tile.
 		 * Every element is accumulated over k in the same order as in the 256-row tiles: results are bit-identical. */
-		return launch_ragged_n(either ? ragged_n_tiling(p, cu_count, four_ok) : RAGGED_N_288, p, pk, grid_wide, cu_count, stream);
+		return launch_ragged_n(either ? ragged_n_tilings(p, cu_count, four_ok) : 1 << RAGGED_N_288, p, pk, grid_wide, cu_count, stream);
 	}
 #define PICK(PK, QK) do { \
 		if (direct) { \

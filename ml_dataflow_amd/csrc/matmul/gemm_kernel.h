@@ -67,6 +67,10 @@ struct GemmParams {
 	float * partial;
 	int split_k;                   /* 0 or 1: off */
 	int kt_per_split;              /* a multiple of 4, as the host plans it; the kernel takes any */
+	/* A ragged-N launch without C goes out on two tilings where even and very uneven groups would be best on different ones; every
+	 * work-group counts the tiles of both from the device prefix sum (ragged_n_choice) and the kernel that loses returns at
+	 * once.  The bits of the two tilings, or 0: run */
+	int candidates;
 	/* Operands copied to padded rows (single problems on the direct kernel only; 0: not padded): elements from one k-row
 	 * to the next of a k-major operand, and the k-rows a k-major operand has where K was rounded up for a k-contiguous one
 	 * (those past them read as zero, like the padding they are multiplied with) */
@@ -216,11 +220,39 @@ __device__ __forceinline__ long count_tiles(const GemmParams & p) {
  * 42 us on 192 (53 on 288), 24 groups of 512 rows, 1536 x 3008, 134 (158).  They are charged 7 % per byte: a round of
  * them costs 0-8 % more per k-tile and fetched row than one of 288 (2.6-3.7 ns for K of 1408-4096), most where the
  * weights of many m-tiles come from HBM (64 groups of about 375 rows, 2048 x 4096: 407 us on 384, 434 on 224).
- * All sides are scaled by the k-tiles of a tile; the host compares them for the tiles it expects (ragged_n_tiling). */
+ * All sides are scaled by the k-tiles of a tile; the host compares them for the tiles it expects (ragged_n_tilings). */
 #define WIDE_TILE_COST(rounds, k_tiles) ((rounds) * (256 + 384) * (103 * (k_tiles) + 160))
 #define NARROW_TILE_COST(rounds, k_tiles) ((rounds) * (256 + 288) * 100 * (k_tiles))
 #define FINER_TILE_COST(rounds, rows, k_tiles) ((rounds) * (256 + (rows)) * 107 * (k_tiles))
 enum { RAGGED_N_288, RAGGED_N_384, RAGGED_N_224, RAGGED_N_192, RAGGED_N_TILINGS };
+
+__host__ __device__ __forceinline__ int ragged_n_rows(int tiling) {
+	return tiling == RAGGED_N_288 ? 288 : tiling == RAGGED_N_384 ? 384 : tiling == RAGGED_N_224 ? 224 : 192;
+}
+__host__ __device__ __forceinline__ long ragged_n_cost(int tiling, long rounds, long k_tiles) {
+	return tiling == RAGGED_N_384 ? WIDE_TILE_COST(rounds, k_tiles) : tiling == RAGGED_N_288 ? NARROW_TILE_COST(rounds, k_tiles)
+		 : FINER_TILE_COST(rounds, ragged_n_rows(tiling), k_tiles);
+}
+
+/* the cheaper of the two candidates for the group sizes at hand */
+__device__ __forceinline__ int ragged_n_choice(const GemmParams & p) {
+	const int lane = threadIdx.x & 63;
+	const int first = __ffs(p.candidates) - 1, second = 31 - __clz(p.candidates);
+	const int first_rows = ragged_n_rows(first), second_rows = ragged_n_rows(second);
+	int first_tiles = 0, second_tiles = 0;
+	for (int g = lane; g < p.num_groups; g += 64) {
+		const int rows = p.cumsum[g] - (g ? p.cumsum[g - 1] : 0);
+		first_tiles += (rows + first_rows - 1) / first_rows;
+		second_tiles += (rows + second_rows - 1) / second_rows;
+	}
+	const unsigned int groups = gridDim.x;
+	const unsigned int tiles_m = (unsigned int) (p.M + 255) / 256;
+	const long k_tiles = (p.K + BK - 1) / BK;
+	const unsigned int first_all = (unsigned int) __builtin_amdgcn_readlane(wave_inclusive_sum(first_tiles), 63) * tiles_m;
+	const unsigned int second_all = (unsigned int) __builtin_amdgcn_readlane(wave_inclusive_sum(second_tiles), 63) * tiles_m;
+	const bool take_second = ragged_n_cost(second, (second_all + groups - 1) / groups, k_tiles) < ragged_n_cost(first, (first_all + groups - 1) / groups, k_tiles);
+	return __builtin_amdgcn_readfirstlane(take_second ? second : first);
+}
 
 /* Order of the tiles of one problem (tiles_m x tiles_n of them, `lid` counts them): the work-groups of a die run 32
  * consecutive tiles at a time, and what they fetch is one operand panel per distinct m-tile plus one per distinct
@@ -1156,7 +1188,11 @@ gemm_bf16_stream_kernel(GemmParams p) {
 	const int wm = (wave % WAVES_M) * WTM;
 	const int wn = (wave / WAVES_M) * WTN;
 
-	static_assert(MODE != MODE_RAGGED_N || BN == 256 || BN == 288 || BN == 224 || BN == 192, "a tiling of ragged_n_tiling, or the one for launches with C");
+	static_assert(MODE != MODE_RAGGED_N || BN == 256 || BN == 288 || BN == 224 || BN == 192, "a tiling of ragged_n_tilings, or the one for launches with C");
+	constexpr int TILING = BN == 288 ? RAGGED_N_288 : BN == 224 ? RAGGED_N_224 : RAGGED_N_192;
+	if (MODE == MODE_RAGGED_N && p.candidates && ragged_n_choice(p) != TILING) {
+		return;                                             /* the other tiling's launch does the work */
+	}
 	const long total = count_tiles<BM, BN, MODE>(p);
 	const long chunk = (total + 7) >> 3;                    /* tiles per die */
 	const long die = blockIdx.x & 7;
