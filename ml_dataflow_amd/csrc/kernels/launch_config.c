@@ -309,6 +309,15 @@ int default_rms_norm_bwd_w_combine_set_launch_config(Hip_Launch_Config * cfg, Da
 	return 0;
 }
 
+int amd_rms_norm_bwd_w_few_rows_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {
+	(void) handle; (void) fn;
+	if (check_row_len("rms_norm_bwd_w", ARG_INT(op, 1))) {
+		return -1;
+	}
+	set_1d(cfg, (unsigned int) ((ARG_INT(op, 1) + 63) / 64), 1024, 0);
+	return 0;
+}
+
 /* ---- AdamW (backends/nvidia/src/ops/src/native/src/optimizer/adamw_step_config.c) ---- */
 
 int default_adamw_step_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {

@@ -236,3 +236,63 @@ default_rms_norm_bwd_w_combine_bf16_kernel(const int * __restrict__ num_orig_blo
 		dW[col] = f32_to_bf16(t);
 	}
 }
+
+/* Both halves in one launch, for few rows: a work-group owns 64 columns and all rows.  Each of its 128 groups of eight lanes
+ * takes every 128th row (128 contiguous bytes a row), the sums of the groups are added through the LDS and on to dW.  The two
+ * launches it replaces are bound by their submission, 3.7 us each, and the second by its 512 partial rows; this one by the
+ * load path of a compute unit, which each row takes 256 bytes through: 4.0 us up to 768 rows (7.4-11.6 before), 4.7 at 1024 x
+ * 2048 (9.2).  More rows are left to the two launches, which spread them over all compute units.
+ * Launch: grid = ceil(n_cols / 64), block = 1024.
+ * `blocks`: what the two-launch form records as its number of work-groups, recorded here for callers that read it. */
+#define FEW_ROWS_LANES 128
+extern "C" __global__ void __launch_bounds__(FEW_ROWS_LANES * 8)
+amd_rms_norm_bwd_w_few_rows_bf16_bf16_kernel(int n_rows, int n_cols, const float * __restrict__ fwd_rms_vals, const bf16_t * __restrict__ X_inp,
+											 const bf16_t * __restrict__ upstream_dX, bf16_t * dW, int blocks, int * __restrict__ ret_num_blocks_launched) {
+	__shared__ float partial[FEW_ROWS_LANES][WAVE + 1];
+	__shared__ float wave_sum[COMBINE_WAVES][WAVE];
+	static_assert(FEW_ROWS_LANES * 8 == COMBINE_WAVES * WAVE, "sixteen waves add up the partial sums");
+	if (blockIdx.x == 0 && threadIdx.x == 0) {
+		*ret_num_blocks_launched = blocks;
+	}
+	const int row_lane = threadIdx.x >> 3;
+	const int nvec = n_cols >> 3;
+	const int v = blockIdx.x * 8 + (threadIdx.x & 7);
+	float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+	if (v < nvec) {
+		#pragma unroll 4
+		for (int row = row_lane; row < n_rows; row += FEW_ROWS_LANES) {
+			const size_t off = (size_t) row * n_cols;
+			const float r = fwd_rms_vals[row];
+			float fx[8], fg[8];
+			unpack8(((const u32x4 *) (X_inp + off))[v], fx);
+			unpack8(((const u32x4 *) (upstream_dX + off))[v], fg);
+			#pragma unroll
+			for (int e = 0; e < 8; e++) {
+				acc[e] += (fg[e] * fx[e]) * r;
+			}
+		}
+	}
+	#pragma unroll
+	for (int e = 0; e < 8; e++) {
+		partial[row_lane][(threadIdx.x & 7) * 8 + e] = acc[e];
+	}
+	__syncthreads();
+	const int lane = threadIdx.x & (WAVE - 1);
+	const int wave = threadIdx.x / WAVE;
+	float sum = 0.0f;
+	#pragma unroll
+	for (int i = 0; i < FEW_ROWS_LANES / COMBINE_WAVES; i++) {
+		sum += partial[wave * (FEW_ROWS_LANES / COMBINE_WAVES) + i][lane];
+	}
+	wave_sum[wave][lane] = sum;
+	__syncthreads();
+	const int col = blockIdx.x * WAVE + lane;
+	if (wave == 0 && col < n_cols) {
+		float t = bf16_to_f32(dW[col]);
+		#pragma unroll
+		for (int w = 0; w < COMBINE_WAVES; w++) {
+			t += wave_sum[w][lane];
+		}
+		dW[col] = f32_to_bf16(t);
+	}
+}

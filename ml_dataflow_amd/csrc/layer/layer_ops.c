@@ -1,10 +1,10 @@
 /* layer_ops.c -- skeletons and submission of the layer driver's own ops (see layer_ops.h) */
 #include "layer_ops.h"
 #include "../ops/skeletons.h"
+#include "../ops/stand_in.h"
 #include "dataflow_amd_ops.h"
 
 #include <stdio.h>
-#include <string.h>
 
 static int submit(Dataflow_Handle * handle, Op * op, int stream_id, const char * what) {
 	if ((handle->submit_op)(handle, op, stream_id)) {
@@ -21,40 +21,24 @@ void layer_set_route_tokens_skeleton(Op_Skeleton * skeleton) {
 	dataflow_fill_skeleton(skeleton, "amd_route_tokens", DATAFLOW_BF16, DATAFLOW_NONE, 17, t);
 }
 
-static Hip_Function * registered(Dataflow_Handle * handle, Op_Skeleton * skeleton) {
-	Hip_Function * fn = NULL;
-	return dataflow_find_table(&handle->op_table, skeleton->identifier.fingerprint, false, (void **) &fn) >= 0 ? fn : NULL;
-}
-
-/* the implementations in the table of the ops that routing consists of; 0 where one is not there */
-static int routing_implementations(Dataflow_Handle * handle, const void * implementations[HIP_MAX_STOOD_IN]) {
-	Op_Skeleton skeletons[HIP_MAX_STOOD_IN];
+static void stood_in_skeletons(Op_Skeleton skeletons[3]) {
 	dataflow_set_matmul_skeleton(&skeletons[0]);
 	dataflow_set_default_select_experts_skeleton(&skeletons[1], DATAFLOW_BF16);
 	dataflow_set_default_build_expert_mapping_skeleton(&skeletons[2]);
-	for (int i = 0; i < HIP_MAX_STOOD_IN; i++) {
-		const Hip_Function * fn = registered(handle, &skeletons[i]);
-		implementations[i] = !fn ? NULL : fn->is_native ? fn->function_handle : (const void *) fn->hip_external_func;
-		if (!implementations[i]) {
-			return 0;
-		}
-	}
-	return 1;
 }
 
 int layer_bind_route_tokens(Dataflow_Handle * handle) {
-	Op_Skeleton skeleton;
+	Op_Skeleton skeleton, of[3];
 	layer_set_route_tokens_skeleton(&skeleton);
-	Hip_Function * fn = registered(handle, &skeleton);
-	return fn && routing_implementations(handle, fn->stands_in_for) ? 0 : -1;
+	stood_in_skeletons(of);
+	return stand_in_bind(handle, &skeleton, of, 3);
 }
 
 int layer_has_route_tokens(Dataflow_Handle * handle) {
-	Op_Skeleton skeleton;
+	Op_Skeleton skeleton, of[3];
 	layer_set_route_tokens_skeleton(&skeleton);
-	const Hip_Function * fn = registered(handle, &skeleton);
-	const void * now[HIP_MAX_STOOD_IN];
-	return fn && routing_implementations(handle, now) && memcmp(now, fn->stands_in_for, sizeof(now)) == 0;
+	stood_in_skeletons(of);
+	return stand_in_usable(handle, &skeleton, of, 3);
 }
 
 int layer_submit_route_tokens(Dataflow_Handle * handle, int stream_id, int num_tokens, int num_experts, int top_k, int model_dim,

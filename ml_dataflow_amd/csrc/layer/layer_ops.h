@@ -18,10 +18,7 @@
 #define LAYER_ROUTE_MAX_EXPERTS 512
 #define LAYER_ROUTE_WORKSPACE(tokens, experts) (((uint64_t) (tokens) + 31) / 32 * (2 * (uint64_t) (experts) + 16) + 256)
 LAYER_OPS_HIDDEN void layer_set_route_tokens_skeleton(Op_Skeleton * skeleton);
-/* The op is used where it is what the ops it stands in for would do: where the handle's table holds it and, under matmul,
- * select_experts and build_expert_mapping, the implementations that stood there when it was registered (_bind notes them,
- * behind its registration).  A program that registers the ops one by one, or puts its own in the place of one of those,
- * has its layer routed op by op. */
+/* stands in for matmul, select_experts and build_expert_mapping (../ops/stand_in.h); _bind goes behind its registration */
 LAYER_OPS_HIDDEN int layer_bind_route_tokens(Dataflow_Handle * handle);
 LAYER_OPS_HIDDEN int layer_has_route_tokens(Dataflow_Handle * handle);
 LAYER_OPS_HIDDEN int layer_submit_route_tokens(Dataflow_Handle * handle, int stream_id, int num_tokens, int num_experts, int top_k, int model_dim,

@@ -9,6 +9,7 @@
  */
 #include "dataflow_amd_ops.h"
 #include "skeletons.h"
+#include "stand_in.h"
 
 #include <pthread.h>
 #include <stdatomic.h>
@@ -555,6 +556,28 @@ int dataflow_submit_default_rms_norm_bwd_x(Dataflow_Handle * handle, int stream_
 
 /* two submissions, as in the reference: partial sums per work-group into the workspace (a 256-byte header with
  * the work-group count, then fp32 rows), then the reduction into dW */
+void dataflow_set_amd_rms_norm_bwd_w_few_rows_skeleton(Op_Skeleton * skeleton) {
+	const DataflowDatatype t[8] = {I_S, I_S, DATAFLOW_FP32, DATAFLOW_BF16, DATAFLOW_BF16, DATAFLOW_BF16, I_S, DATAFLOW_INT};
+	fill_skeleton(skeleton, "amd_rms_norm_bwd_w_few_rows", DATAFLOW_BF16, DATAFLOW_BF16, 8, t);
+}
+
+static void few_rows_stood_in(Op_Skeleton of[2]) {
+	dataflow_set_default_rms_norm_bwd_w_skeleton(&of[0], DATAFLOW_BF16, DATAFLOW_BF16);
+	dataflow_set_default_rms_norm_bwd_w_combine_skeleton(&of[1], DATAFLOW_BF16);
+}
+
+int dataflow_bind_amd_rms_norm_bwd_w_few_rows(Dataflow_Handle * handle) {
+	Op_Skeleton op, of[2];
+	dataflow_set_amd_rms_norm_bwd_w_few_rows_skeleton(&op);
+	few_rows_stood_in(of);
+	return stand_in_bind(handle, &op, of, 2);
+}
+
+/* Up to this many rows one launch does both halves, its work-groups walking all the rows.  Both forms at 1536 rows, us: 512
+ * columns 6.0 against 8.2, 2048 6.0 against 10.2, 4096 10.6 against 13.2, 8192 12.5 against 21.9; at 2048 rows 7.3 / 8.9,
+ * 13.4 / 10.9, 15.2 / 14.3 and 16.0 / 24.1; up to 768 rows 4-6 against 7-18. */
+#define FEW_ROWS 1536
+
 int dataflow_submit_default_rms_norm_bwd_w(Dataflow_Handle * handle, int stream_id,
 										   DataflowDatatype fwd_dt, DataflowDatatype bwd_dt,
 										   int n_rows, int n_cols, float eps, float * fwd_rms_vals,
@@ -567,8 +590,21 @@ int dataflow_submit_default_rms_norm_bwd_w(Dataflow_Handle * handle, int stream_
 	int * ret_num_blocks_launched = (int *) workspace;
 	float * dW_workspace = (float *) ((char *) workspace + 256);
 	Op op;
-	dataflow_set_default_rms_norm_bwd_w_skeleton(&op.op_skeleton, fwd_dt, bwd_dt);
 	void ** a = op.op_args;
+	if (n_rows >= 1 && n_rows <= FEW_ROWS && n_cols >= 8 && (n_cols & 7) == 0 && fwd_dt == DATAFLOW_BF16 && bwd_dt == DATAFLOW_BF16
+		&& workspaceBytes >= 256 + (uint64_t) n_cols * 4) {
+		Op_Skeleton of[2];
+		dataflow_set_amd_rms_norm_bwd_w_few_rows_skeleton(&op.op_skeleton);
+		few_rows_stood_in(of);
+		if (stand_in_usable(handle, &op.op_skeleton, of, 2)) {
+			const uint64_t room = (workspaceBytes - 256) / ((uint64_t) n_cols * 4);
+			int blocks = room < (uint64_t) n_rows ? (int) room : n_rows;
+			a[0] = &n_rows; a[1] = &n_cols; a[2] = &fwd_rms_vals; a[3] = &X_inp; a[4] = &upstream_dX; a[5] = &dW;
+			a[6] = &blocks; a[7] = &ret_num_blocks_launched;
+			return submit(handle, &op, stream_id, "rms norm bwd w (few rows)");
+		}
+	}
+	dataflow_set_default_rms_norm_bwd_w_skeleton(&op.op_skeleton, fwd_dt, bwd_dt);
 	a[0] = &n_rows; a[1] = &n_cols; a[2] = &eps; a[3] = &fwd_rms_vals; a[4] = &X_inp; a[5] = &upstream_dX;
 	a[6] = &dW_workspace; a[7] = &ret_num_blocks_launched; a[8] = &workspaceBytes;
 	if (submit(handle, &op, stream_id, "rms norm bwd w")) {

@@ -8,4 +8,8 @@
 __attribute__((visibility("hidden"))) void dataflow_fill_skeleton(Op_Skeleton * skeleton, const char * base, DataflowDatatype dt0, DataflowDatatype dt1,
 																  int num_args, const DataflowDatatype * arg_dtypes);
 
+/* rms_norm_bwd_w and its combine for few rows, in one launch (dataflow_submit_default_rms_norm_bwd_w submits it) */
+__attribute__((visibility("hidden"))) void dataflow_set_amd_rms_norm_bwd_w_few_rows_skeleton(Op_Skeleton * skeleton);
+__attribute__((visibility("hidden"))) int dataflow_bind_amd_rms_norm_bwd_w_few_rows(Dataflow_Handle * handle);
+
 #endif

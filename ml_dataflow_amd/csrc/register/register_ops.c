@@ -13,6 +13,7 @@
 #include "dataflow_amd.h"
 #include "dataflow_amd_ops.h"
 #include "../layer/layer_ops.h"
+#include "../ops/skeletons.h"
 
 #include <dlfcn.h>
 #include <limits.h>
@@ -149,26 +150,27 @@ static int register_external(Dataflow_Handle * handle, const char * dir) {
 	return added;
 }
 
-/* the layer driver's own ops: in the table like the others, but no part of the operator interface (and of the count that
- * registration reports) */
-static int register_layer_ops(Dataflow_Handle * handle, const char * dir) {
-	enum { N = 1 };
-	Op_Skeleton skeletons[N];
-	layer_set_route_tokens_skeleton(&skeletons[0]);
-	char * symbols[N] = {"amd_route_tokens"};
-	char * init_symbols[N] = {"amd_matmul_init"};
-	char lib[PATH_MAX];
-	snprintf(lib, sizeof(lib), "%s/%s", dir, MATMUL_LIB);
-	int added = (handle->register_external_code)(handle, lib, N, skeletons, symbols, init_symbols);
-	if (added != N) {
-		fprintf(stderr, "Error: failed to register the layer's ops, expected %d functions, got %d...\n", N, added);
+/* the ops that stand in for sequences of others: in the table like the others, but no part of the operator interface (and
+ * of the count that registration reports) */
+static int register_stand_ins(Dataflow_Handle * handle, const char * dir) {
+	Op_Skeleton skeleton;
+	char path[PATH_MAX], config_lib[PATH_MAX];
+	layer_set_route_tokens_skeleton(&skeleton);
+	char * symbol = "amd_route_tokens", * init_symbol = "amd_matmul_init";
+	snprintf(path, sizeof(path), "%s/%s", dir, MATMUL_LIB);
+	if ((handle->register_external_code)(handle, path, 1, &skeleton, &symbol, &init_symbol) != 1 || layer_bind_route_tokens(handle)) {
+		fprintf(stderr, "Error: failed to register the layer's routing op, which needs the matmul, select_experts and build_expert_mapping in the table...\n");
 		return -1;
 	}
-	if (layer_bind_route_tokens(handle)) {
-		fprintf(stderr, "Error: the layer's routing op needs the matmul, select_experts and build_expert_mapping in the table...\n");
+	dataflow_set_amd_rms_norm_bwd_w_few_rows_skeleton(&skeleton);
+	char * kernel = "amd_rms_norm_bwd_w_few_rows_bf16_bf16_kernel", * launch = "amd_rms_norm_bwd_w_few_rows_set_launch_config", * none = NULL;
+	snprintf(path, sizeof(path), "%s/%s", dir, NATIVE_CODE_FILE);
+	snprintf(config_lib, sizeof(config_lib), "%s/%s", dir, NATIVE_CONFIG_LIB);
+	if ((handle->register_native_code)(handle, path, config_lib, 1, &skeleton, &kernel, &launch, &none) != 1 || dataflow_bind_amd_rms_norm_bwd_w_few_rows(handle)) {
+		fprintf(stderr, "Error: failed to register the norm's weight gradient over few rows, which needs rms_norm_bwd_w and its combine in the table...\n");
 		return -1;
 	}
-	return added;
+	return 0;
 }
 
 int dataflow_register_default_ops(Dataflow_Handle * dataflow_handle) {
@@ -185,7 +187,7 @@ int dataflow_register_default_ops(Dataflow_Handle * dataflow_handle) {
 		return -1;
 	}
 	int native = register_native(dataflow_handle, dir);
-	if (native < 0 || register_layer_ops(dataflow_handle, dir) < 0) {
+	if (native < 0 || register_stand_ins(dataflow_handle, dir) < 0) {
 		return -1;
 	}
 	return external + native;

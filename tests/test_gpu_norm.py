@@ -101,6 +101,27 @@ def test_rms_norm_bwd_w(backend, oracle, rows, cols, groups):
     assert np.percentile(bf16_ulp_diff(got, want), 99) <= 1
 
 
+@pytest.mark.parametrize("rows", [1, 2, 127, 128, 129, 511, 1024, 1535, 1536, 1537])
+@pytest.mark.parametrize("cols", [8, 56, 72, 520])
+def test_rms_norm_bwd_w_few_rows_and_more(backend, rows, cols):
+    """One launch up to 1536 rows, two above: row counts at the edges of its 128 row lanes and of the rule, columns at those of
+    its 64.  Whole numbers whose sums fp32 holds exactly in any order, so the result is exact up to its rounding to bf16."""
+    print("case rms_norm_bwd_w few rows=%d cols=%d" % (rows, cols), flush=True)
+    be = backend
+    rng = np.random.default_rng(rows + cols)
+    x, g = rng.integers(-4, 5, (rows, cols)), rng.integers(-4, 5, (rows, cols))
+    rms = np.exp2(rng.integers(-1, 2, rows)).astype(np.float32)
+    start = rng.integers(-8, 9, cols)
+    d_X, d_G, d_rms, d_dW = be.upload(f32_to_bf16(x.astype(np.float32))), be.upload(f32_to_bf16(g.astype(np.float32))), be.upload(rms), be.upload(f32_to_bf16(start.astype(np.float32)))
+    ws_bytes = 256 + 512 * cols * 4
+    d_ws = be.alloc(ws_bytes)
+    assert be.lib.dataflow_submit_default_rms_norm_bwd_w(be.hp, CS, BF, BF, rows, cols, EPS, d_rms.ptr, d_X.ptr, d_G.ptr, d_dW.ptr, ws_bytes, d_ws.ptr) == 0
+    be.sync(CS)
+    assert int(be.read(d_ws.ptr, (1,), np.int32)[0]) == min(rows, 512)
+    want = f32_to_bf16((start + (x * g * rms[:, None].astype(np.float64)).sum(axis=0)).astype(np.float32))
+    assert (be.read(d_dW.ptr, (cols,), np.uint16) == want).all()
+
+
 def test_rms_norm_rejects_bad_shapes_and_small_workspace(backend):
     be = backend
     buf = be.alloc(4096)

@@ -154,6 +154,49 @@ def test_the_benchmark_times_the_ops_the_layer_submits(schedule, first):
     assert len(rows) == len(submitted) and all(name in work for name, _ in rows)
 
 
+NORM_OPS = ("default_rms_norm_bwd_w_BF16_BF16", "default_rms_norm_bwd_w_combine_BF16")
+NORM_FEW_ROWS = "amd_rms_norm_bwd_w_few_rows_BF16_BF16"
+
+
+@pytest.mark.parametrize("replaced", [None, *NORM_OPS])
+def test_the_norms_weight_gradient_over_few_rows_gives_way_to_a_replaced_half(replaced):
+    """one op where the table is as registration leaves it and the rows are few; two where they are not, where a half of it has
+    another implementation, and (refused or not, as before) where the workspace is too small"""
+    noting = NotingHandle(C.sizeof(HipFunction))
+    lib, hp = noting.lib, C.pointer(noting.h)
+    skeletons = {}
+    for name, setter in zip(NORM_OPS, (lambda sk: lib.dataflow_set_default_rms_norm_bwd_w_skeleton(sk, B.DATAFLOW_BF16, B.DATAFLOW_BF16),
+                                       lambda sk: lib.dataflow_set_default_rms_norm_bwd_w_combine_skeleton(sk, B.DATAFLOW_BF16))):
+        skeletons[name] = B.OpSkeleton()
+        setter(C.byref(skeletons[name]))
+    few = skeletons[NORM_FEW_ROWS] = B.OpSkeleton()
+    few.header.op_nickname = NORM_FEW_ROWS.encode()
+    few.header.num_args = 8
+    few.header.arg_dtypes = (C.c_int * B.MAX_OP_ARGS)(*([B.DATAFLOW_INT_SCALAR] * 2 + [B.DATAFLOW_FP32] + [B.DATAFLOW_BF16] * 3 + [B.DATAFLOW_INT_SCALAR, B.DATAFLOW_INT]))
+    assert lib.dataflow_do_fingerprinting(C.byref(few.header), C.sizeof(few.header), few.fingerprint) == 0
+
+    def submit(rows, workspace_bytes=1 << 20):
+        noting.names.clear()
+        assert lib.dataflow_submit_default_rms_norm_bwd_w(hp, 1, B.DATAFLOW_BF16, B.DATAFLOW_BF16, rows, 64, 1e-5, 1 << 24, 2 << 24, 3 << 24, 4 << 24,
+                                                          workspace_bytes, 5 << 24) == 0
+        return tuple(noting.names)
+
+    def insert(name, implementation, **fields):
+        fn = HipFunction(op_skeleton=skeletons[name], is_native=True, function_handle=implementation, **fields)
+        assert lib.dataflow_insert_table(C.byref(noting.h.op_table), C.cast(skeletons[name].fingerprint, C.c_void_p), C.cast(C.byref(fn), C.c_void_p)) == 0
+
+    for i, name in enumerate(NORM_OPS):
+        insert(name, 0x1000 * (i + 1))
+    assert submit(16) == NORM_OPS                                   # ops registered one by one
+    insert(NORM_FEW_ROWS, 0x4000, stands_in_for=(C.c_void_p * 3)(0x1000, 0x2000, None))
+    if replaced:
+        assert lib.dataflow_remove_table(C.byref(noting.h.op_table), C.cast(skeletons[replaced].fingerprint, C.c_void_p), None) == 0
+        insert(replaced, 0x5000)
+    expected = NORM_OPS if replaced else (NORM_FEW_ROWS,)
+    assert submit(1) == expected and submit(1536) == expected
+    assert submit(1537) == NORM_OPS and submit(0) == NORM_OPS and submit(16, 300) == NORM_OPS
+
+
 @pytest.mark.gpu
 def test_gpu_replaced_select_experts_is_the_one_that_runs():
     """registration notes the real implementations; the op sequence takes over when one of them is exchanged for the same
