@@ -109,7 +109,8 @@ def submit_route_tokens(be, layer, T, d_X, d_bias, stream_id):
 
 def replay_step_with_events(be, layer, T, d_X, d_out, d_dY, d_dX, d_bias, backward, ev, stream, fused, first=False):
     """Submits the grouped (or fused) schedule op by op (same ops, same order as amd_moe_layer_forward/_backward, all
-    on the compute stream) with an event pair around every launch; returns [(kernel class, ms)].  first: the weight-gradient
+    on the compute stream; a small layer's up-projection and activation, one op there, as the two it stands in for) with an
+    event pair around every launch; returns [(kernel class, ms)].  first: the weight-gradient
     GEMMs as AMD_MOE_FIRST_MICRO_BATCH runs them (beta = 0, no C operand)."""
     from ml_dataflow_amd import binding as B
     lib, hp, L = be.lib, be.hp, layer.L

@@ -53,6 +53,15 @@ __device__ __forceinline__ u32x4 pack8(const float f[8]) {
 	return v;
 }
 
+/* o = x1 / (1 + exp(-x1)) * x3 in fp32 (swiglu.cu:66-151) */
+__device__ __forceinline__ void swiglu8(const float x1[8], const float x3[8], float o[8]) {
+	#pragma unroll
+	for (int i = 0; i < 8; i++) {
+		float silu = x1[i] / (1.0f + __expf(-x1[i]));
+		o[i] = silu * x3[i];
+	}
+}
+
 /* sum over the 64 lanes of a wave; every lane gets the total */
 __device__ __forceinline__ float wave_sum(float v) {
 	#pragma unroll

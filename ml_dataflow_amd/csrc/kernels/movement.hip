@@ -242,11 +242,7 @@ default_swiglu_bf16_kernel(int num_rows, int num_cols, const bf16_t * x_w1, cons
 	float a[8], b[8], o[8];
 	unpack8(__builtin_nontemporal_load(((const u32x4 *) x_w1) + v), a);
 	unpack8(__builtin_nontemporal_load(((const u32x4 *) x_w3) + v), b);
-	#pragma unroll
-	for (int i = 0; i < 8; i++) {
-		float silu = a[i] / (1.0f + __expf(-a[i]));
-		o[i] = silu * b[i];
-	}
+	swiglu8(a, b, o);
 	((u32x4 *) out)[v] = pack8(o);
 }
 
@@ -596,11 +592,7 @@ amd_swiglu_strided_bf16_kernel(int num_rows, int num_cols, int x_row_stride, con
 	float a[8], b[8], o[8];
 	unpack8(__builtin_nontemporal_load(((const u32x4 *) x_w1) + src), a);
 	unpack8(__builtin_nontemporal_load(((const u32x4 *) x_w3) + src), b);
-	#pragma unroll
-	for (int i = 0; i < 8; i++) {
-		float silu = a[i] / (1.0f + __expf(-a[i]));
-		o[i] = silu * b[i];
-	}
+	swiglu8(a, b, o);
 	((u32x4 *) out)[v] = pack8(o);
 }
 

@@ -21,7 +21,7 @@ void layer_set_route_tokens_skeleton(Op_Skeleton * skeleton) {
 	dataflow_fill_skeleton(skeleton, "amd_route_tokens", DATAFLOW_BF16, DATAFLOW_NONE, 17, t);
 }
 
-static void stood_in_skeletons(Op_Skeleton skeletons[3]) {
+static void route_tokens_stood_in(Op_Skeleton skeletons[3]) {
 	dataflow_set_matmul_skeleton(&skeletons[0]);
 	dataflow_set_default_select_experts_skeleton(&skeletons[1], DATAFLOW_BF16);
 	dataflow_set_default_build_expert_mapping_skeleton(&skeletons[2]);
@@ -30,15 +30,51 @@ static void stood_in_skeletons(Op_Skeleton skeletons[3]) {
 int layer_bind_route_tokens(Dataflow_Handle * handle) {
 	Op_Skeleton skeleton, of[3];
 	layer_set_route_tokens_skeleton(&skeleton);
-	stood_in_skeletons(of);
+	route_tokens_stood_in(of);
 	return stand_in_bind(handle, &skeleton, of, 3);
 }
 
 int layer_has_route_tokens(Dataflow_Handle * handle) {
 	Op_Skeleton skeleton, of[3];
 	layer_set_route_tokens_skeleton(&skeleton);
-	stood_in_skeletons(of);
+	route_tokens_stood_in(of);
 	return stand_in_usable(handle, &skeleton, of, 3);
+}
+
+void layer_set_up_swiglu_skeleton(Op_Skeleton * skeleton) {
+	const DataflowDatatype t[12] = {DATAFLOW_INT_SCALAR, DATAFLOW_INT_SCALAR, DATAFLOW_INT_SCALAR, DATAFLOW_INT_SCALAR, DATAFLOW_INT, DATAFLOW_BF16,
+									DATAFLOW_UINT64_SCALAR, DATAFLOW_BF16, DATAFLOW_INT, DATAFLOW_INT_SCALAR, DATAFLOW_BF16, DATAFLOW_BF16};
+	dataflow_fill_skeleton(skeleton, "amd_up_swiglu", DATAFLOW_BF16, DATAFLOW_NONE, 12, t);
+}
+
+static void up_swiglu_stood_in(Op_Skeleton skeletons[2]) {
+	dataflow_set_amd_grouped_matmul_gathered_skeleton(&skeletons[0]);
+	dataflow_set_amd_swiglu_strided_skeleton(&skeletons[1], DATAFLOW_BF16);
+}
+
+int layer_bind_up_swiglu(Dataflow_Handle * handle) {
+	Op_Skeleton skeleton, of[2];
+	layer_set_up_swiglu_skeleton(&skeleton);
+	up_swiglu_stood_in(of);
+	return stand_in_bind(handle, &skeleton, of, 2);
+}
+
+int layer_has_up_swiglu(Dataflow_Handle * handle) {
+	Op_Skeleton skeleton, of[2];
+	layer_set_up_swiglu_skeleton(&skeleton);
+	up_swiglu_stood_in(of);
+	return stand_in_usable(handle, &skeleton, of, 2);
+}
+
+int layer_submit_up_swiglu(Dataflow_Handle * handle, int stream_id, int expert_dim, int model_dim, int num_rows, int num_experts,
+							 int * expert_counts_cumsum, void * w13, uint64_t expert_stride_bytes, void * X, int * expert_mapping, int num_tokens,
+							 void * x13, void * h) {
+	Op op;
+	layer_set_up_swiglu_skeleton(&op.op_skeleton);
+	void ** a = op.op_args;
+	a[0] = &expert_dim; a[1] = &model_dim; a[2] = &num_rows; a[3] = &num_experts; a[4] = &expert_counts_cumsum; a[5] = &w13; a[6] = &expert_stride_bytes;
+	a[7] = &X; a[8] = &expert_mapping; a[9] = &num_tokens; a[10] = &x13; a[11] = &h;
+	return submit(handle, &op, stream_id, "up projection and swiglu");
 }
 
 int layer_submit_route_tokens(Dataflow_Handle * handle, int stream_id, int num_tokens, int num_experts, int top_k, int model_dim,

@@ -26,4 +26,19 @@ LAYER_OPS_HIDDEN int layer_submit_route_tokens(Dataflow_Handle * handle, int str
 								uint16_t * chosen_experts, int * expert_counts, int * expert_counts_cumsum, int * host_expert_counts,
 								int * expert_mapping, int * token_mapping, uint64_t workspace_bytes, void * workspace);
 
+/* The up-projections of the fused schedule and their activation: what dataflow_submit_amd_grouped_matmul_gathered (x1 | x3 of routed row
+ * r side by side, from row expert_mapping[r] of X) and dataflow_submit_amd_swiglu_strided leave, bit for bit.  All pointers
+ * 16-byte aligned; X and one expert's w1 below 4 GiB.  Stands in for those two.
+ * Submitted for up to LAYER_UP_SWIGLU_VALUES values of x1 | x3: there the GEMM runs on tiles whose epilogue can compute the
+ * activation, one launch less in a chain of six that launches are most of (forwards, us: 256 tokens, dim 512
+ * 28.6 -> 26.6; 16 tokens, 64 experts, dim 4096 264.6 -> 258.8).  Beyond, the
+ * GEMM's persistent kernels have no room for it, and the activation's own launch streams at the rate of the memory. */
+#define LAYER_UP_SWIGLU_VALUES (1u << 23)
+LAYER_OPS_HIDDEN void layer_set_up_swiglu_skeleton(Op_Skeleton * skeleton);
+LAYER_OPS_HIDDEN int layer_bind_up_swiglu(Dataflow_Handle * handle);
+LAYER_OPS_HIDDEN int layer_has_up_swiglu(Dataflow_Handle * handle);
+LAYER_OPS_HIDDEN int layer_submit_up_swiglu(Dataflow_Handle * handle, int stream_id, int expert_dim, int model_dim, int num_rows, int num_experts,
+							 int * expert_counts_cumsum, void * w13, uint64_t expert_stride_bytes, void * X, int * expert_mapping, int num_tokens,
+							 void * x13, void * h);
+
 #endif

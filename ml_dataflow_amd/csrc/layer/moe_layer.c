@@ -256,7 +256,14 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 		 * much) and the token rows are fetched once for both products. */
 		L->saved_side_by_side = 1;
 		void * x13 = L->x1;
-		if (gather_allowed(T, D)) {
+		const int gathered = gather_allowed(T, D);
+		const uintptr_t pointers = (uintptr_t) X | (uintptr_t) L->w1 | (uintptr_t) x13 | (uintptr_t) L->kernel_workspace | (uintptr_t) L->expert_stride_bytes;
+		const int activated = gathered && (uint64_t) T * K * 2 * H <= LAYER_UP_SWIGLU_VALUES && (pointers & 15) == 0
+			&& (uint64_t) (H + 64) * D * 2u <= 0xFFFFFFFFull && layer_has_up_swiglu(h);
+		if (activated) {
+			CHECK(layer_submit_up_swiglu(h, cs, H, D, T * K, E, L->expert_counts_cumsum, L->w1, L->expert_stride_bytes, X, L->expert_mapping, T, x13, L->kernel_workspace),
+				  "failed to submit up projection and swiglu");
+		} else if (gathered) {
 			/* no dispatch copy: the GEMM's loaders fetch row expert_mapping[r] of X for routed row r themselves (the
 			 * same values reach the same multiplies, so the result is that of the copy + GEMM below, bit for bit) */
 			CHECK(dataflow_submit_amd_grouped_matmul_gathered(h, cs, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, 2 * H, D, T * K,
@@ -269,8 +276,10 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 													 E, L->expert_counts_cumsum, 1.0f, 0.0f, L->w1, L->expert_stride_bytes, L->expert_zones, NULL, x13, 0),
 				  "failed to submit grouped w1|w3 matmul");
 		}
-		CHECK(dataflow_submit_amd_swiglu_strided(h, cs, dt, T * K, H, 2 * H, x13, (uint8_t *) x13 + (uint64_t) H * el, L->kernel_workspace),
-			  "failed to submit strided swiglu");
+		if (!activated) {
+			CHECK(dataflow_submit_amd_swiglu_strided(h, cs, dt, T * K, H, 2 * H, x13, (uint8_t *) x13 + (uint64_t) H * el, L->kernel_workspace),
+				  "failed to submit strided swiglu");
+		}
 		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, D, H, T * K,
 												 E, L->expert_counts_cumsum, 1.0f, 0.0f, L->w2, L->expert_stride_bytes, L->kernel_workspace, NULL, L->expert_zones, 0),
 			  "failed to submit grouped w2 matmul");

@@ -74,10 +74,10 @@ static int launch_staged(const GemmParams & p, long grid, hipStream_t stream) {
 }
 
 /* direct-to-LDS kernel: static LDS */
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PK, bool QK, int MODE, int GATHER = GATHER_NONE>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PK, bool QK, int MODE, int GATHER = GATHER_NONE, bool SWIGLU = false>
 static int launch_direct_tile(const GemmParams & p, long grid, hipStream_t stream) {
 	constexpr int threads = WAVES_M * WAVES_N * 64;
-	hipLaunchKernelGGL((gemm_bf16_direct_kernel<BM, BN, WAVES_M, WAVES_N, PK, QK, MODE, GATHER, STAGES>), dim3((unsigned int) ((grid + 7) & ~7L)), dim3(threads), 0, stream, p);
+	hipLaunchKernelGGL((gemm_bf16_direct_kernel<BM, BN, WAVES_M, WAVES_N, PK, QK, MODE, GATHER, STAGES, SWIGLU>), dim3((unsigned int) ((grid + 7) & ~7L)), dim3(threads), 0, stream, p);
 	return check_launch();
 }
 
@@ -142,15 +142,15 @@ static int choose_tile(int mode, const GemmParams & p, long cu_count, bool persi
 }
 
 /* the direct kernel on one of its tiles */
-template <bool PK, bool QK, int MODE, int GATHER = GATHER_NONE>
+template <bool PK, bool QK, int MODE, int GATHER = GATHER_NONE, bool SWIGLU = false>
 static int launch_direct(const GemmParams & p, int which, hipStream_t stream) {
 	const long grid = grid_of(which, MODE, p);
 	switch (which) {
-		case TILE_64x32: return launch_direct_tile<64, 32, 2, 2, 4, PK, QK, MODE, GATHER>(p, grid, stream);
-		case TILE_64x64: return launch_direct_tile<64, 64, 2, 2, 4, PK, QK, MODE, GATHER>(p, grid, stream);
-		case TILE_64x128: return launch_direct_tile<64, 128, 2, 2, 3, PK, QK, MODE, GATHER>(p, grid, stream);
-		case TILE_128x128: return launch_direct_tile<128, 128, 4, 2, 3, PK, QK, MODE, GATHER>(p, grid, stream);
-		default: return launch_direct_tile<128, 128, 4, 2, 2, PK, QK, MODE, GATHER>(p, grid, stream);
+		case TILE_64x32: return launch_direct_tile<64, 32, 2, 2, 4, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
+		case TILE_64x64: return launch_direct_tile<64, 64, 2, 2, 4, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
+		case TILE_64x128: return launch_direct_tile<64, 128, 2, 2, 3, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
+		case TILE_128x128: return launch_direct_tile<128, 128, 4, 2, 3, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
+		default: return launch_direct_tile<128, 128, 4, 2, 2, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
 	}
 }
 
@@ -929,6 +929,72 @@ extern "C" int amd_grouped_matmul(Dataflow_Handle * dataflow_handle, int stream_
 	}
 	fprintf(stderr, "Error: unknown ragged dimension %d...\n", ragged);
 	return -1;
+}
+
+/* The activation behind an up-projection on the persistent kernels, as amd_swiglu_strided_bf16_kernel (kernels/movement.hip) */
+__global__ void __launch_bounds__(256) up_swiglu_kernel(const bf16_t * __restrict__ x13, bf16_t * __restrict__ h, long long rows, int half) {
+	const int per_row = half >> 3;
+	const long long v = (long long) blockIdx.x * 256 + threadIdx.x;
+	if (v >= rows * per_row) {
+		return;
+	}
+	const long long r = v / per_row;
+	const u32x4 * const x = (const u32x4 *) (x13 + r * 2 * half) + (v - r * per_row);
+	float a[8], b[8], o[8];
+	unpack8(__builtin_nontemporal_load(x), a);
+	unpack8(__builtin_nontemporal_load(x + per_row), b);
+	swiglu8(a, b, o);
+	((u32x4 *) h)[v] = pack8(o);
+}
+
+/* The layer's up-projection and its activation in one op (../layer/layer_ops.h): x1 | x3 side by side per routed row and h.  Few
+ * rows run on the direct kernel, whose epilogue then computes h; where the GEMM is large enough for the persistent kernels the
+ * activation follows in a launch of its own. */
+extern "C" int amd_up_swiglu(Dataflow_Handle * dataflow_handle, int stream_id, Op * op, void * op_extra) {
+	void ** a = op->op_args;
+	GemmParams p;
+	memset(&p, 0, sizeof(p));
+	const int half = *((int *) a[0]);
+	p.M = 2 * half;
+	p.K = *((int *) a[1]);
+	p.N = *((int *) a[2]);
+	p.num_groups = *((int *) a[3]);
+	p.cumsum = (const int *) *((uint64_t *) a[4]);
+	p.A = (const bf16_t *) *((uint64_t *) a[5]);
+	const uint64_t strideA_bytes = *((uint64_t *) a[6]);
+	p.strideA = (long long) (strideA_bytes / 2);
+	p.B = (const bf16_t *) *((uint64_t *) a[7]);
+	p.gather = (const int *) *((uint64_t *) a[8]);
+	p.gather_rows = *((int *) a[9]);
+	p.D = (bf16_t *) *((uint64_t *) a[10]);
+	p.h = (bf16_t *) *((uint64_t *) a[11]);
+	p.alpha = 1.0f;
+	const bool aligned = aligned16(p.A) && aligned16(p.B) && aligned16(p.D) && aligned16(p.h) && (strideA_bytes & 15) == 0 && (p.K & 7) == 0 && (half & 7) == 0;
+	if (half < 8 || half > (1 << 24) || p.K < 8 || p.K > (1 << 22) || p.N < 1 || p.num_groups < 1 || !p.cumsum || !p.A || !p.B || !p.gather || !p.D || !p.h || !aligned
+		|| p.gather_rows < 1 || (uint64_t) p.gather_rows * (uint64_t) p.K * 2u > 0xFFFFFFFFull || (uint64_t) (half + 64) * (uint64_t) p.K * 2u > 0xFFFFFFFFull) {
+		fprintf(stderr, "Error: bad arguments of the up-projection op (expert dim %d, model dim %d, %d rows, %d groups)...\n", half, p.K, p.N, p.num_groups);
+		return -1;
+	}
+	hipStream_t stream;
+	if (resolve_stream(dataflow_handle, stream_id, &stream)) {
+		return -1;
+	}
+	if (hipSetDevice(dataflow_handle->device_id) != hipSuccess) {
+		fprintf(stderr, "Error: hipSetDevice failed in the up-projection op...\n");
+		return -1;
+	}
+	const long cu_count = extra_cu_count(op_extra);
+	const int tile = choose_tile(MODE_RAGGED_N, p, cu_count);
+	if (tile != TILE_BIG && kernel_choice == AMD_MATMUL_KERNEL_AUTO) {
+		return launch_direct<false, false, MODE_RAGGED_N, GATHER_Q_ROWS, true>(p, tile, stream);
+	}
+	if (launch_gemm<MODE_RAGGED_N>(p, 1, 0, true, tiles_of(p.M, 256) * ((long) p.N / 256 + p.num_groups), tiles_of(p.M, 128) * ((long) p.N / 128 + p.num_groups),
+								   cu_count, stream, tiles_of(p.M, 256) * ((long) p.N / 192 + p.num_groups))) {
+		return -1;
+	}
+	const long long vectors = (long long) p.N * (half >> 3);
+	hipLaunchKernelGGL(up_swiglu_kernel, dim3((unsigned int) ((vectors + 255) / 256)), dim3(256), 0, stream, (const bf16_t *) p.D, p.h, (long long) p.N, half);
+	return check_launch();
 }
 
 /* The layer's routing in one op (../layer/layer_ops.h): router product, selection, counts, prefix sum, permutation. */

@@ -28,8 +28,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-typedef uint16_t bf16_t;
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#include "../kernels/moe_common.h"
+
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -71,6 +71,9 @@ struct GemmParams {
 	 * work-group counts the tiles of both from the device prefix sum (ragged_n_choice) and the kernel that loses returns at
 	 * once.  The bits of the two tilings, or 0: run */
 	int candidates;
+	/* the layer's up-projection with its activation (SWIGLU form of the direct kernel): A is w1 over w3, M / 2 rows each, and
+	 * h[n * M / 2 + m] = silu(D[n * M + m]) * D[n * M + M / 2 + m] */
+	bf16_t * h;
 	/* Operands copied to padded rows (single problems on the direct kernel only; 0: not padded): elements from one k-row
 	 * to the next of a k-major operand, and the k-rows a k-major operand has where K was rounded up for a k-contiguous one
 	 * (those past them read as zero, like the padding they are multiplied with) */
@@ -99,13 +102,7 @@ __device__ __forceinline__ uint32_t f2bf(float f) {
 	return bits >> 16;
 }
 
-/* two fp32 -> one packed pair of bf16 (round to nearest even) in a single v_cvt_pk_bf16_f32 */
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pack2_bf16(float lo, float hi) {
-	const f32x2_t v = {lo, hi};
-	return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
-}
+__device__ __forceinline__ uint32_t pack2_bf16(float lo, float hi) { return pack_bf16(lo, hi); }
 
 /* Element offset of 16-byte chunk c of row r inside a k-contiguous [rows][64] LDS tile.  A row is 128 bytes, so
  * two rows span the 64 banks; XOR-ing the chunk index with bits 1..3 of the row makes the sixteen 16-byte reads of
@@ -978,12 +975,52 @@ __device__ __forceinline__ bf16x8 read_fragment(const bf16_t * tile, int row_bas
 	}
 }
 
+/* The epilogue of the SWIGLU form: x1 and x3 of a row's columns sit in the two halves of the tile.  The whole tile is staged in the
+ * LDS as bf16 (rows of BM + 8 elements), then a lane takes 8 columns of both halves of a row, writes x1 and x3 and, from the rounded
+ * values, as the activation's own kernel computes it, h.  M / 2 is a multiple of 8, all three outputs 16-byte aligned. */
+template <int BM, int BN, int THREADS, int TM, int TN>
+__device__ __forceinline__ void store_swiglu_tile(const Tile & t, const GemmParams & p, f32x4_t (&acc)[TM][TN], int wm, int wn, int lane, bf16_t * staged) {
+	constexpr int PITCH = BM + 8;
+	constexpr int CHUNKS = BM / 16;                     /* of 8 columns, in a half */
+	#pragma unroll
+	for (int j = 0; j < TN; j++) {
+		#pragma unroll
+		for (int i = 0; i < TM; i++) {
+			u32x2 v;
+			v.x = pack2_bf16(acc[i][j][0], acc[i][j][1]);
+			v.y = pack2_bf16(acc[i][j][2], acc[i][j][3]);
+			*((u32x2 *) (staged + (wn + j * 16 + (lane & 15)) * PITCH + wm + i * 16 + ((lane >> 4) << 2))) = v;
+		}
+	}
+	__syncthreads();
+	const int half = t.M >> 1;
+	bf16_t * const h = p.h + ((t.D - p.D) >> 1);        /* of this group's first row */
+	for (int item = threadIdx.x; item < BN * CHUNKS; item += THREADS) {
+		const int r = item / CHUNKS, c = item % CHUNKS;
+		const int n = t.n0 + r, m = (t.m0 >> 1) + c * 8;
+		if (n >= t.N || m >= half) {
+			continue;
+		}
+		const u32x4 x1 = *((const u32x4 *) (staged + r * PITCH + c * 8)), x3 = *((const u32x4 *) (staged + r * PITCH + BM / 2 + c * 8));
+		float a[8], b[8], o[8];
+		unpack8(x1, a);
+		unpack8(x3, b);
+		swiglu8(a, b, o);
+		bf16_t * const d = t.D + (long long) n * t.M + m;
+		*((u32x4 *) d) = x1;
+		*((u32x4 *) (d + half)) = x3;
+		*((u32x4 *) (h + (long long) n * half + m)) = pack8(o);
+	}
+}
+
 /* STAGES LDS stages keep STAGES - 1 k-tiles in flight per work-group.  Problems of few tiles are short streams of operand
  * bytes with nothing to reuse: a k-tile costs them the memory round trip divided by the k-tiles in flight, so they run on
  * three or four stages of small tiles (1408 x 2048 x 256: 30 us with 128 x 128 tiles and two stages, 23 us with four, 10.5
  * us with 64 x 64 tiles and four; eight stages leave room for one work-group per compute unit and lose what they gain).
- * Two stages where two work-groups of a compute unit hide each other's waits (the host's table of tiles). */
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool P_KMAJOR, bool Q_KMAJOR, int MODE, int GATHER = 0, int STAGES = 2>
+ * Two stages where two work-groups of a compute unit hide each other's waits (the host's table of tiles).
+ * SWIGLU: the first half of a tile's rows of P are rows of w1, the second half the same rows of w3 (GemmParams::h); a lane's two
+ * loads of P per k-tile are then M / 2 rows apart. */
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool P_KMAJOR, bool Q_KMAJOR, int MODE, int GATHER = 0, int STAGES = 2, bool SWIGLU = false>
 __global__ void __launch_bounds__(WAVES_M * WAVES_N * 64)
 gemm_bf16_direct_kernel(GemmParams p) {
 	static_assert(STAGES >= 2 && STAGES <= 8, "at least two stages");
@@ -1046,6 +1083,11 @@ gemm_bf16_direct_kernel(GemmParams p) {
 	const int k_rows = MODE == MODE_SINGLE && p.k_rows ? p.k_rows : t.K;
 	if (GATHER == GATHER_P_KROWS) {
 		ldP.init_gather_k(t.P, t.Pmap, t.m0, t.M, t.K, p.gather_rows);
+	} else if (SWIGLU) {
+		static_assert(!SWIGLU || (!P_KMAJOR && MODE == MODE_RAGGED_N && THREADS / 8 == BM / 2), "two loads of P per lane and k-tile, one of either half");
+		static_assert(!SWIGLU || BN * (BM + 8) <= STAGES * (BM + BN) * BK, "the staged tile must fit in the stages");
+		ldP.init(t.P, t.m0 >> 1, t.M, t.K);
+		ldP.step = (uint32_t) (t.M >> 1) * (uint32_t) t.K * 2u;
 	} else {
 		ldP.init(t.P, t.m0, t.M, P_KMAJOR ? k_rows : t.K, MODE == MODE_SINGLE && p.pitchA ? p.pitchA : t.M);
 	}
@@ -1132,7 +1174,11 @@ gemm_bf16_direct_kernel(GemmParams p) {
 		store_partial<TM, TN>(t, p.partial + (long long) split * t.M * t.N, acc, wm, wn, lane);
 		return;
 	}
-	write_tile<TM, TN>(t, p, acc, wm, wn, lane, wave, (void *) stages);
+	if constexpr (SWIGLU) {
+		store_swiglu_tile<BM, BN, THREADS, TM, TN>(t, p, acc, wm, wn, lane, stage0);
+	} else {
+		write_tile<TM, TN>(t, p, acc, wm, wn, lane, wave, (void *) stages);
+	}
 }
 
 /* --------------------------------------------------------------------------------------------

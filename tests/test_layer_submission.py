@@ -154,6 +154,45 @@ def test_the_benchmark_times_the_ops_the_layer_submits(schedule, first):
     assert len(rows) == len(submitted) and all(name in work for name, _ in rows)
 
 
+UP_OPS = ["amd_grouped_matmul_gathered", "amd_swiglu_strided_BF16"]
+
+
+@pytest.mark.parametrize("replaced", [None, *UP_OPS])
+def test_the_up_projection_op_gives_way_to_a_replaced_one(replaced):
+    """the fused schedule submits gather, GEMM and activation as one op where the table is as registration leaves it and the layer
+    is small; as two where one of them has another implementation, or a limit of the op does not hold"""
+    noting = NotingHandle(C.sizeof(HipFunction))
+    lib, skeletons = noting.lib, {}
+    for name, setter in zip(UP_OPS, (lib.dataflow_set_amd_grouped_matmul_gathered_skeleton, lambda sk: lib.dataflow_set_amd_swiglu_strided_skeleton(sk, B.DATAFLOW_BF16))):
+        skeletons[name] = B.OpSkeleton()
+        setter(C.byref(skeletons[name]))
+    both = skeletons["amd_up_swiglu_BF16"] = B.OpSkeleton()
+    both.header.op_nickname = b"amd_up_swiglu_BF16"
+    both.header.num_args = 12
+    both.header.arg_dtypes = (C.c_int * B.MAX_OP_ARGS)(*([B.DATAFLOW_INT_SCALAR] * 4 + [B.DATAFLOW_INT, B.DATAFLOW_BF16, B.DATAFLOW_UINT64_SCALAR, B.DATAFLOW_BF16, B.DATAFLOW_INT,
+                                                                                       B.DATAFLOW_INT_SCALAR, B.DATAFLOW_BF16, B.DATAFLOW_BF16]))
+    assert lib.dataflow_do_fingerprinting(C.byref(both.header), C.sizeof(both.header), both.fingerprint) == 0
+
+    def insert(name, implementation, **fields):
+        fn = HipFunction(op_skeleton=skeletons[name], is_native="swiglu_strided" in name, **{"function_handle" if "swiglu_strided" in name else "hip_external_func": implementation}, **fields)
+        assert lib.dataflow_insert_table(C.byref(noting.h.op_table), C.cast(skeletons[name].fingerprint, C.c_void_p), C.cast(C.byref(fn), C.c_void_p)) == 0
+
+    def up(**changes):
+        return [name for name in noting.forward(B.AMD_MOE_FUSED, **changes) if name in skeletons]
+
+    for i, name in enumerate(UP_OPS):
+        insert(name, 0x1000 * (i + 1))
+    assert up() == UP_OPS
+    insert("amd_up_swiglu_BF16", 0x4000, stands_in_for=(C.c_void_p * 3)(0x1000, 0x2000, None))
+    if replaced:
+        assert lib.dataflow_remove_table(C.byref(noting.h.op_table), C.cast(skeletons[replaced].fingerprint, C.c_void_p), None) == 0
+        insert(replaced, 0x5000)
+    assert up() == (UP_OPS if replaced else ["amd_up_swiglu_BF16"])
+    assert up(x1=(7 << 24) + 8) == UP_OPS and up(kernel_workspace=(9 << 24) + 8) == UP_OPS     # off a 16-byte boundary
+    large = 1 << 16                                                                            # T K 2 H = 10 M values
+    assert up(expert_dim=large, w3=(2 << 24) + large * D * 2, w1=2 << 24, dw1=3 << 24, dw3=(3 << 24) + large * D * 2) == UP_OPS
+
+
 NORM_OPS = ("default_rms_norm_bwd_w_BF16_BF16", "default_rms_norm_bwd_w_combine_BF16")
 NORM_FEW_ROWS = "amd_rms_norm_bwd_w_few_rows_BF16_BF16"
 
