@@ -92,11 +92,14 @@ static long tiles_of(long extent, long tile) { return (extent + tile - 1) / tile
  * alone), the persistent 256 x 256: 1.1-1.4.  So the cheapest tile is the one with the least (rounds of tiles over the
  * compute units) x (cost of a k-tile), small tiles while they still fit one round and larger ones behind that.  1408 x
  * 2048 x 256 takes 10 us on 64 x 64 tiles (29 on 128 x 128 with one k-tile in flight, which this replaced), 4096 x 4096 x
- * 512 31 us on 64 x 128 (55), 4096 x 4096 x 2048 66 us on pairs of 128 x 128 (92 on the persistent kernel).  The rule has
- * no term per tile and is applied at every K: how the tiles compare where K is so short that a tile's epilogue takes as
- * long as its k-tiles (short groups of a ragged-K launch) has not been measured. */
+ * 512 31 us on 64 x 128 (55), 4096 x 4096 x 2048 66 us on pairs of 128 x 128 (92 on the persistent kernel).  The
+ * costs are in hundredths of a microsecond.  A single problem's rounds are charged half a microsecond each on top, and a
+ * partial last round of the persistent kernel 60 % of a whole one plus the rest by its share (270 tiles of 256 x 256, 3840 x
+ * 3328 x 4582, take 104 us, in pairs of 128 x 128 146).  Ragged launches have no term per tile: how the tiles compare
+ * where K is so short that a tile's epilogue takes as long as its k-tiles (short groups of a ragged-K launch) has not been measured. */
 enum { TILE_64x32, TILE_64x64, TILE_64x128, TILE_128x128, TILE_128x128_PAIR, TILE_BIG, NUM_TILES };
 static const struct { int bm, bn, cost; } TILES[NUM_TILES] = {{64, 32, 21}, {64, 64, 25}, {64, 128, 36}, {128, 128, 58}, {128, 128, 50}, {256, 256, 130}};
+#define TILE_ROUND_COST 50
 #define TILE_PAIR_COST_ALONE 62      /* of a k-tile of the pair's tile where it has the compute unit to itself, or its lines come from HBM */
 
 /* tiles of the launch for tile `which`.  Ragged N: the group sizes are on the device; a group of the mean size has on
@@ -122,7 +125,23 @@ static long grid_of(int which, int mode, const GemmParams & p) {
 	return tiles_of(p.M, TILES[which].bm) * ((long) p.N / TILES[which].bn + (p.N < p.num_groups ? p.N : p.num_groups));
 }
 
-static int choose_tile(int mode, const GemmParams & p, long cu_count, bool persistent_ok = true) {
+static long tile_cost(int which, int mode, const GemmParams & p, long cu_count) {
+	const long tiles = tiles_in_launch(which, mode, p);
+	const bool alone = which == TILE_128x128_PAIR && (tiles <= cu_count || mode == MODE_RAGGED_N);
+	const long cost = alone ? TILE_PAIR_COST_ALONE : TILES[which].cost;
+	if (mode != MODE_SINGLE) {
+		return tiles_of(tiles, cu_count) * cost;
+	}
+	const long round = tiles_of(p.K, BK) * cost + TILE_ROUND_COST;
+	const long full = tiles / cu_count, left = tiles % cu_count;
+	if (which == TILE_BIG && full > 0) {
+		return full * round + (left ? round * (3 * cu_count + 2 * left) / (5 * cu_count) : 0);
+	}
+	return (full + (left ? 1 : 0)) * round;
+}
+
+/* the cheapest tile; `cost`: what it costs (single problems: hundredths of a microsecond) */
+static int choose_tile(int mode, const GemmParams & p, long cu_count, bool persistent_ok = true, long * cost = NULL) {
 	const bool big_ok = persistent_ok && p.M >= 256 && (mode == MODE_RAGGED_N || p.N >= 256);
 	int best = TILE_64x32;
 	long best_cost = 0;
@@ -130,13 +149,14 @@ static int choose_tile(int mode, const GemmParams & p, long cu_count, bool persi
 		if (which == TILE_BIG && !big_ok) {
 			continue;
 		}
-		const long tiles = tiles_in_launch(which, mode, p);
-		const bool alone = which == TILE_128x128_PAIR && (tiles <= cu_count || mode == MODE_RAGGED_N);
-		const long cost = tiles_of(tiles, cu_count) * (alone ? TILE_PAIR_COST_ALONE : TILES[which].cost);
-		if (which == 0 || cost < best_cost) {
+		const long c = tile_cost(which, mode, p, cu_count);
+		if (which == 0 || c < best_cost) {
 			best = which;
-			best_cost = cost;
+			best_cost = c;
 		}
+	}
+	if (cost) {
+		*cost = best_cost;
 	}
 	return best;
 }
@@ -154,23 +174,24 @@ static int launch_direct(const GemmParams & p, int which, hipStream_t stream) {
 	}
 }
 
-/* The partial products of a split along K (few tiles): the direct kernel with four stages, on 64 x 64 tiles where one side
- * has no more rows than that (the router's GEMMs of up to 64 experts: half of a 128 x 128 tile would be padding) */
-static int launch_split(const GemmParams & p, int transa, int transb, hipStream_t stream) {
+/* The partial products of a split along K, on one of the direct kernel's tiles with more than two stages */
+template <bool PK, bool QK>
+static int launch_split_layout(const GemmParams & p, int tile, hipStream_t stream) {
+	const long grid = tiles_in_launch(tile, MODE_SINGLE, p) * p.split_k;
+	switch (tile) {
+		case TILE_64x32: return launch_direct_tile<64, 32, 2, 2, 4, PK, QK, MODE_SINGLE>(p, grid, stream);
+		case TILE_64x64: return launch_direct_tile<64, 64, 2, 2, 4, PK, QK, MODE_SINGLE>(p, grid, stream);
+		case TILE_64x128: return launch_direct_tile<64, 128, 2, 2, 3, PK, QK, MODE_SINGLE>(p, grid, stream);
+		default: return launch_direct_tile<128, 128, 2, 2, 4, PK, QK, MODE_SINGLE>(p, grid, stream);
+	}
+}
+static int launch_split(const GemmParams & p, int tile, int transa, int transb, hipStream_t stream) {
 	const bool pk = !transa;
 	const bool qk = transb != 0;
-	const bool narrow = p.M <= 64 || p.N <= 64;
-	const long tiles = narrow ? tiles_of(p.M, 64) * tiles_of(p.N, 64) : tiles_of(p.M, 128) * tiles_of(p.N, 128);
-	const long grid = tiles * p.split_k;
-#define SPLIT(PK, QK) do { \
-		return narrow ? launch_direct_tile<64, 64, 2, 2, 4, PK, QK, MODE_SINGLE>(p, grid, stream) \
-					  : launch_direct_tile<128, 128, 2, 2, 4, PK, QK, MODE_SINGLE>(p, grid, stream); \
-	} while (0)
-	if (!pk && !qk) { SPLIT(false, false); }
-	if (pk && !qk) { SPLIT(true, false); }
-	if (pk && qk) { SPLIT(true, true); }
-	SPLIT(false, true);
-#undef SPLIT
+	if (!pk && !qk) { return launch_split_layout<false, false>(p, tile, stream); }
+	if (pk && !qk) { return launch_split_layout<true, false>(p, tile, stream); }
+	if (pk && qk) { return launch_split_layout<true, true>(p, tile, stream); }
+	return launch_split_layout<false, true>(p, tile, stream);
 }
 
 /* streaming kernel: one persistent work-group per compute unit (LDS allows no more), a multiple of 8 so every die gets the same share */
@@ -522,41 +543,80 @@ static long extra_cu_count(void * op_extra) {
 	return op_extra ? ((MatmulExtra *) op_extra)->cu_count : 256;
 }
 
-/* Few tiles and a long K (the router's GEMMs: 64 experts on one side): split K over the idle compute units, fp32 partial
- * sums in `workspace`, added up by the pass behind.  Without a workspace that is large enough (and 16-byte aligned) the
- * problem runs unsplit; `must_fit`: that is an error instead.  1 and the split in `p`, 0: unsplit, -1: error. */
-static int plan_split(GemmParams & p, bool direct, float * workspace, uint64_t workspace_bytes, long cu_count, bool must_fit) {
-	const bool big = tiles_of(p.M, 256) * tiles_of(p.N, 256) >= cu_count / 2 && p.M >= 256 && p.N >= 256;     /* enough tiles as it is */
+/* Few tiles and a long K (the router's GEMMs: up to 64 experts on one side; projections of few tokens): K split over the
+ * compute units that the tiles leave idle, fp32 partial sums in `workspace` (16-byte aligned), added up by the pass behind.
+ * Split where the cheapest tile and number of splits that the workspace holds cost less than the problem unsplit: the k-tiles
+ * of a split at the tile's cost (the 128 x 128 tile has four waves here: 0.66), 4 us for the pass behind and its 3 TB/s over the partial
+ * sums.  Over 310 problems (8-4096 columns, 16-30000 tokens, K 64-30000) it takes 2 % longer than the best of all tiles and splits; splits
+ * over all idle compute units wherever there were any, on 128 x 128 tiles, took 15 % longer.  1792 x 896 x 937, us: 8.0 unsplit on
+ * 64 x 128 tiles, 19.9 split in two; 2176 x 19234 x 64: 20.9 in six on 64 x 64, 67.9 unsplit.
+ * The router's logits (up to 64 rows of k-contiguous weights) are charged 1 us for the pass and a quarter for each split: the layer's
+ * routing adds up their partial sums in its selection, whose few work-groups wait for a split's loads behind the last ones'.
+ * 0: unsplit; otherwise the split in `p`, and its tile + 1. */
+#define SPLIT_PASS_COST 400
+#define SPLIT_LOGITS_PASS_COST 100
+#define SPLIT_LOGITS_COST 25
+#define SPLIT_LOGITS_MAX_ROWS 64
+#define SPLIT_BYTES_PER_COST 30000          /* 3 TB/s */
+static int plan_split(GemmParams & p, int transa, int transb, bool direct, float * workspace, uint64_t workspace_bytes, long cu_count) {
+	static const int SPLITS[] = {2, 3, 4, 6, 8, 12, 16, 24, 32, 48};
 	const long k_tiles = tiles_of(p.K, BK);
-	long splits = direct && !big ? cu_count / (tiles_of(p.M, 128) * tiles_of(p.N, 128)) : 1;
-	if (splits < 2 || k_tiles < 8 || !workspace || (((uintptr_t) workspace) & 15)) {
+	if (!direct || k_tiles < 4 || !workspace || (((uintptr_t) workspace) & 15)) {
 		return 0;
 	}
-	long per = tiles_of(k_tiles, splits);
-	per = per < 4 ? 4 : (per + 3) & ~3L;                /* at least as many as the kernel's stages */
-	splits = tiles_of(k_tiles, per);
 	const uint64_t count = (uint64_t) p.M * (uint64_t) p.N;
-	if (splits < 2) {
-		return 0;
-	}
-	if (workspace_bytes / 4 / (uint64_t) splits < count) {
-		if (must_fit) {
-			fprintf(stderr, "Error: this %d x %d x %d matmul splits along K into %ld parts of %lu partial sums each, more than the %lu-byte scratch holds; use the matmul op with a workspace...\n",
-					p.M, p.K, p.N, splits, (unsigned long) count, (unsigned long) workspace_bytes);
-			return -1;
+	const bool logits = transa && !transb && p.M <= SPLIT_LOGITS_MAX_ROWS;
+	long least;
+	choose_tile(MODE_SINGLE, p, cu_count, true, &least);
+	int best = 0;
+	for (int tile = TILE_64x32; tile <= TILE_128x128; tile++) {
+		const long tiles = tiles_in_launch(tile, MODE_SINGLE, p);
+		const long cost_of_k_tile = tile == TILE_128x128 ? 66 : TILES[tile].cost;
+		for (int splits_wanted : SPLITS) {
+			const long per = tiles_of(k_tiles, splits_wanted);
+			const long splits = tiles_of(k_tiles, per);
+			if (per < 2 || splits < 2 || tiles * splits > 4 * cu_count || workspace_bytes / 4 / (uint64_t) splits < count) {
+				continue;
+			}
+			const long cost = tiles_of(tiles * splits, cu_count) * (per * cost_of_k_tile + TILE_ROUND_COST) + (logits ? SPLIT_LOGITS_PASS_COST + splits * SPLIT_LOGITS_COST : SPLIT_PASS_COST)
+				+ (long) ((uint64_t) splits * count * 4 / SPLIT_BYTES_PER_COST);
+			if (cost < least) {
+				least = cost;
+				best = tile + 1;
+				p.split_k = (int) splits;
+				p.kt_per_split = (int) per;
+			}
 		}
-		return 0;
 	}
-	p.partial = workspace;
-	p.split_k = (int) splits;
-	p.kt_per_split = (int) per;
-	return 1;
+	if (best) {
+		p.partial = workspace;
+	}
+	return best;
+}
+
+/* amd_matmul_no_alloc's limit: a problem whose 128 x 128 tiles leave half of the compute units idle, with a K of eight k-tiles or
+ * more, needs room for the partial sums of a split over those (a multiple of four k-tiles each) */
+static bool beyond_scratch(const GemmParams & p, bool direct, uint64_t scratch_bytes, long cu_count) {
+	const long k_tiles = tiles_of(p.K, BK);
+	const bool big = tiles_of(p.M, 256) * tiles_of(p.N, 256) >= cu_count / 2 && p.M >= 256 && p.N >= 256;
+	long splits = direct && !big ? cu_count / (tiles_of(p.M, 128) * tiles_of(p.N, 128)) : 1;
+	if (splits < 2 || k_tiles < 8) {
+		return false;
+	}
+	const long per = tiles_of(k_tiles, splits);
+	splits = tiles_of(k_tiles, per < 4 ? 4 : (per + 3) & ~3L);
+	if (splits < 2 || scratch_bytes / 4 / (uint64_t) splits >= (uint64_t) p.M * (uint64_t) p.N) {
+		return false;
+	}
+	fprintf(stderr, "Error: this %d x %d x %d matmul may split along K into %ld parts of %lu partial sums each, more than the %lu-byte scratch holds; use the matmul op with a workspace...\n",
+			p.M, p.K, p.N, splits, (unsigned long) p.M * (unsigned long) p.N, (unsigned long) scratch_bytes);
+	return true;
 }
 
 /* the pass behind the partial products: D from their sums */
 static int launch_split_reduce(const GemmParams & p, hipStream_t stream) {
 	const uint64_t count = (uint64_t) p.M * (uint64_t) p.N;
-	const long blocks = (long) ((count + 255) / 256);
+	const long blocks = (long) ((count + 1023) / 1024);
 	hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned int) (blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream,
 					   (const float *) p.partial, p.split_k, (long long) count, p.alpha, p.beta, p.C, p.D);
 	return check_launch();
@@ -569,8 +629,7 @@ static int launch_split_reduce(const GemmParams & p, hipStream_t stream) {
  * 93.  A copy with its rows padded to a multiple of 8 elements (zeros) in the caller's workspace costs a pass over that
  * operand (4-6 us here), and the copy then runs on the direct kernel, split along K where the matmul op splits.  A training step of
  * that layer (dim 1024, top 8, expert dim 640) takes 5582 us instead of 9998, one of 1132 tokens and 59 experts 717 instead of
- * 792.  Below PAD_MIN_STEPS rounds of staged tiles x k-tiles the staged kernel is done by the time a second launch starts. */
-#define PAD_MIN_STEPS 2
+ * 792; also where the staged kernel has one k-tile to do it takes 12 us, copy and product 10. */
 
 __global__ void __launch_bounds__(256) pad_rows_kernel(const bf16_t * __restrict__ src, long long rows, int extent, int pitch, u32x4 * __restrict__ dst) {
 	const int chunks = pitch >> 3;                       /* 16-byte chunks of a padded row */
@@ -591,9 +650,8 @@ __global__ void __launch_bounds__(256) pad_rows_kernel(const bf16_t * __restrict
 
 /* Copies of the operands of `p` that need one, at the start of the workspace, which is advanced past them; `p` then
  * describes the padded problem.  1: done, 0: does not apply or does not fit (`p` as it was), -1: error. */
-static int pad_operands(GemmParams & p, int transa, int transb, uint8_t *& workspace, uint64_t & workspace_bytes, long cu_count, hipStream_t stream) {
-	if (!workspace || (((uintptr_t) workspace) & 15) || p.K < 1
-		|| tiles_of(tiles_of(p.M, 128) * tiles_of(p.N, 128), cu_count) * tiles_of(p.K, BK) < PAD_MIN_STEPS) {
+static int pad_operands(GemmParams & p, int transa, int transb, uint8_t *& workspace, uint64_t & workspace_bytes, hipStream_t stream) {
+	if (!workspace || (((uintptr_t) workspace) & 15) || p.K < 1) {
 		return 0;
 	}
 	const bool copy_a = !operand_direct_ok(p.A, !transa, p.M, p.K, 0), copy_b = !operand_direct_ok(p.B, transb != 0, p.N, p.K, 0);
@@ -649,8 +707,7 @@ static int launch_padded(const GemmParams & p, int transa, int transb, long cu_c
 }
 
 /* shared by amd_matmul and amd_matmul_no_alloc: checks, kernel choice, launch.  `workspace` (may be NULL) holds the fp32
- * partial sums of a split along K; `must_fit`: a split that the workspace cannot hold is an error instead of running
- * unsplit */
+ * partial sums of a split along K; `must_fit`: a split that the workspace cannot hold is an error (beyond_scratch) */
 static int run_matmul(Dataflow_Handle * dataflow_handle, int stream_id, GemmParams & p, int transa, int transb,
 					  uint8_t * workspace, uint64_t workspace_bytes, long cu_count, bool must_fit) {
 	if (p.M < 0 || p.N < 0 || p.K < 0 || !p.D || ((p.M > 0 && p.N > 0 && p.K > 0) && (!p.A || !p.B))) {
@@ -671,17 +728,16 @@ static int run_matmul(Dataflow_Handle * dataflow_handle, int stream_id, GemmPara
 	const bool direct = operand_direct_ok(p.A, !transa, p.M, p.K, 0) && operand_direct_ok(p.B, transb != 0, p.N, p.K, 0);
 	const long grid_big = tiles_of(p.M, 256) * tiles_of(p.N, 256);
 	const long grid_small = tiles_of(p.M, 128) * tiles_of(p.N, 128);
-	const int padded = direct ? 0 : pad_operands(p, transa, transb, workspace, workspace_bytes, cu_count, stream);
+	const int padded = direct ? 0 : pad_operands(p, transa, transb, workspace, workspace_bytes, stream);
 	if (padded < 0) {
 		return -1;
 	}
-	/* a padded problem whose split does not fit runs unsplit: it was never refused for that */
-	const int split = plan_split(p, direct || padded, (float *) workspace, workspace_bytes, cu_count, must_fit && !padded);
-	if (split < 0) {
+	if (must_fit && !padded && beyond_scratch(p, direct, workspace_bytes, cu_count)) {
 		return -1;
 	}
+	const int split = plan_split(p, transa, transb, direct || padded, (float *) workspace, workspace_bytes, cu_count);
 	if (split) {
-		if (launch_split(p, transa, transb, stream)) {
+		if (launch_split(p, split - 1, transa, transb, stream)) {
 			return -1;
 		}
 		return launch_split_reduce(p, stream);
@@ -1054,8 +1110,9 @@ extern "C" int amd_route_tokens(Dataflow_Handle * dataflow_handle, int stream_id
 	/* The product is split where the matmul op splits it, by the whole workspace: another order of the sums would be another
 	 * rounding of the logits.  Selection adds up the partial sums itself if the counts fit behind them; if they do not, the
 	 * sums are reduced first and the counts then overwrite them. */
-	if (plan_split(p, direct, (float *) workspace, workspace_bytes, cu_count, false)) {
-		if (launch_split(p, 1, 0, stream)) {
+	const int split = plan_split(p, 1, 0, direct, (float *) workspace, workspace_bytes, cu_count);
+	if (split) {
+		if (launch_split(p, split - 1, 1, 0, stream)) {
 			return -1;
 		}
 		const uint64_t partial_bytes = ((uint64_t) p.split_k * (uint64_t) r.T * (uint64_t) r.E * sizeof(float) + 255) & ~255UL;

@@ -66,7 +66,7 @@ struct GemmParams {
 	 * (no alpha, beta or C) to partial[ks][n * M + m]; splitk_reduce_kernel turns them into D */
 	float * partial;
 	int split_k;                   /* 0 or 1: off */
-	int kt_per_split;              /* a multiple of 4, as the host plans it; the kernel takes any */
+	int kt_per_split;
 	/* A ragged-N launch without C goes out on two tilings where even and very uneven groups would be best on different ones; every
 	 * work-group counts the tiles of both from the device prefix sum (ragged_n_choice) and the kernel that loses returns at
 	 * once.  The bits of the two tilings, or 0: run */
@@ -491,17 +491,39 @@ __device__ __forceinline__ void store_partial(const Tile & t, float * dst, f32x4
 	}
 }
 
-/* D = bf16(alpha * sum over splits of partial + beta * C); one element per thread and step, neighbours coalesce */
+/* D = bf16(alpha * sum over splits of partial + beta * C), the splits in order.  Four elements per lane and step where the
+ * arrays allow 16-byte accesses, four splits' loads in flight: a launch is a chain of memory round trips, not of bytes. */
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float * __restrict__ partial, int splits, long long count,
 															  float alpha, float beta, const bf16_t * C, bf16_t * D) {
 	const long long stride = (long long) gridDim.x * blockDim.x;
-	for (long long i = (long long) blockIdx.x * blockDim.x + threadIdx.x; i < count; i += stride) {
+	const long long first = (long long) blockIdx.x * blockDim.x + threadIdx.x;
+	const bool use_c = C != nullptr && beta != 0.0f;
+	if ((count & 3) == 0 && (((uintptr_t) D) & 7) == 0 && (!use_c || (((uintptr_t) C) & 7) == 0)) {
+		for (long long i = first; i < (count >> 2); i += stride) {
+			const u32x2 c = use_c ? ((const u32x2 *) C)[i] : u32x2{0u, 0u};
+			f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+			#pragma unroll 4
+			for (int s = 0; s < splits; s++) {
+				sum += *((const f32x4_t *) (partial + (long long) s * count + 4 * i));
+			}
+			f32x4_t r = alpha * sum;
+			if (use_c) {
+				r.x = __builtin_fmaf(beta, bf2f(c.x & 0xffffu), r.x);
+				r.y = __builtin_fmaf(beta, bf2f(c.x >> 16), r.y);
+				r.z = __builtin_fmaf(beta, bf2f(c.y & 0xffffu), r.z);
+				r.w = __builtin_fmaf(beta, bf2f(c.y >> 16), r.w);
+			}
+			((u32x2 *) D)[i] = u32x2{pack2_bf16(r.x, r.y), pack2_bf16(r.z, r.w)};
+		}
+		return;
+	}
+	for (long long i = first; i < count; i += stride) {
 		float sum = 0.0f;
 		for (int s = 0; s < splits; s++) {
 			sum += partial[(long long) s * count + i];
 		}
 		float r = alpha * sum;
-		if (C != nullptr && beta != 0.0f) {
+		if (use_c) {
 			r = __builtin_fmaf(beta, bf2f(C[i]), r);
 		}
 		D[i] = (bf16_t) f2bf(r);

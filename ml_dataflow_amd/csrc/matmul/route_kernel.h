@@ -90,13 +90,30 @@ __device__ __forceinline__ void route_stage_quads(const RouteParams & p, uint32_
 				}
 			}
 		} else if (partial) {
-			for (int s = 0; s < p.splits; s++) {
+			/* rows that are no whole quads: element loads, as many in flight (55 experts, 80 tokens: 19 us one split behind the other) */
+			const long long last = (long long) p.splits * count - 1;
+			for (int s0 = 0; s0 < p.splits; s0 += SPLITS) {
+				float q[SPLITS][AHEAD][4];
 				#pragma unroll
-				for (int u = 0; u < AHEAD; u++) {
+				for (int s = 0; s < SPLITS; s++) {
 					#pragma unroll
-					for (int j = 0; j < 4; j++) {
-						const long long x = (long long) s * count + at[u] + j;
-						sum[u][j] += x < (long long) p.splits * count ? partial[x] : 0.0f;      /* past the row's end: not used */
+					for (int u = 0; u < AHEAD; u++) {
+						#pragma unroll
+						for (int j = 0; j < 4; j++) {
+							q[s][u][j] = partial[min((long long) min(s0 + s, p.splits - 1) * count + at[u] + j, last)];      /* past the row's end: not used */
+						}
+					}
+				}
+				#pragma unroll
+				for (int s = 0; s < SPLITS; s++) {
+					if (s0 + s < p.splits) {
+						#pragma unroll
+						for (int u = 0; u < AHEAD; u++) {
+							#pragma unroll
+							for (int j = 0; j < 4; j++) {
+								sum[u][j] += q[s][u][j];
+							}
+						}
 					}
 				}
 			}

@@ -498,6 +498,33 @@ def test_matmul_split_k_through_the_workspace(backend, oracle, transa, transb, M
     check_matmul(got, O.matmul(oracle, transa, transb, M, K, N, A, Bm, alpha=0.5, beta=1.0, Cin=Cin), K)
 
 
+@pytest.mark.parametrize("transa,transb,M,K,N", [
+    (1, 0, 56, 3776, 104), (0, 1, 2624, 5656, 56), (1, 0, 3776, 3968, 120), (1, 0, 128, 8192, 2048),      # split on 64 x 32, 64 x 64, 64 x 128 tiles
+    (0, 0, 1408, 3264, 184), (0, 0, 576, 3904, 98), (0, 1, 56, 1032, 1008),                              # partial last tiles and splits
+    (1, 0, 57, 2048, 101), (0, 0, 72, 1544, 37)])                                                        # an odd number of results
+def test_matmul_split_tiles_and_their_sum(backend, oracle, transa, transb, M, K, N):
+    """The tiles a split along K runs on and the pass that adds up its partial sums, in quads and one by one, with and without C,
+    and with C and D off an 8-byte boundary."""
+    print("case split tile ta=%d tb=%d M=%d K=%d N=%d" % (transa, transb, M, K, N), flush=True)
+    be, rng = backend, np.random.default_rng(M + K + N)
+    A = normal_bf16(rng, (M, K) if transa else (K, M))
+    Bm = normal_bf16(rng, (K, N) if transb else (N, K), 0.05)
+    Cin = normal_bf16(rng, (N, M))
+    big = 64 * M * N * 4 + 4 * (M + N + 64) * (K + 64)
+    plain, scaled = O.matmul(oracle, transa, transb, M, K, N, A, Bm), O.matmul(oracle, transa, transb, M, K, N, A, Bm, alpha=0.5, beta=1.0, Cin=Cin)
+    check_matmul(run_gpu_matmul(be, transa, transb, M, K, N, A, Bm, 1.0, 0.0, None, big), plain, K)
+    got = run_gpu_matmul(be, transa, transb, M, K, N, A, Bm, 0.5, 1.0, Cin, big)
+    check_matmul(got, scaled, K)
+    d_A, d_B, d_D, d_ws = be.upload(A), be.upload(Bm), be.upload(np.concatenate([[np.uint16(7)], Cin.reshape(-1)]).astype(np.uint16)), be.alloc(big)
+    assert be.lib.dataflow_submit_matmul(be.hp, CS, BF, BF, BF, BF, B.DATAFLOW_FP32, transa, transb, M, K, N, 0.5, 1.0,
+                                         d_A.ptr, d_B.ptr, d_D.ptr + 2, d_D.ptr + 2, big, d_ws.ptr) == 0
+    be.sync(CS)
+    after = be.read(d_D.ptr, (N * M + 1,), np.uint16)
+    assert after[0] == 7 and (after[1:].reshape(N, M) == got).all()        # the same sums, rounded once
+    for buf in (d_A, d_B, d_D, d_ws):
+        buf.free()
+
+
 @pytest.mark.parametrize("transa,transb", [(1, 0), (0, 0), (0, 1), (1, 1)])
 @pytest.mark.parametrize("M,K,N", [(72, 200, 33), (8, 8, 32), (1000, 136, 1000), (1024, 64, 968), (2048, 264, 1000), (2000, 56, 1024), (4000, 72, 1000), (4096, 520, 2000)])
 def test_matmul_tiles_of_the_direct_kernel(backend, oracle, transa, transb, M, K, N):
