@@ -278,9 +278,36 @@ __device__ __forceinline__ void tile_in_problem(int lid, int tiles_m, int tiles_
 	}
 }
 
-/* tile `id` (0 <= id < count_tiles) of the launch; false if it has nothing to do */
+/* The groups of a ragged-K launch, up to 64 of them: lane l holds the end of group l's rows, and which group's tiles come l-th */
+struct KGroups { int end, order; };
+
+/* Groups whose tiles differ in their k-tiles go largest first.  uneven: the dearest tile costs half as much again as the mean one (in
+ * k-tiles: its own, and RAGGED_K_EPILOGUE for its store, which takes 6 us of a work-group's share of the memory's rate) */
+#define RAGGED_K_EPILOGUE 6
+__device__ __forceinline__ KGroups k_groups(const GemmParams & p, int lane, bool & uneven) {
+	KGroups k;
+	k.end = lane < p.num_groups ? p.cumsum[lane] : 0;
+	int start = wave_lane_below(k.end, 0);
+	asm volatile("" : "+v"(start));      /* the compiler would fold shift and difference into one instruction, whose results are wrong here */
+	const int rows = lane < p.num_groups ? k.end - start : 0;
+	const int cost = rows > 0 ? max(2, (rows + BK - 1) / BK) + RAGGED_K_EPILOGUE : 0;
+	const float sum = (float) __builtin_amdgcn_readlane(wave_inclusive_sum(cost), 63);
+	k.order = lane;
+	uneven = __ballot((float) cost * (float) p.num_groups > 1.5f * sum) != 0;
+	if (uneven) {
+		int rank = 0;
+		for (int j = 0; j < p.num_groups; j++) {
+			const int other = __builtin_amdgcn_readlane(cost, j);
+			rank += other > cost || (other == cost && j < lane) ? 1 : 0;
+		}
+		k.order = __builtin_amdgcn_ds_permute((lane < p.num_groups ? rank : lane) << 2, lane);
+	}
+	return k;
+}
+
+/* tile `id` (0 <= id < count_tiles) of the launch; false if it has nothing to do.  k: of a ragged-K launch of up to 64 groups */
 template <int BM, int BN, int MODE>
-__device__ __forceinline__ bool resolve_tile_id(const GemmParams & p, long id, Tile & t) {
+__device__ __forceinline__ bool resolve_tile_id(const GemmParams & p, long id, Tile & t, const KGroups & k = KGroups()) {
 	const int tiles_m = (p.M + BM - 1) / BM;
 	if (MODE == MODE_SINGLE) {
 		t.P = p.A; t.Q = p.B; t.Qmap = nullptr; t.Pmap = nullptr; t.C = p.C; t.D = p.D;
@@ -311,10 +338,12 @@ __device__ __forceinline__ bool resolve_tile_id(const GemmParams & p, long id, T
 	}
 	const int tiles_n = (p.N + BN - 1) / BN;
 	const unsigned int per_group = (unsigned int) tiles_m * (unsigned int) tiles_n;
-	const int g = (int) ((unsigned int) id / per_group);
-	const unsigned int r = (unsigned int) id - (unsigned int) g * per_group;
-	const int hi = p.cumsum[g];
-	const int lo = g ? p.cumsum[g - 1] : 0;
+	const int at = (int) ((unsigned int) id / per_group);
+	const unsigned int r = (unsigned int) id - (unsigned int) at * per_group;
+	const bool in_lanes = p.num_groups <= 64;
+	const int g = in_lanes ? __builtin_amdgcn_readlane(k.order, at) : at;
+	const int hi = in_lanes ? __builtin_amdgcn_readlane(k.end, g) : p.cumsum[g];
+	const int lo = g == 0 ? 0 : in_lanes ? __builtin_amdgcn_readlane(k.end, g - 1) : p.cumsum[g - 1];
 	if (hi - lo <= 0) {
 		return false;                                 /* no rows: D keeps its value */
 	}
@@ -1266,14 +1295,57 @@ gemm_bf16_stream_kernel(GemmParams p) {
 	const long die = blockIdx.x & 7;
 	const long stride = gridDim.x >> 3;                     /* work-groups per die (the grid is a multiple of 8) */
 	long local = blockIdx.x >> 3;
+	/* Ragged K over uneven groups: an equal count of tiles is no equal share (with a Zipf router one die had most of the multiplies).
+	 * There the dies take 32 consecutive tiles in turn, to and fro, of the groups in order of their rows: work-group i the
+	 * i-th tile, the i-th from the end of the second round and so on, in two steps that alternate; the tiles behind the last
+	 * whole round (from k_whole on) are spread over the dies, one (k_last) to a work-group.  us: 26 groups of 11700 rows,
+	 * 3968 x 2944, shares falling with the rank's power 1.2, 776 -> 350, 24 of 15768, 1472 x 1600, power 0.6, 192 -> 137; over 60
+	 * uneven launches 1.17x.  Groups of similar rows stay with the equal count, whose order keeps a die on one group (0.0 % apart
+	 * over 30 launches). */
+	KGroups groups = {0, 0};
+	unsigned int k_id = 0, k_step = 0, k_other_step = 0, k_limit = 0, k_whole = 0, k_last = 0;
+	if (MODE == MODE_RAGGED_K) {
+		bool uneven = false;
+		if (p.num_groups <= 64) {
+			groups = k_groups(p, lane, uneven);
+		}
+		k_id = (unsigned int) (die * chunk + local);
+		k_step = k_other_step = (unsigned int) stride;
+		k_limit = k_whole = (unsigned int) min((die + 1) * chunk, total);
+		k_last = 0xFFFFFFFFu;
+		if (uneven) {
+			const unsigned int rest = (unsigned int) total % gridDim.x, share = (rest + 7) >> 3, at = (unsigned int) (die * share + local);
+			k_limit = (unsigned int) total;
+			k_whole = k_limit - rest;
+			k_last = local < share && at < rest ? k_whole + at : 0xFFFFFFFFu;
+			k_id = (unsigned int) (die * stride + local);
+			k_step = 2 * (gridDim.x - k_id) - 1;
+			k_other_step = 2 * k_id + 1;
+			if (k_whole == 0) {
+				k_id = k_last;
+			}
+		}
+	}
+#define ST_K_NEXT(id_, step_, other_) do { \
+		const unsigned int s_ = step_; \
+		step_ = other_; \
+		other_ = s_; \
+		id_ = id_ >= k_whole ? 0xFFFFFFFFu : id_ + s_ >= k_whole ? k_last : id_ + s_; \
+	} while (0)
 
 	Tile cur;
 	bool have = false;
-	for (; local < chunk; local += stride) {
-		const long id = die * chunk + local;
-		if (id < total && resolve_tile_id<BM, BN, MODE>(p, id, cur)) {
-			have = true;
-			break;
+	if (MODE == MODE_RAGGED_K) {
+		while (k_id < k_limit && !(have = resolve_tile_id<BM, BN, MODE>(p, k_id, cur, groups))) {
+			ST_K_NEXT(k_id, k_step, k_other_step);
+		}
+	} else {
+		for (; local < chunk; local += stride) {
+			const long id = die * chunk + local;
+			if (id < total && resolve_tile_id<BM, BN, MODE>(p, id, cur)) {
+				have = true;
+				break;
+			}
 		}
 	}
 	if (!have) {
@@ -1318,13 +1390,14 @@ gemm_bf16_stream_kernel(GemmParams p) {
 #define ST_PEEK_NEXT() do { \
 		if (GATHER == GATHER_P_KROWS && wave < (WAVES_M * WAVES_N) / 2 && ld_live && ld_kt == ld_tiles - 1) { \
 			Tile ahead_; \
-			for (long l_ = local + stride; l_ < chunk; l_ += stride) { \
-				const long id_ = die * chunk + l_; \
-				if (id_ < total && resolve_tile_id<BM, BN, MODE>(p, id_, ahead_)) { \
+			unsigned int k_ = k_id, sa_ = k_step, sb_ = k_other_step; \
+			ST_K_NEXT(k_, sa_, sb_); \
+			while (k_ < k_limit && !peeked) { \
+				if (resolve_tile_id<BM, BN, MODE>(p, k_, ahead_, groups)) { \
 					peek_val = ahead_.Pmap[min(lane, ahead_.K - 1)]; \
 					peeked = true; \
-					break; \
 				} \
+				ST_K_NEXT(k_, sa_, sb_); \
 			} \
 		} \
 	} while (0)
@@ -1332,11 +1405,18 @@ gemm_bf16_stream_kernel(GemmParams p) {
 		ST_PEEK_NEXT(); \
 		if (ld_live && ld_kt == ld_tiles) { \
 			has_next = false; \
-			for (local += stride; local < chunk; local += stride) { \
-				const long id_ = die * chunk + local; \
-				if (id_ < total && resolve_tile_id<BM, BN, MODE>(p, id_, nxt)) { \
-					has_next = true; \
-					break; \
+			if (MODE == MODE_RAGGED_K) { \
+				ST_K_NEXT(k_id, k_step, k_other_step); \
+				while (k_id < k_limit && !(has_next = resolve_tile_id<BM, BN, MODE>(p, k_id, nxt, groups))) { \
+					ST_K_NEXT(k_id, k_step, k_other_step); \
+				} \
+			} else { \
+				for (local += stride; local < chunk; local += stride) { \
+					const long id_ = die * chunk + local; \
+					if (id_ < total && resolve_tile_id<BM, BN, MODE>(p, id_, nxt)) { \
+						has_next = true; \
+						break; \
+					} \
 				} \
 			} \
 			ld_live = has_next; \
@@ -1477,6 +1557,7 @@ gemm_bf16_stream_kernel(GemmParams p) {
 		has_next = false;
 	}
 	WAIT_VMCNT(0);
+#undef ST_K_NEXT
 #undef ST_INIT_LOADERS
 #undef ST_PEEK_NEXT
 #undef ST_ISSUE_NEXT

@@ -893,6 +893,41 @@ def test_grouped_matmul_ragged_k(backend, oracle, G, M, N, total):
             check_matmul(got[g], want, hi - lo)
 
 
+@pytest.mark.parametrize("G,M,N,shares", [(40, 1024, 1024, "one"), (33, 1088, 896, "power"), (64, 512, 1088, "power"), (70, 768, 1024, "power"), (9, 2048, 1280, "few"),
+                                          (150, 512, 768, "one")])
+def test_grouped_matmul_ragged_k_over_uneven_groups(backend, G, M, N, shares):
+    """up to 64 groups whose rows differ much the persistent kernel deals in order of their rows and in turn: every tile of every group,
+    with the bits of the group's own matmul, groups without rows untouched; with and without C"""
+    print("case grouped-K uneven G=%d M=%d N=%d %s" % (G, M, N, shares), flush=True)
+    be = backend
+    rng = np.random.default_rng(G + M)
+    if shares == "one":                                     # nearly all rows in one group, the rest with none to three
+        counts = rng.integers(0, 4, G)
+        counts[G // 3] = 1500
+    elif shares == "few":                                   # no rows in most groups, one of them the first
+        counts = np.where(np.arange(G) % 4 == 2, 700, 0)
+    else:
+        counts = rng.permutation((1200 / np.arange(1, G + 1)).astype(int)) + rng.integers(0, 3, G) * (rng.random(G) < 0.5)
+        counts[G // 2] = 0
+    total, incl = int(counts.sum()), np.cumsum(counts).astype(np.int32)
+    A, Bm, C0 = normal_bf16(rng, (total, M)), normal_bf16(rng, (total, N), 0.1), normal_bf16(rng, (G, N, M))
+    d_A, d_B, d_cum = be.upload(A), be.upload(Bm), be.upload(incl)
+    for beta, c_dt in ((0.0, B.DATAFLOW_NONE), (1.0, BF)):
+        d_got, d_want = be.upload(C0), be.upload(C0)
+        assert be.lib.dataflow_submit_amd_grouped_matmul(be.hp, CS, BF, BF, c_dt, BF, B.DATAFLOW_FP32, 0, 1, B.AMD_GROUPED_RAGGED_K, M, 0, N, G, d_cum.ptr,
+                                                         1.0, beta, d_A.ptr, 0, d_B.ptr, d_got.ptr if beta else None, d_got.ptr, N * M * 2) == 0
+        for g in np.flatnonzero(counts):
+            lo, n, ptr = int(incl[g] - counts[g]), int(counts[g]), d_want.ptr + int(g) * N * M * 2
+            assert be.lib.dataflow_submit_matmul(be.hp, CS, BF, BF, c_dt, BF, B.DATAFLOW_FP32, 0, 1, M, n, N, 1.0, beta, d_A.ptr + lo * M * 2, d_B.ptr + lo * N * 2,
+                                                 ptr if beta else None, ptr, 0, None) == 0
+        be.sync(CS)
+        got, want = be.read(d_got.ptr, (G, N, M), np.uint16), be.read(d_want.ptr, (G, N, M), np.uint16)
+        if not beta:
+            want[counts == 0] = 0
+        assert (got == want).all(), "beta %g: %d elements differ, groups %s" % (beta, int((got != want).sum()), np.unique(np.nonzero(got != want)[0])[:8])
+        d_got.free(), d_want.free()
+
+
 def test_submit_errors_are_reported(backend):
     be = backend
     d = be.alloc(4096)
