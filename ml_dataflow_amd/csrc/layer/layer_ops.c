@@ -77,6 +77,46 @@ int layer_submit_up_swiglu(Dataflow_Handle * handle, int stream_id, int expert_d
 	return submit(handle, &op, stream_id, "up projection and swiglu");
 }
 
+void layer_set_up_swiglu_apart_skeleton(Op_Skeleton * skeleton, int which) {
+	const DataflowDatatype t[13] = {DATAFLOW_INT_SCALAR, DATAFLOW_INT_SCALAR, DATAFLOW_INT_SCALAR, DATAFLOW_INT_SCALAR, DATAFLOW_INT, DATAFLOW_BF16,
+									DATAFLOW_UINT64_SCALAR, DATAFLOW_BF16, DATAFLOW_INT, DATAFLOW_INT_SCALAR, DATAFLOW_BF16, DATAFLOW_BF16, DATAFLOW_BF16};
+	dataflow_fill_skeleton(skeleton, which == LAYER_UP_SWIGLU_EXPERT ? "amd_up_swiglu_expert" : "amd_up_swiglu_grouped", DATAFLOW_BF16, DATAFLOW_NONE, 13, t);
+}
+
+static int up_swiglu_apart_stood_in(Op_Skeleton skeletons[3], int which) {
+	dataflow_set_default_swiglu_skeleton(&skeletons[0], DATAFLOW_BF16);
+	if (which == LAYER_UP_SWIGLU_EXPERT) {
+		dataflow_set_matmul_skeleton(&skeletons[1]);
+		return 2;
+	}
+	dataflow_set_amd_grouped_matmul_skeleton(&skeletons[1]);
+	dataflow_set_default_prepare_experts_skeleton(&skeletons[2], DATAFLOW_BF16, DATAFLOW_BF16);
+	return 3;
+}
+
+int layer_bind_up_swiglu_apart(Dataflow_Handle * handle, int which) {
+	Op_Skeleton skeleton, of[3];
+	layer_set_up_swiglu_apart_skeleton(&skeleton, which);
+	return stand_in_bind(handle, &skeleton, of, up_swiglu_apart_stood_in(of, which));
+}
+
+int layer_has_up_swiglu_apart(Dataflow_Handle * handle, int which) {
+	Op_Skeleton skeleton, of[3];
+	layer_set_up_swiglu_apart_skeleton(&skeleton, which);
+	return stand_in_usable(handle, &skeleton, of, up_swiglu_apart_stood_in(of, which));
+}
+
+int layer_submit_up_swiglu_apart(Dataflow_Handle * handle, int stream_id, int which, int expert_dim, int model_dim, int num_rows, int num_experts,
+							 int * expert_counts_cumsum, void * w13, uint64_t expert_stride_bytes, void * X, int * expert_mapping, int num_tokens,
+							 void * x1, void * x3, void * h) {
+	Op op;
+	layer_set_up_swiglu_apart_skeleton(&op.op_skeleton, which);
+	void ** a = op.op_args;
+	a[0] = &expert_dim; a[1] = &model_dim; a[2] = &num_rows; a[3] = &num_experts; a[4] = &expert_counts_cumsum; a[5] = &w13; a[6] = &expert_stride_bytes;
+	a[7] = &X; a[8] = &expert_mapping; a[9] = &num_tokens; a[10] = &x1; a[11] = &h; a[12] = &x3;
+	return submit(handle, &op, stream_id, "up projections and swiglu");
+}
+
 int layer_submit_route_tokens(Dataflow_Handle * handle, int stream_id, int num_tokens, int num_experts, int top_k, int model_dim,
 							  void * X, void * w_router, void * logit_bias, void * x_routed, float * token_expert_weights,
 							  uint16_t * chosen_experts, int * expert_counts, int * expert_counts_cumsum, int * host_expert_counts,

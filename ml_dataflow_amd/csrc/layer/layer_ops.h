@@ -34,6 +34,24 @@ LAYER_OPS_HIDDEN int layer_submit_route_tokens(Dataflow_Handle * handle, int str
  * 28.6 -> 26.6; 16 tokens, 64 experts, dim 4096 264.6 -> 258.8).  Beyond, the
  * GEMM's persistent kernels have no room for it, and the activation's own launch streams at the rate of the memory. */
 #define LAYER_UP_SWIGLU_VALUES (1u << 23)
+/* The same with x1 and x3 as arrays of their own, for weights that lie behind each other (w3 at w1 + expert_dim * model_dim), always on
+ * the tiles whose epilogue computes the activation.
+ * Of the grouped schedule, where it stands in for prepare_experts, the two grouped matmuls, which run on two streams that meet
+ * before and behind them (12 us each), and swiglu: up to 2^36 multiplies, beyond which the persistent kernels gain more than
+ * that (training steps, us: 1908 tokens, top 4, dims 2048 / 640 587 -> 552, 1326, top 3, 3392 / 1792 1616 -> 1580, 1445, top 2,
+ * 2112 / 640 391 -> 378; at 1.5 times the limit, 1913, top 5, 3264 / 1664, 1740 -> 1758).
+ * Of one expert's packed rows in the per-expert schedule, for the two matmuls and swiglu, up to LAYER_UP_SWIGLU_VALUES: a chain
+ * of four launches per expert becomes two (16 experts of 256 rows, dims 2048 / 1408 1314 -> 1228; 60 of 570, 2624 / 1536
+ * 7256 -> 6777). */
+#define LAYER_UP_SWIGLU_GROUPED_MULTIPLIES (1ull << 36)
+enum { LAYER_UP_SWIGLU_GROUPED, LAYER_UP_SWIGLU_EXPERT };
+LAYER_OPS_HIDDEN void layer_set_up_swiglu_apart_skeleton(Op_Skeleton * skeleton, int which);
+LAYER_OPS_HIDDEN int layer_bind_up_swiglu_apart(Dataflow_Handle * handle, int which);
+LAYER_OPS_HIDDEN int layer_has_up_swiglu_apart(Dataflow_Handle * handle, int which);
+/* _EXPERT: num_experts 1, no prefix sum, no mapping, num_tokens = num_rows */
+LAYER_OPS_HIDDEN int layer_submit_up_swiglu_apart(Dataflow_Handle * handle, int stream_id, int which, int expert_dim, int model_dim, int num_rows, int num_experts,
+							 int * expert_counts_cumsum, void * w13, uint64_t expert_stride_bytes, void * X, int * expert_mapping, int num_tokens,
+							 void * x1, void * x3, void * h);
 LAYER_OPS_HIDDEN void layer_set_up_swiglu_skeleton(Op_Skeleton * skeleton);
 LAYER_OPS_HIDDEN int layer_bind_up_swiglu(Dataflow_Handle * handle);
 LAYER_OPS_HIDDEN int layer_has_up_swiglu(Dataflow_Handle * handle);

@@ -193,6 +193,14 @@ static int stream_wait(Dataflow_Handle * h, int waiter, int signaller) {
 	return 0;
 }
 
+/* may the up-projections of an expert's rows and their activation be one op with x1 and x3 apart, where the rows are few enough? */
+static int up_swiglu_apart(Dataflow_Handle * h, const Amd_Moe_Layer * L, int which) {
+	const uint64_t H = L->expert_dim, D = L->model_dim;
+	const uintptr_t pointers = (uintptr_t) L->w1 | (uintptr_t) L->expert_stride_bytes | (uintptr_t) L->x1 | (uintptr_t) L->x3 | (uintptr_t) L->kernel_workspace
+		| (uintptr_t) (L->kernel_workspace_bytes / 2) | (uintptr_t) L->expert_zones;
+	return up_weights_stacked(L) && (pointers & 15) == 0 && (H & 7) == 0 && (D & 7) == 0 && (H + 64) * D * 2u <= 0xFFFFFFFFull && layer_has_up_swiglu_apart(h, which);
+}
+
 /* ------------------------------------------------------------------ forward */
 
 /* the routing as the reference submits it, op by op */
@@ -288,18 +296,23 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 		return 0;
 	}
 	if (schedule != AMD_MOE_PER_EXPERT) {
-		CHECK(dataflow_submit_default_prepare_experts(h, cs, dt, dt, T, D, K, X, L->token_mapping, L->expert_zones), "failed to submit prepare experts");
-		/* The two up-projections are independent: the second goes to the secondary stream, so its work-groups move
-		 * into the compute units that the first one's last, partial round of tiles leaves idle. */
-		CHECK(stream_wait(h, ss, cs), "secondary stream could not wait for the compute stream");
-		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, H, D, T * K,
-												 E, L->expert_counts_cumsum, 1.0f, 0.0f, L->w1, L->expert_stride_bytes, L->expert_zones, NULL, L->x1, 0),
-			  "failed to submit grouped w1 matmul");
-		CHECK(dataflow_submit_amd_grouped_matmul(h, ss, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, H, D, T * K,
-												 E, L->expert_counts_cumsum, 1.0f, 0.0f, L->w3, L->expert_stride_bytes, L->expert_zones, NULL, L->x3, 0),
-			  "failed to submit grouped w3 matmul");
-		CHECK(stream_wait(h, cs, ss), "compute stream could not wait for the secondary stream");
-		CHECK(dataflow_submit_default_swiglu(h, cs, dt, T * K, H, L->x1, L->x3, L->kernel_workspace), "failed to submit swiglu");
+		if ((uint64_t) T * K * 2 * H * D <= LAYER_UP_SWIGLU_GROUPED_MULTIPLIES && gather_allowed(T, D) && ((uintptr_t) X & 15) == 0 && up_swiglu_apart(h, L, LAYER_UP_SWIGLU_GROUPED)) {
+			CHECK(layer_submit_up_swiglu_apart(h, cs, LAYER_UP_SWIGLU_GROUPED, H, D, T * K, E, L->expert_counts_cumsum, L->w1, L->expert_stride_bytes, X,
+											   L->expert_mapping, T, L->x1, L->x3, L->kernel_workspace), "failed to submit grouped up projections and swiglu");
+		} else {
+			CHECK(dataflow_submit_default_prepare_experts(h, cs, dt, dt, T, D, K, X, L->token_mapping, L->expert_zones), "failed to submit prepare experts");
+			/* The two up-projections are independent: the second goes to the secondary stream, so its work-groups move
+			 * into the compute units that the first one's last, partial round of tiles leaves idle. */
+			CHECK(stream_wait(h, ss, cs), "secondary stream could not wait for the compute stream");
+			CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, H, D, T * K,
+													 E, L->expert_counts_cumsum, 1.0f, 0.0f, L->w1, L->expert_stride_bytes, L->expert_zones, NULL, L->x1, 0),
+				  "failed to submit grouped w1 matmul");
+			CHECK(dataflow_submit_amd_grouped_matmul(h, ss, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, H, D, T * K,
+													 E, L->expert_counts_cumsum, 1.0f, 0.0f, L->w3, L->expert_stride_bytes, L->expert_zones, NULL, L->x3, 0),
+				  "failed to submit grouped w3 matmul");
+			CHECK(stream_wait(h, cs, ss), "compute stream could not wait for the secondary stream");
+			CHECK(dataflow_submit_default_swiglu(h, cs, dt, T * K, H, L->x1, L->x3, L->kernel_workspace), "failed to submit swiglu");
+		}
 		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, D, H, T * K,
 												 E, L->expert_counts_cumsum, 1.0f, 0.0f, L->w2, L->expert_stride_bytes, L->kernel_workspace, NULL, L->expert_zones, 0),
 			  "failed to submit grouped w2 matmul");
@@ -328,6 +341,7 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 	int streams[2] = {cs, ss};
 	int which = 0;
 	uint64_t row = 0;
+	const int up_in_one = up_swiglu_apart(h, L, LAYER_UP_SWIGLU_EXPERT);
 	for (int e = 0; e < E; e++) {                                           /* :2848-2940 */
 		int n = L->host_expert_counts[e];
 		if (n == 0) {
@@ -345,11 +359,16 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 		/* the expert GEMMs get no workspace (the reference hands cuBLASLt the rest of this half, :2894-2897): with one,
 		 * a small expert would be split along K and round differently from the same expert inside the grouped launch */
 		int s = streams[which];
-		CHECK(dataflow_submit_matmul(h, s, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, H, D, n, 1.0f, 0.0f,
-									 expert_ptr(L->w1, L->expert_stride_bytes, e), zone, NULL, x1, 0, NULL), "failed to submit w1 matmul");
-		CHECK(dataflow_submit_matmul(h, s, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, H, D, n, 1.0f, 0.0f,
-									 expert_ptr(L->w3, L->expert_stride_bytes, e), zone, NULL, x3, 0, NULL), "failed to submit w3 matmul");
-		CHECK(dataflow_submit_default_swiglu(h, s, dt, n, H, x1, x3, temp), "failed to submit swiglu");
+		if (up_in_one && (uint64_t) n * 2 * H <= LAYER_UP_SWIGLU_VALUES && (uint64_t) n * D * 2u <= 0xFFFFFFFFull) {
+			CHECK(layer_submit_up_swiglu_apart(h, s, LAYER_UP_SWIGLU_EXPERT, H, D, n, 1, NULL, expert_ptr(L->w1, L->expert_stride_bytes, e), 0, zone, NULL, n,
+											   x1, x3, temp), "failed to submit up projections and swiglu");
+		} else {
+			CHECK(dataflow_submit_matmul(h, s, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, H, D, n, 1.0f, 0.0f,
+										 expert_ptr(L->w1, L->expert_stride_bytes, e), zone, NULL, x1, 0, NULL), "failed to submit w1 matmul");
+			CHECK(dataflow_submit_matmul(h, s, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, H, D, n, 1.0f, 0.0f,
+										 expert_ptr(L->w3, L->expert_stride_bytes, e), zone, NULL, x3, 0, NULL), "failed to submit w3 matmul");
+			CHECK(dataflow_submit_default_swiglu(h, s, dt, n, H, x1, x3, temp), "failed to submit swiglu");
+		}
 		CHECK(dataflow_submit_matmul(h, s, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, D, H, n, 1.0f, 0.0f,
 									 expert_ptr(L->w2, L->expert_stride_bytes, e), temp, NULL, zone, 0, NULL), "failed to submit w2 matmul");
 		row += (uint64_t) n;

@@ -1003,9 +1003,10 @@ __global__ void __launch_bounds__(256) up_swiglu_kernel(const bf16_t * __restric
 	((u32x4 *) h)[v] = pack8(o);
 }
 
-/* The layer's up-projection and its activation in one op (../layer/layer_ops.h): x1 | x3 side by side per routed row and h.  Few
+/* The layer's up-projection and its activation in one op (../layer/layer_ops.h): x1 | x3 of the routed rows and h.  Few
  * rows run on the direct kernel, whose epilogue then computes h; where the GEMM is large enough for the persistent kernels the
- * activation follows in a launch of its own. */
+ * activation follows in a launch of its own.  A thirteenth argument, x3: the two halves of a row go to arrays of their own, always
+ * on the direct kernel; without a prefix sum the rows are those of one expert, packed. */
 extern "C" int amd_up_swiglu(Dataflow_Handle * dataflow_handle, int stream_id, Op * op, void * op_extra) {
 	void ** a = op->op_args;
 	GemmParams p;
@@ -1025,8 +1026,14 @@ extern "C" int amd_up_swiglu(Dataflow_Handle * dataflow_handle, int stream_id, O
 	p.D = (bf16_t *) *((uint64_t *) a[10]);
 	p.h = (bf16_t *) *((uint64_t *) a[11]);
 	p.alpha = 1.0f;
-	const bool aligned = aligned16(p.A) && aligned16(p.B) && aligned16(p.D) && aligned16(p.h) && (strideA_bytes & 15) == 0 && (p.K & 7) == 0 && (half & 7) == 0;
-	if (half < 8 || half > (1 << 24) || p.K < 8 || p.K > (1 << 22) || p.N < 1 || p.num_groups < 1 || !p.cumsum || !p.A || !p.B || !p.gather || !p.D || !p.h || !aligned
+	bool aligned = aligned16(p.A) && aligned16(p.B) && aligned16(p.D) && aligned16(p.h) && (strideA_bytes & 15) == 0 && (p.K & 7) == 0 && (half & 7) == 0;
+	const bool apart = op->op_skeleton.header.num_args == 13, single = apart && !p.cumsum && !p.gather && p.num_groups == 1;
+	if (apart) {
+		const uint64_t x3 = *((uint64_t *) a[12]);
+		aligned = aligned && (x3 & 15) == 0 && x3 && x3 != (uint64_t) p.D;
+		p.x3_apart = ((long long) x3 - (long long) (uint64_t) p.D) / 2;
+	}
+	if (half < 8 || half > (1 << 24) || p.K < 8 || p.K > (1 << 22) || p.N < 1 || p.num_groups < 1 || !p.A || !p.B || (!single && (!p.cumsum || !p.gather)) || !p.D || !p.h || !aligned
 		|| p.gather_rows < 1 || (uint64_t) p.gather_rows * (uint64_t) p.K * 2u > 0xFFFFFFFFull || (uint64_t) (half + 64) * (uint64_t) p.K * 2u > 0xFFFFFFFFull) {
 		fprintf(stderr, "Error: bad arguments of the up-projection op (expert dim %d, model dim %d, %d rows, %d groups)...\n", half, p.K, p.N, p.num_groups);
 		return -1;
@@ -1040,6 +1047,12 @@ extern "C" int amd_up_swiglu(Dataflow_Handle * dataflow_handle, int stream_id, O
 		return -1;
 	}
 	const long cu_count = extra_cu_count(op_extra);
+	if (single) {
+		return launch_direct<false, false, MODE_SINGLE, GATHER_NONE, true>(p, choose_tile(MODE_SINGLE, p, cu_count, false), stream);
+	}
+	if (apart) {
+		return launch_direct<false, false, MODE_RAGGED_N, GATHER_Q_ROWS, true>(p, choose_tile(MODE_RAGGED_N, p, cu_count, false), stream);
+	}
 	const int tile = choose_tile(MODE_RAGGED_N, p, cu_count);
 	if (tile != TILE_BIG && kernel_choice == AMD_MATMUL_KERNEL_AUTO) {
 		return launch_direct<false, false, MODE_RAGGED_N, GATHER_Q_ROWS, true>(p, tile, stream);

@@ -72,8 +72,10 @@ struct GemmParams {
 	 * once.  The bits of the two tilings, or 0: run */
 	int candidates;
 	/* the layer's up-projection with its activation (SWIGLU form of the direct kernel): A is w1 over w3, M / 2 rows each, and
-	 * h[n * M / 2 + m] = silu(D[n * M + m]) * D[n * M + M / 2 + m] */
+	 * h[n * M / 2 + m] = silu(D[n * M + m]) * D[n * M + M / 2 + m].  x3_apart: 0, or x1 and x3 are two arrays with rows of M / 2, D
+	 * the first and x3_apart elements on the second */
 	bf16_t * h;
+	long long x3_apart;
 	/* Operands copied to padded rows (single problems on the direct kernel only; 0: not padded): elements from one k-row
 	 * to the next of a k-major operand, and the k-rows a k-major operand has where K was rounded up for a k-contiguous one
 	 * (those past them read as zero, like the padding they are multiplied with) */
@@ -1045,7 +1047,11 @@ __device__ __forceinline__ void store_swiglu_tile(const Tile & t, const GemmPara
 	}
 	__syncthreads();
 	const int half = t.M >> 1;
-	bf16_t * const h = p.h + ((t.D - p.D) >> 1);        /* of this group's first row */
+	const long long before = (t.D - p.D) >> 1;          /* elements of h, and of x1 or x3 alone, in front of this group's first row */
+	bf16_t * const h = p.h + before;
+	bf16_t * const x = p.x3_apart ? p.D + before : t.D;
+	const int pitch = p.x3_apart ? half : t.M;
+	const long long to_x3 = p.x3_apart ? p.x3_apart : half;
 	for (int item = threadIdx.x; item < BN * CHUNKS; item += THREADS) {
 		const int r = item / CHUNKS, c = item % CHUNKS;
 		const int n = t.n0 + r, m = (t.m0 >> 1) + c * 8;
@@ -1057,9 +1063,9 @@ __device__ __forceinline__ void store_swiglu_tile(const Tile & t, const GemmPara
 		unpack8(x1, a);
 		unpack8(x3, b);
 		swiglu8(a, b, o);
-		bf16_t * const d = t.D + (long long) n * t.M + m;
+		bf16_t * const d = x + (long long) n * pitch + m;
 		*((u32x4 *) d) = x1;
-		*((u32x4 *) (d + half)) = x3;
+		*((u32x4 *) (d + to_x3)) = x3;
 		*((u32x4 *) (h + (long long) n * half + m)) = pack8(o);
 	}
 }
@@ -1135,7 +1141,7 @@ gemm_bf16_direct_kernel(GemmParams p) {
 	if (GATHER == GATHER_P_KROWS) {
 		ldP.init_gather_k(t.P, t.Pmap, t.m0, t.M, t.K, p.gather_rows);
 	} else if (SWIGLU) {
-		static_assert(!SWIGLU || (!P_KMAJOR && MODE == MODE_RAGGED_N && THREADS / 8 == BM / 2), "two loads of P per lane and k-tile, one of either half");
+		static_assert(!SWIGLU || (!P_KMAJOR && MODE != MODE_RAGGED_K && THREADS / 8 == BM / 2), "two loads of P per lane and k-tile, one of either half");
 		static_assert(!SWIGLU || BN * (BM + 8) <= STAGES * (BM + BN) * BK, "the staged tile must fit in the stages");
 		ldP.init(t.P, t.m0 >> 1, t.M, t.K);
 		ldP.step = (uint32_t) (t.M >> 1) * (uint32_t) t.K * 2u;

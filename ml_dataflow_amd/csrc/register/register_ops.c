@@ -168,6 +168,13 @@ static int register_stand_ins(Dataflow_Handle * handle, const char * dir) {
 		fprintf(stderr, "Error: failed to register the layer's up-projection op, which needs the gathered grouped matmul and the strided swiglu in the table...\n");
 		return -1;
 	}
+	for (int which = LAYER_UP_SWIGLU_GROUPED; which <= LAYER_UP_SWIGLU_EXPERT; which++) {
+		layer_set_up_swiglu_apart_skeleton(&skeleton, which);
+		if ((handle->register_external_code)(handle, path, 1, &skeleton, &symbol, &init_symbol) != 1 || layer_bind_up_swiglu_apart(handle, which)) {
+			fprintf(stderr, "Error: failed to register the layer's up-projection ops, which need the matmuls, prepare_experts and swiglu in the table...\n");
+			return -1;
+		}
+	}
 	dataflow_set_amd_rms_norm_bwd_w_few_rows_skeleton(&skeleton);
 	char * kernel = "amd_rms_norm_bwd_w_few_rows_bf16_bf16_kernel", * launch = "amd_rms_norm_bwd_w_few_rows_set_launch_config", * none = NULL;
 	snprintf(path, sizeof(path), "%s/%s", dir, NATIVE_CODE_FILE);

@@ -254,6 +254,39 @@ def test_up_projection_with_its_activation_gives_the_bits_of_the_two_ops(backend
         assert (a == b).all(), "%s differs in %d of %d elements" % (name, int((a != b).sum()), a.size)
 
 
+@pytest.mark.parametrize("T,D,E,K,H", [(1, 64, 2, 1, 8), (7, 72, 3, 2, 24), (40, 136, 5, 3, 56), (100, 256, 4, 2, 136), (256, 512, 8, 2, 1024),
+                                       (700, 64, 4, 2, 1000), (640, 200, 8, 4, 1000), (1200, 96, 2, 2, 1664), (6000, 64, 3, 2, 1792)])
+def test_up_projections_apart_in_one_op_give_the_bits_of_the_separate_ones(backend, T, D, E, K, H):
+    """x1, x3, h and the output of the grouped schedule with its up-projections and activation as one op and op by op
+    (AMD_MOE_NO_GATHER), and of the per-expert schedule, whose experts take that op each; those of the last sizes are beyond its limit"""
+    print("case up swiglu apart T=%d D=%d E=%d K=%d H=%d" % (T, D, E, K, H), flush=True)
+    be = backend
+    rng = np.random.default_rng(T + D + H)
+    Wr, W1, W3, W2 = make_weights(rng, D, E, H)
+    W1[0] = normal_bf16(rng, W1[0].shape, 10.0)
+    X, resid = normal_bf16(rng, (T, D), 2.0), normal_bf16(rng, (T, D))
+    runs = []
+    for schedule, packed in ((B.AMD_MOE_GROUPED, True), (B.AMD_MOE_GROUPED, False), (B.AMD_MOE_PER_EXPERT, False)):
+        if packed:
+            os.environ["AMD_MOE_NO_GATHER"] = "1"
+        try:
+            layer = MoeLayer(be, T, D, E, K, H)
+            layer.load_weights(Wr, W1, W3, W2)
+            d_X, d_out = be.upload(X), be.upload(resid)
+            layer.forward(T, d_X.ptr, d_out.ptr, None, schedule)
+            be.sync()
+        finally:
+            os.environ.pop("AMD_MOE_NO_GATHER", None)
+        runs.append((be.read(d_out.ptr, (T, D), np.uint16), be.read(layer.L.x1, (T * K, H), np.uint16), be.read(layer.L.x3, (T * K, H), np.uint16),
+                     be.read(layer.L.kernel_workspace, (T * K, H), np.uint16)))
+        layer.free()
+        for d in (d_X, d_out):
+            d.free()
+    for schedule, run, names in (("grouped", runs[1], ("out", "x1", "x3", "h")), ("per expert", runs[2], ("out", "x1", "x3"))):
+        for name, a, b in zip(names, runs[0], run):
+            assert (a == b).all(), "%s: %s differs in %d of %d elements" % (schedule, name, int((a != b).sum()), a.size)
+
+
 @pytest.mark.parametrize("schedule", [B.AMD_MOE_FUSED, B.AMD_MOE_GROUPED])
 def test_two_runs_give_the_same_bits(backend, schedule):
     """nothing in the path depends on the order in which work-groups run: the rows of an expert are in token order

@@ -193,6 +193,51 @@ def test_the_up_projection_op_gives_way_to_a_replaced_one(replaced):
     assert up(expert_dim=large, w3=(2 << 24) + large * D * 2, w1=2 << 24, dw1=3 << 24, dw3=(3 << 24) + large * D * 2) == UP_OPS
 
 
+UP_APART = {B.AMD_MOE_GROUPED: ("amd_up_swiglu_grouped_BF16", ("amd_grouped_matmul", "default_swiglu_BF16", "default_prepare_experts_BF16_BF16")),
+            B.AMD_MOE_PER_EXPERT: ("amd_up_swiglu_expert_BF16", ("default_matmul", "default_swiglu_BF16"))}
+
+
+@pytest.mark.parametrize("schedule,replaced", [(s, r) for s, (_, ops) in UP_APART.items() for r in (None, *ops)])
+def test_the_up_projection_ops_with_results_apart_give_way_to_a_replaced_one(schedule, replaced):
+    """as above for the schedules that keep x1 and x3 in arrays of their own"""
+    noting = NotingHandle(C.sizeof(HipFunction))
+    lib, skeletons = noting.lib, {}
+    one_op, ops = UP_APART[schedule]
+    setters = {"amd_grouped_matmul": lib.dataflow_set_amd_grouped_matmul_skeleton, "default_matmul": lib.dataflow_set_matmul_skeleton,
+               "default_swiglu_BF16": lambda sk: lib.dataflow_set_default_swiglu_skeleton(sk, B.DATAFLOW_BF16),
+               "default_prepare_experts_BF16_BF16": lambda sk: lib.dataflow_set_default_prepare_experts_skeleton(sk, B.DATAFLOW_BF16, B.DATAFLOW_BF16)}
+    for name in ops:
+        skeletons[name] = B.OpSkeleton()
+        setters[name](C.byref(skeletons[name]))
+    both = skeletons[one_op] = B.OpSkeleton()
+    both.header.op_nickname = one_op.encode()
+    both.header.num_args = 13
+    both.header.arg_dtypes = (C.c_int * B.MAX_OP_ARGS)(*([B.DATAFLOW_INT_SCALAR] * 4 + [B.DATAFLOW_INT, B.DATAFLOW_BF16, B.DATAFLOW_UINT64_SCALAR, B.DATAFLOW_BF16, B.DATAFLOW_INT,
+                                                                                       B.DATAFLOW_INT_SCALAR] + [B.DATAFLOW_BF16] * 3))
+    assert lib.dataflow_do_fingerprinting(C.byref(both.header), C.sizeof(both.header), both.fingerprint) == 0
+
+    def insert(name, implementation, **fields):
+        native = "matmul" not in name and name != one_op
+        fn = HipFunction(op_skeleton=skeletons[name], is_native=native, **{"function_handle" if native else "hip_external_func": implementation}, **fields)
+        assert lib.dataflow_insert_table(C.byref(noting.h.op_table), C.cast(skeletons[name].fingerprint, C.c_void_p), C.cast(C.byref(fn), C.c_void_p)) == 0
+
+    def swiglus(**changes):
+        return [name for name in noting.forward(schedule, **changes) if "swiglu" in name]
+
+    times = E if schedule == B.AMD_MOE_PER_EXPERT else 1
+    for i, name in enumerate(ops):
+        insert(name, 0x1000 * (i + 1))
+    assert swiglus() == ["default_swiglu_BF16"] * times
+    table = {name: 0x1000 * (i + 1) for i, name in enumerate(ops)}
+    order = [n for n in ("default_swiglu_BF16", "amd_grouped_matmul", "default_matmul", "default_prepare_experts_BF16_BF16") if n in table]
+    insert(one_op, 0x7000, stands_in_for=(C.c_void_p * 3)(*[table[n] for n in order]))
+    if replaced:
+        assert lib.dataflow_remove_table(C.byref(noting.h.op_table), C.cast(skeletons[replaced].fingerprint, C.c_void_p), None) == 0
+        insert(replaced, 0x6000)
+    assert swiglus() == ([ops[1]] if replaced else [one_op]) * times
+    assert swiglus(x1=(7 << 24) + 8) == swiglus(kernel_workspace=(9 << 24) + 8) == swiglus(w3=1 << 40) == [ops[1]] * times     # off a 16-byte boundary; not stacked
+
+
 NORM_OPS = ("default_rms_norm_bwd_w_BF16_BF16", "default_rms_norm_bwd_w_combine_BF16")
 NORM_FEW_ROWS = "amd_rms_norm_bwd_w_few_rows_BF16_BF16"
 
