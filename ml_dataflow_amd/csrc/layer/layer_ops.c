@@ -117,6 +117,35 @@ int layer_submit_up_swiglu_apart(Dataflow_Handle * handle, int stream_id, int wh
 	return submit(handle, &op, stream_id, "up projections and swiglu");
 }
 
+void layer_set_matmul_twin_skeleton(Op_Skeleton * skeleton) {
+	const DataflowDatatype t[11] = {DATAFLOW_INT_SCALAR, DATAFLOW_INT_SCALAR, DATAFLOW_INT_SCALAR, DATAFLOW_FP32_SCALAR, DATAFLOW_BF16, DATAFLOW_BF16, DATAFLOW_BF16,
+									DATAFLOW_BF16, DATAFLOW_BF16, DATAFLOW_BF16, DATAFLOW_BF16};
+	dataflow_fill_skeleton(skeleton, "amd_matmul_twin", DATAFLOW_BF16, DATAFLOW_NONE, 11, t);
+}
+
+int layer_bind_matmul_twin(Dataflow_Handle * handle) {
+	Op_Skeleton skeleton, of;
+	layer_set_matmul_twin_skeleton(&skeleton);
+	dataflow_set_matmul_skeleton(&of);
+	return stand_in_bind(handle, &skeleton, &of, 1);
+}
+
+int layer_has_matmul_twin(Dataflow_Handle * handle) {
+	Op_Skeleton skeleton, of;
+	layer_set_matmul_twin_skeleton(&skeleton);
+	dataflow_set_matmul_skeleton(&of);
+	return stand_in_usable(handle, &skeleton, &of, 1);
+}
+
+int layer_submit_matmul_twin(Dataflow_Handle * handle, int stream_id, int M, int K, int N, float beta, void * A,
+							 void * B1, void * C1, void * D1, void * B2, void * C2, void * D2) {
+	Op op;
+	layer_set_matmul_twin_skeleton(&op.op_skeleton);
+	void ** a = op.op_args;
+	a[0] = &M; a[1] = &K; a[2] = &N; a[3] = &beta; a[4] = &A; a[5] = &B1; a[6] = &C1; a[7] = &D1; a[8] = &B2; a[9] = &C2; a[10] = &D2;
+	return submit(handle, &op, stream_id, "twin matmul");
+}
+
 int layer_submit_route_tokens(Dataflow_Handle * handle, int stream_id, int num_tokens, int num_experts, int top_k, int model_dim,
 							  void * X, void * w_router, void * logit_bias, void * x_routed, float * token_expert_weights,
 							  uint16_t * chosen_experts, int * expert_counts, int * expert_counts_cumsum, int * host_expert_counts,

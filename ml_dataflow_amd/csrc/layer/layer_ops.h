@@ -59,4 +59,14 @@ LAYER_OPS_HIDDEN int layer_submit_up_swiglu(Dataflow_Handle * handle, int stream
 							 int * expert_counts_cumsum, void * w13, uint64_t expert_stride_bytes, void * X, int * expert_mapping, int num_tokens,
 							 void * x13, void * h);
 
+/* An expert's dW1 and dW3 of the per-expert schedule, which differ in B, C and D: what two dataflow_submit_matmul without a
+ * workspace leave, bit for bit; stands in for the matmul.  One launch where the two together run on the direct kernel's tiles, which
+ * an expert's few hundred rows leave half of the compute units without (training steps, us: 16 experts of 256 rows, dims 2048 /
+ * 1408 1232 -> 1188, 60 of 570, 2624 / 1536 6773 -> 6435); two where they are large enough for the persistent one. */
+LAYER_OPS_HIDDEN void layer_set_matmul_twin_skeleton(Op_Skeleton * skeleton);
+LAYER_OPS_HIDDEN int layer_bind_matmul_twin(Dataflow_Handle * handle);
+LAYER_OPS_HIDDEN int layer_has_matmul_twin(Dataflow_Handle * handle);
+LAYER_OPS_HIDDEN int layer_submit_matmul_twin(Dataflow_Handle * handle, int stream_id, int M, int K, int N, float beta, void * A,
+							 void * B1, void * C1, void * D1, void * B2, void * C2, void * D2);
+
 #endif

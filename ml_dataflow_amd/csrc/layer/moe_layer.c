@@ -586,6 +586,7 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 		int streams[2] = {cs, ss};
 		int which = 0;
 		uint64_t row = 0;
+		const int twin = layer_has_matmul_twin(h);
 		for (int e = 0; e < E; e++) {
 			int n = L->host_expert_counts[e];
 			if (n == 0) {
@@ -596,8 +597,12 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 			uint8_t * dx3 = (uint8_t *) L->dx3 + row * H * el;
 			void * dw1 = expert_ptr(L->dw1, S, e), * dw3 = expert_ptr(L->dw3, S, e);
 			int s = streams[which];
-			CHECK(dataflow_submit_matmul(h, s, dt, dt, wc_dt, dt, cdt, 0, 1, D, n, H, 1.0f, wbeta, zone, dx1, WGRAD_C(dw1), dw1, 0, NULL), "failed to submit dW1 matmul");
-			CHECK(dataflow_submit_matmul(h, s, dt, dt, wc_dt, dt, cdt, 0, 1, D, n, H, 1.0f, wbeta, zone, dx3, WGRAD_C(dw3), dw3, 0, NULL), "failed to submit dW3 matmul");
+			if (twin) {
+				CHECK(layer_submit_matmul_twin(h, s, D, n, H, wbeta, zone, dx1, WGRAD_C(dw1), dw1, dx3, WGRAD_C(dw3), dw3), "failed to submit dW1 and dW3 matmul");
+			} else {
+				CHECK(dataflow_submit_matmul(h, s, dt, dt, wc_dt, dt, cdt, 0, 1, D, n, H, 1.0f, wbeta, zone, dx1, WGRAD_C(dw1), dw1, 0, NULL), "failed to submit dW1 matmul");
+				CHECK(dataflow_submit_matmul(h, s, dt, dt, wc_dt, dt, cdt, 0, 1, D, n, H, 1.0f, wbeta, zone, dx3, WGRAD_C(dw3), dw3, 0, NULL), "failed to submit dW3 matmul");
+			}
 			row += (uint64_t) n;
 			which ^= 1;
 		}

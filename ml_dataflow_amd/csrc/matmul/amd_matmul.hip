@@ -163,8 +163,8 @@ static int choose_tile(int mode, const GemmParams & p, long cu_count, bool persi
 
 /* the direct kernel on one of its tiles */
 template <bool PK, bool QK, int MODE, int GATHER = GATHER_NONE, bool SWIGLU = false>
-static int launch_direct(const GemmParams & p, int which, hipStream_t stream) {
-	const long grid = grid_of(which, MODE, p);
+static int launch_direct(const GemmParams & p, int which, hipStream_t stream, int problems = 1) {
+	const long grid = grid_of(which, MODE, p) * problems;
 	switch (which) {
 		case TILE_64x32: return launch_direct_tile<64, 32, 2, 2, 4, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
 		case TILE_64x64: return launch_direct_tile<64, 64, 2, 2, 4, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
@@ -860,6 +860,50 @@ extern "C" int amd_matmul(Dataflow_Handle * dataflow_handle, int stream_id, Op *
 	const uint64_t workspace_bytes = *((uint64_t *) a[17]);
 	uint8_t * workspace = (uint8_t *) *((uint64_t *) a[18]);
 	return run_matmul(dataflow_handle, stream_id, p, transa, transb, workspace, workspace_bytes, extra_cu_count(op_extra), false);
+}
+
+/* Two products with the same A, both operands k-major: what amd_matmul leaves without a workspace for (A, B, C, D) and for (A, B2,
+ * C2, D2), bit for bit (../layer/layer_ops.h).  On the direct kernel's tiles one launch does both. */
+extern "C" int amd_matmul_twin(Dataflow_Handle * dataflow_handle, int stream_id, Op * op, void * op_extra) {
+	void ** a = op->op_args;
+	GemmParams p;
+	memset(&p, 0, sizeof(p));
+	p.M = *((int *) a[0]);
+	p.K = *((int *) a[1]);
+	p.N = *((int *) a[2]);
+	p.beta = *((float *) a[3]);
+	p.alpha = 1.0f;
+	p.A = (const bf16_t *) *((uint64_t *) a[4]);
+	p.B = (const bf16_t *) *((uint64_t *) a[5]);
+	p.C = p.beta == 0.0f ? NULL : (const bf16_t *) *((uint64_t *) a[6]);
+	p.D = (bf16_t *) *((uint64_t *) a[7]);
+	GemmParams second = p;
+	second.B = (const bf16_t *) *((uint64_t *) a[8]);
+	second.C = p.beta == 0.0f ? NULL : (const bf16_t *) *((uint64_t *) a[9]);
+	second.D = (bf16_t *) *((uint64_t *) a[10]);
+	const long cu_count = extra_cu_count(op_extra);
+	if (p.M >= 1 && p.K >= 1 && p.N >= 1 && p.N <= (1 << 24) && p.A && p.B && p.D && second.B && second.D && (p.C == NULL) == (second.C == NULL) && kernel_choice == AMD_MATMUL_KERNEL_AUTO
+		&& operand_direct_ok(p.A, true, p.M, p.K, 0) && operand_direct_ok(p.B, true, p.N, p.K, 0) && operand_direct_ok(second.B, true, p.N, p.K, 0)) {
+		GemmParams both = p;
+		both.N = 2 * p.N;
+		const int tile = choose_tile(MODE_SINGLE, both, cu_count);
+		if (tile != TILE_BIG) {
+			p.B_twin = second.B;
+			p.C_twin = second.C;
+			p.D_twin = second.D;
+			hipStream_t stream;
+			if (resolve_stream(dataflow_handle, stream_id, &stream)) {
+				return -1;
+			}
+			if (hipSetDevice(dataflow_handle->device_id) != hipSuccess) {
+				fprintf(stderr, "Error: hipSetDevice failed in the twin matmul...\n");
+				return -1;
+			}
+			return launch_direct<true, true, MODE_SINGLE>(p, tile, stream, 2);
+		}
+	}
+	return run_matmul(dataflow_handle, stream_id, p, 0, 1, NULL, 0, cu_count, false)
+		|| run_matmul(dataflow_handle, stream_id, second, 0, 1, NULL, 0, cu_count, false) ? -1 : 0;
 }
 
 /* D = alpha * op(A) op(B) + beta * C like amd_matmul (same kernels, same split along K, bit-identical results), for

@@ -81,6 +81,10 @@ struct GemmParams {
 	 * (those past them read as zero, like the padding they are multiplied with) */
 	int pitchA, pitchB;
 	int k_rows;
+	/* a second single problem of the same shape and A behind the first, on the direct kernel (NULL D_twin: none) */
+	const bf16_t * B_twin;
+	const bf16_t * C_twin;
+	bf16_t * D_twin;
 };
 
 struct Tile {
@@ -369,11 +373,15 @@ __device__ __forceinline__ bool resolve_tile(const GemmParams & p, Tile & t) {
 	if (MODE == MODE_SINGLE) {
 		const int tiles_n = (p.N + BN - 1) / BN;
 		long total = (long) tiles_m * tiles_n;
-		long id = xcd_remap(blockIdx.x, total);
+		long id = xcd_remap(blockIdx.x, p.D_twin ? 2 * total : total);
+		t.P = p.A; t.Q = p.B; t.Qmap = nullptr; t.Pmap = nullptr; t.C = p.C; t.D = p.D;
+		if (p.D_twin && id >= total) {
+			id -= total;
+			t.Q = p.B_twin; t.C = p.C_twin; t.D = p.D_twin;
+		}
 		if (id >= total) {
 			return false;
 		}
-		t.P = p.A; t.Q = p.B; t.Qmap = nullptr; t.Pmap = nullptr; t.C = p.C; t.D = p.D;
 		t.M = p.M; t.N = p.N; t.K = p.K;
 		const int tn = (int) ((unsigned int) id / (unsigned int) tiles_m);
 		t.m0 = ((int) id - tn * tiles_m) * BM;

@@ -928,6 +928,42 @@ def test_grouped_matmul_ragged_k_over_uneven_groups(backend, G, M, N, shares):
         d_got.free(), d_want.free()
 
 
+# the direct kernel's tiles, k tails, odd sizes (two calls of the general path) and sizes of the persistent kernel (two calls)
+@pytest.mark.parametrize("M,K,N,off", [(8, 1, 8, 0), (64, 70, 40, 0), (136, 64, 104, 0), (1024, 100, 896, 0), (2048, 256, 1408, 0), (2304, 65, 2048, 0), (64, 33, 41, 0),
+                                       (64, 40, 64, 1), (4096, 64, 4096, 0)])
+def test_twin_matmul_gives_the_bits_of_two(backend, M, K, N, off):
+    """the layer's op for dW1 and dW3 of an expert, which no wrapper of the interface submits (csrc/layer/layer_ops.c)"""
+    print("case twin M=%d K=%d N=%d off=%d" % (M, K, N, off), flush=True)
+    be = backend
+    rng = np.random.default_rng(M + K + N)
+    sk = B.OpSkeleton()
+    sk.header.op_nickname = b"amd_matmul_twin_BF16"
+    sk.header.num_args = 11
+    sk.header.arg_dtypes = (C.c_int * B.MAX_OP_ARGS)(*([B.DATAFLOW_INT_SCALAR] * 3 + [B.DATAFLOW_FP32_SCALAR] + [B.DATAFLOW_BF16] * 7))
+    assert be.lib.dataflow_do_fingerprinting(C.byref(sk.header), C.sizeof(sk.header), sk.fingerprint) == 0
+    A, B1, B2 = normal_bf16(rng, (K, M)), normal_bf16(rng, (K, N), 0.1), normal_bf16(rng, (K * N + off,), 0.1)
+    C1, C2 = normal_bf16(rng, (N, M)), normal_bf16(rng, (N, M))
+    d_A, d_B1, d_B2 = be.upload(A), be.upload(B1), be.upload(B2)
+    for beta in (0.0, 1.0):
+        got, want = [be.upload(C1), be.upload(C2)], [be.upload(C1), be.upload(C2)]
+        bs = [d_B1.ptr, d_B2.ptr + 2 * off]
+        cs = [d.ptr if beta else 0 for d in got]
+        values = [C.c_int(M), C.c_int(K), C.c_int(N), C.c_float(beta)] + [C.c_uint64(v) for v in (d_A.ptr, bs[0], cs[0], got[0].ptr, bs[1], cs[1], got[1].ptr)]
+        op = B.Op(op_skeleton=sk)
+        for i, v in enumerate(values):
+            op.op_args[i] = C.addressof(v)
+        assert be.h.submit_op(be.hp, C.byref(op), CS) == 0
+        for b, d in zip(bs, want):
+            assert be.lib.dataflow_submit_matmul(be.hp, CS, BF, BF, BF if beta else B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 0, 1, M, K, N, 1.0, beta, d_A.ptr, b,
+                                                 d.ptr if beta else None, d.ptr, 0, None) == 0
+        be.sync(CS)
+        for i in range(2):
+            a, b = be.read(got[i].ptr, (N, M), np.uint16), be.read(want[i].ptr, (N, M), np.uint16)
+            assert (a == b).all(), "beta %g, product %d: %d elements differ" % (beta, i, int((a != b).sum()))
+        for d in got + want:
+            d.free()
+
+
 def test_submit_errors_are_reported(backend):
     be = backend
     d = be.alloc(4096)

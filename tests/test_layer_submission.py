@@ -238,6 +238,27 @@ def test_the_up_projection_ops_with_results_apart_give_way_to_a_replaced_one(sch
     assert swiglus(x1=(7 << 24) + 8) == swiglus(kernel_workspace=(9 << 24) + 8) == swiglus(w3=1 << 40) == [ops[1]] * times     # off a 16-byte boundary; not stacked
 
 
+@pytest.mark.parametrize("replaced", [False, True])
+def test_the_twin_matmul_gives_way_to_a_replaced_matmul(replaced):
+    """an expert's dW1 and dW3 of the per-expert schedule: one op where the table is as registration leaves it"""
+    noting = NotingHandle(C.sizeof(HipFunction))
+    lib, hp, layer = noting.lib, C.pointer(noting.h), noting.layer()
+    matmul, twin = B.OpSkeleton(), B.OpSkeleton()
+    lib.dataflow_set_matmul_skeleton(C.byref(matmul))
+    twin.header.op_nickname = b"amd_matmul_twin_BF16"
+    twin.header.num_args = 11
+    twin.header.arg_dtypes = (C.c_int * B.MAX_OP_ARGS)(*([B.DATAFLOW_INT_SCALAR] * 3 + [B.DATAFLOW_FP32_SCALAR] + [B.DATAFLOW_BF16] * 7))
+    assert lib.dataflow_do_fingerprinting(C.byref(twin.header), C.sizeof(twin.header), twin.fingerprint) == 0
+    for sk, implementation, stands_in_for in ((matmul, 0x2000 if replaced else 0x1000, ()), (twin, 0x3000, (0x1000,))):
+        fn = HipFunction(op_skeleton=sk, hip_external_func=implementation, stands_in_for=(C.c_void_p * 3)(*stands_in_for))
+        assert lib.dataflow_insert_table(C.byref(noting.h.op_table), C.cast(sk.fingerprint, C.c_void_p), C.cast(C.byref(fn), C.c_void_p)) == 0
+    assert lib.amd_moe_layer_forward(hp, 1, 2, C.byref(layer), T, 1 << 32, None, 2 << 32, B.AMD_MOE_PER_EXPERT) == 0
+    noting.names.clear()
+    assert lib.amd_moe_layer_backward(hp, 1, 2, C.byref(layer), T, 1 << 32, 3 << 32, 4 << 32, B.AMD_MOE_PER_EXPERT) == 0
+    last = noting.names[noting.names.index("default_prepare_experts_BF16_BF16") + 1:]
+    assert last == (["default_matmul"] * 2 * E if replaced else ["amd_matmul_twin_BF16"] * E) + ["default_matmul"]
+
+
 NORM_OPS = ("default_rms_norm_bwd_w_BF16_BF16", "default_rms_norm_bwd_w_combine_BF16")
 NORM_FEW_ROWS = "amd_rms_norm_bwd_w_few_rows_BF16_BF16"
 
