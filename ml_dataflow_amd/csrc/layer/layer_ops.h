@@ -29,20 +29,22 @@ LAYER_OPS_HIDDEN int layer_submit_route_tokens(Dataflow_Handle * handle, int str
 /* The up-projections of the fused schedule and their activation: what dataflow_submit_amd_grouped_matmul_gathered (x1 | x3 of routed row
  * r side by side, from row expert_mapping[r] of X) and dataflow_submit_amd_swiglu_strided leave, bit for bit.  All pointers
  * 16-byte aligned; X and one expert's w1 below 4 GiB.  Stands in for those two.
- * Submitted for up to LAYER_UP_SWIGLU_VALUES values of x1 | x3: there the GEMM runs on tiles whose epilogue can compute the
+ * Submitted for up to LAYER_UP_SWIGLU_VALUES values of x1 | x3: there the GEMM may run on tiles whose epilogue can compute the
  * activation, one launch less in a chain of six that launches are most of (forwards, us: 256 tokens, dim 512
- * 28.6 -> 26.6; 16 tokens, 64 experts, dim 4096 264.6 -> 258.8).  Beyond, the
- * GEMM's persistent kernels have no room for it, and the activation's own launch streams at the rate of the memory. */
-#define LAYER_UP_SWIGLU_VALUES (1u << 23)
+ * 28.6 -> 26.6; 16 tokens, 64 experts, dim 4096 264.6 -> 258.8; 885 tokens over 34 experts, dims 3904 / 1984 392 -> 385).
+ * Where it runs on the persistent kernels, which have no room for it, the activation is a second launch of the op; beyond the
+ * limit they always are the cheaper ones. */
+#define LAYER_UP_SWIGLU_VALUES (1u << 25)
 /* The same with x1 and x3 as arrays of their own, for weights that lie behind each other (w3 at w1 + expert_dim * model_dim), always on
  * the tiles whose epilogue computes the activation.
  * Of the grouped schedule, where it stands in for prepare_experts, the two grouped matmuls, which run on two streams that meet
  * before and behind them (12 us each), and swiglu: up to 2^36 multiplies, beyond which the persistent kernels gain more than
  * that (training steps, us: 1908 tokens, top 4, dims 2048 / 640 587 -> 552, 1326, top 3, 3392 / 1792 1616 -> 1580, 1445, top 2,
  * 2112 / 640 391 -> 378; at 1.5 times the limit, 1913, top 5, 3264 / 1664, 1740 -> 1758).
- * Of one expert's packed rows in the per-expert schedule, for the two matmuls and swiglu, up to LAYER_UP_SWIGLU_VALUES: a chain
+ * Of one expert's packed rows in the per-expert schedule, for the two matmuls and swiglu, up to LAYER_UP_SWIGLU_EXPERT_VALUES: a chain
  * of four launches per expert becomes two (16 experts of 256 rows, dims 2048 / 1408 1314 -> 1228; 60 of 570, 2624 / 1536
  * 7256 -> 6777). */
+#define LAYER_UP_SWIGLU_EXPERT_VALUES (1u << 23)
 #define LAYER_UP_SWIGLU_GROUPED_MULTIPLIES (1ull << 36)
 enum { LAYER_UP_SWIGLU_GROUPED, LAYER_UP_SWIGLU_EXPERT };
 LAYER_OPS_HIDDEN void layer_set_up_swiglu_apart_skeleton(Op_Skeleton * skeleton, int which);

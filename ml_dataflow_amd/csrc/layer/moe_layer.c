@@ -359,7 +359,7 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 		/* the expert GEMMs get no workspace (the reference hands cuBLASLt the rest of this half, :2894-2897): with one,
 		 * a small expert would be split along K and round differently from the same expert inside the grouped launch */
 		int s = streams[which];
-		if (up_in_one && (uint64_t) n * 2 * H <= LAYER_UP_SWIGLU_VALUES && (uint64_t) n * D * 2u <= 0xFFFFFFFFull) {
+		if (up_in_one && (uint64_t) n * 2 * H <= LAYER_UP_SWIGLU_EXPERT_VALUES && (uint64_t) n * D * 2u <= 0xFFFFFFFFull) {
 			CHECK(layer_submit_up_swiglu_apart(h, s, LAYER_UP_SWIGLU_EXPERT, H, D, n, 1, NULL, expert_ptr(L->w1, L->expert_stride_bytes, e), 0, zone, NULL, n,
 											   x1, x3, temp), "failed to submit up projections and swiglu");
 		} else {

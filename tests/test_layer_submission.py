@@ -189,7 +189,7 @@ def test_the_up_projection_op_gives_way_to_a_replaced_one(replaced):
         insert(replaced, 0x5000)
     assert up() == (UP_OPS if replaced else ["amd_up_swiglu_BF16"])
     assert up(x1=(7 << 24) + 8) == UP_OPS and up(kernel_workspace=(9 << 24) + 8) == UP_OPS     # off a 16-byte boundary
-    large = 1 << 16                                                                            # T K 2 H = 10 M values
+    large = 1 << 18                                                                            # T K 2 H = 42 M values
     assert up(expert_dim=large, w3=(2 << 24) + large * D * 2, w1=2 << 24, dw1=3 << 24, dw3=(3 << 24) + large * D * 2) == UP_OPS
 
 
