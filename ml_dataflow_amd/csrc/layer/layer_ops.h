@@ -33,7 +33,7 @@ LAYER_OPS_HIDDEN int layer_submit_route_tokens(Dataflow_Handle * handle, int str
  * activation, one launch less in a chain of six that launches are most of (forwards, us: 256 tokens, dim 512
  * 28.6 -> 26.6; 16 tokens, 64 experts, dim 4096 264.6 -> 258.8; 885 tokens over 34 experts, dims 3904 / 1984 392 -> 385).
  * Where it runs on the persistent kernels, which have no room for it, the activation is a second launch of the op; beyond the
- * limit they always are the cheaper ones. */
+ * limit they nearly always are the cheaper ones. */
 #define LAYER_UP_SWIGLU_VALUES (1u << 25)
 /* The same with x1 and x3 as arrays of their own, for weights that lie behind each other (w3 at w1 + expert_dim * model_dim), always on
  * the tiles whose epilogue computes the activation.
