@@ -141,7 +141,14 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
 	v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
 	return v;
 }
-__device__ __forceinline__ int wave_lane_below(int v, int first) { return __builtin_amdgcn_update_dpp(first, v, 0x138, 0xF, 0xF, false); }
+/* The move stays an instruction of its own (the empty asm): where the compiler folds it into a difference whose subtrahend it is,
+ * a - below(b), it writes v_subrev_u32_dpp, and there the card moves the lanes of the other operand: the result is below(a) - b.
+ * Measured on all 64 lanes with wave_shr and row_shr; v_add_u32_dpp, v_sub_u32_dpp and v_mov_b32_dpp give what they say. */
+__device__ __forceinline__ int wave_lane_below(int v, int first) {
+	int below = __builtin_amdgcn_update_dpp(first, v, 0x138, 0xF, 0xF, false);
+	asm("" : "+v"(below));
+	return below;
+}
 
 /* ragged N: groups base .. base + 63, one per lane: end and start of the group's rows, tiles of BN rows in the groups up to
  * and including it and in it alone; rows_before: rows of the groups in front of `base` */
@@ -293,8 +300,7 @@ struct KGroups { int end, order; };
 __device__ __forceinline__ KGroups k_groups(const GemmParams & p, int lane, bool & uneven) {
 	KGroups k;
 	k.end = lane < p.num_groups ? p.cumsum[lane] : 0;
-	int start = wave_lane_below(k.end, 0);
-	asm volatile("" : "+v"(start));      /* the compiler would fold shift and difference into one instruction, whose results are wrong here */
+	const int start = wave_lane_below(k.end, 0);
 	const int rows = lane < p.num_groups ? k.end - start : 0;
 	const int cost = rows > 0 ? max(2, (rows + BK - 1) / BK) + RAGGED_K_EPILOGUE : 0;
 	const float sum = (float) __builtin_amdgcn_readlane(wave_inclusive_sum(cost), 63);
