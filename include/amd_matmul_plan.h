@@ -1,0 +1,24 @@
+/*
+ * amd_matmul_plan.h -- what the host's rules in libamd_matmul.so pick for a launch, without one: no device and no handle is
+ * needed, nothing is launched or kept.  For tools that name a launch's kernel and for tests of the rules; no counterpart in
+ * the reference.  Sizes and operand conventions are those of amd_matmul.h; cu_count: compute units of the device (256).
+ */
+#ifndef AMD_MATMUL_PLAN_H
+#define AMD_MATMUL_PLAN_H
+
+#include "dataflow_amd.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* Tiles of an aligned problem that is not split along K: the direct kernel's, or BIG: the persistent kernels */
+enum { AMD_MATMUL_TILE_64x32, AMD_MATMUL_TILE_64x64, AMD_MATMUL_TILE_64x128, AMD_MATMUL_TILE_128x128, AMD_MATMUL_TILE_128x128_PAIR, AMD_MATMUL_TILE_BIG };
+/* has_c: D also takes C (beta is not 0) */
+int amd_matmul_planned_tile(int M, int K, int N, int has_c, int cu_count);
+
+#ifdef __cplusplus
+}
+#endif
+
+#endif

@@ -24,6 +24,7 @@
 #include "dataflow_amd.h"
 #include "dataflow_amd_ops.h"
 #include "amd_matmul.h"
+#include "amd_matmul_plan.h"
 #include "gemm_kernel.h"
 #include "gemm_w4_kernel.h"
 #include "gemm_typed_kernel.h"
@@ -93,14 +94,20 @@ static long tiles_of(long extent, long tile) { return (extent + tile - 1) / tile
  * compute units) x (cost of a k-tile), small tiles while they still fit one round and larger ones behind that.  1408 x
  * 2048 x 256 takes 10 us on 64 x 64 tiles (29 on 128 x 128 with one k-tile in flight, which this replaced), 4096 x 4096 x
  * 512 31 us on 64 x 128 (55), 4096 x 4096 x 2048 66 us on pairs of 128 x 128 (92 on the persistent kernel).  The
- * costs are in hundredths of a microsecond.  A single problem's rounds are charged half a microsecond each on top, and a
- * partial last round of the persistent kernel 60 % of a whole one plus the rest by its share (270 tiles of 256 x 256, 3840 x
- * 3328 x 4582, take 104 us, in pairs of 128 x 128 146).  Ragged launches have no term per tile: with
- * caches that hold nothing of the operands the choice is 0.0 % behind the best of all tiles over 60 ragged-K launches of 4-1500 rows
- * per group, and 2.4 % over 120 ragged-N launches of 4-400. */
-enum { TILE_64x32, TILE_64x64, TILE_64x128, TILE_128x128, TILE_128x128_PAIR, TILE_BIG, NUM_TILES };
-static const struct { int bm, bn, cost; } TILES[NUM_TILES] = {{64, 32, 21}, {64, 64, 25}, {64, 128, 36}, {128, 128, 58}, {128, 128, 50}, {256, 256, 130}};
-#define TILE_ROUND_COST 50
+ * costs are in hundredths of a microsecond.  A single problem's rounds are charged what writing their tiles of D takes (store), the
+ * persistent kernel's also the read of C (the other kernels' is hidden behind their neighbours' k-tiles), and the launch of that
+ * kernel 2 us; a partial last round of it 60 % of a whole one plus the rest by its share (270 tiles of 256 x 256, 3840 x 3328 x 4582,
+ * take 104 us, in pairs of 128 x 128 146).  Without the bytes of C and D a K of one or two k-tiles went to whatever tile has the fewest
+ * rounds: the router's input gradient, 2048 x 32 x 3001 with C, to 96 work-groups of 256 x 256 in 13.3 us, where pairs of 128 x 128 take 9.1
+ * (4096 x 64 x 8192 31.4 and 27.5, 4096 x 64 x 65536 194 and 271, the other way round).  Over 544 products of 64-4096 columns,
+ * 16-65536 tokens, K 8-16384 the choice is 0.8 % behind the best of all tiles, at a flat half a microsecond a round it was 3.5 %.
+ * Ragged launches have no term per tile: with caches that hold nothing of the operands the choice is 0.0 % behind the best of all
+ * tiles over 60 ragged-K launches of 4-1500 rows per group, and 2.4 % over 120 ragged-N launches of 4-400. */
+enum { TILE_64x32 = AMD_MATMUL_TILE_64x32, TILE_64x64 = AMD_MATMUL_TILE_64x64, TILE_64x128 = AMD_MATMUL_TILE_64x128, TILE_128x128 = AMD_MATMUL_TILE_128x128,
+	TILE_128x128_PAIR = AMD_MATMUL_TILE_128x128_PAIR, TILE_BIG = AMD_MATMUL_TILE_BIG, NUM_TILES };
+static const struct { int bm, bn, cost, store; } TILES[NUM_TILES] = {{64, 32, 21, 40}, {64, 64, 25, 60}, {64, 128, 36, 90}, {128, 128, 58, 110}, {128, 128, 50, 110}, {256, 256, 130, 100}};
+#define TILE_BIG_READ_C_COST 320
+#define TILE_BIG_LAUNCH_COST 200
 #define TILE_PAIR_COST_ALONE 62      /* of a k-tile of the pair's tile where it has the compute unit to itself, or its lines come from HBM */
 
 /* tiles of the launch for tile `which`.  Ragged N: the group sizes are on the device; a group of the mean size has on
@@ -133,12 +140,13 @@ static long tile_cost(int which, int mode, const GemmParams & p, long cu_count) 
 	if (mode != MODE_SINGLE) {
 		return tiles_of(tiles, cu_count) * cost;
 	}
-	const long round = tiles_of(p.K, BK) * cost + TILE_ROUND_COST;
+	const bool big = which == TILE_BIG;
+	const long round = tiles_of(p.K, BK) * cost + TILES[which].store + (big && p.C ? TILE_BIG_READ_C_COST : 0);
 	const long full = tiles / cu_count, left = tiles % cu_count;
-	if (which == TILE_BIG && full > 0) {
-		return full * round + (left ? round * (3 * cu_count + 2 * left) / (5 * cu_count) : 0);
+	if (big && full > 0) {
+		return TILE_BIG_LAUNCH_COST + full * round + (left ? round * (3 * cu_count + 2 * left) / (5 * cu_count) : 0);
 	}
-	return (full + (left ? 1 : 0)) * round;
+	return (big ? TILE_BIG_LAUNCH_COST : 0) + (full + (left ? 1 : 0)) * round;
 }
 
 /* the cheapest tile; `cost`: what it costs (single problems: hundredths of a microsecond) */
@@ -160,6 +168,14 @@ static int choose_tile(int mode, const GemmParams & p, long cu_count, bool persi
 		*cost = best_cost;
 	}
 	return best;
+}
+
+extern "C" int amd_matmul_planned_tile(int M, int K, int N, int has_c, int cu_count) {
+	GemmParams p;
+	memset(&p, 0, sizeof(p));
+	p.M = M; p.K = K; p.N = N;
+	p.C = has_c ? (const bf16_t *) scratch_of_device : NULL;      /* any address: the rules look at whether there is one */
+	return choose_tile(MODE_SINGLE, p, cu_count);
 }
 
 /* the direct kernel on one of its tiles */
@@ -554,6 +570,7 @@ static long extra_cu_count(void * op_extra) {
  * The router's logits (up to 64 rows of k-contiguous weights) are charged 1 us for the pass and a quarter for each split: the layer's
  * routing adds up their partial sums in its selection, whose few work-groups wait for a split's loads behind the last ones'.
  * 0: unsplit; otherwise the split in `p`, and its tile + 1. */
+#define SPLIT_ROUND_COST 50                 /* the partial sums' stores, beside their bytes below */
 #define SPLIT_PASS_COST 400
 #define SPLIT_LOGITS_PASS_COST 100
 #define SPLIT_LOGITS_COST 25
@@ -579,7 +596,7 @@ static int plan_split(GemmParams & p, int transa, int transb, bool direct, float
 			if (per < 2 || splits < 2 || tiles * splits > 4 * cu_count || workspace_bytes / 4 / (uint64_t) splits < count) {
 				continue;
 			}
-			const long cost = tiles_of(tiles * splits, cu_count) * (per * cost_of_k_tile + TILE_ROUND_COST) + (logits ? SPLIT_LOGITS_PASS_COST + splits * SPLIT_LOGITS_COST : SPLIT_PASS_COST)
+			const long cost = tiles_of(tiles * splits, cu_count) * (per * cost_of_k_tile + SPLIT_ROUND_COST) + (logits ? SPLIT_LOGITS_PASS_COST + splits * SPLIT_LOGITS_COST : SPLIT_PASS_COST)
 				+ (long) ((uint64_t) splits * count * 4 / SPLIT_BYTES_PER_COST);
 			if (cost < least) {
 				least = cost;

@@ -1,0 +1,54 @@
+"""What the matmul's host rules pick, checked on the CPU against measured times (include/amd_matmul_plan.h)."""
+import ctypes as C
+import os
+
+import pytest
+
+from ml_dataflow_amd import binding as B
+
+CUS = 256
+TILES = ("64x32", "64x64", "64x128", "128x128", "128x128 pair", "256x256")
+
+
+@pytest.fixture(scope="module")
+def plan():
+    B.load_library()                                                   # whose symbols the matmul library uses
+    lib = C.CDLL(os.path.join(B.LIB_DIR, "libamd_matmul.so"))
+    lib.amd_matmul_planned_tile.argtypes = [C.c_int] * 5
+    return lib
+
+
+# M, K, N, C, microseconds on each tile (mean of 20-60 launches back to back, three buffers in turn).  The first eight are
+# the router's input gradient (K is the number of experts): next to no k-tiles, C and D are the time.
+MEASURED = [
+    (1408, 32, 3001, 1, (10.2, 9.57, 8.58, 8.9, 7.69, 11.72)),
+    (2048, 32, 3001, 1, (13.83, 12.25, 11.04, 10.98, 9.06, 13.24)),
+    (2048, 64, 4096, 1, (17.32, 15.59, 11.89, 11.47, 9.82, 14.86)),
+    (2048, 8, 8192, 1, (29.9, 27.14, 20.77, 20.74, 16.09, 18.96)),
+    (2048, 32, 20000, 1, (65.38, 59.74, 44.15, 45.72, 31.99, 41.08)),
+    (4096, 64, 8192, 1, (54.07, 49.68, 37.09, 37.6, 27.52, 31.22)),
+    (4096, 64, 20000, 1, (164.46, 154.14, 121.11, 118.9, 88.88, 65.15)),
+    (4096, 64, 65536, 1, (521.48, 487.84, 383.97, 372.05, 270.83, 194.03)),
+    (256, 4056, 633, 0, (15.83, 20.94, 29.89, 38.63, 52.83, 96.99)),
+    (1216, 2048, 344, 1, (10.77, 12.6, 15.45, 20.65, 23.13, 43.92)),
+    (2176, 768, 296, 1, (8.93, 6.98, 8.88, 10.42, 12.22, 21.8)),
+    (1408, 2784, 632, 0, (22.89, 14.86, 18.63, 25.46, 31.89, 55.73)),
+    (2560, 8744, 640, 0, (149.05, 88.76, 51.7, 70.88, 89.35, 166.0)),
+    (3328, 3248, 680, 0, (75.19, 45.93, 39.04, 29.43, 39.25, 64.31)),
+    (1472, 360, 2944, 1, (16.53, 15.47, 15.26, 15.44, 11.74, 18.32)),
+    (3584, 64, 6733, 1, (41.79, 37.58, 28.31, 28.65, 21.64, 29.85)),
+    (3968, 2280, 10841, 1, (895.96, 522.2, 381.93, 335.38, 321.8, 196.64)),
+    (3008, 112, 33160, 0, (180.55, 137.87, 106.33, 95.73, 81.98, 51.4)),
+]
+
+
+@pytest.mark.parametrize("M,K,N,has_c,us", MEASURED)
+def test_single_problem_runs_on_a_tile_near_the_best(plan, M, K, N, has_c, us):
+    tile = plan.amd_matmul_planned_tile(M, K, N, has_c, CUS)
+    # 10 %: runs of one tile differ by up to 4 %, and two tiles are compared
+    assert us[tile] <= 1.1 * min(us), (TILES[tile], TILES[us.index(min(us))])
+
+
+def test_the_persistent_kernel_needs_a_whole_tile_on_both_sides(plan):
+    assert plan.amd_matmul_planned_tile(255, 4096, 65536, 0, CUS) != 5
+    assert plan.amd_matmul_planned_tile(65536, 4096, 255, 0, CUS) != 5
