@@ -312,13 +312,21 @@ static int launch_ragged_n(int tilings, const GemmParams & p, bool pk, long grid
 	return 0;
 }
 
-/* Tiles of `tile_rows` rows of all groups together.  Even: as an even router deals the rows, a group's share near-normal with the
- * mean's root as standard deviation.  Uneven: shares that fall like a power (0.9) of the group's rank, the largest 4.1 times
- * the mean.  Either is seen at twelve equally likely quantiles.  spread: standard deviation of the result. */
-static double expected_n_tiles(const GemmParams & p, long tile_rows, bool uneven, double * spread) {
+/* Tiles of `tile_rows` rows of all groups together, for one of the distributions that a router may deal the rows in.  EVEN: a group's
+ * share near-normal with the mean's root as standard deviation.  UNEVEN: shares that fall like a power (0.9) of the group's rank, the
+ * largest 4.1 times the mean.  Either is seen at twelve equally likely quantiles.  ONE: 95 % of the rows in one group, the rest even.
+ * spread: standard deviation of the result. */
+enum { ROWS_EVEN, ROWS_UNEVEN, ROWS_IN_ONE, ROWS_DISTRIBUTIONS };
+static double expected_n_tiles(const GemmParams & p, long tile_rows, int rows_dealt, double * spread) {
 	static const double NORMAL[6] = {0.104, 0.319, 0.549, 0.812, 1.150, 1.732};
 	static const double SHARES[12] = {4.122, 1.855, 1.223, 0.921, 0.743, 0.624, 0.540, 0.476, 0.427, 0.387, 0.354, 0.327};
 	const double rows = (double) p.N / p.num_groups, deviation = sqrt(rows);
+	*spread = 0.0;
+	if (rows_dealt == ROWS_IN_ONE) {
+		const int others = p.num_groups - 1;
+		return (double) tiles_of(lrint(0.95 * p.N), tile_rows) + (others ? (double) others * tiles_of(lrint(0.05 * p.N / others), tile_rows) : 0.0);
+	}
+	const bool uneven = rows_dealt == ROWS_UNEVEN;
 	double sum = 0.0, squares = 0.0;
 	for (int i = 0; i < 12; i++) {
 		const double r = rint(uneven ? rows * SHARES[i] : rows + (i & 1 ? -1.0 : 1.0) * NORMAL[i / 2] * deviation);
@@ -333,9 +341,9 @@ static double expected_n_tiles(const GemmParams & p, long tile_rows, bool uneven
 
 /* Rounds of those tiles over the work-groups of a launch; a few tiles more or less decide over a whole round, so half a
  * standard deviation to both sides counts a quarter each */
-static double expected_rounds(const GemmParams & p, long tile_rows, bool uneven, long groups) {
+static double expected_rounds(const GemmParams & p, long tile_rows, int rows_dealt, long groups) {
 	double spread;
-	const double n_tiles = expected_n_tiles(p, tile_rows, uneven, &spread);
+	const double n_tiles = expected_n_tiles(p, tile_rows, rows_dealt, &spread);
 	double rounds = 0.0;
 	for (int side = -1; side <= 1; side++) {
 		rounds += (side ? 0.25 : 0.5) * (double) tiles_of(tiles_of(p.M, 256) * lrint(n_tiles + 0.5 * side * spread), groups);
@@ -343,19 +351,20 @@ static double expected_rounds(const GemmParams & p, long tile_rows, bool uneven,
 	return rounds;
 }
 
-/* expected costs of the tilings, and the cheapest.  No tiling is faster than the weights arrive (STREAMED_WEIGHTS: 6 TB/s). */
+/* expected costs of the tilings, and the cheapest.  No tiling is faster than the weights arrive (STREAMED_WEIGHTS: 6 TB/s).
+ * 384 is never the cheapest where its kernel does not apply, whatever `cost` says of it. */
 #define STREAMED_WEIGHTS(bytes) ((bytes) / 200)
 static double larger(double a, double b) { return a > b ? a : b; }
-static int cheapest_tiling(const GemmParams & p, long groups, bool four_ok, bool uneven, double cost[RAGGED_N_TILINGS]) {
+static int cheapest_tiling(const GemmParams & p, long groups, bool four_ok, int rows_dealt, double cost[RAGGED_N_TILINGS]) {
 	const long k_tiles = tiles_of(p.K, BK);
-	const double narrow = expected_rounds(p, 288, uneven, groups), wide = expected_rounds(p, 384, uneven, groups);
+	const double narrow = expected_rounds(p, 288, rows_dealt, groups), wide = expected_rounds(p, 384, rows_dealt, groups);
 	const double streamed = STREAMED_WEIGHTS((double) p.num_groups * p.M * p.K * 2.0);
 	int best = four_ok && WIDE_TILE_COST(wide, k_tiles) < NARROW_TILE_COST(narrow, k_tiles) ? RAGGED_N_384 : RAGGED_N_288;
 	cost[RAGGED_N_288] = larger(NARROW_TILE_COST(narrow, k_tiles), streamed);
 	cost[RAGGED_N_384] = larger(WIDE_TILE_COST(wide, k_tiles), streamed);
 	for (int tiling = RAGGED_N_224; tiling <= RAGGED_N_192; tiling++) {
 		const long rows = ragged_n_rows(tiling);
-		cost[tiling] = larger(FINER_TILE_COST(expected_rounds(p, rows, uneven, groups), rows, k_tiles), streamed);
+		cost[tiling] = larger(FINER_TILE_COST(expected_rounds(p, rows, rows_dealt, groups), rows, k_tiles), streamed);
 		if (cost[tiling] < cost[best]) {
 			best = tiling;
 		}
@@ -363,21 +372,54 @@ static int cheapest_tiling(const GemmParams & p, long groups, bool four_ok, bool
 	return best;
 }
 
-/* The tilings a ragged-N launch without C goes out on, as bits: the cheapest for the group sizes that an even router gives, and where
- * that one costs 5 % and 4 us more than another with very uneven groups, that other one too: the sizes are on the device, whose
+/* The tilings a ragged-N launch without C goes out on, as bits: the cheapest for the group sizes that an even router gives, and a
+ * second one where that one costs 5 % and 4 us more than the cheapest with UNEVEN group sizes, or 10 % and 15 us more with nearly all
+ * rows IN_ONE group: of the others the one that leaves the smaller of the worst cases.  The sizes are on the device, whose
  * work-groups then agree on one of the two from the real sizes (ragged_n_choice).  A launch that loses costs 3 us, so both
- * go out only there.  Over 310 launches of the layer's kind (8-64 experts, 30-9000 rows each, K 512-4096) one launch on the
- * expected tiling takes 1.9 % longer than the best of all tilings and this rule 2.5 %; up to three launches, among them 288 always,
- * took 4.7 %.  With a Zipf router, whose largest group is eight times the mean (100 launches), 4.5, 3.2 and 5.6 %: one of
- * 2979 tokens, 36 experts, top 4, dim 832 lost 9 % to the single launch.  us: a training step of 65536 tokens, 64 experts, dim
- * 4096 37.75 -> 36.99 ms, a forward of 8192 tokens, 32 experts, dim 2048 638 -> 622. */
-#define SECOND_TILING_MARGIN 121000
+ * go out only there.  Over 310 launches of the layer's kind (8-64 experts, 30-9000 rows each, K 512-4096) with even groups one launch on
+ * the expected tiling takes 1.9 % longer than the best of all tilings; up to three launches, among them 288 always,
+ * took 4.7 %.  A training step of 65536 tokens, 64 experts, dim 4096 37.75 -> 36.99 ms, a forward of 8192 tokens, 32 experts, dim
+ * 2048 638 -> 622 us.  Over 341 launches whose rows lie in one, two or four of 8-64 experts to 95 % or are dealt by Zipf routers, this
+ * rule is 3.4 % behind the best, without the second list 4.8 %, up to three launches 6.8 %; 17 / 41 of them are more than 3 % slower
+ * than those three launches and 4 / 27 more than 8 % (1024 x 3072, 41 groups, 6205 of 6478 rows in one: 90 / 136 us, on 288 alone 87). */
+#define SECOND_TILING_MARGIN 121000          /* 4 us */
+#define IN_ONE_TILING_MARGIN 454000          /* 15 us */
 static int ragged_n_tilings(const GemmParams & p, long cu_count, bool four_ok) {
+	static const struct { double share; double margin; } SECOND[ROWS_DISTRIBUTIONS] = {{0.0, 0.0}, {1.05, SECOND_TILING_MARGIN}, {1.10, IN_ONE_TILING_MARGIN}};
 	long groups = cu_count & ~7L;
 	groups = groups < 8 ? 8 : groups;
-	double even[RAGGED_N_TILINGS], uneven[RAGGED_N_TILINGS];
-	const int first = cheapest_tiling(p, groups, four_ok, false, even), second = cheapest_tiling(p, groups, four_ok, true, uneven);
-	return uneven[first] < 1.05 * uneven[second] + SECOND_TILING_MARGIN ? 1 << first : 1 << first | 1 << second;
+	double cost[ROWS_DISTRIBUTIONS][RAGGED_N_TILINGS];
+	int cheapest[ROWS_DISTRIBUTIONS];
+	for (int dealt = 0; dealt < ROWS_DISTRIBUTIONS; dealt++) {
+		cheapest[dealt] = cheapest_tiling(p, groups, four_ok, dealt, cost[dealt]);
+	}
+	const int first = cheapest[ROWS_EVEN];
+	int second = first;
+	double least = 0.0;                             /* the worst case with `first` and `second`, over the cheapest's cost */
+	for (int tiling = 0; tiling < RAGGED_N_TILINGS; tiling++) {
+		double worst = 0.0;
+		for (int dealt = ROWS_UNEVEN; dealt < ROWS_DISTRIBUTIONS; dealt++) {
+			const double best = cost[dealt][cheapest[dealt]];
+			if (cost[dealt][first] < SECOND[dealt].share * best + SECOND[dealt].margin) {
+				continue;
+			}
+			const double with = (cost[dealt][tiling] < cost[dealt][first] ? cost[dealt][tiling] : cost[dealt][first]) / best;
+			worst = with > worst ? with : worst;
+		}
+		if (tiling != first && worst > 0.0 && (four_ok || tiling != RAGGED_N_384) && (second == first || worst < least || (worst == least && cost[ROWS_EVEN][tiling] < cost[ROWS_EVEN][second]))) {
+			second = tiling;
+			least = worst;
+		}
+	}
+	return 1 << first | 1 << second;
+}
+
+extern "C" int amd_matmul_planned_tilings(int M, int K, int N, int num_groups, int cu_count) {
+	GemmParams p;
+	memset(&p, 0, sizeof(p));
+	p.M = M; p.K = K; p.N = N;
+	p.num_groups = num_groups;
+	return ragged_n_tilings(p, cu_count, w4_ok(p));
 }
 
 static long round_up8(long v) { return (v + 7) & ~7L; }

@@ -15,6 +15,7 @@ def plan():
     B.load_library()                                                   # whose symbols the matmul library uses
     lib = C.CDLL(os.path.join(B.LIB_DIR, "libamd_matmul.so"))
     lib.amd_matmul_planned_tile.argtypes = [C.c_int] * 5
+    lib.amd_matmul_planned_tilings.argtypes = [C.c_int] * 5
     return lib
 
 
@@ -52,3 +53,28 @@ def test_single_problem_runs_on_a_tile_near_the_best(plan, M, K, N, has_c, us):
 def test_the_persistent_kernel_needs_a_whole_tile_on_both_sides(plan):
     assert plan.amd_matmul_planned_tile(255, 4096, 65536, 0, CUS) != 5
     assert plan.amd_matmul_planned_tile(65536, 4096, 255, 0, CUS) != 5
+
+
+# M, K, rows, groups, how the rows are dealt, microseconds on tiles of 288, 384, 224 and 192 token rows (0: not on that kernel)
+MEASURED_TILINGS = [
+    (1024, 3072, 6478, 41, "95 % in one group", (87.4, 89.7, 137.3, 137.1)),
+    (3776, 1664, 4305, 15, "95 % in one group", (84.5, 104.0, 75.3, 94.3)),
+    (576, 3008, 33286, 34, "95 % in one group", (153.8, 153.2, 184.6, 175.8)),
+    (3456, 3904, 4716, 36, "95 % in four groups", (308.8, 308.3, 292.8, 358.4)),
+    (1280, 3584, 27778, 43, "95 % in two groups", (289.8, 321.1, 333.1, 321.3)),
+    (3456, 3520, 8050, 25, "95 % in two groups", (274.6, 272.2, 321.2, 313.5)),
+    (3584, 1408, 7774, 26, "Zipf, 1.2", (115.5, 132.8, 107.0, 103.1)),
+    (832, 3584, 43635, 15, "even", (279.6, 249.7, 300.0, 285.1)),
+    (2688, 1920, 10017, 21, "even", (96.2, 114.8, 111.0, 103.0)),
+    (3072, 2624, 6042, 57, "even", (226.6, 225.4, 221.0, 219.8)),
+]
+
+
+@pytest.mark.parametrize("M,K,rows,groups,dealt,us", MEASURED_TILINGS)
+def test_a_good_tiling_for_uneven_rows_is_among_those_that_go_out(plan, M, K, rows, groups, dealt, us):
+    tilings = plan.amd_matmul_planned_tilings(M, K, rows, groups, CUS)
+    assert 1 <= bin(tilings).count("1") <= 2
+    assert not (tilings & 2 and K % 128)                               # 384 rows: whole pairs of k-tiles
+    best = min(t for bit, t in enumerate(us) if tilings >> bit & 1)
+    # 13 %: the cost of the launch that loses, and what the rule leaves on the table (largest entry of this list: 12 %)
+    assert best <= 1.13 * min(us), tilings
