@@ -62,6 +62,18 @@ __device__ __forceinline__ void swiglu8(const float x1[8], const float x3[8], fl
 	}
 }
 
+/* out[r][i] = silu(x1[r][i]) * x3[r][i] for the 8 elements of vector v, counted over rows of per_row vectors; row r of x1 and x3
+ * starts row_stride elements after row r - 1, out is packed */
+__device__ __forceinline__ void swiglu_strided_vector(size_t v, size_t per_row, size_t row_stride, const bf16_t * x1, const bf16_t * x3, bf16_t * out) {
+	const size_t r = v / per_row;
+	const size_t src = (r * row_stride >> 3) + (v - r * per_row);
+	float a[8], b[8], o[8];
+	unpack8(__builtin_nontemporal_load(((const u32x4 *) x1) + src), a);
+	unpack8(__builtin_nontemporal_load(((const u32x4 *) x3) + src), b);
+	swiglu8(a, b, o);
+	((u32x4 *) out)[v] = pack8(o);
+}
+
 /* sum over the 64 lanes of a wave; every lane gets the total */
 __device__ __forceinline__ float wave_sum(float v) {
 	#pragma unroll

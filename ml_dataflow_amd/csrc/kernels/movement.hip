@@ -587,13 +587,7 @@ amd_swiglu_strided_bf16_kernel(int num_rows, int num_cols, int x_row_stride, con
 	if (v >= nvec) {
 		return;
 	}
-	const size_t r = v / (size_t) per_row;
-	const size_t src = (r * (size_t) x_row_stride >> 3) + (v - r * (size_t) per_row);
-	float a[8], b[8], o[8];
-	unpack8(__builtin_nontemporal_load(((const u32x4 *) x_w1) + src), a);
-	unpack8(__builtin_nontemporal_load(((const u32x4 *) x_w3) + src), b);
-	swiglu8(a, b, o);
-	((u32x4 *) out)[v] = pack8(o);
+	swiglu_strided_vector(v, (size_t) per_row, (size_t) x_row_stride, x_w1, x_w3, out);
 }
 
 /* What remains of the expert-side backward between the hidden-gradient GEMM and the input-gradient GEMMs when the

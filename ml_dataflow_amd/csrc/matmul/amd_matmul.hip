@@ -1091,26 +1091,34 @@ extern "C" int amd_grouped_matmul(Dataflow_Handle * dataflow_handle, int stream_
 	return -1;
 }
 
-/* The activation behind an up-projection on the persistent kernels, as amd_swiglu_strided_bf16_kernel (kernels/movement.hip) */
-__global__ void __launch_bounds__(256) up_swiglu_kernel(const bf16_t * __restrict__ x13, bf16_t * __restrict__ h, long long rows, int half) {
+/* The activation behind an up-projection on kernels whose epilogue does not compute it */
+__global__ void __launch_bounds__(256) up_swiglu_kernel(const bf16_t * x1, const bf16_t * x3, int row_stride, bf16_t * h, long long rows, int half) {
 	const int per_row = half >> 3;
 	const long long v = (long long) blockIdx.x * 256 + threadIdx.x;
-	if (v >= rows * per_row) {
-		return;
+	if (v < rows * per_row) {
+		swiglu_strided_vector((size_t) v, (size_t) per_row, (size_t) row_stride, x1, x3, h);
 	}
-	const long long r = v / per_row;
-	const u32x4 * const x = (const u32x4 *) (x13 + r * 2 * half) + (v - r * per_row);
-	float a[8], b[8], o[8];
-	unpack8(__builtin_nontemporal_load(x), a);
-	unpack8(__builtin_nontemporal_load(x + per_row), b);
-	swiglu8(a, b, o);
-	((u32x4 *) h)[v] = pack8(o);
+}
+static int launch_up_swiglu(const GemmParams & p, int half, const bf16_t * x3, int row_stride, hipStream_t stream) {
+	const long long vectors = (long long) p.N * (half >> 3);
+	hipLaunchKernelGGL(up_swiglu_kernel, dim3((unsigned int) ((vectors + 255) / 256)), dim3(256), 0, stream, (const bf16_t *) p.D, x3, row_stride, p.h, (long long) p.N, half);
+	return check_launch();
+}
+
+/* a GEMM of the up-projection as the matmul ops launch it */
+static int launch_up_projection(const GemmParams & p, bool single, long cu_count, hipStream_t stream) {
+	if (single) {
+		return launch_gemm<MODE_SINGLE>(p, 1, 0, true, tiles_of(p.M, 256) * tiles_of(p.N, 256), tiles_of(p.M, 128) * tiles_of(p.N, 128), cu_count, stream);
+	}
+	return launch_gemm<MODE_RAGGED_N>(p, 1, 0, true, tiles_of(p.M, 256) * ((long) p.N / 256 + p.num_groups), tiles_of(p.M, 128) * ((long) p.N / 128 + p.num_groups),
+									  cu_count, stream, tiles_of(p.M, 256) * ((long) p.N / 192 + p.num_groups));
 }
 
 /* The layer's up-projection and its activation in one op (../layer/layer_ops.h): x1 | x3 of the routed rows and h.  Few
  * rows run on the direct kernel, whose epilogue then computes h; where the GEMM is large enough for the persistent kernels the
- * activation follows in a launch of its own.  A thirteenth argument, x3: the two halves of a row go to arrays of their own, always
- * on the direct kernel; without a prefix sum the rows are those of one expert, packed. */
+ * activation follows in a launch of its own.  A thirteenth argument, x3: the two halves of a row go to arrays of their own,
+ * on the direct kernel; without a prefix sum the rows are those of one expert, packed.  A caller that named a kernel
+ * (amd_matmul_select_kernel) has the GEMMs and the activation launched as the ops this one stands in for launch them. */
 extern "C" int amd_up_swiglu(Dataflow_Handle * dataflow_handle, int stream_id, Op * op, void * op_extra) {
 	void ** a = op->op_args;
 	GemmParams p;
@@ -1151,6 +1159,18 @@ extern "C" int amd_up_swiglu(Dataflow_Handle * dataflow_handle, int stream_id, O
 		return -1;
 	}
 	const long cu_count = extra_cu_count(op_extra);
+	const bool named = kernel_choice != AMD_MATMUL_KERNEL_AUTO;
+	if (apart && named) {
+		GemmParams one = p, three = p;
+		one.M = three.M = half;
+		one.x3_apart = three.x3_apart = 0;
+		three.A = p.A + (long long) half * p.K;
+		three.D = p.D + p.x3_apart;
+		if (launch_up_projection(one, single, cu_count, stream) || launch_up_projection(three, single, cu_count, stream)) {
+			return -1;
+		}
+		return launch_up_swiglu(p, half, three.D, half, stream);
+	}
 	if (single) {
 		return launch_direct<false, false, MODE_SINGLE, GATHER_NONE, true>(p, choose_tile(MODE_SINGLE, p, cu_count, false), stream);
 	}
@@ -1158,16 +1178,13 @@ extern "C" int amd_up_swiglu(Dataflow_Handle * dataflow_handle, int stream_id, O
 		return launch_direct<false, false, MODE_RAGGED_N, GATHER_Q_ROWS, true>(p, choose_tile(MODE_RAGGED_N, p, cu_count, false), stream);
 	}
 	const int tile = choose_tile(MODE_RAGGED_N, p, cu_count);
-	if (tile != TILE_BIG && kernel_choice == AMD_MATMUL_KERNEL_AUTO) {
+	if (tile != TILE_BIG && !named) {
 		return launch_direct<false, false, MODE_RAGGED_N, GATHER_Q_ROWS, true>(p, tile, stream);
 	}
-	if (launch_gemm<MODE_RAGGED_N>(p, 1, 0, true, tiles_of(p.M, 256) * ((long) p.N / 256 + p.num_groups), tiles_of(p.M, 128) * ((long) p.N / 128 + p.num_groups),
-								   cu_count, stream, tiles_of(p.M, 256) * ((long) p.N / 192 + p.num_groups))) {
+	if (launch_up_projection(p, false, cu_count, stream)) {
 		return -1;
 	}
-	const long long vectors = (long long) p.N * (half >> 3);
-	hipLaunchKernelGGL(up_swiglu_kernel, dim3((unsigned int) ((vectors + 255) / 256)), dim3(256), 0, stream, (const bf16_t *) p.D, p.h, (long long) p.N, half);
-	return check_launch();
+	return launch_up_swiglu(p, half, p.D + half, 2 * half, stream);
 }
 
 /* The layer's routing in one op (../layer/layer_ops.h): router product, selection, counts, prefix sum, permutation. */
