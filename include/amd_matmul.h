@@ -30,13 +30,15 @@ int amd_grouped_matmul(Dataflow_Handle * dataflow_handle, int stream_id, Op * op
 
 /* No counterpart in the reference.  For callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid it): D = alpha * op(A) op(B) + beta * C exactly as the matmul op computes
- * it with a workspace of 8 MiB (same kernels, same split along K, bit-identical results; to_trans_a / to_trans_b, M, K, N and the array layouts
- * as for dataflow_submit_matmul), with the fp32 partial sums of the split kept in a device array of the library itself
- * instead of a caller's workspace.  The call makes no allocation of any kind.  C is ignored when NULL or beta == 0.
- * Limit: a problem of few tiles and a long K (its 128 x 128 tiles leave half of the compute units idle, K is 512 or more) is
+ * it with a workspace that holds its split (same kernels, same split along K, bit-identical results; to_trans_a / to_trans_b, M, K, N and
+ * the array layouts as for dataflow_submit_matmul), with the fp32 partial sums of the split kept in a device array of the library itself,
+ * 64 MiB on each device, instead of a caller's workspace; 64 MiB hold every split that the op makes on a device of 256 compute
+ * units.  The call makes no allocation of any kind.  C is ignored when NULL or beta == 0.
+ * Limit: a problem of few tiles and a long K (its 128 x 128 tiles leave half of the compute units idle, K is more than 448) is
  * refused with -1 where a split over those compute units needs more than 8 MiB of partial sums (splits * M * N * 4 bytes).
- * Operands whose rows are not 16-byte aligned, which the op copies to padded rows in the workspace, are copied to the
- * same array where copies and partial sums fit; where they do not, the problem runs as the op runs it without a workspace.
+ * Operands whose rows are not 16-byte aligned, which the op copies to padded rows in its workspace, are copied to the
+ * same array: there the results are those of the op with a workspace of exactly 64 MiB, which copies and partial sums share; where the
+ * copies do not fit, the problem runs as the op runs it without a workspace.
  * Every call on a device shares that device's array: calls that overlap on one device (two streams, two host
  * threads) race on it.  Needs a handle on which dataflow_register_default_ops has run (that is where the array's
  * address on the handle's device is looked up). */

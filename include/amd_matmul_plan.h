@@ -17,6 +17,9 @@ enum { AMD_MATMUL_TILE_64x32, AMD_MATMUL_TILE_64x64, AMD_MATMUL_TILE_64x128, AMD
 /* has_c: D also takes C (beta is not 0) */
 int amd_matmul_planned_tile(int M, int K, int N, int has_c, int cu_count);
 
+/* Parts into which the matmul op splits K of an aligned problem with a workspace of that size (1: not split) */
+int amd_matmul_planned_splits(int to_trans_a, int to_trans_b, int M, int K, int N, int has_c, uint64_t workspace_bytes, int cu_count);
+
 /* Tilings of the token rows that a ragged-N launch without C goes out on where it runs on the persistent kernels: the sum of
  * one or two of these bits (D 16-byte aligned); with two, the device picks one from the group sizes */
 enum { AMD_MATMUL_ROWS_288 = 1, AMD_MATMUL_ROWS_384 = 2, AMD_MATMUL_ROWS_224 = 4, AMD_MATMUL_ROWS_192 = 8 };

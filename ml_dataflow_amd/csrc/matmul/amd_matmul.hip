@@ -38,10 +38,11 @@ struct MatmulExtra {
 };
 
 /* Scratch of amd_matmul_no_alloc: the fp32 partial sums of a split along K, which amd_matmul keeps in the caller's
- * workspace.  A file-scope device array: every GPU the library runs on holds its own copy at its own address until the
- * process ends.  In host code the name is only a handle for hipGetSymbolAddress; the address of each device's copy is
- * looked up once per device in amd_matmul_init and everything below uses that pointer. */
-#define AMD_MATMUL_SCRATCH_BYTES (8u << 20)
+ * workspace.  64 MiB hold every split that plan_split makes on 256 compute units (four work-groups each, 64 KiB of sums per work-group), so
+ * the call splits as the op does with any workspace that is large enough.  A file-scope device array: every GPU the library runs on holds
+ * its own copy at its own address until the process ends.  In host code the name is only a handle for hipGetSymbolAddress; the address of
+ * each device's copy is looked up once per device in amd_matmul_init and everything below uses that pointer. */
+#define AMD_MATMUL_SCRATCH_BYTES (64u << 20)
 #define AMD_MATMUL_MAX_DEVICES 64
 static __device__ __align__(256) unsigned char scratch[AMD_MATMUL_SCRATCH_BYTES];
 static void * scratch_of_device[AMD_MATMUL_MAX_DEVICES];
@@ -602,6 +603,22 @@ static long extra_cu_count(void * op_extra) {
 	return op_extra ? ((MatmulExtra *) op_extra)->cu_count : 256;
 }
 
+/* amd_matmul_no_alloc's limit, part of its interface: a problem whose 128 x 128 tiles leave half of the compute units idle, with a K of
+ * eight k-tiles or more, is refused where the partial sums of a split over those (a multiple of four k-tiles each) are more than 8 MiB.
+ * 0: taken; otherwise that number of splits */
+#define NO_ALLOC_LIMIT_BYTES (8u << 20)
+static long beyond_scratch(const GemmParams & p, bool direct, long cu_count) {
+	const long k_tiles = tiles_of(p.K, BK);
+	const bool big = tiles_of(p.M, 256) * tiles_of(p.N, 256) >= cu_count / 2 && p.M >= 256 && p.N >= 256;
+	long splits = direct && !big ? cu_count / (tiles_of(p.M, 128) * tiles_of(p.N, 128)) : 1;
+	if (splits < 2 || k_tiles < 8) {
+		return 0;
+	}
+	const long per = tiles_of(k_tiles, splits);
+	splits = tiles_of(k_tiles, per < 4 ? 4 : (per + 3) & ~3L);
+	return splits < 2 || (uint64_t) NO_ALLOC_LIMIT_BYTES / 4 / (uint64_t) splits >= (uint64_t) p.M * (uint64_t) p.N ? 0 : splits;
+}
+
 /* Few tiles and a long K (the router's GEMMs: up to 64 experts on one side; projections of few tokens): K split over the
  * compute units that the tiles leave idle, fp32 partial sums in `workspace` (16-byte aligned), added up by the pass behind.
  * Split where the cheapest tile and number of splits that the workspace holds cost less than the problem unsplit: the k-tiles
@@ -654,23 +671,13 @@ static int plan_split(GemmParams & p, int transa, int transb, bool direct, float
 	return best;
 }
 
-/* amd_matmul_no_alloc's limit: a problem whose 128 x 128 tiles leave half of the compute units idle, with a K of eight k-tiles or
- * more, needs room for the partial sums of a split over those (a multiple of four k-tiles each) */
-static bool beyond_scratch(const GemmParams & p, bool direct, uint64_t scratch_bytes, long cu_count) {
-	const long k_tiles = tiles_of(p.K, BK);
-	const bool big = tiles_of(p.M, 256) * tiles_of(p.N, 256) >= cu_count / 2 && p.M >= 256 && p.N >= 256;
-	long splits = direct && !big ? cu_count / (tiles_of(p.M, 128) * tiles_of(p.N, 128)) : 1;
-	if (splits < 2 || k_tiles < 8) {
-		return false;
-	}
-	const long per = tiles_of(k_tiles, splits);
-	splits = tiles_of(k_tiles, per < 4 ? 4 : (per + 3) & ~3L);
-	if (splits < 2 || scratch_bytes / 4 / (uint64_t) splits >= (uint64_t) p.M * (uint64_t) p.N) {
-		return false;
-	}
-	fprintf(stderr, "Error: this %d x %d x %d matmul may split along K into %ld parts of %lu partial sums each, more than the %lu-byte scratch holds; use the matmul op with a workspace...\n",
-			p.M, p.K, p.N, splits, (unsigned long) p.M * (unsigned long) p.N, (unsigned long) scratch_bytes);
-	return true;
+extern "C" int amd_matmul_planned_splits(int to_trans_a, int to_trans_b, int M, int K, int N, int has_c, uint64_t workspace_bytes, int cu_count) {
+	GemmParams p;
+	memset(&p, 0, sizeof(p));
+	p.M = M; p.K = K; p.N = N;
+	p.C = has_c ? (const bf16_t *) scratch_of_device : NULL;
+	/* an aligned workspace at no address in particular: the plan writes nothing */
+	return plan_split(p, to_trans_a, to_trans_b, true, (float *) 4096, workspace_bytes, cu_count) ? p.split_k : 1;
 }
 
 /* the pass behind the partial products: D from their sums */
@@ -792,7 +799,10 @@ static int run_matmul(Dataflow_Handle * dataflow_handle, int stream_id, GemmPara
 	if (padded < 0) {
 		return -1;
 	}
-	if (must_fit && !padded && beyond_scratch(p, direct, workspace_bytes, cu_count)) {
+	const long refused = must_fit && !padded ? beyond_scratch(p, direct, cu_count) : 0;
+	if (refused) {
+		fprintf(stderr, "Error: this %d x %d x %d matmul may split along K into %ld parts of %lu partial sums each, more than the %u bytes of scratch that one call may ask for; use the matmul op with a workspace...\n",
+				p.M, p.K, p.N, refused, (unsigned long) p.M * (unsigned long) p.N, NO_ALLOC_LIMIT_BYTES);
 		return -1;
 	}
 	const int split = plan_split(p, transa, transb, direct || padded, (float *) workspace, workspace_bytes, cu_count);
@@ -969,8 +979,7 @@ extern "C" int amd_matmul_twin(Dataflow_Handle * dataflow_handle, int stream_id,
 /* D = alpha * op(A) op(B) + beta * C like amd_matmul (same kernels, same split along K, bit-identical results), for
  * callers that cannot allocate: the split's partial sums go to the library's own scratch on the handle's device
  * instead of a caller's workspace, and the call makes no allocation of any kind.  BF16 operands and result, fp32
- * accumulation; C is ignored when NULL or beta == 0.  A problem whose split would need more than the scratch
- * (AMD_MATMUL_SCRATCH_BYTES, 8 MiB) is refused with -1.  The scratch keeps the last call's contents (nothing in it
+ * accumulation; C is ignored when NULL or beta == 0.  Refused with -1: see beyond_scratch.  The scratch keeps the last call's contents (nothing in it
  * has to start at zero: every partial sum is written before it is read); it is shared by every call on that device, so
  * calls that overlap on one device -- two streams, two host threads -- race on it. */
 extern "C" int amd_matmul_no_alloc(Dataflow_Handle * dataflow_handle, int stream_id, int to_trans_a, int to_trans_b,

@@ -2,6 +2,7 @@
 import ctypes as C
 import os
 
+import numpy as np
 import pytest
 
 from ml_dataflow_amd import binding as B
@@ -16,6 +17,7 @@ def plan():
     lib = C.CDLL(os.path.join(B.LIB_DIR, "libamd_matmul.so"))
     lib.amd_matmul_planned_tile.argtypes = [C.c_int] * 5
     lib.amd_matmul_planned_tilings.argtypes = [C.c_int] * 5
+    lib.amd_matmul_planned_splits.argtypes = [C.c_int] * 6 + [C.c_uint64, C.c_int]
     return lib
 
 
@@ -78,3 +80,19 @@ def test_a_good_tiling_for_uneven_rows_is_among_those_that_go_out(plan, M, K, ro
     best = min(t for bit, t in enumerate(us) if tilings >> bit & 1)
     # 13 %: the cost of the launch that loses, and what the rule leaves on the table (largest entry of this list: 12 %)
     assert best <= 1.13 * min(us), tilings
+
+
+def test_the_library_scratch_holds_every_split(plan):
+    """amd_matmul_no_alloc leaves the op's bits because no split needs more than its 64 MiB: the plan is the same with any larger
+    workspace."""
+    rng = np.random.default_rng(7)
+    split = 0
+    for _ in range(4000):
+        M, N = (8 * int(v) for v in np.exp(rng.uniform(0.0, np.log(1024.0), size=2)))
+        K = 8 * int(np.exp(rng.uniform(np.log(8.0), np.log(8192.0))))
+        for transa, transb in ((1, 0), (0, 0), (0, 1)):
+            parts = plan.amd_matmul_planned_splits(transa, transb, M, K, N, 1, 64 << 20, CUS)
+            assert parts == 1 or parts * M * N * 4 <= 64 << 20
+            assert parts == plan.amd_matmul_planned_splits(transa, transb, M, K, N, 1, 1 << 40, CUS), (M, K, N)
+            split += parts > 1
+    assert split > 500
