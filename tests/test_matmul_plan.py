@@ -1,6 +1,7 @@
 """What the matmul's host rules pick, checked on the CPU against measured times (include/amd_matmul_plan.h)."""
 import ctypes as C
 import os
+import sys
 
 import numpy as np
 import pytest
@@ -8,6 +9,7 @@ import pytest
 from ml_dataflow_amd import binding as B
 
 CUS = 256
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 TILES = ("64x32", "64x64", "64x128", "128x128", "128x128 pair", "256x256")
 
 
@@ -96,3 +98,14 @@ def test_the_library_scratch_holds_every_split(plan):
             assert parts == plan.amd_matmul_planned_splits(transa, transb, M, K, N, 1, 1 << 40, CUS), (M, K, N)
             split += parts > 1
     assert split > 500
+
+
+@pytest.mark.parametrize("largest,rows", [(6205, 288), (158, 192)])
+def test_bench_names_the_tiling_that_the_work_groups_pick(plan, largest, rows):
+    """both tilings go out for these sizes; the measured times above say which one the uneven groups need"""
+    sys.path.insert(0, ROOT)
+    import bench
+    assert plan.amd_matmul_planned_tilings(1024, 3072, 6478, 41, CUS) == 1 | 8
+    others = [(6478 - largest) // 40] * 40
+    others[0] += 6478 - largest - sum(others)
+    assert bench.ragged_n_tile_rows(1024, 3072, [largest] + others) == rows
