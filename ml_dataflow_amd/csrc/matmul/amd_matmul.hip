@@ -379,8 +379,8 @@ static int cheapest_tiling(const GemmParams & p, long groups, bool four_ok, int 
  * work-groups then agree on one of the two from the real sizes (ragged_n_choice).  A launch that loses costs 3 us, so both
  * go out only there.  Over 310 launches of the layer's kind (8-64 experts, 30-9000 rows each, K 512-4096) with even groups one launch on
  * the expected tiling takes 1.9 % longer than the best of all tilings; up to three launches, among them 288 always,
- * took 4.7 %.  A training step of 65536 tokens, 64 experts, dim 4096 37.75 -> 36.99 ms, a forward of 8192 tokens, 32 experts, dim
- * 2048 638 -> 622 us.  Over 341 launches whose rows lie in one, two or four of 8-64 experts to 95 % or are dealt by Zipf routers, this
+ * took 4.7 %.  A first training step of 3001 tokens, 32 experts, dim 2048 934 -> 905 us, a forward of 8192 tokens 635 -> 632, one with
+ * a Zipf router, whose launches take a second tiling, unchanged.  Over 341 launches whose rows lie in one, two or four of 8-64 experts to 95 % or are dealt by Zipf routers, this
  * rule is 3.4 % behind the best, without the second list 4.8 %, up to three launches 6.8 %; 17 / 41 of them are more than 3 % slower
  * than those three launches and 4 / 27 more than 8 % (1024 x 3072, 41 groups, 6205 of 6478 rows in one: 90 / 136 us, on 288 alone 87). */
 #define SECOND_TILING_MARGIN 121000          /* 4 us */
@@ -627,7 +627,10 @@ static long beyond_scratch(const GemmParams & p, bool direct, long cu_count) {
  * over all idle compute units wherever there were any, on 128 x 128 tiles, took 15 % longer.  1792 x 896 x 937, us: 8.0 unsplit on
  * 64 x 128 tiles, 19.9 split in two; 2176 x 19234 x 64: 20.9 in six on 64 x 64, 67.9 unsplit.
  * The router's logits (up to 64 rows of k-contiguous weights) are charged 1 us for the pass and a quarter for each split: the layer's
- * routing adds up their partial sums in its selection, whose few work-groups wait for a split's loads behind the last ones'.
+ * routing adds up their partial sums in its selection, whose few work-groups wait for a split's loads behind the last ones'.  A
+ * plain product of that form pays for the pass behind all the same, but has to split alike: the routing leaves the matmul's bits.  Over 63
+ * of them (8, 32 and 64 columns, 16-32768 tokens, K 512-4096) that price costs 1.6 us at most (8 or 32 x 2048 x 8192, 11.0 us
+ * against 9.4) and saves 1.3 at 3001 tokens; over all it is 0.6 % faster than the plain one.
  * 0: unsplit; otherwise the split in `p`, and its tile + 1. */
 #define SPLIT_ROUND_COST 50                 /* the partial sums' stores, beside their bytes below */
 #define SPLIT_PASS_COST 400

@@ -130,8 +130,8 @@ __device__ __forceinline__ long xcd_remap(long b, long total) {
 /* Inclusive sum over the lanes of a wave, and the value of the lane below (lane 0: `first`), in cross-lane moves of the
  * vector unit.  Every ragged launch starts with such a scan of the group sizes, a persistent work-group does one per tile
  * with the matrix pipes idle, and a shuffle through the LDS costs about a hundred clocks where a move costs eight (with
- * 32-bit divisions by the tiles of a row: a forward of 256 tokens 30.6 -> 28.9 us, a training step of 8192 tokens, 64
- * experts, dim 4096 5124 -> 5063). */
+ * 32-bit divisions by the tiles of a row: a forward of 256 tokens 30.4 -> 28.8 us, a training step of 8192 tokens, 64
+ * experts, dim 4096 5240 -> 5153, both sides on one card). */
 __device__ __forceinline__ int wave_inclusive_sum(int v) {
 	v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);      /* row_shr:1, 2, 4, 8 */
 	v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
