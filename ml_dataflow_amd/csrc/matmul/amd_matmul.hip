@@ -273,10 +273,11 @@ extern "C" int amd_matmul_select_kernel(int which) {
 	return 0;
 }
 
-/* the four-wave kernel takes whole k-tiles in pairs from k-contiguous operands, 16-byte lines of output, no C */
+/* the four-wave kernel takes whole k-tiles in pairs from k-contiguous operands, 16-byte lines of output, no C; a wave's rows of D
+ * (128 at most) stay below 2 GiB (W4_NO_COLUMN) */
 static bool w4_ok(const GemmParams & p) {
 	return !(p.C && p.beta != 0.0f) && (p.K % 128 == 0) && p.K <= (1 << 21) &&
-		   (p.M % 8 == 0) && ((((uintptr_t) p.D) & 15) == 0);
+		   (p.M % 8 == 0) && p.M <= (1 << 22) && ((((uintptr_t) p.D) & 15) == 0);
 }
 
 /* a ragged-N launch without C on one of its tilings; grid: an upper bound on the tiles */

@@ -154,14 +154,18 @@ __device__ __forceinline__ int wave_lane_below(int v, int first) {
  * and including it and in it alone; rows_before: rows of the groups in front of `base` */
 struct GroupScan { int end, start, incl, mine; };
 template <int BN>
-__device__ __forceinline__ GroupScan scan_groups(const GemmParams & p, int base, int lane, int rows_before) {
+__device__ __forceinline__ GroupScan scan_of_ends(const GemmParams & p, int base, int lane, int rows_before, int end) {
 	const int g = base + lane;
 	GroupScan s;
-	s.end = g < p.num_groups ? p.cumsum[g] : 0;
+	s.end = end;
 	s.start = wave_lane_below(s.end, rows_before);
 	s.mine = g < p.num_groups ? (s.end - s.start + BN - 1) / BN : 0;
 	s.incl = wave_inclusive_sum(s.mine);
 	return s;
+}
+template <int BN>
+__device__ __forceinline__ GroupScan scan_groups(const GemmParams & p, int base, int lane, int rows_before) {
+	return scan_of_ends<BN>(p, base, lane, rows_before, base + lane < p.num_groups ? p.cumsum[base + lane] : 0);
 }
 
 /* ragged N: the group of n-tile `nt` of the launch, its rows and which of its n-tiles that is */
@@ -317,8 +321,9 @@ __device__ __forceinline__ KGroups k_groups(const GemmParams & p, int lane, bool
 	return k;
 }
 
-/* tile `id` (0 <= id < count_tiles) of the launch; false if it has nothing to do.  k: of a ragged-K launch of up to 64 groups */
-template <int BM, int BN, int MODE>
+/* tile `id` (0 <= id < count_tiles) of the launch; false if it has nothing to do.  k: of a ragged-K launch of up to 64 groups; IN_LANES:
+ * and the ends in it of a ragged-N launch of as many */
+template <int BM, int BN, int MODE, bool IN_LANES = false>
 __device__ __forceinline__ bool resolve_tile_id(const GemmParams & p, long id, Tile & t, const KGroups & k = KGroups()) {
 	const int tiles_m = (p.M + BM - 1) / BM;
 	if (MODE == MODE_SINGLE) {
@@ -333,7 +338,14 @@ __device__ __forceinline__ bool resolve_tile_id(const GemmParams & p, long id, T
 	if (MODE == MODE_RAGGED_N) {
 		/* finds the group: a group owns tiles_m * (its n-tiles) consecutive ids */
 		const int nt = (int) ((unsigned int) id / (unsigned int) tiles_m);
-		const FoundGroup f = uniform_group(find_group<BN>(p, threadIdx.x & 63, nt));
+		FoundGroup f = {0, 0, 0, 0};
+		const int lane = IN_LANES ? __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : threadIdx.x & 63;
+		if (IN_LANES && p.num_groups <= 64) {
+			find_in_scan(p, scan_of_ends<BN>(p, 0, lane, 0, k.end), 0, lane, 0, nt, f);
+		} else {
+			f = find_group<BN>(p, lane, nt);
+		}
+		f = uniform_group(f);
 		/* f.nt counts whole rows of tiles_m ids inside the group; redo the split with the blocked order */
 		int tm, tn;
 		tile_in_problem(f.nt * tiles_m + ((int) id - nt * tiles_m), tiles_m, (f.rows + BN - 1) / BN, tm, tn);

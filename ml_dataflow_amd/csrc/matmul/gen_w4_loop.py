@@ -51,7 +51,7 @@ M_BF, M_AF, M_ARD, M_BRD = 128, 176, 192, 200                 # v[0:127]: accumu
 # schedule parameters (W4_OPTS="key=value,..." overrides them for experiments; ablations give wrong results, timing only)
 OPTS = {"abl": "", "pre": 4, "first": 2, "every": 3, "qfirst": 14, "qevery": 13}
 for kv in os.environ.get("W4_OPTS", "").split(","):
-    if "=" in kv:
+    if "=" in kv and kv.split("=", 1)[0] in OPTS:
         k_, v_ = kv.split("=", 1)
         OPTS[k_] = type(OPTS[k_])(v_)
 ABL = set(OPTS["abl"].split("+")) if OPTS["abl"] else set()
@@ -168,6 +168,8 @@ class Mult(Asm):
         for m in range(192):
             s, rem = divmod(m, 96)
             i, j = divmod(rem, 6)
+            if i & 1:
+                j = 5 - j                        # one operand stays from each MFMA to the next: 0.8 % less time at the card's power limit
             a = s * 16 + i
             self.need(("A", a % 4), ("B", s, j))
             self.e("v_mfma_f32_16x16x32_bf16 %s, %s, %s, %s" % (self.acc(i, j), vr(M_AF + (a % 4) * 4, 4), vr(M_BF + s * 24 + j * 4, 4), self.acc(i, j)))
@@ -296,10 +298,82 @@ class Loader(Asm):
 
 # ================================================================================================ four symmetric waves, 256 x 384
 QW_STAGE = 49152         # bytes of one Q stage of the wide tile (384 rows x 64 k)
-D_VP, D_VQ, D_VQ_NEXT = 208, 216, 228                         # this lane's offsets of the wave's 8 chunks of P, 12 of Q, the next tile's Q
+D_VP, D_VQ, D_VQ_NEXT, D_AT = 208, 216, 228, 240              # this lane's offsets of the wave's 8 chunks of P, 12 of Q, the next tile's Q, of D
 
 
-class Wide(Mult):
+class Tail(Asm):
+    """The epilogue of the kernels below, a part of their statements: the compiler, given 256 accumulators or more to read, kept 16 to 40
+    of them in scratch memory, waited there for its own stores, and for every second load of C.  A wave's results are groups of 64 (m) x 16
+    (n), two accumulators of 8 per lane; they leave as whole 128-byte lines without the LDS:
+      1. Pairs of row blocks change lane rows (v_permlane16_swap_b32: lane rows 1 and 3 of block i with lane rows 0 and 2 of block
+         i + 1): a lane then holds m = 8 (grp / 2) .. + 7 of block i + (grp & 1), 16 bytes, and the four lane rows of one n hold 64
+         consecutive bytes.
+      2. Two such pairs (blocks i, i + 1 and i + 2, i + 3) are merged across the halves of a lane row (a DPP rotation by eight
+         lanes, written to one half only): one store carries both pairs of eight n, 128 consecutive bytes per n.
+    The first store of a group carries n = 0-7 (lanes 0-7 of a lane row the first pair, lanes 8-15 the second), the second n = 8-15 (the
+    other way round).  s32 / s33: address of the wave's first element of D, s34: bytes from there to the end of its rows, s35: bytes of 16
+    rows, s38: alpha.  v[at + 2 h], v[at + 2 h + 1]: this lane's offset of the first and the second store of group (0, h), outside any buffer
+    where its columns do not exist.  Rows that do not exist lie past s34.  All stores are issued always: the waits of the next statement
+    count them."""
+
+    def valu(self, text, dst, cross=()):
+        """a vector instruction that writes the registers `dst`; the cross-lane reads `cross` need two others behind their writer"""
+        behind = min([self.count - self.written.get(v, -9) for v in cross] + [3])
+        if behind <= 2:
+            self.e("s_nop %d" % (2 - behind))
+            self.count += 3 - behind
+        self.e(text)
+        for v in dst:
+            self.written[v] = self.count
+        self.count += 1
+
+    def swap(self, a, b):
+        self.valu("v_permlane16_swap_b32 v%d, v%d" % (a, b), (a, b), (a, b))
+
+    def dpp(self, dst, src, ctrl, bank):
+        self.valu("v_mov_b32_dpp v%d, v%d %s row_mask:0xf bank_mask:0x%x" % (dst, src, ctrl, bank), (dst,), (src,))
+
+    def descriptor(self, d, address):
+        for ins in ("s_mov_b32 s%d, s%d" % (d, address), "s_mov_b32 s%d, s%d" % (d + 1, address + 1), "s_mov_b32 s%d, s34" % (d + 2),
+                    "s_mov_b32 s%d, 0x00020000" % (d + 3)):
+            self.e(ins)
+
+    def accumulators(self, group, t, scale):
+        """the 16 results of a group, as registers (copied to t .. t + 15 from the accumulation registers), times alpha"""
+        src = t
+        if group < 16:
+            for r in range(16):
+                self.valu("v_accvgpr_read_b32 v%d, a%d" % (t + r, 16 * group + r), (t + r,))
+        else:
+            src = 16 * (group - 16)
+        if scale:
+            for r in range(16):
+                self.valu("v_mul_f32 v%d, s38, v%d" % (t + r, src + r), (t + r,))
+            src = t
+        return src
+
+    def store_group(self, src, t, at):
+        """16 results to D; t .. t + 3 and t + 16 .. t + 19 carry the stores"""
+        for k in range(8):
+            self.valu("v_cvt_pk_bf16_f32 v%d, v%d, v%d" % (t + k, src + 2 * k, src + 2 * k + 1), (t + k,))
+        for a in (t, t + 1, t + 4, t + 5):
+            self.swap(a, a + 2)
+        for k in range(4):
+            self.valu("v_mov_b32 v%d, v%d" % (t + 16 + k, t + k), (t + 16 + k,))
+        for k in range(4):
+            self.dpp(t + k, t + 4 + k, "row_ror:8", 0xC)
+        for k in range(4):
+            self.dpp(t + 16 + k, t + 4 + k, "row_ror:8", 0x3)
+        self.e("buffer_store_dwordx4 %s, v%d, s[92:95], 0 offen nt" % (vr(t, 4), at))
+        self.e("buffer_store_dwordx4 %s, v%d, s[92:95], 0 offen nt" % (vr(t + 16, 4), at + 1))
+        self.count += 2
+
+    def next_rows(self, at, n):
+        for k in range(n):
+            self.valu("v_add_u32 v%d, s35, v%d" % (at + k, at + k), (at + k,))
+
+
+class Wide(Mult, Tail):
     """gemm_bf16_w4d_kernel: tile 256 (m) x 384 (n) x 64 (k), four waves that all do both jobs.  Wave w multiplies columns
     [96 w, 96 w + 96) of the tile like a multiplying wave above (same fragment reads, same MFMA order) and loads a quarter
     of every k-tile -- chunks 8 w .. 8 w + 7 of P and 12 w .. 12 w + 11 of Q, 20 KiB -- straight into the LDS
@@ -318,11 +392,12 @@ class Wide(Mult):
     the tile has no k-tile g + 2 they switch to the next tile's first one.
 
     s[40:47] this tile's cursor at k-tile 0, s[48:55] the next tile's (empty buffers when there is none), s56 k-tiles
-    (even), s57 bit 0: first tile of the work-group, s58 / s59 bytes per k-tile of P / Q, s61 / s62 LDS address of the
-    wave's first chunk of P / Q in stage 0.  Working registers as in the loader above.
+    (even), s57 bit 0: first tile of the work-group, s58 / s59 bytes per k-tile of P / Q, s60 LDS address of the stages,
+    s61 / s62 of the wave's first chunk of P / Q in stage 0, s63 bytes from s60 to the wave's rows of Q.  Working registers as in the loader above.
 
-    State from statement to statement: stage 0 holds k-tile 0 of the tile, visible to all waves; the Q rows and the first
-    `pre` chunks of P of k-tile 1 are in flight into stage 1; the Q offsets of the tile are in v[D_VQ ...]."""
+    State from statement to statement: stage 0 holds k-tile 0 of the tile, visible to all waves; the rows of Q and P of k-tile 1 are
+    in flight into stage 1, and behind them the 48 stores of the tile before; the Q offsets of the tile are in v[D_VQ ...].  Epilogue as
+    in class Tail; s57 bit 2: alpha is not 1."""
 
     LOADS_P, LOADS_Q = 8, 12
 
@@ -376,7 +451,7 @@ class Wide(Mult):
         else:
             self.advance(which)
 
-    def step(self, p):
+    def step(self, p, start=False):
         after = {}
 
         def at(m, fn):
@@ -386,8 +461,9 @@ class Wide(Mult):
         assert 1 <= pre <= 4 and first + every * (self.LOADS_P - pre - 1) < qfirst
         assert qfirst >= 8 and qfirst + qevery * (self.LOADS_Q - 1) < 179
         # the rest of the P rows of k-tile g + 1, into the other stage
-        for n, u in enumerate(range(pre, self.LOADS_P)):
-            at(first + every * n, lambda u=u: self.dma_p(1 - p, u))
+        if not start:                        # of the first k-tile they are out in front of the epilogue
+            for n, u in enumerate(range(pre, self.LOADS_P)):
+                at(first + every * n, lambda u=u: self.dma_p(1 - p, u))
         # the fragments of Q of k-step 1 first: with them in registers the wave's Q rows of this stage are free
         for j in range(6):
             at(j, lambda j=j: self.read_B(p, 1, j))
@@ -400,7 +476,14 @@ class Wide(Mult):
             at(6 * (a - 4) + 5, lambda a=a: self.read_A(p, a))
 
         def barrier():
-            self.e("s_waitcnt vmcnt(%d)" % self.LOADS_Q)
+            if start:                            # behind the first tile's loads, or the stores of the tile before
+                self.e("s_bitcmp1_b32 s57, 0")
+                self.e("s_cbranch_scc0 7f")
+                self.e("s_waitcnt vmcnt(%d)" % self.LOADS_Q)
+                self.e("7:")
+                self.e("s_waitcnt vmcnt(%d)" % (self.LOADS_Q + 48))
+            else:
+                self.e("s_waitcnt vmcnt(%d)" % self.LOADS_Q)
             self.lds_drain()
             self.barrier()
             self.tail_reads(1 - p, 0)
@@ -413,14 +496,54 @@ class Wide(Mult):
         for m in range(192):
             s, rem = divmod(m, 96)
             i, j = divmod(rem, 6)
+            if i & 1:
+                j = 5 - j                        # one operand stays from each MFMA to the next: 0.8 % less time at the card's power limit
             a = s * 16 + i
             self.need(("A", a % 4), ("B", s, j))
-            self.e("v_mfma_f32_16x16x32_bf16 %s, %s, %s, %s" % (self.acc(i, j), vr(M_AF + (a % 4) * 4, 4), vr(M_BF + s * 24 + j * 4, 4), self.acc(i, j)))
+            self.e("v_mfma_f32_16x16x32_bf16 %s, %s, %s, %s" % (self.acc(i, j), vr(M_AF + (a % 4) * 4, 4), vr(M_BF + s * 24 + j * 4, 4), "0" if start and s == 0 else self.acc(i, j)))
             for fn in after.get(m, []):
                 fn()
 
+    def addresses(self):
+        """fragment read addresses of this lane, from its number (kept out of the compiler's hands: it has eight registers across the
+        statement): row l % 16, chunk 4 s + l / 16 of a k-contiguous operand, four k-rows from 8 (l / 16) on of a k-major one"""
+        e = self.e
+        l15, g4, sw, t = M_BF, M_BF + 1, M_BF + 2, M_BF + 3
+        e("v_mbcnt_lo_u32_b32 v%d, -1, 0" % t)
+        e("v_mbcnt_hi_u32_b32 v%d, -1, v%d" % (t, t))
+        e("v_and_b32 v%d, 15, v%d" % (l15, t))
+        e("v_lshrrev_b32 v%d, 4, v%d" % (g4, t))
+        if self.PKM:                             # k-row 8 g4 + l15 / 4, rows 16 i + 4 (l15 % 4), swizzled as kmajor_swizzle does
+            e("v_lshrrev_b32 v%d, 2, v%d" % (sw, l15))
+            e("v_lshl_add_u32 v%d, v%d, 3, v%d" % (t, g4, sw))
+            e("v_lshlrev_b32 v%d, 5, v%d" % (sw, sw))
+            e("v_and_b32 v%d, 0x60, v%d" % (sw, sw))
+            e("v_and_b32 v%d, 1, v%d" % (t + 1, g4))
+            e("v_lshlrev_b32 v%d, 4, v%d" % (t + 1, t + 1))
+            e("v_xor_b32 v%d, v%d, v%d" % (sw, sw, t + 1))
+            e("v_lshlrev_b32 v%d, 9, v%d" % (t, t))
+            e("v_add_u32 v%d, s60, v%d" % (t, t))
+            e("v_and_b32 v%d, 3, v%d" % (t + 1, l15))
+            e("v_lshlrev_b32 v%d, 2, v%d" % (t + 1, t + 1))
+            for n in range(8):
+                e("v_add_u32 v%d, %d, v%d" % (M_ARD + n, 16 * n, t + 1))
+                e("v_xor_b32 v%d, v%d, v%d" % (M_ARD + n, M_ARD + n, sw))
+                e("v_lshl_add_u32 v%d, v%d, 1, v%d" % (M_ARD + n, M_ARD + n, t))
+        e("v_lshrrev_b32 v%d, 1, v%d" % (sw, l15))
+        e("v_lshlrev_b32 v%d, 7, v%d" % (l15, l15))
+        e("v_add_u32 v%d, s60, v%d" % (l15, l15))
+        for s in range(2):
+            e("v_add_u32 v%d, %d, v%d" % (t, 4 * s, g4))
+            e("v_xor_b32 v%d, v%d, v%d" % (t, t, sw))
+            e("v_lshl_add_u32 v%d, v%d, 4, v%d" % (t, t, l15))
+            if not self.PKM:
+                e("v_mov_b32 v%d, v%d" % (M_ARD + s, t))
+            e("v_add_u32 v%d, s63, v%d" % (M_BRD + 2 * s, t))
+            e("v_add_u32 v%d, %d, v%d" % (M_BRD + 2 * s + 1, QW_STAGE, M_BRD + 2 * s))
+
     def generate(self):
         e = self.e
+        self.addresses()
         self.set_cursor(40, 0)
         self.set_cursor(40, 1)
         e("s_mov_b32 s76, 0")
@@ -434,7 +557,7 @@ class Wide(Mult):
         e("s_barrier")
         self.advance(0)
         self.advance(1)
-        for u in range(OPTS["pre"]):
+        for u in range(self.LOADS_P):
             self.dma_p(1, u)
         for q in range(self.LOADS_Q):
             self.dma_q(1, q)
@@ -445,21 +568,44 @@ class Wide(Mult):
         e("4:")
         for which in range(3):
             self.tail_reads(0, which)
-        e("3:")
-        self.loop_head_state()
-        self.step(0)
-        self.loop_head_state()
-        self.step(1)
-        e("s_add_u32 s76, s76, 2")
-        e("s_cmp_lt_u32 s76, s56")
-        e("s_cbranch_scc1 3b")
+        for first in (True, False):          # the first two k-tiles start the sums
+            if not first:
+                e("3:")
+            self.loop_head_state()
+            self.step(0, first)
+            self.loop_head_state()
+            self.step(1)
+            e("s_add_u32 s76, s76, 2")
+            e("s_cmp_lt_u32 s76, s56")
+            e("s_cbranch_scc0 9f" if first else "s_cbranch_scc1 3b")
+        e("9:")
         e("s_waitcnt lgkmcnt(0)")
+        for u in range(OPTS["pre"], self.LOADS_P):
+            self.dma_p(1, u)
+        self.descriptor(92, 32)
         for _ in range(3):
             e("s_nop 7")
+        e("s_bitcmp1_b32 s57, 2")
+        e("s_cbranch_scc1 10f")
+        self.epilogue(False)
+        e("s_branch 11f")
+        e("10:")
+        self.epilogue(True)
+        e("11:")
         return self.L
 
+    def epilogue(self, scale):
+        self.count, self.written = 0, {}
+        for n in range(24):
+            j, h = divmod(n, 4)
+            if h == 0 and j:
+                self.next_rows(D_AT, 8)
+            t = M_BF + 24 * (n & 1)
+            self.store_group(self.accumulators(6 * h + j, t, scale), t, D_AT + 2 * h)
+
     def clobbers(self):
-        return ["v%d" % i for i in range(M_BF, M_ARD)] + ["s%d" % i for i in range(64, 78)] + ["m0", "scc", "memory"]
+        return ["v%d" % i for i in range(D_VP)] + ["a%d" % i for i in range(256)] + ["s%d" % i for i in range(64, 78)] + \
+               ["s%d" % i for i in range(92, 96)] + ["m0", "scc", "memory"]
 
 
 def main():
@@ -485,12 +631,11 @@ def main():
         f.write('#define W4_LOAD_INPUTS(vp, wr, wr4, sa, sb, sc) "{v[%d:%d]}"(vp), "{v[%d:%d]}"(wr[0]), "{v[%d:%d]}"(wr[1]), "{v[%d:%d]}"(wr4), "{s[40:47]}"(sa), "{s[48:55]}"(sb), "{s[56:63]}"(sc)\n' %
                 (L_VOFFP, L_VOFFP + 31, L_WR, L_WR + 31, L_WR + 32, L_WR + 63, L_WR + 64, L_WR + 67))
         f.write('#define W4_LOAD_INPUTS_NEXT(vn, vn4) "{v[%d:%d]}"(vn), "{v[%d:%d]}"(vn4)\n' % (L_VOFFQ_NEXT, L_VOFFQ_NEXT + 31, L_VOFFQ_NEXT + 32, L_VOFFQ_NEXT + 35))
-        # wide symmetric kernel: accumulator groups as above, fragment read addresses lb, the lane's load offsets vo (8 of P,
-        # 12 of Q, 12 of the next tile's Q), cursors sa, sb and the block sc (k-tiles, flags, bytes per k-tile of P and Q,
-        # unused, LDS address of the wave's first chunk of P and of Q in stage 0, unused)
-        f.write('#define W4D_OUTPUTS(g, vo) W4_MULT_OUTPUTS(g), "+{v[%d:%d]}"(vo)\n' % (D_VP, D_VP + 31))
-        f.write('#define W4D_INPUTS(lb, sa, sb, sc) "{v[%d:%d]}"(lb), "{s[40:47]}"(sa), "{s[48:55]}"(sb), "{s[56:63]}"(sc)\n' % (M_ARD, M_ARD + 15))
-        f.write("#define W4D_VP 0\n#define W4D_VQ %d\n#define W4D_VQ_NEXT %d\n#define W4D_PRE %d\n" % (D_VQ - D_VP, D_VQ_NEXT - D_VP, OPTS["pre"]))
+        # wide symmetric kernel: the lane's load offsets vo (8 of P, 12 of Q, 12 of the next tile's Q) and its eight of D (in and out, though
+        # those of P do not change: of an input the compiler kept a copy in scratch memory), the blocks of scalars sd, sa, sb, sc
+        f.write('#define W4D_OUTPUTS(vo, at) "+{v[%d:%d]}"(vo), "+{v[%d:%d]}"(at)\n' % (D_VP, D_VP + 31, D_AT, D_AT + 7))
+        f.write('#define W4D_INPUTS(sd, sa, sb, sc) "{s[32:39]}"(sd), "{s[40:47]}"(sa), "{s[48:55]}"(sb), "{s[56:63]}"(sc)\n')
+        f.write("#define W4D_VP 0\n#define W4D_VQ %d\n#define W4D_VQ_NEXT %d\n" % (D_VQ - D_VP, D_VQ_NEXT - D_VP))
 
 if __name__ == "__main__":
     main()

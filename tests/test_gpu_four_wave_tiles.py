@@ -1,0 +1,62 @@
+"""What the four-wave GEMM kernels do between two tiles (epilogue, walk over the tiles), at the edges of tiles, groups and k-tiles:
+bit for bit what the eight-wave kernel leaves, which test_gpu_ops.py holds to the oracle, and nothing past the end of D."""
+import ctypes as C
+import os
+
+import numpy as np
+import pytest
+
+from ml_dataflow_amd import binding as B
+from util import normal_bf16
+
+pytestmark = pytest.mark.gpu
+
+BF = B.DATAFLOW_BF16
+CS = 1
+AUTO, EIGHT, FOUR_384 = 0, 8, 384
+GUARD = 4096            # elements behind D that have to stay as they are
+
+
+@pytest.fixture(scope="module")
+def select_kernel(backend):
+    lib = C.CDLL(os.path.join(os.path.dirname(B.__file__), "lib", "libamd_matmul.so"))
+    lib.amd_matmul_select_kernel.argtypes = [C.c_int]
+    yield lib.amd_matmul_select_kernel
+    assert lib.amd_matmul_select_kernel(AUTO) == 0
+
+
+def both(be, select_kernel, other, elements, start, submit):
+    """D of the eight-wave kernel and of `other`, from the same values in it, and the guard behind the second"""
+    got = {}
+    filled = np.concatenate([start.reshape(-1), np.full(GUARD, 0x4242, np.uint16)])
+    for kernel in (EIGHT, other):
+        d_D = be.upload(filled)
+        assert select_kernel(kernel) == 0
+        assert submit(d_D) == 0
+        be.sync(CS)
+        got[kernel] = be.read(d_D.ptr, (elements + GUARD,), np.uint16)
+        d_D.free()
+    assert select_kernel(AUTO) == 0
+    assert (got[other][elements:] == 0x4242).all()
+    bad = got[other] != got[EIGHT]
+    assert not bad.any(), "%d of %d elements differ, first at %s" % (int(bad.sum()), bad.size, np.flatnonzero(bad)[:4].tolist())
+
+
+@pytest.mark.parametrize("transa", [1, 0])
+@pytest.mark.parametrize("alpha", [1.0, -0.75])
+@pytest.mark.parametrize("M,K,groups", [(1304, 128, 70), (264, 384, 64), (2048, 256, 130)])
+def test_ragged_n_many_groups(backend, select_kernel, transa, alpha, M, K, groups):
+    """more groups than lanes, and as many; tiles partial in both directions; a work-group walks over many short tiles"""
+    be = backend
+    rng = np.random.default_rng(M + K + groups + transa)
+    counts = rng.choice([0, 1, 95, 96, 97, 191, 193, 288, 383, 384, 385, 500], size=groups).astype(np.int32)
+    counts[0], counts[-1] = 385, 97
+    total = int(counts.sum())
+    print("case four waves, N: ta=%d alpha=%g M=%d K=%d G=%d rows=%d" % (transa, alpha, M, K, groups, total), flush=True)
+    d_W = be.upload(normal_bf16(rng, (groups, M, K) if transa else (groups, K, M), 0.05))
+    d_X, d_cum = be.upload(normal_bf16(rng, (total, K))), be.upload(np.cumsum(counts).astype(np.int32))
+    both(be, select_kernel, FOUR_384, total * M, np.zeros(total * M, np.uint16), lambda d_D: be.lib.dataflow_submit_amd_grouped_matmul(
+        be.hp, CS, BF, BF, B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, transa, 0, B.AMD_GROUPED_RAGGED_N, M, K, total, groups, d_cum.ptr, alpha, 0.0,
+        d_W.ptr, M * K * 2, d_X.ptr, None, d_D.ptr, 0))
+    for d in (d_W, d_X, d_cum):
+        d.free()
