@@ -397,13 +397,15 @@ class Wide(Mult, Tail):
 
     State from statement to statement: stage 0 holds k-tile 0 of the tile, visible to all waves; the rows of Q and P of k-tile 1 are
     in flight into stage 1, and behind them the 48 stores of the tile before; the Q offsets of the tile are in v[D_VQ ...].  Epilogue as
-    in class Tail; s57 bit 2: alpha is not 1."""
+    in class Tail; s57 bit 2: alpha is not 1.  Three macros: what every tile starts with, the first tile's loads and the loop, the first two
+    steps, which come in front of the loop but stand behind it, and the epilogue."""
 
     LOADS_P, LOADS_Q = 8, 12
 
     def __init__(self, PKM, GATHER):
         Mult.__init__(self, PKM)
         self.GATHER = GATHER
+        self.parts = []
         self.name = "W4D_%s_%s" % ("PKM" if PKM else "PKC", "GATHER" if GATHER else "PACKED")
 
     # which: 0 = P (descriptor s[64:67], bytes left s[72:73]), 1 = Q (s[68:71], s[74:75])
@@ -549,6 +551,7 @@ class Wide(Mult, Tail):
         e("s_mov_b32 s76, 0")
         e("s_bitcmp1_b32 s57, 0")
         e("s_cbranch_scc0 2f")
+        self.part("HEAD")
         for u in range(self.LOADS_P):        # first tile: k-tile 0, then the first loads of k-tile 1
             self.dma_p(0, u)
         for q in range(self.LOADS_Q):
@@ -557,10 +560,19 @@ class Wide(Mult, Tail):
         e("s_barrier")
         self.advance(0)
         self.advance(1)
-        for u in range(self.LOADS_P):
+        for u in range(OPTS["pre"]):
             self.dma_p(1, u)
         for q in range(self.LOADS_Q):
             self.dma_q(1, q)
+        e("s_branch 12f")
+        e("3:")
+        self.two_steps(False)
+        e("s_cbranch_scc1 3b")
+        e("s_branch 9f")
+        self.part("ASM")
+        e("12:")                             # the rest of the first tile's P
+        for u in range(OPTS["pre"], self.LOADS_P):
+            self.dma_p(1, u)
         e("s_branch 4f")
         e("2:")
         self.advance(0)
@@ -568,16 +580,8 @@ class Wide(Mult, Tail):
         e("4:")
         for which in range(3):
             self.tail_reads(0, which)
-        for first in (True, False):          # the first two k-tiles start the sums
-            if not first:
-                e("3:")
-            self.loop_head_state()
-            self.step(0, first)
-            self.loop_head_state()
-            self.step(1)
-            e("s_add_u32 s76, s76, 2")
-            e("s_cmp_lt_u32 s76, s56")
-            e("s_cbranch_scc0 9f" if first else "s_cbranch_scc1 3b")
+        self.two_steps(True)                 # the first two k-tiles start the sums
+        e("s_cbranch_scc1 3b")
         e("9:")
         e("s_waitcnt lgkmcnt(0)")
         for u in range(OPTS["pre"], self.LOADS_P):
@@ -592,7 +596,21 @@ class Wide(Mult, Tail):
         e("10:")
         self.epilogue(True)
         e("11:")
-        return self.L
+        self.part("END")
+        return self.parts
+
+    def part(self, name):
+        """the lines since the last part, as a macro of their own"""
+        self.parts.append(("%s_%s" % (self.name, name), self.L))
+        self.L = []
+
+    def two_steps(self, start):
+        self.loop_head_state()
+        self.step(0, start)
+        self.loop_head_state()
+        self.step(1)
+        self.e("s_add_u32 s76, s76, 2")
+        self.e("s_cmp_lt_u32 s76, s56")
 
     def epilogue(self, scale):
         self.count, self.written = 0, {}
@@ -613,8 +631,11 @@ def main():
     with open(out, "w") as f:
         f.write("/* generated by gen_w4_loop.py -- do not edit */\n")
         for v in (Mult(False), Mult(True), Loader(False), Loader(True), Wide(False, False), Wide(False, True), Wide(True, False), Wide(True, True)):
-            lines = v.generate()
-            f.write("#define %s_ASM \\\n" % v.name + " \\\n".join('\t"%s\\n\\t"' % x for x in lines) + "\n")
+            parts = v.generate()
+            if not isinstance(v, Wide):
+                parts = [(v.name + "_ASM", parts)]
+            for name, lines in parts:
+                f.write("#define %s \\\n" % name + " \\\n".join('\t"%s\\n\\t"' % x for x in lines) + "\n")
             f.write("#define %s_CLOBBERS %s\n" % (v.name, ", ".join('"%s"' % c for c in v.clobbers())))
         # multiplying waves: accumulator groups g[0..23] (group 6 (i / 4) + j holds row blocks 4 (i / 4) .. + 3 of column block
         # j), the lane block lb (fragment read addresses), k-tiles and flags
@@ -635,6 +656,7 @@ def main():
         # those of P do not change: of an input the compiler kept a copy in scratch memory), the blocks of scalars sd, sa, sb, sc
         f.write('#define W4D_OUTPUTS(vo, at) "+{v[%d:%d]}"(vo), "+{v[%d:%d]}"(at)\n' % (D_VP, D_VP + 31, D_AT, D_AT + 7))
         f.write('#define W4D_INPUTS(sd, sa, sb, sc) "{s[32:39]}"(sd), "{s[40:47]}"(sa), "{s[48:55]}"(sb), "{s[56:63]}"(sc)\n')
+        f.write("#define W4D_PRE %d\n" % OPTS["pre"])
         f.write("#define W4D_VP 0\n#define W4D_VQ %d\n#define W4D_VQ_NEXT %d\n" % (D_VQ - D_VP, D_VQ_NEXT - D_VP))
 
 if __name__ == "__main__":
