@@ -161,14 +161,14 @@ def replay_step_with_events(be, layer, T, d_X, d_out, d_dY, d_dX, d_bias, backwa
             grouped("gemm_nn", 0, 0, B.AMD_GROUPED_RAGGED_N, H, D, R, 0.0, L.w2, S, L.expert_zones, None, dh, 0)
             timed("swiglu_bwd_x_routed", lib.dataflow_submit_amd_swiglu_bwd_x_routed, hp, CS, BF, BF, R, H, E, K, 2 * H, 2 * H, L.expert_mapping,
                   L.token_mapping, L.chosen_experts, L.token_expert_weights, L.x1, L.x1 + 2 * H, dh, L.d_routed, L.dx1, L.dx1 + 2 * H, ws)
-            grouped("gemm_nt_dw", 0, 1, B.AMD_GROUPED_RAGGED_K, H, 0, D, wbeta, ws, 0, L.expert_zones, wc(L.dw2), L.dw2, S)
+            grouped("gemm_nt_dw", 0, 1, B.AMD_GROUPED_RAGGED_K, H, R, D, wbeta, ws, 0, L.expert_zones, wc(L.dw2), L.dw2, S)
             grouped("gemm_dx13", 0, 0, B.AMD_GROUPED_RAGGED_N, D, 2 * H, R, 0.0, L.w1, S, L.dx1, None, L.expert_zones, 0)
         else:
             timed("swiglu", lib.dataflow_submit_default_swiglu, hp, CS, BF, R, H, L.x1, L.x3, ws)
             grouped("gemm_tn", 1, 0, B.AMD_GROUPED_RAGGED_N, D, H, R, 0.0, L.w2, S, ws, None, L.expert_zones, 0)
             timed("router_bwd_x", lib.dataflow_submit_amd_router_bwd_x_all, hp, CS, BF, BF, T, D, E, K, L.token_mapping, L.chosen_experts,
                   L.token_expert_weights, L.expert_zones, d_dY.ptr, L.d_routed, L.expert_zones)
-            grouped("gemm_nt_dw", 0, 1, B.AMD_GROUPED_RAGGED_K, H, 0, D, wbeta, ws, 0, L.expert_zones, wc(L.dw2), L.dw2, S)
+            grouped("gemm_nt_dw", 0, 1, B.AMD_GROUPED_RAGGED_K, H, R, D, wbeta, ws, 0, L.expert_zones, wc(L.dw2), L.dw2, S)
             grouped("gemm_nn", 0, 0, B.AMD_GROUPED_RAGGED_N, H, D, R, 0.0, L.w2, S, L.expert_zones, None, L.dx1, 0)
             timed("swiglu_bwd_x", lib.dataflow_submit_default_swiglu_bwd_x, hp, CS, BF, BF, R, H, L.x1, L.x3, L.dx1, L.dx1, L.dx3)
             grouped("gemm_nn", 0, 0, B.AMD_GROUPED_RAGGED_N, D, H, R, 0.0, L.w1, S, L.dx1, None, L.expert_zones, 0)
@@ -183,11 +183,11 @@ def replay_step_with_events(be, layer, T, d_X, d_out, d_dY, d_dX, d_bias, backwa
               L.kernel_workspace_bytes, ws)
         timed("dispatch", lib.dataflow_submit_default_prepare_experts, hp, CS, BF, BF, T, D, K, d_X.ptr, L.token_mapping, L.expert_zones)
         if fused:
-            timed("gemm_dw13", lib.dataflow_submit_amd_grouped_matmul, hp, CS, BF, BF, wdt, BF, F32, 0, 1, B.AMD_GROUPED_RAGGED_K, D, 0, 2 * H, E, cum,
+            timed("gemm_dw13", lib.dataflow_submit_amd_grouped_matmul, hp, CS, BF, BF, wdt, BF, F32, 0, 1, B.AMD_GROUPED_RAGGED_K, D, R, 2 * H, E, cum,
                   1.0, wbeta, L.expert_zones, 0, L.dx1, wc(L.dw1), L.dw1, S)
         else:
-            grouped("gemm_nt_dw", 0, 1, B.AMD_GROUPED_RAGGED_K, D, 0, H, wbeta, L.expert_zones, 0, L.dx1, wc(L.dw1), L.dw1, S)
-            grouped("gemm_nt_dw", 0, 1, B.AMD_GROUPED_RAGGED_K, D, 0, H, wbeta, L.expert_zones, 0, L.dx3, wc(L.dw3), L.dw3, S)
+            grouped("gemm_nt_dw", 0, 1, B.AMD_GROUPED_RAGGED_K, D, R, H, wbeta, L.expert_zones, 0, L.dx1, wc(L.dw1), L.dw1, S)
+            grouped("gemm_nt_dw", 0, 1, B.AMD_GROUPED_RAGGED_K, D, R, H, wbeta, L.expert_zones, 0, L.dx3, wc(L.dw3), L.dw3, S)
         timed("router_gemm", lib.dataflow_submit_matmul, hp, CS, BF, BF, wdt, BF, F32, 0, 1, D, T, E, 1.0, wbeta, d_X.ptr, L.d_routed, wc(L.dw_router), L.dw_router,
               L.kernel_workspace_bytes, ws)
     be.sync(CS)
@@ -218,6 +218,7 @@ MEASURED_TRAFFIC_BYTES = {
 _STREAM = "gemm_bf16_stream_kernel<256, %d, 4, 2, %s>"
 _W4 = "gemm_bf16_w4_kernel<%s>"
 _W4D = "gemm_bf16_w4d_kernel<%s>"
+_W4K = "gemm_bf16_w4k_kernel<%s>"
 FUSED_GEMM_KERNEL_OF_CLASS = {
     "gemm_up13": _STREAM % (288, "false, false, 1, 1"), "gemm_tn": _STREAM % (288, "false, false, 1, 0"),
     "gemm_nn": _STREAM % (288, "true, false, 1, 0"), "gemm_dx13": _STREAM % (288, "true, false, 1, 0"),
@@ -812,6 +813,8 @@ def main():
                 tile_rows = ragged_n_tile_rows(rows_m[cls], k_of[cls], counts)
                 if tile_rows != 384:
                     four[cls] = kernel_of_class[cls].replace("288", str(tile_rows))
+        if args.gemm_kernel == 384 or (args.gemm_kernel == 0 and T * K >= 320 * E):      # the library's rule for the weight gradients
+            four.update(dict.fromkeys(("gemm_nt_dw", "gemm_dw13"), _W4K % "true, 2"))
         kernel_of_class.update(four)
     by_kernel = {}
     for k, v in gemms.items():

@@ -51,13 +51,15 @@ int amd_matmul_no_alloc(Dataflow_Handle * dataflow_handle, int stream_id, int to
  *     (256 x 288 over the token rows of a ragged-N launch).
  *   FOUR_WAVES_384: one wave per SIMD with the accumulators in the accumulation registers, 256 x 384 tiles (12 % fewer
  *     operand bytes per flop), every wave loading straight into the LDS and multiplying, its own token rows reloaded
- *     without the barrier.
+ *     without the barrier.  Where both operands are k-major (ragged K, the weight gradients): 256 x 256 tiles, with C.
  *   FOUR_WAVES: one loading wave (operands through its registers) and three multiplying waves, 256 x 288 tiles.
  *   AUTO (the default): a ragged-N launch runs on the cheapest of the tilings of both (tiles of 384, 288, 224 or 192 token
  *     rows) for the group sizes that an even router gives: the number of tiles, in rounds over the compute units.
- *     For a single problem, whose tiles are known, tiles of 384 against those of 256.  Everything else runs EIGHT_WAVES.
+ *     For a single problem, whose tiles are known, tiles of 384 against those of 256.  Two k-major operands: four waves from K = 256 on,
+ *     ragged K from 320 rows a group on where the caller gave the rows of all groups as K.  Everything else runs EIGHT_WAVES.
  * The four-wave kernels are taken only where their limits hold (no C operand, N-side operand k-contiguous, K a multiple
- * of 128 and at most 2^21, M a multiple of 8, 16-byte aligned D), the eight-wave kernel elsewhere.  Results are
+ * of 128 and at most 2^21, M a multiple of 8, 16-byte aligned D; for two k-major operands M and N multiples of 8, C and D 16-byte
+ * aligned), the eight-wave kernel elsewhere.  Results are
  * bit-identical whichever kernel runs.  The choice is process-wide; the environment variable AMD_MATMUL_KERNEL ("auto",
  * "8", "384" or "4") sets it when the matmul op is registered. */
 #define AMD_MATMUL_KERNEL_AUTO 0

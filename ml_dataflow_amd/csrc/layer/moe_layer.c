@@ -439,7 +439,7 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 														  L->chosen_experts, L->token_expert_weights, x13, (uint8_t *) x13 + (uint64_t) H * el, dh,
 														  L->d_routed, dx13, (uint8_t *) dx13 + (uint64_t) H * el, temp),
 				  "failed to submit routed swiglu bwd x");
-			CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, H, 0, D, E, cum,
+			CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, H, T * K, D, E, cum,
 													 1.0f, wbeta, temp, 0, L->expert_zones, WGRAD_C(L->dw2), L->dw2, S), "failed to submit grouped dW2 matmul");
 			CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, DATAFLOW_NONE, dt, cdt, 0, 0, AMD_GROUPED_RAGGED_N, D, 2 * H, T * K, E, cum,
 													 1.0f, 0.0f, L->w1, S, dx13, NULL, L->expert_zones, 0), "failed to submit grouped dX matmul");
@@ -449,7 +449,7 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 			CHECK(dataflow_submit_amd_swiglu_bwd_x_routed(h, cs, dt, dt, T * K, H, E, K, H, H, L->expert_mapping, L->token_mapping, L->chosen_experts,
 														  L->token_expert_weights, L->x1, L->x3, L->dx1, L->d_routed, L->dx1, L->dx3, temp),
 				  "failed to submit routed swiglu bwd x");
-			CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, H, 0, D, E, cum,
+			CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, H, T * K, D, E, cum,
 													 1.0f, wbeta, temp, 0, L->expert_zones, WGRAD_C(L->dw2), L->dw2, S), "failed to submit grouped dW2 matmul");
 			CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, DATAFLOW_NONE, dt, cdt, 0, 0, AMD_GROUPED_RAGGED_N, D, H, T * K, E, cum,
 													 1.0f, 0.0f, L->w1, S, L->dx1, NULL, L->expert_zones, 0), "failed to submit grouped dX(w1) matmul");
@@ -471,7 +471,7 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 		 * that element of dx1), so the two GEMMs are independent and the second runs on the secondary stream, filling
 		 * the compute units that the first one's last round of tiles leaves idle. */
 		CHECK(stream_wait(h, ss, cs), "secondary stream could not wait for the compute stream");
-		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, H, 0, D, E, cum,
+		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, H, T * K, D, E, cum,
 												 1.0f, wbeta, temp, 0, L->expert_zones, WGRAD_C(L->dw2), L->dw2, S), "failed to submit grouped dW2 matmul");
 		CHECK(dataflow_submit_amd_grouped_matmul(h, ss, dt, dt, DATAFLOW_NONE, dt, cdt, 0, 0, AMD_GROUPED_RAGGED_N, H, D, T * K, E, cum,
 												 1.0f, 0.0f, L->w2, S, L->expert_zones, NULL, L->dx1, 0), "failed to submit grouped dh matmul");
@@ -567,18 +567,18 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 	}
 	if (gathered) {
 		/* no re-dispatch: the GEMM takes the rows of X through expert_mapping (same values, same result) */
-		CHECK(dataflow_submit_amd_grouped_matmul_gathered(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, 0, 2 * H, E, L->expert_counts_cumsum,
+		CHECK(dataflow_submit_amd_grouped_matmul_gathered(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, T * K, 2 * H, E, L->expert_counts_cumsum,
 														  1.0f, wbeta, X, 0, L->dx1, WGRAD_C(L->dw1), L->dw1, S, L->expert_mapping, T),
 			  "failed to submit gathered grouped dW1|dW3 matmul");
 	} else if (side_by_side) {
-		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, 0, 2 * H, E, L->expert_counts_cumsum,
+		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, T * K, 2 * H, E, L->expert_counts_cumsum,
 												 1.0f, wbeta, L->expert_zones, 0, L->dx1, WGRAD_C(L->dw1), L->dw1, S), "failed to submit grouped dW1|dW3 matmul");
 	} else if (schedule != AMD_MOE_PER_EXPERT) {
 		/* independent of each other: the second on the secondary stream, as for the up-projections */
 		CHECK(stream_wait(h, ss, cs), "secondary stream could not wait for the compute stream");
-		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, 0, H, E, L->expert_counts_cumsum,
+		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, T * K, H, E, L->expert_counts_cumsum,
 												 1.0f, wbeta, L->expert_zones, 0, L->dx1, WGRAD_C(L->dw1), L->dw1, S), "failed to submit grouped dW1 matmul");
-		CHECK(dataflow_submit_amd_grouped_matmul(h, ss, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, 0, H, E, L->expert_counts_cumsum,
+		CHECK(dataflow_submit_amd_grouped_matmul(h, ss, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, T * K, H, E, L->expert_counts_cumsum,
 												 1.0f, wbeta, L->expert_zones, 0, L->dx3, WGRAD_C(L->dw3), L->dw3, S), "failed to submit grouped dW3 matmul");
 		CHECK(stream_wait(h, cs, ss), "compute stream could not wait for the secondary stream");
 	} else {

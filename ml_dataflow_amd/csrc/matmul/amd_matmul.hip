@@ -258,6 +258,25 @@ static int launch_w4d(const GemmParams & p, long tiles_upper_bound, long cu_coun
 	return check_launch();
 }
 
+/* the four waves with k-major operands in slices (gemm_w4_kernel.h): same grid rule */
+template <int MODE>
+static int launch_w4k(const GemmParams & p, long tiles, long cu_count, hipStream_t stream) {
+	long grid = cu_count & ~7L;
+	if (grid < 8) {
+		grid = 8;
+	}
+	const long need = (tiles + 7) & ~7L;
+	if (need < grid) {
+		grid = need;
+	}
+	if (p.C && p.beta != 0.0f) {
+		hipLaunchKernelGGL((gemm_bf16_w4k_kernel<true, MODE>), dim3((unsigned int) grid), dim3(256), 0, stream, p);
+	} else {
+		hipLaunchKernelGGL((gemm_bf16_w4k_kernel<false, MODE>), dim3((unsigned int) grid), dim3(256), 0, stream, p);
+	}
+	return check_launch();
+}
+
 /* Which persistent kernel large problems without a C operand run: AMD_MATMUL_KERNEL_EIGHT_WAVES or
  * AMD_MATMUL_KERNEL_FOUR_WAVES (amd_matmul.h).  Process-wide; amd_matmul_select_kernel changes it, the environment
  * variable AMD_MATMUL_KERNEL ("8" or "4") sets the initial value when the op is registered. */
@@ -278,6 +297,22 @@ extern "C" int amd_matmul_select_kernel(int which) {
 static bool w4_ok(const GemmParams & p) {
 	return !(p.C && p.beta != 0.0f) && (p.K % 128 == 0) && p.K <= (1 << 21) &&
 		   (p.M % 8 == 0) && p.M <= (1 << 22) && ((((uintptr_t) p.D) & 15) == 0);
+}
+
+/* the sliced kernel takes and leaves 16-byte pieces of rows of C and D; a wave's 128 rows of D stay below 2 GiB (W4_NO_COLUMN), a
+ * slice of either operand below 4 GiB */
+static bool w4k_ok(const GemmParams & p) {
+	return p.M % 8 == 0 && p.N % 8 == 0 && p.M <= (1 << 22) && p.N <= (1 << 24) && p.strideD % 8 == 0 && ((((uintptr_t) p.D) & 15) == 0) &&
+		   (!(p.C && p.beta != 0.0f) || (((uintptr_t) p.C) & 15) == 0);
+}
+
+/* Where the sliced kernel is the faster one.  Ragged K: from 320 rows a group on, where the caller said how many there are.  Its tiles have
+ * at least 8 slices of 32 k-rows (5 without C), and a fixed part that two waves on a SIMD hide better: us, eight waves and sliced, 32
+ * groups, 2048 x 1408 with C, of 64 rows 77 and 89, of 256 96 and 100, of 320 106 and 106, of 375 114 and 110, of 640 152 and 144; 1024 x
+ * 4096 without C, of 64 65 and 67, of 320 107 and 104, of 640 169 and 163.  One problem: from K = 256 on (4096 x 4096 with C, K 128: 17 and
+ * 17, 512: 29 and 24, 8192: 207 and 196). */
+static bool w4k_pays(int mode, const GemmParams & p) {
+	return mode == MODE_RAGGED_K ? (long) p.K >= 320L * p.num_groups : p.K >= 256;
 }
 
 /* a ragged-N launch without C on one of its tilings; grid: an upper bound on the tiles */
@@ -512,6 +547,11 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 					   : launch_direct<true, true, MODE_RAGGED_K, GATHER_P_KROWS>(p, tile, stream);
 		}
 		return launch_staged<SMALL_TILE, true, true, MODE_RAGGED_K>(p, round_up8(grid_small), stream);
+	}
+	if constexpr (MODE != MODE_RAGGED_N) {
+		if (pk && qk && direct && big && !p.gather && (wide_only || (either && w4k_pays(MODE, p))) && w4k_ok(p)) {
+			return launch_w4k<MODE>(p, grid_big, cu_count, stream);
+		}
 	}
 	if (!pk && !qk) { PICK(false, false); }
 	if (pk && !qk) { PICK(true, false); }

@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """Writes gemm_w4_loop.inc: the k-loops of the four-wave GEMM kernels of gemm_w4_kernel.h as inline-assembly text
-(gemm_bf16_w4_kernel: classes Mult and Loader, described here; gemm_bf16_w4d_kernel: class Wide, described there).  Run
+(gemm_bf16_w4_kernel: classes Mult and Loader, described here; gemm_bf16_w4d_kernel: class Wide, gemm_bf16_w4k_kernel: class Ring, described there).  Run
 by the Makefile; the output is a build product.
 
 The kernel: 256 threads, one wave per SIMD, work-group tile 256 (m) x 288 (n) x 64 (k).  The waves have two roles.
@@ -626,11 +626,263 @@ class Wide(Mult, Tail):
                ["s%d" % i for i in range(92, 96)] + ["m0", "scc", "memory"]
 
 
+# ================================================================================================ four waves, ragged reduction
+R_SLICE, R_SLOTS = 32768, 5                                   # bytes of a slice of both operands (2 x 32 k x 256 rows), slices in the LDS
+R_C, R_PRD, R_QRD, R_VP, R_VQ, R_AT, R_CAT = 64, 192, 200, 208, 212, 216, 220
+
+
+class Ring(Tail):
+    """gemm_bf16_w4k_kernel: tile 256 (m) x 256 (n), both operands k-major, four waves as 2 x 2, each 128 x 128 (8 x 8 blocks, all 256
+    accumulators in a[0:255]).  The stream is one of slices of 32 k, 16 KiB of P behind 16 KiB of Q, in a ring of five slots that runs on
+    across tiles; every wave loads a quarter of each slice (eight chunks of 1 KiB, two k-rows each) straight into the LDS.
+
+    Slice s, two halves of 32 MFMAs, row block by row block: columns 0-3, then 4-7.  All operands of a slice are in registers once, and
+    each is read again right behind its last MFMA: those of columns 4-7 (of this slice) in the first half, between the halves the one
+    barrier, then those of columns 0-3 and row by row those of P (of the next slice), 28 MFMAs in front of their use.  In front of the
+    barrier the wave waits for its loads of slice s + 1, and for its reads of slice s, whose slot takes the loads of slice s + 5: three to
+    four slices, 96 to 128 KiB, are in flight at any time.
+
+    C has 128 registers: its tile is read in the first eight slices, four lines of 16 rows each, and has the rest of the tile's multiplies
+    to arrive; the stores of D go out behind the last multiply and drain under the next tile's.
+
+    s[40:47] the cursor (as for the loader above) of this tile, at slice 0 for the work-group's first tile and at slice 5 for any other,
+    s[48:55] the next tile's at slice 0, s56 slices (at least `least`), s57 bit 0: first tile, bit 2: alpha is not 1, s58 / s59 bytes per
+    slice of P / Q, s60 byte offset of slice 0's slot, s61 / s62 LDS address of the wave's rows of P / Q in slot 0, s63 of its first chunk.
+    s[32:39] as w4_output gives them (D, bytes, bytes of 16 rows, C, alpha, beta).  Working registers: s[64:75] as in the loader above,
+    s76 the slot, s77 scratch, s78 where the loads go, s79 the slice, s[84:87] C's descriptor, s[92:95] D's.
+
+    State from statement to statement: slices 0-4 of the tile are on their way or there, slice 0 visible to all waves; behind them the 32
+    stores of the tile before."""
+
+    LOADS, STORES = 8, 32
+
+    def __init__(self, HAS_C):
+        Asm.__init__(self)
+        self.C = HAS_C
+        self.least = 8 if HAS_C else 5           # slices a tile has at least
+        self.head = 8 if HAS_C else 4            # slices in front of the loop
+        self.name = "W4K_%s" % ("C" if HAS_C else "NOC")
+
+    set_cursor, advance = Wide.set_cursor, Wide.advance
+
+    def need(self, *keys):
+        n = max(self.prod.get(k, -1) for k in keys)
+        if n > self.known_done:
+            after = min(self.issued - 1 - n, 15)
+            self.e("s_waitcnt lgkmcnt(%d)" % after)
+            self.known_done = self.issued - 1 - after
+
+    def read(self, which, n):
+        """operand n (16 rows) of P or Q, both halves of its 32 k"""
+        dst = 4 * n + (0 if which == "P" else 32)
+        addr = (R_PRD if which == "P" else R_QRD) + n
+        self.lds("ds_read_b64_tr_b16 %s, v%d" % (vr(dst, 2), addr))
+        self.lds("ds_read_b64_tr_b16 %s, v%d offset:%d" % (vr(dst + 2, 2), addr, 4 * 512), (which, n))
+
+    def dma(self, u):
+        self.e("s_add_u32 m0, s78, %d" % ((u % 4) * 1024 + (16384 if u >= 4 else 0)))
+        self.e("s_nop 0")
+        self.e("buffer_load_dwordx4 v%d, s[%s], 0 offen lds" % (R_VP + u, "64:67" if u < 4 else "68:71"))
+
+    def load_c(self, j, k):
+        self.e("buffer_load_dwordx4 %s, v%d, s[84:87], 0 offen nt" % (vr(R_C + 16 * j + 4 * k, 4), R_CAT + k))
+        self.e("v_add_u32 v%d, s35, v%d" % (R_CAT + k, R_CAT + k))
+
+    def move_on(self):
+        """the cursor, which stands at slice s79 + 5 of this tile, to the next tile's first one if there is none"""
+        self.e("s_add_u32 s77, s79, %d" % R_SLOTS)
+        self.e("s_cmp_eq_u32 s77, s56")
+        self.e("s_cbranch_scc0 6f")
+        self.set_cursor(48, 0)
+        self.set_cursor(48, 1)
+        self.e("6:")
+
+    def vm_count(self, s):
+        """of the operations behind the loads of slice s + 1, how many may be in flight at the barrier of slice s < head"""
+        ops = []
+        for t in range(1, R_SLOTS):
+            ops += ["L%d" % t] * self.LOADS
+        ops += ["S"] * self.STORES
+        for t in range(s + 1):
+            ops += ["C"] * (4 if self.C else 0)
+            if t < s:
+                ops += ["L%d" % (t + R_SLOTS)] * self.LOADS
+        last = max(n for n, o in enumerate(ops) if o == "L%d" % (s + 1))
+        return min(63, len(ops) - 1 - last)
+
+    def slice(self, s):
+        """s: the slice's number, or None in the loop"""
+        after = {}
+
+        def at(m, fn):
+            after.setdefault(m, []).append(fn)
+
+        e = self.e
+        for n in range(4):
+            at(2 * n, lambda n=n: self.read("Q", 4 + n))
+        # the read addresses move to the next slot (the reads of this one are out)
+        at(8, lambda: e("s_add_u32 s78, s63, s76"))
+        at(8, lambda: e("s_mov_b32 s77, s76"))
+        at(9, lambda: e("s_add_u32 s76, s76, %d" % R_SLICE))
+        at(9, lambda: e("s_cmp_eq_u32 s76, %d" % (R_SLOTS * R_SLICE)))
+        at(9, lambda: e("s_cselect_b32 s76, 0, s76"))
+        at(9, lambda: e("s_sub_u32 s77, s76, s77"))
+        for n in range(16):
+            at(10 + n, lambda n=n: e("v_add_u32 v%d, s77, v%d" % (R_PRD + n, R_PRD + n)))
+        if self.C and s is not None and s < 8:
+            for k in range(4):
+                at(11 + 4 * k, lambda k=k: self.load_c(s, k))
+
+        def barrier():
+            e("s_waitcnt vmcnt(%d)" % (self.LOADS * 3 if s is None else self.vm_count(s)))
+            self.lds_drain()
+            self.barrier()
+        at(31, barrier)
+        for n in range(4):
+            at(32 + n, lambda n=n: self.read("Q", n))
+        for i in range(8):
+            at(35 + 4 * i, lambda i=i: self.read("P", i))
+        at(34, self.move_on)
+        for u in range(self.LOADS):
+            at(36 + 3 * u, lambda u=u: self.dma(u))
+        at(58, lambda: self.advance(0))
+        at(59, lambda: self.advance(1))
+        at(60, lambda: e("s_add_u32 s79, s79, 1"))
+        for m in range(64):
+            half, rem = divmod(m, 32)
+            i, j = divmod(rem, 4)
+            if i & 1:
+                j = 3 - j                        # one operand stays from each MFMA to the next
+            j += 4 * half
+            acc = "a[%d:%d]" % (16 * (8 * (i // 4) + j) + 4 * (i % 4), 16 * (8 * (i // 4) + j) + 4 * (i % 4) + 3)
+            self.need(("P", i), ("Q", j))
+            self.e("v_mfma_f32_16x16x32_bf16 %s, %s, %s, %s" % (acc, vr(4 * i, 4), vr(32 + 4 * j, 4), "0" if s == 0 else acc))
+            for fn in after.get(m, []):
+                fn()
+
+    def entry_state(self):
+        """the reads in flight at the start of a slice, as the second half of the one before leaves them"""
+        self.issued, self.known_done, self.prod = 0, -1, {}
+        keep, self.L = self.L, []
+        for n in range(4):
+            self.read("Q", n)
+        for i in range(8):
+            self.read("P", i)
+        self.L = keep
+
+    def addresses(self):
+        """fragment read addresses of this lane in the slot s60: k-row 8 g4 + l15 / 4, rows 16 i + 4 (l15 % 4), swizzled as
+        kmajor_swizzle does"""
+        e = self.e
+        l15, g4, sw, t, row = 0, 1, 2, 3, 4
+        e("v_mbcnt_lo_u32_b32 v%d, -1, 0" % t)
+        e("v_mbcnt_hi_u32_b32 v%d, -1, v%d" % (t, t))
+        e("v_and_b32 v%d, 15, v%d" % (l15, t))
+        e("v_lshrrev_b32 v%d, 4, v%d" % (g4, t))
+        e("v_lshrrev_b32 v%d, 2, v%d" % (sw, l15))
+        e("v_lshl_add_u32 v%d, v%d, 3, v%d" % (t, g4, sw))
+        e("v_lshlrev_b32 v%d, 5, v%d" % (sw, sw))
+        e("v_and_b32 v%d, 1, v%d" % (row, g4))
+        e("v_lshlrev_b32 v%d, 4, v%d" % (row, row))
+        e("v_xor_b32 v%d, v%d, v%d" % (sw, sw, row))
+        e("v_lshlrev_b32 v%d, 9, v%d" % (t, t))
+        e("v_add_u32 v%d, s60, v%d" % (t, t))
+        e("v_and_b32 v%d, 3, v%d" % (row, l15))
+        e("v_lshlrev_b32 v%d, 2, v%d" % (row, row))
+        for n in range(8):
+            e("v_add_u32 v%d, %d, v%d" % (R_PRD + n, 16 * n, row))
+            e("v_xor_b32 v%d, v%d, v%d" % (R_PRD + n, R_PRD + n, sw))
+            e("v_lshl_add_u32 v%d, v%d, 1, v%d" % (R_PRD + n, R_PRD + n, t))
+            e("v_add_u32 v%d, s62, v%d" % (R_QRD + n, R_PRD + n))
+            e("v_add_u32 v%d, s61, v%d" % (R_PRD + n, R_PRD + n))
+
+    def generate(self):
+        e = self.e
+        self.addresses()
+        self.set_cursor(40, 0)
+        self.set_cursor(40, 1)
+        if self.C:
+            for n, ins in enumerate(("s36", "s37", "s34", "0x00020000")):
+                e("s_mov_b32 s%d, %s" % (84 + n, ins))
+        e("s_mov_b32 s76, s60")
+        e("s_mov_b32 s79, 0")
+        e("s_bitcmp1_b32 s57, 0")
+        e("s_cbranch_scc0 2f")
+        for t in range(R_SLOTS):                 # first tile (its first slot is slot 0)
+            e("s_add_u32 s78, s63, %d" % (t * R_SLICE))
+            for u in range(self.LOADS):
+                self.dma(u)
+            self.advance(0)
+            self.advance(1)
+        e("s_waitcnt vmcnt(0)")
+        e("s_barrier")
+        e("2:")
+        for n in range(4):
+            self.read("Q", n)
+        for i in range(8):
+            self.read("P", i)
+        for s in range(self.head):
+            self.entry_state()
+            self.slice(s)
+        e("s_cmp_lt_u32 s79, s56")
+        e("s_cbranch_scc0 4f")
+        e("3:")
+        self.entry_state()
+        self.slice(None)
+        e("s_cmp_lt_u32 s79, s56")
+        e("s_cbranch_scc1 3b")
+        e("4:")
+        e("s_waitcnt lgkmcnt(0)")
+        self.descriptor(92, 32)
+        if self.C:                               # C is here: 8 loads went out behind it for each slice from the eighth on
+            e("s_cmp_ge_u32 s56, 11")
+            e("s_cbranch_scc1 5f")
+            e("s_waitcnt vmcnt(%d)" % self.LOADS)
+            e("5:")
+            e("s_waitcnt vmcnt(%d)" % (4 * self.LOADS))
+        for _ in range(3):
+            e("s_nop 7")
+        e("s_bitcmp1_b32 s57, 2")
+        e("s_cbranch_scc1 10f")
+        self.epilogue(False)
+        e("s_branch 11f")
+        e("10:")
+        self.epilogue(True)
+        e("11:")
+        return self.L
+
+    def add_c(self, src, c):
+        """beta C on the 16 results from src on; c .. c + 3 and c + 4 .. c + 7: the lines' halves as they were loaded, 16 bytes of each
+        row in a lane.  The swap undoes what the one in front of a store does"""
+        for a in (c, c + 1, c + 4, c + 5):
+            self.swap(a, a + 2)
+        for k in range(8):
+            for half in range(2):
+                self.valu(("v_and_b32 v60, 0xffff0000, v%d" if half else "v_lshlrev_b32 v60, 16, v%d") % (c + k), (60,))
+                self.valu("v_fmac_f32 v%d, s39, v60" % (src + 2 * k + half), (src + 2 * k + half,))
+
+    def epilogue(self, scale):
+        self.count, self.written = 0, {}
+        for n in range(16):
+            j, h = divmod(n, 2)
+            if h == 0 and j:
+                self.next_rows(R_AT, 4)
+            t = 24 * (n & 1)
+            src = self.accumulators(8 * h + j, t, scale)
+            if self.C:
+                self.add_c(src, R_C + 16 * j + 8 * h)
+            self.store_group(src, t, R_AT + 2 * h)
+
+    def clobbers(self):
+        return ["v%d" % i for i in range(R_VP)] + ["a%d" % i for i in range(256)] + ["s%d" % i for i in range(64, 80)] + \
+               ["s%d" % i for i in list(range(84, 88)) + list(range(92, 96))] + ["m0", "scc", "memory"]
+
+
 def main():
     out = sys.argv[1] if len(sys.argv) > 1 else os.path.join(os.path.dirname(os.path.abspath(__file__)), "gemm_w4_loop.inc")
     with open(out, "w") as f:
         f.write("/* generated by gen_w4_loop.py -- do not edit */\n")
-        for v in (Mult(False), Mult(True), Loader(False), Loader(True), Wide(False, False), Wide(False, True), Wide(True, False), Wide(True, True)):
+        for v in (Mult(False), Mult(True), Loader(False), Loader(True), Wide(False, False), Wide(False, True), Wide(True, False), Wide(True, True), Ring(False), Ring(True)):
             parts = v.generate()
             if not isinstance(v, Wide):
                 parts = [(v.name + "_ASM", parts)]
@@ -658,6 +910,11 @@ def main():
         f.write('#define W4D_INPUTS(sd, sa, sb, sc) "{s[32:39]}"(sd), "{s[40:47]}"(sa), "{s[48:55]}"(sb), "{s[56:63]}"(sc)\n')
         f.write("#define W4D_PRE %d\n" % OPTS["pre"])
         f.write("#define W4D_VP 0\n#define W4D_VQ %d\n#define W4D_VQ_NEXT %d\n" % (D_VQ - D_VP, D_VQ_NEXT - D_VP))
+
+        # sliced kernel: the lane's load offsets vo (4 of P, 4 of Q) and its four of D and four of C, the blocks of scalars sd, sa, sb, sc
+        f.write('#define W4K_OUTPUTS(vo, at) "+{v[%d:%d]}"(vo), "+{v[%d:%d]}"(at)\n' % (R_VP, R_VP + 7, R_AT, R_AT + 7))
+        for v in (Ring(False), Ring(True)):
+            f.write("#define %s_LEAST %d\n" % (v.name, v.least))
 
 if __name__ == "__main__":
     main()

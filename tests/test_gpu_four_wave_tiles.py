@@ -60,3 +60,38 @@ def test_ragged_n_many_groups(backend, select_kernel, transa, alpha, M, K, group
         d_W.ptr, M * K * 2, d_X.ptr, None, d_D.ptr, 0))
     for d in (d_W, d_X, d_cum):
         d.free()
+
+
+@pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (1.0, 1.0), (-0.75, 0.0), (1.5, -0.5)])
+@pytest.mark.parametrize("M,N,groups", [(264, 520, 64), (1304, 264, 70), (256, 256, 300)])
+def test_ragged_k_tiles_and_slices(backend, select_kernel, alpha, beta, M, N, groups):
+    """reductions of no slice to more than the ring holds, last slices of 1 to 32 k-rows; tiles partial in both directions"""
+    be = backend
+    rng = np.random.default_rng(M + N + groups)
+    counts = rng.choice([0, 1, 31, 32, 33, 128, 159, 160, 161, 255, 256, 257, 352, 353, 500], size=groups).astype(np.int32)
+    counts[0], counts[-1] = 353, 1
+    total = int(counts.sum())
+    print("case four waves, K: alpha=%g beta=%g M=%d N=%d G=%d rows=%d" % (alpha, beta, M, N, groups, total), flush=True)
+    d_A, d_B = be.upload(normal_bf16(rng, (total, M), 0.05)), be.upload(normal_bf16(rng, (total, N)))
+    d_cum = be.upload(np.cumsum(counts).astype(np.int32))
+    start = normal_bf16(rng, (groups, N, M))
+    both(be, select_kernel, FOUR_384, groups * N * M, start, lambda d_D: be.lib.dataflow_submit_amd_grouped_matmul(
+        be.hp, CS, BF, BF, BF if beta else B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 0, 1, B.AMD_GROUPED_RAGGED_K, M, 0, N, groups, d_cum.ptr, alpha, beta,
+        d_A.ptr, 0, d_B.ptr, d_D.ptr if beta else None, d_D.ptr, N * M * 2))
+    for d in (d_A, d_B, d_cum):
+        d.free()
+
+
+@pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (1.0, 1.0), (0.5, -2.0)])
+@pytest.mark.parametrize("M,N,K", [(4104, 4008, 161), (2816, 4096, 1000), (4096, 4096, 256)])
+def test_k_major_operands_of_one_problem(backend, select_kernel, alpha, beta, M, N, K):
+    """one or two tiles a work-group, partial ones in both directions, a last slice of one k-row, of eight, and a whole one"""
+    be = backend
+    rng = np.random.default_rng(M + N + K)
+    print("case four waves, k-major: alpha=%g beta=%g M=%d N=%d K=%d" % (alpha, beta, M, N, K), flush=True)
+    d_A, d_B, d_ws = be.upload(normal_bf16(rng, (K, M), 0.05)), be.upload(normal_bf16(rng, (K, N))), be.upload(np.zeros(1 << 20, np.uint8))
+    both(be, select_kernel, FOUR_384, N * M, normal_bf16(rng, (N, M)), lambda d_D: be.lib.dataflow_submit_matmul(
+        be.hp, CS, BF, BF, BF if beta else B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 0, 1, M, K, N, alpha, beta,
+        d_A.ptr, d_B.ptr, d_D.ptr if beta else None, d_D.ptr, 1 << 20, d_ws.ptr))
+    for d in (d_A, d_B, d_ws):
+        d.free()
