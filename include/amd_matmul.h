@@ -56,7 +56,7 @@ int amd_matmul_no_alloc(Dataflow_Handle * dataflow_handle, int stream_id, int to
  *   AUTO (the default): a ragged-N launch runs on the cheapest of the tilings of both (tiles of 384, 288, 224 or 192 token
  *     rows) for the group sizes that an even router gives: the number of tiles, in rounds over the compute units.
  *     For a single problem, whose tiles are known, tiles of 384 against those of 256.  Two k-major operands: four waves from K = 256 on,
- *     ragged K from 320 rows a group on where the caller gave the rows of all groups as K.  Everything else runs EIGHT_WAVES.
+ *     ragged K from 320 rows a group on with C, 512 without, where the caller gave the rows of all groups as K.  Everything else runs EIGHT_WAVES.
  * The four-wave kernels are taken only where their limits hold (no C operand, N-side operand k-contiguous, K a multiple
  * of 128 and at most 2^21, M a multiple of 8, 16-byte aligned D; for two k-major operands M and N multiples of 8, C and D 16-byte
  * aligned), the eight-wave kernel elsewhere.  Results are

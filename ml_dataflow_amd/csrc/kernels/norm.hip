@@ -14,6 +14,9 @@
  *
  * All kernels are bandwidth-bound: one 256-thread work-group per row, 16 bytes per lane per access, the row kept
  * in registers between the reduction and the second use (rows up to 8192 elements; longer rows are read twice).
+ * us, forward, bwd_x with X_out and bwd_w of 8192 x 4096 in turn, 604 MB: 113.3 -> 104.7 (5.8 TB/s): dX loaded with x and g instead of
+ * behind the sum 109.6, bwd_x's results stored past the caches 106.8, bwd_w's loads in front of the sums of four rows 104.7.  bwd_x from
+ * the last row to the first, for what the memory-side cache holds of x, was no faster (114.3).
  */
 
 #define NORM_MAX_VEC 4
@@ -112,7 +115,7 @@ default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 	u32x4 * d = (u32x4 *) (dX + (size_t) row * n_cols);
 	u32x4 * xo = X_out ? (u32x4 *) (X_out + (size_t) row * n_cols) : nullptr;
 
-	u32x4 keep_x[NORM_MAX_VEC], keep_g[NORM_MAX_VEC];
+	u32x4 keep_x[NORM_MAX_VEC], keep_g[NORM_MAX_VEC], keep_d[NORM_MAX_VEC];
 	float part[1] = {0.0f};
 	int j = 0;
 	for (int v = threadIdx.x; v < nvec; v += ROW_THREADS, j++) {
@@ -121,6 +124,7 @@ default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 		if (j < NORM_MAX_VEC) {
 			keep_x[j] = qx;
 			keep_g[j] = qg;
+			keep_d[j] = d[v];
 		}
 		float fx[8], fg[8], fw[8], y[8];
 		unpack8(qx, fx);
@@ -132,7 +136,7 @@ default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 			part[0] = __builtin_fmaf(y[i], fg[i], part[0]);
 		}
 		if (xo) {
-			xo[v] = pack8(y);
+			__builtin_nontemporal_store(pack8(y), xo + v);
 		}
 	}
 	block_sum<1>(part, scratch);
@@ -143,20 +147,22 @@ default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 		unpack8(j < NORM_MAX_VEC ? keep_x[j] : x[v], fx);
 		unpack8(j < NORM_MAX_VEC ? keep_g[j] : g[v], fg);
 		unpack8(w[v], fw);
-		unpack8(d[v], fd);
+		unpack8(j < NORM_MAX_VEC ? keep_d[j] : d[v], fd);
 		#pragma unroll
 		for (int i = 0; i < 8; i++) {
 			fd[i] += r * (fg[i] * fw[i] - c_div_n * (fx[i] * r));
 		}
-		d[v] = pack8(fd);
+		__builtin_nontemporal_store(pack8(fd), d + v);
 	}
 }
 
 /* Backward w.r.t. the scale, first half: work-group b sums g * x * r over its share of the rows (a contiguous
  * range, as in the reference) into dW_workspace[b][n_cols] (fp32) and records the number of work-groups.
  * Launch: grid x <= n_rows (chosen so that the workspace holds grid.x * n_cols floats), grid y = column slabs of
- * 2048, block = 256: every thread owns 8 columns and walks down its work-group's rows with 16 loads in flight.
+ * 2048, block = 256: every thread owns 8 columns and walks down its work-group's rows, four at a time: left to itself the compiler keeps
+ * two or three loads in flight (30 registers) and not eight.  Eight rows at a time take the same 104.7 us in the sequence above.
  * Algorithmic HBM bytes: 4*n_rows*n_cols read, 4*grid*n_cols written. */
+#define BWD_W_ROWS 4
 extern "C" __global__ void __launch_bounds__(ROW_THREADS)
 default_rms_norm_bwd_w_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const float * __restrict__ fwd_rms_vals,
 										const bf16_t * __restrict__ X_inp, const bf16_t * __restrict__ upstream_dX,
@@ -182,13 +188,35 @@ default_rms_norm_bwd_w_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 		return;
 	}
 	float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-	#pragma unroll 8
-	for (int i = 0; i < rows; i++) {
-		const size_t off = (size_t) (first + i) * n_cols;
+	const u32x4 * x = (const u32x4 *) (X_inp + (size_t) first * n_cols) + v;
+	const u32x4 * g = (const u32x4 *) (upstream_dX + (size_t) first * n_cols) + v;
+	int i = 0;
+	for (; i + BWD_W_ROWS <= rows; i += BWD_W_ROWS) {
+		u32x4 qx[BWD_W_ROWS], qg[BWD_W_ROWS];
+		float r[BWD_W_ROWS];
+		#pragma unroll
+		for (int k = 0; k < BWD_W_ROWS; k++) {
+			qx[k] = __builtin_nontemporal_load(x + (size_t) (i + k) * nvec);
+			qg[k] = __builtin_nontemporal_load(g + (size_t) (i + k) * nvec);
+			r[k] = fwd_rms_vals[first + i + k];
+		}
+		__builtin_amdgcn_sched_barrier(0);              /* the loads stay in front of the sums */
+		#pragma unroll
+		for (int k = 0; k < BWD_W_ROWS; k++) {
+			float fx[8], fg[8];
+			unpack8(qx[k], fx);
+			unpack8(qg[k], fg);
+			#pragma unroll
+			for (int e = 0; e < 8; e++) {
+				acc[e] += (fg[e] * fx[e]) * r[k];
+			}
+		}
+	}
+	for (; i < rows; i++) {
 		const float r = fwd_rms_vals[first + i];
 		float fx[8], fg[8];
-		unpack8(__builtin_nontemporal_load(((const u32x4 *) (X_inp + off)) + v), fx);
-		unpack8(__builtin_nontemporal_load(((const u32x4 *) (upstream_dX + off)) + v), fg);
+		unpack8(__builtin_nontemporal_load(x + (size_t) i * nvec), fx);
+		unpack8(__builtin_nontemporal_load(g + (size_t) i * nvec), fg);
 		#pragma unroll
 		for (int e = 0; e < 8; e++) {
 			acc[e] += (fg[e] * fx[e]) * r;

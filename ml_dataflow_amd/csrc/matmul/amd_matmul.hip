@@ -306,13 +306,13 @@ static bool w4k_ok(const GemmParams & p) {
 		   (!(p.C && p.beta != 0.0f) || (((uintptr_t) p.C) & 15) == 0);
 }
 
-/* Where the sliced kernel is the faster one.  Ragged K: from 320 rows a group on, where the caller said how many there are.  Its tiles have
- * at least 8 slices of 32 k-rows (5 without C), and a fixed part that two waves on a SIMD hide better: us, eight waves and sliced, 32
- * groups, 2048 x 1408 with C, of 64 rows 77 and 89, of 256 96 and 100, of 320 106 and 106, of 375 114 and 110, of 640 152 and 144; 1024 x
- * 4096 without C, of 64 65 and 67, of 320 107 and 104, of 640 169 and 163.  One problem: from K = 256 on (4096 x 4096 with C, K 128: 17 and
- * 17, 512: 29 and 24, 8192: 207 and 196). */
+/* Where the sliced kernel is the faster one.  Ragged K, where the caller said how many rows there are: from 320 a group on with C, from
+ * 512 without.  Its tiles have at least 8 slices of 32 k-rows (5 without C), and a fixed part that two waves on a SIMD hide better: us,
+ * eight waves and sliced, 32 groups, 2048 x 1408 with C, of 64 rows 77 and 89, of 256 96 and 100, of 320 106 and 106, of 375 114 and 110,
+ * of 640 152 and 144; 1024 x 4096 without C, of 64 65 and 67, of 375 118 and 117, of 512 146 and 140, 2048 x 1408 without, of 375 85 and
+ * 89, of 640 125 and 126.  One problem: from K = 256 on (4096 x 4096 with C, K 128: 17 and 17, 512: 29 and 24, 8192: 207 and 196). */
 static bool w4k_pays(int mode, const GemmParams & p) {
-	return mode == MODE_RAGGED_K ? (long) p.K >= 320L * p.num_groups : p.K >= 256;
+	return mode == MODE_RAGGED_K ? (long) p.K >= (p.C && p.beta != 0.0f ? 320L : 512L) * p.num_groups : p.K >= 256;
 }
 
 /* a ragged-N launch without C on one of its tilings; grid: an upper bound on the tiles */
