@@ -49,7 +49,8 @@ __device__ __forceinline__ float sort_key16_value(uint32_t key) {
  * mirror pairs a lane with one from the other half, which is all a reduction needs */
 template <int CTRL>
 __device__ __forceinline__ uint32_t key_min_step(uint32_t key) {
-	const uint32_t other = (uint32_t) __builtin_amdgcn_update_dpp((int) key, (int) key, CTRL, 0xF, 0xF, false);
+	/* every lane has a partner; with the identity of min in its place the compiler folds the move into the minimum */
+	const uint32_t other = (uint32_t) __builtin_amdgcn_update_dpp(-1, (int) key, CTRL, 0xF, 0xF, false);
 	return min(key, other);
 }
 
@@ -62,7 +63,7 @@ template <int LANES>
 struct SelectSlot {
 	uint32_t key;                                          /* this lane's slot */
 	uint32_t min_key;                                      /* the smallest slot of the group: the same in every lane */
-	uint32_t max_key16;                                    /* largest value that entered */
+	uint32_t max_key16;                                    /* largest value that entered: the first expert to have it always enters */
 	int slot, K;
 	bool live;
 
@@ -73,30 +74,28 @@ struct SelectSlot {
 	}
 
 	/* experts [c0, c0 + count) in order; `row`: their sort keys, two per dword (an odd count's last partner is -inf and
-	 * never enters) */
+	 * never enters).  A step is a chain: which lane holds the smallest key, the larger of that key and the expert's, the smallest
+	 * again.  What does not depend on the step before is kept out of it: the expert's key is 0 where its logit can never enter, so
+	 * that one unsigned maximum is the rule above, and the largest value that entered is the largest there is.  16 tokens, 64 experts,
+	 * top 8 in one work-group: 8.9 -> 8.3 us; 65536 tokens, selection and mapping: 42.3 -> 39.9.  Keys read four pairs ahead: no faster. */
 	__device__ __forceinline__ void walk(const uint32_t * row, int c0, int count) {
 		for (int j = 0; j < count; j += 2) {
 			const uint32_t pair = row[j >> 1];
-			#pragma unroll
-			for (int h = 0; h < 2; h++) {
-				const uint32_t k16 = h ? (pair >> 16) : (pair & 0xFFFFu);
-				const bool enters = k16 > (min_key >> 16);      /* the same in every lane of the group */
-				max_key16 = enters ? max(max_key16, k16) : max_key16;
-				if (enters && key == min_key) {
-					key = (k16 << 16) | (0xFFFFu - (uint32_t) (c0 + j + h));
-				}
-				if (LANES > 1) {
-					uint32_t m = key_min_step<0xB1>(key);
-					if (LANES > 2) { m = key_min_step<0x4E>(m); }
-					if (LANES > 4) { m = key_min_step<0x141>(m); }
-					if (LANES > 8) { m = key_min_step<0x140>(m); }
-					if (LANES > 16) { m = min(m, (uint32_t) __shfl_xor((int) m, 16, WAVE)); }
-					min_key = m;
-				} else {
-					min_key = key;
-				}
-			}
+			step(pair & 0xFFFFu, c0 + j);
+			step(pair >> 16, c0 + j + 1);
 		}
+	}
+
+	__device__ __forceinline__ void step(uint32_t k16, int expert) {
+		const uint32_t entry = k16 > KEY16_NEG_INF ? (k16 << 16) | (0xFFFFu - (uint32_t) expert) : 0u;
+		max_key16 = max(max_key16, k16);
+		key = key == min_key ? max(key, entry) : key;
+		min_key = key;
+		if (LANES > 1) { min_key = key_min_step<0xB1>(min_key); }
+		if (LANES > 2) { min_key = key_min_step<0x4E>(min_key); }
+		if (LANES > 4) { min_key = key_min_step<0x141>(min_key); }
+		if (LANES > 8) { min_key = key_min_step<0x140>(min_key); }
+		if (LANES > 16) { min_key = min(min_key, (uint32_t) __shfl_xor((int) min_key, 16, WAVE)); }
 	}
 
 	/* softmax over the K slots, summed in slot order; the reference subtracts the max in bf16 before expf
