@@ -240,7 +240,7 @@ def ragged_n_tile_rows(M, K, counts, work_groups=256):
     def rounds(tile_rows):
         return -(-(-(-M // 256) * sum(-(-int(c) // tile_rows) for c in counts)) // work_groups)
 
-    cost = {288: rounds(288) * 544 * 100 * kt, 384: rounds(384) * 640 * (103 * kt + 160)}
+    cost = {288: rounds(288) * 544 * 100 * kt, 384: rounds(384) * 640 * (95 * kt + 210)}
     cost.update({rows: rounds(rows) * (256 + rows) * 107 * kt for rows in (224, 192)})
     return out[-1] if cost[out[-1]] < cost[out[0]] else out[0]
 
@@ -475,7 +475,7 @@ def tiling_sweep(args):
             tiles_m, kt = -(-M // 256), -(-K // 64)
             narrow = -(-tiles_m * int(sum(-(-int(c) // 288) for c in counts)) // 256)
             wide = -(-tiles_m * int(sum(-(-int(c) // 384) for c in counts)) // 256)
-            rule = 384 if wide * 640 * (103 * kt + 160) < narrow * 544 * 100 * kt else 8
+            rule = 384 if wide * 640 * (95 * kt + 210) < narrow * 544 * 100 * kt else 8
             cases.append({"groups": G, "M": M, "K": K, "rows": rows if kind == "even" else "%d %s" % (rows, kind), "ms_8": round(best[8], 4),
                           "ms_384": round(best[384], 4), "ms_default": round(best[0], 4), "rule": rule})
             for d in (d_W, d_X, d_D, d_cum):

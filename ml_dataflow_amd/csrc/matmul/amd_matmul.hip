@@ -390,6 +390,7 @@ static double expected_rounds(const GemmParams & p, long tile_rows, int rows_dea
 
 /* expected costs of the tilings, and the cheapest.  No tiling is faster than the weights arrive (STREAMED_WEIGHTS: 6 TB/s).
  * 384 is never the cheapest where its kernel does not apply, whatever `cost` says of it. */
+#define WIDE_TILE_COST_UNEVEN(rounds, k_tiles) ((rounds) * (256 + 384) * (103 * (k_tiles) + 160))
 #define STREAMED_WEIGHTS(bytes) ((bytes) / 200)
 static double larger(double a, double b) { return a > b ? a : b; }
 static int cheapest_tiling(const GemmParams & p, long groups, bool four_ok, int rows_dealt, double cost[RAGGED_N_TILINGS]) {
@@ -398,7 +399,10 @@ static int cheapest_tiling(const GemmParams & p, long groups, bool four_ok, int 
 	const double streamed = STREAMED_WEIGHTS((double) p.num_groups * p.M * p.K * 2.0);
 	int best = four_ok && WIDE_TILE_COST(wide, k_tiles) < NARROW_TILE_COST(narrow, k_tiles) ? RAGGED_N_384 : RAGGED_N_288;
 	cost[RAGGED_N_288] = larger(NARROW_TILE_COST(narrow, k_tiles), streamed);
-	cost[RAGGED_N_384] = larger(WIDE_TILE_COST(wide, k_tiles), streamed);
+	/* a second tiling costs every launch 3 us: the lists that ask for one go on charging the larger tile 8-10 % more, so that it is asked for
+	 * where that tile gains at least as much (at its own price the up-projections of 32 groups of 512 rows, 1408 x 2048, went out on
+	 * two tilings, and a grouped training step of 4096 tokens took 1405 us instead of 1389) */
+	cost[RAGGED_N_384] = larger(rows_dealt == ROWS_EVEN ? WIDE_TILE_COST(wide, k_tiles) : WIDE_TILE_COST_UNEVEN(wide, k_tiles), streamed);
 	for (int tiling = RAGGED_N_224; tiling <= RAGGED_N_192; tiling++) {
 		const long rows = ragged_n_rows(tiling);
 		cost[tiling] = larger(FINER_TILE_COST(expected_rounds(p, rows, rows_dealt, groups), rows, k_tiles), streamed);
@@ -494,7 +498,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 		groups = groups < 8 ? 8 : groups;
 		const long wide = tiles_of(tiles, groups), narrow = tiles_of(grid_big, groups);
 		const long k_tiles = tiles_of(p.K, BK);
-		if (wide_only || wide * (256 + 384) * (103 * k_tiles + 160) < narrow * (256 + 256) * 100 * k_tiles) {
+		if (wide_only || wide * (256 + 384) * (95 * k_tiles + 210) < narrow * (256 + 256) * 100 * k_tiles) {
 			if (pk) { return launch_w4d<true, MODE_SINGLE>(p, tiles, cu_count, stream); }
 			return launch_w4d<false, MODE_SINGLE>(p, tiles, cu_count, stream);
 		}

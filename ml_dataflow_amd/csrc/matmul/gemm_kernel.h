@@ -226,16 +226,17 @@ __device__ __forceinline__ long count_tiles(const GemmParams & p) {
 
 /* Which tiling of the token rows is cheapest for this launch.  A launch takes (rounds of tiles over the work-groups) x
  * (time of a tile), and a k-tile step is paced by the bytes it fetches: 256 + 288 rows against 256 + 384 rows of 128
- * bytes, the larger tile at 3 % fewer bytes per clock plus what 1.6 k-tiles take per tile (its tiles change over
- * with fewer loads in flight; measured over group sizes of 256-2048 rows, K of 1024-4096 and the layer's launches: 3-7 %
- * at 64 k-tiles, 7-15 % at 16).  The 384 tiling wins where the groups are long enough to fill its tiles and the rounds
- * come out even; with short or very uneven groups the narrower tiles waste less.  Tiles of 224 and 192 rows serve the
+ * bytes, the larger tile at 5 % less per byte plus what 2 k-tiles take per tile.  Over 48 launches of 32 and 64 groups of 300-1500 rows
+ * dealt at random, K of 1024-4096, timed on both, the rule's choice is 0.1 % behind the better one (3 % more per byte and 1.6 k-tiles,
+ * which held before that kernel's epilogue was generated, 0.6 %, up to 10).  us on 288 and 384: 32 groups of 1024 rows, 2816 x 2048, 348
+ * and 330, of 1500, 2048 x 2816, 501 and 456, 64 groups of 1500, 1024 x 4096, 727 and 657, of 512 259 and 276.
+ * The 384 tiling wins where the groups are long enough to fill its tiles and the rounds come out even; with short or very uneven groups the narrower tiles waste less.  Tiles of 224 and 192 rows serve the
  * sizes between: 32 groups of 430 rows, 1408 x 2048, take 85 us in two rounds of 224 and 97 in two of 288; 170 rows
  * 42 us on 192 (53 on 288), 24 groups of 512 rows, 1536 x 3008, 134 (158).  They are charged 7 % per byte: a round of
  * them costs 0-8 % more per k-tile and fetched row than one of 288 (2.6-3.7 ns for K of 1408-4096), most where the
  * weights of many m-tiles come from HBM (64 groups of about 375 rows, 2048 x 4096: 407 us on 384, 434 on 224).
  * All sides are scaled by the k-tiles of a tile; the host compares them for the tiles it expects (ragged_n_tilings). */
-#define WIDE_TILE_COST(rounds, k_tiles) ((rounds) * (256 + 384) * (103 * (k_tiles) + 160))
+#define WIDE_TILE_COST(rounds, k_tiles) ((rounds) * (256 + 384) * (95 * (k_tiles) + 210))
 #define NARROW_TILE_COST(rounds, k_tiles) ((rounds) * (256 + 288) * 100 * (k_tiles))
 #define FINER_TILE_COST(rounds, rows, k_tiles) ((rounds) * (256 + (rows)) * 107 * (k_tiles))
 enum { RAGGED_N_288, RAGGED_N_384, RAGGED_N_224, RAGGED_N_192, RAGGED_N_TILINGS };
