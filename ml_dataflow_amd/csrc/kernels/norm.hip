@@ -163,6 +163,7 @@ default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
  * two or three loads in flight (30 registers) and not eight.  Eight rows at a time take the same 104.7 us in the sequence above.
  * Algorithmic HBM bytes: 4*n_rows*n_cols read, 4*grid*n_cols written. */
 #define BWD_W_ROWS 4
+#define BWD_W_SLABS 4          /* rows of four slabs and more go one by one: the three passes of 32768 x 8192 take 823 us, in fours 834 */
 extern "C" __global__ void __launch_bounds__(ROW_THREADS)
 default_rms_norm_bwd_w_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const float * __restrict__ fwd_rms_vals,
 										const bf16_t * __restrict__ X_inp, const bf16_t * __restrict__ upstream_dX,
@@ -191,7 +192,7 @@ default_rms_norm_bwd_w_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 	const u32x4 * x = (const u32x4 *) (X_inp + (size_t) first * n_cols) + v;
 	const u32x4 * g = (const u32x4 *) (upstream_dX + (size_t) first * n_cols) + v;
 	int i = 0;
-	for (; i + BWD_W_ROWS <= rows; i += BWD_W_ROWS) {
+	for (; gridDim.y < BWD_W_SLABS && i + BWD_W_ROWS <= rows; i += BWD_W_ROWS) {
 		u32x4 qx[BWD_W_ROWS], qg[BWD_W_ROWS];
 		float r[BWD_W_ROWS];
 		#pragma unroll
@@ -212,6 +213,7 @@ default_rms_norm_bwd_w_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 			}
 		}
 	}
+	#pragma unroll 8
 	for (; i < rows; i++) {
 		const float r = fwd_rms_vals[first + i];
 		float fx[8], fg[8];
