@@ -197,16 +197,17 @@ def replay_step_with_events(be, layer, T, d_X, d_out, d_dY, d_dX, d_bias, backwa
 # HBM bytes per launch (average over the launches of a class) from two hardware counter runs of this script with
 # --calibration-copy (rocprofv3 --pmc FETCH_SIZE, then WRITE_SIZE), each scaled by what the counter reads for the
 # calibration copy of known size (fetch x1.985, write x1.000).  Only valid for the workload and the schedule (fused) they were taken on.
+# The weight gradients (gemm_nt_dw, gemm_dw13) have no entry: the counters were taken on the kernel they ran on before.
 TRAFFIC_SOURCE = ("profiles/moe_layer_%s_hbm_traffic.md: hardware counters of two separate runs of this script, not of this run")
 MEASURED_TRAFFIC_BYTES = {
     "config4_fwdbwd_8192x4096_e64k8_h1024": {
-        "gemm_up13": 2589760385, "gemm_tn": 1458409166, "gemm_nn": 1540948489, "gemm_nt_dw": 1862856075, "gemm_dx13": 2281766452,
-        "gemm_dw13": 3738749644, "dispatch_scaled": 605606034, "swiglu": 400721551, "swiglu_bwd_x_routed": 822827377, "combine": 668834607,
+        "gemm_up13": 2589760385, "gemm_tn": 1458409166, "gemm_nn": 1540948489, "gemm_dx13": 2281766452,
+        "dispatch_scaled": 605606034, "swiglu": 400721551, "swiglu_bwd_x_routed": 822827377, "combine": 668834607,
         "combine_grad": 601168066, "dispatch": 604555665,
     },
     "config5_fwdbwd_65536x4096_e64k8_h1024": {
-        "gemm_up13": 21330367076, "gemm_tn": 12462374745, "gemm_nn": 9885439367, "gemm_nt_dw": 9458770557, "gemm_dx13": 33712088322,
-        "gemm_dw13": 18547757374, "dispatch_scaled": 4844596105, "swiglu": 3205532585, "swiglu_bwd_x_routed": 6617731110, "combine": 5350080114,
+        "gemm_up13": 21330367076, "gemm_tn": 12462374745, "gemm_nn": 9885439367, "gemm_dx13": 33712088322,
+        "dispatch_scaled": 4844596105, "swiglu": 3205532585, "swiglu_bwd_x_routed": 6617731110, "combine": 5350080114,
         "combine_grad": 4808782033, "dispatch": 4836259094,
     },
 }
