@@ -96,47 +96,52 @@ default_rms_norm_recompute_bf16_kernel(int n_rows, int n_cols, const bf16_t * __
 
 /* Backward w.r.t. the input, accumulated into dX; X_out (nullable) receives the recomputed forward output.
  * Launch: grid = n_rows, block = 256.
- * Algorithmic HBM bytes: 6*n_rows*n_cols read (x, g, dX), 2*n_rows*n_cols written (+2*n_rows*n_cols for X_out). */
-extern "C" __global__ void __launch_bounds__(ROW_THREADS)
-default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const float * __restrict__ fwd_rms_vals,
-										const bf16_t * __restrict__ rms_weight, const bf16_t * __restrict__ X_inp,
-										const bf16_t * __restrict__ upstream_dX, bf16_t * dX, bf16_t * X_out) {
-	__shared__ float scratch[ROW_WAVES];
-	(void) eps;
-	const int row = blockIdx.x;
-	if (row >= n_rows) {
-		return;
-	}
+ * Algorithmic HBM bytes: 6*n_rows*n_cols read (x, g, dX), 2*n_rows*n_cols written (+2*n_rows*n_cols for X_out).
+ *
+ * Two forms, by the rows.  A compute unit holds six of the work-groups (80 registers: the row's x, g and dX stay in them), 256 compute units
+ * 1536.  Beyond that, MANY_ROWS, rows wait for their sums while others load: dX is loaded with x and g, behind the scale, as loads come
+ * back in order and the sum would wait for dX too; results pass the caches by.  Up to 1536 rows everything is in flight at once,
+ * an early load of dX has nothing to hide behind, and the next kernel finds what was stored in the memory-side cache: dX behind the sum,
+ * plain stores.  us, forward, bwd_x and bwd_w in turn over one set of arrays, few-rows form and the other: 1120 x 7232 34.1 and 35.5, 1536 x
+ * 6144 39.6 and 40.8, 2048 x 8192 64.1 and 62.4, 8192 x 4096 102.3 and 99.6, over eight sets 71.5 and 65.9 for 2048 x 8192, 113.0 and 104.8
+ * for 8192 x 4096.  At 83 registers, five work-groups a compute unit, and with dX in front of the scale the other form took 36.2 at 1120 x 7232,
+ * 79.2 at 3000 x 7232 (77.6 now).  Left: 1537 to 1792 rows, which the few-rows form alone, 67 registers, would hold at once: 2-6 % slower than there
+ * when all arrays are in the caches, within 2 % when none is (from 4096 columns on). */
+#define BWD_X_FEW_ROWS (6 * 256)
+template <bool MANY_ROWS>
+__device__ __forceinline__ void
+rms_norm_bwd_x_row(int n_cols, float r, const u32x4 * __restrict__ x, const u32x4 * __restrict__ g, const u32x4 * __restrict__ w, u32x4 * d, u32x4 * xo, float * scratch) {
 	const int nvec = n_cols >> 3;
-	const float r = fwd_rms_vals[row];
-	const u32x4 * x = (const u32x4 *) (X_inp + (size_t) row * n_cols);
-	const u32x4 * g = (const u32x4 *) (upstream_dX + (size_t) row * n_cols);
-	const u32x4 * w = (const u32x4 *) rms_weight;
-	u32x4 * d = (u32x4 *) (dX + (size_t) row * n_cols);
-	u32x4 * xo = X_out ? (u32x4 *) (X_out + (size_t) row * n_cols) : nullptr;
-
 	u32x4 keep_x[NORM_MAX_VEC], keep_g[NORM_MAX_VEC], keep_d[NORM_MAX_VEC];
 	float part[1] = {0.0f};
 	int j = 0;
 	for (int v = threadIdx.x; v < nvec; v += ROW_THREADS, j++) {
 		const u32x4 qx = x[v];
 		const u32x4 qg = __builtin_nontemporal_load(g + v);
+		const u32x4 qw = w[v];
+		__builtin_amdgcn_sched_barrier(0);              /* loads come back in order: dX's behind what the sum needs */
 		if (j < NORM_MAX_VEC) {
 			keep_x[j] = qx;
 			keep_g[j] = qg;
-			keep_d[j] = d[v];
+			if (MANY_ROWS) {
+				keep_d[j] = d[v];
+			}
 		}
 		float fx[8], fg[8], fw[8], y[8];
 		unpack8(qx, fx);
 		unpack8(qg, fg);
-		unpack8(w[v], fw);
+		unpack8(qw, fw);
 		#pragma unroll
 		for (int i = 0; i < 8; i++) {
 			y[i] = (fx[i] * r) * fw[i];
 			part[0] = __builtin_fmaf(y[i], fg[i], part[0]);
 		}
 		if (xo) {
-			__builtin_nontemporal_store(pack8(y), xo + v);
+			if (MANY_ROWS) {
+				__builtin_nontemporal_store(pack8(y), xo + v);
+			} else {
+				xo[v] = pack8(y);
+			}
 		}
 	}
 	block_sum<1>(part, scratch);
@@ -147,12 +152,39 @@ default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 		unpack8(j < NORM_MAX_VEC ? keep_x[j] : x[v], fx);
 		unpack8(j < NORM_MAX_VEC ? keep_g[j] : g[v], fg);
 		unpack8(w[v], fw);
-		unpack8(j < NORM_MAX_VEC ? keep_d[j] : d[v], fd);
+		unpack8(MANY_ROWS && j < NORM_MAX_VEC ? keep_d[j] : d[v], fd);
 		#pragma unroll
 		for (int i = 0; i < 8; i++) {
 			fd[i] += r * (fg[i] * fw[i] - c_div_n * (fx[i] * r));
 		}
-		__builtin_nontemporal_store(pack8(fd), d + v);
+		if (MANY_ROWS) {
+			__builtin_nontemporal_store(pack8(fd), d + v);
+		} else {
+			d[v] = pack8(fd);
+		}
+	}
+}
+
+extern "C" __global__ void __launch_bounds__(ROW_THREADS)
+default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const float * __restrict__ fwd_rms_vals,
+										const bf16_t * __restrict__ rms_weight, const bf16_t * __restrict__ X_inp,
+										const bf16_t * __restrict__ upstream_dX, bf16_t * dX, bf16_t * X_out) {
+	__shared__ float scratch[ROW_WAVES];
+	(void) eps;
+	const int row = blockIdx.x;
+	if (row >= n_rows) {
+		return;
+	}
+	const float r = fwd_rms_vals[row];
+	const u32x4 * x = (const u32x4 *) (X_inp + (size_t) row * n_cols);
+	const u32x4 * g = (const u32x4 *) (upstream_dX + (size_t) row * n_cols);
+	const u32x4 * w = (const u32x4 *) rms_weight;
+	u32x4 * d = (u32x4 *) (dX + (size_t) row * n_cols);
+	u32x4 * xo = X_out ? (u32x4 *) (X_out + (size_t) row * n_cols) : nullptr;
+	if (n_rows > BWD_X_FEW_ROWS) {
+		rms_norm_bwd_x_row<true>(n_cols, r, x, g, w, d, xo, scratch);
+	} else {
+		rms_norm_bwd_x_row<false>(n_cols, r, x, g, w, d, xo, scratch);
 	}
 }
 

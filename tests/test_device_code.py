@@ -51,3 +51,12 @@ def test_no_lane_move_in_a_reversed_operation_of_the_matmul_library(tmp_path):
     text = subprocess.run([objdump, "-d", str(tmp_path / objects[0])], check=True, capture_output=True, text=True).stdout
     assert "_dpp" in text
     assert not REVERSED_WITH_LANE_MOVE.search(text)
+
+
+def test_six_work_groups_of_the_norms_backward_fit_a_compute_unit(tmp_path):
+    """the number that its rule for few rows counts with (norm.hip): 512 registers a lane of a SIMD, four waves a work-group, one on each"""
+    text = assembly(os.path.join(CSRC, "kernels", "hip_kernels.hip"), tmp_path)
+    entry = next(e for e in text[text.index("amdhsa.kernels:"):].split("  - .agpr_count:") if ".symbol:         default_rms_norm_bwd_x_bf16_bf16_kernel.kd" in e)
+    count = {name: int(re.search(r"\.%s: +(\d+)" % name, entry).group(1)) for name in ("vgpr_count", "vgpr_spill_count", "private_segment_fixed_size")}
+    assert count["vgpr_count"] <= 80 and 512 // 80 == 6
+    assert count["vgpr_spill_count"] == 0 and count["private_segment_fixed_size"] == 0

@@ -122,6 +122,29 @@ def test_rms_norm_bwd_w_few_rows_and_more(backend, rows, cols):
     assert (be.read(d_dW.ptr, (cols,), np.uint16) == want).all()
 
 
+@pytest.mark.parametrize("with_out", [True, False])
+@pytest.mark.parametrize("rows,cols", [(1536, 64), (1536, 4104), (1536, 8200), (1537, 64), (1537, 2056), (1537, 8192), (1537, 8200), (1800, 6152)])
+def test_rms_norm_bwd_x_with_few_rows_and_more(backend, rows, cols, with_out):
+    """Up to 1536 rows and beyond are two forms of one kernel: a row's result has the same bits from either.  The first 700 rows alone
+    run on the first form, and so do all 1536."""
+    print("case rms_norm_bwd_x forms rows=%d cols=%d out=%d" % (rows, cols, with_out), flush=True)
+    be = backend
+    rng = np.random.default_rng(rows + cols)
+    X, G, W, start = normal_bf16(rng, (rows, cols), 1.5), normal_bf16(rng, (rows, cols)), normal_bf16(rng, (cols,)), normal_bf16(rng, (rows, cols), 0.5)
+    rms = (0.5 + rng.random(rows)).astype(np.float32)
+    d_X, d_G, d_W, d_rms = be.upload(X), be.upload(G), be.upload(W), be.upload(rms)
+    got = {}
+    for n in (700, rows):
+        d_dX, d_out = be.upload(start), be.upload(np.full((rows, cols), 0x4242, np.uint16))
+        assert be.lib.dataflow_submit_default_rms_norm_bwd_x(be.hp, CS, BF, BF, n, cols, EPS, d_rms.ptr, d_W.ptr, d_X.ptr, d_G.ptr, d_dX.ptr, d_out.ptr if with_out else None) == 0
+        be.sync(CS)
+        got[n] = be.read(d_dX.ptr, (rows, cols), np.uint16), be.read(d_out.ptr, (rows, cols), np.uint16)
+        assert (got[n][0][n:] == start[n:]).all() and (got[n][1][n if with_out else 0:] == 0x4242).all()
+    for few, many in zip(got[700], got[rows]):
+        assert (few[:700] == many[:700]).all()
+    assert (got[rows][0] != start).any(axis=1).all()
+
+
 def test_rms_norm_rejects_bad_shapes_and_small_workspace(backend):
     be = backend
     buf = be.alloc(4096)
