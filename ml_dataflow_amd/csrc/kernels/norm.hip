@@ -195,7 +195,10 @@ default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
  * two or three loads in flight (30 registers) and not eight.  Eight rows at a time take the same 104.7 us in the sequence above.
  * Algorithmic HBM bytes: 4*n_rows*n_cols read, 4*grid*n_cols written. */
 #define BWD_W_ROWS 4
-#define BWD_W_SLABS 4          /* rows of four slabs and more go one by one: the three passes of 32768 x 8192 take 823 us, in fours 834 */
+/* From this row length on the rows go one by one, by the loop that the compiler leaves two or three loads in flight: us alone, one by one
+ * and in fours, 8192 x 4480 33.4 and 31.7, 16384 x 4544 55.8 and 54.9, 16384 x 4608 56.2 and 55.7 (from memory 56.1 and 56.7), 16384 x 5120 58.7
+ * and 62.1, 32768 x 6144 127 and 137, 32768 x 8192 166 and 185. */
+#define BWD_W_FOURS_COLS 4608
 extern "C" __global__ void __launch_bounds__(ROW_THREADS)
 default_rms_norm_bwd_w_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const float * __restrict__ fwd_rms_vals,
 										const bf16_t * __restrict__ X_inp, const bf16_t * __restrict__ upstream_dX,
@@ -224,7 +227,7 @@ default_rms_norm_bwd_w_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 	const u32x4 * x = (const u32x4 *) (X_inp + (size_t) first * n_cols) + v;
 	const u32x4 * g = (const u32x4 *) (upstream_dX + (size_t) first * n_cols) + v;
 	int i = 0;
-	for (; gridDim.y < BWD_W_SLABS && i + BWD_W_ROWS <= rows; i += BWD_W_ROWS) {
+	for (; n_cols < BWD_W_FOURS_COLS && i + BWD_W_ROWS <= rows; i += BWD_W_ROWS) {
 		u32x4 qx[BWD_W_ROWS], qg[BWD_W_ROWS];
 		float r[BWD_W_ROWS];
 		#pragma unroll

@@ -122,6 +122,23 @@ def test_rms_norm_bwd_w_few_rows_and_more(backend, rows, cols):
     assert (be.read(d_dW.ptr, (cols,), np.uint16) == want).all()
 
 
+@pytest.mark.parametrize("rows,cols", [(1537, 4600), (1537, 4608), (4099, 4600), (4099, 4608), (6200, 72), (2048, 6152)])
+def test_rms_norm_bwd_w_rows_in_fours_and_one_by_one(backend, rows, cols):
+    """Three to twelve rows a work-group, on both sides of the row length from which on they go one by one.  Whole numbers as above: exact."""
+    print("case rms_norm_bwd_w fours rows=%d cols=%d" % (rows, cols), flush=True)
+    be = backend
+    rng = np.random.default_rng(rows + cols)
+    x, g = rng.integers(-4, 5, (rows, cols)).astype(np.float32), rng.integers(-4, 5, (rows, cols)).astype(np.float32)
+    rms = np.exp2(rng.integers(-1, 2, rows)).astype(np.float32)
+    d_X, d_G, d_rms, d_dW = be.upload(f32_to_bf16(x)), be.upload(f32_to_bf16(g)), be.upload(rms), be.upload(np.zeros(cols, np.uint16))
+    ws_bytes = 256 + 512 * cols * 4
+    d_ws = be.alloc(ws_bytes)
+    assert be.lib.dataflow_submit_default_rms_norm_bwd_w(be.hp, CS, BF, BF, rows, cols, EPS, d_rms.ptr, d_X.ptr, d_G.ptr, d_dW.ptr, ws_bytes, d_ws.ptr) == 0
+    be.sync(CS)
+    want = f32_to_bf16(np.einsum("rc,r->c", x * g, rms, dtype=np.float64).astype(np.float32))
+    assert (be.read(d_dW.ptr, (cols,), np.uint16) == want).all()
+
+
 @pytest.mark.parametrize("with_out", [True, False])
 @pytest.mark.parametrize("rows,cols", [(1536, 64), (1536, 4104), (1536, 8200), (1537, 64), (1537, 2056), (1537, 8192), (1537, 8200), (1800, 6152)])
 def test_rms_norm_bwd_x_with_few_rows_and_more(backend, rows, cols, with_out):
