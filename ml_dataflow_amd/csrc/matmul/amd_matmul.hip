@@ -388,21 +388,20 @@ static double expected_rounds(const GemmParams & p, long tile_rows, int rows_dea
 	return rounds;
 }
 
-/* expected costs of the tilings, and the cheapest.  No tiling is faster than the weights arrive (STREAMED_WEIGHTS: 6 TB/s).
- * 384 is never the cheapest where its kernel does not apply, whatever `cost` says of it. */
-#define WIDE_TILE_COST_UNEVEN(rounds, k_tiles) ((rounds) * (256 + 384) * (103 * (k_tiles) + 160))
+/* expected costs of the tilings, and the cheapest by them.  No tiling is faster than the weights arrive (STREAMED_WEIGHTS: 6 TB/s).
+ * 384 is never the cheapest where its kernel does not apply, whatever `cost` says of it.  `second`: for uneven rows beside another tiling, see
+ * ragged_n_tilings. */
+#define WIDE_TILE_COST_SECOND(rounds, k_tiles) ((rounds) * (256 + 384) * (103 * (k_tiles) + 160))
 #define STREAMED_WEIGHTS(bytes) ((bytes) / 200)
 static double larger(double a, double b) { return a > b ? a : b; }
-static int cheapest_tiling(const GemmParams & p, long groups, bool four_ok, int rows_dealt, double cost[RAGGED_N_TILINGS]) {
+static int cheapest_tiling(const GemmParams & p, long groups, bool four_ok, int rows_dealt, bool second, double cost[RAGGED_N_TILINGS]) {
 	const long k_tiles = tiles_of(p.K, BK);
 	const double narrow = expected_rounds(p, 288, rows_dealt, groups), wide = expected_rounds(p, 384, rows_dealt, groups);
 	const double streamed = STREAMED_WEIGHTS((double) p.num_groups * p.M * p.K * 2.0);
-	int best = four_ok && WIDE_TILE_COST(wide, k_tiles) < NARROW_TILE_COST(narrow, k_tiles) ? RAGGED_N_384 : RAGGED_N_288;
+	const double surcharge = second ? larger(WIDE_TILE_COST_SECOND(wide, k_tiles) - WIDE_TILE_COST(wide, k_tiles), 0.0) : 0.0;
+	int best = four_ok && surcharge + WIDE_TILE_COST(wide, k_tiles) < NARROW_TILE_COST(narrow, k_tiles) ? RAGGED_N_384 : RAGGED_N_288;
 	cost[RAGGED_N_288] = larger(NARROW_TILE_COST(narrow, k_tiles), streamed);
-	/* a second tiling costs every launch 3 us: the lists that ask for one go on charging the larger tile 8-10 % more, so that it is asked for
-	 * where that tile gains at least as much (at its own price the up-projections of 32 groups of 512 rows, 1408 x 2048, went out on
-	 * two tilings, and a grouped training step of 4096 tokens took 1405 us instead of 1389) */
-	cost[RAGGED_N_384] = larger(rows_dealt == ROWS_EVEN ? WIDE_TILE_COST(wide, k_tiles) : WIDE_TILE_COST_UNEVEN(wide, k_tiles), streamed);
+	cost[RAGGED_N_384] = larger(surcharge + WIDE_TILE_COST(wide, k_tiles), streamed);
 	for (int tiling = RAGGED_N_224; tiling <= RAGGED_N_192; tiling++) {
 		const long rows = ragged_n_rows(tiling);
 		cost[tiling] = larger(FINER_TILE_COST(expected_rounds(p, rows, rows_dealt, groups), rows, k_tiles), streamed);
@@ -422,7 +421,13 @@ static int cheapest_tiling(const GemmParams & p, long groups, bool four_ok, int 
  * took 4.7 %.  A first training step of 3001 tokens, 32 experts, dim 2048 934 -> 905 us, a forward of 8192 tokens 635 -> 632, one with
  * a Zipf router, whose launches take a second tiling, unchanged.  Over 341 launches whose rows lie in one, two or four of 8-64 experts to 95 % or are dealt by Zipf routers, this
  * rule is 3.4 % behind the best, without the second list 4.8 %, up to three launches 6.8 %; 17 / 41 of them are more than 3 % slower
- * than those three launches and 4 / 27 more than 8 % (1024 x 3072, 41 groups, 6205 of 6478 rows in one: 90 / 136 us, on 288 alone 87). */
+ * than those three launches and 4 / 27 more than 8 % (1024 x 3072, 41 groups, 6205 of 6478 rows in one: 90 / 136 us, on 288 alone 87).
+ * As a second tiling beside another one 384 is charged 4 to 8 % more from 1024 k on (its price before its epilogue was generated): at its own
+ * price the up-projections of 32 groups of 512 rows, 1408 x 2048, went out on two tilings, and a grouped training step of 4096 tokens took 1405 us
+ * instead of 1389.  Where 384 is the first, UNEVEN compares at its own price: 18 launches to which the surcharge added 288 take, rows
+ * dealt by a Zipf router, 3 % less on 384 alone (3648 x 1792, 61 groups, 22868 rows: 385 us on both, 288 chosen, 366; 17 launches more, to which
+ * neither adds it, 3-12 % less on 384 than on 288).  IN_ONE charges it always: there the narrower tile is the better one by up to
+ * 45 % (2176 x 896, 26 groups, 7056 rows: 53 us with 224, 71 without). */
 #define SECOND_TILING_MARGIN 121000          /* 4 us */
 #define IN_ONE_TILING_MARGIN 454000          /* 15 us */
 static int ragged_n_tilings(const GemmParams & p, long cu_count, bool four_ok) {
@@ -431,10 +436,10 @@ static int ragged_n_tilings(const GemmParams & p, long cu_count, bool four_ok) {
 	groups = groups < 8 ? 8 : groups;
 	double cost[ROWS_DISTRIBUTIONS][RAGGED_N_TILINGS];
 	int cheapest[ROWS_DISTRIBUTIONS];
-	for (int dealt = 0; dealt < ROWS_DISTRIBUTIONS; dealt++) {
-		cheapest[dealt] = cheapest_tiling(p, groups, four_ok, dealt, cost[dealt]);
+	const int first = cheapest[ROWS_EVEN] = cheapest_tiling(p, groups, four_ok, ROWS_EVEN, false, cost[ROWS_EVEN]);
+	for (int dealt = ROWS_UNEVEN; dealt < ROWS_DISTRIBUTIONS; dealt++) {
+		cheapest[dealt] = cheapest_tiling(p, groups, four_ok, dealt, dealt == ROWS_IN_ONE || first != RAGGED_N_384, cost[dealt]);
 	}
-	const int first = cheapest[ROWS_EVEN];
 	int second = first;
 	double least = 0.0;                             /* the worst case with `first` and `second`, over the cheapest's cost */
 	for (int tiling = 0; tiling < RAGGED_N_TILINGS; tiling++) {

@@ -84,6 +84,21 @@ def test_a_good_tiling_for_uneven_rows_is_among_those_that_go_out(plan, M, K, ro
     assert best <= 1.13 * min(us), tilings
 
 
+# M, K, rows, groups, microseconds with rows dealt by a Zipf router on 288 and on 384 token rows alone
+MEASURED_BESIDE_384 = [
+    (3648, 1792, 22868, 61, (385, 366)), (3072, 1536, 30368, 50, (307, 292)), (3456, 1792, 30066, 27, (383, 357)), (3392, 1792, 31425, 22, (385, 361)),
+    (2176, 1024, 41136, 47, (197, 193)), (3840, 1536, 30783, 17, (334, 324)), (2368, 4096, 58539, 53, (1147, 995)), (1280, 3328, 90517, 52, (677, 632)),
+    (4096, 2048, 47615, 45, (720, 679)), (3712, 3584, 30358, 20, (713, 674)), (1920, 3584, 55494, 51, (762, 673)),
+]
+
+
+@pytest.mark.parametrize("M,K,rows,groups,us", MEASURED_BESIDE_384)
+def test_no_second_tiling_beside_384_where_uneven_rows_run_best_on_it(plan, M, K, rows, groups, us):
+    """one price for both sides of a comparison: the 384 tiling is not chosen at one and then found too dear at another"""
+    assert us[1] < us[0]
+    assert plan.amd_matmul_planned_tilings(M, K, rows, groups, CUS) == 2
+
+
 def test_the_library_scratch_holds_every_split(plan):
     """amd_matmul_no_alloc leaves the op's bits because no split needs more than its 64 MiB: the plan is the same with any larger
     workspace."""
