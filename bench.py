@@ -814,8 +814,9 @@ def main():
                 tile_rows = ragged_n_tile_rows(rows_m[cls], k_of[cls], counts)
                 if tile_rows != 384:
                     four[cls] = kernel_of_class[cls].replace("288", str(tile_rows))
-        if args.gemm_kernel == 384 or (args.gemm_kernel == 0 and T * K >= 320 * E):      # the library's rule for the weight gradients
-            four.update(dict.fromkeys(("gemm_nt_dw", "gemm_dw13"), _W4K % "true, 2"))
+        for cls, M, N in (("gemm_nt_dw", H, D), ("gemm_dw13", D, 2 * H)):
+            if args.gemm_kernel == 384 or (args.gemm_kernel == 0 and mm.amd_matmul_planned_sliced(M, T * K, N, E, 1, 256)):
+                four[cls] = _W4K % "true, 2"
         kernel_of_class.update(four)
     by_kernel = {}
     for k, v in gemms.items():

@@ -55,8 +55,9 @@ int amd_matmul_no_alloc(Dataflow_Handle * dataflow_handle, int stream_id, int to
  *   FOUR_WAVES: one loading wave (operands through its registers) and three multiplying waves, 256 x 288 tiles.
  *   AUTO (the default): a ragged-N launch runs on the cheapest of the tilings of both (tiles of 384, 288, 224 or 192 token
  *     rows) for the group sizes that an even router gives: the number of tiles, in rounds over the compute units.
- *     For a single problem, whose tiles are known, tiles of 384 against those of 256.  Two k-major operands: four waves from K = 256 on,
- *     ragged K from 320 rows a group on with C, 512 without, where the caller gave the rows of all groups as K.  Everything else runs EIGHT_WAVES.
+ *     For a single problem, whose tiles are known, tiles of 384 against those of 256.  Two k-major operands, where they run on the 256 x 256 tile: four
+ *     waves from 512 rows a group (ragged K, the rows of all groups given as K) or K = 256 to 512 on with C, from 640 or K = 1024 without, from 2048
+ *     where one round of tiles is all (amd_matmul_planned_sliced of amd_matmul_plan.h).  Everything else runs EIGHT_WAVES.
  * The four-wave kernels are taken only where their limits hold (no C operand, N-side operand k-contiguous, K a multiple
  * of 128 and at most 2^21, M a multiple of 8, 16-byte aligned D; for two k-major operands M and N multiples of 8, C and D 16-byte
  * aligned), the eight-wave kernel elsewhere.  Results are

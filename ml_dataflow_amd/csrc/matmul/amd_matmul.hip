@@ -306,13 +306,22 @@ static bool w4k_ok(const GemmParams & p) {
 		   (!(p.C && p.beta != 0.0f) || (((uintptr_t) p.C) & 15) == 0);
 }
 
-/* Where the sliced kernel is the faster one.  Ragged K, where the caller said how many rows there are: from 320 a group on with C, from
- * 512 without.  Its tiles have at least 8 slices of 32 k-rows (5 without C), and a fixed part that two waves on a SIMD hide better: us,
- * eight waves and sliced, 32 groups, 2048 x 1408 with C, of 64 rows 77 and 89, of 256 96 and 100, of 320 106 and 106, of 375 114 and 110,
- * of 640 152 and 144; 1024 x 4096 without C, of 64 65 and 67, of 375 118 and 117, of 512 146 and 140, 2048 x 1408 without, of 375 85 and
- * 89, of 640 125 and 126.  One problem: from K = 256 on (4096 x 4096 with C, K 128: 17 and 17, 512: 29 and 24, 8192: 207 and 196). */
-static bool w4k_pays(int mode, const GemmParams & p) {
-	return mode == MODE_RAGGED_K ? (long) p.K >= (p.C && p.beta != 0.0f ? 320L : 512L) * p.num_groups : p.K >= 256;
+/* The k-rows a tile has to have, in the mean, for the sliced kernel to be the faster one.  Its tiles have at least 8 slices of 32 k-rows
+ * (5 without C), and a fixed part that two waves on a SIMD hide better; what it gains, beside the loads in flight, is the read of C.
+ * Time on it over time on eight waves.
+ * Ragged K, the groups' sizes on the device, 36 launches of 8-60 groups, 512-4096 x 512-4096, several rounds of tiles, even rows and rows dealt by a
+ * Zipf router, most of whose groups are shorter than the mean.  With C: 320 rows a group 0.985 and 1.068 (at worst 1.07 and 1.11), 384 0.982 and
+ * 1.035, 448 0.976 and 1.008, 512 0.975 and 0.990 (1.02 and 1.03), 640 0.970 and 0.966.  Without: 512 0.996 and 0.978 (1.06 and 1.02), 640 0.990
+ * and 0.961 (1.03 and 1.01).  In one round or less (14 launches of 150-240 tiles): with C 512 0.938 and 1.007, without 1024 1.021 and
+ * 0.975, 1536 0.984 and 0.937 (1.04 and 0.98), 2048 0.930 and 0.889.
+ * One problem (14 of one round, 5 of more): with C, K 256 0.91 in one round, 0.99 (1.05) in more, 512 0.88; without, in one round 512 1.04,
+ * 1024 1.017, 1536 0.998 (1.013), 2048 0.988, in more 512 0.994 (1.02), 1024 0.972.  The lines lie where neither distribution loses. */
+static bool w4k_pays(int mode, const GemmParams & p, long tiles, long cu_count) {
+	const bool reads_c = p.C && p.beta != 0.0f, one_round = tiles <= cu_count;
+	if (mode == MODE_RAGGED_K) {
+		return (long) p.K >= (reads_c ? 512L : one_round ? 2048L : 640L) * p.num_groups;
+	}
+	return p.K >= (reads_c ? (one_round ? 256 : 512) : one_round ? 2048 : 1024);
 }
 
 /* a ragged-N launch without C on one of its tilings; grid: an upper bound on the tiles */
@@ -468,6 +477,17 @@ extern "C" int amd_matmul_planned_tilings(int M, int K, int N, int num_groups, i
 	return ragged_n_tilings(p, cu_count, w4_ok(p));
 }
 
+extern "C" int amd_matmul_planned_sliced(int M, int K, int N, int num_groups, int has_c, int cu_count) {
+	GemmParams p;
+	memset(&p, 0, sizeof(p));
+	p.M = M; p.K = K; p.N = N;
+	p.num_groups = num_groups;
+	p.C = has_c ? (const bf16_t *) scratch_of_device : NULL;
+	p.beta = has_c ? 1.0f : 0.0f;
+	const int mode = num_groups ? MODE_RAGGED_K : MODE_SINGLE;
+	return choose_tile(mode, p, cu_count) == TILE_BIG && w4k_ok(p) && w4k_pays(mode, p, tiles_in_launch(TILE_BIG, mode, p), cu_count);
+}
+
 static long round_up8(long v) { return (v + 7) & ~7L; }
 
 #define BIG_TILE 256, 256, 4, 2          /* 8 waves, wave tile 64 x 128 */
@@ -558,7 +578,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 		return launch_staged<SMALL_TILE, true, true, MODE_RAGGED_K>(p, round_up8(grid_small), stream);
 	}
 	if constexpr (MODE != MODE_RAGGED_N) {
-		if (pk && qk && direct && big && !p.gather && (wide_only || (either && w4k_pays(MODE, p))) && w4k_ok(p)) {
+		if (pk && qk && direct && big && !p.gather && (wide_only || (either && w4k_pays(MODE, p, grid_big, cu_count))) && w4k_ok(p)) {
 			return launch_w4k<MODE>(p, grid_big, cu_count, stream);
 		}
 	}

@@ -19,6 +19,7 @@ def plan():
     lib = C.CDLL(os.path.join(B.LIB_DIR, "libamd_matmul.so"))
     lib.amd_matmul_planned_tile.argtypes = [C.c_int] * 5
     lib.amd_matmul_planned_tilings.argtypes = [C.c_int] * 5
+    lib.amd_matmul_planned_sliced.argtypes = [C.c_int] * 6
     lib.amd_matmul_planned_splits.argtypes = [C.c_int] * 6 + [C.c_uint64, C.c_int]
     return lib
 
@@ -97,6 +98,58 @@ def test_no_second_tiling_beside_384_where_uneven_rows_run_best_on_it(plan, M, K
     """one price for both sides of a comparison: the 384 tiling is not chosen at one and then found too dear at another"""
     assert us[1] < us[0]
     assert plan.amd_matmul_planned_tilings(M, K, rows, groups, CUS) == 2
+
+
+# M, K (ragged: rows of all groups), N, groups (0: one problem), C, microseconds on eight waves and on the sliced kernel: even rows, rows of a Zipf router
+MEASURED_SLICED = [
+    (1024, 65536, 4096, 64, 1, (586.9, 555.3), (667.2, 606.2)),
+    (4096, 65536, 2048, 64, 1, (1156.6, 1083.7), (1198.9, 1121.4)),
+    (1408, 16384, 2048, 32, 1, (144.5, 138.8), (170.3, 166.4)),
+    (2048, 12000, 2816, 32, 1, (210.4, 204.9), (217.5, 227.9)),
+    (1408, 12000, 2048, 32, 1, (118.1, 108.4), (128.5, 134.2)),
+    (3072, 13824, 1408, 36, 1, (206.1, 211.4), (208.8, 227.2)),
+    (3392, 24192, 2048, 54, 1, (495.8, 485.9), (510.1, 531.2)),
+    (3136, 12096, 1920, 27, 1, (226.5, 221.7), (230.4, 243.5)),
+    (3072, 23040, 1408, 36, 1, (283.9, 284.9), (304.4, 301.9)),
+    (896, 5120, 1344, 10, 1, (26.1, 24.2), (39.9, 40.9)),
+    (1024, 14336, 1024, 14, 1, (38.3, 35.5), (84.1, 80.7)),
+    (1024, 65536, 4096, 64, 0, (522.9, 487.9), (622.6, 552.8)),
+    (1856, 30720, 512, 60, 0, (87.5, 91.4), (174.5, 162.4)),
+    (1856, 46080, 512, 60, 0, (115.4, 116.9), (243.5, 219.4)),
+    (1024, 23552, 1600, 46, 0, (107.6, 113.5), (172.3, 165.0)),
+    (3136, 17280, 1920, 27, 0, (248.9, 244.1), (266.7, 260.0)),
+    (1152, 11700, 576, 13, 0, (27.8, 29.6), (68.9, 68.2)),
+    (896, 10240, 1344, 10, 0, (32.2, 34.2), (69.0, 68.0)),
+    (1024, 28672, 1024, 14, 0, (65.6, 58.3), (182.3, 151.9)),
+    (960, 45056, 1088, 11, 0, (109.5, 98.2), (289.0, 249.1)),
+    (3392, 256, 2880, 0, 0, (12.0, 13.4)),
+    (2496, 512, 3712, 0, 0, (16.4, 17.6)),
+    (2880, 1024, 3008, 0, 0, (25.4, 26.1)),
+    (3200, 4096, 2624, 0, 0, (80.4, 78.2)),
+    (4096, 512, 6144, 0, 0, (32.2, 32.8)),
+    (8192, 1024, 4096, 0, 0, (61.2, 58.6)),
+    (2752, 22084, 3968, 0, 0, (467.2, 418.4)),
+    (3456, 256, 4032, 0, 1, (19.4, 17.7)),
+    (3776, 1000, 4032, 0, 1, (38.3, 34.3)),
+    (5120, 256, 5120, 0, 1, (36.7, 38.5)),
+    (8192, 512, 4096, 0, 1, (49.8, 42.5)),
+]
+
+
+@pytest.mark.parametrize("case", MEASURED_SLICED)
+def test_the_sliced_kernel_runs_where_neither_even_nor_uneven_rows_lose_by_it(plan, case):
+    M, K, N, groups, has_c = case[:5]
+    ratios = [sliced / eight for eight, sliced in case[5:]]
+    if plan.amd_matmul_planned_sliced(M, K, N, groups, has_c, CUS):
+        assert max(ratios) <= 1.03, ratios                             # two runs of one kernel differ by up to 1 %, two kernels are compared
+    else:
+        assert max(ratios) > 1.0 or max(ratios) > 0.97 and groups == 0, ratios
+
+
+@pytest.mark.parametrize("M,K,N,groups,has_c", [(64, 65536, 4096, 8, 1), (1028, 65536, 4096, 64, 1), (1024, 65536, 4092, 64, 1), (1024, 0, 4096, 64, 1), (1 << 23, 4096, 256, 0, 1)])
+def test_what_the_sliced_kernel_does_not_take(plan, M, K, N, groups, has_c):
+    """no whole tile, rows that are not 16-byte aligned, rows that the caller did not tell, a wave's rows of D beyond 2 GiB"""
+    assert plan.amd_matmul_planned_sliced(M, K, N, groups, has_c, CUS) == 0
 
 
 def test_the_library_scratch_holds_every_split(plan):
