@@ -815,7 +815,7 @@ def main():
                 if tile_rows != 384:
                     four[cls] = kernel_of_class[cls].replace("288", str(tile_rows))
         for cls, M, N in (("gemm_nt_dw", H, D), ("gemm_dw13", D, 2 * H)):
-            if args.gemm_kernel == 384 or (args.gemm_kernel == 0 and mm.amd_matmul_planned_sliced(M, T * K, N, E, 1, 256)):
+            if mm.amd_matmul_planned_sliced(M, T * K, N, E, 1, 256):
                 four[cls] = _W4K % "true, 2"
         kernel_of_class.update(four)
     by_kernel = {}

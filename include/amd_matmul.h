@@ -46,12 +46,13 @@ int amd_matmul_no_alloc(Dataflow_Handle * dataflow_handle, int stream_id, int to
 						int M, int K, int N, float alpha, float beta, void * A, void * B, void * C, void * D);
 
 /* No counterpart in the reference (cuBLASLt picks its kernels by heuristic, matmul_helper.c:527-600): which persistent
- * kernel large problems without a C operand run on.
+ * kernel large problems run on, without a C operand or with two k-major operands.
  *   EIGHT_WAVES: two waves per SIMD, operands straight from global memory into one of two LDS stages, 256 x 256 tiles
  *     (256 x 288 over the token rows of a ragged-N launch).
  *   FOUR_WAVES_384: one wave per SIMD with the accumulators in the accumulation registers, 256 x 384 tiles (12 % fewer
  *     operand bytes per flop), every wave loading straight into the LDS and multiplying, its own token rows reloaded
- *     without the barrier.  Where both operands are k-major (ragged K, the weight gradients): 256 x 256 tiles, with C.
+ *     without the barrier.  Where both operands are k-major (ragged K, the weight gradients): 256 x 256 tiles, also with C,
+ *     from as many k-rows on as for AUTO; below, EIGHT_WAVES.
  *   FOUR_WAVES: one loading wave (operands through its registers) and three multiplying waves, 256 x 288 tiles.
  *   AUTO (the default): a ragged-N launch runs on the cheapest of the tilings of both (tiles of 384, 288, 224 or 192 token
  *     rows) for the group sizes that an even router gives: the number of tiles, in rounds over the compute units.
@@ -59,8 +60,8 @@ int amd_matmul_no_alloc(Dataflow_Handle * dataflow_handle, int stream_id, int to
  *     waves from 512 rows a group (ragged K, the rows of all groups given as K) or K = 256 to 512 on with C, from 640 or K = 1024 without, from 2048
  *     where one round of tiles is all (amd_matmul_planned_sliced of amd_matmul_plan.h).  Everything else runs EIGHT_WAVES.
  * The four-wave kernels are taken only where their limits hold (no C operand, N-side operand k-contiguous, K a multiple
- * of 128 and at most 2^21, M a multiple of 8, 16-byte aligned D; for two k-major operands M and N multiples of 8, C and D 16-byte
- * aligned), the eight-wave kernel elsewhere.  Results are
+ * of 128 and at most 2^21, M a multiple of 8 and at most 2^22, 16-byte aligned D; for two k-major operands M and N multiples of 8, M at most 2^22, N at
+ * most 2^24, C and D 16-byte aligned and the groups of D a multiple of 16 bytes apart), the eight-wave kernel elsewhere.  Results are
  * bit-identical whichever kernel runs.  The choice is process-wide; the environment variable AMD_MATMUL_KERNEL ("auto",
  * "8", "384" or "4") sets it when the matmul op is registered. */
 #define AMD_MATMUL_KERNEL_AUTO 0

@@ -27,7 +27,7 @@ int amd_matmul_planned_tilings(int M, int K, int N, int num_groups, int cu_count
 
 /* 1: two k-major operands, that is to_trans_a == 0 and to_trans_b == 1, run on the four-wave kernel that takes them in slices (FOUR_WAVES_384 of
  * amd_matmul.h), 0: on the eight-wave kernel or on a smaller tile.  num_groups: of a ragged-K launch, K then being the rows of all groups together; 0:
- * one problem, not split along K.  Aligned operands, C and D. */
+ * one problem, not split along K.  Aligned operands, C and D; a kernel named with amd_matmul_select_kernel counts. */
 int amd_matmul_planned_sliced(int M, int K, int N, int num_groups, int has_c, int cu_count);
 
 #ifdef __cplusplus

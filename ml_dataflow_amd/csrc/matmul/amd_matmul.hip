@@ -277,9 +277,8 @@ static int launch_w4k(const GemmParams & p, long tiles, long cu_count, hipStream
 	return check_launch();
 }
 
-/* Which persistent kernel large problems without a C operand run: AMD_MATMUL_KERNEL_EIGHT_WAVES or
- * AMD_MATMUL_KERNEL_FOUR_WAVES (amd_matmul.h).  Process-wide; amd_matmul_select_kernel changes it, the environment
- * variable AMD_MATMUL_KERNEL ("8" or "4") sets the initial value when the op is registered. */
+/* Which persistent kernel large problems run, one of AMD_MATMUL_KERNEL_* (amd_matmul.h).  Process-wide; amd_matmul_select_kernel changes it, the
+ * environment variable AMD_MATMUL_KERNEL ("auto", "8", "384" or "4") sets the initial value when the op is registered. */
 static int kernel_choice = AMD_MATMUL_KERNEL_DEFAULT;
 
 extern "C" int amd_matmul_select_kernel(int which) {
@@ -322,6 +321,18 @@ static bool w4k_pays(int mode, const GemmParams & p, long tiles, long cu_count) 
 		return (long) p.K >= (reads_c ? 512L : one_round ? 2048L : 640L) * p.num_groups;
 	}
 	return p.K >= (reads_c ? (one_round ? 256 : 512) : one_round ? 2048 : 1024);
+}
+
+/* whether two k-major operands on the 256 x 256 tile run on it: also where a caller named FOUR_WAVES_384, whose weight gradients of few rows ran
+ * on eight waves before there was another kernel for them (32 groups of 64 rows, 2048 x 1408 with C, 77 us, 89 on the sliced one) */
+static bool takes_sliced(int mode, const GemmParams & p, long tiles, long cu_count) {
+	return (kernel_choice == AMD_MATMUL_KERNEL_AUTO || kernel_choice == AMD_MATMUL_KERNEL_FOUR_WAVES_384) && w4k_ok(p) && w4k_pays(mode, p, tiles, cu_count);
+}
+
+/* a caller that named one of the persistent kernels gets it wherever it has enough tiles for half the compute units */
+static int tile_of_launch(int mode, const GemmParams & p, long grid_big, long cu_count) {
+	const bool named = kernel_choice != AMD_MATMUL_KERNEL_AUTO && p.M >= 256 && (mode == MODE_RAGGED_N ? (long) p.N / 256 * tiles_of(p.M, 256) : p.N >= 256 ? grid_big : 0) >= 128;
+	return named ? TILE_BIG : choose_tile(mode, p, cu_count);
 }
 
 /* a ragged-N launch without C on one of its tilings; grid: an upper bound on the tiles */
@@ -485,7 +496,8 @@ extern "C" int amd_matmul_planned_sliced(int M, int K, int N, int num_groups, in
 	p.C = has_c ? (const bf16_t *) scratch_of_device : NULL;
 	p.beta = has_c ? 1.0f : 0.0f;
 	const int mode = num_groups ? MODE_RAGGED_K : MODE_SINGLE;
-	return choose_tile(mode, p, cu_count) == TILE_BIG && w4k_ok(p) && w4k_pays(mode, p, tiles_in_launch(TILE_BIG, mode, p), cu_count);
+	const long tiles = tiles_in_launch(TILE_BIG, mode, p);
+	return tile_of_launch(mode, p, tiles, cu_count) == TILE_BIG && takes_sliced(mode, p, tiles, cu_count);
 }
 
 static long round_up8(long v) { return (v + 7) & ~7L; }
@@ -505,9 +517,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 	if (grid_big <= 0 || grid_small <= 0) {
 		return 0;
 	}
-	/* a caller that named one of the persistent kernels gets it wherever it has enough tiles for half the compute units */
-	const bool named = kernel_choice != AMD_MATMUL_KERNEL_AUTO && p.M >= 256 && (MODE == MODE_RAGGED_N ? (long) p.N / 256 * tiles_of(p.M, 256) : p.N >= 256 ? grid_big : 0) >= 128;
-	const int tile = named ? TILE_BIG : choose_tile(MODE, p, cu_count);
+	const int tile = tile_of_launch(MODE, p, grid_big, cu_count);
 	const bool big = tile == TILE_BIG;
 	const bool four_ok = direct && big && !qk && w4_ok(p);
 	const bool wide_only = kernel_choice == AMD_MATMUL_KERNEL_FOUR_WAVES_384;
@@ -578,7 +588,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 		return launch_staged<SMALL_TILE, true, true, MODE_RAGGED_K>(p, round_up8(grid_small), stream);
 	}
 	if constexpr (MODE != MODE_RAGGED_N) {
-		if (pk && qk && direct && big && !p.gather && (wide_only || (either && w4k_pays(MODE, p, grid_big, cu_count))) && w4k_ok(p)) {
+		if (pk && qk && direct && big && !p.gather && takes_sliced(MODE, p, grid_big, cu_count)) {
 			return launch_w4k<MODE>(p, grid_big, cu_count, stream);
 		}
 	}

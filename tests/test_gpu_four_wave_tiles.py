@@ -21,8 +21,18 @@ GUARD = 4096            # elements behind D that have to stay as they are
 def select_kernel(backend):
     lib = C.CDLL(os.path.join(os.path.dirname(B.__file__), "lib", "libamd_matmul.so"))
     lib.amd_matmul_select_kernel.argtypes = [C.c_int]
+    lib.amd_matmul_planned_sliced.argtypes = [C.c_int] * 6
     yield lib.amd_matmul_select_kernel
     assert lib.amd_matmul_select_kernel(AUTO) == 0
+
+
+def runs_sliced(select_kernel, kernel, M, K, N, groups, has_c):
+    """what the library says of a launch (amd_matmul_plan.h): a comparison of the eight-wave kernel with itself shows nothing"""
+    lib = C.CDLL(os.path.join(os.path.dirname(B.__file__), "lib", "libamd_matmul.so"))
+    assert select_kernel(kernel) == 0
+    sliced = lib.amd_matmul_planned_sliced(M, K, N, groups, int(has_c), 256)
+    assert select_kernel(AUTO) == 0
+    return sliced == 1
 
 
 def both(be, select_kernel, other, elements, start, submit):
@@ -71,21 +81,25 @@ def test_ragged_k_tiles_and_slices(backend, select_kernel, alpha, beta, M, N, gr
     counts = rng.choice([0, 1, 31, 32, 33, 128, 159, 160, 161, 255, 256, 257, 352, 353, 500], size=groups).astype(np.int32)
     counts[0], counts[-1] = 353, 1
     total = int(counts.sum())
+    rows = 2048 * groups                                               # what K says decides on the kernel only: here, that it is the sliced one
+    assert runs_sliced(select_kernel, FOUR_384, M, rows, N, groups, beta)
     print("case four waves, K: alpha=%g beta=%g M=%d N=%d G=%d rows=%d" % (alpha, beta, M, N, groups, total), flush=True)
     d_A, d_B = be.upload(normal_bf16(rng, (total, M), 0.05)), be.upload(normal_bf16(rng, (total, N)))
     d_cum = be.upload(np.cumsum(counts).astype(np.int32))
     start = normal_bf16(rng, (groups, N, M))
     both(be, select_kernel, FOUR_384, groups * N * M, start, lambda d_D: be.lib.dataflow_submit_amd_grouped_matmul(
-        be.hp, CS, BF, BF, BF if beta else B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 0, 1, B.AMD_GROUPED_RAGGED_K, M, 0, N, groups, d_cum.ptr, alpha, beta,
+        be.hp, CS, BF, BF, BF if beta else B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 0, 1, B.AMD_GROUPED_RAGGED_K, M, rows, N, groups, d_cum.ptr, alpha, beta,
         d_A.ptr, 0, d_B.ptr, d_D.ptr if beta else None, d_D.ptr, N * M * 2))
     for d in (d_A, d_B, d_cum):
         d.free()
 
 
-@pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (1.0, 1.0), (0.5, -2.0)])
-@pytest.mark.parametrize("M,N,K", [(4104, 4008, 161), (2816, 4096, 1000), (4096, 4096, 256)])
+@pytest.mark.parametrize("alpha,beta,M,N,K", [(1.0, 0.0, 4104, 4008, 1057), (1.0, 1.0, 4104, 4008, 545), (0.5, -2.0, 4104, 4008, 545),
+                                              (1.0, 0.0, 2816, 4096, 2056), (1.0, 1.0, 2816, 4096, 1000), (0.5, -2.0, 2816, 4096, 1000),
+                                              (1.0, 0.0, 4096, 4096, 2048), (1.0, 1.0, 4096, 4096, 256), (0.5, -2.0, 4096, 4096, 256)])
 def test_k_major_operands_of_one_problem(backend, select_kernel, alpha, beta, M, N, K):
     """one or two tiles a work-group, partial ones in both directions, a last slice of one k-row, of eight, and a whole one"""
+    assert runs_sliced(select_kernel, FOUR_384, M, K, N, 0, beta)
     be = backend
     rng = np.random.default_rng(M + N + K)
     print("case four waves, k-major: alpha=%g beta=%g M=%d N=%d K=%d" % (alpha, beta, M, N, K), flush=True)

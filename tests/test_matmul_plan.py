@@ -152,6 +152,17 @@ def test_what_the_sliced_kernel_does_not_take(plan, M, K, N, groups, has_c):
     assert plan.amd_matmul_planned_sliced(M, K, N, groups, has_c, CUS) == 0
 
 
+def test_a_named_kernel_does_not_bring_the_sliced_one_for_few_rows(plan):
+    few, many = (2048, 64 * 32, 1408, 32, 1, CUS), (2048, 640 * 32, 1408, 32, 1, CUS)
+    try:
+        for kernel, expected in ((384, 1), (8, 0), (4, 0), (0, 1)):
+            assert plan.amd_matmul_select_kernel(kernel) == 0
+            assert plan.amd_matmul_planned_sliced(*many) == expected
+            assert plan.amd_matmul_planned_sliced(*few) == 0
+    finally:
+        assert plan.amd_matmul_select_kernel(0) == 0
+
+
 def test_the_library_scratch_holds_every_split(plan):
     """amd_matmul_no_alloc leaves the op's bits because no split needs more than its 64 MiB: the plan is the same with any larger
     workspace."""
