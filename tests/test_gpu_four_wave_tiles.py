@@ -50,11 +50,12 @@ def both(be, select_kernel, other, elements, start, submit):
     assert (got[other][elements:] == 0x4242).all()
     bad = got[other] != got[EIGHT]
     assert not bad.any(), "%d of %d elements differ, first at %s" % (int(bad.sum()), bad.size, np.flatnonzero(bad)[:4].tolist())
+    return got[other][:elements]
 
 
 @pytest.mark.parametrize("transa", [1, 0])
 @pytest.mark.parametrize("alpha", [1.0, -0.75])
-@pytest.mark.parametrize("M,K,groups", [(1304, 128, 70), (264, 384, 64), (2048, 256, 130)])
+@pytest.mark.parametrize("M,K,groups", [(1304, 128, 70), (520, 384, 64), (2048, 256, 130)])
 def test_ragged_n_many_groups(backend, select_kernel, transa, alpha, M, K, groups):
     """more groups than lanes, and as many; tiles partial in both directions; a work-group walks over many short tiles"""
     be = backend
@@ -62,6 +63,7 @@ def test_ragged_n_many_groups(backend, select_kernel, transa, alpha, M, K, group
     counts = rng.choice([0, 1, 95, 96, 97, 191, 193, 288, 383, 384, 385, 500], size=groups).astype(np.int32)
     counts[0], counts[-1] = 385, 97
     total = int(counts.sum())
+    assert total // 256 * -(-M // 256) >= 128                          # from there on a named kernel runs, not the direct one on both sides
     print("case four waves, N: ta=%d alpha=%g M=%d K=%d G=%d rows=%d" % (transa, alpha, M, K, groups, total), flush=True)
     d_W = be.upload(normal_bf16(rng, (groups, M, K) if transa else (groups, K, M), 0.05))
     d_X, d_cum = be.upload(normal_bf16(rng, (total, K))), be.upload(np.cumsum(counts).astype(np.int32))
@@ -109,3 +111,34 @@ def test_k_major_operands_of_one_problem(backend, select_kernel, alpha, beta, M,
         d_A.ptr, d_B.ptr, d_D.ptr if beta else None, d_D.ptr, 1 << 20, d_ws.ptr))
     for d in (d_A, d_B, d_ws):
         d.free()
+
+
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+def test_ragged_k_by_default_with_c_apart_and_gaps_between_groups(backend, select_kernel, beta):
+    """the caller's count of rows as K, no kernel named; C in an array of its own, which stays as it is; groups of D further apart than they are long"""
+    be = backend
+    M = N = 1016
+    groups, gap = 32, 72
+    rng = np.random.default_rng(5)
+    counts = rng.choice([0, 1, 33, 352, 640, 700, 760, 1200], size=groups).astype(np.int32)
+    counts[3], counts[-1] = 3500, 6000
+    total = int(counts.sum())
+    assert runs_sliced(select_kernel, AUTO, M, total, N, groups, beta)
+    print("case four waves, K by default: beta=%g rows=%d" % (beta, total), flush=True)
+    stride = N * M + gap
+    d_A, d_B = be.upload(normal_bf16(rng, (total, M), 0.05)), be.upload(normal_bf16(rng, (total, N)))
+    d_cum = be.upload(np.cumsum(counts).astype(np.int32))
+    c = normal_bf16(rng, (groups * stride,))
+    d_C = be.upload(c)
+    start = np.full(groups * stride, 0x3131, np.uint16)
+
+    def submit(d_D):
+        return be.lib.dataflow_submit_amd_grouped_matmul(be.hp, CS, BF, BF, BF if beta else B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 0, 1, B.AMD_GROUPED_RAGGED_K, M, total, N, groups,
+                                                         d_cum.ptr, 1.0, beta, d_A.ptr, 0, d_B.ptr, d_C.ptr if beta else None, d_D.ptr, stride * 2)
+    d = both(be, select_kernel, AUTO, groups * stride, start, submit).reshape(groups, stride)
+    assert (d[:, N * M:] == 0x3131).all()
+    untouched = (counts == 0) & (beta != 0.0)
+    assert (d[untouched] == 0x3131).all() and (d[~untouched, :N * M] != 0x3131).any(axis=1).all()
+    assert (be.read(d_C.ptr, (groups * stride,), np.uint16) == c).all()
+    for buffer in (d_A, d_B, d_C, d_cum):
+        buffer.free()
