@@ -25,6 +25,9 @@ int amd_matmul_planned_splits(int to_trans_a, int to_trans_b, int M, int K, int 
 enum { AMD_MATMUL_ROWS_288 = 1, AMD_MATMUL_ROWS_384 = 2, AMD_MATMUL_ROWS_224 = 4, AMD_MATMUL_ROWS_192 = 8 };
 int amd_matmul_planned_tilings(int M, int K, int N, int num_groups, int cu_count);
 
+/* 1: one problem without C and with to_trans_b == 0, not split along K, runs on tiles of 256 x 384, 0: on 256 x 256 or a smaller tile */
+int amd_matmul_planned_wide(int M, int K, int N, int cu_count);
+
 /* 1: two k-major operands, that is to_trans_a == 0 and to_trans_b == 1, run on the four-wave kernel that takes them in slices (FOUR_WAVES_384 of
  * amd_matmul.h), 0: on the eight-wave kernel or on a smaller tile.  num_groups: of a ragged-K launch, K then being the rows of all groups together; 0:
  * one problem, not split along K.  Aligned operands, C and D; a kernel named with amd_matmul_select_kernel counts. */

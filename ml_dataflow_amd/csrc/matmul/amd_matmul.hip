@@ -329,6 +329,20 @@ static bool takes_sliced(int mode, const GemmParams & p, long tiles, long cu_cou
 	return (kernel_choice == AMD_MATMUL_KERNEL_AUTO || kernel_choice == AMD_MATMUL_KERNEL_FOUR_WAVES_384) && w4k_ok(p) && w4k_pays(mode, p, tiles, cu_count);
 }
 
+/* A single problem without C, whose tiles are known here: `wide` tiles of 256 x 384 against `narrow` ones of 256 x 256 on the eight-wave kernel.  A
+ * round costs the bytes of its k-tiles and a part of its own, a last round that is not full, as fewer work-groups share the card's power and
+ * memory, a half (wide: seven tenths) and the rest by its share.  Over 260 problems beside the 170 of the fit, M 512-8192, K 128-4096, N 1024-32768,
+ * half of them such that the prices disagree, the choice is 0.1 % behind the better one, at worst 3.6 %.  Whole rounds at the prices of
+ * the ragged launches were 1.6 % behind (3200 x 3456 x 22783, 3.05 rounds of 384: 5 % slower on them; K 128 in less than a round: 16 % faster), at those
+ * prices before the epilogue was generated 1.3 %. */
+static bool single_wide_is_cheaper(long wide, long narrow, long k_tiles, long cu_count) {
+	const long groups = (cu_count & ~7L) < 8 ? 8 : cu_count & ~7L;
+	const long wide_left = wide % groups, narrow_left = narrow % groups;
+	const long wide_rounds = wide / groups * 10 * groups + (wide_left ? 7 * groups + 3 * wide_left : 0);
+	const long narrow_rounds = narrow / groups * 10 * groups + (narrow_left ? 5 * groups + 5 * narrow_left : 0);
+	return wide_rounds * (256 + 384) * (105 * k_tiles + 250) < narrow_rounds * (256 + 256) * (100 * k_tiles + 150);
+}
+
 /* a caller that named one of the persistent kernels gets it wherever it has enough tiles for half the compute units */
 static int tile_of_launch(int mode, const GemmParams & p, long grid_big, long cu_count) {
 	const bool named = kernel_choice != AMD_MATMUL_KERNEL_AUTO && p.M >= 256 && (mode == MODE_RAGGED_N ? (long) p.N / 256 * tiles_of(p.M, 256) : p.N >= 256 ? grid_big : 0) >= 128;
@@ -488,6 +502,14 @@ extern "C" int amd_matmul_planned_tilings(int M, int K, int N, int num_groups, i
 	return ragged_n_tilings(p, cu_count, w4_ok(p));
 }
 
+extern "C" int amd_matmul_planned_wide(int M, int K, int N, int cu_count) {
+	GemmParams p;
+	memset(&p, 0, sizeof(p));
+	p.M = M; p.K = K; p.N = N;
+	return choose_tile(MODE_SINGLE, p, cu_count) == TILE_BIG && w4_ok(p)
+		&& single_wide_is_cheaper(tiles_of(M, 256) * tiles_of(N, 384), tiles_in_launch(TILE_BIG, MODE_SINGLE, p), tiles_of(K, BK), cu_count);
+}
+
 extern "C" int amd_matmul_planned_sliced(int M, int K, int N, int num_groups, int has_c, int cu_count) {
 	GemmParams p;
 	memset(&p, 0, sizeof(p));
@@ -526,14 +548,8 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 		return launch_ragged_n(1 << RAGGED_N_384, p, pk, grid_wide, cu_count, stream);
 	}
 	if (MODE == MODE_SINGLE && four_ok && p.split_k <= 1 && (wide_only || either)) {
-		/* a single problem's tiles are known here: the same rule as for the ragged launches, against the 256 x 256 tiles
-		 * the eight-wave kernel walks a single problem in */
 		const long tiles = tiles_of(p.M, 256) * tiles_of(p.N, 384);
-		long groups = cu_count & ~7L;
-		groups = groups < 8 ? 8 : groups;
-		const long wide = tiles_of(tiles, groups), narrow = tiles_of(grid_big, groups);
-		const long k_tiles = tiles_of(p.K, BK);
-		if (wide_only || wide * (256 + 384) * (95 * k_tiles + 210) < narrow * (256 + 256) * 100 * k_tiles) {
+		if (wide_only || single_wide_is_cheaper(tiles, grid_big, tiles_of(p.K, BK), cu_count)) {
 			if (pk) { return launch_w4d<true, MODE_SINGLE>(p, tiles, cu_count, stream); }
 			return launch_w4d<false, MODE_SINGLE>(p, tiles, cu_count, stream);
 		}

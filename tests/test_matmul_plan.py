@@ -19,6 +19,7 @@ def plan():
     lib = C.CDLL(os.path.join(B.LIB_DIR, "libamd_matmul.so"))
     lib.amd_matmul_planned_tile.argtypes = [C.c_int] * 5
     lib.amd_matmul_planned_tilings.argtypes = [C.c_int] * 5
+    lib.amd_matmul_planned_wide.argtypes = [C.c_int] * 4
     lib.amd_matmul_planned_sliced.argtypes = [C.c_int] * 6
     lib.amd_matmul_planned_splits.argtypes = [C.c_int] * 6 + [C.c_uint64, C.c_int]
     return lib
@@ -98,6 +99,38 @@ def test_no_second_tiling_beside_384_where_uneven_rows_run_best_on_it(plan, M, K
     """one price for both sides of a comparison: the 384 tiling is not chosen at one and then found too dear at another"""
     assert us[1] < us[0]
     assert plan.amd_matmul_planned_tilings(M, K, rows, groups, CUS) == 2
+
+
+# M, K, N, microseconds on tiles of 256 x 256 and of 256 x 384
+MEASURED_WIDE = [
+    (2432, 384, 18396, 39.0, 40.4),
+    (3840, 128, 5274, 16.2, 13.6),
+    (4992, 1920, 10936, 179.6, 185.8),
+    (3264, 1920, 19539, 190.8, 185.6),
+    (7552, 1536, 7035, 144.2, 147.9),
+    (3328, 1280, 17198, 126.6, 129.9),
+    (2240, 1920, 23712, 179.6, 185.4),
+    (1024, 128, 22846, 16.5, 15.1),
+    (3712, 128, 6084, 16.0, 14.1),
+    (2880, 1408, 19412, 136.5, 141.2),
+    (1088, 128, 16353, 15.7, 13.4),
+    (5376, 896, 28840, 245.6, 236.8),
+    (3072, 2816, 24654, 341.1, 352.4),
+    (2944, 3328, 24894, 385.8, 396.9),
+    (2304, 1664, 23957, 155.3, 159.3),
+    (3968, 384, 11021, 38.1, 39.2),
+    (4224, 3200, 2048, 62.7, 85.6),
+    (3264, 768, 26466, 121.3, 117.6),
+    (3264, 768, 5203, 39.5, 28.1),
+    (2752, 128, 4469, 10.0, 13.6),
+]
+
+
+@pytest.mark.parametrize("M,K,N,narrow,wide", MEASURED_WIDE)
+def test_single_problem_runs_on_the_better_width(plan, M, K, N, narrow, wide):
+    chosen = wide if plan.amd_matmul_planned_wide(M, K, N, CUS) else narrow
+    assert chosen <= 1.04 * min(narrow, wide)                          # what the rule leaves on the table: 3.6 % at most over 260 problems, near K = 384
+    assert plan.amd_matmul_planned_wide(M, K + 64, N, CUS) == 0        # whole pairs of k-tiles only
 
 
 # M, K (ragged: rows of all groups), N, groups (0: one problem), C, microseconds on eight waves and on the sliced kernel: even rows, rows of a Zipf router
