@@ -1,0 +1,200 @@
+"""The generated statements of the four-wave kernels that load straight into the LDS (gen_w4_loop.py, classes Wide and Ring), executed: scalar
+registers, branches, the queue of memory operations that s_waitcnt vmcnt counts.  A work-group's tiles one behind the other, as the kernels give them."""
+import os
+import re
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+MASK = 0xFFFFFFFF
+P_BYTES, Q_BYTES = 0x1000, 0x2000                # of a slice or k-tile of either operand
+CHUNK = 1024
+
+
+@pytest.fixture(scope="module")
+def macros(tmp_path_factory):
+    out = tmp_path_factory.mktemp("loop") / "loop.inc"
+    env = {k: v for k, v in os.environ.items() if k != "W4_OPTS"}
+    subprocess.run([sys.executable, os.path.join(ROOT, "ml_dataflow_amd", "csrc", "matmul", "gen_w4_loop.py"), str(out)], check=True, env=env, cwd=ROOT)
+    return dict(re.findall(r"#define (\w+)(.*?)(?=\n#define|\Z)", out.read_text(), re.S))
+
+
+def lines_of(macros, *names):
+    return [line for name in names for line in re.findall(r'"([^"]*?)\\n\\t"', macros[name])]
+
+
+class Machine:
+    """what one wave of the work-group does with a statement"""
+
+    def __init__(self, lines):
+        self.lines = lines
+        self.s = {"m0": 0}
+        self.queue = []                          # memory operations in flight, oldest first
+        self.loads = []                          # every load into the LDS: (operand, address, place in the LDS)
+        self.mfmas = self.from_zero = self.stores = self.barriers = 0
+        self.at_barrier = self.at_load = self.at_epilogue = lambda: None
+
+    def value(self, name):
+        return self.s[name] if re.fullmatch(r"s\d+|m0", name) else int(name, 0) & MASK
+
+    def target(self, at, label):
+        number, direction = label[:-1], label[-1]
+        places = range(at + 1, len(self.lines)) if direction == "f" else range(at - 1, -1, -1)
+        return next(i for i in places if self.lines[i] == number + ":")
+
+    def run(self):
+        at, scc, last_mfma = 0, 0, False
+        while at < len(self.lines):
+            op, _, rest = self.lines[at].partition(" ")
+            a = [x.strip() for x in rest.split(",")]
+            at += 1
+            if op == "s_mov_b32":
+                self.s[a[0]] = self.value(a[1])
+            elif op in ("s_add_u32", "s_addc_u32"):
+                total = self.value(a[1]) + self.value(a[2]) + (scc if op == "s_addc_u32" else 0)
+                self.s[a[0]], scc = total & MASK, int(total > MASK)
+            elif op in ("s_sub_u32", "s_subb_u32"):
+                total = self.value(a[1]) - self.value(a[2]) - (scc if op == "s_subb_u32" else 0)
+                self.s[a[0]], scc = total & MASK, int(total < 0)
+            elif op.startswith("s_cmp_"):
+                x, y = self.value(a[0]), self.value(a[1])
+                scc = int({"lg": x != y, "eq": x == y, "lt": x < y, "ge": x >= y}[op.split("_")[2]])
+            elif op == "s_cselect_b32":
+                self.s[a[0]] = self.value(a[1]) if scc else self.value(a[2])
+            elif op == "s_bitcmp1_b32":
+                scc = self.value(a[0]) >> int(a[1]) & 1
+            elif op in ("s_cbranch_scc0", "s_cbranch_scc1"):
+                if scc == int(op[-1]):
+                    at = self.target(at - 1, a[0])
+            elif op == "s_branch":
+                at = self.target(at - 1, a[0])
+            elif op == "s_barrier":
+                self.at_barrier()
+                self.barriers += 1
+            elif op == "s_waitcnt":
+                left = re.search(r"vmcnt\((\d+)\)", rest)
+                if left:
+                    assert int(left.group(1)) <= 63          # the field's width
+                    self.queue = self.queue[len(self.queue) - int(left.group(1)):] if len(self.queue) > int(left.group(1)) else self.queue
+            elif op == "buffer_load_dwordx4" and rest.endswith(" lds"):
+                operand, base = ("P", 64) if "s[64:67]" in rest else ("Q", 68)
+                self.loads.append((operand, self.s["s%d" % base] | self.s["s%d" % (base + 1)] << 32, self.s["m0"]))
+                self.queue.append(len(self.loads) - 1)
+                self.at_load()
+            elif op == "buffer_load_dwordx4":
+                assert "s[84:87]" in rest
+                self.queue.append("C")
+            elif op == "buffer_store_dwordx4":
+                assert "s[92:95]" in rest
+                self.stores += 1
+                self.queue.append("D")
+            elif op.startswith("v_mfma"):
+                self.mfmas += 1
+                self.from_zero += a[-1] == "0"
+                last_mfma = True
+            elif op.startswith("v_accvgpr_read") and last_mfma:
+                self.at_epilogue()
+                last_mfma = False
+            else:
+                assert op[0] == "v" or op.startswith("ds_read") or op == "s_nop" or op[:-1].isdigit(), op
+
+
+def cursor(tile, at):
+    """both operands of tile `tile` at slice or k-tile `at`, none of a tile that does not exist"""
+    if tile is None:
+        return [0] * 8
+    p, q = (tile + 1 << 32) + at * P_BYTES, (tile + 1 << 36) + at * Q_BYTES
+    return [p & MASK, p >> 32, 0, 1, q & MASK, q >> 32, 0, 1]
+
+
+def give(machine, first_register, values):
+    for n, v in enumerate(values):
+        machine.s["s%d" % (first_register + n)] = v
+
+
+@pytest.mark.parametrize("scaled", [0, 4])
+@pytest.mark.parametrize("name,least", [("W4K_C", 8), ("W4K_NOC", 5)])
+def test_sliced_kernel_waits_for_what_it_reads(macros, name, least, scaled):
+    slot_bytes, slots, per_slice = 32768, 5, 8
+    tiles = [least, least + 1, least + 2, least, 11, 12, 40, least, 9, 23]
+    start = [sum(tiles[:t]) for t in range(len(tiles))]                    # the stream's slice that the tile begins with
+    m = Machine(lines_of(macros, name + "_ASM"))
+
+    def slices_there():
+        """slices whose loads have all arrived, this wave's"""
+        waiting = [x for x in m.queue if isinstance(x, int)]
+        return (waiting[0] if waiting else len(m.loads)) // per_slice
+
+    def at_barrier():
+        if m.barriers == 0:
+            assert slices_there() == slots                                 # the first tile's first loads
+        else:
+            assert slices_there() > m.barriers, (name, m.barriers)         # barrier b lets all waves at slice b of the stream
+
+    def at_load():
+        operand, address, place = m.loads[-1]
+        g, u = divmod(len(m.loads) - 1, per_slice)
+        assert g < slots or m.barriers > g - slots + 1                     # every wave is done with the slice whose slot it takes
+        assert place == 4096 * 2 + g % slots * slot_bytes + u % 4 * CHUNK + (16384 if u >= 4 else 0)
+        tile = max(t for t in range(len(tiles)) if start[t] <= g)
+        if g - start[tile] < tiles[tile]:
+            assert (operand, address) == (("P", (tile + 1 << 32) + (g - start[tile]) * P_BYTES), ("Q", (tile + 1 << 36) + (g - start[tile]) * Q_BYTES))[u // 4]
+
+    def at_epilogue():
+        assert "C" not in m.queue
+
+    m.at_barrier, m.at_load, m.at_epilogue = at_barrier, at_load, at_epilogue
+    for t, slices in enumerate(tiles):
+        before = m.mfmas, m.from_zero, m.stores, m.barriers, len(m.loads)
+        give(m, 32, [7, 0, 1 << 20, 512, 9, 0, 0x3f800000, 0x3f800000])
+        give(m, 40, cursor(t, 0) if t == 0 else cursor(t if slices > slots else None, slots))
+        give(m, 48, cursor(t + 1 if t + 1 < len(tiles) else None, 0))
+        give(m, 56, [slices, (t == 0) | scaled, P_BYTES, Q_BYTES, start[t] % slots * slot_bytes, 0, 16384, 4096 * 2])
+        m.run()
+        assert m.mfmas - before[0] == 64 * slices and m.from_zero - before[1] == 64
+        assert m.stores - before[2] == 32
+        assert m.barriers - before[3] == slices + (t == 0)
+        assert len(m.loads) - before[4] == per_slice * (slices + (slots if t == 0 else 0))
+
+
+@pytest.mark.parametrize("scaled", [0, 4])
+@pytest.mark.parametrize("name", ["W4D_PKC_PACKED", "W4D_PKC_GATHER", "W4D_PKM_PACKED", "W4D_PKM_GATHER"])
+def test_wide_kernel_waits_for_what_it_reads(macros, name, scaled):
+    stage_p, stage_q, place_p, place_q, of_p, of_q = 32768, 49152, 8 * CHUNK, 65536 + 12 * CHUNK, 8, 12
+    tiles = [2, 4, 2, 2, 6, 16, 2, 10]
+    start = [sum(tiles[:t]) for t in range(len(tiles))]
+    m = Machine(lines_of(macros, name + "_HEAD", name + "_ASM", name + "_END"))
+
+    def k_tiles(operand, of):
+        mine = [n for n, load in enumerate(m.loads) if load[0] == operand]
+        waiting = {x for x in m.queue if isinstance(x, int)}
+        return next((n for n, load in enumerate(mine) if load in waiting), len(mine)) // of
+
+    def at_barrier():
+        there = min(k_tiles("P", of_p), k_tiles("Q", of_q))
+        assert there >= 1 if m.barriers == 0 else there > m.barriers, (name, m.barriers)
+
+    def at_load():
+        operand, address, place = m.loads[-1]
+        g, u = divmod(sum(load[0] == operand for load in m.loads) - 1, of_p if operand == "P" else of_q)
+        assert place == (place_p + g % 2 * stage_p if operand == "P" else place_q + g % 2 * stage_q) + u * CHUNK
+        if operand == "P":
+            assert g < 2 or m.barriers > g - 1                             # P is shared: every wave is done with the k-tile whose stage it takes
+        tile = max(t for t in range(len(tiles)) if start[t] <= g)
+        if g - start[tile] < tiles[tile]:
+            assert address == ((tile + 1 << 32) + (g - start[tile]) * P_BYTES if operand == "P" else (tile + 1 << 36) + (g - start[tile]) * Q_BYTES)
+
+    m.at_barrier, m.at_load = at_barrier, at_load
+    for t, count in enumerate(tiles):
+        before = m.mfmas, m.from_zero, m.stores, m.barriers, len(m.loads)
+        give(m, 32, [7, 0, 1 << 20, 512, 0, 0, 0x3f800000, 0])
+        give(m, 40, cursor(t, 0))
+        give(m, 48, cursor(t + 1 if t + 1 < len(tiles) else None, 0))
+        give(m, 56, [count, (t == 0) | scaled, P_BYTES, Q_BYTES, 0, place_p, place_q, 65536])
+        m.run()
+        assert m.mfmas - before[0] == 192 * count and m.from_zero - before[1] == 96
+        assert m.stores - before[2] == 48
+        assert m.barriers - before[3] == count + (t == 0)
+        assert len(m.loads) - before[4] == (of_p + of_q) * (count + (2 if t == 0 else 0))

@@ -35,8 +35,9 @@ def test_generated_k_loop_defines_what_the_kernel_uses_and_is_reproducible(tmp_p
     text = run_generator(tmp_path)
     assert text == run_generator(tmp_path)                                     # no dependence on time, hashing order or the environment
     kernel = open(os.path.join(ROOT, "ml_dataflow_amd", "csrc", "matmul", "gemm_w4_kernel.h")).read()
-    used = set(re.findall(r"\bW4D?_(?:MULT|LOAD|M|PKC|PKM|OUTPUTS|INPUTS|VP|VQ)_?[A-Z0-9_]*\b", kernel))
-    defined = set(re.findall(r"#define (W4D?_[A-Z0-9_]+)", text))
+    used = set(re.findall(r"\bW4[DK]?_(?:MULT|LOAD|M|PKC|PKM|C|NOC|OUTPUTS|INPUTS|VP|VQ)_?[A-Z0-9_]*\b", kernel))
+    defined = set(re.findall(r"#define (W4[DK]?_[A-Z0-9_]+)", text))
+    assert {"W4D_PKM_GATHER_END", "W4K_C_ASM", "W4K_NOC_LEAST"} <= used
     assert used and used <= defined, sorted(used - defined)
     # per k-tile of a multiplying wave: 16 x 6 accumulator groups, two k-steps -> 192 MFMAs in each of its two loop bodies' steps
     for name in ("W4_MULT_PKC_ASM", "W4_MULT_PKM_ASM"):
