@@ -197,18 +197,18 @@ def replay_step_with_events(be, layer, T, d_X, d_out, d_dY, d_dX, d_bias, backwa
 # HBM bytes per launch (average over the launches of a class) from two hardware counter runs of this script with
 # --calibration-copy (rocprofv3 --pmc FETCH_SIZE, then WRITE_SIZE), each scaled by what the counter reads for the
 # calibration copy of known size (fetch x1.985, write x1.000).  Only valid for the workload and the schedule (fused) they were taken on.
-# The weight gradients (gemm_nt_dw, gemm_dw13) have no entry: the counters were taken on the kernel they ran on before.
+# Taken on gemm_bf16_w4k_kernel for the weight gradients and gemm_bf16_w4d_kernel for the other grouped GEMMs.
 TRAFFIC_SOURCE = ("profiles/moe_layer_%s_hbm_traffic.md: hardware counters of two separate runs of this script, not of this run")
 MEASURED_TRAFFIC_BYTES = {
     "config4_fwdbwd_8192x4096_e64k8_h1024": {
-        "gemm_up13": 2589760385, "gemm_tn": 1458409166, "gemm_nn": 1540948489, "gemm_dx13": 2281766452,
-        "dispatch_scaled": 605606034, "swiglu": 400721551, "swiglu_bwd_x_routed": 822827377, "combine": 668834607,
-        "combine_grad": 601168066, "dispatch": 604555665,
+        "gemm_up13": 2161455558, "gemm_tn": 1371280124, "gemm_nn": 1535730842, "gemm_nt_dw": 1854822314, "gemm_dx13": 2206062164,
+        "gemm_dw13": 3748477803, "dispatch_scaled": 605606686, "swiglu": 400734208, "swiglu_bwd_x_routed": 822825787, "combine": 668830825,
+        "combine_grad": 601176532, "dispatch": 604556391,
     },
     "config5_fwdbwd_65536x4096_e64k8_h1024": {
-        "gemm_up13": 21330367076, "gemm_tn": 12462374745, "gemm_nn": 9885439367, "gemm_dx13": 33712088322,
-        "dispatch_scaled": 4844596105, "swiglu": 3205532585, "swiglu_bwd_x_routed": 6617731110, "combine": 5350080114,
-        "combine_grad": 4808782033, "dispatch": 4836259094,
+        "gemm_up13": 18470144588, "gemm_tn": 11482951390, "gemm_nn": 9339866922, "gemm_nt_dw": 16609306740, "gemm_dx13": 29595429204,
+        "gemm_dw13": 41511091429, "dispatch_scaled": 4844596061, "swiglu": 3205541793, "swiglu_bwd_x_routed": 6617716932, "combine": 5350069289,
+        "combine_grad": 4808784480, "dispatch": 4836258995,
     },
 }
 
@@ -754,7 +754,8 @@ def main():
         assert mm.amd_matmul_select_kernel(args.gemm_kernel) == 0
         gemm_kernel_ab = {"kernel": other, "ms_per_step_median": round(other_steps[len(other_steps) // 2], 4), "ms_per_step_min": round(other_steps[0], 4),
                           "gemm_avg_ms": {k: round(float(np.mean(v)), 4) for k, v in other_classes.items() if k.startswith("gemm")},
-                          "note": "ragged-N launches without a C operand only (up13, tn, nn, dx13); the weight-gradient launches run the eight-wave kernel either way"}
+                          "note": "kernel 8: every GEMM on the eight-wave kernel; kernel 4: the ragged-N launches without a C operand (up13, tn, nn, dx13) on the four-wave kernel with "
+                                  "a loading wave, the weight gradients on the eight-wave one"}
     # the first micro-batch of an accumulation: weight gradients written with beta = 0 and no C operand.  Reported beside the
     # accumulating steps above, which stay the headline (every later micro-batch, and every step of the reference, is one of those)
     first_mb = None
