@@ -632,9 +632,9 @@ def main():
                          "grouped: the reference's op sequence with grouped launches (10 expert GEMMs); per_expert: the reference's "
                          "own schedule (host sync after routing, one launch per expert and op)")
     ap.add_argument("--gemm-kernel", type=int, default=0, choices=[0, 8, 4, 384],
-                    help="persistent GEMM kernel of the large launches without a C operand (amd_matmul_select_kernel): 0 = the library's "
-                         "default (per launch, decided on the device from the group sizes: 8 or 384); 8 = eight waves, loads straight "
-                         "into the LDS, 256 x 288 tiles; 384 = four waves that all load and multiply, 256 x 384 tiles; 4 = one loading "
+                    help="persistent GEMM kernel of the large launches (amd_matmul_select_kernel): 0 = the library's default, per launch; 8 = eight waves, "
+                         "loads straight into the LDS; 384 = four waves that all load and multiply, 256 x 384 tiles without a C operand, 256 x 256 in "
+                         "slices for two k-major operands (the weight gradients) of enough rows; 4 = for launches without a C operand, one loading "
                          "wave and three multiplying waves.  Another one (4 beside 8, else 8) is timed after the step loop and "
                          "reported under gemm_kernel_ab")
     ap.add_argument("--no-cpu-baseline", action="store_true")

@@ -102,6 +102,8 @@ static long tiles_of(long extent, long tile) { return (extent + tile - 1) / tile
  * rounds: the router's input gradient, 2048 x 32 x 3001 with C, to 96 work-groups of 256 x 256 in 13.3 us, where pairs of 128 x 128 take 9.1
  * (4096 x 64 x 8192 31.4 and 27.5, 4096 x 64 x 65536 194 and 271, the other way round).  Over 544 products of 64-4096 columns,
  * 16-65536 tokens, K 8-16384 the choice is 0.8 % behind the best of all tiles, at a flat half a microsecond a round it was 3.5 %.
+ * BIG's cost and its read of C are those of the eight-wave kernel, also where the problem then runs on 256 x 384 tiles or on the sliced kernel, which
+ * reads C under the multiplies (3776 x 1000 x 4032 with C 38 us on eight waves, 34 on that one): there the choice leans to the smaller tiles.
  * Ragged launches have no term per tile: with caches that hold nothing of the operands the choice is 0.0 % behind the best of all
  * tiles over 60 ragged-K launches of 4-1500 rows per group, and 2.4 % over 120 ragged-N launches of 4-400. */
 enum { TILE_64x32 = AMD_MATMUL_TILE_64x32, TILE_64x64 = AMD_MATMUL_TILE_64x64, TILE_64x128 = AMD_MATMUL_TILE_64x128, TILE_128x128 = AMD_MATMUL_TILE_128x128,

@@ -300,7 +300,8 @@ __device__ __forceinline__ void tile_in_problem(int lid, int tiles_m, int tiles_
 struct KGroups { int end, order; };
 
 /* Groups whose tiles differ in their k-tiles go largest first.  uneven: the dearest tile costs half as much again as the mean one (in
- * k-tiles: its own, and RAGGED_K_EPILOGUE for its store, which takes 6 us of a work-group's share of the memory's rate) */
+ * k-tiles: its own, and RAGGED_K_EPILOGUE for its store, which takes 6 us of a work-group's share of the memory's rate on the eight-wave
+ * kernel; the sliced one hides a part of it, and goes by the same line) */
 #define RAGGED_K_EPILOGUE 6
 __device__ __forceinline__ KGroups k_groups(const GemmParams & p, int lane, bool & uneven) {
 	KGroups k;
