@@ -181,10 +181,22 @@ extern "C" int amd_matmul_planned_tile(int M, int K, int N, int has_c, int cu_co
 	return choose_tile(MODE_SINGLE, p, cu_count);
 }
 
+/* Few rows per group: a launch is bound by the weights of the groups that have any, and where these have one tile of rows each line of the
+ * weights is read by one work-group.  Such lines are loaded non-temporally: rows of 8 KiB, 128 bytes at a time, stream at 6.0-6.6 TB/s
+ * so and at 5.3 with plain loads (whole arrays in order: 7.1 and 6.25).  Forwards, us: 16 tokens, 64 experts, top 8, 4096 x 1024 258 -> 229; 50 tokens, 42 experts,
+ * 3584 x 1600 287 -> 253; 4 tokens, 43 experts, 1792 x 1216 61 -> 55.  A group with more tiles of rows keeps plain loads (712 tokens dealt to 35 experts by a Zipf
+ * router, non-temporal throughout: 104 -> 118), and so do launches whose weights are few enough to be found in the 256 MiB memory-side cache
+ * (7 tokens, 55 experts, top 2, 512 x 1472, over three sets of weights: 32.4 -> 33.7; over fourteen 37.8 -> 34.5). */
+#define STREAM_WEIGHTS_BYTES (48u << 20)
+static bool streams_weights(const GemmParams & p) {
+	return (uint64_t) (p.N < p.num_groups ? p.N : p.num_groups) * (uint64_t) p.M * (uint64_t) p.K * 2u > STREAM_WEIGHTS_BYTES;
+}
+
 /* the direct kernel on one of its tiles */
 template <bool PK, bool QK, int MODE, int GATHER = GATHER_NONE, bool SWIGLU = false>
-static int launch_direct(const GemmParams & p, int which, hipStream_t stream, int problems = 1) {
+static int launch_direct(GemmParams p, int which, hipStream_t stream, int problems = 1) {
 	const long grid = grid_of(which, MODE, p) * problems;
+	p.stream_weights = MODE == MODE_RAGGED_N && streams_weights(p);
 	switch (which) {
 		case TILE_64x32: return launch_direct_tile<64, 32, 2, 2, 4, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
 		case TILE_64x64: return launch_direct_tile<64, 64, 2, 2, 4, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);

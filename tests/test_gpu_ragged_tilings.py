@@ -96,3 +96,40 @@ def test_group_of_every_row_at_the_edges_of_the_scan(backend, G, kernel, M, K, r
     assert (be.read(d_D.ptr, (rows, M), np.uint16) == as_bf16(want)).all()
     for d in (d_W, d_X, d_cum, d_D):
         d.free()
+
+
+# rows of a group on both sides of one tile of 32, 64 and 128 rows, each mean on another of those tiles
+FEW_ROWS = {
+    "32": [0, 1, 31, 32, 33, 2, 16, 64, 65, 0, 30, 7, 32, 31, 5, 1],
+    "64": [63, 64, 65, 1, 0, 32, 33, 128, 129, 60, 64, 63, 40, 90, 50, 64],
+    "128": [127, 128, 129, 255, 256, 257, 0, 1, 100, 128, 127, 140, 90, 120, 128, 110],
+}
+
+
+@pytest.mark.parametrize("gathered", [False, True])
+@pytest.mark.parametrize("transa", [1, 0])
+@pytest.mark.parametrize("name", sorted(FEW_ROWS))
+def test_streamed_weights_bit_identical(backend, name, transa, gathered):
+    """16 groups with 64 MiB of weights: enough that those of groups with one tile of rows are loaded non-temporally; against one plain
+    matmul a group, which loads them as ever.  Every element is accumulated over k in the same order: bit for bit."""
+    be, M, K = backend, 2048, 1032
+    counts = np.array(FEW_ROWS[name], dtype=np.int32)
+    G, total, src_rows = len(counts), int(counts.sum()), 333
+    print("case streamed weights %s ta=%d gathered=%s rows=%d" % (name, transa, gathered, total), flush=True)
+    rng = np.random.default_rng(total + transa)
+    W, X, row_map = normal_bf16(rng, (G * M * K,), 0.05), normal_bf16(rng, (src_rows if gathered else total, K)), rng.integers(0, src_rows, size=total).astype(np.int32)
+    ends = np.cumsum(counts).astype(np.int32)
+    d_W, d_X, d_packed, d_cum, d_map = be.upload(W), be.upload(X), be.upload(np.ascontiguousarray(X[row_map]) if gathered else X), be.upload(ends), be.upload(row_map)
+    d_D, d_E = (be.upload(np.full((total, M), 0x4242, dtype=np.uint16)) for _ in range(2))
+    head = (be.hp, CS, BF, BF, B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, transa, 0, B.AMD_GROUPED_RAGGED_N, M, K, total, G, d_cum.ptr, 1.0, 0.0,
+            d_W.ptr, M * K * 2, d_X.ptr, None, d_D.ptr, 0)
+    assert (be.lib.dataflow_submit_amd_grouped_matmul_gathered(*head, d_map.ptr, src_rows) if gathered else be.lib.dataflow_submit_amd_grouped_matmul(*head)) == 0
+    for g in range(G):
+        first = int(ends[g] - counts[g])
+        assert be.lib.dataflow_submit_matmul(be.hp, CS, BF, BF, B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, transa, 0, M, K, int(counts[g]), 1.0, 0.0,
+                                             d_W.ptr + g * M * K * 2, d_packed.ptr + first * K * 2, None, d_E.ptr + first * M * 2, 0, None) == 0
+    be.sync(CS)
+    bad = be.read(d_D.ptr, (total, M), np.uint16) != be.read(d_E.ptr, (total, M), np.uint16)
+    assert not bad.any(), "%d of %d elements differ, first at %s" % (int(bad.sum()), bad.size, np.argwhere(bad)[:4].tolist())
+    for d in (d_W, d_X, d_packed, d_cum, d_map, d_D, d_E):
+        d.free()
