@@ -127,21 +127,21 @@ class Mult(Asm):
         dst = M_BF + s * 24 + j * 4
         self.lds("ds_read_b128 %s, v%d offset:%d" % (vr(dst, 4), M_BRD + s * 2 + stage, j * 2048), ("B", s, j))
 
-    def tail_reads(self, stage, which):
+    def tail_reads(self, stage, which, blocks=6):
         if which == 0:
             self.read_B(stage, 0, 0)
             self.read_A(stage, 0)
-            for j in range(1, 6):
+            for j in range(1, blocks):
                 self.read_B(stage, 0, j)
             self.read_A(stage, 1)
         else:
             self.read_A(stage, 1 + which)
 
-    def loop_head_state(self):
+    def loop_head_state(self, blocks=6):
         self.issued, self.known_done, self.prod = 0, -1, {}
         keep, self.L = self.L, []
         for which in range(3):
-            self.tail_reads(0, which)
+            self.tail_reads(0, which, blocks)
         self.L = keep
 
     def step(self, p):
@@ -298,6 +298,7 @@ class Loader(Asm):
 
 # ================================================================================================ four symmetric waves, 256 x 384
 QW_STAGE = 49152         # bytes of one Q stage of the wide tile (384 rows x 64 k)
+SHORT = (5, 4, 3, 2)     # column blocks of a wave in a tile of fewer rows
 D_VP, D_VQ, D_VQ_NEXT, D_AT = 208, 216, 228, 240              # this lane's offsets of the wave's 8 chunks of P, 12 of Q, the next tile's Q, of D
 
 
@@ -395,8 +396,11 @@ class Wide(Mult, Tail):
     (even), s57 bit 0: first tile of the work-group, s58 / s59 bytes per k-tile of P / Q, s60 LDS address of the stages,
     s61 / s62 of the wave's first chunk of P / Q in stage 0, s63 bytes from s60 to the wave's rows of Q.  Working registers as in the loader above.
 
+    Short tiles: a tile of at most 64 n rows, n one of SHORT, has bit 14 - n of s57 set, and wave w multiplies rows [16 n w, 16 n w + 16 n) of
+    it, n column blocks instead of six: the steps are the same with fewer multiplies.  Its loads of Q from the 2 n-th on carry offsets that read zeros.
+
     State from statement to statement: stage 0 holds k-tile 0 of the tile, visible to all waves; the rows of Q and P of k-tile 1 are
-    in flight into stage 1, and behind them the 48 stores of the tile before; the Q offsets of the tile are in v[D_VQ ...].  Epilogue as
+    in flight into stage 1, and behind them the 48 stores of the tile before; the Q offsets of the tile are in v[D_VQ ...], those of the next in v[D_VQ_NEXT ...].  Epilogue as
     in class Tail; s57 bit 2: alpha is not 1.  Three macros: what every tile starts with, the first tile's loads and the loop, the first two
     steps, which come in front of the loop but stand behind it, and the epilogue."""
 
@@ -443,7 +447,7 @@ class Wide(Mult, Tail):
             e("s_cmp_eq_u32 s77, s56")
             e("s_cbranch_scc0 5f")
             self.set_cursor(48, which)
-            if self.GATHER and which == 1:
+            if which == 1:
                 for q in range(12):
                     e("v_mov_b32 v%d, v%d" % (D_VQ + q, D_VQ_NEXT + q))
             e("s_branch 6f")
@@ -453,29 +457,34 @@ class Wide(Mult, Tail):
         else:
             self.advance(which)
 
-    def step(self, p, start=False):
+    def step(self, p, start=False, blocks=6):
+        """`blocks`: column blocks of a wave"""
         after = {}
 
         def at(m, fn):
             after.setdefault(m, []).append(fn)
 
-        pre, first, every, qfirst, qevery = OPTS["pre"], OPTS["first"], OPTS["every"], OPTS["qfirst"], OPTS["qevery"]
+        count, behind = 32 * blocks, 30 * blocks - 1         # MFMAs; the one behind which two of the four slots of P's fragments are free again
+        pre, first, every, qfirst, qevery = (OPTS[k] for k in ("pre", "first", "every", "qfirst", "qevery"))
+        if blocks < 6:                           # all twelve loads of Q go out (the next tile may have the rows), closer together
+            every, qfirst = min(every, blocks - 1), min(qfirst, 4 * blocks)
+            qevery = (behind - 1 - qfirst) // (self.LOADS_Q - 1)
         assert 1 <= pre <= 4 and first + every * (self.LOADS_P - pre - 1) < qfirst
-        assert qfirst >= 8 and qfirst + qevery * (self.LOADS_Q - 1) < 179
+        assert qfirst >= 8 and qfirst + qevery * (self.LOADS_Q - 1) < behind
         # the rest of the P rows of k-tile g + 1, into the other stage
         if not start:                        # of the first k-tile they are out in front of the epilogue
             for n, u in enumerate(range(pre, self.LOADS_P)):
                 at(first + every * n, lambda u=u: self.dma_p(1 - p, u))
         # the fragments of Q of k-step 1 first: with them in registers the wave's Q rows of this stage are free
-        for j in range(6):
+        for j in range(blocks):
             at(j, lambda j=j: self.read_B(p, 1, j))
         # this wave's Q rows of k-tile g + 2, into the stage being multiplied
-        at(qfirst, lambda: self.need(*[("B", 1, j) for j in range(6)]))
+        at(qfirst, lambda: self.need(*[("B", 1, j) for j in range(blocks)]))
         at(qfirst, lambda: self.move_on(1, p == 0))
         for q in range(self.LOADS_Q):
             at(qfirst + qevery * q, lambda q=q: self.dma_q(p, q))
         for a in range(4, 32):
-            at(6 * (a - 4) + 5, lambda a=a: self.read_A(p, a))
+            at(blocks * (a - 3) - 1, lambda a=a: self.read_A(p, a))
 
         def barrier():
             if start:                            # behind the first tile's loads, or the stores of the tile before
@@ -488,18 +497,18 @@ class Wide(Mult, Tail):
                 self.e("s_waitcnt vmcnt(%d)" % self.LOADS_Q)
             self.lds_drain()
             self.barrier()
-            self.tail_reads(1 - p, 0)
-        at(179, barrier)
-        at(180, lambda: self.move_on(0, p == 0))
+            self.tail_reads(1 - p, 0, blocks)
+        at(behind, barrier)
+        at(behind + 1, lambda: self.move_on(0, p == 0))
         for u in range(pre):
-            at(180 + 3 * u, lambda u=u: self.dma_p(p, u))
-        at(185, lambda: self.tail_reads(1 - p, 1))
-        at(191, lambda: self.tail_reads(1 - p, 2))
-        for m in range(192):
-            s, rem = divmod(m, 96)
-            i, j = divmod(rem, 6)
+            at(behind + 1 + blocks * u // 2, lambda u=u: self.dma_p(p, u))
+        at(behind + blocks, lambda: self.tail_reads(1 - p, 1))
+        at(behind + 2 * blocks, lambda: self.tail_reads(1 - p, 2))
+        for m in range(count):
+            s, rem = divmod(m, 16 * blocks)
+            i, j = divmod(rem, blocks)
             if i & 1:
-                j = 5 - j                        # one operand stays from each MFMA to the next: 0.8 % less time at the card's power limit
+                j = blocks - 1 - j               # one operand stays from each MFMA to the next: 0.8 % less time at the card's power limit
             a = s * 16 + i
             self.need(("A", a % 4), ("B", s, j))
             self.e("v_mfma_f32_16x16x32_bf16 %s, %s, %s, %s" % (self.acc(i, j), vr(M_AF + (a % 4) * 4, 4), vr(M_BF + s * 24 + j * 4, 4), "0" if start and s == 0 else self.acc(i, j)))
@@ -578,10 +587,24 @@ class Wide(Mult, Tail):
         self.advance(0)
         self.advance(1)
         e("4:")
+        for blocks in SHORT:
+            e("s_bitcmp1_b32 s57, %d" % (14 - blocks))
+            e("s_cbranch_scc1 %df" % (30 + blocks))
         for which in range(3):
             self.tail_reads(0, which)
         self.two_steps(True)                 # the first two k-tiles start the sums
         e("s_cbranch_scc1 3b")
+        e("s_branch 9f")
+        for blocks in SHORT:
+            e("%d:" % (30 + blocks))
+            for which in range(3):
+                self.tail_reads(0, which, blocks)
+            self.two_steps(True, blocks)
+            e("s_cbranch_scc0 9f")
+            e("%d:" % (40 + blocks))
+            self.two_steps(False, blocks)
+            e("s_cbranch_scc1 %db" % (40 + blocks))
+            e("s_branch 9f")
         e("9:")
         e("s_waitcnt lgkmcnt(0)")
         for u in range(OPTS["pre"], self.LOADS_P):
@@ -604,11 +627,11 @@ class Wide(Mult, Tail):
         self.parts.append(("%s_%s" % (self.name, name), self.L))
         self.L = []
 
-    def two_steps(self, start):
-        self.loop_head_state()
-        self.step(0, start)
-        self.loop_head_state()
-        self.step(1)
+    def two_steps(self, start, blocks=6):
+        self.loop_head_state(blocks)
+        self.step(0, start, blocks)
+        self.loop_head_state(blocks)
+        self.step(1, False, blocks)
         self.e("s_add_u32 s76, s76, 2")
         self.e("s_cmp_lt_u32 s76, s56")
 

@@ -198,3 +198,107 @@ def test_wide_kernel_waits_for_what_it_reads(macros, name, scaled):
         assert m.stores - before[2] == 48
         assert m.barriers - before[3] == count + (t == 0)
         assert len(m.loads) - before[4] == (of_p + of_q) * (count + (2 if t == 0 else 0))
+
+
+class Operands(Machine):
+    """... and the fragments of P and Q that its multiplies take: what each register holds, or has on the way from the LDS"""
+
+    class Lines(list):
+        """the statement, each line looked at as it is executed"""
+
+        def __getitem__(self, at):
+            line = list.__getitem__(self, at)
+            self.look(line)
+            return line
+
+    def __init__(self, lines):
+        super().__init__(self.Lines(lines))
+        self.lines.look = self.look
+        self.plain = lines
+        self.held, self.on_the_way, self.multiplied = {}, [], []
+
+    def target(self, at, label):
+        places = range(at + 1, len(self.plain)) if label[-1] == "f" else range(at - 1, -1, -1)
+        return next(i for i in places if self.plain[i] == label[:-1] + ":")
+
+    def look(self, line):
+        if line.startswith("ds_read"):
+            numbers = [int(x) for x in re.findall(r"\d+", line.split(" ", 1)[1])]
+            offset = numbers[-1] if "offset" in line else 0
+            self.on_the_way.append((list(range(numbers[0], numbers[1] + 1)), (numbers[2], offset)))
+            for r in self.on_the_way[-1][0]:
+                self.held[r] = None
+        elif "lgkmcnt" in line:
+            left = int(re.search(r"lgkmcnt\((\d+)\)", line).group(1))
+            while len(self.on_the_way) > left:
+                registers, what = self.on_the_way.pop(0)
+                for r in registers:
+                    self.held[r] = what
+        elif line.startswith("v_mfma"):
+            regs = re.findall(r"([av])\[(\d+):(\d+)\]", line)
+            first = lambda n: [self.held[r] for r in range(int(regs[n][1]), int(regs[n][2]) + 1)]
+            self.multiplied.append((regs[0][0] + regs[0][1], first(1), first(2)))
+
+
+@pytest.mark.parametrize("blocks", [6, 5, 4, 3, 2])
+@pytest.mark.parametrize("name", ["W4D_PKC_PACKED", "W4D_PKC_GATHER", "W4D_PKM_PACKED", "W4D_PKM_GATHER"])
+def test_wide_kernel_multiplies_short_tiles(macros, name, blocks):
+    """Tiles of `blocks` column blocks a wave among full ones: every multiply's operands, where the loads go and when."""
+    stage_p, stage_q, place_p, place_q, of_p, of_q = 32768, 49152, 8 * CHUNK, 65536 + 12 * CHUNK, 8, 12
+    tiles = [(2, 6), (4, blocks), (2, blocks), (6, 6), (2, blocks), (16, blocks), (8, 6), (4, blocks)]
+    start = [sum(n for n, _ in tiles[:t]) for t in range(len(tiles))]
+    m = Operands(lines_of(macros, name + "_HEAD", name + "_ASM", name + "_END"))
+    kmajor, M_ARD, M_BRD = "PKM" in name, 192, 200
+
+    def there(operand, of):
+        mine = [n for n, load in enumerate(m.loads) if load[0] == operand]
+        waiting = {x for x in m.queue if isinstance(x, int)}
+        return next((n for n, load in enumerate(mine) if load in waiting), len(mine)) // of
+
+    def at_barrier():
+        k = min(there("P", of_p), there("Q", of_q))
+        assert k >= 1 if m.barriers == 0 else k > m.barriers, (name, m.barriers)
+
+    def at_load():
+        operand, address, place = m.loads[-1]
+        g, u = divmod(sum(load[0] == operand for load in m.loads) - 1, of_p if operand == "P" else of_q)
+        assert place == (place_p + g % 2 * stage_p if operand == "P" else place_q + g % 2 * stage_q) + u * CHUNK
+        if operand == "P":
+            assert g < 2 or m.barriers > g - 1
+        else:
+            # the wave's own rows: every fragment of the k-tile whose stage this takes is in its registers
+            assert g < 2 or not [what for _, what in m.on_the_way if what[0] in (M_BRD + g % 2, M_BRD + 2 + g % 2) and m.barriers <= g - 1]
+        tile = max(t for t in range(len(tiles)) if start[t] <= g)
+        k = g - start[tile]
+        if k < tiles[tile][0]:
+            assert address == ((tile + 1 << 32) + k * P_BYTES if operand == "P" else (tile + 1 << 36) + k * Q_BYTES)
+
+    m.at_barrier, m.at_load = at_barrier, at_load
+    for t, (count, nb) in enumerate(tiles):
+        before = m.mfmas, m.from_zero, m.stores, m.barriers, len(m.loads)
+        m.multiplied = []
+        give(m, 32, [7, 0, 1 << 20, 512, 0, 0, 0x3f800000, 0])
+        give(m, 40, cursor(t, 0))
+        give(m, 48, cursor(t + 1 if t + 1 < len(tiles) else None, 0))
+        give(m, 56, [count, (t == 0) | (0 if nb == 6 else 1 << 14 - nb), P_BYTES, Q_BYTES, 0, place_p, place_q, 65536])
+        m.run()
+        assert m.mfmas - before[0] == 32 * nb * count and m.from_zero - before[1] == 16 * nb
+        assert m.stores - before[2] == 48
+        assert m.barriers - before[3] == count + (t == 0)
+        assert len(m.loads) - before[4] == (of_p + of_q) * (count + (2 if t == 0 else 0))
+        want = set()
+        for k in range(count):
+            stage = k & 1
+            for s in range(2):
+                for i in range(16):
+                    for j in range(nb):
+                        group, low = (i // 4) * 6 + j, (i % 4) * 4
+                        acc = "a%d" % (16 * group + low) if group < 16 else "v%d" % (16 * (group - 16) + low)
+                        if kmajor:
+                            at = stage * 32768 + s * 32 * 512 + (i // 8) * 256
+                            a = [(M_ARD + i % 8, at)] * 2 + [(M_ARD + i % 8, at + 4 * 512)] * 2
+                        else:
+                            a = [(M_ARD + s, stage * 32768 + i * 2048)] * 4
+                        want.add((k, acc, tuple(a), tuple([(M_BRD + 2 * s + stage, j * 2048)] * 4)))
+        got = {(n // (32 * nb), acc, tuple(a), tuple(b)) for n, (acc, a, b) in enumerate(m.multiplied)}
+        assert got == want and len(m.multiplied) == len(want)
