@@ -397,10 +397,11 @@ class Wide(Mult, Tail):
     s61 / s62 of the wave's first chunk of P / Q in stage 0, s63 bytes from s60 to the wave's rows of Q.  Working registers as in the loader above.
 
     Short tiles: a tile of at most 64 n rows, n one of SHORT, has bit 14 - n of s57 set, and wave w multiplies rows [16 n w, 16 n w + 16 n) of
-    it, n column blocks instead of six: the steps are the same with fewer multiplies.  Its loads of Q from the 2 n-th on carry offsets that read zeros.
+    it, n column blocks instead of six: the steps are the same with fewer multiplies.  Its loads of Q from the 2 n-th on read zeros.
 
     State from statement to statement: stage 0 holds k-tile 0 of the tile, visible to all waves; the rows of Q and P of k-tile 1 are
-    in flight into stage 1, and behind them the 48 stores of the tile before; the Q offsets of the tile are in v[D_VQ ...], those of the next in v[D_VQ_NEXT ...].  Epilogue as
+    in flight into stage 1, and behind them the 48 stores of the tile before; the Q offsets of the tile are in v[D_VQ ...], of
+    gathered rows those of the next in v[D_VQ_NEXT ...].  Epilogue as
     in class Tail; s57 bit 2: alpha is not 1.  Three macros: what every tile starts with, the first tile's loads and the loop, the first two
     steps, which come in front of the loop but stand behind it, and the epilogue."""
 
@@ -447,7 +448,7 @@ class Wide(Mult, Tail):
             e("s_cmp_eq_u32 s77, s56")
             e("s_cbranch_scc0 5f")
             self.set_cursor(48, which)
-            if which == 1:
+            if self.GATHER and which == 1:
                 for q in range(12):
                     e("v_mov_b32 v%d, v%d" % (D_VQ + q, D_VQ_NEXT + q))
             e("s_branch 6f")
