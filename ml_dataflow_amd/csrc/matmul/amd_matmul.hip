@@ -1390,7 +1390,12 @@ extern "C" int amd_route_tokens(Dataflow_Handle * dataflow_handle, int stream_id
 	 * Its one compute unit adds up the partial sums at 20-30 GB/s a wave: bounded, so that it stays below a launch. */
 	if (r.T <= ROUTE_SMALL_TOKENS && r.T * lanes <= ROUTE_SMALL_THREADS && (long) r.T * r.E * (r.splits > 1 ? r.splits : 1) <= ROUTE_SMALL_PARTIALS) {
 		int threads = (r.T * lanes + WAVE - 1) / WAVE * WAVE;
-		threads = threads < 256 ? 256 : threads;
+		/* The logits are added up by all its waves, four experts of a token each, before the selection's have work: a wave for every 64 of
+		 * those up to eight waves, and sixteen waves from 2048 on.  us, as many as the selection has and so: 32 tokens, 52 experts, top 2 8.1 and 7.0,
+		 * 68, 38 and 4 14.2 and 9.7, 256, 64 and 2 17.7 and 13.7; sixteen at 68 tokens 11.0. */
+		const long sums = r.T * tiles_of(r.E < ROUTE_CHUNK ? r.E : ROUTE_CHUNK, 4);
+		const long wanted = sums > 2048 ? ROUTE_SMALL_THREADS : sums > 512 ? 512 : sums < 256 ? 256 : tiles_of(sums, WAVE) * WAVE;
+		threads = threads < wanted ? (int) wanted : threads;
 		hipLaunchKernelGGL(route_small_kernel, dim3(1), dim3((unsigned int) threads), 0, stream, r, lanes);
 		return check_launch();
 	}

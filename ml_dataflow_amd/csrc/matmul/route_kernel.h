@@ -379,7 +379,7 @@ __global__ void __launch_bounds__(ROUTE_MAP_THREADS) route_map_kernel(RouteParam
 }
 
 /* Selection and permutation of few tokens in one work-group: T * lanes <= 1024, T <= 256.
- * Launch: grid = 1, block = T * lanes rounded up to whole waves, at least 256. */
+ * Launch: grid = 1, block = T * lanes rounded up to whole waves, or more waves where there are more sums to add up. */
 __global__ void __launch_bounds__(ROUTE_SMALL_THREADS) route_small_kernel(RouteParams p, int lanes) {
 	__shared__ uint32_t tile[ROUTE_SMALL_TOKENS * ROUTE_ROW_DWORDS];
 	__shared__ uint16_t ids[ROUTE_SMALL_THREADS];

@@ -152,3 +152,21 @@ def test_routing_writes_logits_at_any_element(backend):
     around = be.read(d_logits.ptr, (T * E + 8,), np.uint16)
     assert around[0] == 0x1234 and (around[T * E + 1:] == 0x1234).all()
     layer.free()
+
+
+@pytest.mark.parametrize("T,E,K", [(64, 16, 1), (65, 16, 1), (127, 16, 2), (128, 16, 2), (129, 16, 2), (68, 38, 4), (32, 52, 2), (255, 32, 2), (256, 32, 2),
+                                   (256, 33, 2), (256, 64, 2), (256, 100, 1)])
+def test_few_tokens_at_the_edges_of_the_waves_that_add_up(backend, T, E, K):
+    """256, 512 and 2048 quads of sums, where the single work-group gets more waves than its selection needs"""
+    print("case routing waves T=%d E=%d K=%d" % (T, E, K), flush=True)
+    be, D = backend, 512
+    rng = np.random.default_rng(T + E + K)
+    layer = MoeLayer(be, T, D, E, K, 256)
+    L = layer.L
+    X, Wr = normal_bf16(rng, (T, D)), normal_bf16(rng, (E, D), 0.02)
+    d_X, d_out = be.upload(X), be.alloc(T * D * 2)
+    be.write(L.w_router, Wr)
+    be.zero(L.w1, E * L.expert_stride_bytes)
+    compare(be, L, layer, T, E, K, D, d_X, d_out, None)
+    layer.free()
+    d_X.free(), d_out.free()
