@@ -36,9 +36,9 @@
  *                       and backward must both use this schedule or neither.  The stacked up-projection fetches the
  *                       rows of X through expert_mapping itself while X is below 4 GiB (no dispatch copy); with
  *                       AMD_MOE_NO_GATHER set in the environment it takes the copy + packed form that otherwise
- *                       only runs beyond that size.  The stacked dW1 | dW3 GEMM runs on a re-dispatched copy of X (the
- *                       faster form for a reduction over scattered rows); with AMD_MOE_BWD_GATHER set in the
- *                       environment it gathers the rows too.  Test hooks: every form gives the same bits.
+ *                       only runs beyond that size.  The stacked dW1 | dW3 GEMM gathers the rows of X too where that is the
+ *                       faster form (amd_moe_layer_backward_gathers), or everywhere with AMD_MOE_BWD_GATHER set in the
+ *                       environment, and runs on a re-dispatched copy of X otherwise.  Test hooks: every form gives the same bits.
  * All functions return 0 on success and -1 on error with a message on stderr.
  */
 #ifndef MOE_LAYER_H
@@ -141,6 +141,10 @@ int amd_moe_layer_forward(Dataflow_Handle * handle, int compute_stream_id, int s
  * compute stream first if the forward did not, because it reads host_expert_counts); the fused schedule only its own. */
 int amd_moe_layer_backward(Dataflow_Handle * handle, int compute_stream_id, int secondary_stream_id,
 						   Amd_Moe_Layer * layer, int num_tokens, void * X, void * dY, void * dX, int schedule);
+
+/* 1: the fused backward over that many tokens takes the rows of X for dW1 | dW3 through expert_mapping (w1 and w3 back to back), 0: from a
+ * copy in expert_zones.  The same bits either way. */
+int amd_moe_layer_backward_gathers(const Amd_Moe_Layer * layer, int num_tokens, int first_micro_batch);
 
 /* ---- the reference's files, as far as this layer meets them ---- */
 

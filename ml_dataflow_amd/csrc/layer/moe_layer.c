@@ -382,6 +382,31 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 
 /* ------------------------------------------------------------------ backward */
 
+/* The stacked dW1 | dW3 GEMM can take the k-rows of X through expert_mapping (no re-dispatch), as the up-projection does in the
+ * forward.  On the sliced kernel, which finds the rows with a few instructions a slice, that saves the copy and more: X is an eighth
+ * of its copies and stays in the memory-side cache (64 groups of 1024 rows, 4096 x 2048 with C, us: packed 1150, gathered 1096, the copy 92; of 8192 rows, X
+ * 512 MiB, 7168, 7448 and 913).  Training steps: 8192 tokens, 64 experts, top 8, 4096 x 1024 4878 -> 4823, 65536 36677 -> 35705; 45 drawn ones 0.99-1.03x.
+ * It does where that kernel runs (its lines, matmul/amd_matmul.hip, one for both directions of the accumulation), the copy is worth it and the
+ * rows are not read again too often: with wide experts each k-row is fetched for every 256 columns of 2H, scattered (expert dims of 1664-2048 0.992-1.002x), and
+ * short rows make tiles whose chain of slices is the longer one (dim 576, a Zipf router: 0.947).  On eight waves, with fewer rows, the copy + packed form is
+ * the faster one (425 rows an expert 0.982). */
+#define BWD_GATHER_MEAN_ROWS 512
+#define BWD_GATHER_MEAN_ROWS_FIRST 640
+#define BWD_GATHER_LEAST_DIM 1280
+#define BWD_GATHER_MOST_EXPERT_DIM 1536
+int amd_moe_layer_backward_gathers(const Amd_Moe_Layer * L, int T, int first_micro_batch) {
+	const uint64_t rows = (uint64_t) T * L->top_k, E = L->num_experts, D = L->model_dim, H = L->expert_dim;
+	const uint64_t tiles = (D + 255) / 256 * ((2 * H + 255) / 256) * E;
+	if (!gather_allowed(T, L->model_dim)) {
+		return 0;
+	}
+	if (getenv("AMD_MOE_BWD_GATHER") != NULL) {
+		return 1;
+	}
+	return rows >= (first_micro_batch ? BWD_GATHER_MEAN_ROWS_FIRST : BWD_GATHER_MEAN_ROWS) * E && D >= BWD_GATHER_LEAST_DIM && H <= BWD_GATHER_MOST_EXPERT_DIM
+		&& 2 * H >= 256 && (!first_micro_batch || tiles > 256 || rows >= 2048 * E);
+}
+
 int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L, int T, void * X, void * dY, void * dX, int schedule) {
 	/* first micro-batch of an accumulation: the weight gradients are written (beta = 0, no C operand), not added to */
 	const int first_micro_batch = (schedule & AMD_MOE_FIRST_MICRO_BATCH) != 0;
@@ -556,12 +581,7 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 								 L->kernel_workspace_bytes, L->kernel_workspace), "failed to submit router dX matmul");
 
 	/* bwd_w: re-dispatch the inputs (:4062-4066), dW1 / dW3 (:4101-4148), dWr (:4174-4181) */
-	/* The stacked dW1 | dW3 GEMM can take the k-rows of X through expert_mapping (no re-dispatch), as the up-projection
-	 * does in the forward; here that form loses: a k-row of a tile is a 512-byte piece of a scattered row of X, and the
-	 * launch takes longer by more than the copy costs (config 4: 5.47 against 5.39 ms per step, config 5: 38.6 against
-	 * 38.0).  The copy + packed form is the default; AMD_MOE_BWD_GATHER in the environment selects the gathered one,
-	 * which gives the same bits. */
-	const int gathered = side_by_side && gather_allowed(T, D) && getenv("AMD_MOE_BWD_GATHER") != NULL;
+	const int gathered = side_by_side && amd_moe_layer_backward_gathers(L, T, first_micro_batch);
 	if (!gathered) {
 		CHECK(dataflow_submit_default_prepare_experts(h, cs, dt, dt, T, D, K, X, L->token_mapping, L->expert_zones), "failed to submit prepare experts (bwd_w)");
 	}

@@ -273,7 +273,7 @@ static int launch_w4d(const GemmParams & p, long tiles_upper_bound, long cu_coun
 }
 
 /* the four waves with k-major operands in slices (gemm_w4_kernel.h): same grid rule */
-template <int MODE>
+template <int MODE, int GATHER = GATHER_NONE>
 static int launch_w4k(const GemmParams & p, long tiles, long cu_count, hipStream_t stream) {
 	long grid = cu_count & ~7L;
 	if (grid < 8) {
@@ -284,9 +284,9 @@ static int launch_w4k(const GemmParams & p, long tiles, long cu_count, hipStream
 		grid = need;
 	}
 	if (p.C && p.beta != 0.0f) {
-		hipLaunchKernelGGL((gemm_bf16_w4k_kernel<true, MODE>), dim3((unsigned int) grid), dim3(256), 0, stream, p);
+		hipLaunchKernelGGL((gemm_bf16_w4k_kernel<true, MODE, GATHER>), dim3((unsigned int) grid), dim3(256), 0, stream, p);
 	} else {
-		hipLaunchKernelGGL((gemm_bf16_w4k_kernel<false, MODE>), dim3((unsigned int) grid), dim3(256), 0, stream, p);
+		hipLaunchKernelGGL((gemm_bf16_w4k_kernel<false, MODE, GATHER>), dim3((unsigned int) grid), dim3(256), 0, stream, p);
 	}
 	return check_launch();
 }
@@ -317,6 +317,11 @@ static bool w4_ok(const GemmParams & p) {
 static bool w4k_ok(const GemmParams & p) {
 	return p.M % 8 == 0 && p.N % 8 == 0 && p.M <= (1 << 22) && p.N <= (1 << 24) && p.strideD % 8 == 0 && ((((uintptr_t) p.D) & 15) == 0) &&
 		   (!(p.C && p.beta != 0.0f) || (((uintptr_t) p.C) & 15) == 0);
+}
+
+/* gathered k-rows: a row that does not exist, and a lane's column behind it, lie outside a source of this size */
+static bool w4k_gather_ok(const GemmParams & p) {
+	return (uint64_t) p.gather_rows * (uint64_t) p.M * 2u <= 0xFFFFF000ull;
 }
 
 /* The k-rows a tile has to have, in the mean, for the sliced kernel to be the faster one.  Its tiles have at least 8 slices of 32 k-rows
@@ -611,6 +616,9 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 	}
 	if (MODE == MODE_RAGGED_K && p.gather) {
 		/* gathered A: the k-rows of the reduction are fetched through the row map (both operands are k-major here) */
+		if (direct && big && w4k_gather_ok(p) && takes_sliced(MODE, p, grid_big, cu_count)) {
+			return launch_w4k<MODE_RAGGED_K, GATHER_P_KROWS>(p, grid_big, cu_count, stream);
+		}
 		if (direct) {
 			return big ? launch_stream<BIG_TILE, true, true, MODE_RAGGED_K, GATHER_P_KROWS>(p, grid_big, cu_count, stream)
 					   : launch_direct<true, true, MODE_RAGGED_K, GATHER_P_KROWS>(p, tile, stream);

@@ -653,6 +653,7 @@ class Wide(Mult, Tail):
 # ================================================================================================ four waves, ragged reduction
 R_SLICE, R_SLOTS = 32768, 5                                   # bytes of a slice of both operands (2 x 32 k x 256 rows), slices in the LDS
 R_C, R_PRD, R_QRD, R_VP, R_VQ, R_AT, R_CAT = 64, 192, 200, 208, 212, 216, 220
+R_MAP, R_MAPN, R_MAP0, R_MAP1, R_SEL, R_SEL0, R_KB, R_COL, R_T = 224, 225, 226, 227, 228, 229, 230, 231, 233      # gathered k-rows
 
 
 class Ring(Tail):
@@ -676,16 +677,82 @@ class Ring(Tail):
     s76 the slot, s77 scratch, s78 where the loads go, s79 the slice, s[84:87] C's descriptor, s[92:95] D's.
 
     State from statement to statement: slices 0-4 of the tile are on their way or there, slice 0 visible to all waves; behind them the 32
-    stores of the tile before."""
+    stores of the tile before.
+
+    GATHER: the k-rows of P are scattered over a source, by a map.  The cursor of P stays at the tile's first column of the source; s42 the
+    source's bytes from there, s43 its rows, s58 bytes of one of them (s50 and s51 of the next tile).  s[80:83] / s[88:91] buffers over this / the
+    next tile's map.  A wave's rows of eight slices, 8 r + j the j-th row of the r-th slice, are held one per lane, as the byte offset of the
+    source's row (R_MAP; a row that does not exist, outside any buffer), each load takes its two from there by a ds_bpermute, and the
+    offsets of the next eight slices are on their way (R_MAPN; of the next tile's first sixteen R_MAP0 and R_MAP1, which therefore are asked
+    for a tile ahead: a load between two tiles would wait for the stores in front of it).  R_SEL: where the slice's first row is, four bytes a
+    lane; R_KB, R_SEL0, R_COL: this lane's place in the map, in a slice, and column of the source, of even and of odd loads.  s96 bytes of the
+    map to the eight slices behind those held, s97 slices to them.  A tile has eight slices at least.  State: R_MAP the tile's first eight slices, R_SEL at
+    the sixth of them, R_MAPN the next eight."""
 
     LOADS, STORES = 8, 32
 
-    def __init__(self, HAS_C):
+    def __init__(self, HAS_C, GATHER=False):
         Asm.__init__(self)
-        self.C = HAS_C
-        self.least = 8 if HAS_C else 5           # slices a tile has at least
+        self.C, self.GATHER = HAS_C, GATHER
+        self.least = 8 if HAS_C or GATHER else 5           # slices a tile has at least
         self.head = 8 if HAS_C else 4            # slices in front of the loop
-        self.name = "W4K_%s" % ("C" if HAS_C else "NOC")
+        self.name = "W4K_%s%s" % ("C" if HAS_C else "NOC", "_GATHER" if GATHER else "")
+
+    def set_p(self, src):
+        """the buffer of P, gathered"""
+        for n, ins in enumerate(("s%d" % src, "s%d" % (src + 1), "s%d" % (src + 2), "0x00020000")):
+            self.e("s_mov_b32 s%d, %s" % (64 + n, ins))
+
+    def load_map(self, dst, buffer, at=None):
+        self.e("buffer_load_dword v%d, v%d, s[%d:%d], 0 offen" % (dst, R_KB if at is None else at, buffer, buffer + 3))
+
+    def hold(self, raw, buffer, at=None):
+        """the offsets of the rows `raw`, entries of the map from byte `at` (a register) or 0 on"""
+        e = self.e
+        where = R_KB
+        if at:
+            e("v_add_u32 v%d, %s, v%d" % (R_T, at, R_KB))
+            where = R_T
+        e("v_cmp_gt_u32 vcc, s%d, v%d" % (buffer + 2, where))
+        e("v_min_u32 v%d, s43, v%d" % (R_MAP, raw))
+        e("v_mul_lo_u32 v%d, v%d, s58" % (R_MAP, R_MAP))
+        e("v_mov_b32 v%d, 0xfffffc00" % R_T)
+        e("v_cndmask_b32 v%d, v%d, v%d, vcc" % (R_MAP, R_T, R_MAP))
+
+    def next_rows_of_map(self):
+        """in front of the loads of slice s79 + 5: its rows among those held"""
+        e = self.e
+        e("s_sub_u32 s97, s97, 1")
+        e("s_add_u32 s77, s79, %d" % R_SLOTS)
+        e("s_cmp_eq_u32 s77, s56")
+        e("s_cbranch_scc1 21f")
+        e("s_cmp_eq_u32 s97, 0")
+        e("s_cbranch_scc0 23f")
+        self.hold(R_MAPN, 80, "s96")             # the next eight slices of the tile
+        e("s_mov_b32 s97, 8")
+        e("s_add_u32 s96, s96, 1024")
+        e("s_add_u32 s77, s77, 8")
+        e("s_cmp_lt_u32 s77, s56")               # and those behind them, if there are any
+        e("s_cbranch_scc0 23f")
+        e("v_add_u32 v%d, s96, v%d" % (R_T, R_KB))
+        self.load_map(R_MAPN, 80, R_T)
+        e("s_branch 23f")
+        e("21:")                                 # the next tile's first eight
+        e("s_waitcnt vmcnt(%d)" % (3 * self.LOADS))        # asked for at least three slices ago
+        self.hold(R_MAP0, 88)
+        e("v_mov_b32 v%d, v%d" % (R_MAPN, R_MAP1))
+        e("v_mov_b32 v%d, v%d" % (R_SEL, R_SEL0))
+        e("s_mov_b32 s97, 16")                   # no more than five of them are loaded in this statement
+        e("23:")
+
+    def take_rows(self, u):
+        self.lds("ds_bpermute_b32 v%d, v%d, v%d offset:%d" % (R_VP + u, R_SEL, R_MAP, 8 * u))
+
+    def add_column(self, u):
+        self.e("v_add_u32 v%d, v%d, v%d" % (R_VP + u, R_COL + (u & 1), R_VP + u))
+
+    def next_slice_of_map(self):
+        self.e("v_add_u32 v%d, 32, v%d" % (R_SEL, R_SEL))
 
     set_cursor, advance = Wide.set_cursor, Wide.advance
 
@@ -717,7 +784,10 @@ class Ring(Tail):
         self.e("s_add_u32 s77, s79, %d" % R_SLOTS)
         self.e("s_cmp_eq_u32 s77, s56")
         self.e("s_cbranch_scc0 6f")
-        self.set_cursor(48, 0)
+        if self.GATHER:
+            self.set_p(48)
+        else:
+            self.set_cursor(48, 0)
         self.set_cursor(48, 1)
         self.e("6:")
 
@@ -726,7 +796,7 @@ class Ring(Tail):
         ops = []
         for t in range(1, R_SLOTS):
             ops += ["L%d" % t] * self.LOADS
-        ops += ["S"] * self.STORES
+        ops += ["S"] * self.STORES + (["M"] * 2 if self.GATHER else [])
         for t in range(s + 1):
             ops += ["C"] * (4 if self.C else 0)
             if t < s:
@@ -753,6 +823,12 @@ class Ring(Tail):
         at(9, lambda: e("s_sub_u32 s77, s76, s77"))
         for n in range(16):
             at(10 + n, lambda n=n: e("v_add_u32 v%d, s77, v%d" % (R_PRD + n, R_PRD + n)))
+        if self.GATHER:
+            at(7, self.next_rows_of_map)
+            for u in range(4):
+                at(12 + 3 * u, lambda u=u: self.take_rows(u))
+                at(32 + u // 2, lambda u=u: self.add_column(u))
+            at(35, self.next_slice_of_map)
         if self.C and s is not None and s < 8:
             for k in range(4):
                 at(11 + 4 * k, lambda k=k: self.load_c(s, k))
@@ -769,7 +845,8 @@ class Ring(Tail):
         at(34, self.move_on)
         for u in range(self.LOADS):
             at(36 + 3 * u, lambda u=u: self.dma(u))
-        at(58, lambda: self.advance(0))
+        if not self.GATHER:
+            at(58, lambda: self.advance(0))
         at(59, lambda: self.advance(1))
         at(60, lambda: e("s_add_u32 s79, s79, 1"))
         for m in range(64):
@@ -823,24 +900,49 @@ class Ring(Tail):
     def generate(self):
         e = self.e
         self.addresses()
-        self.set_cursor(40, 0)
+        if self.GATHER:
+            self.set_p(40)
+        else:
+            self.set_cursor(40, 0)
         self.set_cursor(40, 1)
         if self.C:
             for n, ins in enumerate(("s36", "s37", "s34", "0x00020000")):
                 e("s_mov_b32 s%d, %s" % (84 + n, ins))
         e("s_mov_b32 s76, s60")
         e("s_mov_b32 s79, 0")
+        if self.GATHER:
+            e("s_mov_b32 s96, 1024")
+            e("s_mov_b32 s97, 4")                # slices 5, 6 and 7 are held; counted down in front of each
         e("s_bitcmp1_b32 s57, 0")
         e("s_cbranch_scc0 2f")
+        if self.GATHER:
+            self.load_map(R_MAP0, 80)
+            e("v_add_u32 v%d, s96, v%d" % (R_T, R_KB))
+            self.load_map(R_MAPN, 80, R_T)
+            e("s_waitcnt vmcnt(0)")
+            self.hold(R_MAP0, 80)
+            e("v_mov_b32 v%d, v%d" % (R_SEL, R_SEL0))
         for t in range(R_SLOTS):                 # first tile (its first slot is slot 0)
             e("s_add_u32 s78, s63, %d" % (t * R_SLICE))
+            if self.GATHER:
+                for u in range(4):
+                    self.take_rows(u)
+                e("s_waitcnt lgkmcnt(0)")
+                for u in range(4):
+                    self.add_column(u)
+                self.next_slice_of_map()
             for u in range(self.LOADS):
                 self.dma(u)
-            self.advance(0)
+            if not self.GATHER:
+                self.advance(0)
             self.advance(1)
         e("s_waitcnt vmcnt(0)")
         e("s_barrier")
         e("2:")
+        if self.GATHER:
+            self.load_map(R_MAP0, 88)
+            e("v_add_u32 v%d, s96, v%d" % (R_T, R_KB))
+            self.load_map(R_MAP1, 88, R_T)
         for n in range(4):
             self.read("Q", n)
         for i in range(8):
@@ -899,14 +1001,14 @@ class Ring(Tail):
 
     def clobbers(self):
         return ["v%d" % i for i in range(R_VP)] + ["a%d" % i for i in range(256)] + ["s%d" % i for i in range(64, 80)] + \
-               ["s%d" % i for i in list(range(84, 88)) + list(range(92, 96))] + ["m0", "scc", "memory"]
+               ["s%d" % i for i in list(range(84, 88)) + list(range(92, 98 if self.GATHER else 96))] + (["vcc"] if self.GATHER else []) + ["m0", "scc", "memory"]
 
 
 def main():
     out = sys.argv[1] if len(sys.argv) > 1 else os.path.join(os.path.dirname(os.path.abspath(__file__)), "gemm_w4_loop.inc")
     with open(out, "w") as f:
         f.write("/* generated by gen_w4_loop.py -- do not edit */\n")
-        for v in (Mult(False), Mult(True), Loader(False), Loader(True), Wide(False, False), Wide(False, True), Wide(True, False), Wide(True, True), Ring(False), Ring(True)):
+        for v in (Mult(False), Mult(True), Loader(False), Loader(True), Wide(False, False), Wide(False, True), Wide(True, False), Wide(True, True), Ring(False), Ring(True), Ring(False, True), Ring(True, True)):
             parts = v.generate()
             if not isinstance(v, Wide):
                 parts = [(v.name + "_ASM", parts)]
@@ -937,7 +1039,11 @@ def main():
 
         # sliced kernel: the lane's load offsets vo (4 of P, 4 of Q) and its four of D and four of C, the blocks of scalars sd, sa, sb, sc
         f.write('#define W4K_OUTPUTS(vo, at) "+{v[%d:%d]}"(vo), "+{v[%d:%d]}"(at)\n' % (R_VP, R_VP + 7, R_AT, R_AT + 7))
-        for v in (Ring(False), Ring(True)):
+        # gathered k-rows: the registers from R_MAP on and the two buffers over maps
+        f.write('#define W4K_GATHER_OUTPUTS(vg) "+{v[%d:%d]}"(vg)\n' % (R_MAP, R_MAP + 15))
+        f.write('#define W4K_GATHER_INPUTS(mc, mn) "{s[80:83]}"(mc), "{s[88:91]}"(mn)\n')
+        f.write("#define W4K_SEL0 %d\n#define W4K_KB %d\n#define W4K_COL %d\n" % (R_SEL0 - R_MAP, R_KB - R_MAP, R_COL - R_MAP))
+        for v in (Ring(False), Ring(True), Ring(False, True), Ring(True, True)):
             f.write("#define %s_LEAST %d\n" % (v.name, v.least))
 
 if __name__ == "__main__":

@@ -86,6 +86,10 @@ class Machine:
             elif op == "buffer_load_dwordx4":
                 assert "s[84:87]" in rest
                 self.queue.append("C")
+            elif op == "buffer_load_dword":
+                assert "s[80:83]" in rest or "s[88:91]" in rest
+                self.maps_asked = getattr(self, "maps_asked", 0) + 1
+                self.queue.append(("map", self.maps_asked))
             elif op == "buffer_store_dwordx4":
                 assert "s[92:95]" in rest
                 self.stores += 1
@@ -98,7 +102,7 @@ class Machine:
                 self.at_epilogue()
                 last_mfma = False
             else:
-                assert op[0] == "v" or op.startswith("ds_read") or op == "s_nop" or op[:-1].isdigit(), op
+                assert op[0] == "v" or op.startswith(("ds_read", "ds_bpermute")) or op == "s_nop" or op[:-1].isdigit(), op
 
 
 def cursor(tile, at):
@@ -302,3 +306,134 @@ def test_wide_kernel_multiplies_short_tiles(macros, name, blocks):
                         want.add((k, acc, tuple(a), tuple([(M_BRD + 2 * s + stage, j * 2048)] * 4)))
         got = {(n // (32 * nb), acc, tuple(a), tuple(b)) for n, (acc, a, b) in enumerate(m.multiplied)}
         assert got == want and len(m.multiplied) == len(want)
+
+
+class Gathering(Machine):
+    """... and, lane by lane, the registers with which a wave finds the rows of its loads of P"""
+
+    MAP0 = 224                                   # first of them in the statement
+
+    class Lines(list):
+        def __getitem__(self, at):
+            line = list.__getitem__(self, at)
+            self.look(line)
+            return line
+
+    def __init__(self, lines, maps):
+        super().__init__(self.Lines(lines))
+        self.lines.look = self.look
+        self.plain, self.maps = lines, maps
+        self.v, self.pending, self.vcc, self.taken = {}, {}, None, []
+
+    def target(self, at, label):
+        places = range(at + 1, len(self.plain)) if label[-1] == "f" else range(at - 1, -1, -1)
+        return next(i for i in places if self.plain[i] == label[:-1] + ":")
+
+    def lanes(self, name):
+        if name[0] == "v" and name[1:].isdigit():
+            n = int(name[1:])
+            if n in self.pending:                # of a load of the map: there once it is no longer in the queue
+                assert not [x for x in self.queue if isinstance(x, tuple) and x[1] == self.pending[n][0]], name
+                self.v[n] = self.pending.pop(n)[1]
+            assert n not in [x for x, _ in self.taken], name
+            return list(self.v[n])
+        return [self.value(name)] * 64
+
+    def look(self, line):
+        op, _, rest = line.partition(" ")
+        a = [x.strip() for x in rest.replace(" offset:", ", ").replace(" offen", "").split(",")]
+        if op == "s_waitcnt" and "lgkmcnt(0)" in rest:
+            for n, value in self.taken:
+                self.v[n] = value
+            self.taken = []
+        if op.startswith("buffer_load_dwordx4") or not a[0].startswith("v") or not (a[0] == "vcc" or a[0][1:].isdigit() and (self.MAP0 <= int(a[0][1:]) < 240 or 208 <= int(a[0][1:]) < 212)):
+            return
+        n = None if a[0] == "vcc" else int(a[0][1:])
+        if op == "buffer_load_dword":
+            buffer = int(re.search(r"s\[(\d+):", rest).group(1))
+            entries, bytes_ = self.maps.get(self.s["s%d" % buffer], []), self.s["s%d" % (buffer + 2)]
+            assert n not in self.pending or not [x for x in self.queue if isinstance(x, tuple) and x[1] == self.pending[n][0]]
+            self.pending[n] = (getattr(self, "maps_asked", 0) + 1, [entries[x // 4] if x < bytes_ else 0 for x in self.lanes(a[1])])
+            return
+        if n in self.pending:                    # written behind the load, which is over
+            self.lanes(a[0])
+        if op == "v_cmp_gt_u32":
+            self.vcc = [x > y for x, y in zip(self.lanes(a[1]), self.lanes(a[2]))]
+        elif op == "v_cndmask_b32":
+            self.v[n] = [y if c else x for x, y, c in zip(self.lanes(a[1]), self.lanes(a[2]), self.vcc)]
+        elif op == "ds_bpermute_b32":
+            where, what = self.lanes(a[1]), self.lanes(a[2])
+            self.taken.append((n, [what[(x + int(a[3]) >> 2) & 63] for x in where]))
+        elif op == "v_mov_b32":
+            self.v[n] = self.lanes(a[1])
+        else:
+            do = {"v_add_u32": lambda x, y: x + y & MASK, "v_min_u32": min, "v_mul_lo_u32": lambda x, y: x * y & MASK}[op]
+            self.v[n] = [do(x, y) for x, y in zip(self.lanes(a[1]), self.lanes(a[2]))]
+
+
+@pytest.mark.parametrize("wave", [0, 3])
+@pytest.mark.parametrize("name,with_c", [("W4K_C_GATHER", 4), ("W4K_NOC_GATHER", 0)])
+def test_sliced_kernel_finds_the_rows_of_gathered_loads(macros, name, with_c, wave):
+    """the offsets of every load of P against the map, tiles of 8 to 40 slices whose last one is not full, rows outside the source"""
+    import random
+    rng = random.Random(wave)
+    slot_bytes, slots, per_slice, pitch, source_rows = 32768, 5, 8, 512, 1000
+    rows = [250, 256, 257, 300, 512, 513, 1280, 100, 255, 700, 256, 513]
+    tiles = [max(8, -(-r // 32)) for r in rows]
+    start = [sum(tiles[:t]) for t in range(len(tiles))]
+    maps = {(t + 1) << 20: [rng.choice([rng.randrange(source_rows)] * 9 + [MASK]) for _ in range(r)] for t, r in enumerate(rows)}
+    m = Gathering(lines_of(macros, name + "_ASM"), maps)
+
+    def swizzle(k):
+        return (k & 3) << 2 ^ (k >> 3 & 1) << 1
+
+    m.v[230] = [4 * (32 * (l >> 3) + 8 * wave + (l & 7)) for l in range(64)]
+    m.v[229] = [4 * (l >> 5) for l in range(64)]
+    for odd in range(2):
+        m.v[231 + odd] = [((l & 31) ^ swizzle(8 * wave + 2 * odd + (l >> 5))) * 16 for l in range(64)]
+
+    def slices_there():
+        waiting = [x for x in m.queue if isinstance(x, int)]
+        return (waiting[0] if waiting else len(m.loads)) // per_slice
+
+    def at_barrier():
+        assert slices_there() == slots if m.barriers == 0 else slices_there() > m.barriers, (name, m.barriers)
+
+    def at_load():
+        operand, address, place = m.loads[-1]
+        g, u = divmod(len(m.loads) - 1, per_slice)
+        assert g < slots or m.barriers > g - slots + 1
+        assert place == 4096 * 2 + g % slots * slot_bytes + u % 4 * CHUNK + (16384 if u >= 4 else 0)
+        t = max(t for t in range(len(tiles)) if start[t] <= g)
+        k = g - start[t]
+        if k >= tiles[t]:
+            return
+        if u >= 4:
+            assert (operand, address) == ("Q", (t + 1 << 36) + k * Q_BYTES)
+            return
+        assert (operand, address) == ("P", t + 1 << 32)
+        for l in range(64):
+            row = 32 * k + 8 * wave + 2 * u + (l >> 5)
+            column = ((l & 31) ^ swizzle(row)) * 16
+            got = m.lanes("v%d" % (208 + u))[l]
+            if row < rows[t] and maps[(t + 1) << 20][row] < source_rows:
+                assert got == maps[(t + 1) << 20][row] * pitch + column
+            else:
+                assert got >= source_rows * pitch                          # outside the source: zeros
+
+    m.at_barrier, m.at_load = at_barrier, at_load
+    for t, slices in enumerate(tiles):
+        before = m.mfmas, m.from_zero, m.stores, m.barriers, len(m.loads)
+        following = t + 1 if t + 1 < len(tiles) else None
+        source = lambda n: [0, n + 1, source_rows * pitch, source_rows] if n is not None else [0, 0, 0, source_rows]
+        give(m, 32, [7, 0, 1 << 20, 512, 9, 0, 0x3f800000, 0x3f800000])
+        give(m, 40, source(t) + cursor(t, 0 if t == 0 else slots)[4:])
+        give(m, 48, source(following) + cursor(following, 0)[4:])
+        give(m, 56, [slices, t == 0, pitch, Q_BYTES, start[t] % slots * slot_bytes, 0, 16384, 4096 * 2])
+        give(m, 80, [(t + 1) << 20, 0, 4 * rows[t], 0x20000])
+        give(m, 88, [(t + 2) << 20, 0, 4 * rows[t + 1], 0x20000] if following is not None else [0, 0, 0, 0x20000])
+        m.run()
+        assert m.mfmas - before[0] == 64 * slices and m.from_zero - before[1] == 64
+        assert m.stores - before[2] == 32
+        assert m.barriers - before[3] == slices + (t == 0)
+        assert len(m.loads) - before[4] == per_slice * (slices + (slots if t == 0 else 0))

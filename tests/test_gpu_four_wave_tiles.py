@@ -142,3 +142,29 @@ def test_ragged_k_by_default_with_c_apart_and_gaps_between_groups(backend, selec
     assert (be.read(d_C.ptr, (groups * stride,), np.uint16) == c).all()
     for buffer in (d_A, d_B, d_C, d_cum):
         buffer.free()
+
+
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+@pytest.mark.parametrize("M,N,groups", [(520, 264, 70), (1304, 512, 24)])
+def test_ragged_k_gathered_rows_on_slices(backend, select_kernel, beta, M, N, groups):
+    """Rows of a group on both sides of a slice, of the eight slices whose rows a wave holds and of the fewest a tile has; entries outside the
+    source; groups without rows; more groups than lanes.  The sliced kernel against the eight-wave one, which gathers too."""
+    be = backend
+    counts = np.array([0, 1, 31, 32, 33, 255, 256, 257, 288, 289, 511, 512, 513, 0, 3000, 2047, 2048, 2049, 160, 161, 96, 768, 1025, 1500], dtype=np.int32)
+    counts = np.concatenate([counts, np.full(groups - len(counts), 900, np.int32)])
+    total, src_rows = int(counts.sum()), 1237
+    # lines of the sliced kernel: 512 rows a group in the mean with C, 640 without
+    assert runs_sliced(select_kernel, FOUR_384, M, total, N, groups, beta != 0.0) and total >= 640 * groups
+    print("case gathered slices M=%d N=%d groups=%d rows=%d beta=%g" % (M, N, groups, total, beta), flush=True)
+    rng = np.random.default_rng(M + groups)
+    row_map = rng.integers(0, src_rows, total).astype(np.int32)
+    row_map[rng.integers(0, total, 50)] = -1
+    row_map[rng.integers(0, total, 50)] = src_rows
+    d_A, d_B = be.upload(normal_bf16(rng, (src_rows, M))), be.upload(normal_bf16(rng, (total, N), 0.05))
+    d_cum, d_map = be.upload(np.cumsum(counts).astype(np.int32)), be.upload(row_map)
+    both(be, select_kernel, FOUR_384, groups * N * M, normal_bf16(rng, (groups * N * M,)),
+         lambda d_D: be.lib.dataflow_submit_amd_grouped_matmul_gathered(be.hp, CS, BF, BF, BF if beta else B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 0, 1, B.AMD_GROUPED_RAGGED_K,
+                                                                        M, total, N, groups, d_cum.ptr, 1.0, beta, d_A.ptr, 0, d_B.ptr, d_D.ptr if beta else None, d_D.ptr,
+                                                                        N * M * 2, d_map.ptr, src_rows))
+    for d in (d_A, d_B, d_cum, d_map):
+        d.free()

@@ -154,6 +154,18 @@ def test_the_benchmark_times_the_ops_the_layer_submits(schedule, first):
     assert len(rows) == len(submitted) and all(name in work for name, _ in rows)
 
 
+@pytest.mark.parametrize("tokens,first,gathers", [(0, False, False), (2047, False, False), (2048, False, True), (2559, True, False), (2560, True, True)])
+def test_the_backward_gathers_where_experts_have_the_rows(tokens, first, gathers):
+    """dim 1280, 8 experts, top 2: the lines are 512 and 640 rows an expert; not with wide experts, narrow rows or an environment that forbids it"""
+    lib = B.load_library()
+    layer = B.AmdMoeLayer(model_dim=1280, num_experts=8, top_k=2, expert_dim=1536)
+    assert lib.amd_moe_layer_backward_gathers(C.byref(layer), tokens, first) == gathers
+    for name, value in (("model_dim", 1272), ("expert_dim", 1544)):
+        other = B.AmdMoeLayer(model_dim=1280, num_experts=8, top_k=2, expert_dim=1536)
+        setattr(other, name, value)
+        assert lib.amd_moe_layer_backward_gathers(C.byref(other), tokens, first) == 0
+
+
 UP_OPS = ["amd_grouped_matmul_gathered", "amd_swiglu_strided_BF16"]
 
 
