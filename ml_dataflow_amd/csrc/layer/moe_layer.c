@@ -181,6 +181,9 @@ static void * expert_ptr(void * base, uint64_t stride, int e) {
 /* the two streams meet: `waiter` will not run past this point before `signaller` reaches it
  * (dataflow_transformer.c:2814-2826) */
 static int stream_wait(Dataflow_Handle * h, int waiter, int signaller) {
+	if (waiter == signaller) {
+		return 0;                                          /* a stream is in order with itself */
+	}
 	void * state = (h->get_stream_state)(h, signaller);
 	if (!state) {
 		fprintf(stderr, "Error: failed to get stream state for stream #%d...\n", signaller);
@@ -191,6 +194,18 @@ static int stream_wait(Dataflow_Handle * h, int waiter, int signaller) {
 		return -1;
 	}
 	return 0;
+}
+
+/* The stream of the second of two independent grouped matmuls (grouped schedule).  On the secondary one its work-groups move into the compute units
+ * that the first one's last, partial round of tiles leaves idle; on the compute stream nothing has to meet in front of and behind the pair, and in
+ * a pass that uses one queue alone every other launch follows sooner too.  The second is the better one for small passes.  Training steps, us, two
+ * streams and one: 374 tokens, 28 experts, top 3, 1152 / 576 230 and 184; 590, 25, top 8, 1728 / 512 337 and 298; 551, 32, top 8, 3456 / 896 858 and
+ * 828; 25 with an even router between 2^35 and 2^36 multiplies of the stacked up-projection 0-4 % less, beyond 2^36 up to 2.5 % more (4096, 32, top 4, 2048 / 1408 1410 and 1431).
+ * With a Zipf router a launch can end in the long tiles of one group, which another hides: 34 steps of up to 2498 tokens 0.3 % more to 10 % less,
+ * of 20 with more tokens nine 2-21 % more (40457, 55, top 1, 512 / 1536 2537 and 3221).  No group has more rows than there are tokens. */
+#define ONE_STREAM_MOST_TOKENS 2048
+static int second_stream(const Amd_Moe_Layer * L, int T, int cs, int ss) {
+	return T <= ONE_STREAM_MOST_TOKENS && (uint64_t) T * L->top_k * 2 * L->expert_dim * L->model_dim <= LAYER_UP_SWIGLU_GROUPED_MULTIPLIES ? cs : ss;
 }
 
 /* may the up-projections of an expert's rows and their activation be one op with x1 and x3 apart, where the rows are few enough? */
@@ -301,16 +316,16 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 											   L->expert_mapping, T, L->x1, L->x3, L->kernel_workspace), "failed to submit grouped up projections and swiglu");
 		} else {
 			CHECK(dataflow_submit_default_prepare_experts(h, cs, dt, dt, T, D, K, X, L->token_mapping, L->expert_zones), "failed to submit prepare experts");
-			/* The two up-projections are independent: the second goes to the secondary stream, so its work-groups move
-			 * into the compute units that the first one's last, partial round of tiles leaves idle. */
-			CHECK(stream_wait(h, ss, cs), "secondary stream could not wait for the compute stream");
+			/* The two up-projections are independent (second_stream) */
+			const int second = second_stream(L, T, cs, ss);
+			CHECK(stream_wait(h, second, cs), "secondary stream could not wait for the compute stream");
 			CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, H, D, T * K,
 													 E, L->expert_counts_cumsum, 1.0f, 0.0f, L->w1, L->expert_stride_bytes, L->expert_zones, NULL, L->x1, 0),
 				  "failed to submit grouped w1 matmul");
-			CHECK(dataflow_submit_amd_grouped_matmul(h, ss, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, H, D, T * K,
+			CHECK(dataflow_submit_amd_grouped_matmul(h, second, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, H, D, T * K,
 													 E, L->expert_counts_cumsum, 1.0f, 0.0f, L->w3, L->expert_stride_bytes, L->expert_zones, NULL, L->x3, 0),
 				  "failed to submit grouped w3 matmul");
-			CHECK(stream_wait(h, cs, ss), "compute stream could not wait for the secondary stream");
+			CHECK(stream_wait(h, cs, second), "compute stream could not wait for the secondary stream");
 			CHECK(dataflow_submit_default_swiglu(h, cs, dt, T * K, H, L->x1, L->x3, L->kernel_workspace), "failed to submit swiglu");
 		}
 		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, D, H, T * K,
@@ -493,14 +508,14 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 												   L->expert_zones, dY, L->d_routed, L->expert_zones), "failed to submit router bwd x");
 		/* dW2 += g^T h (:3548-3555) and dh = g W2 (:3568-3575).  The reference writes dh over h, which orders the two;
 		 * here dh goes to the dx1 buffer (swiglu_bwd_x then works in place: it reads an element of dh before it writes
-		 * that element of dx1), so the two GEMMs are independent and the second runs on the secondary stream, filling
-		 * the compute units that the first one's last round of tiles leaves idle. */
-		CHECK(stream_wait(h, ss, cs), "secondary stream could not wait for the compute stream");
+		 * that element of dx1), so the two GEMMs are independent (second_stream). */
+		const int second = second_stream(L, T, cs, ss);
+		CHECK(stream_wait(h, second, cs), "secondary stream could not wait for the compute stream");
 		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, H, T * K, D, E, cum,
 												 1.0f, wbeta, temp, 0, L->expert_zones, WGRAD_C(L->dw2), L->dw2, S), "failed to submit grouped dW2 matmul");
-		CHECK(dataflow_submit_amd_grouped_matmul(h, ss, dt, dt, DATAFLOW_NONE, dt, cdt, 0, 0, AMD_GROUPED_RAGGED_N, H, D, T * K, E, cum,
+		CHECK(dataflow_submit_amd_grouped_matmul(h, second, dt, dt, DATAFLOW_NONE, dt, cdt, 0, 0, AMD_GROUPED_RAGGED_N, H, D, T * K, E, cum,
 												 1.0f, 0.0f, L->w2, S, L->expert_zones, NULL, L->dx1, 0), "failed to submit grouped dh matmul");
-		CHECK(stream_wait(h, cs, ss), "compute stream could not wait for the secondary stream");
+		CHECK(stream_wait(h, cs, second), "compute stream could not wait for the secondary stream");
 		CHECK(dataflow_submit_default_swiglu_bwd_x(h, cs, dt, dt, T * K, H, L->x1, L->x3, L->dx1, L->dx1, L->dx3), "failed to submit swiglu bwd x");
 		/* zone = dx1 W1, zone += dx3 W3 (:3601-3621) */
 		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, DATAFLOW_NONE, dt, cdt, 0, 0, AMD_GROUPED_RAGGED_N, D, H, T * K, E, cum,
@@ -594,13 +609,14 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, T * K, 2 * H, E, L->expert_counts_cumsum,
 												 1.0f, wbeta, L->expert_zones, 0, L->dx1, WGRAD_C(L->dw1), L->dw1, S), "failed to submit grouped dW1|dW3 matmul");
 	} else if (schedule != AMD_MOE_PER_EXPERT) {
-		/* independent of each other: the second on the secondary stream, as for the up-projections */
-		CHECK(stream_wait(h, ss, cs), "secondary stream could not wait for the compute stream");
+		/* independent of each other, as the up-projections */
+		const int second = second_stream(L, T, cs, ss);
+		CHECK(stream_wait(h, second, cs), "secondary stream could not wait for the compute stream");
 		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, T * K, H, E, L->expert_counts_cumsum,
 												 1.0f, wbeta, L->expert_zones, 0, L->dx1, WGRAD_C(L->dw1), L->dw1, S), "failed to submit grouped dW1 matmul");
-		CHECK(dataflow_submit_amd_grouped_matmul(h, ss, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, T * K, H, E, L->expert_counts_cumsum,
+		CHECK(dataflow_submit_amd_grouped_matmul(h, second, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, T * K, H, E, L->expert_counts_cumsum,
 												 1.0f, wbeta, L->expert_zones, 0, L->dx3, WGRAD_C(L->dw3), L->dw3, S), "failed to submit grouped dW3 matmul");
-		CHECK(stream_wait(h, cs, ss), "compute stream could not wait for the secondary stream");
+		CHECK(stream_wait(h, cs, second), "compute stream could not wait for the secondary stream");
 	} else {
 		CHECK(stream_wait(h, ss, cs), "secondary stream could not wait for the compute stream");
 		int streams[2] = {cs, ss};

@@ -166,6 +166,23 @@ def test_the_backward_gathers_where_experts_have_the_rows(tokens, first, gathers
         assert lib.amd_moe_layer_backward_gathers(C.byref(other), tokens, first) == 0
 
 
+@pytest.mark.parametrize("tokens,dim,streams", [(1024, 4096, {1}), (1025, 4096, {1, 2}), (2048, 2048, {1}), (2049, 1024, {1, 2})])
+def test_small_grouped_passes_stay_on_one_stream(tokens, dim, streams):
+    """the lines: 2^36 multiplies of the stacked up-projection, 2048 tokens; a layer whose w3 lies apart from w1 has a pair of matmuls in its forward"""
+    noting, used, met = NotingHandle(), [], []
+    fields = dict(B.DataflowHandle._fields_)
+    on = fields["submit_op"](lambda handle, op, stream: used.append(stream) or 0)
+    meet = fields["submit_dependency"](lambda *a: met.append(a[1]) or 0)
+    noting.h.submit_op, noting.h.submit_dependency = on, meet
+    layer = noting.layer(max_tokens=tokens, model_dim=dim, expert_dim=1024, num_experts=64, top_k=8, expert_stride_bytes=6 * dim * 1024)
+    assert noting.lib.amd_moe_layer_forward(C.pointer(noting.h), 1, 2, C.byref(layer), tokens, 1 << 32, None, 2 << 32, B.AMD_MOE_GROUPED) == 0
+    assert set(used) == streams and set(met) == (streams if len(streams) > 1 else set())
+    used.clear()
+    met.clear()
+    assert noting.lib.amd_moe_layer_backward(C.pointer(noting.h), 1, 2, C.byref(layer), tokens, 1 << 32, 2 << 32, 3 << 32, B.AMD_MOE_GROUPED) == 0
+    assert set(used) == streams and len(met) == (4 if len(streams) > 1 else 0)
+
+
 UP_OPS = ["amd_grouped_matmul_gathered", "amd_swiglu_strided_BF16"]
 
 
