@@ -74,6 +74,41 @@ def test_ragged_n_many_groups(backend, select_kernel, transa, alpha, M, K, group
         d.free()
 
 
+@pytest.mark.parametrize("transa", [1, 0])
+@pytest.mark.parametrize("gathered", [False, True])
+@pytest.mark.parametrize("n_tiles", [20, 48, 60, 70, 112])
+def test_ragged_n_partial_last_rounds(backend, select_kernel, n_tiles, gathered, transa):
+    """A die's last round in pieces: the only round, in two (15 tiles for 32 work-groups), a second one in three and in two (4, 13), none (21), a third in
+    two and three; tiles of few rows, that have fewer blocks of columns than pieces, and of a group of many tiles."""
+    be = backend
+    M, K, src_rows = 1304, 256, 997
+    rng = np.random.default_rng(n_tiles + 2 * gathered + transa)
+    counts = [3500] if n_tiles > 20 else []
+    counts += [1] if n_tiles % 20 == 0 else []
+    while sum(-(-c // 384) for c in counts) < n_tiles:
+        counts.append(int(rng.choice([1, 63, 129, 193, 257, 320, 383, 384, 385, 449, 640, 768])))
+        if sum(-(-c // 384) for c in counts) > n_tiles:
+            counts[-1] = 384
+    counts = np.array(counts[1:] + counts[:1], np.int32)
+    total, groups = int(counts.sum()), len(counts)
+    # the named kernel runs from this many rows on: an upper bound of them is what a launch is told
+    most = max(total, 256 * 22)
+    assert most // 256 * -(-M // 256) >= 128
+    print("case partial last rounds: tiles=%d gathered=%d ta=%d rows=%d groups=%d" % (n_tiles, gathered, transa, total, groups), flush=True)
+    d_W = be.upload(normal_bf16(rng, (groups, M, K) if transa else (groups, K, M), 0.05))
+    d_X = be.upload(normal_bf16(rng, (src_rows if gathered else most, K)))
+    d_cum, d_map = be.upload(np.cumsum(counts).astype(np.int32)), be.upload(rng.integers(-1, src_rows + 1, most).astype(np.int32))
+    args = (be.hp, CS, BF, BF, B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, transa, 0, B.AMD_GROUPED_RAGGED_N, M, K, most, groups, d_cum.ptr, 1.0, 0.0,
+            d_W.ptr, M * K * 2, d_X.ptr, None)
+    if gathered:
+        submit = lambda d_D: be.lib.dataflow_submit_amd_grouped_matmul_gathered(*args, d_D.ptr, 0, d_map.ptr, src_rows)
+    else:
+        submit = lambda d_D: be.lib.dataflow_submit_amd_grouped_matmul(*args, d_D.ptr, 0)
+    both(be, select_kernel, FOUR_384, total * M, np.zeros(total * M, np.uint16), submit)
+    for d in (d_W, d_X, d_cum, d_map):
+        d.free()
+
+
 @pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (1.0, 1.0), (-0.75, 0.0), (1.5, -0.5)])
 @pytest.mark.parametrize("M,N,groups", [(264, 520, 64), (1304, 264, 70), (256, 256, 300)])
 def test_ragged_k_tiles_and_slices(backend, select_kernel, alpha, beta, M, N, groups):
