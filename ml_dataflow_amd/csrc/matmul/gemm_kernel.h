@@ -83,12 +83,12 @@ struct GemmParams {
 	 * (those past them read as zero, like the padding they are multiplied with) */
 	int pitchA, pitchB;
 	int k_rows;
+	/* ragged N on the direct kernel: the weights of groups with one tile of rows are loaded non-temporally (streams_weights) */
+	int stream_weights;
 	/* a second single problem of the same shape and A behind the first, on the direct kernel (NULL D_twin: none) */
 	const bf16_t * B_twin;
 	const bf16_t * C_twin;
 	bf16_t * D_twin;
-	/* ragged N on the direct kernel: the weights of groups with one tile of rows are loaded non-temporally (streams_weights) */
-	int stream_weights;
 };
 
 struct Tile {
