@@ -206,9 +206,9 @@ def replay_step_with_events(be, layer, T, d_X, d_out, d_dY, d_dX, d_bias, backwa
 TRAFFIC_SOURCE = ("profiles/moe_layer_%s_hbm_traffic.md: hardware counters of two separate runs of this script, not of this run")
 MEASURED_TRAFFIC_BYTES = {
     "config4_fwdbwd_8192x4096_e64k8_h1024": {
-        "gemm_up13": 2161455558, "gemm_tn": 1371280124, "gemm_nn": 1535730842, "gemm_nt_dw": 1854822314, "gemm_dx13": 2206062164,
-        "gemm_dw13": 3748477803, "dispatch_scaled": 605606686, "swiglu": 400734208, "swiglu_bwd_x_routed": 822825787, "combine": 668830825,
-        "combine_grad": 601176532, "dispatch": 604556391,
+        "gemm_up13": 3496291835, "gemm_tn": 1431075660, "gemm_nn": 2115575916, "gemm_nt_dw": 1850063536, "gemm_dx13": 2728310496,
+        "gemm_dw13": 3750854003, "dispatch_scaled": 605606411, "swiglu": 400734999, "swiglu_bwd_x_routed": 822810773, "combine": 668832146,
+        "combine_grad": 601176166,
     },
     "config5_fwdbwd_65536x4096_e64k8_h1024": {
         "gemm_up13": 18470144588, "gemm_tn": 11482951390, "gemm_nn": 9339866922, "gemm_nt_dw": 16609306740, "gemm_dx13": 29595429204,
