@@ -211,9 +211,9 @@ MEASURED_TRAFFIC_BYTES = {
         "combine_grad": 601176166,
     },
     "config5_fwdbwd_65536x4096_e64k8_h1024": {
-        "gemm_up13": 18470144588, "gemm_tn": 11482951390, "gemm_nn": 9339866922, "gemm_nt_dw": 16609306740, "gemm_dx13": 29595429204,
-        "gemm_dw13": 41511091429, "dispatch_scaled": 4844596061, "swiglu": 3205541793, "swiglu_bwd_x_routed": 6617716932, "combine": 5350069289,
-        "combine_grad": 4808784480, "dispatch": 4836258995,
+        "gemm_up13": 18140215299, "gemm_tn": 11598692544, "gemm_nn": 9610729576, "gemm_nt_dw": 18076972731, "gemm_dx13": 31305495330,
+        "gemm_dw13": 29264811696, "dispatch_scaled": 4844597161, "swiglu": 3205540481, "swiglu_bwd_x_routed": 6617719634, "combine": 5350067597,
+        "combine_grad": 4808785202,
     },
 }
 
