@@ -252,7 +252,13 @@ static int row_kernel_config(Hip_Launch_Config * cfg, Op * op, const char * name
 
 int default_rms_norm_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {
 	(void) handle; (void) fn;
-	return row_kernel_config(cfg, op, "rms_norm");
+	if (row_kernel_config(cfg, op, "rms_norm")) {
+		return -1;
+	}
+	if (ARG_INT(op, 1) <= 1024 && ARG_INT(op, 0) >= 8192) {
+		cfg->gridDimX = ((unsigned int) ARG_INT(op, 0) + 3) / 4;          /* rows on one wave each: NORM_WAVE_ROW_COLS, norm.hip */
+	}
+	return 0;
 }
 
 int default_rms_norm_recompute_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {

@@ -21,13 +21,81 @@
 
 #define NORM_MAX_VEC 4
 
-/* r[row], out = bf16((x * r) * w).  Launch: grid = n_rows, block = 256.
+__device__ __forceinline__ void add_squares(u32x4 q, float & sum) {
+	float f[8];
+	unpack8(q, f);
+	#pragma unroll
+	for (int i = 0; i < 8; i++) {
+		sum = __builtin_fmaf(f[i], f[i], sum);
+	}
+}
+
+__device__ __forceinline__ u32x4 normed(u32x4 x, u32x4 w, float r) {
+	float f[8], g[8], y[8];
+	unpack8(x, f);
+	unpack8(w, g);
+	#pragma unroll
+	for (int i = 0; i < 8; i++) {
+		y[i] = (f[i] * r) * g[i];
+	}
+	return pack8(y);
+}
+
+/* A row of up to 1024 columns on one wave.  On a work-group such a row keeps two of its waves idle or more, and all four meet twice for a sum; here nothing
+ * meets and both loads of x and w are out at once.  The vectors of a lane are those that two of the four waves would have, summed by wave and added in
+ * their order: the same bits.  us, over several sets of arrays, a work-group a row and so: 32768 x 512 19.8 and 12.2, 16384 x 960 13.4 and 11.8, 12000 x
+ * 1024 11.4 and 9.5, 8192 x 576 7.8 and 6.1, 8192 x 1024 8.7 and 7.7.  From 2048 columns on (8192 rows 12.1 and 12.4) and with fewer rows (3000 x
+ * 1600 5.6 and 6.7) rows on a work-group, which spread over more waves, are the faster ones.  Those with their loads in front of the sum, unrolled,
+ * took 1-4 % less from 5120 columns on and 4 % more at 2048: 68 registers, seven work-groups a compute unit instead of eight. */
+#define NORM_WAVE_ROW_COLS 1024                          /* launch_config.c has these two as well */
+#define NORM_WAVE_ROW_LEAST_ROWS 8192
+#define NORM_WAVE_ROW_VEC (NORM_WAVE_ROW_COLS / 8 / WAVE)
+__device__ __forceinline__ void rms_norm_wave_row(int n_cols, float eps, const u32x4 * x, const u32x4 * __restrict__ w, u32x4 * o, float * rms) {
+	const int nvec = n_cols >> 3, lane = threadIdx.x & (WAVE - 1);
+	u32x4 keep[NORM_WAVE_ROW_VEC], scale[NORM_WAVE_ROW_VEC];
+	#pragma unroll
+	for (int j = 0; j < NORM_WAVE_ROW_VEC; j++) {
+		if (lane + j * WAVE < nvec) {
+			keep[j] = x[lane + j * WAVE];
+		}
+	}
+	#pragma unroll
+	for (int j = 0; j < NORM_WAVE_ROW_VEC; j++) {
+		if (lane + j * WAVE < nvec) {
+			scale[j] = w[lane + j * WAVE];
+		}
+	}
+	float sum = 0.0f;
+	#pragma unroll
+	for (int j = 0; j < NORM_WAVE_ROW_VEC; j++) {
+		if (j * WAVE < nvec) {                           /* uniform */
+			float part = 0.0f;
+			if (lane + j * WAVE < nvec) {
+				add_squares(keep[j], part);
+			}
+			sum += wave_sum(part);
+		}
+	}
+	const float r = rsqrtf(sum * (1.0f / (float) n_cols) + eps);
+	if (lane == 0 && rms) {
+		*rms = r;
+	}
+	#pragma unroll
+	for (int j = 0; j < NORM_WAVE_ROW_VEC; j++) {
+		if (lane + j * WAVE < nvec) {
+			o[lane + j * WAVE] = normed(keep[j], scale[j], r);
+		}
+	}
+}
+
+/* r[row], out = bf16((x * r) * w).  Launch: block = 256, grid = n_rows, or a quarter of them for rows on one wave.
  * Algorithmic HBM bytes: 2*n_rows*n_cols read, 2*n_rows*n_cols + 4*n_rows written (w stays in cache). */
 extern "C" __global__ void __launch_bounds__(ROW_THREADS)
 default_rms_norm_bf16_kernel(int n_rows, int n_cols, float eps, const bf16_t * __restrict__ rms_weight,
 							 const bf16_t * __restrict__ X, bf16_t * __restrict__ out, float * __restrict__ rms_vals) {
 	__shared__ float scratch[ROW_WAVES];
-	const int row = blockIdx.x;
+	const bool wave_rows = n_cols <= NORM_WAVE_ROW_COLS && n_rows >= NORM_WAVE_ROW_LEAST_ROWS;
+	const int row = wave_rows ? (int) (blockIdx.x * ROW_WAVES + threadIdx.x / WAVE) : (int) blockIdx.x;
 	if (row >= n_rows) {
 		return;
 	}
@@ -35,6 +103,10 @@ default_rms_norm_bf16_kernel(int n_rows, int n_cols, float eps, const bf16_t * _
 	const u32x4 * x = (const u32x4 *) (X + (size_t) row * n_cols);
 	u32x4 * o = (u32x4 *) (out + (size_t) row * n_cols);
 	const u32x4 * w = (const u32x4 *) rms_weight;
+	if (wave_rows) {
+		rms_norm_wave_row(n_cols, eps, x, w, o, rms_vals ? rms_vals + row : nullptr);
+		return;
+	}
 
 	u32x4 keep[NORM_MAX_VEC];
 	float part[1] = {0.0f};

@@ -54,6 +54,31 @@ def test_rms_norm_forward_and_recompute(backend, oracle, rows, cols):
     assert (be.read(d_X.ptr, (rows, cols), np.uint16) == got).all()
 
 
+# rows on one wave, four to a work-group (8192 rows and more of up to 1024 columns), give the bits of rows on a work-group (two calls of half the rows)
+@pytest.mark.parametrize("rows,cols", [(8192, 8), (8193, 64), (8195, 512), (8194, 520), (8192, 1016), (8193, 1024), (8192, 1032)])
+def test_rms_norm_rows_on_a_wave(backend, rows, cols):
+    print("case rms_norm rows=%d cols=%d" % (rows, cols), flush=True)
+    be = backend
+    rng = np.random.default_rng(rows * 3 + cols)
+    X = normal_bf16(rng, (rows, cols), 1.5)
+    X[5], X[6, 0], X[7, cols - 1] = 0, 0x7F80, 0x7FC0                  # a row of zeros, an infinity, a NaN
+    W = f32_to_bf16(1.0 + 0.1 * rng.standard_normal(cols).astype(np.float32))
+    d_X, d_W = be.upload(X), be.upload(W)
+    d_out, d_rms, d_part, d_prms = be.alloc(rows * cols * 2), be.alloc(rows * 4), be.alloc(rows * cols * 2), be.alloc(rows * 4)
+    assert be.lib.dataflow_submit_default_rms_norm(be.hp, CS, BF, rows, cols, EPS, d_W.ptr, d_X.ptr, d_out.ptr, d_rms.ptr) == 0
+    half = rows // 2
+    for first, n in ((0, half), (half, rows - half)):
+        at = first * cols * 2
+        assert be.lib.dataflow_submit_default_rms_norm(be.hp, CS, BF, n, cols, EPS, d_W.ptr, d_X.ptr + at, d_part.ptr + at, d_prms.ptr + first * 4) == 0
+    be.sync(CS)
+    assert (be.read(d_rms.ptr, (rows,), np.uint32) == be.read(d_prms.ptr, (rows,), np.uint32)).all()
+    assert (be.read(d_out.ptr, (rows, cols), np.uint16) == be.read(d_part.ptr, (rows, cols), np.uint16)).all()
+    # the statistic is optional, and the output may alias the input
+    assert be.lib.dataflow_submit_default_rms_norm(be.hp, CS, BF, rows, cols, EPS, d_W.ptr, d_X.ptr, d_X.ptr, None) == 0
+    be.sync(CS)
+    assert (be.read(d_X.ptr, (rows, cols), np.uint16) == be.read(d_part.ptr, (rows, cols), np.uint16)).all()
+
+
 @pytest.mark.parametrize("with_out", [True, False])
 @pytest.mark.parametrize("rows,cols", SHAPES)
 def test_rms_norm_bwd_x(backend, oracle, rows, cols, with_out):
