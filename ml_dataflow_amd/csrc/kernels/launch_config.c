@@ -250,15 +250,20 @@ static int row_kernel_config(Hip_Launch_Config * cfg, Op * op, const char * name
 	return 0;
 }
 
-int default_rms_norm_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {
-	(void) handle; (void) fn;
-	if (row_kernel_config(cfg, op, "rms_norm")) {
+/* the forward and bwd_x: long launches over short rows have one of them on a wave (NORM_WAVE_ROW_COLS, norm.hip) */
+static int norm_rows_config(Hip_Launch_Config * cfg, Op * op, const char * name) {
+	if (row_kernel_config(cfg, op, name)) {
 		return -1;
 	}
 	if (ARG_INT(op, 1) <= 1024 && ARG_INT(op, 0) >= 8192) {
-		cfg->gridDimX = ((unsigned int) ARG_INT(op, 0) + 3) / 4;          /* rows on one wave each: NORM_WAVE_ROW_COLS, norm.hip */
+		cfg->gridDimX = ((unsigned int) ARG_INT(op, 0) + 3) / 4;
 	}
 	return 0;
+}
+
+int default_rms_norm_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {
+	(void) handle; (void) fn;
+	return norm_rows_config(cfg, op, "rms_norm");
 }
 
 int default_rms_norm_recompute_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {
@@ -268,7 +273,7 @@ int default_rms_norm_recompute_set_launch_config(Hip_Launch_Config * cfg, Datafl
 
 int default_rms_norm_bwd_x_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {
 	(void) handle; (void) fn;
-	return row_kernel_config(cfg, op, "rms_norm_bwd_x");
+	return norm_rows_config(cfg, op, "rms_norm_bwd_x");
 }
 
 /* As many work-groups as the workspace has room for partial rows, at most 512 and at most one per row.

@@ -95,7 +95,7 @@ default_rms_norm_bf16_kernel(int n_rows, int n_cols, float eps, const bf16_t * _
 							 const bf16_t * __restrict__ X, bf16_t * __restrict__ out, float * __restrict__ rms_vals) {
 	__shared__ float scratch[ROW_WAVES];
 	const bool wave_rows = n_cols <= NORM_WAVE_ROW_COLS && n_rows >= NORM_WAVE_ROW_LEAST_ROWS;
-	const int row = wave_rows ? (int) (blockIdx.x * ROW_WAVES + threadIdx.x / WAVE) : (int) blockIdx.x;
+	const int row = wave_rows ? (int) (blockIdx.x * ROW_WAVES) + __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE)) : (int) blockIdx.x;
 	if (row >= n_rows) {
 		return;
 	}
@@ -167,7 +167,7 @@ default_rms_norm_recompute_bf16_kernel(int n_rows, int n_cols, const bf16_t * __
 }
 
 /* Backward w.r.t. the input, accumulated into dX; X_out (nullable) receives the recomputed forward output.
- * Launch: grid = n_rows, block = 256.
+ * Launch: block = 256, grid = n_rows, or a quarter of them for rows on one wave.
  * Algorithmic HBM bytes: 6*n_rows*n_cols read (x, g, dX), 2*n_rows*n_cols written (+2*n_rows*n_cols for X_out).
  *
  * Two forms, by the rows.  A compute unit holds six of the work-groups (80 registers: the row's x, g and dX stay in them), 256 compute units
@@ -237,13 +237,74 @@ rms_norm_bwd_x_row(int n_cols, float r, const u32x4 * __restrict__ x, const u32x
 	}
 }
 
+/* The same for a row on one wave, as in the forward (rms_norm_wave_row), all of its loads out at once.  us, forward, bwd_x
+ * and bwd_w in turn, bwd_x with a row on a work-group and so: 32768 x 512 74.2 and 60.9, 16384 x 960 58.5 and 55.1, 12000 x 1024 49.5 and 47.0, 8192 x
+ * 1024 37.1 and 34.6, 8192 x 576 31.1 and 26.8.  The row's number is made uniform: in vector registers its addresses would take the kernel from 80 to
+ * 91, five work-groups a compute unit (8192 x 4096 104.2 and 106.1). */
+__device__ __forceinline__ void
+rms_norm_bwd_x_wave_row(int n_cols, float r, const u32x4 * __restrict__ x, const u32x4 * __restrict__ g, const u32x4 * __restrict__ w, u32x4 * d, u32x4 * xo) {
+	const int nvec = n_cols >> 3, lane = threadIdx.x & (WAVE - 1);
+	u32x4 qx[NORM_WAVE_ROW_VEC], qg[NORM_WAVE_ROW_VEC], qw[NORM_WAVE_ROW_VEC], qd[NORM_WAVE_ROW_VEC];
+	#pragma unroll
+	for (int j = 0; j < NORM_WAVE_ROW_VEC; j++) {
+		const int v = lane + j * WAVE;
+		if (v < nvec) {
+			qx[j] = x[v];
+			qg[j] = __builtin_nontemporal_load(g + v);
+			qw[j] = w[v];
+			qd[j] = d[v];
+		}
+	}
+	float sum = 0.0f;
+	#pragma unroll
+	for (int j = 0; j < NORM_WAVE_ROW_VEC; j++) {
+		const int v = lane + j * WAVE;
+		if (j * WAVE < nvec) {                           /* uniform */
+			float part = 0.0f;
+			if (v < nvec) {
+				float fx[8], fg[8], fw[8], y[8];
+				unpack8(qx[j], fx);
+				unpack8(qg[j], fg);
+				unpack8(qw[j], fw);
+				#pragma unroll
+				for (int i = 0; i < 8; i++) {
+					y[i] = (fx[i] * r) * fw[i];
+					part = __builtin_fmaf(y[i], fg[i], part);
+				}
+				if (xo) {
+					__builtin_nontemporal_store(pack8(y), xo + v);
+				}
+			}
+			sum += wave_sum(part);
+		}
+	}
+	const float c_div_n = sum / (float) n_cols;
+	#pragma unroll
+	for (int j = 0; j < NORM_WAVE_ROW_VEC; j++) {
+		const int v = lane + j * WAVE;
+		if (v < nvec) {
+			float fx[8], fg[8], fw[8], fd[8];
+			unpack8(qx[j], fx);
+			unpack8(qg[j], fg);
+			unpack8(qw[j], fw);
+			unpack8(qd[j], fd);
+			#pragma unroll
+			for (int i = 0; i < 8; i++) {
+				fd[i] += r * (fg[i] * fw[i] - c_div_n * (fx[i] * r));
+			}
+			__builtin_nontemporal_store(pack8(fd), d + v);
+		}
+	}
+}
+
 extern "C" __global__ void __launch_bounds__(ROW_THREADS)
 default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const float * __restrict__ fwd_rms_vals,
 										const bf16_t * __restrict__ rms_weight, const bf16_t * __restrict__ X_inp,
 										const bf16_t * __restrict__ upstream_dX, bf16_t * dX, bf16_t * X_out) {
 	__shared__ float scratch[ROW_WAVES];
 	(void) eps;
-	const int row = blockIdx.x;
+	const bool wave_rows = n_cols <= NORM_WAVE_ROW_COLS && n_rows >= NORM_WAVE_ROW_LEAST_ROWS;
+	const int row = wave_rows ? (int) (blockIdx.x * ROW_WAVES) + __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE)) : (int) blockIdx.x;
 	if (row >= n_rows) {
 		return;
 	}
@@ -253,7 +314,9 @@ default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 	const u32x4 * w = (const u32x4 *) rms_weight;
 	u32x4 * d = (u32x4 *) (dX + (size_t) row * n_cols);
 	u32x4 * xo = X_out ? (u32x4 *) (X_out + (size_t) row * n_cols) : nullptr;
-	if (n_rows > BWD_X_FEW_ROWS) {
+	if (wave_rows) {
+		rms_norm_bwd_x_wave_row(n_cols, r, x, g, w, d, xo);
+	} else if (n_rows > BWD_X_FEW_ROWS) {
 		rms_norm_bwd_x_row<true>(n_cols, r, x, g, w, d, xo, scratch);
 	} else {
 		rms_norm_bwd_x_row<false>(n_cols, r, x, g, w, d, xo, scratch);
