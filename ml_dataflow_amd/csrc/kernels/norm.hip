@@ -45,8 +45,7 @@ __device__ __forceinline__ u32x4 normed(u32x4 x, u32x4 w, float r) {
  * meets and both loads of x and w are out at once.  The vectors of a lane are those that two of the four waves would have, summed by wave and added in
  * their order: the same bits.  us, over several sets of arrays, a work-group a row and so: 32768 x 512 19.8 and 12.2, 16384 x 960 13.4 and 11.8, 12000 x
  * 1024 11.4 and 9.5, 8192 x 576 7.8 and 6.1, 8192 x 1024 8.7 and 7.7.  From 2048 columns on (8192 rows 12.1 and 12.4) and with fewer rows (3000 x
- * 1600 5.6 and 6.7) rows on a work-group, which spread over more waves, are the faster ones.  Those with their loads in front of the sum, unrolled,
- * took 1-4 % less from 5120 columns on and 4 % more at 2048: 68 registers, seven work-groups a compute unit instead of eight. */
+ * 1600 5.6 and 6.7) rows on a work-group, which spread over more waves, are the faster ones. */
 #define NORM_WAVE_ROW_COLS 1024                          /* launch_config.c has these two as well */
 #define NORM_WAVE_ROW_LEAST_ROWS 8192
 #define NORM_WAVE_ROW_VEC (NORM_WAVE_ROW_COLS / 8 / WAVE)
@@ -88,6 +87,61 @@ __device__ __forceinline__ void rms_norm_wave_row(int n_cols, float eps, const u
 	}
 }
 
+/* Many long rows, one on a work-group: all loads of a lane's first four vectors are out before the first is waited for, those of w in front of the sum's
+ * barriers.  The loop in the kernel below, a round trip to memory a vector twice over, stays for rows of up to 4608 columns, where it is
+ * the faster one (2048 x 2048 4.8 and 5.0 us), and for fewer rows: at 2048 x 8192 this form is the faster one too (11.7 and 11.2), but the three norm
+ * passes together, over arrays that just miss the memory-side cache, took 62.2 and 63.6.  us, that loop and this form: 8192 x 4672 30.9 and
+ * 28.4, 20000 x 5120 75.0 and 71.7, 3000 x 7232 15.5 and 14.5, 2500 x 8192 14.4 and 14.2, 8192 x 8192 52.9 and 47.9, 32768 x 8192 185 and 183, 3000 x 10048 23.3
+ * and 22.2.  62 registers: eight work-groups a compute unit, as before. */
+#define NORM_UNROLLED_COLS 4608
+#define NORM_UNROLLED_LEAST_ROWS 2500
+__device__ __forceinline__ void rms_norm_unrolled_row(int n_cols, float eps, const u32x4 * x, const u32x4 * __restrict__ w, u32x4 * o, float * rms, float * scratch) {
+	const int nvec = n_cols >> 3;
+	u32x4 keep[NORM_MAX_VEC], scale[NORM_MAX_VEC];
+	float part[1] = {0.0f};
+	#pragma unroll
+	for (int j = 0; j < NORM_MAX_VEC; j++) {
+		const int v = threadIdx.x + j * ROW_THREADS;
+		if (v < nvec) {
+			keep[j] = x[v];
+		}
+	}
+	__builtin_amdgcn_sched_barrier(0);                      /* the loads of x are out before the first is waited for */
+	#pragma unroll
+	for (int j = 0; j < NORM_MAX_VEC; j++) {
+		if ((int) (threadIdx.x + j * ROW_THREADS) < nvec) {
+			add_squares(keep[j], part[0]);
+		}
+	}
+	#pragma unroll 1
+	for (int v = threadIdx.x + NORM_MAX_VEC * ROW_THREADS; v < nvec; v += ROW_THREADS) {
+		add_squares(x[v], part[0]);
+	}
+	#pragma unroll
+	for (int j = 0; j < NORM_MAX_VEC; j++) {
+		const int v = threadIdx.x + j * ROW_THREADS;
+		if (v < nvec) {
+			scale[j] = w[v];
+		}
+	}
+	block_sum<1>(part, scratch);
+	const float r = rsqrtf(part[0] * (1.0f / (float) n_cols) + eps);
+	if (threadIdx.x == 0 && rms) {
+		*rms = r;
+	}
+	#pragma unroll
+	for (int j = 0; j < NORM_MAX_VEC; j++) {
+		const int v = threadIdx.x + j * ROW_THREADS;
+		if (v < nvec) {
+			o[v] = normed(keep[j], scale[j], r);
+		}
+	}
+	#pragma unroll 1
+	for (int v = threadIdx.x + NORM_MAX_VEC * ROW_THREADS; v < nvec; v += ROW_THREADS) {
+		o[v] = normed(x[v], w[v], r);
+	}
+}
+
 /* r[row], out = bf16((x * r) * w).  Launch: block = 256, grid = n_rows, or a quarter of them for rows on one wave.
  * Algorithmic HBM bytes: 2*n_rows*n_cols read, 2*n_rows*n_cols + 4*n_rows written (w stays in cache). */
 extern "C" __global__ void __launch_bounds__(ROW_THREADS)
@@ -105,6 +159,10 @@ default_rms_norm_bf16_kernel(int n_rows, int n_cols, float eps, const bf16_t * _
 	const u32x4 * w = (const u32x4 *) rms_weight;
 	if (wave_rows) {
 		rms_norm_wave_row(n_cols, eps, x, w, o, rms_vals ? rms_vals + row : nullptr);
+		return;
+	}
+	if (n_cols > NORM_UNROLLED_COLS && n_rows >= NORM_UNROLLED_LEAST_ROWS) {
+		rms_norm_unrolled_row(n_cols, eps, x, w, o, rms_vals ? rms_vals + row : nullptr, scratch);
 		return;
 	}
 

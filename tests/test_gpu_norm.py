@@ -54,9 +54,10 @@ def test_rms_norm_forward_and_recompute(backend, oracle, rows, cols):
     assert (be.read(d_X.ptr, (rows, cols), np.uint16) == got).all()
 
 
-# rows on one wave, four to a work-group (8192 rows and more of up to 1024 columns), give the bits of rows on a work-group (two calls of half the rows)
-@pytest.mark.parametrize("rows,cols", [(8192, 8), (8193, 64), (8195, 512), (8194, 520), (8192, 1016), (8193, 1024), (8192, 1032)])
-def test_rms_norm_rows_on_a_wave(backend, rows, cols):
+# rows on one wave, four to a work-group (8192 rows and more of up to 1024 columns), and unrolled ones (2500 and more of over 4608) give the bits of rows on a work-group (two calls of half the rows)
+@pytest.mark.parametrize("rows,cols", [(8192, 8), (8193, 64), (8195, 512), (8194, 520), (8192, 1016), (8193, 1024), (8192, 1032),
+                                       (2500, 4608), (2500, 4616), (2501, 8192), (2500, 8200)])
+def test_rms_norm_rows_on_a_wave_and_unrolled(backend, rows, cols):
     print("case rms_norm rows=%d cols=%d" % (rows, cols), flush=True)
     be = backend
     rng = np.random.default_rng(rows * 3 + cols)
