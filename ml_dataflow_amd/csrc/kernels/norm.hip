@@ -12,7 +12,8 @@
  * Sums run over a row (or over rows) in fp32 in an order the reference leaves to its launch shape; results agree
  * within fp32 rounding of the sums.
  *
- * All kernels are bandwidth-bound: one 256-thread work-group per row, 16 bytes per lane per access, the row kept
+ * All kernels are bandwidth-bound: one 256-thread work-group per row (forward and bwd_x: one wave where rows are short
+ * and many), 16 bytes per lane per access, the row kept
  * in registers between the reduction and the second use (rows up to 8192 elements; longer rows are read twice).
  * us, forward, bwd_x with X_out and bwd_w of 8192 x 4096 in turn, 604 MB: 113.3 -> 104.7 (5.8 TB/s): dX loaded with x and g instead of
  * behind the sum 109.6, bwd_x's results stored past the caches 106.8, bwd_w's loads in front of the sums of four rows 104.7.  bwd_x from
