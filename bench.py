@@ -181,7 +181,7 @@ def replay_step_with_events(be, layer, T, d_X, d_out, d_dY, d_dX, d_bias, backwa
         timed("router_gate_bwd_x", lib.dataflow_submit_router_gate_bwd_x, hp, CS, BF, BF, T, E, K, L.chosen_experts, L.token_expert_weights, L.d_routed)
         timed("router_gemm", lib.dataflow_submit_matmul, hp, CS, BF, BF, BF, BF, F32, 0, 0, D, E, T, 1.0, 1.0, L.w_router, L.d_routed, d_dX.ptr, d_dX.ptr,
               L.kernel_workspace_bytes, ws)
-        gathers = fused and lib.amd_moe_layer_backward_gathers(C.byref(L), T, int(first))
+        gathers = fused and lib.amd_moe_layer_backward_gathers(hp, C.byref(L), T, d_X.ptr, int(first))
         if not gathers:
             timed("dispatch", lib.dataflow_submit_default_prepare_experts, hp, CS, BF, BF, T, D, K, d_X.ptr, L.token_mapping, L.expert_zones)
         if gathers:
@@ -820,7 +820,7 @@ def main():
                 tile_rows = ragged_n_tile_rows(rows_m[cls], k_of[cls], counts)
                 if tile_rows != 384:
                     four[cls] = kernel_of_class[cls].replace("288", str(tile_rows))
-        gathers = be.lib.amd_moe_layer_backward_gathers(C.byref(layer.L), T, 0)
+        gathers = be.lib.amd_moe_layer_backward_gathers(be.hp, C.byref(layer.L), T, d_X.ptr, 0)
         for cls, M, N in (("gemm_nt_dw", H, D), ("gemm_dw13", D, 2 * H)):
             if mm.amd_matmul_planned_sliced(M, T * K, N, E, 1, 256):
                 four[cls] = _W4K % ("true, 2, 2" if cls == "gemm_dw13" and gathers else "true, 2, 0")

@@ -142,9 +142,10 @@ int amd_moe_layer_forward(Dataflow_Handle * handle, int compute_stream_id, int s
 int amd_moe_layer_backward(Dataflow_Handle * handle, int compute_stream_id, int secondary_stream_id,
 						   Amd_Moe_Layer * layer, int num_tokens, void * X, void * dY, void * dX, int schedule);
 
-/* 1: the fused backward over that many tokens takes the rows of X for dW1 | dW3 through expert_mapping (w1 and w3 back to back), 0: from a
- * copy in expert_zones.  The same bits either way. */
-int amd_moe_layer_backward_gathers(const Amd_Moe_Layer * layer, int num_tokens, int first_micro_batch);
+/* 1: the fused backward over that many rows of X takes them for dW1 | dW3 through expert_mapping, 0: from a copy in expert_zones.  The same bits
+ * either way.  It gathers where w1 and w3 lie back to back, the ops are those of registration and the matmul says that the launch runs on its sliced
+ * kernel, with the compute units of the handle and the kernel named with amd_matmul_select_kernel (amd_matmul.h). */
+int amd_moe_layer_backward_gathers(Dataflow_Handle * handle, const Amd_Moe_Layer * layer, int num_tokens, void * X, int first_micro_batch);
 
 /* ---- the reference's files, as far as this layer meets them ---- */
 

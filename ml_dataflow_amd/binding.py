@@ -227,7 +227,7 @@ SIGNATURES = {
     "amd_moe_layer_alloc": (_I, [_H, C.POINTER(AmdMoeLayer), _I, _I, _I, _I, _I]),
     "amd_moe_layer_free": (None, [_H, C.POINTER(AmdMoeLayer)]),
     "amd_moe_layer_forward": (_I, [_H, _I, _I, C.POINTER(AmdMoeLayer), _I, _P, _P, _P, _I]),
-    "amd_moe_layer_backward_gathers": (_I, [C.POINTER(AmdMoeLayer), _I, _I]),
+    "amd_moe_layer_backward_gathers": (_I, [_H, C.POINTER(AmdMoeLayer), _I, _P, _I]),
     "amd_moe_layer_backward": (_I, [_H, _I, _I, C.POINTER(AmdMoeLayer), _I, _P, _P, _P, _I]),
     "amd_moe_block_weight_offsets": (_I, [_I, _I, _I, _I, _I, _DT, _I, C.POINTER(AmdMoeBlockOffsets)]),
     "amd_moe_layer_load_block_file": (_I, [_H, _I, C.POINTER(AmdMoeLayer), C.c_char_p, _I, _I, _I, _P]),

@@ -146,6 +146,38 @@ int layer_submit_matmul_twin(Dataflow_Handle * handle, int stream_id, int M, int
 	return submit(handle, &op, stream_id, "twin matmul");
 }
 
+void layer_set_gathers_k_rows_skeleton(Op_Skeleton * skeleton) {
+	const DataflowDatatype t[10] = {DATAFLOW_INT_SCALAR, DATAFLOW_INT_SCALAR, DATAFLOW_INT_SCALAR, DATAFLOW_INT_SCALAR, DATAFLOW_BF16, DATAFLOW_INT_SCALAR, DATAFLOW_BF16,
+									DATAFLOW_BF16, DATAFLOW_BF16, DATAFLOW_UINT64_SCALAR};
+	dataflow_fill_skeleton(skeleton, "amd_gathers_k_rows", DATAFLOW_BF16, DATAFLOW_NONE, 10, t);
+}
+
+static void gathers_k_rows_stood_in(Op_Skeleton skeletons[3]) {
+	dataflow_set_amd_grouped_matmul_gathered_skeleton(&skeletons[0]);
+	dataflow_set_amd_grouped_matmul_skeleton(&skeletons[1]);
+	dataflow_set_default_prepare_experts_skeleton(&skeletons[2], DATAFLOW_BF16, DATAFLOW_BF16);
+}
+
+int layer_bind_gathers_k_rows(Dataflow_Handle * handle) {
+	Op_Skeleton skeleton, of[3];
+	layer_set_gathers_k_rows_skeleton(&skeleton);
+	gathers_k_rows_stood_in(of);
+	return stand_in_bind(handle, &skeleton, of, 3);
+}
+
+int layer_gathers_k_rows(Dataflow_Handle * handle, int model_dim, int num_rows, int stacked_dim, int num_experts, void * X, int num_tokens,
+						 void * dx13, int accumulate, void * dw13, uint64_t expert_stride_bytes) {
+	Op op;
+	Op_Skeleton of[3];
+	layer_set_gathers_k_rows_skeleton(&op.op_skeleton);
+	gathers_k_rows_stood_in(of);
+	void * C = accumulate ? dw13 : NULL;
+	void ** a = op.op_args;
+	a[0] = &model_dim; a[1] = &num_rows; a[2] = &stacked_dim; a[3] = &num_experts; a[4] = &X; a[5] = &num_tokens; a[6] = &dx13; a[7] = &C; a[8] = &dw13;
+	a[9] = &expert_stride_bytes;
+	return stand_in_ask(handle, &op, of, 3);
+}
+
 int layer_submit_route_tokens(Dataflow_Handle * handle, int stream_id, int num_tokens, int num_experts, int top_k, int model_dim,
 							  void * X, void * w_router, void * logit_bias, void * x_routed, float * token_expert_weights,
 							  uint16_t * chosen_experts, int * expert_counts, int * expert_counts_cumsum, int * host_expert_counts,

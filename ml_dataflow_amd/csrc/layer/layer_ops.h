@@ -71,4 +71,12 @@ LAYER_OPS_HIDDEN int layer_has_matmul_twin(Dataflow_Handle * handle);
 LAYER_OPS_HIDDEN int layer_submit_matmul_twin(Dataflow_Handle * handle, int stream_id, int M, int K, int N, float beta, void * A,
 							 void * B1, void * C1, void * D1, void * B2, void * C2, void * D2);
 
+/* dW1 | dW3 of the fused schedule: would the gathered grouped matmul over the rows of X run on the kernel that makes up for the copy it saves
+ * (the sliced one)?  Asked of the library that launches it, with the launch's operands; nothing runs on the device.  dw, if C is read: accumulate.
+ * 0 where it, the grouped matmul or prepare_experts, which the copy + packed form consists of, is not the one of registration. */
+LAYER_OPS_HIDDEN void layer_set_gathers_k_rows_skeleton(Op_Skeleton * skeleton);
+LAYER_OPS_HIDDEN int layer_bind_gathers_k_rows(Dataflow_Handle * handle);
+LAYER_OPS_HIDDEN int layer_gathers_k_rows(Dataflow_Handle * handle, int model_dim, int num_rows, int stacked_dim, int num_experts, void * X, int num_tokens,
+							 void * dx13, int accumulate, void * dw13, uint64_t expert_stride_bytes);
+
 #endif

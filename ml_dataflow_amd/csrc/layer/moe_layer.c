@@ -398,28 +398,28 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 /* ------------------------------------------------------------------ backward */
 
 /* The stacked dW1 | dW3 GEMM can take the k-rows of X through expert_mapping (no re-dispatch), as the up-projection does in the
- * forward.  On the sliced kernel, which finds the rows with a few instructions a slice, that saves the copy and more: X is an eighth
- * of its copies and stays in the memory-side cache (64 groups of 1024 rows, 4096 x 2048 with C, us: packed 1150, gathered 1096, the copy 92; of 8192 rows, X
- * 512 MiB, 7168, 7448 and 913).  Training steps: 8192 tokens, 64 experts, top 8, 4096 x 1024 4878 -> 4823, 65536 36677 -> 35705; 45 drawn ones 0.99-1.03x.
- * It does where that kernel runs (its lines, matmul/amd_matmul.hip, one for both directions of the accumulation), the copy is worth it and the
- * rows are not read again too often: with wide experts each k-row is fetched for every 256 columns of 2H, scattered (expert dims of 1664-2048 0.992-1.002x), and
- * short rows make tiles whose chain of slices is the longer one (dim 576, a Zipf router: 0.947).  On eight waves, with fewer rows, the copy + packed form is
- * the faster one (425 rows an expert 0.982). */
-#define BWD_GATHER_MEAN_ROWS 512
-#define BWD_GATHER_MEAN_ROWS_FIRST 640
+ * forward.  The launch is the slower one for it, also on the sliced kernel, which finds the rows with a few instructions a slice, but by less than the
+ * copy.  In the step, us, the copy, the packed launch behind it and the gathered one: 8192 tokens, 64 experts, top 8, 4096 x 1024 92, 1099 and 1149, in a
+ * first micro-batch 92, 990 and 1059, 65536 tokens 919, 6933 and 7412.  (By itself the launch finds X, an eighth of its copies, in the memory-side
+ * cache: 1150 and 1096.)  Whole steps, both forms in turn on one card: 4845 -> 4792, first 4703 -> 4667, 65536 36012 -> 35430, first 35973 -> 35295; 16
+ * drawn ones of 844-14991 rows an expert, even and Zipf routers, accumulating and first, 0.962-1.009 of the packed form's time, 0.991 in the mean of either
+ * direction.
+ * The matmul itself says whether the launch runs on the sliced kernel (layer_gathers_k_rows); on eight waves a lane waits for its entry of the map, which
+ * costs more than the copy: the steps above, that kernel named, packed and gathered 5327 and 5444, first 5189 and 5333, 38097 and 38855, 37907 and 38714.
+ * Two lines beside that: with wide experts each k-row is fetched for every 256 columns of 2H, scattered (expert dims of 1664-2048 0.998-1.008, of 1536
+ * 0.996-1.007), and short rows make tiles whose chain of slices is the longer one (dim 576, a Zipf router: 1.056). */
 #define BWD_GATHER_LEAST_DIM 1280
 #define BWD_GATHER_MOST_EXPERT_DIM 1536
-int amd_moe_layer_backward_gathers(const Amd_Moe_Layer * L, int T, int first_micro_batch) {
-	const uint64_t rows = (uint64_t) T * L->top_k, E = L->num_experts, D = L->model_dim, H = L->expert_dim;
-	const uint64_t tiles = (D + 255) / 256 * ((2 * H + 255) / 256) * E;
-	if (!gather_allowed(T, L->model_dim)) {
+int amd_moe_layer_backward_gathers(Dataflow_Handle * h, const Amd_Moe_Layer * L, int T, void * X, int first_micro_batch) {
+	const int D = L->model_dim, E = L->num_experts, K = L->top_k, H = L->expert_dim;
+	if (!up_weights_stacked(L) || !gather_allowed(T, D)) {
 		return 0;
 	}
 	if (getenv("AMD_MOE_BWD_GATHER") != NULL) {
 		return 1;
 	}
-	return rows >= (first_micro_batch ? BWD_GATHER_MEAN_ROWS_FIRST : BWD_GATHER_MEAN_ROWS) * E && D >= BWD_GATHER_LEAST_DIM && H <= BWD_GATHER_MOST_EXPERT_DIM
-		&& 2 * H >= 256 && (!first_micro_batch || tiles > 256 || rows >= 2048 * E);
+	return D >= BWD_GATHER_LEAST_DIM && H <= BWD_GATHER_MOST_EXPERT_DIM
+		&& layer_gathers_k_rows(h, D, T * K, 2 * H, E, X, T, L->dx1, !first_micro_batch, L->dw1, L->expert_stride_bytes);
 }
 
 int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L, int T, void * X, void * dY, void * dX, int schedule) {
@@ -596,7 +596,7 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 								 L->kernel_workspace_bytes, L->kernel_workspace), "failed to submit router dX matmul");
 
 	/* bwd_w: re-dispatch the inputs (:4062-4066), dW1 / dW3 (:4101-4148), dWr (:4174-4181) */
-	const int gathered = side_by_side && amd_moe_layer_backward_gathers(L, T, first_micro_batch);
+	const int gathered = side_by_side && amd_moe_layer_backward_gathers(h, L, T, X, first_micro_batch);
 	if (!gathered) {
 		CHECK(dataflow_submit_default_prepare_experts(h, cs, dt, dt, T, D, K, X, L->token_mapping, L->expert_zones), "failed to submit prepare experts (bwd_w)");
 	}

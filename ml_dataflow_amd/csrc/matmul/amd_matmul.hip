@@ -362,6 +362,17 @@ static bool single_wide_is_cheaper(long wide, long narrow, long k_tiles, long cu
 	return wide_rounds * (256 + 384) * (105 * k_tiles + 250) < narrow_rounds * (256 + 256) * (100 * k_tiles + 150);
 }
 
+/* a ragged reduction's operands have their rows packed along k (or gathered): group bases are aligned where M and N are multiples of 8 */
+static bool operand_direct_ok(const void * base, bool kmajor, long rows, long K, long group_stride_elems);
+static bool ragged_k_direct_ok(const GemmParams & p) {
+	return operand_direct_ok(p.A, true, p.M, p.K, 0) && operand_direct_ok(p.B, true, p.N, p.K, 0) && (p.strideD % 4 == 0);
+}
+
+/* whether it runs on the sliced kernel with its k-rows gathered; `tile`: of the launch */
+static bool gathers_on_sliced(const GemmParams & p, bool direct, int tile, long tiles, long cu_count) {
+	return direct && tile == TILE_BIG && w4k_gather_ok(p) && takes_sliced(MODE_RAGGED_K, p, tiles, cu_count);
+}
+
 /* a caller that named one of the persistent kernels gets it wherever it has enough tiles for half the compute units */
 static int tile_of_launch(int mode, const GemmParams & p, long grid_big, long cu_count) {
 	const bool named = kernel_choice != AMD_MATMUL_KERNEL_AUTO && p.M >= 256 && (mode == MODE_RAGGED_N ? (long) p.N / 256 * tiles_of(p.M, 256) : p.N >= 256 ? grid_big : 0) >= 128;
@@ -616,7 +627,7 @@ static int launch_gemm(const GemmParams & p, int transa, int transb, bool direct
 	}
 	if (MODE == MODE_RAGGED_K && p.gather) {
 		/* gathered A: the k-rows of the reduction are fetched through the row map (both operands are k-major here) */
-		if (direct && big && w4k_gather_ok(p) && takes_sliced(MODE, p, grid_big, cu_count)) {
+		if (gathers_on_sliced(p, direct, tile, grid_big, cu_count)) {
 			return launch_w4k<MODE_RAGGED_K, GATHER_P_KROWS>(p, grid_big, cu_count, stream);
 		}
 		if (direct) {
@@ -1202,8 +1213,7 @@ extern "C" int amd_grouped_matmul(Dataflow_Handle * dataflow_handle, int stream_
 			fprintf(stderr, "Error: ragged-K grouped matmul needs to_trans_a == 0 and to_trans_b == 1...\n");
 			return -1;
 		}
-		/* both operands have their rows packed along k: group bases are aligned when M and N are multiples of 8 */
-		const bool direct = operand_direct_ok(p.A, true, p.M, p.K, 0) && operand_direct_ok(p.B, true, p.N, p.K, 0) && (p.strideD % 4 == 0);
+		const bool direct = ragged_k_direct_ok(p);
 		const long grid_big = tiles_of(p.M, 256) * tiles_of(p.N, 256) * p.num_groups;
 		const long grid_small = tiles_of(p.M, 128) * tiles_of(p.N, 128) * p.num_groups;
 		if (p.C == nullptr) {
@@ -1219,6 +1229,31 @@ extern "C" int amd_grouped_matmul(Dataflow_Handle * dataflow_handle, int stream_
 	}
 	fprintf(stderr, "Error: unknown ragged dimension %d...\n", ragged);
 	return -1;
+}
+
+/* The layer's question in front of its dW1 | dW3 (../layer/layer_ops.h), answered by the launch's own rules: 1 where the gathered form runs on
+ * the sliced kernel.  Launches nothing. */
+extern "C" int amd_gathers_k_rows(Dataflow_Handle * dataflow_handle, int stream_id, Op * op, void * op_extra) {
+	(void) dataflow_handle; (void) stream_id;
+	void ** a = op->op_args;
+	GemmParams p;
+	memset(&p, 0, sizeof(p));
+	p.M = *((int *) a[0]);
+	p.K = *((int *) a[1]);
+	p.N = *((int *) a[2]);
+	p.num_groups = *((int *) a[3]);
+	p.A = (const bf16_t *) *((uint64_t *) a[4]);
+	p.gather_rows = *((int *) a[5]);
+	p.B = (const bf16_t *) *((uint64_t *) a[6]);
+	p.C = (const bf16_t *) *((uint64_t *) a[7]);
+	p.beta = p.C ? 1.0f : 0.0f;
+	p.D = (bf16_t *) *((uint64_t *) a[8]);
+	p.strideD = (long long) (*((uint64_t *) a[9]) / 2);
+	if (p.M < 1 || p.N < 1 || p.num_groups < 1 || p.gather_rows < 1) {
+		return 0;
+	}
+	const long cu_count = extra_cu_count(op_extra), tiles = tiles_in_launch(TILE_BIG, MODE_RAGGED_K, p);
+	return gathers_on_sliced(p, ragged_k_direct_ok(p), tile_of_launch(MODE_RAGGED_K, p, tiles, cu_count), tiles, cu_count);
 }
 
 /* The activation behind an up-projection on kernels whose epilogue does not compute it */

@@ -36,3 +36,8 @@ int stand_in_usable(Dataflow_Handle * handle, Op_Skeleton * op, Op_Skeleton * of
 	}
 	return fn != NULL;
 }
+
+int stand_in_ask(Dataflow_Handle * handle, Op * op, Op_Skeleton * of, int n) {
+	const Hip_Function * fn = registered(handle, &op->op_skeleton);
+	return fn && fn->hip_external_func && stand_in_usable(handle, &op->op_skeleton, of, n) ? (fn->hip_external_func)(handle, -1, op, fn->op_extra) : 0;
+}

@@ -14,5 +14,7 @@
 __attribute__((visibility("hidden"))) int stand_in_bind(Dataflow_Handle * handle, Op_Skeleton * op, Op_Skeleton * of, int n);
 /* may `op` be submitted in their place? */
 __attribute__((visibility("hidden"))) int stand_in_usable(Dataflow_Handle * handle, Op_Skeleton * op, Op_Skeleton * of, int n);
+/* asks an external op that answers on the host (what it returns) instead of launching anything; 0 where it may not be used in their place */
+__attribute__((visibility("hidden"))) int stand_in_ask(Dataflow_Handle * handle, Op * op, Op_Skeleton * of, int n);
 
 #endif

@@ -181,6 +181,12 @@ static int register_stand_ins(Dataflow_Handle * handle, const char * dir) {
 		fprintf(stderr, "Error: failed to register the layer's twin matmul, which needs the matmul in the table...\n");
 		return -1;
 	}
+	layer_set_gathers_k_rows_skeleton(&skeleton);
+	symbol = "amd_gathers_k_rows";
+	if ((handle->register_external_code)(handle, path, 1, &skeleton, &symbol, &init_symbol) != 1 || layer_bind_gathers_k_rows(handle)) {
+		fprintf(stderr, "Error: failed to register the layer's question about gathered rows, which needs the grouped matmuls and prepare_experts in the table...\n");
+		return -1;
+	}
 	dataflow_set_amd_rms_norm_bwd_w_few_rows_skeleton(&skeleton);
 	char * kernel = "amd_rms_norm_bwd_w_few_rows_bf16_bf16_kernel", * launch = "amd_rms_norm_bwd_w_few_rows_set_launch_config", * none = NULL;
 	snprintf(path, sizeof(path), "%s/%s", dir, NATIVE_CODE_FILE);

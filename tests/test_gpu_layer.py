@@ -192,8 +192,8 @@ def test_schedules_agree_bit_for_bit(backend, T, D, E, K, H):
 @pytest.mark.parametrize("T,D,E,K,H", [(1024, 512, 16, 4, 384), (4096, 1024, 8, 4, 512)])
 def test_fused_schedule_without_gathered_loads_gives_the_same_bits(backend, T, D, E, K, H):
     """The stacked GEMMs of the fused schedule either fetch the rows of X through expert_mapping in their own loaders or run
-    on a dispatched copy (the up-projection for an X of 4 GiB and more, the dW1 | dW3 GEMM by default); AMD_MOE_BWD_GATHER
-    makes the backward gather too, AMD_MOE_NO_GATHER forces the copy everywhere.  Same values into the same multiplies:
+    on a dispatched copy (the up-projection for an X of 4 GiB and more, the dW1 | dW3 GEMM where amd_moe_layer_backward_gathers answers 0, as it
+    does here); AMD_MOE_BWD_GATHER makes the backward gather all the same, on eight waves and smaller tiles, AMD_MOE_NO_GATHER forces the copy everywhere.  Same values into the same multiplies:
     every output and gradient agrees bit for bit."""
     be = backend
     rng = np.random.default_rng(31)
@@ -219,6 +219,49 @@ def test_fused_schedule_without_gathered_loads_gives_the_same_bits(backend, T, D
             d.free()
     for i, (a, b) in enumerate(zip(*runs)):
         assert (a == b).all(), "output %d differs between the gathered and the packed form" % i
+
+
+# both directions of the accumulation; partial tiles on both sides, experts of uneven rows
+@pytest.mark.parametrize("T,D,E,K,H,first", [(2100, 1296, 8, 2, 520, False), (1301, 1296, 8, 4, 904, False), (1301, 1296, 8, 4, 904, True)])
+def test_rows_gathered_by_default_give_the_bits_of_the_copy(backend, T, D, E, K, H, first):
+    """dW1 | dW3 as the fused backward runs it by itself, where it takes the rows of X through expert_mapping on the sliced kernel, against the copy:
+    an expert without rows, gradients that were there before; with the eight-wave kernel named it is the copy by itself."""
+    print("case gathered by default T=%d D=%d E=%d K=%d H=%d first=%d" % (T, D, E, K, H, first), flush=True)
+    be = backend
+    mm = C.CDLL(os.path.join(B.LIB_DIR, "libamd_matmul.so"))
+    rng = np.random.default_rng(T + E)
+    Wr, W1, W3, W2 = make_weights(rng, D, E, H)
+    X, dY = normal_bf16(rng, (T, D)), normal_bf16(rng, (T, D))
+    bias = normal_bf16(rng, (1, E)).repeat(T, 0)
+    bias[:, 3] = 0xC7C3                                             # -99840: no token takes this expert
+    before = normal_bf16(rng, (E, 2 * H * D), 0.02)
+    layer = MoeLayer(be, T, D, E, K, H)
+    layer.load_weights(Wr, W1, W3, W2)
+    d_X, d_bias, d_out, d_dY, d_dX = be.upload(X), be.upload(bias), be.alloc(T * D * 2), be.upload(dY), be.alloc(T * D * 2)
+    layer.forward(T, d_X.ptr, d_out.ptr, d_bias.ptr, B.AMD_MOE_FUSED)
+    runs = []
+    for name in ("default", "eight waves", "copy"):
+        for e in range(E):
+            be.write(layer.expert_ptr(layer.L.dw1, e), before[e])
+        os.environ.pop("AMD_MOE_NO_GATHER", None)
+        try:
+            if name == "copy":
+                os.environ["AMD_MOE_NO_GATHER"] = "1"
+            if name == "eight waves":
+                assert mm.amd_matmul_select_kernel(8) == 0
+            gathers = be.lib.amd_moe_layer_backward_gathers(be.hp, C.byref(layer.L), T, d_X.ptr, int(first))
+            assert gathers == (name == "default")
+            layer.backward(T, d_X.ptr, d_dY.ptr, d_dX.ptr, B.AMD_MOE_FUSED, first_micro_batch=first)
+            be.sync()
+        finally:
+            os.environ.pop("AMD_MOE_NO_GATHER", None)
+            assert mm.amd_matmul_select_kernel(0) == 0
+        runs.append(np.stack([be.read(layer.expert_ptr(layer.L.dw1, e), (2 * H * D,), np.uint16) for e in range(E)]))
+    layer.free()
+    for d in (d_X, d_bias, d_out, d_dY, d_dX):
+        d.free()
+    assert (runs[0] == runs[2]).all() and (runs[1] == runs[2]).all()
+    assert (runs[2][3] == (0 if first else before[3])).all() and (runs[2][0] != before[0]).mean() > 0.5
 
 
 # one per work-group tile of the fused up-projection (64 x 32, 64 x 64, 64 x 128, 128 x 128 and the persistent kernels with a launch

@@ -154,16 +154,101 @@ def test_the_benchmark_times_the_ops_the_layer_submits(schedule, first):
     assert len(rows) == len(submitted) and all(name in work for name, _ in rows)
 
 
+GATHERING_OPS = ("amd_grouped_matmul_gathered", "amd_grouped_matmul", "default_prepare_experts_BF16_BF16")
+ALIGNED_X = 1 << 32
+AUTO, EIGHT_WAVES, FOUR_WAVES, FOUR_WAVES_384 = 0, 8, 4, 384          # include/amd_matmul.h
+
+
+class AskingHandle(NotingHandle):
+    """with the library's answer about gathered rows in the table, and under the three ops it speaks for what it was registered beside"""
+
+    def __init__(self, matmul):
+        super().__init__(C.sizeof(HipFunction))
+        lib, self.skeletons = self.lib, {}
+        setters = (lib.dataflow_set_amd_grouped_matmul_gathered_skeleton, lib.dataflow_set_amd_grouped_matmul_skeleton,
+                   lambda sk: lib.dataflow_set_default_prepare_experts_skeleton(sk, B.DATAFLOW_BF16, B.DATAFLOW_BF16))
+        for i, (name, setter) in enumerate(zip(GATHERING_OPS, setters)):
+            self.skeletons[name] = B.OpSkeleton()
+            setter(C.byref(self.skeletons[name]))
+            self.insert(name, 0x1000 * (i + 1))
+        answer = self.skeletons["answer"] = B.OpSkeleton()
+        answer.header.op_nickname = b"amd_gathers_k_rows_BF16"
+        answer.header.num_args = 10
+        answer.header.arg_dtypes = (C.c_int * B.MAX_OP_ARGS)(*([B.DATAFLOW_INT_SCALAR] * 4 + [B.DATAFLOW_BF16, B.DATAFLOW_INT_SCALAR] + [B.DATAFLOW_BF16] * 3 + [B.DATAFLOW_UINT64_SCALAR]))
+        assert lib.dataflow_do_fingerprinting(C.byref(answer.header), C.sizeof(answer.header), answer.fingerprint) == 0
+        self.insert("answer", C.cast(matmul.amd_gathers_k_rows, C.c_void_p).value, stands_in_for=(C.c_void_p * 3)(0x1000, 0x2000, 0x3000))
+
+    def insert(self, name, implementation, **fields):
+        native = "prepare" in name
+        fn = HipFunction(op_skeleton=self.skeletons[name], is_native=native, **{"function_handle" if native else "hip_external_func": implementation}, **fields)
+        assert self.lib.dataflow_insert_table(C.byref(self.h.op_table), C.cast(self.skeletons[name].fingerprint, C.c_void_p), C.cast(C.byref(fn), C.c_void_p)) == 0
+
+    def replace(self, name):
+        assert self.lib.dataflow_remove_table(C.byref(self.h.op_table), C.cast(self.skeletons[name].fingerprint, C.c_void_p), None) == 0
+        self.insert(name, 0x5000)
+
+    def gathers(self, layer, tokens, first, X=ALIGNED_X):
+        return self.lib.amd_moe_layer_backward_gathers(C.pointer(self.h), C.byref(layer), tokens, X, first)
+
+
+@pytest.fixture
+def matmul():
+    import os
+    B.load_library()
+    lib = C.CDLL(os.path.join(B.LIB_DIR, "libamd_matmul.so"))
+    yield lib
+    assert lib.amd_matmul_select_kernel(AUTO) == 0
+
+
+def stacked_layer(dim, experts, top_k, hidden):
+    up = 2 * dim * hidden
+    return B.AmdMoeLayer(model_dim=dim, num_experts=experts, top_k=top_k, expert_dim=hidden, dx1=2 << 32, w1=3 << 32, w3=(3 << 32) + up, dw1=4 << 32, dw3=(4 << 32) + up,
+                         expert_stride_bytes=3 * up)
+
+
 @pytest.mark.parametrize("tokens,first,gathers", [(0, False, False), (2047, False, False), (2048, False, True), (2559, True, False), (2560, True, True)])
-def test_the_backward_gathers_where_experts_have_the_rows(tokens, first, gathers):
-    """dim 1280, 8 experts, top 2: the lines are 512 and 640 rows an expert; not with wide experts, narrow rows or an environment that forbids it"""
-    lib = B.load_library()
-    layer = B.AmdMoeLayer(model_dim=1280, num_experts=8, top_k=2, expert_dim=1536)
-    assert lib.amd_moe_layer_backward_gathers(C.byref(layer), tokens, first) == gathers
-    for name, value in (("model_dim", 1272), ("expert_dim", 1544)):
-        other = B.AmdMoeLayer(model_dim=1280, num_experts=8, top_k=2, expert_dim=1536)
-        setattr(other, name, value)
-        assert lib.amd_moe_layer_backward_gathers(C.byref(other), tokens, first) == 0
+def test_the_backward_gathers_where_experts_have_the_rows(matmul, tokens, first, gathers):
+    """dim 1280, 8 experts, top 2: the lines are 512 and 640 rows an expert; not with wide experts, narrow rows, w3 apart from w1, an X off a 16-byte boundary, one of
+    4 GiB or an environment that forbids it"""
+    handle, layer = AskingHandle(matmul), stacked_layer(1280, 8, 2, 1536)
+    assert handle.gathers(layer, tokens, first) == gathers
+    assert handle.gathers(layer, tokens, first, ALIGNED_X + 8) == 0
+    apart = stacked_layer(1280, 8, 2, 1536)
+    apart.w3 += 256
+    for other in (stacked_layer(1272, 8, 2, 1536), stacked_layer(1280, 8, 2, 1544), apart):
+        assert handle.gathers(other, tokens, first) == 0
+    assert handle.gathers(layer, (1 << 32) // 2 // 1280 + 1, first) == 0
+
+
+def test_the_backward_gathers_only_where_the_sliced_kernel_runs(matmul):
+    """over drawn layers, with every kernel a program can name: the answer is that of the launch's own plan, within the layer's two lines"""
+    import random
+    rng, handle, told = random.Random(1), AskingHandle(matmul), {}
+    for _ in range(4000):
+        dim, hidden, experts, top_k = 64 * rng.randint(8, 64), 64 * rng.randint(8, 32), rng.randint(1, 64), rng.randint(1, 8)
+        tokens, first = int(2 ** rng.uniform(8, 16)), rng.random() < 0.5
+        if rng.random() < 0.3:                                          # about a round of tiles: where the lines of one and of more rounds meet
+            experts = max(1, min(64, 256 // (-(-dim // 256) * -(-2 * hidden // 256)) + rng.randint(-1, 1)))
+        if top_k > experts or tokens * dim * 2 > 0xFFFFFFFF:
+            continue
+        for kernel in (AUTO, EIGHT_WAVES, FOUR_WAVES, FOUR_WAVES_384):
+            assert matmul.amd_matmul_select_kernel(kernel) == 0
+            sliced = matmul.amd_matmul_planned_sliced(dim, tokens * top_k, 2 * hidden, experts, int(not first), 256)
+            answer = handle.gathers(stacked_layer(dim, experts, top_k, hidden), tokens, first)
+            assert answer == (sliced and dim >= 1280 and hidden <= 1536), (kernel, tokens, dim, experts, top_k, hidden, first)
+            told[kernel] = told.get(kernel, 0) + answer
+    assert told[AUTO] > 500 and told[FOUR_WAVES_384] > 500 and told[EIGHT_WAVES] == told[FOUR_WAVES] == 0
+
+
+@pytest.mark.parametrize("replaced", [None, *GATHERING_OPS])
+def test_the_gathered_gradient_gives_way_to_a_replaced_op(matmul, replaced):
+    """the rows go through a copy where a program has put its own op in the place of one of the three, and where the table has no answer"""
+    handle, layer = AskingHandle(matmul), stacked_layer(4096, 64, 8, 1024)
+    if replaced:
+        handle.replace(replaced)
+    assert handle.gathers(layer, 8192, False) == (replaced is None)
+    bare = NotingHandle(C.sizeof(HipFunction))
+    assert bare.lib.amd_moe_layer_backward_gathers(C.pointer(bare.h), C.byref(layer), 8192, ALIGNED_X, False) == 0
 
 
 @pytest.mark.parametrize("tokens,dim,streams", [(1024, 4096, {1}), (1025, 4096, {1, 2}), (2048, 2048, {1}), (2049, 1024, {1, 2})])
