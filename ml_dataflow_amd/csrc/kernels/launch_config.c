@@ -8,6 +8,7 @@
  * A grid of 0 tells the handle there is nothing to launch.
  */
 #include "dataflow_amd.h"
+#include "norm_rows.h"
 
 #include <stdint.h>
 #include <stdio.h>
@@ -250,13 +251,13 @@ static int row_kernel_config(Hip_Launch_Config * cfg, Op * op, const char * name
 	return 0;
 }
 
-/* the forward and bwd_x: long launches over short rows have one of them on a wave (NORM_WAVE_ROW_COLS, norm.hip) */
+/* the forward and bwd_x: long launches over short rows have one of them on a wave (norm_rows.h) */
 static int norm_rows_config(Hip_Launch_Config * cfg, Op * op, const char * name) {
 	if (row_kernel_config(cfg, op, name)) {
 		return -1;
 	}
-	if (ARG_INT(op, 1) <= 1024 && ARG_INT(op, 0) >= 8192) {
-		cfg->gridDimX = ((unsigned int) ARG_INT(op, 0) + 3) / 4;
+	if (NORM_ROWS_ON_WAVES(ARG_INT(op, 0), ARG_INT(op, 1))) {
+		cfg->gridDimX = ((unsigned int) ARG_INT(op, 0) + NORM_WAVE_ROWS_PER_GROUP - 1) / NORM_WAVE_ROWS_PER_GROUP;
 	}
 	return 0;
 }

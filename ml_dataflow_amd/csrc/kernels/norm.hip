@@ -20,6 +20,8 @@
  * the last row to the first, for what the memory-side cache holds of x, was no faster (114.3).
  */
 
+#include "norm_rows.h"
+
 #define NORM_MAX_VEC 4
 
 __device__ __forceinline__ void add_squares(u32x4 q, float & sum) {
@@ -47,8 +49,7 @@ __device__ __forceinline__ u32x4 normed(u32x4 x, u32x4 w, float r) {
  * their order: the same bits.  us, over several sets of arrays, a work-group a row and so: 32768 x 512 19.8 and 12.2, 16384 x 960 13.4 and 11.8, 12000 x
  * 1024 11.4 and 9.5, 8192 x 576 7.8 and 6.1, 8192 x 1024 8.7 and 7.7.  From 2048 columns on (8192 rows 12.1 and 12.4) and with fewer rows (3000 x
  * 1600 5.6 and 6.7) rows on a work-group, which spread over more waves, are the faster ones. */
-#define NORM_WAVE_ROW_COLS 1024                          /* launch_config.c has these two as well */
-#define NORM_WAVE_ROW_LEAST_ROWS 8192
+static_assert(NORM_WAVE_ROWS_PER_GROUP == ROW_WAVES, "a row to each wave of a work-group");
 #define NORM_WAVE_ROW_VEC (NORM_WAVE_ROW_COLS / 8 / WAVE)
 __device__ __forceinline__ void rms_norm_wave_row(int n_cols, float eps, const u32x4 * x, const u32x4 * __restrict__ w, u32x4 * o, float * rms) {
 	const int nvec = n_cols >> 3, lane = threadIdx.x & (WAVE - 1);
@@ -149,7 +150,7 @@ extern "C" __global__ void __launch_bounds__(ROW_THREADS)
 default_rms_norm_bf16_kernel(int n_rows, int n_cols, float eps, const bf16_t * __restrict__ rms_weight,
 							 const bf16_t * __restrict__ X, bf16_t * __restrict__ out, float * __restrict__ rms_vals) {
 	__shared__ float scratch[ROW_WAVES];
-	const bool wave_rows = n_cols <= NORM_WAVE_ROW_COLS && n_rows >= NORM_WAVE_ROW_LEAST_ROWS;
+	const bool wave_rows = NORM_ROWS_ON_WAVES(n_rows, n_cols);
 	const int row = wave_rows ? (int) (blockIdx.x * ROW_WAVES) + __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE)) : (int) blockIdx.x;
 	if (row >= n_rows) {
 		return;
@@ -362,7 +363,7 @@ default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 										const bf16_t * __restrict__ upstream_dX, bf16_t * dX, bf16_t * X_out) {
 	__shared__ float scratch[ROW_WAVES];
 	(void) eps;
-	const bool wave_rows = n_cols <= NORM_WAVE_ROW_COLS && n_rows >= NORM_WAVE_ROW_LEAST_ROWS;
+	const bool wave_rows = NORM_ROWS_ON_WAVES(n_rows, n_cols);
 	const int row = wave_rows ? (int) (blockIdx.x * ROW_WAVES) + __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE)) : (int) blockIdx.x;
 	if (row >= n_rows) {
 		return;
