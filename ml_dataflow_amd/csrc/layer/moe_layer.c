@@ -202,9 +202,13 @@ static int stream_wait(Dataflow_Handle * h, int waiter, int signaller) {
  * streams and one: 374 tokens, 28 experts, top 3, 1152 / 576 230 and 184; 590, 25, top 8, 1728 / 512 337 and 298; 551, 32, top 8, 3456 / 896 858 and
  * 828; 25 with an even router between 2^35 and 2^36 multiplies of the stacked up-projection 0-4 % less, beyond 2^36 up to 2.5 % more (4096, 32, top 4, 2048 / 1408 1410 and 1431).
  * With a Zipf router a launch can end in the long tiles of one group, which another hides: 34 steps of up to 2498 tokens 0.3 % more to 10 % less,
- * of 20 with more tokens nine 2-21 % more (40457, 55, top 1, 512 / 1536 2537 and 3221).  No group has more rows than there are tokens. */
+ * of 20 with more tokens nine 2-21 % more (40457, 55, top 1, 512 / 1536 2537 and 3221).  No group has more rows than there are tokens.  An id that the handle does not have
+ * is passed on, to be refused where the streams meet. */
 #define ONE_STREAM_MOST_TOKENS 2048
-static int second_stream(const Amd_Moe_Layer * L, int T, int cs, int ss) {
+static int second_stream(Dataflow_Handle * h, const Amd_Moe_Layer * L, int T, int cs, int ss) {
+	if (h->num_streams > 0 && (ss < 0 || ss >= h->num_streams)) {
+		return ss;
+	}
 	return T <= ONE_STREAM_MOST_TOKENS && (uint64_t) T * L->top_k * 2 * L->expert_dim * L->model_dim <= LAYER_UP_SWIGLU_GROUPED_MULTIPLIES ? cs : ss;
 }
 
@@ -317,7 +321,7 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 		} else {
 			CHECK(dataflow_submit_default_prepare_experts(h, cs, dt, dt, T, D, K, X, L->token_mapping, L->expert_zones), "failed to submit prepare experts");
 			/* The two up-projections are independent (second_stream) */
-			const int second = second_stream(L, T, cs, ss);
+			const int second = second_stream(h, L, T, cs, ss);
 			CHECK(stream_wait(h, second, cs), "secondary stream could not wait for the compute stream");
 			CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, DATAFLOW_NONE, dt, cdt, 1, 0, AMD_GROUPED_RAGGED_N, H, D, T * K,
 													 E, L->expert_counts_cumsum, 1.0f, 0.0f, L->w1, L->expert_stride_bytes, L->expert_zones, NULL, L->x1, 0),
@@ -509,7 +513,7 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 		/* dW2 += g^T h (:3548-3555) and dh = g W2 (:3568-3575).  The reference writes dh over h, which orders the two;
 		 * here dh goes to the dx1 buffer (swiglu_bwd_x then works in place: it reads an element of dh before it writes
 		 * that element of dx1), so the two GEMMs are independent (second_stream). */
-		const int second = second_stream(L, T, cs, ss);
+		const int second = second_stream(h, L, T, cs, ss);
 		CHECK(stream_wait(h, second, cs), "secondary stream could not wait for the compute stream");
 		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, H, T * K, D, E, cum,
 												 1.0f, wbeta, temp, 0, L->expert_zones, WGRAD_C(L->dw2), L->dw2, S), "failed to submit grouped dW2 matmul");
@@ -610,7 +614,7 @@ int amd_moe_layer_backward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * 
 												 1.0f, wbeta, L->expert_zones, 0, L->dx1, WGRAD_C(L->dw1), L->dw1, S), "failed to submit grouped dW1|dW3 matmul");
 	} else if (schedule != AMD_MOE_PER_EXPERT) {
 		/* independent of each other, as the up-projections */
-		const int second = second_stream(L, T, cs, ss);
+		const int second = second_stream(h, L, T, cs, ss);
 		CHECK(stream_wait(h, second, cs), "secondary stream could not wait for the compute stream");
 		CHECK(dataflow_submit_amd_grouped_matmul(h, cs, dt, dt, wc_dt, dt, cdt, 0, 1, AMD_GROUPED_RAGGED_K, D, T * K, H, E, L->expert_counts_cumsum,
 												 1.0f, wbeta, L->expert_zones, 0, L->dx1, WGRAD_C(L->dw1), L->dw1, S), "failed to submit grouped dW1 matmul");

@@ -268,6 +268,20 @@ def test_small_grouped_passes_stay_on_one_stream(tokens, dim, streams):
     assert set(used) == streams and len(met) == (4 if len(streams) > 1 else 0)
 
 
+def test_small_grouped_passes_refuse_a_secondary_stream_that_is_none():
+    """they submit nothing to it, but an id the handle does not have stays an error, as in a large pass"""
+    noting = NotingHandle()
+    noting.h.num_streams = 3
+    refuse = dict(B.DataflowHandle._fields_)["submit_dependency"](lambda handle, stream, state: 0 if 0 <= stream < 3 else -1)
+    noting.h.submit_dependency = refuse
+    for tokens in (16, 4096):
+        layer = noting.layer(max_tokens=tokens, model_dim=4096, expert_dim=1024, num_experts=64, top_k=8, expert_stride_bytes=6 * 4096 * 1024)
+        for secondary, answer in ((2, 0), (3, -1), (-1, -1)):
+            args = (C.pointer(noting.h), 1, secondary, C.byref(layer), tokens, 1 << 32)
+            assert noting.lib.amd_moe_layer_forward(*args, None, 2 << 32, B.AMD_MOE_GROUPED) == answer
+            assert noting.lib.amd_moe_layer_backward(*args, 2 << 32, 3 << 32, B.AMD_MOE_GROUPED) == answer
+
+
 UP_OPS = ["amd_grouped_matmul_gathered", "amd_swiglu_strided_BF16"]
 
 
