@@ -404,10 +404,10 @@ int amd_moe_layer_forward(Dataflow_Handle * h, int cs, int ss, Amd_Moe_Layer * L
 /* The stacked dW1 | dW3 GEMM can take the k-rows of X through expert_mapping (no re-dispatch), as the up-projection does in the
  * forward.  The launch is the slower one for it, also on the sliced kernel, which finds the rows with a few instructions a slice, but by less than the
  * copy.  In the step, us, the copy, the packed launch behind it and the gathered one: 8192 tokens, 64 experts, top 8, 4096 x 1024 92, 1099 and 1149, in a
- * first micro-batch 92, 990 and 1059, 65536 tokens 919, 6933 and 7412.  (By itself the launch finds X, an eighth of its copies, in the memory-side
- * cache: 1150 and 1096.)  Whole steps, both forms in turn on one card: 4845 -> 4792, first 4703 -> 4667, 65536 36012 -> 35430, first 35973 -> 35295; 16
- * drawn ones of 844-14991 rows an expert, even and Zipf routers, accumulating and first, 0.962-1.009 of the packed form's time, 0.991 in the mean of either
- * direction.
+ * first micro-batch 92, 990 and 1059, 65536 tokens 919, 6933 and 7412.  (By itself the gathered launch is the faster one, 1150 and 1096: the likely cause,
+ * not measured, is that it then finds X, an eighth of its copies, in the memory-side cache.)  Whole steps, both forms in turn on one card: 4845 -> 4792,
+ * first 4703 -> 4667, 65536 tokens 36012 -> 35430, first 35973 -> 35295; 16 drawn ones of 844-14991 rows an expert, even and Zipf routers, accumulating and
+ * first, 0.962-1.009 of the packed form's time, 0.991 in the mean of either direction.
  * The matmul itself says whether the launch runs on the sliced kernel (layer_gathers_k_rows); on eight waves a lane waits for its entry of the map, which
  * costs more than the copy: the steps above, that kernel named, packed and gathered 5327 and 5444, first 5189 and 5333, 38097 and 38855, 37907 and 38714.
  * Two lines beside that: with wide experts each k-row is fetched for every 256 columns of 2H, scattered (expert dims of 1664-2048 0.998-1.008, of 1536

@@ -186,7 +186,11 @@ extern "C" int amd_matmul_planned_tile(int M, int K, int N, int has_c, int cu_co
  * so and at 5.3 with plain loads (whole arrays in order: 7.1 and 6.25).  Forwards, us: 16 tokens, 64 experts, top 8, 4096 x 1024 258 -> 229; 50 tokens, 42 experts,
  * 3584 x 1600 287 -> 253; 4 tokens, 43 experts, 1792 x 1216 61 -> 55.  A group with more tiles of rows keeps plain loads (712 tokens dealt to 35 experts by a Zipf
  * router, non-temporal throughout: 104 -> 118), and so do launches whose weights are few enough to be found in the 256 MiB memory-side cache
- * (7 tokens, 55 experts, top 2, 512 x 1472, over three sets of weights: 32.4 -> 33.7; over fourteen 37.8 -> 34.5). */
+ * (7 tokens, 55 experts, top 2, 512 x 1472, over three sets of weights: 32.4 -> 33.7; over fourteen 37.8 -> 34.5).
+ * The line is drawn for a program whose layers together have more weights than the cache holds.  Forwards of 16 tokens over many layers and over one
+ * in a loop, us: 16 experts, 2048 x 1024 (192 MiB in all, 128 in the launch) 61.4 -> 55.0 and 46.0 -> 52.9, 24 (288 and 192) 75.9 -> 68.3 and 68.6 -> 67.2, 32 (384 and 256)
+ * 89.7 -> 81.0 and 89.2 -> 79.4; 32 experts, 1024 x 1024 52.4 -> 47.2 and 42.9 -> 45.0; 64 tokens, 32, 2048 x 768 79.5 -> 72.2 and 67.3 -> 72.1.  So a single layer of 72 to
+ * some 290 MiB that is run again and again loses 5-15 % by it, and from there on nothing is found in the cache either way. */
 #define STREAM_WEIGHTS_BYTES (48u << 20)
 static bool streams_weights(const GemmParams & p) {
 	return (uint64_t) (p.N < p.num_groups ? p.N : p.num_groups) * (uint64_t) p.M * (uint64_t) p.K * 2u > STREAM_WEIGHTS_BYTES;
@@ -351,9 +355,10 @@ static bool takes_sliced(int mode, const GemmParams & p, long tiles, long cu_cou
 /* A single problem without C, whose tiles are known here: `wide` tiles of 256 x 384 against `narrow` ones of 256 x 256 on the eight-wave kernel.  A
  * round costs the bytes of its k-tiles and a part of its own, a last round that is not full, as fewer work-groups share the card's power and
  * memory, a half (wide: seven tenths) and the rest by its share.  Over 260 problems beside the 170 of the fit, M 512-8192, K 128-4096, N 1024-32768,
- * half of them such that the prices disagree, the choice is 0.1 % behind the better one, at worst 3.6 %.  Whole rounds at the prices of
- * the ragged launches were 1.6 % behind (3200 x 3456 x 22783, 3.05 rounds of 384: 5 % slower on them; K 128 in less than a round: 16 % faster), at those
- * prices before the epilogue was generated 1.3 %. */
+ * half of them such that the prices disagree, the choice was 0.1 % behind the better one, at worst 3.6 %, when a partial round of 384 went out in whole
+ * tiles.  In pieces (W4DWalk) it costs less than these prices say: over 260 drawn problems, M 512-8192, K 128-4096, N 1024-32768, the choice is 0.6 %
+ * behind, in 16 of them more than 3 %, each time 256 where 384 would be the faster one with a last round that is half full or less (2432 x 3712 x 20930, 2.15
+ * rounds, 322 us and 281, 5184 x 384 x 6808, 1.48, 40 and 35).  Whole rounds at the prices of the ragged launches were 1.6 % behind before that. */
 static bool single_wide_is_cheaper(long wide, long narrow, long k_tiles, long cu_count) {
 	const long groups = (cu_count & ~7L) < 8 ? 8 : cu_count & ~7L;
 	const long wide_left = wide % groups, narrow_left = narrow % groups;
@@ -481,11 +486,15 @@ static int cheapest_tiling(const GemmParams & p, long groups, bool four_ok, int 
  * rows IN_ONE group: of the others the one that leaves the smaller of the worst cases.  The sizes are on the device, whose
  * work-groups then agree on one of the two from the real sizes (ragged_n_choice).  A launch that loses costs 3 us, so both
  * go out only there.  Over 310 launches of the layer's kind (8-64 experts, 30-9000 rows each, K 512-4096) with even groups one launch on
- * the expected tiling takes 1.9 % longer than the best of all tilings; up to three launches, among them 288 always,
+ * the expected tiling took 1.9 % longer than the best of all tilings; up to three launches, among them 288 always,
  * took 4.7 %.  A first training step of 3001 tokens, 32 experts, dim 2048 934 -> 905 us, a forward of 8192 tokens 635 -> 632, one with
  * a Zipf router, whose launches take a second tiling, unchanged.  Over 341 launches whose rows lie in one, two or four of 8-64 experts to 95 % or are dealt by Zipf routers, this
- * rule is 3.4 % behind the best, without the second list 4.8 %, up to three launches 6.8 %; 17 / 41 of them are more than 3 % slower
+ * rule was 3.4 % behind the best, without the second list 4.8 %, up to three launches 6.8 %; 17 / 41 of them were more than 3 % slower
  * than those three launches and 4 / 27 more than 8 % (1024 x 3072, 41 groups, 6205 of 6478 rows in one: 90 / 136 us, on 288 alone 87).
+ * All these with tiles of 384 that took as long as full ones.  With that kernel's short tiles and pieces, which the prices do not know, over 212 launches
+ * of the same ranges that reach these kernels: even rows 2.7 % behind the best tiling (at worst 18), Zipf routers 2.1 (21), 95 % in one group 2.6 (22),
+ * nearly always for another tiling where 384 is the faster one by now (44 groups of 236 rows, 1024 x 3968: 130 us on 288, 110 on 384); 384
+ * throughout 2.4, 2.1 and 2.3 (39, 55 and 28).
  * As a second tiling beside another one 384 is charged 4 to 8 % more from 1024 k on (its price before its epilogue was generated): at its own
  * price the up-projections of 32 groups of 512 rows, 1408 x 2048, went out on two tilings, and a grouped training step of 4096 tokens took 1405 us
  * instead of 1389.  Where 384 is the first, UNEVEN compares at its own price: 18 launches to which the surcharge added 288 take, rows
@@ -1434,7 +1443,7 @@ extern "C" int amd_route_tokens(Dataflow_Handle * dataflow_handle, int stream_id
 	if (r.T <= ROUTE_SMALL_TOKENS && r.T * lanes <= ROUTE_SMALL_THREADS && (long) r.T * r.E * (r.splits > 1 ? r.splits : 1) <= ROUTE_SMALL_PARTIALS) {
 		int threads = (r.T * lanes + WAVE - 1) / WAVE * WAVE;
 		/* The logits are added up by all its waves, four experts of a token each, before the selection's have work: a wave for every 64 of
-		 * those up to eight waves, and sixteen waves from 2048 on.  us, as many as the selection has and so: 32 tokens, 52 experts, top 2 8.1 and 7.0,
+		 * those up to eight waves, and sixteen waves beyond 2048.  us, as many as the selection has and so: 32 tokens, 52 experts, top 2 8.1 and 7.0,
 		 * 68, 38 and 4 14.2 and 9.7, 256, 64 and 2 17.7 and 13.7; sixteen at 68 tokens 11.0. */
 		const long sums = r.T * tiles_of(r.E < ROUTE_CHUNK ? r.E : ROUTE_CHUNK, 4);
 		const long wanted = sums > 2048 ? ROUTE_SMALL_THREADS : sums > 512 ? 512 : sums < 256 ? 256 : tiles_of(sums, WAVE) * WAVE;

@@ -231,8 +231,9 @@ __device__ __forceinline__ long count_tiles(const GemmParams & p) {
 /* Which tiling of the token rows is cheapest for this launch.  A launch takes (rounds of tiles over the work-groups) x
  * (time of a tile), and a k-tile step is paced by the bytes it fetches: 256 + 288 rows against 256 + 384 rows of 128
  * bytes, the larger tile at 5 % less per byte plus what 2 k-tiles take per tile.  Over 48 launches of 32 and 64 groups of 300-1500 rows
- * dealt at random, K of 1024-4096, timed on both, the rule's choice is 0.1 % behind the better one (3 % more per byte and 1.6 k-tiles,
- * which held before that kernel's epilogue was generated, 0.6 %, up to 10).  us on 288 and 384: 32 groups of 1024 rows, 2816 x 2048, 348
+ * dealt at random, K of 1024-4096, timed on both, the rule's choice was 0.1 % behind the better one, when every tile took as long as a full one.
+ * The prices still are those of full tiles and full rounds, although a group's last tile and a partial last round cost the 384 tiling less since
+ * (w4d_blocks, W4DWalk): ragged_n_tilings has what that leaves behind.  us on 288 and 384 then: 32 groups of 1024 rows, 2816 x 2048, 348
  * and 330, of 1500, 2048 x 2816, 501 and 456, 64 groups of 1500, 1024 x 4096, 727 and 657, of 512 259 and 276.
  * The 384 tiling wins where the groups are long enough to fill its tiles and the rounds come out even; with short or very uneven groups the narrower tiles waste less.  Tiles of 224 and 192 rows serve the
  * sizes between: 32 groups of 430 rows, 1408 x 2048, take 85 us in two rounds of 224 and 97 in two of 288; 170 rows
