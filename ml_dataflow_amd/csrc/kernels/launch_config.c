@@ -251,20 +251,32 @@ static int row_kernel_config(Hip_Launch_Config * cfg, Op * op, const char * name
 	return 0;
 }
 
-/* the forward and bwd_x: long launches over short rows have one of them on a wave (norm_rows.h) */
-static int norm_rows_config(Hip_Launch_Config * cfg, Op * op, const char * name) {
+/* four rows to a work-group (norm_rows.h); a lane holds the row's vectors in registers */
+static int wave_rows_config(Hip_Launch_Config * cfg, Op * op, const char * name) {
 	if (row_kernel_config(cfg, op, name)) {
 		return -1;
 	}
-	if (NORM_ROWS_ON_WAVES(ARG_INT(op, 0), ARG_INT(op, 1))) {
-		cfg->gridDimX = ((unsigned int) ARG_INT(op, 0) + NORM_WAVE_ROWS_PER_GROUP - 1) / NORM_WAVE_ROWS_PER_GROUP;
+	if (ARG_INT(op, 1) > NORM_WAVE_ROW_COLS) {
+		fprintf(stderr, "Error: %s with a row on a wave takes up to %d columns, got %d...\n", name, NORM_WAVE_ROW_COLS, ARG_INT(op, 1));
+		return -1;
 	}
+	cfg->gridDimX = ((unsigned int) ARG_INT(op, 0) + NORM_WAVE_ROWS_PER_GROUP - 1) / NORM_WAVE_ROWS_PER_GROUP;
 	return 0;
+}
+
+int amd_rms_norm_wave_rows_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {
+	(void) handle; (void) fn;
+	return wave_rows_config(cfg, op, "rms_norm");
+}
+
+int amd_rms_norm_bwd_x_wave_rows_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {
+	(void) handle; (void) fn;
+	return wave_rows_config(cfg, op, "rms_norm_bwd_x");
 }
 
 int default_rms_norm_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {
 	(void) handle; (void) fn;
-	return norm_rows_config(cfg, op, "rms_norm");
+	return row_kernel_config(cfg, op, "rms_norm");
 }
 
 int default_rms_norm_recompute_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {
@@ -274,7 +286,7 @@ int default_rms_norm_recompute_set_launch_config(Hip_Launch_Config * cfg, Datafl
 
 int default_rms_norm_bwd_x_set_launch_config(Hip_Launch_Config * cfg, Dataflow_Handle * handle, Hip_Function * fn, Op * op) {
 	(void) handle; (void) fn;
-	return norm_rows_config(cfg, op, "rms_norm_bwd_x");
+	return row_kernel_config(cfg, op, "rms_norm_bwd_x");
 }
 
 /* As many work-groups as the workspace has room for partial rows, at most 512 and at most one per row.

@@ -46,8 +46,8 @@ __device__ __forceinline__ u32x4 normed(u32x4 x, u32x4 w, float r) {
 
 /* A row of up to 1024 columns on one wave.  On a work-group such a row keeps two of its waves idle or more, and all four meet twice for a sum; here nothing
  * meets and both loads of x and w are out at once.  The vectors of a lane are those that two of the four waves would have, summed by wave and added in
- * their order: the same bits.  us, over several sets of arrays, a work-group a row and so: 32768 x 512 19.8 and 12.2, 16384 x 960 13.4 and 11.8, 12000 x
- * 1024 11.4 and 9.5, 8192 x 576 7.8 and 6.1, 8192 x 1024 8.7 and 7.7.  From 2048 columns on (8192 rows 12.1 and 12.4) and with fewer rows (3000 x
+ * their order: the same bits.  us, over sets of arrays beyond the caches, a work-group a row and so: 32768 x 512 26.7 and 14.4, 12000 x 1024 15.0 and 12.5,
+ * 8192 x 576 10.2 and 7.0, 8192 x 1024 11.1 and 8.2.  From 2048 columns on (8192 rows 12.1 and 12.4) and with fewer rows (3000 x
  * 1600 5.6 and 6.7) rows on a work-group, which spread over more waves, are the faster ones. */
 static_assert(NORM_WAVE_ROWS_PER_GROUP == ROW_WAVES, "a row to each wave of a work-group");
 #define NORM_WAVE_ROW_VEC (NORM_WAVE_ROW_COLS / 8 / WAVE)
@@ -66,6 +66,9 @@ __device__ __forceinline__ void rms_norm_wave_row(int n_cols, float eps, const u
 			scale[j] = w[lane + j * WAVE];
 		}
 	}
+	/* one wait for all of them: in the branches below it would be for the stores in front as well (100000 x 256 31.5 and 28.5 us) */
+	static_assert(NORM_WAVE_ROW_VEC == 2, "the vectors named here");
+	asm volatile("" : "+v"(keep[0]), "+v"(keep[1]), "+v"(scale[0]), "+v"(scale[1]));
 	float sum = 0.0f;
 	#pragma unroll
 	for (int j = 0; j < NORM_WAVE_ROW_VEC; j++) {
@@ -95,8 +98,6 @@ __device__ __forceinline__ void rms_norm_wave_row(int n_cols, float eps, const u
  * passes together, over arrays that just miss the memory-side cache, took 62.2 and 63.6.  us, that loop and this form: 8192 x 4672 30.9 and
  * 28.4, 20000 x 5120 75.0 and 71.7, 3000 x 7232 15.5 and 14.5, 2500 x 8192 14.4 and 14.2, 8192 x 8192 52.9 and 47.9, 32768 x 8192 185 and 183, 3000 x 10048 23.3
  * and 22.2.  62 registers: eight work-groups a compute unit, as before. */
-#define NORM_UNROLLED_COLS 4608
-#define NORM_UNROLLED_LEAST_ROWS 2500
 __device__ __forceinline__ void rms_norm_unrolled_row(int n_cols, float eps, const u32x4 * x, const u32x4 * __restrict__ w, u32x4 * o, float * rms, float * scratch) {
 	const int nvec = n_cols >> 3;
 	u32x4 keep[NORM_MAX_VEC], scale[NORM_MAX_VEC];
@@ -144,14 +145,13 @@ __device__ __forceinline__ void rms_norm_unrolled_row(int n_cols, float eps, con
 	}
 }
 
-/* r[row], out = bf16((x * r) * w).  Launch: block = 256, grid = n_rows, or a quarter of them for rows on one wave.
+/* r[row], out = bf16((x * r) * w).  Launch: grid = n_rows, block = 256.
  * Algorithmic HBM bytes: 2*n_rows*n_cols read, 2*n_rows*n_cols + 4*n_rows written (w stays in cache). */
 extern "C" __global__ void __launch_bounds__(ROW_THREADS)
 default_rms_norm_bf16_kernel(int n_rows, int n_cols, float eps, const bf16_t * __restrict__ rms_weight,
 							 const bf16_t * __restrict__ X, bf16_t * __restrict__ out, float * __restrict__ rms_vals) {
 	__shared__ float scratch[ROW_WAVES];
-	const bool wave_rows = NORM_ROWS_ON_WAVES(n_rows, n_cols);
-	const int row = wave_rows ? (int) (blockIdx.x * ROW_WAVES) + __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE)) : (int) blockIdx.x;
+	const int row = blockIdx.x;
 	if (row >= n_rows) {
 		return;
 	}
@@ -159,14 +159,6 @@ default_rms_norm_bf16_kernel(int n_rows, int n_cols, float eps, const bf16_t * _
 	const u32x4 * x = (const u32x4 *) (X + (size_t) row * n_cols);
 	u32x4 * o = (u32x4 *) (out + (size_t) row * n_cols);
 	const u32x4 * w = (const u32x4 *) rms_weight;
-	if (wave_rows) {
-		rms_norm_wave_row(n_cols, eps, x, w, o, rms_vals ? rms_vals + row : nullptr);
-		return;
-	}
-	if (n_cols > NORM_UNROLLED_COLS && n_rows >= NORM_UNROLLED_LEAST_ROWS) {
-		rms_norm_unrolled_row(n_cols, eps, x, w, o, rms_vals ? rms_vals + row : nullptr, scratch);
-		return;
-	}
 
 	u32x4 keep[NORM_MAX_VEC];
 	float part[1] = {0.0f};
@@ -201,6 +193,32 @@ default_rms_norm_bf16_kernel(int n_rows, int n_cols, float eps, const bf16_t * _
 	}
 }
 
+/* The two forms are kernels of their own, submitted in the place of the one above (../ops/dataflow_ops.c, norm_rows.h).  As branches of it their two tests,
+ * a dozen scalar instructions in front of a row's first load, made every other launch the slower one: us, without and with them, 26970 x 1344 33.5 and
+ * 34.6, 9000 x 1344 13.9 and 14.3, 8000 x 1024 11.1 and 11.5, 8192 x 4096 26.0 and 26.2, 20000 x 3072 47.0 and 47.5 (one test costs nothing, the
+ * cheapest arrangement of two 0.1-2.6 %; the 62 registers of the long form cost it nothing).  Launch: block = 256, grid = a quarter of n_rows, rounded up,
+ * and n_rows. */
+extern "C" __global__ void __launch_bounds__(ROW_THREADS)
+amd_rms_norm_wave_rows_bf16_kernel(int n_rows, int n_cols, float eps, const bf16_t * __restrict__ rms_weight,
+								   const bf16_t * __restrict__ X, bf16_t * __restrict__ out, float * __restrict__ rms_vals) {
+	const int row = (int) (blockIdx.x * ROW_WAVES) + __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE));
+	if (row < n_rows) {
+		rms_norm_wave_row(n_cols, eps, (const u32x4 *) (X + (size_t) row * n_cols), (const u32x4 *) rms_weight, (u32x4 *) (out + (size_t) row * n_cols),
+						  rms_vals ? rms_vals + row : nullptr);
+	}
+}
+
+extern "C" __global__ void __launch_bounds__(ROW_THREADS)
+amd_rms_norm_long_rows_bf16_kernel(int n_rows, int n_cols, float eps, const bf16_t * __restrict__ rms_weight,
+								   const bf16_t * __restrict__ X, bf16_t * __restrict__ out, float * __restrict__ rms_vals) {
+	__shared__ float scratch[ROW_WAVES];
+	const int row = blockIdx.x;
+	if (row < n_rows) {
+		rms_norm_unrolled_row(n_cols, eps, (const u32x4 *) (X + (size_t) row * n_cols), (const u32x4 *) rms_weight, (u32x4 *) (out + (size_t) row * n_cols),
+							  rms_vals ? rms_vals + row : nullptr, scratch);
+	}
+}
+
 /* out = bf16((x * r) * w) with r read from rms_vals.  Launch: grid = n_rows, block = 256. */
 extern "C" __global__ void __launch_bounds__(ROW_THREADS)
 default_rms_norm_recompute_bf16_kernel(int n_rows, int n_cols, const bf16_t * __restrict__ rms_weight,
@@ -227,7 +245,7 @@ default_rms_norm_recompute_bf16_kernel(int n_rows, int n_cols, const bf16_t * __
 }
 
 /* Backward w.r.t. the input, accumulated into dX; X_out (nullable) receives the recomputed forward output.
- * Launch: block = 256, grid = n_rows, or a quarter of them for rows on one wave.
+ * Launch: grid = n_rows, block = 256.
  * Algorithmic HBM bytes: 6*n_rows*n_cols read (x, g, dX), 2*n_rows*n_cols written (+2*n_rows*n_cols for X_out).
  *
  * Two forms, by the rows.  A compute unit holds six of the work-groups (80 registers: the row's x, g and dX stay in them), 256 compute units
@@ -297,10 +315,9 @@ rms_norm_bwd_x_row(int n_cols, float r, const u32x4 * __restrict__ x, const u32x
 	}
 }
 
-/* The same for a row on one wave, as in the forward (rms_norm_wave_row), all of its loads out at once.  us, forward, bwd_x
- * and bwd_w in turn, bwd_x with a row on a work-group and so: 32768 x 512 74.2 and 60.9, 16384 x 960 58.5 and 55.1, 12000 x 1024 49.5 and 47.0, 8192 x
- * 1024 37.1 and 34.6, 8192 x 576 31.1 and 26.8.  The row's number is made uniform: in vector registers its addresses would take the kernel from 80 to
- * 91, five work-groups a compute unit (8192 x 4096 104.2 and 106.1). */
+/* The same for a row on one wave, as in the forward (rms_norm_wave_row), all of its loads out at once.  us, over sets of arrays beyond the caches, a row on
+ * a work-group and so: 32768 x 512 41.0 and 29.3, 12000 x 1024 24.2 and 23.3, 8192 x 576 14.8 and 11.4, 8192 x 1024 18.4 and 17.1.  The row's number is made uniform: its
+ * addresses stay in scalar registers. */
 __device__ __forceinline__ void
 rms_norm_bwd_x_wave_row(int n_cols, float r, const u32x4 * __restrict__ x, const u32x4 * __restrict__ g, const u32x4 * __restrict__ w, u32x4 * d, u32x4 * xo) {
 	const int nvec = n_cols >> 3, lane = threadIdx.x & (WAVE - 1);
@@ -363,8 +380,7 @@ default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 										const bf16_t * __restrict__ upstream_dX, bf16_t * dX, bf16_t * X_out) {
 	__shared__ float scratch[ROW_WAVES];
 	(void) eps;
-	const bool wave_rows = NORM_ROWS_ON_WAVES(n_rows, n_cols);
-	const int row = wave_rows ? (int) (blockIdx.x * ROW_WAVES) + __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE)) : (int) blockIdx.x;
+	const int row = blockIdx.x;
 	if (row >= n_rows) {
 		return;
 	}
@@ -374,12 +390,23 @@ default_rms_norm_bwd_x_bf16_bf16_kernel(int n_rows, int n_cols, float eps, const
 	const u32x4 * w = (const u32x4 *) rms_weight;
 	u32x4 * d = (u32x4 *) (dX + (size_t) row * n_cols);
 	u32x4 * xo = X_out ? (u32x4 *) (X_out + (size_t) row * n_cols) : nullptr;
-	if (wave_rows) {
-		rms_norm_bwd_x_wave_row(n_cols, r, x, g, w, d, xo);
-	} else if (n_rows > BWD_X_FEW_ROWS) {
+	if (n_rows > BWD_X_FEW_ROWS) {
 		rms_norm_bwd_x_row<true>(n_cols, r, x, g, w, d, xo, scratch);
 	} else {
 		rms_norm_bwd_x_row<false>(n_cols, r, x, g, w, d, xo, scratch);
+	}
+}
+
+/* a row on a wave, in a kernel of its own, as in the forward; launch: grid = a quarter of n_rows, block = 256 */
+extern "C" __global__ void __launch_bounds__(ROW_THREADS)
+amd_rms_norm_bwd_x_wave_rows_bf16_bf16_kernel(int n_rows, int n_cols, const float * __restrict__ fwd_rms_vals,
+											  const bf16_t * __restrict__ rms_weight, const bf16_t * __restrict__ X_inp,
+											  const bf16_t * __restrict__ upstream_dX, bf16_t * dX, bf16_t * X_out) {
+	const int row = (int) (blockIdx.x * ROW_WAVES) + __builtin_amdgcn_readfirstlane((int) (threadIdx.x / WAVE));
+	if (row < n_rows) {
+		const size_t at = (size_t) row * n_cols;
+		rms_norm_bwd_x_wave_row(n_cols, fwd_rms_vals[row], (const u32x4 *) (X_inp + at), (const u32x4 *) (upstream_dX + at), (const u32x4 *) rms_weight,
+								(u32x4 *) (dX + at), X_out ? (u32x4 *) (X_out + at) : nullptr);
 	}
 }
 

@@ -9,6 +9,7 @@
  */
 #include "dataflow_amd_ops.h"
 #include "skeletons.h"
+#include "../kernels/norm_rows.h"
 #include "stand_in.h"
 
 #include <pthread.h>
@@ -522,11 +523,49 @@ int dataflow_submit_amd_swiglu_strided(Dataflow_Handle * handle, int stream_id, 
 
 /* ---- RMS norm wrappers (libdataflowops/src/submit_ops/norm_ops.c:3-120) ---- */
 
+void dataflow_set_amd_rms_norm_form_skeleton(Op_Skeleton * skeleton, int form) {
+	const DataflowDatatype fwd[7] = {I_S, I_S, F_S, DATAFLOW_BF16, DATAFLOW_BF16, DATAFLOW_BF16, DATAFLOW_FP32};
+	const DataflowDatatype bwd[8] = {I_S, I_S, DATAFLOW_FP32, DATAFLOW_BF16, DATAFLOW_BF16, DATAFLOW_BF16, DATAFLOW_BF16, DATAFLOW_BF16};
+	if (form == NORM_FORM_BWD_X_WAVE_ROWS) {
+		fill_skeleton(skeleton, "amd_rms_norm_bwd_x_wave_rows", DATAFLOW_BF16, DATAFLOW_BF16, 8, bwd);
+	} else if (form == NORM_FORM_LONG_ROWS) {
+		fill_skeleton(skeleton, "amd_rms_norm_long_rows", DATAFLOW_BF16, DATAFLOW_NONE, 7, fwd);
+	} else {
+		fill_skeleton(skeleton, "amd_rms_norm_wave_rows", DATAFLOW_BF16, DATAFLOW_NONE, 7, fwd);
+	}
+}
+
+static void norm_form_stood_in(Op_Skeleton * of, int form) {
+	if (form == NORM_FORM_BWD_X_WAVE_ROWS) {
+		dataflow_set_default_rms_norm_bwd_x_skeleton(of, DATAFLOW_BF16, DATAFLOW_BF16);
+	} else {
+		dataflow_set_default_rms_norm_skeleton(of, DATAFLOW_BF16);
+	}
+}
+
+int dataflow_bind_amd_rms_norm_form(Dataflow_Handle * handle, int form) {
+	Op_Skeleton op, of;
+	dataflow_set_amd_rms_norm_form_skeleton(&op, form);
+	norm_form_stood_in(&of, form);
+	return stand_in_bind(handle, &op, &of, 1);
+}
+
+/* 1, and the form's skeleton in `skeleton`, where it may be submitted */
+static int norm_form_usable(Dataflow_Handle * handle, Op_Skeleton * skeleton, int form) {
+	Op_Skeleton of;
+	dataflow_set_amd_rms_norm_form_skeleton(skeleton, form);
+	norm_form_stood_in(&of, form);
+	return stand_in_usable(handle, skeleton, &of, 1);
+}
+
 int dataflow_submit_default_rms_norm(Dataflow_Handle * handle, int stream_id, DataflowDatatype fwd_dt,
 									 int n_rows, int n_cols, float eps,
 									 void * rms_weight, void * X, void * out, float * rms_vals) {
 	Op op;
-	dataflow_set_default_rms_norm_skeleton(&op.op_skeleton, fwd_dt);
+	const int form = NORM_ROWS_ON_WAVES(n_rows, n_cols) ? NORM_FORM_WAVE_ROWS : NORM_LONG_ROWS(n_rows, n_cols) ? NORM_FORM_LONG_ROWS : -1;
+	if (form < 0 || fwd_dt != DATAFLOW_BF16 || !norm_form_usable(handle, &op.op_skeleton, form)) {
+		dataflow_set_default_rms_norm_skeleton(&op.op_skeleton, fwd_dt);
+	}
 	void ** a = op.op_args;
 	a[0] = &n_rows; a[1] = &n_cols; a[2] = &eps; a[3] = &rms_weight; a[4] = &X; a[5] = &out; a[6] = &rms_vals;
 	return submit(handle, &op, stream_id, "rms norm");
@@ -547,8 +586,13 @@ int dataflow_submit_default_rms_norm_bwd_x(Dataflow_Handle * handle, int stream_
 										   int n_rows, int n_cols, float eps, float * fwd_rms_vals,
 										   void * rms_weight, void * X_inp, void * upstream_dX, void * dX, void * X_out) {
 	Op op;
-	dataflow_set_default_rms_norm_bwd_x_skeleton(&op.op_skeleton, fwd_dt, bwd_dt);
 	void ** a = op.op_args;
+	if (NORM_ROWS_ON_WAVES(n_rows, n_cols) && fwd_dt == DATAFLOW_BF16 && bwd_dt == DATAFLOW_BF16
+		&& norm_form_usable(handle, &op.op_skeleton, NORM_FORM_BWD_X_WAVE_ROWS)) {
+		a[0] = &n_rows; a[1] = &n_cols; a[2] = &fwd_rms_vals; a[3] = &rms_weight; a[4] = &X_inp; a[5] = &upstream_dX; a[6] = &dX; a[7] = &X_out;
+		return submit(handle, &op, stream_id, "rms norm bwd x (rows on waves)");
+	}
+	dataflow_set_default_rms_norm_bwd_x_skeleton(&op.op_skeleton, fwd_dt, bwd_dt);
 	a[0] = &n_rows; a[1] = &n_cols; a[2] = &eps; a[3] = &fwd_rms_vals; a[4] = &rms_weight; a[5] = &X_inp;
 	a[6] = &upstream_dX; a[7] = &dX; a[8] = &X_out;
 	return submit(handle, &op, stream_id, "rms norm bwd x");

@@ -12,4 +12,9 @@ __attribute__((visibility("hidden"))) void dataflow_fill_skeleton(Op_Skeleton * 
 __attribute__((visibility("hidden"))) void dataflow_set_amd_rms_norm_bwd_w_few_rows_skeleton(Op_Skeleton * skeleton);
 __attribute__((visibility("hidden"))) int dataflow_bind_amd_rms_norm_bwd_w_few_rows(Dataflow_Handle * handle);
 
+/* the norm over short rows, one on a wave, and over long ones (dataflow_submit_default_rms_norm and its bwd_x submit them, kernels/norm_rows.h) */
+enum { NORM_FORM_WAVE_ROWS, NORM_FORM_LONG_ROWS, NORM_FORM_BWD_X_WAVE_ROWS, NORM_FORMS };
+__attribute__((visibility("hidden"))) void dataflow_set_amd_rms_norm_form_skeleton(Op_Skeleton * skeleton, int form);
+__attribute__((visibility("hidden"))) int dataflow_bind_amd_rms_norm_form(Dataflow_Handle * handle, int form);
+
 #endif

@@ -187,12 +187,27 @@ static int register_stand_ins(Dataflow_Handle * handle, const char * dir) {
 		fprintf(stderr, "Error: failed to register the layer's question about gathered rows, which needs the grouped matmuls and prepare_experts in the table...\n");
 		return -1;
 	}
-	dataflow_set_amd_rms_norm_bwd_w_few_rows_skeleton(&skeleton);
-	char * kernel = "amd_rms_norm_bwd_w_few_rows_bf16_bf16_kernel", * launch = "amd_rms_norm_bwd_w_few_rows_set_launch_config", * none = NULL;
+	/* the norm's own: its forms, and behind them its weight gradient over few rows */
+	enum { N = NORM_FORMS + 1 };
+	char * kernels[N] = {"amd_rms_norm_wave_rows_bf16_kernel", "amd_rms_norm_long_rows_bf16_kernel", "amd_rms_norm_bwd_x_wave_rows_bf16_bf16_kernel",
+						 "amd_rms_norm_bwd_w_few_rows_bf16_bf16_kernel"};
+	char * launches[N] = {"amd_rms_norm_wave_rows_set_launch_config", "default_rms_norm_set_launch_config", "amd_rms_norm_bwd_x_wave_rows_set_launch_config",
+						  "amd_rms_norm_bwd_w_few_rows_set_launch_config"};
+	char * none[N] = {NULL};
+	Op_Skeleton norms[N];
+	for (int form = 0; form < NORM_FORMS; form++) {
+		dataflow_set_amd_rms_norm_form_skeleton(&norms[form], form);
+	}
+	dataflow_set_amd_rms_norm_bwd_w_few_rows_skeleton(&norms[NORM_FORMS]);
 	snprintf(path, sizeof(path), "%s/%s", dir, NATIVE_CODE_FILE);
 	snprintf(config_lib, sizeof(config_lib), "%s/%s", dir, NATIVE_CONFIG_LIB);
-	if ((handle->register_native_code)(handle, path, config_lib, 1, &skeleton, &kernel, &launch, &none) != 1 || dataflow_bind_amd_rms_norm_bwd_w_few_rows(handle)) {
-		fprintf(stderr, "Error: failed to register the norm's weight gradient over few rows, which needs rms_norm_bwd_w and its combine in the table...\n");
+	int bound = (handle->register_native_code)(handle, path, config_lib, N, norms, kernels, launches, none) == N
+		&& dataflow_bind_amd_rms_norm_bwd_w_few_rows(handle) == 0;
+	for (int form = 0; form < NORM_FORMS && bound; form++) {
+		bound = dataflow_bind_amd_rms_norm_form(handle, form) == 0;
+	}
+	if (!bound) {
+		fprintf(stderr, "Error: failed to register the norm over short, long and few rows, which needs rms_norm, its bwd_x, bwd_w and combine in the table...\n");
 		return -1;
 	}
 	return 0;

@@ -230,21 +230,22 @@ def test_missing_artifacts_fail_loudly(monkeypatch, tmp_path):
         B.load_library()
 
 
-@pytest.mark.parametrize("op", ["default_rms_norm", "default_rms_norm_bwd_x"])
-def test_the_norms_grid_follows_the_kernels_rule_for_rows_on_waves(op):
-    """the host's grid and the kernel's choice of a row come from one definition (kernels/norm_rows.h), and the grid holds every row"""
+@pytest.mark.parametrize("op,on_waves", [("default_rms_norm", False), ("default_rms_norm_bwd_x", False), ("amd_rms_norm_wave_rows", True), ("amd_rms_norm_bwd_x_wave_rows", True)])
+def test_the_norms_grid_holds_every_row(op, on_waves):
+    """the limits of rows on waves are in one place (kernels/norm_rows.h), a row that a wave cannot hold is refused, and the grid has a place for each"""
     kernels = os.path.join(ROOT, "ml_dataflow_amd", "csrc", "kernels")
     rule = {name: int(value) for name, value in re.findall(r"#define (NORM_WAVE_\w+) (\d+)\n", open(os.path.join(kernels, "norm_rows.h")).read())}
     cols, least, per_group = (rule[name] for name in ("NORM_WAVE_ROW_COLS", "NORM_WAVE_ROW_LEAST_ROWS", "NORM_WAVE_ROWS_PER_GROUP"))
     for name in ("norm.hip", "launch_config.c"):
         text = open(os.path.join(kernels, name)).read()
-        assert '#include "norm_rows.h"' in text and "NORM_ROWS_ON_WAVES(" in text
-        assert not re.search(r"#define\s+NORM_WAVE_ROW_(COLS|LEAST_ROWS)\b", text)
+        assert '#include "norm_rows.h"' in text and not re.search(r"#define\s+NORM_WAVE_ROW_(COLS|LEAST_ROWS)\b", text)
     set_config = getattr(C.CDLL(os.path.join(B.LIB_DIR, "libhip_kernels_config.so")), op + "_set_launch_config")
     for n_rows in (0, 1, least - 1, least, least + 1, least + per_group, 2 ** 31 - 1):
         for n_cols in (8, cols - 8, cols, cols + 8):
             rows, width, launch, op_args = C.c_int(n_rows), C.c_int(n_cols), (C.c_uint * 16)(), B.Op()
             op_args.op_args[0], op_args.op_args[1] = C.addressof(rows), C.addressof(width)
+            if on_waves and n_cols > cols:
+                assert set_config(C.byref(launch), None, None, C.byref(op_args)) == -1
+                continue
             assert set_config(C.byref(launch), None, None, C.byref(op_args)) == 0
-            on_waves = n_cols <= cols and n_rows >= least
             assert launch[0] == (-(-n_rows // per_group) if on_waves else n_rows) and launch[3] == 64 * per_group

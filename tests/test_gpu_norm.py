@@ -169,7 +169,7 @@ def test_rms_norm_bwd_w_rows_in_fours_and_one_by_one(backend, rows, cols):
 @pytest.mark.parametrize("rows,cols", [(1536, 64), (1536, 4104), (1536, 8200), (1537, 64), (1537, 2056), (1537, 8192), (1537, 8200), (1800, 6152),
                                        (8192, 8), (8193, 64), (8195, 512), (8194, 520), (8193, 1024), (8192, 1032)])
 def test_rms_norm_bwd_x_with_few_rows_and_more(backend, rows, cols, with_out):
-    """Up to 1536 rows, beyond and 8192 rows of up to 1024 columns, one on a wave, are three forms of one kernel: a row's result has the same
+    """Up to 1536 rows and beyond are two forms of one kernel, 8192 rows of up to 1024 columns, one on a wave, have their own: a row's result has the same
     bits from each.  The first 700 rows alone run on the first form, and so do all 1536."""
     print("case rms_norm_bwd_x forms rows=%d cols=%d out=%d" % (rows, cols, with_out), flush=True)
     be = backend

@@ -430,6 +430,53 @@ def test_the_norms_weight_gradient_over_few_rows_gives_way_to_a_replaced_half(re
     assert submit(1537) == NORM_OPS and submit(0) == NORM_OPS and submit(16, 300) == NORM_OPS
 
 
+NORM_FORMS = {"amd_rms_norm_wave_rows_BF16": [B.DATAFLOW_INT_SCALAR] * 2 + [B.DATAFLOW_FP32_SCALAR] + [B.DATAFLOW_BF16] * 3 + [B.DATAFLOW_FP32],
+              "amd_rms_norm_bwd_x_wave_rows_BF16_BF16": [B.DATAFLOW_INT_SCALAR] * 2 + [B.DATAFLOW_FP32] + [B.DATAFLOW_BF16] * 5}
+NORM_FORMS["amd_rms_norm_long_rows_BF16"] = NORM_FORMS["amd_rms_norm_wave_rows_BF16"]
+
+
+@pytest.mark.parametrize("replaced", [False, True])
+def test_the_norms_forms_by_rows_and_columns_and_only_beside_what_they_stand_in_for(replaced):
+    """a row on a wave from 8192 rows of up to 1024 columns on, long rows from 2500 of over 4608 columns on (forward), the op itself elsewhere, in another
+    type, and everywhere where the table has another implementation under it or none of the forms"""
+    noting = NotingHandle(C.sizeof(HipFunction))
+    lib, hp, forward, bwd_x = noting.lib, C.pointer(noting.h), B.OpSkeleton(), B.OpSkeleton()
+    lib.dataflow_set_default_rms_norm_skeleton(C.byref(forward), B.DATAFLOW_BF16)
+    lib.dataflow_set_default_rms_norm_bwd_x_skeleton(C.byref(bwd_x), B.DATAFLOW_BF16, B.DATAFLOW_BF16)
+
+    def insert(skeleton, implementation, stands_in_for=None):
+        fn = HipFunction(op_skeleton=skeleton, is_native=True, function_handle=implementation, stands_in_for=(C.c_void_p * 3)(stands_in_for, None, None))
+        assert lib.dataflow_insert_table(C.byref(noting.h.op_table), C.cast(skeleton.fingerprint, C.c_void_p), C.cast(C.byref(fn), C.c_void_p)) == 0
+
+    def submitted(rows, cols, dt=B.DATAFLOW_BF16):
+        noting.names.clear()
+        assert lib.dataflow_submit_default_rms_norm(hp, 1, dt, rows, cols, 1e-5, 1 << 24, 2 << 24, 3 << 24, 4 << 24) == 0
+        assert lib.dataflow_submit_default_rms_norm_bwd_x(hp, 1, dt, dt, rows, cols, 1e-5, 4 << 24, 1 << 24, 2 << 24, 3 << 24, 5 << 24, None) == 0
+        return tuple(noting.names)
+
+    plain = ("default_rms_norm_BF16", "default_rms_norm_bwd_x_BF16_BF16")
+    insert(forward, 0x1000)
+    insert(bwd_x, 0x2000)
+    assert submitted(8192, 1024) == submitted(2500, 4616) == plain
+    for name, tags in NORM_FORMS.items():
+        form = B.OpSkeleton()
+        form.header.op_nickname, form.header.num_args = name.encode(), len(tags)
+        form.header.arg_dtypes = (C.c_int * B.MAX_OP_ARGS)(*tags)
+        assert lib.dataflow_do_fingerprinting(C.byref(form.header), C.sizeof(form.header), form.fingerprint) == 0
+        insert(form, 0x3000, 0x2000 if "bwd_x" in name else 0x1000)
+    if replaced:
+        for skeleton in (forward, bwd_x):
+            assert lib.dataflow_remove_table(C.byref(noting.h.op_table), C.cast(skeleton.fingerprint, C.c_void_p), None) == 0
+            insert(skeleton, 0x5000)
+    waves = plain if replaced else ("amd_rms_norm_wave_rows_BF16", "amd_rms_norm_bwd_x_wave_rows_BF16_BF16")
+    long_rows = plain if replaced else ("amd_rms_norm_long_rows_BF16", plain[1])
+    assert submitted(8192, 1024) == submitted(8192, 8) == submitted(1 << 20, 1024) == waves
+    assert submitted(2500, 4616) == submitted(65536, 16384) == long_rows
+    for rows, cols in ((8191, 1024), (8192, 1032), (0, 64), (1, 8), (2499, 4616), (2500, 4608), (8192, 4096)):
+        assert submitted(rows, cols) == plain
+    assert submitted(8192, 512, B.DATAFLOW_FP16)[0] == "default_rms_norm_FP16"
+
+
 @pytest.mark.gpu
 def test_gpu_replaced_select_experts_is_the_one_that_runs():
     """registration notes the real implementations; the op sequence takes over when one of them is exchanged for the same
