@@ -76,10 +76,10 @@ static int launch_staged(const GemmParams & p, long grid, hipStream_t stream) {
 }
 
 /* direct-to-LDS kernel: static LDS */
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PK, bool QK, int MODE, int GATHER = GATHER_NONE, bool SWIGLU = false>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PK, bool QK, int MODE, int GATHER = GATHER_NONE, bool SWIGLU = false, bool ONCE = false>
 static int launch_direct_tile(const GemmParams & p, long grid, hipStream_t stream) {
 	constexpr int threads = WAVES_M * WAVES_N * 64;
-	hipLaunchKernelGGL((gemm_bf16_direct_kernel<BM, BN, WAVES_M, WAVES_N, PK, QK, MODE, GATHER, STAGES, SWIGLU>), dim3((unsigned int) ((grid + 7) & ~7L)), dim3(threads), 0, stream, p);
+	hipLaunchKernelGGL((gemm_bf16_direct_kernel<BM, BN, WAVES_M, WAVES_N, PK, QK, MODE, GATHER, STAGES, SWIGLU, ONCE>), dim3((unsigned int) ((grid + 7) & ~7L)), dim3(threads), 0, stream, p);
 	return check_launch();
 }
 
@@ -190,23 +190,38 @@ extern "C" int amd_matmul_planned_tile(int M, int K, int N, int has_c, int cu_co
  * The line is drawn for a program whose layers together have more weights than the cache holds.  Forwards of 16 tokens over many layers and over one
  * in a loop, us: 16 experts, 2048 x 1024 (192 MiB in all, 128 in the launch) 61.4 -> 55.0 and 46.0 -> 52.9, 24 (288 and 192) 75.9 -> 68.3 and 68.6 -> 67.2, 32 (384 and 256)
  * 89.7 -> 81.0 and 89.2 -> 79.4; 32 experts, 1024 x 1024 52.4 -> 47.2 and 42.9 -> 45.0; 64 tokens, 32, 2048 x 768 79.5 -> 72.2 and 67.3 -> 72.1.  So a single layer of 72 to
- * some 290 MiB that is run again and again loses 5-15 % by it, and from there on nothing is found in the cache either way. */
+ * some 290 MiB that is run again and again loses 5-15 % by it, and from there on nothing is found in the cache either way.
+ * It is another instance of the kernel, with a copy of the loop for each kind of load: a choice between two copies that no group of a launch needs cost it
+ * about 1 % (900 tokens, 8 experts, top 2, 1024 x 1024 51.8 -> 52.4, 1624, 23, 2, 3328 x 512 137.7 -> 138.8).  So it is taken only where the mean group has no
+ * more rows than a tile: over 44 drawn forwards, 27 of them so, even and Zipf routers, 0.88-1.00 of the time without (two of 14 and 24 tokens, whose few experts stay in
+ * the cache, 1.05), the others 1.00, and no Zipf router with more rows gained by it (0.996-1.005). */
 #define STREAM_WEIGHTS_BYTES (48u << 20)
-static bool streams_weights(const GemmParams & p) {
-	return (uint64_t) (p.N < p.num_groups ? p.N : p.num_groups) * (uint64_t) p.M * (uint64_t) p.K * 2u > STREAM_WEIGHTS_BYTES;
+static bool streams_weights(const GemmParams & p, int tile_rows) {
+	const long filled = p.N < p.num_groups ? p.N : p.num_groups;
+	return p.N <= tile_rows * filled && (uint64_t) filled * (uint64_t) p.M * (uint64_t) p.K * 2u > STREAM_WEIGHTS_BYTES;
+}
+
+/* one tile of the direct kernel, with or without them */
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PK, bool QK, int MODE, int GATHER, bool SWIGLU>
+static int launch_direct_either(const GemmParams & p, long grid, hipStream_t stream) {
+	if constexpr (MODE == MODE_RAGGED_N) {
+		if (streams_weights(p, BN)) {
+			return launch_direct_tile<BM, BN, WAVES_M, WAVES_N, STAGES, PK, QK, MODE, GATHER, SWIGLU, true>(p, grid, stream);
+		}
+	}
+	return launch_direct_tile<BM, BN, WAVES_M, WAVES_N, STAGES, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
 }
 
 /* the direct kernel on one of its tiles */
 template <bool PK, bool QK, int MODE, int GATHER = GATHER_NONE, bool SWIGLU = false>
-static int launch_direct(GemmParams p, int which, hipStream_t stream, int problems = 1) {
+static int launch_direct(const GemmParams & p, int which, hipStream_t stream, int problems = 1) {
 	const long grid = grid_of(which, MODE, p) * problems;
-	p.stream_weights = MODE == MODE_RAGGED_N && streams_weights(p);
 	switch (which) {
-		case TILE_64x32: return launch_direct_tile<64, 32, 2, 2, 4, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
-		case TILE_64x64: return launch_direct_tile<64, 64, 2, 2, 4, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
-		case TILE_64x128: return launch_direct_tile<64, 128, 2, 2, 3, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
-		case TILE_128x128: return launch_direct_tile<128, 128, 4, 2, 3, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
-		default: return launch_direct_tile<128, 128, 4, 2, 2, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
+		case TILE_64x32: return launch_direct_either<64, 32, 2, 2, 4, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
+		case TILE_64x64: return launch_direct_either<64, 64, 2, 2, 4, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
+		case TILE_64x128: return launch_direct_either<64, 128, 2, 2, 3, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
+		case TILE_128x128: return launch_direct_either<128, 128, 4, 2, 3, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
+		default: return launch_direct_either<128, 128, 4, 2, 2, PK, QK, MODE, GATHER, SWIGLU>(p, grid, stream);
 	}
 }
 

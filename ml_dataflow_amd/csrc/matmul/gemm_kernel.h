@@ -83,8 +83,6 @@ struct GemmParams {
 	 * (those past them read as zero, like the padding they are multiplied with) */
 	int pitchA, pitchB;
 	int k_rows;
-	/* ragged N on the direct kernel: the weights of groups with one tile of rows are loaded non-temporally (streams_weights) */
-	int stream_weights;
 	/* a second single problem of the same shape and A behind the first, on the direct kernel (NULL D_twin: none) */
 	const bf16_t * B_twin;
 	const bf16_t * C_twin;
@@ -1120,8 +1118,9 @@ __device__ __forceinline__ void store_swiglu_tile(const Tile & t, const GemmPara
  * us with 64 x 64 tiles and four; eight stages leave room for one work-group per compute unit and lose what they gain).
  * Two stages where two work-groups of a compute unit hide each other's waits (the host's table of tiles).
  * SWIGLU: the first half of a tile's rows of P are rows of w1, the second half the same rows of w3 (GemmParams::h); a lane's two
- * loads of P per k-tile are then M / 2 rows apart. */
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool P_KMAJOR, bool Q_KMAJOR, int MODE, int GATHER = 0, int STAGES = 2, bool SWIGLU = false>
+ * loads of P per k-tile are then M / 2 rows apart.
+ * ONCE: the weights of groups with one tile of rows are loaded non-temporally (ragged N; the host's streams_weights). */
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool P_KMAJOR, bool Q_KMAJOR, int MODE, int GATHER = 0, int STAGES = 2, bool SWIGLU = false, bool ONCE = false>
 __global__ void __launch_bounds__(WAVES_M * WAVES_N * 64)
 gemm_bf16_direct_kernel(GemmParams p) {
 	static_assert(STAGES >= 2 && STAGES <= 8, "at least two stages");
@@ -1269,8 +1268,9 @@ gemm_bf16_direct_kernel(GemmParams p) {
 			}
 		}
 	};
-	if constexpr (MODE == MODE_RAGGED_N) {
-		if (p.stream_weights && t.N <= BN) {           /* the group's rows fit one tile: each line of its weights goes to one work-group */
+	if constexpr (ONCE) {
+		static_assert(MODE == MODE_RAGGED_N, "the groups' weights are streamed");
+		if (t.N <= BN) {                               /* the group's rows fit one tile: each line of its weights goes to one work-group */
 			multiply(std::true_type());
 		} else {
 			multiply(std::false_type());

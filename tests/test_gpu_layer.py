@@ -265,9 +265,9 @@ def test_rows_gathered_by_default_give_the_bits_of_the_copy(backend, T, D, E, K,
 
 
 # one per work-group tile of the fused up-projection (64 x 32, 64 x 64, 64 x 128, 128 x 128 and the persistent kernels with a launch
-# behind), expert dims on and off half a tile, k tails, groups without rows
+# behind), expert dims on and off half a tile, k tails, groups without rows, weights that are loaded non-temporally (last)
 @pytest.mark.parametrize("T,D,E,K,H", [(1, 64, 2, 1, 8), (7, 72, 3, 2, 24), (40, 136, 5, 3, 56), (100, 256, 4, 2, 136), (256, 512, 8, 2, 1024),
-                                       (700, 64, 4, 2, 1000), (640, 200, 8, 4, 1000), (3000, 64, 3, 1, 1000), (1141, 256, 8, 2, 1792)])
+                                       (700, 64, 4, 2, 1000), (640, 200, 8, 4, 1000), (3000, 64, 3, 1, 1000), (1141, 256, 8, 2, 1792), (40, 1032, 16, 2, 1024)])
 def test_up_projection_with_its_activation_gives_the_bits_of_the_two_ops(backend, T, D, E, K, H):
     """x1 | x3, h and the output of the op that does both, against the dispatched copy, the GEMM and the activation as three ops
     (AMD_MOE_NO_GATHER); x1 reaches several hundred, where exp overflows and underflows."""
@@ -298,7 +298,7 @@ def test_up_projection_with_its_activation_gives_the_bits_of_the_two_ops(backend
 
 
 @pytest.mark.parametrize("T,D,E,K,H", [(1, 64, 2, 1, 8), (7, 72, 3, 2, 24), (40, 136, 5, 3, 56), (100, 256, 4, 2, 136), (256, 512, 8, 2, 1024),
-                                       (700, 64, 4, 2, 1000), (640, 200, 8, 4, 1000), (1200, 96, 2, 2, 1664), (6000, 64, 3, 2, 1792)])
+                                       (700, 64, 4, 2, 1000), (640, 200, 8, 4, 1000), (1200, 96, 2, 2, 1664), (6000, 64, 3, 2, 1792), (40, 1032, 16, 2, 1024)])
 def test_up_projections_apart_in_one_op_give_the_bits_of_the_separate_ones(backend, T, D, E, K, H):
     """x1, x3, h and the output of the grouped schedule with its up-projections and activation as one op and op by op
     (AMD_MOE_NO_GATHER), and of the per-expert schedule, whose experts take that op each; those of the last sizes are beyond its limit"""

@@ -103,6 +103,7 @@ FEW_ROWS = {
     "32": [0, 1, 31, 32, 33, 2, 16, 64, 65, 0, 30, 7, 32, 31, 5, 1],
     "64": [63, 64, 65, 1, 0, 32, 33, 128, 129, 60, 64, 63, 40, 90, 50, 64],
     "128": [127, 128, 129, 255, 256, 257, 0, 1, 100, 128, 127, 140, 90, 120, 128, 110],
+    "128 in the mean": [127, 128, 129, 1, 0, 100, 128, 127, 90, 120, 128, 110, 64, 257, 126, 3],
 }
 
 
@@ -110,7 +111,7 @@ FEW_ROWS = {
 @pytest.mark.parametrize("transa", [1, 0])
 @pytest.mark.parametrize("name", sorted(FEW_ROWS))
 def test_streamed_weights_bit_identical(backend, name, transa, gathered):
-    """16 groups with 64 MiB of weights: enough that those of groups with one tile of rows are loaded non-temporally; against one plain
+    """16 groups with 64 MiB of weights: enough that those of groups with one tile of rows are loaded non-temporally where the mean group has one; against one plain
     matmul a group, which loads them as ever.  Every element is accumulated over k in the same order: bit for bit."""
     be, M, K = backend, 2048, 1032
     counts = np.array(FEW_ROWS[name], dtype=np.int32)
