@@ -193,12 +193,16 @@ extern "C" int amd_matmul_planned_tile(int M, int K, int N, int has_c, int cu_co
  * some 290 MiB that is run again and again loses 5-15 % by it, and from there on nothing is found in the cache either way.
  * It is another instance of the kernel, with a copy of the loop for each kind of load: a choice between two copies that no group of a launch needs cost it
  * about 1 % (900 tokens, 8 experts, top 2, 1024 x 1024 51.8 -> 52.4, 1624, 23, 2, 3328 x 512 137.7 -> 138.8).  So it is taken only where the mean group has no
- * more rows than a tile: over 44 drawn forwards, 27 of them so, even and Zipf routers, 0.88-1.00 of the time without (two of 14 and 24 tokens, whose few experts stay in
- * the cache, 1.05), the others 1.00, and no Zipf router with more rows gained by it (0.996-1.005). */
+ * more rows than a tile, and no more than 96: over sets of weights beyond the cache, even and Zipf routers, 27 drawn forwards with fewer rows 0.88-1.00 of the time without (two of 14
+ * and 24 tokens, whose few experts stay in the cache, 1.05), 17 with more than a tile 1.00; between 96 and 128 rows it is 0.96-1.03 (1259 tokens, 61 experts, top 5,
+ * 3712 x 1152 416 -> 428, 1540, 16, 1, 1792 x 1280 103 -> 99).  Training steps of one layer, whose backward finds in the cache what plain loads of the
+ * forward leave there: 36 drawn ones 0.93-1.03, 0.972 in the mean; above 1.01 only where weights of 290-450 MiB meet 64-110 rows an expert (608 tokens, 41, 5,
+ * 2304 x 832 450 -> 460). */
 #define STREAM_WEIGHTS_BYTES (48u << 20)
+#define STREAM_WEIGHTS_MOST_ROWS 96
 static bool streams_weights(const GemmParams & p, int tile_rows) {
-	const long filled = p.N < p.num_groups ? p.N : p.num_groups;
-	return p.N <= tile_rows * filled && (uint64_t) filled * (uint64_t) p.M * (uint64_t) p.K * 2u > STREAM_WEIGHTS_BYTES;
+	const long filled = p.N < p.num_groups ? p.N : p.num_groups, rows = tile_rows < STREAM_WEIGHTS_MOST_ROWS ? tile_rows : STREAM_WEIGHTS_MOST_ROWS;
+	return p.N <= rows * filled && (uint64_t) filled * (uint64_t) p.M * (uint64_t) p.K * 2u > STREAM_WEIGHTS_BYTES;
 }
 
 /* one tile of the direct kernel, with or without them */

@@ -103,7 +103,7 @@ FEW_ROWS = {
     "32": [0, 1, 31, 32, 33, 2, 16, 64, 65, 0, 30, 7, 32, 31, 5, 1],
     "64": [63, 64, 65, 1, 0, 32, 33, 128, 129, 60, 64, 63, 40, 90, 50, 64],
     "128": [127, 128, 129, 255, 256, 257, 0, 1, 100, 128, 127, 140, 90, 120, 128, 110],
-    "128 in the mean": [127, 128, 129, 1, 0, 100, 128, 127, 90, 120, 128, 110, 64, 257, 126, 3],
+    "96 in the mean": [127, 128, 129, 1, 0, 100, 128, 127, 90, 120, 128, 10, 64, 255, 126, 3],
 }
 
 
