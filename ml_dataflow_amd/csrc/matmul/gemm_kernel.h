@@ -1198,8 +1198,8 @@ gemm_bf16_direct_kernel(GemmParams p) {
 	}
 
 	/* the descriptors end with the operand of this problem: anything outside reads as zero */
-#define ISSUE_STAGE(addr, kt_) do { \
-		ldP.template issue<decltype(p_once)::value>((addr), (kt_), t.K, wave); \
+#define ISSUE_STAGE(once, addr, kt_) do { \
+		ldP.template issue<once>((addr), (kt_), t.K, wave); \
 		ldQ.issue((addr) + BM * BK * 2, (kt_), t.K, wave); \
 	} while (0)
 
@@ -1230,58 +1230,74 @@ gemm_bf16_direct_kernel(GemmParams p) {
 	 * k-tile kt.  The loads have the whole multiply phase to land.
 	 * Loads past the last k-tile are out of range of the buffer and fill LDS with zeros: an odd tile count
 	 * costs one multiply of a zero tile instead of control flow around 256 live accumulators. */
-	/* In two copies: with a branch at each load the loop's schedule is lost (the router's logits of 8192 tokens 14.7 -> 17.1 us). */
-	const auto multiply = [&](auto p_once) {
-		if constexpr (STAGES == 2) {
-			ISSUE_STAGE(stage0_addr, kt_begin);
-			for (int kt = kt_begin; kt < k_tiles; kt += 2) {
-				WAIT_VMCNT(0);
-				__syncthreads();
-				ISSUE_STAGE(stage1_addr, kt + 1);
-				COMPUTE_STAGE(stage0);
-				WAIT_VMCNT(0);
-				__syncthreads();
-				ISSUE_STAGE(stage0_addr, kt + 2);
-				COMPUTE_STAGE(stage1);
+	/* More than two stages.  Iteration for k-tile kt (stage kt mod STAGES): the loads of kt .. kt + STAGES - 2 are out; wait until only those
+	 * behind kt are (loads complete in order), barrier -- kt is visible, and nobody reads the stage of kt-1 any more --
+	 * start the load of kt + STAGES - 1 into that stage, multiply kt.  Loads that run ahead past the end are never
+	 * multiplied. */
+	constexpr uint32_t STAGE_BYTES = (BM + BN) * BK * 2;
+	static_assert(STAGES == 2 || (STAGES - 2) * LOADS_PER_STAGE < 64, "vmcnt is a 6-bit counter");
+#define MULTIPLY_TILES(once) do { \
+		if constexpr (STAGES == 2) { \
+			ISSUE_STAGE(once, stage0_addr, kt_begin); \
+			for (int kt = kt_begin; kt < k_tiles; kt += 2) { \
+				WAIT_VMCNT(0); \
+				__syncthreads(); \
+				ISSUE_STAGE(once, stage1_addr, kt + 1); \
+				COMPUTE_STAGE(stage0); \
+				WAIT_VMCNT(0); \
+				__syncthreads(); \
+				ISSUE_STAGE(once, stage0_addr, kt + 2); \
+				COMPUTE_STAGE(stage1); \
+			} \
+		} else { \
+			_Pragma("unroll") \
+			for (int u = 0; u < STAGES - 1; u++) { \
+				ISSUE_STAGE(once, stage0_addr + u * STAGE_BYTES, kt_begin + u); \
+			} \
+			for (int kt = kt_begin; kt < k_tiles; kt += STAGES) { \
+				_Pragma("unroll") \
+				for (int u = 0; u < STAGES; u++) { \
+					if (kt + u < k_tiles) { \
+						WAIT_VMCNT((STAGES - 2) * LOADS_PER_STAGE); \
+						__syncthreads(); \
+						ISSUE_STAGE(once, stage0_addr + ((u + STAGES - 1) % STAGES) * STAGE_BYTES, kt + u + STAGES - 1); \
+						COMPUTE_STAGE(stages[u]); \
+					} \
+				} \
+			} \
+		} \
+	} while (0)
+
+	/* ONCE: the loop in two copies; with a branch at each load its schedule is lost (the router's logits of 8192 tokens 14.7 -> 17.1 us).  The 64 x 32
+	 * tile has it in a closure: there the compiler leaves the accumulators in their registers, which it otherwise copies from one kind to the other in every
+	 * k-tile (forward of 256 tokens, dim 512, 26.4 and 25.5 us).  Larger tiles are the slower ones for it: 5380 x 640 x 3648 on 128 x 128, gradient of the weight,
+	 * 50.6 and 51.8. */
+	if constexpr (BN == 32) {
+		const auto multiply = [&](auto once) { MULTIPLY_TILES(decltype(once)::value); };
+		if constexpr (ONCE) {
+			if (t.N <= BN) {                           /* the group's rows fit one tile: each line of its weights goes to one work-group */
+				multiply(std::true_type());
+			} else {
+				multiply(std::false_type());
 			}
-		} else {
-			/* Iteration for k-tile kt (stage kt mod STAGES): the loads of kt .. kt + STAGES - 2 are out; wait until only those
-			 * behind kt are (loads complete in order), barrier -- kt is visible, and nobody reads the stage of kt-1 any more --
-			 * start the load of kt + STAGES - 1 into that stage, multiply kt.  Loads that run ahead past the end are never
-			 * multiplied. */
-			constexpr uint32_t STAGE_BYTES = (BM + BN) * BK * 2;
-			static_assert((STAGES - 2) * LOADS_PER_STAGE < 64, "vmcnt is a 6-bit counter");
-			#pragma unroll
-			for (int u = 0; u < STAGES - 1; u++) {
-				ISSUE_STAGE(stage0_addr + u * STAGE_BYTES, kt_begin + u);
-			}
-			for (int kt = kt_begin; kt < k_tiles; kt += STAGES) {
-				#pragma unroll
-				for (int u = 0; u < STAGES; u++) {
-					if (kt + u < k_tiles) {
-						WAIT_VMCNT((STAGES - 2) * LOADS_PER_STAGE);
-						__syncthreads();
-						ISSUE_STAGE(stage0_addr + ((u + STAGES - 1) % STAGES) * STAGE_BYTES, kt + u + STAGES - 1);
-						COMPUTE_STAGE(stages[u]);
-					}
-				}
-			}
-		}
-	};
-	if constexpr (ONCE) {
-		static_assert(MODE == MODE_RAGGED_N, "the groups' weights are streamed");
-		if (t.N <= BN) {                               /* the group's rows fit one tile: each line of its weights goes to one work-group */
-			multiply(std::true_type());
 		} else {
 			multiply(std::false_type());
 		}
+	} else if constexpr (ONCE) {
+		if (t.N <= BN) {
+			MULTIPLY_TILES(true);
+		} else {
+			MULTIPLY_TILES(false);
+		}
 	} else {
-		multiply(std::false_type());
+		MULTIPLY_TILES(false);
 	}
+	static_assert(!ONCE || MODE == MODE_RAGGED_N, "the groups' weights are streamed");
 	WAIT_VMCNT(0);                             /* drain the trailing (zero-filling) loads before the LDS is released */
 	__syncthreads();
 #undef ISSUE_STAGE
 #undef COMPUTE_STAGE
+#undef MULTIPLY_TILES
 
 	if (split >= 0) {
 		store_partial<TM, TN>(t, p.partial + (long long) split * t.M * t.N, acc, wm, wn, lane);
