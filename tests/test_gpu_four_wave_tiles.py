@@ -109,6 +109,31 @@ def test_ragged_n_partial_last_rounds(backend, select_kernel, n_tiles, gathered,
         d.free()
 
 
+@pytest.mark.parametrize("gathered", [False, True])
+@pytest.mark.parametrize("groups,tiles", [(20, 2), (33, 2), (16, 8), (20, 3), (17, 4)])
+def test_ragged_n_groups_of_the_same_tiles(backend, select_kernel, groups, tiles, gathered):
+    """Groups of as many tiles each, four tiles high: 8, 16 and 32 of them go into a die's 32 work-groups, whose last tiles are not cut then, 12 do not;
+    partial last rounds, rows of a group from one in its last tile to all."""
+    be = backend
+    M, K, src_rows = 1016, 256, 997
+    rng = np.random.default_rng(groups + tiles)
+    counts = (384 * (tiles - 1) + rng.choice([1, 63, 64, 65, 128, 129, 192, 193, 257, 320, 383, 384], size=groups)).astype(np.int32)
+    counts[0], counts[-1] = 384 * tiles, 384 * (tiles - 1) + 1
+    total = int(counts.sum())
+    assert total // 256 * -(-M // 256) >= 128                          # from there on a named kernel runs, not the direct one on both sides
+    print("case groups of the same tiles: groups=%d tiles=%d gathered=%d rows=%d" % (groups, tiles, gathered, total), flush=True)
+    d_W, d_X = be.upload(normal_bf16(rng, (groups, M, K), 0.05)), be.upload(normal_bf16(rng, (src_rows if gathered else total, K)))
+    d_cum, d_map = be.upload(np.cumsum(counts).astype(np.int32)), be.upload(rng.integers(-1, src_rows + 1, total).astype(np.int32))
+    args = (be.hp, CS, BF, BF, B.DATAFLOW_NONE, BF, B.DATAFLOW_FP32, 1, 0, B.AMD_GROUPED_RAGGED_N, M, K, total, groups, d_cum.ptr, 1.0, 0.0, d_W.ptr, M * K * 2, d_X.ptr, None)
+    if gathered:
+        submit = lambda d_D: be.lib.dataflow_submit_amd_grouped_matmul_gathered(*args, d_D.ptr, 0, d_map.ptr, src_rows)
+    else:
+        submit = lambda d_D: be.lib.dataflow_submit_amd_grouped_matmul(*args, d_D.ptr, 0)
+    both(be, select_kernel, FOUR_384, total * M, np.zeros(total * M, np.uint16), submit)
+    for d in (d_W, d_X, d_cum, d_map):
+        d.free()
+
+
 @pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (1.0, 1.0), (-0.75, 0.0), (1.5, -0.5)])
 @pytest.mark.parametrize("M,N,groups", [(264, 520, 64), (1304, 264, 70), (256, 256, 300)])
 def test_ragged_k_tiles_and_slices(backend, select_kernel, alpha, beta, M, N, groups):
